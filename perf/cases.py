@@ -249,8 +249,8 @@ def work(case):
 
 
 def tolerance(case):
-    # about four times what the outputs measure against the same step in 64 bits, relative: fp16 2.1e-4 (attention 2.9e-4), bf16 1.7e-3 (one
-    # rounding to the output type after fp32 sums), fp32 products at most 6e-7 (an order of the sums; 1.3e-6 with other orders of a long K)
+    # four times or so what the outputs measure against the same step in 64 bits, relative: fp16 2.1e-4 (attention 2.9e-4), bf16 1.7e-3 (one
+    # rounding to the output type after fp32 sums), fp32 products at most 6e-7 (K = 1024; twice that leaves room for the order of a longer sum)
     dt = case["dtype"]
     if case["family"] == "gemm" and dt == "int8":
         return "exact"
