@@ -200,6 +200,10 @@ static int sub_round_split(const KernelEntry* k, int64_t tiles, int64_t kt) {
   return split;
 }
 
+// K tile of the kernel that stages through registers against the one of the same tile that transfers straight to LDS (fp16 NN, us,
+// registers against copy + LDS transfers on 128x128 tiles: 4095x4097x4001 304 / 227, 1999x4099x3001 154 / 100, 1001x999x1003 31 / 21)
+static constexpr double kStagedFactor = 1.6;
+
 static double estimated_cost(const KernelEntry* k, const frisk_gemm_desc* d, bool may_split = false) {
   const int64_t tiles = ((d->M + k->bm - 1) / k->bm) * ((d->N + k->bn - 1) / k->bn);
   const double kt = (double)((d->K + k->bk - 1) / k->bk);
@@ -231,7 +235,7 @@ static double estimated_cost(const KernelEntry* k, const frisk_gemm_desc* d, boo
     // 3 + 3 tiles when the grid is one wave, 2 + 2 (two work-groups per CU) beyond
     c = k->stages >= 3 ? (tiles <= 256 ? 0.46 : 0.55) : (tiles <= 256 ? 0.55 : 0.52);
   }
-  if (k->guard) c *= 3.0;
+  if (k->guard && !k->edge) c *= kStagedFactor;
   if (k->bm == 32 && k->wk > 1) {
     // The 32x32 kernel streams B.  With a ring of 4 tiles one work-group fills a CU: whole rounds of 256, each paying its
     // own start (measured 14.8 us for 256 tiles, 35.8 for 512).  With a ring of 2 two work-groups share a CU: slower alone
@@ -381,7 +385,7 @@ static double small_grid_time(const SmallGridModel& m, const KernelEntry* k, con
   }
   t += (double)full * whole + (rest ? last : 0.0);
   if (split > 1) t += m.r0 + m.r1 * ((double)d->M * (double)d->N * split * 4.0 / 1e6);
-  return k->guard ? 3.0 * t : t;
+  return k->guard && !k->edge ? kStagedFactor * t : t;
 }
 // the split of a variant: among the powers of two the rule admits, the one the model makes fastest; *cost receives its time
 static int small_grid_split(const KernelEntry* k, const frisk_gemm_desc* d, bool no_split, double* cost = nullptr) {
@@ -405,7 +409,26 @@ static double small_grid_cost(const KernelEntry* k, const frisk_gemm_desc* d, bo
   return t;
 }
 
-static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_model, bool force_guard = false, bool no_split = false) {
+// What a launch knows beyond the descriptor: pointers off 16-byte boundaries (C: or a column-scale pointer off its vector), and
+// whether there is a workspace to use.
+struct PlanContext { bool a_off = false, b_off = false, c_off = false, no_workspace = false; };
+// Operands that are copied to aligned rows in the workspace before the product runs, and where they go.
+struct Repack { bool a = false, b = false; int64_t lda = 0, ldb = 0; size_t b_offset = 0, bytes = 0; };
+
+static Repack repack_of(const frisk_gemm_desc* d, bool a, bool b) {
+  Repack r;
+  const int es = elem_size(d->dtype_ab), per16 = 16 / es;
+  r.a = a; r.b = b;
+  const int64_t a_rows = d->transA ? d->K : d->M, a_cols = d->transA ? d->M : d->K, b_rows = d->transB ? d->N : d->K, b_cols = d->transB ? d->K : d->N;
+  r.lda = (a_cols + per16 - 1) / per16 * per16;
+  r.ldb = (b_cols + per16 - 1) / per16 * per16;
+  if (a) r.b_offset = ((size_t)a_rows * (size_t)r.lda * es + 255) & ~(size_t)255;
+  r.bytes = r.b_offset + (b ? (size_t)b_rows * (size_t)r.ldb * es : 0);
+  return r;
+}
+
+static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_model, const PlanContext& ctx = {}, Repack* repack = nullptr) {
+  const bool no_split = ctx.no_workspace;
   int st = validate(d);
   if (st != FRISK_OK) return st;
   if (!plan) return fail(FRISK_ERR_NULL, "plan is null");
@@ -418,7 +441,12 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
   if (d->epilogue == FRISK_EPI_TENSOR_SCALE) plan->bytes += 8.0;
   plan->split_k = 1;
 
-  const bool rows_aligned = (d->lda * es) % 16 == 0 && (d->ldb * es) % 16 == 0 && (d->ldc * os) % 16 == 0;
+  const bool a_aligned = (d->lda * es) % 16 == 0 && !ctx.a_off, b_aligned = (d->ldb * es) % 16 == 0 && !ctx.b_off;
+  const bool rows_aligned = a_aligned && b_aligned && (d->ldc * os) % 16 == 0 && !ctx.c_off;
+  // what it would take to put the operands' rows on 16-byte boundaries, in bytes and in microseconds: a dependent launch, and every
+  // byte read and written once
+  const Repack packed = repack_of(d, !a_aligned, !b_aligned);
+  const double repack_cost = packed.bytes ? 4.0 + (double)packed.bytes / 2.2e6 : 0.0;
   const auto& ks = kernels();
   int best = -1;
   double best_cost = 0.0;
@@ -448,26 +476,30 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
       // a kernel whose loop needs a minimum of K tiles: per slice when the descriptor asks for a split
       if (k->min_k_tiles > 1 && (d->K + k->bk - 1) / k->bk / (want_split && d->split_k > 1 ? d->split_k : 1) < k->min_k_tiles) continue;
       // the fast kernels need whole tiles and rows that start on 16-byte boundaries; their edge variants take any M and N (and
-      // are left out where the plain twin fits); the guarded ones take anything
+      // are left out where the plain twin fits)
       const bool whole_mn = d->M % k->bm == 0 && d->N % k->bn == 0;
-      if (!k->guard && (force_guard || !rows_aligned || d->K % k->bk || (k->edge ? whole_mn : !whole_mn))) continue;
-      // the guarded kernels that move whole 16-byte chunks: aligned rows and pointers, K a whole number of chunks
-      if (k->guard && k->edge && (force_guard || !rows_aligned || d->K % (16 / es))) continue;
+      if (!k->guard && (!rows_aligned || d->K % k->bk || (k->edge ? whole_mn : !whole_mn))) continue;
+      // the edge kernels once more under their guarded names: K off the K tile (a whole number of chunks), and anything at all,
+      // with A and B copied to aligned rows where theirs are not
+      if (k->guard == 1 && k->edge && (!rows_aligned || d->K % (16 / es))) continue;
+      if (k->guard == 2 && packed.bytes && (no_split || d->split_k != 0)) continue;
       // ... and address a tile's chunks by 32-bit lane offsets from its first row: the stored rows of one tile must span
       // less than 4 GiB
-      const double span_a = (double)d->lda * es * (d->transA ? k->bk : k->bm), span_b = (double)d->ldb * es * (d->transB ? k->bn : k->bk);
-      if (!k->guard && (span_a >= 4294967296.0 || span_b >= 4294967296.0)) continue;
+      const double span_a = (double)(packed.a ? packed.lda : d->lda) * es * (d->transA ? k->bk : k->bm),
+                   span_b = (double)(packed.b ? packed.ldb : d->ldb) * es * (d->transB ? k->bn : k->bk);
+      if ((!k->guard || k->edge) && (span_a >= 4294967296.0 || span_b >= 4294967296.0)) continue;
       if (k->guard && best >= 0 && !ks[best]->guard) continue;  // never a guarded kernel when a fast one fits
       double cost = small && !want_split ? small_grid_cost(k, d, no_split) : estimated_cost(k, d, !want_split && !no_split && d->split_k == 0);
       // (a 32-row edge tile above 64 rows streams B once per 32 rows where the 64-row tile wastes at most as much: 130x11008x4096
       // NT 64.5 against 53.5 us)
       if (k->edge && k->bm == 32 && d->M > 64 && !d->tile_m) continue;
-      if (k->edge && !k->guard) {
+      if (k->edge) {
         // the models see whole tiles; rows and columns beyond M and N are work all the same (a 64-row tile on 32 rows is no
         // better than the 32-row tile that fits): the square root of the covered area over M x N, as a penalty
         const double covered = (double)((d->M + k->bm - 1) / k->bm * k->bm) * (double)((d->N + k->bn - 1) / k->bn * k->bn);
         cost *= std::sqrt(covered / ((double)d->M * (double)d->N));
       }
+      if (k->guard == 2) cost += repack_cost;
       // ties: the first listed variant is the tuned default
       if (best < 0 || (ks[best]->guard && !k->guard) || cost < best_cost) { best = (int)i; best_cost = cost; }
     }
@@ -502,11 +534,15 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
   plan->stages_b = k->stages_b;
   plan->grid_x = (int)((d->N + k->bn - 1) / k->bn);
   plan->grid_y = (int)((d->M + k->bm - 1) / k->bm);
-  plan->guarded = k->guard;
+  plan->guarded = k->guard != 0;
   plan->xcd_remap = ((int64_t)plan->grid_x * plan->grid_y) % 8 == 0;
   fill_layout(&plan->lds_a, !d->transA, es, frag_bytes(d->dtype_ab), k->bm, k->bk, k->wm * k->wn * k->wk, with_model, k->atom);
   fill_layout(&plan->lds_b, d->transB != 0, es, frag_bytes(d->dtype_ab), k->bn, k->bk, k->wm * k->wn * k->wk, with_model, k->atom);
   plan->workspace_bytes = 0;
+  if (k->guard == 2 && packed.bytes) {
+    plan->workspace_bytes = packed.bytes;
+    if (repack) *repack = packed;
+  }
   // Split K over the grid's y dimension when the tile grid alone leaves most CUs idle (skinny problems are
   // bound by streaming the large operand, which needs many work-groups in flight).  Slices hold whole K tiles.
   const int64_t kt = d->K / k->bk, tiles = (int64_t)plan->grid_x * plan->grid_y;
@@ -603,7 +639,12 @@ size_t frisk_hip_workspace_bytes(const frisk_gemm_desc* desc) {
 int frisk_hip_gemm(const frisk_gemm_desc* desc, const void* A, const void* B, void* C, const float* scaleA,
                    const float* scaleB, void* workspace, size_t workspace_bytes, void* stream) {
   frisk_gemm_plan plan;
-  int st = make_plan(desc, &plan, false);
+  Repack repack;
+  PlanContext ctx;
+  ctx.a_off = (uintptr_t)A & 15;
+  ctx.b_off = (uintptr_t)B & 15;
+  ctx.c_off = ((uintptr_t)C & 15) || (desc && desc->epilogue == FRISK_EPI_ROW_COL_SCALE && ((uintptr_t)scaleB & 15));
+  int st = make_plan(desc, &plan, false, ctx, &repack);
   if (st != FRISK_OK) return st;
   if (desc->M == 0 || desc->N == 0) return FRISK_OK;
   if (!A || !B || !C) return fail(FRISK_ERR_NULL, "A, B and C must be device pointers");
@@ -611,19 +652,15 @@ int frisk_hip_gemm(const frisk_gemm_desc* desc, const void* A, const void* B, vo
   const uintptr_t es = (uintptr_t)elem_size(desc->dtype_ab), os = (uintptr_t)elem_size(desc->dtype_out);
   if (((uintptr_t)A | (uintptr_t)B) & (es - 1) || (uintptr_t)C & (os - 1) || (((uintptr_t)scaleA | (uintptr_t)scaleB) & 3))
     return fail(FRISK_ERR_ALIGNMENT, "pointers must be aligned to their element size");
-  const bool ptrs16 = ((((uintptr_t)A | (uintptr_t)B | (uintptr_t)C) & 15) == 0) &&
-                      !(desc->epilogue == FRISK_EPI_ROW_COL_SCALE && ((uintptr_t)scaleB & 15));
-  if (!ptrs16 && !plan.guarded) {  // the fast kernels move 16-byte chunks: fall back to the guarded kernel
-    st = make_plan(desc, &plan, false, true);
-    if (st != FRISK_OK) return st;
-  }
   if (plan.workspace_bytes > 0 && (!workspace || workspace_bytes < plan.workspace_bytes)) {
     // an explicit split_k needs its workspace; the planner's own choice degrades to a single pass without one
     if (desc->split_k > 1) return fail(FRISK_ERR_WORKSPACE, "split_k=%d needs %zu bytes of workspace", desc->split_k, plan.workspace_bytes);
-    st = make_plan(desc, &plan, false, plan.guarded != 0, true);
+    ctx.no_workspace = true;
+    repack = Repack{};
+    st = make_plan(desc, &plan, false, ctx);
     if (st != FRISK_OK) return st;
   }
-  if ((plan.split_k > 1 || plan.tail_split > 1) && ((uintptr_t)workspace & 15)) return fail(FRISK_ERR_ALIGNMENT, "workspace must be 16-byte aligned");
+  if (plan.workspace_bytes > 0 && ((uintptr_t)workspace & 15)) return fail(FRISK_ERR_ALIGNMENT, "workspace must be 16-byte aligned");
   if (!device_ok()) return fail(FRISK_ERR_DEVICE, "no gfx950 device is current");
 
   GemmParams p;
@@ -644,7 +681,20 @@ int frisk_hip_gemm(const frisk_gemm_desc* desc, const void* A, const void* B, vo
   p.tail_kt = plan.tail_split > 1 ? p.kt_per_slice / plan.tail_split : 0;
   p.tile_m = k->bm; p.tile_n = k->bn;
   p.k_rotate = 1;
-  hipError_t e = k->launch(p, (hipStream_t)stream);
+  hipError_t e = hipSuccess;
+  if (repack.bytes) {
+    RepackParams r;
+    auto side = [&](RepackParams::Side& s, bool on, const void* src, void* dst, int64_t rows, int64_t cols, int64_t ld, int64_t dst_ld) {
+      if (on) s = {src, dst, ld * (int64_t)es, dst_ld * (int64_t)es, rows, cols * (int64_t)es};
+    };
+    side(r.a, repack.a, A, workspace, desc->transA ? desc->K : desc->M, desc->transA ? desc->M : desc->K, desc->lda, repack.lda);
+    side(r.b, repack.b, B, (char*)workspace + repack.b_offset, desc->transB ? desc->N : desc->K, desc->transB ? desc->K : desc->N, desc->ldb, repack.ldb);
+    if (repack.a) { p.A = r.a.dst; p.lda = repack.lda; }
+    if (repack.b) { p.B = r.b.dst; p.ldb = repack.ldb; }
+    e = launch_repack(r, (hipStream_t)stream);
+    if (e != hipSuccess) return fail(FRISK_ERR_DEVICE, "launch of the copy to aligned rows failed: %s", hipGetErrorString(e));
+  }
+  e = k->launch(p, (hipStream_t)stream);
   if (e != hipSuccess) return fail(FRISK_ERR_DEVICE, "launch of %s failed: %s", k->name, hipGetErrorString(e));
   if (plan.split_k > 1) {
     e = launch_splitk_reduce(p, desc->dtype_acc == FRISK_I32, (hipStream_t)stream);

@@ -57,10 +57,11 @@ struct KernelEntry {
   int bm, bn, bk, wm, wn;
   int stages, stages_b;  // LDS ring depth for A and for B (stages_b >= stages)
   int wk;  // waves splitting the K steps of a tile (1 = none)
-  int guard;  // 1: handles any shape / leading dimension (slower staging)
+  int guard;  // 1: named guarded: K off the K tile (with edge), or any alignment, staged through registers (without); 2: an edge kernel for
+              // any K, C and alignment, A and B being copied to aligned rows first
   int splitk;  // 1: compiled with the split-K store path
   int atom;  // rows and columns of the MFMA atom: 32 (32x32xK) or 16 (16x16x2K)
-  int edge;  // 1: M and N need not be multiples of the tile (K, and the alignment of rows and pointers, as for the plain kernels)
+  int edge;  // 1: M and N need not be multiples of the tile (and, without split-K, neither K nor the alignment of C matters)
   int lds_bytes;
   int min_k_tiles;  // fewest K tiles the kernel's loop is written for
   hipError_t (*launch)(const GemmParams&, hipStream_t);
@@ -71,6 +72,13 @@ struct KernelEntry {
 hipError_t launch_splitk_reduce(const GemmParams& p, int acc_is_int, hipStream_t stream);
 // the same for the tiles of a tail split
 hipError_t launch_tail_reduce(const GemmParams& p, int acc_is_int, hipStream_t stream);
+
+// Copies A and / or B to rows that start on 16-byte boundaries (repack.hip), the bytes behind a row's last one up to the next
+// boundary zero.  A side with no rows is left out.
+struct RepackParams {
+  struct Side { const void* src = nullptr; void* dst = nullptr; int64_t src_ld = 0, dst_ld = 0, rows = 0, row_bytes = 0; } a, b;  // bytes
+};
+hipError_t launch_repack(const RepackParams& p, hipStream_t stream);
 
 // defined in kernels_*.hip (two tables per element type: kernels_<type>.hip and kernels_<type>_2.hip)
 extern const KernelEntry kKernelsF16[];

@@ -73,12 +73,11 @@ typedef enum frisk_status {
  * Supported (dtype_ab -> dtype_acc -> dtype_out):
  *   F32->F32->F32, F16->F32->{F16,F32}, BF16->F32->{BF16,F32},
  *   I8->I32->{I32, F16 with ROW_COL_SCALE}, E4M3->F32->{BF16,F32} (NONE or TENSOR_SCALE)
- * tile_* and waves_* = 0 let the planner choose.  With rows and pointers on 16-byte boundaries and K a multiple of
- * the K tile (64 elements of 16 bits, 128 of 8 bits, 32 of fp32) the fast kernels run, for any M and N (where those
- * are no multiples of the tile, variants of the same kernels whose stores are checked against M and N); anything
- * else (K off the K tile, odd leading dimensions, element-aligned pointers, K = 0) runs a bounds-checked kernel with
- * the same arithmetic: one that moves 16-byte chunks while rows and pointers are aligned and K is a whole number of
- * chunks, an element-wise one otherwise.
+ * tile_* and waves_* = 0 let the planner choose.  With rows and pointers on 16-byte boundaries the fast kernels run,
+ * for any M, N and K (where those are no multiples of the tile, variants of the same kernels whose stores are checked
+ * against M and N and whose last K tile is cleared beyond K).  Where rows or pointers of A or B lie off those
+ * boundaries the operands are first copied to aligned rows in the workspace, if one is passed and split_k is 0 and the
+ * problem is large enough to repay it; a kernel that stages them through registers runs otherwise.
  */
 typedef struct frisk_gemm_desc {
   int32_t abi_version; /* FRISK_HIP_ABI_VERSION */
@@ -128,7 +127,7 @@ typedef struct frisk_gemm_plan {
   int32_t grid_x, grid_y;            /* work-group grid (tiles along N, tiles along M) */
   int32_t split_k;                   /* >1: partial sums go through the workspace */
   int32_t xcd_remap;                 /* 1: work-group ids are remapped so each XCD owns a compact block of tiles */
-  int32_t guarded;                   /* 1: a bounds-checked kernel runs (K off the K tile, unaligned rows or pointers) */
+  int32_t guarded;                   /* 1: K off the K tile, or unaligned rows or pointers */
   frisk_lds_layout lds_a, lds_b;
   size_t workspace_bytes;
   double flops;                      /* 2.M.N.K */
@@ -152,8 +151,8 @@ const char* frisk_hip_last_error(void);
 int frisk_hip_plan(const frisk_gemm_desc* desc, frisk_gemm_plan* plan);
 
 /* Pure host: bytes of device workspace `frisk_hip_gemm` wants for this descriptor: split_k * M * N * 4 when the
- * plan splits K, tail_split * tail_tiles * tile_m * tile_n * 4 for a tail split, else 0.  With split_k = 0 in the
- * descriptor a launch without workspace still runs, unsplit. */
+ * plan splits K, tail_split * tail_tiles * tile_m * tile_n * 4 for a tail split, the size of the operands with padded rows
+ * where they are copied, else 0.  With split_k = 0 in the descriptor a launch without workspace still runs, unsplit. */
 size_t frisk_hip_workspace_bytes(const frisk_gemm_desc* desc);
 
 /* Launch on `stream` (a hipStream_t, may be NULL for the default stream).

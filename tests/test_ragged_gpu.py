@@ -1,0 +1,96 @@
+"""Problems off the tiles on the device: a K that is no multiple of the K tile on the edge kernels, rows off 16-byte boundaries staged
+through registers (no workspace) and copied to aligned rows first (workspace).  Operands end with their last element, and the
+bytes around C are checked for stray writes."""
+import numpy as np
+import pytest
+
+import oracle as O
+from helpers import DEFAULT_OUT, TOL, from_dev, make_operand, stored_shapes, to_dev
+
+BK = {O.F32: 32, O.F16: 64, O.BF16: 64, O.I8: 128, O.E4M3: 128}
+ES = {O.F32: 4, O.F16: 2, O.BF16: 2, O.I8: 1, O.E4M3: 1}
+OUT_NP = {O.F32: np.float32, O.F16: np.uint16, O.BF16: np.uint16, O.I32: np.int32}
+
+
+def launch(hip, dtype, A, B, M, N, K, transA, transB, aligned, workspace=True, ldc_extra=0, **kw):
+    """A and B as stored, each row padded to a multiple of 16 bytes (`aligned`) or followed by one more element"""
+    import torch
+    per = 16 // ES[dtype]
+
+    def rows(x):
+        cols = x.shape[1]
+        ld = (cols + per - 1) // per * per if aligned else cols + 1 - (cols & 1)  # odd: no row but the first on a boundary
+        buf = np.zeros((x.shape[0], ld), x.dtype)
+        buf[:, :cols] = x
+        return to_dev(buf.reshape(-1)[:(x.shape[0] - 1) * ld + cols]), ld
+
+    (dA, lda), (dB, ldb) = rows(A), rows(B)
+    out = DEFAULT_OUT[dtype]
+    ldc = N + ldc_extra
+    guard = np.full(64 + M * ldc, 0x55, dtype=np.uint8).astype(OUT_NP[out])
+    dC = to_dev(guard)
+    d = hip.make_desc(dtype, M, N, K, dtype_out=out, transA=bool(transA), transB=bool(transB), lda=lda, ldb=ldb, ldc=ldc, **kw)
+    need = hip.workspace_bytes(d) if workspace else 0
+    ws = torch.full((max(need, 16),), 0xFF, dtype=torch.uint8, device="cuda")  # NaNs of every float type
+    hip.gemm(d, dA.data_ptr(), dB.data_ptr(), dC.data_ptr() + 32 * guard.itemsize, None, None, ws.data_ptr() if need else None, need,
+             torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    got = from_dev(dC, OUT_NP[out], (64 + M * ldc,))
+    inner = got[32:32 + M * ldc].reshape(M, ldc)
+    assert np.array_equal(got[:32], guard[:32]) and np.array_equal(got[32 + M * ldc:], guard[32 + M * ldc:]), "write outside C"
+    assert np.array_equal(inner[:, N:], guard[:M * ldc_extra].reshape(M, ldc_extra)), "write between the rows of C"
+    return inner[:, :N], hip.kernel_names()[hip.plan(d).kernel_id], need
+
+
+def verify(dtype, got, A, B, transA, transB):
+    if dtype == O.I8:
+        assert np.array_equal(got, O.gemm_i32(A, B, transA, transB))
+    else:
+        r = O.compare(DEFAULT_OUT[dtype], np.ascontiguousarray(got), O.gemm_f64(dtype, A, B, transA, transB))
+        assert r["nonfinite"] == 0 and r["max_rel"] <= TOL[dtype] and r["fro_rel"] <= TOL[dtype], r
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [O.F16, O.BF16, O.I8, O.E4M3, O.F32])
+@pytest.mark.parametrize("transA,transB", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_a_partial_last_k_tile_on_the_edge_kernels(hip, dtype, transA, transB):
+    """one to eight K tiles (every path through the prologue, the unrolled loop and the drain), the last one of 1 element up to all
+    but one, on both edge tiles; C rows off 16-byte boundaries"""
+    bk, big = BK[dtype], 128 if dtype == O.F32 else 256
+    M, N = 150, 301
+    for tile, ks in (((big, big, 0), (1, bk - 1, bk + 1, 2 * bk - 3, 2 * bk + 1, 3 * bk + 5, 8 * bk - 1)), ((big // 2, big // 2, 0), (7, bk + 3, 2 * bk + bk // 2, 4 * bk - 1))):
+        for K in ks:
+            A = make_operand(dtype, *stored_shapes(M, N, K, transA, transB)[0], seed=81, tensor=0, scale=0.5)
+            B = make_operand(dtype, *stored_shapes(M, N, K, transA, transB)[1], seed=81, tensor=1, scale=0.5)
+            got, name, need = launch(hip, dtype, A, B, M, N, K, transA, transB, True, ldc_extra=1, tile=tile, stages=2 if tile[0] != 256 else 3)
+            assert name.endswith("_guard") and need == 0, name
+            verify(dtype, got, A, B, transA, transB)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [O.F16, O.F32])
+def test_infinities_before_k_do_not_leak_into_the_cleared_part_of_a_k_tile(hip, dtype):
+    """the chunks fetched in place of those beyond K repeat values of the operand: an infinity among them must not meet a zero"""
+    M, N, K = 64, 64, BK[dtype] + 5
+    A = make_operand(dtype, M, K, seed=82, tensor=0, scale=0.5)
+    B = make_operand(dtype, K, N, seed=82, tensor=1, scale=0.5)
+    A[3, K - 1] = O.encode(dtype, np.array([np.inf], np.float32))[0]
+    B[K - 1, :] = O.encode(dtype, np.full(N, 0.25, np.float32))
+    got, _, _ = launch(hip, dtype, A, B, M, N, K, 0, 0, True)
+    f = got.astype(np.float32) if dtype == O.F32 else got.view(np.float16).astype(np.float32)
+    assert np.all(np.isposinf(f[3])) and np.all(np.isfinite(np.delete(f, 3, axis=0)))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [O.F16, O.BF16, O.I8, O.E4M3, O.F32])
+@pytest.mark.parametrize("transA,transB", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_rows_off_16_byte_boundaries(hip, dtype, transA, transB):
+    """sizes around a chunk, a tile and a K tile; once without a workspace (staged through registers) and once with (copied first)"""
+    bk = BK[dtype]
+    for (M, N, K) in ((1, 3, 5), (3, 130, 1), (17, 9, bk + 1), (129, 127, 2 * bk), (255, 131, 3 * bk - 1), (301, 515, 5 * bk + 7)):
+        A = make_operand(dtype, *stored_shapes(M, N, K, transA, transB)[0], seed=83, tensor=0, scale=0.5)
+        B = make_operand(dtype, *stored_shapes(M, N, K, transA, transB)[1], seed=83, tensor=1, scale=0.5)
+        for kw in (dict(workspace=False), dict(split_k=1), dict(tile=(128, 128, 0) if dtype == O.F32 else (256, 256, 0))):
+            got, name, need = launch(hip, dtype, A, B, M, N, K, transA, transB, False, **kw)
+            assert name.endswith("_guard") and (need > 0) == ("tile" in kw), (name, need)
+            verify(dtype, got, A, B, transA, transB)
