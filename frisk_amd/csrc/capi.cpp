@@ -849,7 +849,6 @@ int frisk_hip_elementwise(const frisk_elementwise_desc* d, const void* const* in
   for (int k = 0; k < d->n_inputs; ++k) dense = dense && d->in_col_stride[k] == 1 && d->in_row_stride[k] == d->cols;
   p.rows = dense ? 1 : d->rows;
   p.cols = dense ? d->rows * d->cols : d->cols;
-  bool vec = p.cols % 8 == 0 && rows_on_16_bytes(d->out_dtype, out, dense ? 0 : d->out_ld);
   for (int k = 0; k < d->n_inputs; ++k) {
     const int dt = d->in_dtype[k];
     if (dt != FRISK_F32 && dt != FRISK_F16 && dt != FRISK_BF16) return fail(FRISK_ERR_DTYPE, "elementwise operand %d: element type %d is not f32, f16 or bf16", k, dt);
@@ -857,13 +856,12 @@ int frisk_hip_elementwise(const frisk_elementwise_desc* d, const void* const* in
     if (d->in_row_stride[k] < 0) return fail(FRISK_ERR_SHAPE, "elementwise operand %d: negative row stride", k);
     if (!inputs[k]) return fail(FRISK_ERR_NULL, "elementwise operand %d: pointer is null", k);
     if ((uintptr_t)inputs[k] & (uintptr_t)(elem_size(dt) - 1)) return fail(FRISK_ERR_ALIGNMENT, "elementwise operand %d: pointer is not aligned to its element size", k);
-    if (d->in_col_stride[k] == 1) vec = vec && rows_on_16_bytes(dt, inputs[k], dense ? 0 : d->in_row_stride[k]);
     p.in[k] = inputs[k]; p.in_row_stride[k] = d->in_row_stride[k]; p.in_dtype[k] = dt; p.in_col_stride[k] = d->in_col_stride[k];
   }
   if (!device_ok()) return fail(FRISK_ERR_DEVICE, "no gfx950 device is current");
   p.out = out; p.out_ld = d->out_ld; p.out_dtype = d->out_dtype; p.n_ops = d->n_ops;
   for (int i = 0; i < d->n_ops; ++i) { p.op[i] = d->op[i]; p.arg[i] = d->arg[i]; p.imm[i] = d->imm[i]; }
-  hipError_t e = launch_elementwise(p, vec ? 1 : 0, (hipStream_t)stream);
+  hipError_t e = launch_elementwise(p, (hipStream_t)stream);
   if (e != hipSuccess) return fail(FRISK_ERR_DEVICE, "elementwise launch failed: %s", hipGetErrorString(e));
   return FRISK_OK;
 }

@@ -3,11 +3,17 @@
 // the value.  The reference defines the op and lowers it nowhere.  Here the expression arrives as a postfix program (at
 // most FRISK_EW_MAX_OPS steps over FRISK_EW_MAX_INPUTS operands) and ONE kernel interprets it: no run-time compilation.
 //
-// A lane evaluates 8 consecutive columns at a time through 16-byte accesses; the program counter and every opcode are
-// wave-uniform (the program sits in registers, a step is a lane read and a scalar branch), and the evaluation stack lives
-// in registers: one switch on (stack depth, opcode) names the slots each snippet touches, so nothing is indexed at run
-// time.  All arithmetic is fp32; the result is rounded once to the output type.  A one-step program moves 5.3 TB/s,
-// y = log2(max(x, c) / (x + c)) (8 steps, one IEEE division) 2.2 TB/s on a 32768 x 8192 f16 view.
+// What bounds it is the vector pipe and the dispatch of a step, not memory, so the host first turns the postfix steps into steps of a
+// machine with a top value: a binary operation whose right operand is an input or a constant takes it directly, and only a value
+// that must survive goes below the top.  A lane evaluates 8 consecutive columns at a time.  The loop over the steps is written as inline
+// assembly over fixed registers: a step is two lane reads of the program, a jump to its handler and 8 vector instructions in
+// place, the operand picked by the register index mode.  (As a C++ switch the compiler joins the values of all cases after every
+// step by register moves: 327 vector, 300 scalar and 120 branch instructions per group of 8 columns for (x - s * c) * g + b; here
+// 136, 171 and 35.)  That body on 8192 x 8192 f16: 139 us before, 62.7 now (a plain copy: 41); log2(max(x, c) / (x + c)), bound by
+// the vector pipe in its division, 125 -> 71.5; rows off 16-byte boundaries (4095 x 8191) 370 -> 51.
+// Operands that are the same for every row stay in registers while the lane's columns do, values of one per row stay one
+// register, and what the next group needs from memory is fetched while the current one is evaluated.  All arithmetic is
+// fp32; the result is rounded once to the output type.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include "tile_ops.h"
@@ -16,159 +22,359 @@ namespace frisk {
 namespace {
 
 typedef unsigned v4u __attribute__((ext_vector_type(4)));
-static_assert(FRISK_EW_MAX_STACK == 6, "the interpreter below names six stack slots");
+// 16 bytes that start on any element: loads and stores of this type are one instruction at any address
+typedef unsigned v4u_any __attribute__((ext_vector_type(4), aligned(2)));
+constexpr int V = 8;  // columns per lane and step
 
-// element (row, col .. col + V - 1) of operand k as floats; cs = 0 broadcasts one element along the row
-template <int V, bool VEC>
-__device__ __forceinline__ void load_operand(const EwParams& p, int k, int64_t row, int64_t col, int64_t cols, float (&out)[V]) {
-  const int dt = p.in_dtype[k];
-  const int64_t base = row * p.in_row_stride[k] + (p.in_col_stride[k] ? col : 0);
-  const char* ptr = (const char*)p.in[k];
-  if (!p.in_col_stride[k]) {
-    float x;
-    if (dt == FRISK_F32) x = ((const float*)ptr)[base];
-    else if (dt == FRISK_F16) x = (float)((const _Float16*)ptr)[base];
-    else x = (float)((const __bf16*)ptr)[base];
+// The machine.  Registers of a lane, 8 columns each: top v[16:23] and the slots v[24 + 8 j : 31 + 8 j], which a step names by 8 j:
+// below the top S0 (j = 0) and, in deep programs, S1 .. S4 (j = 5 .. 8); X (1) what a step fetched or a quotient's divisor; COL0, COL1
+// (2, 3) operands that are the same for every row; WALK2 (4) the second operand that walks the rows.  v14, v15: values of one per row.
+// A step is (handler << 24) | (input of STEP_FETCH << 8) | register index; constants lie beside it.  Suffix V: operand in a slot, S: constant,
+// R: value of the row.  STEP_END .. STEP_DIV* leave the assembly; the quotient and the fetch are C++.
+enum Step {
+  STEP_END = 0, STEP_MORE, STEP_FETCH, STEP_DIVV, STEP_RDIVV, STEP_DIVS, STEP_DIVR,  // leave the assembly
+  STEP_SAVE, STEP_LOADV, STEP_LOADS, STEP_LOADR, STEP_ADDV, STEP_ADDS, STEP_ADDR, STEP_SUBV, STEP_RSUBV, STEP_SUBR, STEP_MULV, STEP_MULS, STEP_MULR,
+  STEP_MAXV, STEP_MAXS, STEP_MAXR, STEP_MINV, STEP_MINS, STEP_MINR, STEP_NEG, STEP_EXP2, STEP_LOG2
+};
+constexpr int kSlotS0 = 0, kSlotX = 8, kSlotCol0 = 16, kSlotCol1 = 24, kSlotWalk2 = 32, kSlotS1 = 40;
+constexpr int kChunk = 64;  // steps in one register of a wave, one per lane; STEP_MORE goes on to the second register
+struct EwSteps {
+  int code[2 * kChunk];
+  float imm[2 * kChunk];
+  int depth;              // most values below the top at any time
+  int head, walk2;        // operands fetched a group ahead: the one the program starts with, and another that walks the rows (-1: none)
+  int col0, col1;         // operands that are the same for every row, kept in registers while the columns stay
+  int row0, row1;         // operands of one value per row, fetched a group ahead
+};
+
+// ---- the interpreter loop.  EACH: one instruction per column.  Handlers lie 256 bytes apart, in the order of Step; NEXT fetches
+// the step s51 counts and jumps to its handler.  s50 holds the step being run, s56 its constant.  (A lane select written by a scalar
+// instruction, the index mode and a jump need no wait states; a vector instruction that reads an exponential or a logarithm needs one.)
+#define EW_EACH(I) ".irp e,0,1,2,3,4,5,6,7\n" I "\n.endr\n"
+#define EW_NEXT                                                                                                              \
+  "v_readlane_b32 s50, v12, s51\nv_readlane_b32 s56, v13, s51\ns_addk_i32 s51, 1\ns_lshr_b32 s52, s50, 16\n"              \
+  "s_add_u32 s54, s48, s52\ns_addc_u32 s55, s49, 0\ns_setpc_b64 s[54:55]\n"
+#define EW_HANDLER(BODY) ".p2align 8\n" BODY EW_NEXT
+#define EW_LEAVE(BODY) ".p2align 8\n" BODY "s_branch .Lew_out%=\n"
+#define EW_INDEXED(I) "s_set_gpr_idx_on s50, gpr_idx(SRC0)\n" EW_EACH(I) "s_set_gpr_idx_off\n"
+#define EW_V(OP) EW_HANDLER(EW_INDEXED(OP " v[16+\\e], v[24+\\e], v[16+\\e]"))
+#define EW_S(OP) EW_HANDLER(EW_EACH(OP " v[16+\\e], s56, v[16+\\e]"))
+#define EW_R(OP) EW_HANDLER(EW_INDEXED(OP " v[16+\\e], v14, v[16+\\e]"))
+// maximum and minimum ignore a NaN operand, a signalling one too: both sides go through X and a maximum with themselves first
+#define EW_QUIET_TOP EW_EACH("v_max_f32 v[16+\\e], v[16+\\e], v[16+\\e]")
+#define EW_MV(OP)                                                                                                            \
+  EW_HANDLER("s_set_gpr_idx_on s50, gpr_idx(SRC0,SRC1)\n" EW_EACH("v_max_f32 v[32+\\e], v[24+\\e], v[24+\\e]")       \
+             "s_set_gpr_idx_off\n" EW_QUIET_TOP EW_EACH(OP " v[16+\\e], v[32+\\e], v[16+\\e]"))
+#define EW_MS(OP) EW_HANDLER(EW_QUIET_TOP EW_EACH(OP " v[16+\\e], s56, v[16+\\e]"))
+#define EW_MR(OP)                                                                                                            \
+  EW_HANDLER("s_set_gpr_idx_on s50, gpr_idx(SRC0,SRC1)\nv_max_f32 v32, v14, v14\ns_set_gpr_idx_off\n" EW_QUIET_TOP          \
+             EW_EACH(OP " v[16+\\e], v32, v[16+\\e]"))
+#define EW_INTERPRETER                                                                                                       \
+  "s_getpc_b64 s[48:49]\n.Lew_here%=:\ns_add_u32 s48, s48, (.Lew_handlers%=-.Lew_here%=)&4294967295\n"                     \
+  "s_addc_u32 s49, s49, (.Lew_handlers%=-.Lew_here%=)>>32\n" EW_NEXT ".p2align 8\n.Lew_handlers%=:\n"                       \
+  EW_LEAVE("") EW_LEAVE("") EW_LEAVE("")                                                                   /* END MORE FETCH */ \
+  EW_LEAVE(EW_INDEXED("v_mov_b32 v[32+\\e], v[24+\\e]"))                                                        /* DIVV */  \
+  EW_LEAVE(EW_EACH("v_mov_b32 v[32+\\e], v[16+\\e]") EW_INDEXED("v_mov_b32 v[16+\\e], v[24+\\e]"))            /* RDIVV */ \
+  EW_LEAVE(EW_EACH("v_mov_b32 v[32+\\e], s56")) EW_LEAVE(EW_INDEXED("v_mov_b32 v[32+\\e], v14"))          /* DIVS DIVR */ \
+  EW_HANDLER("s_set_gpr_idx_on s50, gpr_idx(DST)\n" EW_EACH("v_mov_b32 v[24+\\e], v[16+\\e]") "s_set_gpr_idx_off\n") /* SAVE */ \
+  EW_HANDLER(EW_INDEXED("v_mov_b32 v[16+\\e], v[24+\\e]")) EW_HANDLER(EW_EACH("v_mov_b32 v[16+\\e], s56"))           \
+  EW_HANDLER(EW_INDEXED("v_mov_b32 v[16+\\e], v14"))                                               /* LOADV LOADS LOADR */ \
+  EW_V("v_add_f32") EW_S("v_add_f32") EW_R("v_add_f32")                                                                      \
+  EW_V("v_subrev_f32") EW_V("v_sub_f32") EW_R("v_subrev_f32")                                             /* SUBV RSUBV SUBR */ \
+  EW_V("v_mul_f32") EW_S("v_mul_f32") EW_R("v_mul_f32")                                                                      \
+  EW_MV("v_max_f32") EW_MS("v_max_f32") EW_MR("v_max_f32") EW_MV("v_min_f32") EW_MS("v_min_f32") EW_MR("v_min_f32")          \
+  EW_HANDLER(EW_EACH("v_xor_b32 v[16+\\e], 0x80000000, v[16+\\e]"))                                               /* NEG */  \
+  EW_HANDLER(EW_EACH("v_exp_f32 v[16+\\e], v[16+\\e]") "s_nop 0\n")                                                     \
+  EW_HANDLER(EW_EACH("v_log_f32 v[16+\\e], v[16+\\e]") "s_nop 0\n")                                                     \
+  ".Lew_out%=:\n"
+#define EW_CLOBBERS "s48", "s49", "s52", "s54", "s55", "s56", "scc"
+
+typedef float v8f __attribute__((ext_vector_type(8)));
+
+struct Raw { v4u a, b; };  // 8 elements of a 32-bit operand, or (a) of a 16-bit one
+
+__device__ __forceinline__ Raw load_raw(const char* at, int dt, bool streamed) {
+  Raw r;
+  if (streamed) {
+    r.a = __builtin_nontemporal_load((const v4u_any*)at);
+    if (dt == FRISK_F32) r.b = __builtin_nontemporal_load((const v4u_any*)at + 1);
+  } else {
+    r.a = *(const v4u_any*)at;
+    if (dt == FRISK_F32) r.b = *((const v4u_any*)at + 1);
+  }
+  return r;
+}
+// the first `valid` (1 to 7) of 8 elements
+__device__ __forceinline__ Raw load_raw_partial(const char* at, int dt, int valid) {
+  unsigned w[8] = {0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
-    for (int e = 0; e < V; ++e) out[e] = x;
+  for (int e = 0; e < V; ++e) {
+    if (e >= valid) continue;
+    if (dt == FRISK_F32) w[e] = ((const unsigned*)at)[e];
+    else w[e / 2] |= (unsigned)((const uint16_t*)at)[e] << (16 * (e & 1));
+  }
+  return Raw{v4u{w[0], w[1], w[2], w[3]}, v4u{w[4], w[5], w[6], w[7]}};
+}
+template <class F> __device__ __forceinline__ void to_float(const Raw& r, int dt, F& out) {
+  if (dt == FRISK_F32) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const unsigned lo = r.a[e], hi = r.b[e];  // copy first: bit_cast applied to a vector element reads element 0
+      out[e] = __builtin_bit_cast(float, lo);
+      out[4 + e] = __builtin_bit_cast(float, hi);
+    }
+  } else if (dt == FRISK_F16) {
+    typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+    const h8 h = __builtin_bit_cast(h8, r.a);
+#pragma unroll
+    for (int e = 0; e < V; ++e) out[e] = (float)h[e];
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) { out[2 * e] = __builtin_bit_cast(float, r.a[e] << 16); out[2 * e + 1] = __builtin_bit_cast(float, r.a[e] & 0xffff0000u); }
+  }
+}
+__device__ __forceinline__ float load_one(const char* at, int dt) {
+  if (dt == FRISK_F32) return *(const float*)at;
+  if (dt == FRISK_F16) return (float)*(const _Float16*)at;
+  return (float)*(const __bf16*)at;
+}
+__device__ __forceinline__ void store_group(char* at, int dt, const v8f& r, int valid) {
+  if (valid >= V) {
+    if (dt == FRISK_F32) {
+      v4u a, b;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) { const float lo = r[e], hi = r[4 + e]; a[e] = __builtin_bit_cast(unsigned, lo); b[e] = __builtin_bit_cast(unsigned, hi); }
+      *(v4u_any*)at = a;
+      *((v4u_any*)at + 1) = b;
+    } else if (dt == FRISK_F16) {
+      typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+      h8 h;
+#pragma unroll
+      for (int e = 0; e < V; ++e) h[e] = (_Float16)r[e];
+      __builtin_nontemporal_store(__builtin_bit_cast(v4u, h), (v4u_any*)at);
+    } else {
+      typedef __bf16 b8 __attribute__((ext_vector_type(8)));
+      b8 h;
+#pragma unroll
+      for (int e = 0; e < V; ++e) h[e] = (__bf16)r[e];
+      __builtin_nontemporal_store(__builtin_bit_cast(v4u, h), (v4u_any*)at);
+    }
     return;
   }
-  if constexpr (VEC) {
 #pragma unroll
-    for (int c = 0; c < V / 8; ++c) {  // 8 columns at a time: 32 bytes of a 32-bit operand, 16 of a 16-bit one
-      if (dt == FRISK_F32) {
-        const v4u* q = (const v4u*)(ptr + (base + 8 * c) * 4);
-        const v4u a = __builtin_nontemporal_load(q), b = __builtin_nontemporal_load(q + 1);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const unsigned lo = a[e], hi = b[e];  // copy first: bit_cast applied to a vector element reads element 0
-          out[8 * c + e] = __builtin_bit_cast(float, lo);
-          out[8 * c + 4 + e] = __builtin_bit_cast(float, hi);
-        }
-      } else {
-        const v4u a = __builtin_nontemporal_load((const v4u*)(ptr + (base + 8 * c) * 2));
-        if (dt == FRISK_F16) {
-          typedef _Float16 h8 __attribute__((ext_vector_type(8)));
-          const h8 h = __builtin_bit_cast(h8, a);
-#pragma unroll
-          for (int e = 0; e < 8; ++e) out[8 * c + e] = (float)h[e];
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) { out[8 * c + 2 * e] = __builtin_bit_cast(float, a[e] << 16); out[8 * c + 2 * e + 1] = __builtin_bit_cast(float, a[e] & 0xffff0000u); }
-        }
-      }
-    }
-  } else {
-#pragma unroll
-    for (int e = 0; e < V; ++e) {
-      float x = 0.f;
-      if (col + e < cols) {
-        if (dt == FRISK_F32) x = ((const float*)ptr)[base + e];
-        else if (dt == FRISK_F16) x = (float)((const _Float16*)ptr)[base + e];
-        else x = (float)((const __bf16*)ptr)[base + e];
-      }
-      out[e] = x;
-    }
+  for (int e = 0; e < V; ++e) {
+    if (e >= valid) continue;
+    if (dt == FRISK_F32) ((float*)at)[e] = r[e];
+    else if (dt == FRISK_F16) ((_Float16*)at)[e] = (_Float16)r[e];
+    else ((__bf16*)at)[e] = (__bf16)r[e];
   }
 }
 
-template <int V> __device__ __forceinline__ void ew_store(const EwParams& p, int64_t at, const float (&r)[V]) {
-  char* dst = (char*)p.out;
-  if constexpr (V > 1) {
-#pragma unroll
-    for (int c = 0; c < V / 8; ++c) {
-      if (p.out_dtype == FRISK_F32) {
-        v4u a, b;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) { a[e] = __builtin_bit_cast(unsigned, r[8 * c + e]); b[e] = __builtin_bit_cast(unsigned, r[8 * c + 4 + e]); }
-        __builtin_nontemporal_store(a, (v4u*)(dst + (at + 8 * c) * 4));
-        __builtin_nontemporal_store(b, (v4u*)(dst + (at + 8 * c) * 4) + 1);
-      } else if (p.out_dtype == FRISK_F16) {
-        typedef _Float16 h8 __attribute__((ext_vector_type(8)));
-        h8 h;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) h[e] = (_Float16)r[8 * c + e];
-        __builtin_nontemporal_store(__builtin_bit_cast(v4u, h), (v4u*)(dst + (at + 8 * c) * 2));
-      } else {
-        typedef __bf16 b8 __attribute__((ext_vector_type(8)));
-        b8 h;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) h[e] = (__bf16)r[8 * c + e];
-        __builtin_nontemporal_store(__builtin_bit_cast(v4u, h), (v4u*)(dst + (at + 8 * c) * 2));
-      }
-    }
-  } else {
-    if (p.out_dtype == FRISK_F32) ((float*)dst)[at] = r[0];
-    else if (p.out_dtype == FRISK_F16) ((_Float16*)dst)[at] = (_Float16)r[0];
-    else ((__bf16*)dst)[at] = (__bf16)r[0];
-  }
-}
-
-// The interpreter.  The evaluation stack is six plain arrays s0 .. s5 (slot k of the stack is sk); one switch on
-// (stack depth, opcode) selects a straight-line snippet in which the slots an opcode touches are named, so nothing is ever
-// indexed at run time and the stack stays in registers.  The host has checked that no step underflows or overflows.
-template <int V> __global__ void __launch_bounds__(256) elementwise_kernel(EwParams p, int lanes_log2) {
-  constexpr bool VEC = V > 1;
-  const int64_t groups = (p.cols + V - 1) / V;
+// DT: element type of the operands that walk the rows and of the output (-1: mixed, read from the arguments).  AHEAD: the operands
+// named in EwSteps beside `head` are held or fetched ahead (44 more registers for 32-bit operands, 32 for 16-bit ones).  DEPTH: values
+// below the top the program needs.  UNIFORM_ROW: a wave's lanes lie in one row (rows of at least 64 groups).
+template <int DT, bool AHEAD, int DEPTH, bool UNIFORM_ROW> __global__ void __launch_bounds__(256) elementwise_kernel(EwParams p, EwSteps prog, int lanes_log2) {
   const int lanes = 1 << lanes_log2, row_step = 256 >> lanes_log2;
-  const int lane_group = threadIdx.x & (lanes - 1), lane_row = threadIdx.x >> lanes_log2;
-  // The program sits in three registers, step i in lane i (FRISK_EW_MAX_OPS <= 64): a step is fetched with a lane read
-  // instead of a dependent scalar load from the kernel arguments, whose latency every step of every element group paid.
-  static_assert(FRISK_EW_MAX_OPS <= 64, "one program step per lane of a wave");
-  const int my_step = (threadIdx.x & 63) < FRISK_EW_MAX_OPS ? (int)(threadIdx.x & 63) : 0;
-  int ops_reg = p.op[my_step], args_reg = p.arg[my_step];
-  float imms_reg = p.imm[my_step];
-  // pinned here, with every lane active: the lane reads below happen inside loops that lanes leave at different times,
-  // and a load that the compiler moved down to its use there would fill only the lanes still running
-  asm volatile("" : "+v"(ops_reg), "+v"(args_reg), "+v"(imms_reg));
-  for (int64_t row = (int64_t)blockIdx.y * row_step + lane_row; row < p.rows; row += (int64_t)gridDim.y * row_step)
-    for (int64_t g = (int64_t)blockIdx.x * lanes + lane_group; g < groups; g += (int64_t)gridDim.x * lanes) {
-      const int64_t col = g * V;
-      float s0[V], s1[V], s2[V], s3[V], s4[V], s5[V];
-      int sp = 0;
-      for (int pc = 0; pc < p.n_ops; ++pc) {
-        const int op = __builtin_amdgcn_readlane(ops_reg, pc), arg = __builtin_amdgcn_readlane(args_reg, pc);
-        const float imm = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, imms_reg), pc));
-#define FRISK_EW_EACH(STMT) _Pragma("unroll") for (int e = 0; e < V; ++e) { STMT; }
-#define FRISK_EW_PUSH(SP, NEXT)                                                                                  \
-  case SP * 16 + FRISK_EW_INPUT: load_operand<V, VEC>(p, arg, row, col, p.cols, NEXT); sp = SP + 1; break;     \
-  case SP * 16 + FRISK_EW_CONST: FRISK_EW_EACH(NEXT[e] = imm) sp = SP + 1; break;
-#define FRISK_EW_UNARY(SP, TOP)                                                                                  \
-  case SP * 16 + FRISK_EW_NEG: FRISK_EW_EACH(TOP[e] = -TOP[e]) break;                                            \
-  case SP * 16 + FRISK_EW_EXP2: FRISK_EW_EACH(TOP[e] = __builtin_amdgcn_exp2f(TOP[e])) break;                    \
-  case SP * 16 + FRISK_EW_LOG2: FRISK_EW_EACH(TOP[e] = __builtin_amdgcn_logf(TOP[e])) break; /* v_log_f32: base 2 */
-#define FRISK_EW_BINARY(SP, A, B) /* the operand pushed first (A) is the left one; MAX / MIN ignore a NaN operand */ \
-  case SP * 16 + FRISK_EW_ADD: FRISK_EW_EACH(A[e] = A[e] + B[e]) sp = SP - 1; break;                            \
-  case SP * 16 + FRISK_EW_SUB: FRISK_EW_EACH(A[e] = A[e] - B[e]) sp = SP - 1; break;                            \
-  case SP * 16 + FRISK_EW_MUL: FRISK_EW_EACH(A[e] = A[e] * B[e]) sp = SP - 1; break;                            \
-  case SP * 16 + FRISK_EW_DIV: FRISK_EW_EACH(A[e] = A[e] / B[e]) sp = SP - 1; break;                            \
-  case SP * 16 + FRISK_EW_MAX: FRISK_EW_EACH(A[e] = __builtin_fmaxf(A[e], B[e])) sp = SP - 1; break;            \
-  case SP * 16 + FRISK_EW_MIN: FRISK_EW_EACH(A[e] = __builtin_fminf(A[e], B[e])) sp = SP - 1; break;
-        switch (sp * 16 + op) {  // wave-uniform
-          FRISK_EW_PUSH(0, s0)
-          FRISK_EW_PUSH(1, s1) FRISK_EW_UNARY(1, s0)
-          FRISK_EW_PUSH(2, s2) FRISK_EW_UNARY(2, s1) FRISK_EW_BINARY(2, s0, s1)
-          FRISK_EW_PUSH(3, s3) FRISK_EW_UNARY(3, s2) FRISK_EW_BINARY(3, s1, s2)
-          FRISK_EW_PUSH(4, s4) FRISK_EW_UNARY(4, s3) FRISK_EW_BINARY(4, s2, s3)
-          FRISK_EW_PUSH(5, s5) FRISK_EW_UNARY(5, s4) FRISK_EW_BINARY(5, s3, s4)
-          FRISK_EW_UNARY(6, s5) FRISK_EW_BINARY(6, s4, s5)
-          default: break;
-        }
-#undef FRISK_EW_EACH
-#undef FRISK_EW_PUSH
-#undef FRISK_EW_UNARY
-#undef FRISK_EW_BINARY
-      }
-      ew_store<V>(p, row * p.out_ld + col, s0);
+  const int lane_group = threadIdx.x & (lanes - 1);
+  int lane_row = threadIdx.x >> lanes_log2;
+  if constexpr (UNIFORM_ROW) lane_row = __builtin_amdgcn_readfirstlane(lane_row);
+  const int64_t groups = (p.cols + V - 1) / V, slabs = (groups + lanes - 1) >> lanes_log2, row_blocks = (p.rows + row_step - 1) / row_step;
+  const bool ragged = p.cols % V != 0;
+  // step i of a chunk of the program in lane i: a lane read instead of a dependent scalar load
+  int code_reg[2], imm_reg[2];
+#pragma unroll
+  for (int c = 0; c < 2; ++c) { code_reg[c] = prog.code[c * kChunk + (threadIdx.x & 63)]; imm_reg[c] = __builtin_bit_cast(int, prog.imm[c * kChunk + (threadIdx.x & 63)]); }
+  auto type_of = [&](int k) { return DT >= 0 ? DT : p.in_dtype[k]; };
+  // where this lane is in step (rb, slab): lanes beyond the view repeat its last row or group and store nothing
+  struct Place { int64_t row; int off, valid; bool live; };
+  auto place = [&](int64_t rb_, int64_t slab_) {
+    Place q;
+    const int64_t row = rb_ * row_step + lane_row, left = groups - (slab_ << lanes_log2);
+    q.live = row < p.rows && lane_group < left;
+    q.row = row < p.rows ? row : p.rows - 1;
+    q.off = lane_group < left ? lane_group : (int)left - 1;
+    const int64_t rest = p.cols - ((slab_ << lanes_log2) + q.off) * V;
+    q.valid = rest < V ? (int)rest : V;
+    return q;
+  };
+  // element (row, first column of the group) of operand k, whose elements are of type dt
+  auto operand_at = [&](int k, int dt, bool walks, const Place& q, int64_t slab_) {
+    const int es = dt == FRISK_F32 ? 4 : 2;
+    const char* base = (const char*)p.in[k] + q.row * (p.in_row_stride[k] * es);
+    return walks ? base + (slab_ << lanes_log2) * (V * es) + (unsigned)(q.off * (V * es)) : base;
+  };
+  auto fetch = [&](int k, int dt, const Place& q, int64_t slab_, bool streamed) {
+    const char* at = operand_at(k, dt, true, q, slab_);
+    if (!ragged || q.valid >= V) return load_raw(at, dt, streamed);
+    return load_raw_partial(at, dt, q.valid);
+  };
+  auto fetch_row = [&](int k, const Place& q) {
+    const char* at = operand_at(k, p.in_dtype[k], false, q, 0);
+    return p.in_dtype[k] == FRISK_F32 ? *(const unsigned*)at : (unsigned)*(const uint16_t*)at;
+  };
+  auto row_value = [&](int k, unsigned bits) {
+    if (p.in_dtype[k] == FRISK_F32) return __builtin_bit_cast(float, bits);
+    if (p.in_dtype[k] == FRISK_F16) return (float)__builtin_bit_cast(_Float16, (uint16_t)bits);
+    return __builtin_bit_cast(float, bits << 16);
+  };
+
+  int64_t rb = blockIdx.y, slab = blockIdx.x;
+  if (rb >= row_blocks || slab >= slabs) return;
+  Place here = place(rb, slab);
+  Raw ahead{}, ahead2{};
+  unsigned row0 = 0, row1 = 0;
+  v8f col0{}, col1{};
+  auto fetch_ahead = [&](const Place& q, int64_t slab_) {
+    if (prog.head >= 0) ahead = fetch(prog.head, type_of(prog.head), q, slab_, true);
+    if constexpr (AHEAD) {
+      if (prog.walk2 >= 0) ahead2 = fetch(prog.walk2, type_of(prog.walk2), q, slab_, true);
+      if (prog.row0 >= 0) row0 = fetch_row(prog.row0, q);
+      if (prog.row1 >= 0) row1 = fetch_row(prog.row1, q);
     }
+  };
+  auto fetch_cols = [&](const Place& q, int64_t slab_) {
+    if constexpr (AHEAD) {
+      if (prog.col0 >= 0) to_float(fetch(prog.col0, p.in_dtype[prog.col0], q, slab_, false), p.in_dtype[prog.col0], col0);
+      if (prog.col1 >= 0) to_float(fetch(prog.col1, p.in_dtype[prog.col1], q, slab_, false), p.in_dtype[prog.col1], col1);
+    }
+  };
+  fetch_ahead(here, slab);
+  fetch_cols(here, slab);
+  for (;;) {
+    int64_t next_rb = rb, next_slab = slab + gridDim.x;
+    if (next_slab >= slabs) { next_slab = blockIdx.x; next_rb += gridDim.y; }
+    const bool more = next_rb < row_blocks;
+    const Place there = place(more ? next_rb : rb, more ? next_slab : slab);
+    v8f top, s0, s1, s2, s3, s4, x, walk2;
+    asm volatile("" : "=v"(top), "=v"(s0), "=v"(x), "=v"(walk2));  // written by the program before it reads them
+    if constexpr (DEPTH > 1) asm volatile("" : "=v"(s1), "=v"(s2), "=v"(s3), "=v"(s4));
+    float row_a = 0.f, row_b = 0.f;
+    if (prog.head >= 0) to_float(ahead, type_of(prog.head), top);
+    if constexpr (AHEAD) {
+      if (prog.walk2 >= 0) to_float(ahead2, type_of(prog.walk2), walk2);
+      if (prog.row0 >= 0) row_a = row_value(prog.row0, row0);
+      if (prog.row1 >= 0) row_b = row_value(prog.row1, row1);
+    }
+    if (more) fetch_ahead(there, next_slab);
+    int pc = 0, code = code_reg[0], imm = imm_reg[0];
+    for (;;) {
+      int step;
+      if constexpr (AHEAD && DEPTH > 1)
+        asm volatile(EW_INTERPRETER : "={s50}"(step), "+{s51}"(pc), "+{v[16:23]}"(top), "+{v[24:31]}"(s0), "+{v[32:39]}"(x), "+{v[64:71]}"(s1), "+{v[72:79]}"(s2),
+                     "+{v[80:87]}"(s3), "+{v[88:95]}"(s4) : "{v12}"(code), "{v13}"(imm), "{v14}"(row_a), "{v15}"(row_b), "{v[40:47]}"(col0), "{v[48:55]}"(col1),
+                     "{v[56:63]}"(walk2) : EW_CLOBBERS);
+      else if constexpr (AHEAD)
+        asm volatile(EW_INTERPRETER : "={s50}"(step), "+{s51}"(pc), "+{v[16:23]}"(top), "+{v[24:31]}"(s0), "+{v[32:39]}"(x) : "{v12}"(code), "{v13}"(imm),
+                     "{v14}"(row_a), "{v15}"(row_b), "{v[40:47]}"(col0), "{v[48:55]}"(col1), "{v[56:63]}"(walk2) : EW_CLOBBERS);
+      else if constexpr (DEPTH > 1)
+        asm volatile(EW_INTERPRETER : "={s50}"(step), "+{s51}"(pc), "+{v[16:23]}"(top), "+{v[24:31]}"(s0), "+{v[32:39]}"(x), "+{v[64:71]}"(s1), "+{v[72:79]}"(s2),
+                     "+{v[80:87]}"(s3), "+{v[88:95]}"(s4) : "{v12}"(code), "{v13}"(imm) : EW_CLOBBERS);
+      else
+        asm volatile(EW_INTERPRETER : "={s50}"(step), "+{s51}"(pc), "+{v[16:23]}"(top), "+{v[24:31]}"(s0), "+{v[32:39]}"(x) : "{v12}"(code), "{v13}"(imm) : EW_CLOBBERS);
+      const int what = step >> 24;
+      if (what == STEP_END) break;
+      if (what == STEP_FETCH) {
+        const int k = (step >> 8) & 15;
+        if (p.in_col_stride[k]) to_float(fetch(k, p.in_dtype[k], here, slab, false), p.in_dtype[k], x);
+        else x = v8f{} + row_value(k, fetch_row(k, here));
+      } else if (what == STEP_MORE) {
+        code = code_reg[1];
+        imm = imm_reg[1];
+        pc = 0;
+      } else {
+#pragma unroll
+        for (int e = 0; e < V; ++e) top[e] = top[e] / x[e];
+      }
+    }
+    if (here.live) {
+      const int dt = DT >= 0 ? DT : p.out_dtype, es = dt == FRISK_F32 ? 4 : 2;
+      char* at = (char*)p.out + here.row * (p.out_ld * es) + (slab << lanes_log2) * (V * es) + (unsigned)(here.off * (V * es));
+      store_group(at, dt, top, here.valid);
+    }
+    if (!more) break;
+    if (next_slab != slab) fetch_cols(there, next_slab);
+    rb = next_rb;
+    slab = next_slab;
+    here = there;
+  }
+}
+
+// The postfix program as steps.  `ahead`: inputs may be held in slots (else each mention is fetched where it stands).
+EwSteps steps_of(const EwParams& p, bool ahead) {
+  EwSteps s{};
+  s.head = s.walk2 = s.col0 = s.col1 = s.row0 = s.row1 = -1;
+  int n = 0, below = -1;  // steps so far, values below the top
+  auto emit = [&](int what, int index = 0, float imm = 0.f, int input = 0) {
+    if (n == kChunk - 1) s.code[n++] = STEP_MORE << 24;
+    s.code[n] = what << 24 | input << 8 | index;
+    s.imm[n++] = imm;
+  };
+  auto slot_below = [](int depth) { return depth == 1 ? kSlotS0 : kSlotS1 + 8 * (depth - 2); };  // of the depth-th value below the top
+  const int by_slot[6] = {STEP_ADDV, STEP_SUBV, STEP_MULV, STEP_DIVV, STEP_MAXV, STEP_MINV};
+  const int by_const[6] = {STEP_ADDS, STEP_ADDS, STEP_MULS, STEP_DIVS, STEP_MAXS, STEP_MINS};  // x - c is x + (-c)
+  const int by_row[6] = {STEP_ADDR, STEP_SUBR, STEP_MULR, STEP_DIVR, STEP_MAXR, STEP_MINR};
+  const int from_below[6] = {STEP_ADDV, STEP_RSUBV, STEP_MULV, STEP_RDIVV, STEP_MAXV, STEP_MINV};  // the value below is the left operand
+  bool seen[FRISK_EW_MAX_INPUTS] = {};
+  for (int i = 0; i < p.n_ops; ++i) {
+    const int op = p.op[i];
+    if (op == FRISK_EW_INPUT || op == FRISK_EW_CONST) {
+      const int k = op == FRISK_EW_INPUT ? p.arg[i] : 0, next = i + 1 < p.n_ops ? p.op[i + 1] : -1;
+      const bool walks = p.in_col_stride[k] != 0;
+      if (op == FRISK_EW_INPUT && !seen[k]) {
+        seen[k] = true;
+        if (i == 0 && walks) s.head = k;
+        else if (!ahead) {}
+        else if (!walks) { if (s.row0 < 0) s.row0 = k; else if (s.row1 < 0) s.row1 = k; }
+        else if (p.in_row_stride[k] == 0 && p.rows > 1) { if (s.col0 < 0) s.col0 = k; else if (s.col1 < 0) s.col1 = k; }
+        else if (s.walk2 < 0) s.walk2 = k;
+      }
+      const bool fused = next >= FRISK_EW_ADD && next <= FRISK_EW_MIN;  // pushed only to be the right operand of the next step
+      if (!fused && ++below > 0) emit(STEP_SAVE, slot_below(below));
+      if (below > s.depth) s.depth = below;
+      const int which = fused ? next - FRISK_EW_ADD : 0;
+      if (op == FRISK_EW_CONST) emit(fused ? by_const[which] : STEP_LOADS, 0, fused && next == FRISK_EW_SUB ? -p.imm[i] : p.imm[i]);
+      else if (k == s.row0 || k == s.row1) emit(fused ? by_row[which] : STEP_LOADR, k == s.row1);
+      else if (i == 0 && k == s.head) {}  // the top starts with it
+      else {
+        const int slot = k == s.walk2 ? kSlotWalk2 : k == s.col0 ? kSlotCol0 : k == s.col1 ? kSlotCol1 : kSlotX;
+        if (slot == kSlotX) emit(STEP_FETCH, 0, 0.f, k);
+        emit(fused ? by_slot[which] : STEP_LOADV, slot);
+      }
+      i += fused;
+    } else if (op <= FRISK_EW_MIN) {
+      emit(from_below[op - FRISK_EW_ADD], slot_below(below));
+      --below;
+    } else {
+      emit(op == FRISK_EW_NEG ? STEP_NEG : op == FRISK_EW_EXP2 ? STEP_EXP2 : STEP_LOG2);
+    }
+  }
+  emit(STEP_END);
+  return s;
+}
+// two postfix steps make at most four steps (a value saved, fetched, loaded and combined from below)
+static_assert(2 * FRISK_EW_MAX_OPS + 2 <= 2 * kChunk, "a program fits into two chunks");
+
+template <int DT, bool AHEAD> void launch_typed(const dim3& grid, const EwParams& p, const EwSteps& prog, int lanes_log2, hipStream_t s) {
+#define FRISK_EW_LAUNCH(DEPTH)                                                                                                         \
+  if (lanes_log2 >= 6) hipLaunchKernelGGL((elementwise_kernel<DT, AHEAD, DEPTH, true>), grid, dim3(256), 0, s, p, prog, lanes_log2);   \
+  else hipLaunchKernelGGL((elementwise_kernel<DT, AHEAD, DEPTH, false>), grid, dim3(256), 0, s, p, prog, lanes_log2);
+  if (prog.depth <= 1) { FRISK_EW_LAUNCH(1) } else { FRISK_EW_LAUNCH(5) }
+#undef FRISK_EW_LAUNCH
 }
 
 }  // namespace
 
-hipError_t launch_elementwise(const EwParams& p, int vec_ok, hipStream_t s) {
-  // columns per lane and step: 8 through 16-byte accesses, else single elements.  (16 per lane halve the interpreter's cost
-  // per element but need 173 registers: two waves per SIMD keep too few bytes in flight, 3.2 against 5.3 TB/s for a copy.)
-  const int V = vec_ok ? 8 : 1;
+hipError_t launch_elementwise(const EwParams& p, hipStream_t s) {
+  // one type for everything that moves with the rows: the kernels for it; mixed types: the one that looks at each operand's type,
+  // which holds nothing ahead but the first operand
+  EwSteps prog = steps_of(p, true);
+  int dt = p.out_dtype;
+  bool ahead = prog.walk2 >= 0 || prog.col0 >= 0 || prog.row0 >= 0;
+  if ((prog.head >= 0 && p.in_dtype[prog.head] != dt) || (prog.walk2 >= 0 && p.in_dtype[prog.walk2] != dt)) {
+    dt = -1;
+    ahead = false;
+    prog = steps_of(p, false);
+  }
   const int64_t groups = (p.cols + V - 1) / V;
   int lanes_log2 = 0;
   while (lanes_log2 < 8 && ((int64_t)1 << lanes_log2) < groups) ++lanes_log2;
@@ -180,8 +386,12 @@ hipError_t launch_elementwise(const EwParams& p, int vec_ok, hipStream_t s) {
   if (gx * gy > cap) gy = (cap + gx - 1) / gx;
   if (gy > 65535) gy = 65535;
   const dim3 grid((unsigned)gx, (unsigned)gy);
-  if (V == 8) hipLaunchKernelGGL(elementwise_kernel<8>, grid, dim3(256), 0, s, p, lanes_log2);
-  else hipLaunchKernelGGL(elementwise_kernel<1>, grid, dim3(256), 0, s, p, lanes_log2);
+  switch (dt) {
+    case FRISK_F32: if (ahead) launch_typed<FRISK_F32, true>(grid, p, prog, lanes_log2, s); else launch_typed<FRISK_F32, false>(grid, p, prog, lanes_log2, s); break;
+    case FRISK_F16: if (ahead) launch_typed<FRISK_F16, true>(grid, p, prog, lanes_log2, s); else launch_typed<FRISK_F16, false>(grid, p, prog, lanes_log2, s); break;
+    case FRISK_BF16: if (ahead) launch_typed<FRISK_BF16, true>(grid, p, prog, lanes_log2, s); else launch_typed<FRISK_BF16, false>(grid, p, prog, lanes_log2, s); break;
+    default: launch_typed<-1, false>(grid, p, prog, lanes_log2, s); break;
+  }
   return hipGetLastError();
 }
 

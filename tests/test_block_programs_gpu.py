@@ -1,0 +1,77 @@
+"""The interpreter of frisk.block bodies at the edges of its step machine: programs of more than one chunk of steps, the deepest stack,
+every operation with its right operand a constant, a value of the row, a value of the column, a second walking operand or a
+value from below, more broadcast operands than there are slots, mixed element types, rows of any length and alignment."""
+import numpy as np
+import pytest
+
+import oracle as O
+from oracle import tile_ops as T
+
+ES = {O.F32: 4, O.F16: 2, O.BF16: 2}
+TOL = {O.F32: 3e-6, O.F16: 1e-3, O.BF16: 8e-3}
+BINARY = ["add", "sub", "mul", "div", "max", "min"]
+
+
+def run(hip, prog, operands, out_dt, rows, cols, in_place=None):
+    """operands: (dtype, kind, values as float) with kind walk | row | col | one; walking rows are one element longer than cols"""
+    import torch
+    bufs, ins, refs = [], [], []
+    for dt, kind, vals in operands:
+        st = O.encode(dt, np.ascontiguousarray(vals, dtype=np.float32).reshape(-1))
+        dec = O.decode(dt, st).astype(np.float64)
+        if kind == "walk":
+            padded = np.zeros((rows, cols + 1), st.dtype)
+            padded[:, :cols] = st.reshape(rows, cols)
+            bufs.append(torch.from_numpy(padded.view(np.uint8).reshape(-1).copy()).cuda())
+            ins.append((dt, cols + 1, 1))
+            refs.append(dec.reshape(rows, cols))
+        else:
+            bufs.append(torch.from_numpy(st.view(np.uint8).reshape(-1).copy()).cuda())
+            ins.append({"row": (dt, 1, 0), "col": (dt, 0, 1), "one": (dt, 0, 0)}[kind])
+            refs.append(dec.reshape({"row": (rows, 1), "col": (1, cols), "one": (1, 1)}[kind]))
+    want = T.elementwise(prog, refs, rows, cols)
+    out = torch.full((rows * (cols + 1) * ES[out_dt],), 0xEE, dtype=torch.uint8, device="cuda") if in_place is None else bufs[in_place]
+    before = out.cpu().numpy().view(O.NP_STORAGE[out_dt]).reshape(rows, cols + 1)[:, cols].copy()
+    hip.elementwise(hip.make_elementwise_desc(prog, ins, out_dt, rows, cols, out_ld=cols + 1), [b.data_ptr() for b in bufs], out.data_ptr(),
+                    torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    full = out.cpu().numpy().view(O.NP_STORAGE[out_dt]).reshape(rows, cols + 1)
+    assert np.array_equal(full[:, cols], before), "written between the rows"
+    got = O.decode(out_dt, np.ascontiguousarray(full[:, :cols])).astype(np.float64).reshape(rows, cols)
+    err = np.abs(got - want) / np.maximum(np.abs(want), 1.0)  # the operands are of the order of 1: so are the fp32 roundings inside
+    assert np.all(np.isfinite(want)) and err.max() <= TOL[out_dt], (prog, rows, cols, err.max())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", [O.F32, O.F16, O.BF16])
+@pytest.mark.parametrize("rows,cols", [(1, 1), (3, 7), (5, 64), (130, 513), (4, 20001)])
+def test_every_operation_with_every_kind_of_right_operand(hip, dt, rows, cols):
+    u = lambda n, t: O.uniform(n, 101, t, 0.5, 2.0)
+    ops = [(dt, "walk", u(rows * cols, 0)), (O.F32, "row", u(rows, 1)), (dt, "row", u(rows, 2)), (dt, "col", u(cols, 3)), (O.F32, "col", u(cols, 4)), (dt, "walk", u(rows * cols, 5)),
+           (dt, "one", u(1, 6)), (dt, "col", u(cols, 7))]
+    x = ("input", 0)
+    for op in BINARY:
+        for right in ([("const", 1.25)], *[[("input", k)] for k in range(8)], [x, ("const", 0.5), "add"]):
+            run(hip, [x] + right + [op], ops, dt, rows, cols)
+    run(hip, [x, "neg", "exp2", "log2", ("input", 5), "max"], ops, dt, rows, cols, in_place=0)
+
+
+@pytest.mark.gpu
+def test_long_and_deep_programs_and_mixed_types(hip):
+    rows, cols = 37, 300
+    u = lambda n, t: O.uniform(n, 102, t, 0.5, 1.5)
+    same = [(O.F16, "walk", u(rows * cols, 0)), (O.F16, "col", u(cols, 1)), (O.F16, "row", u(rows, 2)), (O.F16, "walk", u(rows * cols, 3)), (O.F16, "walk", u(rows * cols, 4))]
+    mixed = [(O.F32, "walk", u(rows * cols, 0)), (O.F16, "col", u(cols, 1)), (O.BF16, "row", u(rows, 2)), (O.BF16, "walk", u(rows * cols, 3)), (O.F16, "walk", u(rows * cols, 4))]
+    inputs = [("input", k) for k in range(5)]
+    # six values, folded from the top down; the divisor is at least 0.5 + 0.5 * 0.5, so that no rounding is magnified by more than 3 (a first
+    # form divided by a difference that came within 1e-5 of zero)
+    deep = inputs + [("input", 0)] + ["mul", "add", "div", "sub", "max"]
+    long_ = inputs[:4] + ["mul", "add", "sub"]                                               # then 40 more steps: 47 of 48
+    long_ += [s for k in range(20) for s in (("input", k % 5), ("add", "mul", "max", "min")[k % 4])]
+    unfused = [("input", 3)]                                                                # values saved, fetched, loaded and combined from below: two chunks
+    for k in range(11):
+        unfused += [("input", 4), "neg", "neg", "max" if k % 2 else "mul"]
+    for ops in (same, mixed):
+        for out in (O.F16, O.F32):
+            for prog in (deep, long_, unfused):
+                run(hip, prog, ops, out, rows, cols)
