@@ -175,15 +175,21 @@ static void fill_layout(frisk_lds_layout* L, bool kcontig, int es, int fragb, in
 // With a kernel that has the split-K store path, the last tiles % 256 tiles (at most half a round) are computed by 2, 4 or
 // 8 work-groups each, every one taking an equal share of the K tiles (at least 4).  Returns that count, 1 for no split.
 static int tail_split_of(const KernelEntry* k, int64_t tiles, int64_t kt, bool whole_k_tiles) {
-  if (!k->splitk || k->bm < 128 || k->wk > 1 || !whole_k_tiles || tiles <= 256) return 1;
+  // the edge kernels deal any number of K tiles: their last slice may be shorter (us unsplit / split: bf16 3000x11008x4096 NT, 516
+  // tiles, 248 / 212; fp16 4097x4097x4096 NT, 289 tiles, 161 / 126; 4095x4097x4001 NN with its copy to aligned rows 204 / 150)
+  const bool edge = k->edge && !k->splitk && (int64_t)k->bm * k->bn >= 256 * 256;
+  if (!edge && (!k->splitk || k->bm < 128 || k->wk > 1 || !whole_k_tiles)) return 1;
+  if (tiles <= 256) return 1;
   const int64_t rest = tiles % 256;
   if (rest == 0 || rest > 128) return 1;
   // shallower slices do not repay the second launch (measured); the 8-bit kernels run a K tile of twice the depth in the same
   // time, so the summing pass weighs twice as much against their slices (fp8 5120x4096x4096: 64 tiles in 4 slices of 8 K tiles
   // 92.4 us, unsplit 84, 256x128 tiles 81.4)
   const int min_slice = elem_size(k->dtype) == 1 ? 16 : 8;
-  for (int s = 8; s >= 2; s /= 2)
-    if (rest * s <= 256 && kt % s == 0 && kt / s >= min_slice) return s;
+  for (int s = 8; s >= 2; s /= 2) {
+    const int64_t per = (kt + s - 1) / s;
+    if (rest * s <= 256 && (edge ? (s - 1) * per < kt : kt % s == 0) && per >= min_slice) return s;
+  }
   return 1;
 }
 
@@ -254,7 +260,7 @@ static double estimated_cost(const KernelEntry* k, const frisk_gemm_desc* d, boo
     if (cs > 1) return kt / cs * c * (0.6 + 0.4 * rest_fill * cs) * 1.08 + 5.0 + 0.07 * (double)(tiles * cs);
   }
   double cost = (double)full * kt * c;
-  if (const int ts = tail_split_of(k, tiles, (int64_t)kt, d->K % k->bk == 0); ts > 1) {
+  if (const int ts = (k->edge && !k->splitk && !may_split) ? 1 : tail_split_of(k, tiles, (int64_t)kt, d->K % k->bk == 0); ts > 1) {
     // the last `rest` tiles as ts work-groups each, a ts-th of the K tiles apiece, plus the pass that sums them
     // (a dependent launch, and rest * ts tiles of 32-bit partial sums to read)
     return cost + kt / ts * c * (0.6 + 0.4 * rest_fill * ts) + 5.0 + 0.04 * (double)(rest * ts);
@@ -414,6 +420,9 @@ static double small_grid_cost(const KernelEntry* k, const frisk_gemm_desc* d, bo
 struct PlanContext { bool a_off = false, b_off = false, c_off = false, no_workspace = false; };
 // Operands that are copied to aligned rows in the workspace before the product runs, and where they go.
 struct Repack { bool a = false, b = false; int64_t lda = 0, ldb = 0; size_t b_offset = 0, bytes = 0; };
+// What a launch needs of a plan beyond the public structure: the copies, and the tail split of an edge kernel (whose slices may
+// differ in length), its partial sums behind the copies in the workspace.
+struct LaunchExtras { Repack repack; int tail_split = 1, tail_tiles = 0; size_t partial_offset = 0; };
 
 static Repack repack_of(const frisk_gemm_desc* d, bool a, bool b) {
   Repack r;
@@ -427,7 +436,7 @@ static Repack repack_of(const frisk_gemm_desc* d, bool a, bool b) {
   return r;
 }
 
-static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_model, const PlanContext& ctx = {}, Repack* repack = nullptr) {
+static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_model, const PlanContext& ctx = {}, LaunchExtras* extras = nullptr) {
   const bool no_split = ctx.no_workspace;
   int st = validate(d);
   if (st != FRISK_OK) return st;
@@ -541,7 +550,15 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
   plan->workspace_bytes = 0;
   if (k->guard == 2 && packed.bytes) {
     plan->workspace_bytes = packed.bytes;
-    if (repack) *repack = packed;
+    if (extras) extras->repack = packed;
+  }
+  if (k->edge && !k->splitk && !no_split && d->split_k == 0) {
+    const int64_t edge_tiles = (int64_t)plan->grid_x * plan->grid_y;
+    if (const int ts = tail_split_of(k, edge_tiles, (d->K + k->bk - 1) / k->bk, false); ts > 1) {
+      const size_t offset = (plan->workspace_bytes + 255) & ~(size_t)255;
+      plan->workspace_bytes = offset + (size_t)ts * (size_t)(edge_tiles % 256) * (size_t)k->bm * (size_t)k->bn * 4;
+      if (extras) { extras->tail_split = ts; extras->tail_tiles = (int)(edge_tiles % 256); extras->partial_offset = offset; }
+    }
   }
   // Split K over the grid's y dimension when the tile grid alone leaves most CUs idle (skinny problems are
   // bound by streaming the large operand, which needs many work-groups in flight).  Slices hold whole K tiles.
@@ -639,12 +656,12 @@ size_t frisk_hip_workspace_bytes(const frisk_gemm_desc* desc) {
 int frisk_hip_gemm(const frisk_gemm_desc* desc, const void* A, const void* B, void* C, const float* scaleA,
                    const float* scaleB, void* workspace, size_t workspace_bytes, void* stream) {
   frisk_gemm_plan plan;
-  Repack repack;
+  LaunchExtras extras;
   PlanContext ctx;
   ctx.a_off = (uintptr_t)A & 15;
   ctx.b_off = (uintptr_t)B & 15;
   ctx.c_off = ((uintptr_t)C & 15) || (desc && desc->epilogue == FRISK_EPI_ROW_COL_SCALE && ((uintptr_t)scaleB & 15));
-  int st = make_plan(desc, &plan, false, ctx, &repack);
+  int st = make_plan(desc, &plan, false, ctx, &extras);
   if (st != FRISK_OK) return st;
   if (desc->M == 0 || desc->N == 0) return FRISK_OK;
   if (!A || !B || !C) return fail(FRISK_ERR_NULL, "A, B and C must be device pointers");
@@ -656,8 +673,8 @@ int frisk_hip_gemm(const frisk_gemm_desc* desc, const void* A, const void* B, vo
     // an explicit split_k needs its workspace; the planner's own choice degrades to a single pass without one
     if (desc->split_k > 1) return fail(FRISK_ERR_WORKSPACE, "split_k=%d needs %zu bytes of workspace", desc->split_k, plan.workspace_bytes);
     ctx.no_workspace = true;
-    repack = Repack{};
-    st = make_plan(desc, &plan, false, ctx);
+    extras = LaunchExtras{};
+    st = make_plan(desc, &plan, false, ctx, &extras);
     if (st != FRISK_OK) return st;
   }
   if (plan.workspace_bytes > 0 && ((uintptr_t)workspace & 15)) return fail(FRISK_ERR_ALIGNMENT, "workspace must be 16-byte aligned");
@@ -674,11 +691,13 @@ int frisk_hip_gemm(const frisk_gemm_desc* desc, const void* A, const void* B, vo
   const KernelEntry* k = kernels()[plan.kernel_id];
   p.split_k = plan.split_k;
   p.kt_per_slice = (int)((desc->K + k->bk - 1) / k->bk) / plan.split_k;
-  p.partial = plan.split_k > 1 || plan.tail_split > 1 ? workspace : nullptr;
-  p.tail_split = plan.tail_split;
-  p.tail_tiles = plan.tail_tiles;
-  p.tail_from = p.tiles_m * p.tiles_n - plan.tail_tiles;
-  p.tail_kt = plan.tail_split > 1 ? p.kt_per_slice / plan.tail_split : 0;
+  const Repack& repack = extras.repack;
+  const int tail_split = std::max(plan.tail_split, extras.tail_split);
+  p.partial = plan.split_k > 1 || tail_split > 1 ? (char*)workspace + extras.partial_offset : nullptr;
+  p.tail_split = tail_split;
+  p.tail_tiles = extras.tail_split > 1 ? extras.tail_tiles : plan.tail_tiles;
+  p.tail_from = p.tiles_m * p.tiles_n - p.tail_tiles;
+  p.tail_kt = tail_split > 1 ? (p.kt_per_slice + tail_split - 1) / tail_split : 0;
   p.tile_m = k->bm; p.tile_n = k->bn;
   p.k_rotate = 1;
   hipError_t e = hipSuccess;
@@ -700,7 +719,7 @@ int frisk_hip_gemm(const frisk_gemm_desc* desc, const void* A, const void* B, vo
     e = launch_splitk_reduce(p, desc->dtype_acc == FRISK_I32, (hipStream_t)stream);
     if (e != hipSuccess) return fail(FRISK_ERR_DEVICE, "launch of the split-K reduction failed: %s", hipGetErrorString(e));
   }
-  if (plan.tail_split > 1) {
+  if (tail_split > 1) {
     e = launch_tail_reduce(p, desc->dtype_acc == FRISK_I32, (hipStream_t)stream);
     if (e != hipSuccess) return fail(FRISK_ERR_DEVICE, "launch of the tail reduction failed: %s", hipGetErrorString(e));
   }

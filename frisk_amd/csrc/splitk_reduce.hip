@@ -81,6 +81,7 @@ template <bool INT_ACC> __global__ void __launch_bounds__(256) tail_reduce_kerne
   for (int id = blockIdx.x * 256 + threadIdx.x; id < quads; id += gridDim.x * 256) {
     const int r = id / quads_per_row, c = (id % quads_per_row) * 4;
     const int64_t m = (int64_t)tm * BM + r, n = (int64_t)tn * BN + c;
+    if (m >= p.M || n >= p.N) continue;
     int isum[4] = {0, 0, 0, 0};
     float fsum[4] = {0.f, 0.f, 0.f, 0.f};
     r_v4i v[8];  // a tail has 2, 4 or 8 slices: all fetched before the first addition, added in slice order
@@ -100,10 +101,11 @@ template <bool INT_ACC> __global__ void __launch_bounds__(256) tail_reduce_kerne
       for (int e = 0; e < 4; ++e) sb[e] = p.scaleB[0];
     } else if (p.epilogue == FRISK_EPI_ROW_COL_SCALE) {
       sa = p.scaleA[m];
-      for (int e = 0; e < 4; ++e) sb[e] = p.scaleB[n + e];
+      for (int e = 0; e < 4; ++e) if (n + e < p.N) sb[e] = p.scaleB[n + e];
     }
     const bool accum = p.accumulate != 0;
     for (int e = 0; e < 4; ++e) {
+      if (n + e >= p.N) break;
       const int64_t at = m * p.ldc + n + e;
       if (INT_ACC && p.dtype_out == FRISK_I32) {
         int* q = (int*)p.C + at;

@@ -94,3 +94,18 @@ def test_rows_off_16_byte_boundaries(hip, dtype, transA, transB):
             got, name, need = launch(hip, dtype, A, B, M, N, K, transA, transB, False, **kw)
             assert name.endswith("_guard") and (need > 0) == ("tile" in kw), (name, need)
             verify(dtype, got, A, B, transA, transB)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,transA,transB,aligned", [(O.F16, 0, 0, True), (O.BF16, 1, 0, True), (O.I8, 0, 1, False), (O.E4M3, 0, 1, True)])
+def test_tail_split_of_an_edge_kernel(hip, dtype, transA, transB, aligned):
+    """257 to 272 tiles of 256 x 256: the tiles behind the first round are computed in slices of K of unequal length (the last one
+    partial), their sums and the checked stores in the second kernel"""
+    bk = BK[dtype]
+    M, N, K = 16 * 256 + 3, 15 * 256 + 17, (8 if bk == 64 else 16) * bk * 4 - bk - 8
+    A = make_operand(dtype, *stored_shapes(M, N, K, transA, transB)[0], seed=84, tensor=0, scale=0.5)
+    B = make_operand(dtype, *stored_shapes(M, N, K, transA, transB)[1], seed=84, tensor=1, scale=0.5)
+    got, name, need = launch(hip, dtype, A, B, M, N, K, transA, transB, aligned, ldc_extra=1)
+    tiles = 16  # 17 x 16 tiles
+    assert "256x256" in name and need >= 2 * tiles * 256 * 256 * 4, (name, need)
+    verify(dtype, got, A, B, transA, transB)
