@@ -118,6 +118,28 @@ static void wave_partition(int policy, int64_t M, int64_t N, int num_waves, int 
   *wn = (int)std::max<int64_t>(1, n_w);
 }
 
+// The compiled variants of one element type and pair of layouts, in table order, with what the planner would otherwise work out
+// for each of them on every call: which wave policies their wave grid satisfies (computeWarpPartition gives it for their tile and
+// wave count).  A launch of a 128x128x128 product spent 0.75 of its 3.9 us of host time walking the whole table.
+struct Variant { const KernelEntry* k; int id; bool policy[3]; };
+static const std::vector<Variant>& variants(int dtype, bool transA, bool transB) {
+  static const std::vector<std::vector<Variant>> all = [] {
+    std::vector<std::vector<Variant>> v(6 * 4);
+    const auto& ks = kernels();
+    for (size_t i = 0; i < ks.size(); ++i) {
+      Variant x{ks[i], (int)i, {}};
+      for (int policy = 0; policy < 3; ++policy) {
+        int wm = 0, wn = 0;
+        wave_partition(policy, x.k->bm, x.k->bn, x.k->wm * x.k->wn, x.k->atom, x.k->atom, &wm, &wn);
+        x.policy[policy] = wm == x.k->wm && wn == x.k->wn;
+      }
+      v[(size_t)(x.k->dtype * 4 + x.k->transA * 2 + x.k->transB)].push_back(x);
+    }
+    return v;
+  }();
+  return all[(size_t)(dtype * 4 + (transA ? 2 : 0) + (transB ? 1 : 0))];
+}
+
 static int validate(const frisk_gemm_desc* d) {
   if (!d) return fail(FRISK_ERR_NULL, "descriptor is null");
   if (d->abi_version != FRISK_HIP_ABI_VERSION)
@@ -149,7 +171,7 @@ static int validate(const frisk_gemm_desc* d) {
   return FRISK_OK;
 }
 
-static void fill_layout(frisk_lds_layout* L, bool kcontig, int es, int fragb, int mn, int bk, int nw, bool with_model, int atom) {
+static void fill_layout(frisk_lds_layout* L, bool kcontig, int es, int fragb, int mn, int bk, int nw, int atom) {
   TileShape t{kcontig ? mn : bk, (kcontig ? bk : mn) * es, kcontig, es, fragb, mn, bk, atom};
   Swizzle s = default_swizzle(kcontig, es, t.rowb, atom);
   L->rows = t.rows;
@@ -164,8 +186,8 @@ static void fill_layout(frisk_lds_layout* L, bool kcontig, int es, int fragb, in
   L->read_instr = kcontig ? 0 : (es == 4 ? 3 : (es == 2 ? 1 : 2));
   int atoms = mn / atom < 4 ? mn / atom : 4;
   int n_access = atoms * ((bk * es) / frag_kstep_bytes(fragb, atom)) * frag_instr_count(kcontig, es, fragb);
-  // evaluating the bank model costs ~0.1 ms of host time: only when the caller asks for the plan
-  L->read_cycles = (with_model && n_access) ? (float)swizzle_read_cycles(t, s) / (float)n_access : 0.f;
+  // evaluating the bank model costs ~0.1 ms of host time
+  L->read_cycles = n_access ? (float)swizzle_read_cycles(t, s) / (float)n_access : 0.f;
   // the direct-to-LDS transfer writes 64 consecutive 16-byte slots: no conflicts by construction
   L->write_cycles = 16.f;
   (void)nw;
@@ -457,16 +479,15 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
   const Repack packed = repack_of(d, !a_aligned, !b_aligned);
   const double repack_cost = packed.bytes ? 4.0 + (double)packed.bytes / 2.2e6 : 0.0;
   const auto& ks = kernels();
+  const auto& list = variants(d->dtype_ab, d->transA != 0, d->transB != 0);
   int best = -1;
   double best_cost = 0.0;
   bool policy_excluded = false;
-  bool any_layout = false, tile_requested = d->tile_m || d->tile_n || d->tile_k || d->waves_m || d->waves_n || d->stages || d->atom;
+  const bool any_layout = !list.empty(), tile_requested = d->tile_m || d->tile_n || d->tile_k || d->waves_m || d->waves_n || d->stages || d->atom;
   const bool small = small_grid(d);
   auto search = [&](bool want_split) {
-    for (size_t i = 0; i < ks.size(); ++i) {
-      const KernelEntry* k = ks[i];
-      if (k->dtype != d->dtype_ab || k->transA != (d->transA != 0) || k->transB != (d->transB != 0)) continue;
-      any_layout = true;
+    for (const Variant& v : list) {
+      const KernelEntry* k = v.k;
       if (d->tile_m && d->tile_m != k->bm) continue;
       if (d->tile_n && d->tile_n != k->bn) continue;
       if (d->tile_k && d->tile_k != k->bk) continue;
@@ -476,11 +497,7 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
       if (d->atom && d->atom != k->atom) continue;
       // frisk.gemm's wave policy (FriskOps.td:248-289) decides the wave grid unless the descriptor names one: only variants
       // whose compiled grid is what computeWarpPartition gives for their tile and wave count under that policy qualify
-      if (!d->waves_m && !d->waves_n) {
-        int pm = 0, pn = 0;
-        wave_partition(d->policy, k->bm, k->bn, k->wm * k->wn, k->atom, k->atom, &pm, &pn);
-        if (pm != k->wm || pn != k->wn) { policy_excluded = true; continue; }
-      }
+      if (!d->waves_m && !d->waves_n && !v.policy[d->policy]) { policy_excluded = true; continue; }
       if (want_split && !k->splitk) continue;
       // a kernel whose loop needs a minimum of K tiles: per slice when the descriptor asks for a split
       if (k->min_k_tiles > 1 && (d->K + k->bk - 1) / k->bk / (want_split && d->split_k > 1 ? d->split_k : 1) < k->min_k_tiles) continue;
@@ -510,7 +527,7 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
       }
       if (k->guard == 2) cost += repack_cost;
       // ties: the first listed variant is the tuned default
-      if (best < 0 || (ks[best]->guard && !k->guard) || cost < best_cost) { best = (int)i; best_cost = cost; }
+      if (best < 0 || (ks[best]->guard && !k->guard) || cost < best_cost) { best = v.id; best_cost = cost; }
     }
   };
   // an explicit split_k looks among the variants with the split-K store path first; if none of them fits, the choice among
@@ -545,8 +562,10 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
   plan->grid_y = (int)((d->M + k->bm - 1) / k->bm);
   plan->guarded = k->guard != 0;
   plan->xcd_remap = ((int64_t)plan->grid_x * plan->grid_y) % 8 == 0;
-  fill_layout(&plan->lds_a, !d->transA, es, frag_bytes(d->dtype_ab), k->bm, k->bk, k->wm * k->wn * k->wk, with_model, k->atom);
-  fill_layout(&plan->lds_b, d->transB != 0, es, frag_bytes(d->dtype_ab), k->bn, k->bk, k->wm * k->wn * k->wk, with_model, k->atom);
+  if (with_model) {  // for the caller of frisk_hip_plan: no launch looks at the LDS layouts
+    fill_layout(&plan->lds_a, !d->transA, es, frag_bytes(d->dtype_ab), k->bm, k->bk, k->wm * k->wn * k->wk, k->atom);
+    fill_layout(&plan->lds_b, d->transB != 0, es, frag_bytes(d->dtype_ab), k->bn, k->bk, k->wm * k->wn * k->wk, k->atom);
+  }
   plan->workspace_bytes = 0;
   if (k->guard == 2 && packed.bytes) {
     plan->workspace_bytes = packed.bytes;
