@@ -642,8 +642,6 @@ static int check_view(const char* what, int dtype, const void* p, int64_t rows, 
   return FRISK_OK;
 }
 
-static bool rows_on_16_bytes(int dtype, const void* p, int64_t ld) { return ((uintptr_t)p & 15) == 0 && (ld * elem_size(dtype)) % 16 == 0; }
-
 }  // namespace frisk
 
 using namespace frisk;
@@ -824,7 +822,7 @@ int frisk_hip_fill(int dtype, void* dst, int64_t rows, int64_t cols, int64_t ld,
   if (rows == 0 || cols == 0) return FRISK_OK;
   if (!device_ok()) return fail(FRISK_ERR_DEVICE, "no gfx950 device is current");
   if (ld == cols) { cols *= rows; rows = 1; ld = cols; }  // a dense view is one long row
-  hipError_t e = launch_fill(dtype, dst, rows, cols, ld, value, rows_on_16_bytes(dtype, dst, ld), (hipStream_t)stream);
+  hipError_t e = launch_fill(dtype, dst, rows, cols, ld, value, (hipStream_t)stream);
   if (e != hipSuccess) return fail(FRISK_ERR_DEVICE, "fill launch failed: %s", hipGetErrorString(e));
   return FRISK_OK;
 }
@@ -836,8 +834,7 @@ int frisk_hip_copy(int src_dtype, const void* src, int64_t src_ld, int dst_dtype
   if (rows == 0 || cols == 0) return FRISK_OK;
   if (!device_ok()) return fail(FRISK_ERR_DEVICE, "no gfx950 device is current");
   if (src_ld == cols && dst_ld == cols) { cols *= rows; rows = 1; src_ld = dst_ld = cols; }
-  const int vec = rows_on_16_bytes(src_dtype, src, src_ld) && rows_on_16_bytes(dst_dtype, dst, dst_ld);
-  hipError_t e = launch_copy(src_dtype, src, src_ld, dst_dtype, dst, dst_ld, rows, cols, vec, (hipStream_t)stream);
+  hipError_t e = launch_copy(src_dtype, src, src_ld, dst_dtype, dst, dst_ld, rows, cols, (hipStream_t)stream);
   if (e != hipSuccess) return fail(FRISK_ERR_DEVICE, "copy launch failed: %s", hipGetErrorString(e));
   return FRISK_OK;
 }
@@ -851,12 +848,9 @@ int frisk_hip_copy_tiles(int src_dtype, const void* src, int64_t src_ld, int dst
   if (n0 > INT32_MAX || n1 > INT32_MAX || n0 * n1 > INT32_MAX) return fail(FRISK_ERR_SHAPE, "tiled copy: more than 2^31-1 tiles");
   if (tile_rows == 0 || tile_cols == 0 || n0 == 0 || n1 == 0) return FRISK_OK;
   if (!device_ok()) return fail(FRISK_ERR_DEVICE, "no gfx950 device is current");
-  const int ss = elem_size(src_dtype), ds = elem_size(dst_dtype);
-  const bool steps16 = (src_step0 * ss) % 16 == 0 && (src_step1 * ss) % 16 == 0 && (dst_step0 * ds) % 16 == 0 && (dst_step1 * ds) % 16 == 0;
-  const int vec = steps16 && rows_on_16_bytes(src_dtype, src, src_ld) && rows_on_16_bytes(dst_dtype, dst, dst_ld);
   TilePlacement t;
   t.n0 = n0; t.n1 = n1; t.src_step0 = src_step0; t.src_step1 = src_step1; t.dst_step0 = dst_step0; t.dst_step1 = dst_step1;
-  hipError_t e = launch_copy_tiles(src_dtype, src, src_ld, dst_dtype, dst, dst_ld, tile_rows, tile_cols, t, vec, (hipStream_t)stream);
+  hipError_t e = launch_copy_tiles(src_dtype, src, src_ld, dst_dtype, dst, dst_ld, tile_rows, tile_cols, t, (hipStream_t)stream);
   if (e != hipSuccess) return fail(FRISK_ERR_DEVICE, "tiled copy launch failed: %s", hipGetErrorString(e));
   return FRISK_OK;
 }
@@ -923,8 +917,7 @@ int frisk_hip_reduce(int dtype, const void* src, int64_t rows, int64_t cols, int
   int slices = (rows > 0 && cols > 0) ? reduce_slices(dtype, rows, cols, dim) : 1;
   // without a (large enough, 4-byte aligned) workspace the reduction runs unsplit: same result, fewer work-groups
   if (slices > 1 && (!workspace || workspace_bytes < (size_t)slices * (size_t)kept * 4 || ((uintptr_t)workspace & 3))) slices = 1;
-  hipError_t e = launch_reduce(dtype, src, rows, cols, ld, dim, kind, clear ? 1 : 0, dst, (float*)workspace, slices, rows_on_16_bytes(dtype, src, ld),
-                               (hipStream_t)stream);
+  hipError_t e = launch_reduce(dtype, src, rows, cols, ld, dim, kind, clear ? 1 : 0, dst, (float*)workspace, slices, (hipStream_t)stream);
   if (e != hipSuccess) return fail(FRISK_ERR_DEVICE, "reduce launch failed: %s", hipGetErrorString(e));
   return FRISK_OK;
 }
@@ -943,11 +936,10 @@ int frisk_hip_softmax(int dtype, const void* src, int64_t src_ld, void* dst, int
   if ((uintptr_t)lse & 3) return fail(FRISK_ERR_ALIGNMENT, "lse must be 4-byte aligned");
   if (rows == 0 || cols == 0) return FRISK_OK;
   if (!device_ok()) return fail(FRISK_ERR_DEVICE, "no gfx950 device is current");
-  const int rows_aligned = rows_on_16_bytes(dtype, src, src_ld) && rows_on_16_bytes(dtype, dst, dst_ld);
   int slices = softmax_slices(dtype, rows, cols);
   // without a (large enough, 4-byte aligned) workspace the rows are not split: same result, fewer work-groups
   if (slices > 1 && (!workspace || workspace_bytes < (size_t)rows * (size_t)slices * 8 || ((uintptr_t)workspace & 3))) slices = 1;
-  hipError_t e = launch_softmax_rows(dtype, src, src_ld, dst, dst_ld, rows, cols, scale_log2, lse, rows_aligned, (float*)workspace, slices, (hipStream_t)stream);
+  hipError_t e = launch_softmax_rows(dtype, src, src_ld, dst, dst_ld, rows, cols, scale_log2, lse, (float*)workspace, slices, (hipStream_t)stream);
   if (e != hipSuccess) return fail(FRISK_ERR_DEVICE, "softmax launch failed: %s", hipGetErrorString(e));
   return FRISK_OK;
 }

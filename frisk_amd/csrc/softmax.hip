@@ -5,8 +5,8 @@
 // wave and combined by shuffles; longer rows get a work-group of 256 lanes each.  Rows of up to 64 elements per lane are
 // read once and held in registers (maximum, exponentials, sum, scaling: one read and one write of HBM per element);
 // longer rows take the sketch's two sweeps with a running maximum and sum per lane, the second sweep re-reading x.
-// A lane moves 16 bytes at a time where rows start on 16-byte boundaries; groups that are not whole and, in the
-// work-group kernels, any view whose row length is not a whole number of groups are walked element by element.
+// A lane moves 16 bytes at a time, wherever the rows start; only a row's last group, when it is not whole, is walked element by
+// element (4095 x 8191 f16: 55.5 us while rows off 16-byte boundaries went element by element, 31.5 now).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include "tile_ops.h"
@@ -15,11 +15,44 @@ namespace frisk {
 namespace {
 
 typedef unsigned v4u __attribute__((ext_vector_type(4)));
+// 16 bytes that start on any element: loads and stores of this type are one instruction at any address
+typedef unsigned v4u_any __attribute__((ext_vector_type(4), aligned(2)));
 
 template <int DT> struct SElem;
 template <> struct SElem<FRISK_F32> { typedef float T; static __device__ float load(const T& x) { return x; } static __device__ T store(float x) { return x; } };
 template <> struct SElem<FRISK_F16> { typedef _Float16 T; static __device__ float load(const T& x) { return (float)x; } static __device__ T store(float x) { return (_Float16)x; } };
 template <> struct SElem<FRISK_BF16> { typedef __bf16 T; static __device__ float load(const T& x) { return (float)x; } static __device__ T store(float x) { return (__bf16)x; } };
+
+// group g (G elements, 16 bytes) of a row of cols elements as floats times c; -inf beyond the row
+template <int DT, bool STREAMED> __device__ __forceinline__ void load_group(const typename SElem<DT>::T* x, int64_t g, int64_t cols, float c, float (&v)[16 / sizeof(typename SElem<DT>::T)]) {
+  typedef typename SElem<DT>::T T;
+  constexpr int G = 16 / (int)sizeof(T);
+  const int64_t left = cols - g * G;
+  T in[G];
+  if (left >= G) {
+    if constexpr (STREAMED) *(v4u*)in = __builtin_nontemporal_load((const v4u_any*)(x + g * G));
+    else *(v4u*)in = *(const v4u_any*)(x + g * G);
+#pragma unroll
+    for (int e = 0; e < G; ++e) v[e] = SElem<DT>::load(in[e]) * c;
+  } else {
+#pragma unroll
+    for (int e = 0; e < G; ++e) v[e] = e < left ? SElem<DT>::load(x[g * G + e]) * c : -INFINITY;
+  }
+}
+template <int DT, bool WHOLE = false> __device__ __forceinline__ void store_group(typename SElem<DT>::T* y, int64_t g, int64_t cols, const float (&v)[16 / sizeof(typename SElem<DT>::T)]) {
+  typedef typename SElem<DT>::T T;
+  constexpr int G = 16 / (int)sizeof(T);
+  const int64_t left = cols - g * G;
+  T out[G];
+#pragma unroll
+  for (int e = 0; e < G; ++e) out[e] = SElem<DT>::store(v[e]);
+  if (WHOLE || left >= G) __builtin_nontemporal_store(*(const v4u*)out, (v4u_any*)(y + g * G));
+  else {
+#pragma unroll
+    for (int e = 0; e < G; ++e)
+      if (e < left) y[g * G + e] = out[e];
+  }
+}
 
 // (maximum, sum of 2^(v - maximum)) pairs combine associatively
 struct MaxSum {
@@ -57,31 +90,39 @@ __device__ __forceinline__ MaxSum block_merge(MaxSum v, float* lds) {
   return r;
 }
 
-// Longer rows, a work-group each.  NPT > 0: the row fits in NPT 16-byte groups per lane and is kept in registers.  NPT == 0: two sweeps, 16-byte
-// groups when `vec`, single elements otherwise.
-template <int DT, int NPT>
+// Longer rows, a work-group each.  NPT > 0: the row fits in NPT 16-byte groups per lane and is kept in registers.  NPT == 0: two sweeps.
+// WHOLE: the row is a whole number of groups (the code for a last one that is not costs 8 % where no row needs it).
+template <int DT, int NPT, bool WHOLE>
 __global__ void __launch_bounds__(256) softmax_rows_kernel(const typename SElem<DT>::T* src, int64_t sld, typename SElem<DT>::T* dst, int64_t dld, int64_t rows,
-                                                           int64_t cols, float c, float* lse, int vec) {
+                                                           int64_t cols, float c, float* lse) {
   typedef typename SElem<DT>::T T;
   constexpr int G = 16 / (int)sizeof(T);
+  const int64_t groups = (cols + G - 1) / G;
   __shared__ float lds[8];
   for (int64_t r = blockIdx.x; r < rows; r += gridDim.x) {
     const T* x = src + r * sld;
     T* y = dst + r * dld;
     if constexpr (NPT > 0) {
-      const int64_t groups = cols / G;
       float v[NPT][G];
+      // every whole group is requested before the first is used; the row's last group, if it is not whole, comes behind them
+      T in[NPT][G];
+#pragma unroll
+      for (int q = 0; q < NPT; ++q) {
+        const int64_t g = (int64_t)q * 256 + threadIdx.x;
+        if (g * G + G <= cols) *(v4u*)in[q] = __builtin_nontemporal_load((const v4u_any*)(x + g * G));
+      }
       float mx = -INFINITY;
 #pragma unroll
       for (int q = 0; q < NPT; ++q) {
         const int64_t g = (int64_t)q * 256 + threadIdx.x;
-        T in[G];
-        if (g < groups) *(v4u*)in = __builtin_nontemporal_load((const v4u*)(x + g * G));
 #pragma unroll
-        for (int e = 0; e < G; ++e) {
-          v[q][e] = g < groups ? SElem<DT>::load(in[e]) * c : -INFINITY;
-          mx = fmaxf(mx, v[q][e]);
-        }
+        for (int e = 0; e < G; ++e) v[q][e] = -INFINITY;
+        if (g * G + G <= cols) {
+#pragma unroll
+          for (int e = 0; e < G; ++e) v[q][e] = SElem<DT>::load(in[q][e]) * c;
+        } else if (!WHOLE && g < groups) load_group<DT, true>(x, g, cols, c, v[q]);
+#pragma unroll
+        for (int e = 0; e < G; ++e) mx = fmaxf(mx, v[q][e]);
       }
       const MaxSum top = block_merge(MaxSum{mx, 1.f}, lds);  // only the maximum is used here
       float sum = 0.f;
@@ -97,38 +138,27 @@ __global__ void __launch_bounds__(256) softmax_rows_kernel(const typename SElem<
 #pragma unroll
       for (int q = 0; q < NPT; ++q) {
         const int64_t g = (int64_t)q * 256 + threadIdx.x;
-        if (g < groups) {
-          T out[G];
 #pragma unroll
-          for (int e = 0; e < G; ++e) out[e] = SElem<DT>::store(v[q][e] * inv);
-          __builtin_nontemporal_store(*(const v4u*)out, (v4u*)(y + g * G));
-        }
+        for (int e = 0; e < G; ++e) v[q][e] *= inv;
+        if (g < groups) store_group<DT, WHOLE>(y, g, cols, v[q]);
       }
       if (lse && threadIdx.x == 0) lse[r] = top.m + __builtin_amdgcn_logf(all.l);
     } else {
       MaxSum acc = {-INFINITY, 0.f};
-      if (vec) {
-        for (int64_t g = threadIdx.x; g < cols / G; g += 256) {
-          T in[G];
-          *(v4u*)in = *(const v4u*)(x + g * G);
+      for (int64_t g = threadIdx.x; g < groups; g += 256) {
+        float v[G];
+        load_group<DT, false>(x, g, cols, c, v);
 #pragma unroll
-          for (int e = 0; e < G; ++e) acc.add(SElem<DT>::load(in[e]) * c);
-        }
-      } else {
-        for (int64_t j = threadIdx.x; j < cols; j += 256) acc.add(SElem<DT>::load(x[j]) * c);
+        for (int e = 0; e < G; ++e) acc.add(v[e]);
       }
       const MaxSum all = block_merge(acc, lds);
       const float ref = all.m + __builtin_amdgcn_logf(all.l);  // log2 of the denominator
-      if (vec) {
-        for (int64_t g = threadIdx.x; g < cols / G; g += 256) {
-          T in[G], out[G];
-          *(v4u*)in = *(const v4u*)(x + g * G);
+      for (int64_t g = threadIdx.x; g < groups; g += 256) {
+        float v[G];
+        load_group<DT, false>(x, g, cols, c, v);
 #pragma unroll
-          for (int e = 0; e < G; ++e) out[e] = SElem<DT>::store(__builtin_amdgcn_exp2f(SElem<DT>::load(in[e]) * c - ref));
-          __builtin_nontemporal_store(*(const v4u*)out, (v4u*)(y + g * G));
-        }
-      } else {
-        for (int64_t j = threadIdx.x; j < cols; j += 256) y[j] = SElem<DT>::store(__builtin_amdgcn_exp2f(SElem<DT>::load(x[j]) * c - ref));
+        for (int e = 0; e < G; ++e) v[e] = __builtin_amdgcn_exp2f(v[e] - ref);
+        store_group<DT>(y, g, cols, v);
       }
       if (lse && threadIdx.x == 0) lse[r] = ref;
     }
@@ -136,11 +166,10 @@ __global__ void __launch_bounds__(256) softmax_rows_kernel(const typename SElem<
 }
 
 // Rows of at most 256 groups of 16 bytes: 2^lanes_log2 <= 64 lanes of one wave share a row, each holding up to NPT groups in
-// registers, and combine maximum and sum by shuffles (no LDS, no barrier); a work-group holds 256 >> lanes_log2 rows.  Any
-// alignment: a group that is not a whole, aligned 16 bytes is walked element by element.
+// registers, and combine maximum and sum by shuffles (no LDS, no barrier); a work-group holds 256 >> lanes_log2 rows.
 template <int DT, int NPT>
 __global__ void __launch_bounds__(256) softmax_short_rows_kernel(const typename SElem<DT>::T* src, int64_t sld, typename SElem<DT>::T* dst, int64_t dld, int64_t rows,
-                                                                 int64_t cols, float c, float* lse, int vec, int lanes_log2) {
+                                                                 int64_t cols, float c, float* lse, int lanes_log2) {
   typedef typename SElem<DT>::T T;
   constexpr int G = 16 / (int)sizeof(T);
   const int lanes = 1 << lanes_log2, lane = threadIdx.x & (lanes - 1), rows_per_group = 256 >> lanes_log2;
@@ -156,8 +185,8 @@ __global__ void __launch_bounds__(256) softmax_short_rows_kernel(const typename 
 #pragma unroll
     for (int q = 0; q < NPT; ++q) {
       const int64_t c0 = (int64_t)(q * lanes + lane) * G;
-      whole[q] = live && vec && c0 + G <= cols;
-      if (whole[q]) *(v4u*)in[q] = __builtin_nontemporal_load((const v4u*)(x + c0));
+      whole[q] = live && c0 + G <= cols;
+      if (whole[q]) *(v4u*)in[q] = __builtin_nontemporal_load((const v4u_any*)(x + c0));
     }
     float mx = -INFINITY;
 #pragma unroll
@@ -188,7 +217,7 @@ __global__ void __launch_bounds__(256) softmax_short_rows_kernel(const typename 
         T out[G];
 #pragma unroll
         for (int e = 0; e < G; ++e) out[e] = SElem<DT>::store(v[q][e] * inv);
-        __builtin_nontemporal_store(*(const v4u*)out, (v4u*)(y + c0));
+        __builtin_nontemporal_store(*(const v4u*)out, (v4u_any*)(y + c0));
       } else if (live) {
 #pragma unroll
         for (int e = 0; e < G; ++e)
@@ -204,21 +233,17 @@ __global__ void __launch_bounds__(256) softmax_short_rows_kernel(const typename 
 // second launch: every work-group merges the row's pairs and writes its share of exp2(x * c - log-sum).  Two reads and
 // one write per element, as in the two sweeps above, but on rows x slices work-groups instead of rows.
 template <int DT>
-__global__ void __launch_bounds__(256) softmax_split_stats_kernel(const typename SElem<DT>::T* src, int64_t sld, int64_t cols, float c, float* partial, int vec) {
+__global__ void __launch_bounds__(256) softmax_split_stats_kernel(const typename SElem<DT>::T* src, int64_t sld, int64_t cols, float c, float* partial) {
   typedef typename SElem<DT>::T T;
   constexpr int G = 16 / (int)sizeof(T);
   __shared__ float lds[8];
   const T* x = src + (int64_t)blockIdx.x * sld;
   MaxSum acc = {-INFINITY, 0.f};
-  if (vec) {
-    for (int64_t g = (int64_t)blockIdx.y * 256 + threadIdx.x; g < cols / G; g += (int64_t)gridDim.y * 256) {
-      T in[G];
-      *(v4u*)in = *(const v4u*)(x + g * G);
+  for (int64_t g = (int64_t)blockIdx.y * 256 + threadIdx.x; g * G < cols; g += (int64_t)gridDim.y * 256) {
+    float v[G];
+    load_group<DT, false>(x, g, cols, c, v);
 #pragma unroll
-      for (int e = 0; e < G; ++e) acc.add(SElem<DT>::load(in[e]) * c);
-    }
-  } else {
-    for (int64_t j = (int64_t)blockIdx.y * 256 + threadIdx.x; j < cols; j += (int64_t)gridDim.y * 256) acc.add(SElem<DT>::load(x[j]) * c);
+    for (int e = 0; e < G; ++e) acc.add(v[e]);
   }
   const MaxSum all = block_merge(acc, lds);
   if (threadIdx.x == 0) {
@@ -230,7 +255,7 @@ __global__ void __launch_bounds__(256) softmax_split_stats_kernel(const typename
 
 template <int DT>
 __global__ void __launch_bounds__(256) softmax_split_write_kernel(const typename SElem<DT>::T* src, int64_t sld, typename SElem<DT>::T* dst, int64_t dld, int64_t cols,
-                                                                  float c, float* lse, const float* partial, int vec) {
+                                                                  float c, float* lse, const float* partial) {
   typedef typename SElem<DT>::T T;
   constexpr int G = 16 / (int)sizeof(T);
   __shared__ float lds[8];
@@ -243,26 +268,20 @@ __global__ void __launch_bounds__(256) softmax_split_write_kernel(const typename
   }
   const MaxSum all = block_merge(acc, lds);
   const float ref = all.m + __builtin_amdgcn_logf(all.l);  // log2 of the denominator
-  if (vec) {
-    for (int64_t g = (int64_t)blockIdx.y * 256 + threadIdx.x; g < cols / G; g += (int64_t)gridDim.y * 256) {
-      T in[G], out[G];
-      *(v4u*)in = __builtin_nontemporal_load((const v4u*)(x + g * G));
+  for (int64_t g = (int64_t)blockIdx.y * 256 + threadIdx.x; g * G < cols; g += (int64_t)gridDim.y * 256) {
+    float v[G];
+    load_group<DT, true>(x, g, cols, c, v);
 #pragma unroll
-      for (int e = 0; e < G; ++e) out[e] = SElem<DT>::store(__builtin_amdgcn_exp2f(SElem<DT>::load(in[e]) * c - ref));
-      __builtin_nontemporal_store(*(const v4u*)out, (v4u*)(y + g * G));
-    }
-  } else {
-    for (int64_t j = (int64_t)blockIdx.y * 256 + threadIdx.x; j < cols; j += (int64_t)gridDim.y * 256)
-      y[j] = SElem<DT>::store(__builtin_amdgcn_exp2f(SElem<DT>::load(x[j]) * c - ref));
+    for (int e = 0; e < G; ++e) v[e] = __builtin_amdgcn_exp2f(v[e] - ref);
+    store_group<DT>(y, g, cols, v);
   }
   if (lse && blockIdx.y == 0 && threadIdx.x == 0) lse[blockIdx.x] = ref;
 }
 
-template <int DT> hipError_t launch_typed(const void* src, int64_t sld, void* dst, int64_t dld, int64_t rows, int64_t cols, float c, float* lse, int rows_aligned,
-                                          float* partial, int slices, hipStream_t s) {
+template <int DT> hipError_t launch_typed(const void* src, int64_t sld, void* dst, int64_t dld, int64_t rows, int64_t cols, float c, float* lse, float* partial,
+                                          int slices, hipStream_t s) {
   typedef typename SElem<DT>::T T;
   constexpr int G = 16 / (int)sizeof(T);
-  const int vec = rows_aligned && cols % G == 0;
   const unsigned grid = (unsigned)(rows < 256 * 64 ? rows : 256 * 64);
   const int64_t per_pass = 256 * (int64_t)G;
   const T* x = (const T*)src;
@@ -270,24 +289,28 @@ template <int DT> hipError_t launch_typed(const void* src, int64_t sld, void* ds
   const int64_t groups = (cols + G - 1) / G;
   if (slices > 1) {
     const dim3 sgrid((unsigned)rows, (unsigned)slices);
-    hipLaunchKernelGGL((softmax_split_stats_kernel<DT>), sgrid, dim3(256), 0, s, x, sld, cols, c, partial, vec);
-    hipLaunchKernelGGL((softmax_split_write_kernel<DT>), sgrid, dim3(256), 0, s, x, sld, y, dld, cols, c, lse, (const float*)partial, vec);
+    hipLaunchKernelGGL((softmax_split_stats_kernel<DT>), sgrid, dim3(256), 0, s, x, sld, cols, c, partial);
+    hipLaunchKernelGGL((softmax_split_write_kernel<DT>), sgrid, dim3(256), 0, s, x, sld, y, dld, cols, c, lse, (const float*)partial);
     return hipGetLastError();
   }
-  if (groups <= 256) {  // here a row that ends in a partial group still moves its whole groups 16 bytes at a time
+  if (groups <= 256) {
     int lanes_log2 = 0;
     while (lanes_log2 < 6 && (int64_t(1) << lanes_log2) < groups) ++lanes_log2;
     const int64_t rows_per_group = 256 >> lanes_log2, blocks = (rows + rows_per_group - 1) / rows_per_group;
     const dim3 sgrid((unsigned)(blocks < (1 << 22) ? blocks : (1 << 22)));
-    if (groups <= 64) hipLaunchKernelGGL((softmax_short_rows_kernel<DT, 1>), sgrid, dim3(256), 0, s, x, sld, y, dld, rows, cols, c, lse, rows_aligned, lanes_log2);
-    else if (groups <= 128) hipLaunchKernelGGL((softmax_short_rows_kernel<DT, 2>), sgrid, dim3(256), 0, s, x, sld, y, dld, rows, cols, c, lse, rows_aligned, lanes_log2);
-    else hipLaunchKernelGGL((softmax_short_rows_kernel<DT, 4>), sgrid, dim3(256), 0, s, x, sld, y, dld, rows, cols, c, lse, rows_aligned, lanes_log2);
+    if (groups <= 64) hipLaunchKernelGGL((softmax_short_rows_kernel<DT, 1>), sgrid, dim3(256), 0, s, x, sld, y, dld, rows, cols, c, lse, lanes_log2);
+    else if (groups <= 128) hipLaunchKernelGGL((softmax_short_rows_kernel<DT, 2>), sgrid, dim3(256), 0, s, x, sld, y, dld, rows, cols, c, lse, lanes_log2);
+    else hipLaunchKernelGGL((softmax_short_rows_kernel<DT, 4>), sgrid, dim3(256), 0, s, x, sld, y, dld, rows, cols, c, lse, lanes_log2);
     return hipGetLastError();
   }
-  if (vec && cols <= 2 * per_pass) hipLaunchKernelGGL((softmax_rows_kernel<DT, 2>), dim3(grid), dim3(256), 0, s, x, sld, y, dld, rows, cols, c, lse, vec);
-  else if (vec && cols <= 4 * per_pass) hipLaunchKernelGGL((softmax_rows_kernel<DT, 4>), dim3(grid), dim3(256), 0, s, x, sld, y, dld, rows, cols, c, lse, vec);
-  else if (vec && cols <= 8 * per_pass) hipLaunchKernelGGL((softmax_rows_kernel<DT, 8>), dim3(grid), dim3(256), 0, s, x, sld, y, dld, rows, cols, c, lse, vec);
-  else hipLaunchKernelGGL((softmax_rows_kernel<DT, 0>), dim3(grid), dim3(256), 0, s, x, sld, y, dld, rows, cols, c, lse, vec);
+#define FRISK_SOFTMAX_ROWS(NPT)                                                                                                                         \
+  if (cols % G == 0) hipLaunchKernelGGL((softmax_rows_kernel<DT, NPT, true>), dim3(grid), dim3(256), 0, s, x, sld, y, dld, rows, cols, c, lse);           \
+  else hipLaunchKernelGGL((softmax_rows_kernel<DT, NPT, false>), dim3(grid), dim3(256), 0, s, x, sld, y, dld, rows, cols, c, lse);
+  if (cols <= 2 * per_pass) { FRISK_SOFTMAX_ROWS(2) }
+  else if (cols <= 4 * per_pass) { FRISK_SOFTMAX_ROWS(4) }
+  else if (cols <= 8 * per_pass) { FRISK_SOFTMAX_ROWS(8) }
+  else hipLaunchKernelGGL((softmax_rows_kernel<DT, 0, false>), dim3(grid), dim3(256), 0, s, x, sld, y, dld, rows, cols, c, lse);
+#undef FRISK_SOFTMAX_ROWS
   return hipGetLastError();
 }
 
@@ -301,13 +324,12 @@ int softmax_slices(int dtype, int64_t rows, int64_t cols) {
   return slices;
 }
 
-// rows_aligned: pointers and leading dimensions put every row of both views on a 16-byte boundary
 hipError_t launch_softmax_rows(int dtype, const void* src, int64_t sld, void* dst, int64_t dld, int64_t rows, int64_t cols, float scale_log2, float* lse,
-                               int rows_aligned, float* partial, int slices, hipStream_t s) {
+                               float* partial, int slices, hipStream_t s) {
   switch (dtype) {
-    case FRISK_F32: return launch_typed<FRISK_F32>(src, sld, dst, dld, rows, cols, scale_log2, lse, rows_aligned, partial, slices, s);
-    case FRISK_F16: return launch_typed<FRISK_F16>(src, sld, dst, dld, rows, cols, scale_log2, lse, rows_aligned, partial, slices, s);
-    default: return launch_typed<FRISK_BF16>(src, sld, dst, dld, rows, cols, scale_log2, lse, rows_aligned, partial, slices, s);
+    case FRISK_F32: return launch_typed<FRISK_F32>(src, sld, dst, dld, rows, cols, scale_log2, lse, partial, slices, s);
+    case FRISK_F16: return launch_typed<FRISK_F16>(src, sld, dst, dld, rows, cols, scale_log2, lse, partial, slices, s);
+    default: return launch_typed<FRISK_BF16>(src, sld, dst, dld, rows, cols, scale_log2, lse, partial, slices, s);
   }
 }
 

@@ -1,7 +1,6 @@
 // frisk.fill, frisk.copy and frisk.reduce on rank-2 views of device memory.  All three are bound by
-// HBM traffic: a lane moves 16 bytes at a time wherever the view allows it (row start and row length
-// multiples of 16 bytes), falls back to single elements otherwise, and a launch covers the view with
-// many more work-groups than the 256 CUs.
+// HBM traffic: a lane moves 16 bytes at a time, wherever the rows start (only a row's last group, when it is not whole, goes element
+// by element), and a launch covers the view with many more work-groups than the 256 CUs.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include "tile_ops.h"
@@ -13,9 +12,11 @@ typedef unsigned v4u __attribute__((ext_vector_type(4)));
 
 // streaming reads: every byte is read once, so the caches are told not to keep it; on stores the hint pays in copy
 // between equally wide types (6.3 against 5.9 TB/s) and changes nothing in fill, so only copy uses it
-__device__ __forceinline__ v4u load16(const void* p) { return __builtin_nontemporal_load((const v4u*)p); }
-__device__ __forceinline__ void store16(void* p, v4u v) { *(v4u*)p = v; }
-__device__ __forceinline__ void store16_stream(void* p, v4u v) { __builtin_nontemporal_store(v, (v4u*)p); }
+// (16 bytes that start on any element: loads and stores of this type are one instruction at any address)
+typedef unsigned v4u_any __attribute__((ext_vector_type(4), aligned(2)));
+__device__ __forceinline__ v4u load16(const void* p) { return __builtin_nontemporal_load((const v4u_any*)p); }
+__device__ __forceinline__ void store16(void* p, v4u v) { *(v4u_any*)p = v; }
+__device__ __forceinline__ void store16_stream(void* p, v4u v) { __builtin_nontemporal_store(v, (v4u_any*)p); }
 
 template <int DT> struct Elem;
 template <> struct Elem<FRISK_F32> { typedef float T; static __device__ float load(const T& x) { return x; } static __device__ T store(float x) { return x; } };
@@ -24,13 +25,12 @@ template <> struct Elem<FRISK_BF16> { typedef __bf16 T; static __device__ float 
 
 // A rows x cols view is cut into groups of G columns (16 bytes of the narrower type) and walked without any division:
 // 2^lanes_log2 lanes of a work-group lie along a row, the remaining 256 >> lanes_log2 across rows, work-groups step
-// along the row in x and down the rows in y.  Every lane handles several groups per step, all loads issued before the
-// first store: two neighbours along the row (4 KiB apart) where the row is long enough to give both of them work
-// (ALONG; more than two measured slower), else the same columns of eight rows.
-constexpr int kPerLaneAlong = 2, kPerLaneAcross = 8;
+// along the row in x and down the rows in y.  Every lane handles several groups per step: ALONG (1, 2 or 4) neighbours along the row
+// (4 KiB apart) where the row is long enough to give them work, or (ALONG 0) the same columns of eight rows.
+constexpr int kPerLaneAcross = 8;
 
-template <bool ALONG> struct Walk {
-  static constexpr int PER = ALONG ? kPerLaneAlong : kPerLaneAcross;
+template <int ALONG> struct Walk {
+  static constexpr int PER = ALONG ? ALONG : kPerLaneAcross;
   int64_t slabs, row_blocks, rows, groups_per_row;
   int lanes, lane_group, lane_row, row_step;
   __device__ Walk(int64_t rows_, int64_t groups_per_row_, int lanes_log2) : rows(rows_), groups_per_row(groups_per_row_) {
@@ -38,9 +38,13 @@ template <bool ALONG> struct Walk {
     row_step = 256 >> lanes_log2;
     lane_group = threadIdx.x & (lanes - 1);
     lane_row = threadIdx.x >> lanes_log2;
-    const int64_t per_x = (int64_t)lanes * (ALONG ? PER : 1), per_y = (int64_t)row_step * (ALONG ? 1 : PER);
-    slabs = (groups_per_row + per_x - 1) / per_x;
-    row_blocks = (rows + per_y - 1) / per_y;
+    // groups of a slab and rows of a row block are powers of two: shifts (a 64-bit division is 150 instructions, and most work-groups
+    // take a single step)
+    constexpr int kPerLog2 = PER == 8 ? 3 : PER == 4 ? 2 : PER == 2 ? 1 : 0;
+    static_assert(PER == 1 << kPerLog2, "groups per lane and step");
+    const int x_log2 = lanes_log2 + (ALONG ? kPerLog2 : 0), y_log2 = 8 - lanes_log2 + (ALONG ? 0 : kPerLog2);
+    slabs = (groups_per_row + ((int64_t)1 << x_log2) - 1) >> x_log2;
+    row_blocks = (rows + ((int64_t)1 << y_log2) - 1) >> y_log2;
   }
   // the u-th group of this lane in step (slab, rb); false when it lies outside the view
   __device__ bool at(int64_t slab, int64_t rb, int u, int64_t& row, int64_t& group) const {
@@ -48,10 +52,14 @@ template <bool ALONG> struct Walk {
     row = (ALONG ? rb : rb * PER + u) * row_step + lane_row;
     return group < groups_per_row && row < rows;
   }
+  // every group of the step (slab, rb) lies inside the view and is whole (wave-uniform)
+  __device__ bool inside(int64_t slab, int64_t rb, int64_t cols, int G) const {
+    return (slab + 1) * (ALONG ? PER : 1) * lanes * G <= cols && (rb + 1) * row_step * (ALONG ? 1 : PER) <= rows;
+  }
 };
 
-template <int DT, bool ALONG> __global__ void __launch_bounds__(256)
-fill_kernel(typename Elem<DT>::T* dst, int64_t rows, int64_t cols, int64_t ld, float value, int vec_ok, int lanes_log2) {
+template <int DT, int ALONG> __global__ void __launch_bounds__(256)
+fill_kernel(typename Elem<DT>::T* dst, int64_t rows, int64_t cols, int64_t ld, float value, int lanes_log2) {
   typedef typename Elem<DT>::T T;
   constexpr int G = 16 / sizeof(T);
   const Walk<ALONG> w(rows, (cols + G - 1) / G, lanes_log2);
@@ -68,14 +76,14 @@ fill_kernel(typename Elem<DT>::T* dst, int64_t rows, int64_t cols, int64_t ld, f
         if (!w.at(slab, rb, u, r, g)) continue;
         const int64_t c0 = g * G;
         T* p = dst + r * ld + c0;
-        if (vec_ok && c0 + G <= cols) store16(p, *(const v4u*)tmp);
+        if (c0 + G <= cols) store16(p, *(const v4u*)tmp);
         else for (int e = 0; e < G && c0 + e < cols; ++e) p[e] = v;
       }
     }
 }
 
-template <int SDT, int DDT, bool ALONG> __device__ __forceinline__ void
-copy_window(const typename Elem<SDT>::T* src, int64_t sld, typename Elem<DDT>::T* dst, int64_t dld, int64_t rows, int64_t cols, int vec_ok, int lanes_log2) {
+template <int SDT, int DDT, int ALONG> __device__ __forceinline__ void
+copy_window(const typename Elem<SDT>::T* src, int64_t sld, typename Elem<DDT>::T* dst, int64_t dld, int64_t rows, int64_t cols, int lanes_log2) {
   typedef typename Elem<SDT>::T S;
   typedef typename Elem<DDT>::T D;
   constexpr int G = 16 / (sizeof(S) < sizeof(D) ? sizeof(S) : sizeof(D));  // 16 bytes of the narrower side, 32 of the wider
@@ -84,12 +92,50 @@ copy_window(const typename Elem<SDT>::T* src, int64_t sld, typename Elem<DDT>::T
   for (int64_t rb = blockIdx.y; rb < w.row_blocks; rb += gridDim.y)
     for (int64_t slab = blockIdx.x; slab < w.slabs; slab += gridDim.x) {
       S in[PER][G];
+      // one group converted and stored
+      auto put = [&](D* dp, const S (&x)[G]) {
+        D out[G];
+#pragma unroll
+        for (int e = 0; e < G; ++e) {
+          if constexpr (SDT == DDT) out[e] = x[e]; else out[e] = Elem<DDT>::store(Elem<SDT>::load(x[e]));
+        }
+#pragma unroll
+        for (int q = 0; q < (int)(G * sizeof(D) / 16); ++q) {
+          // a lane's two stores of a widening copy each cover half of its 32 bytes: the cache has to merge them
+          if constexpr (sizeof(D) > sizeof(S)) store16((v4u*)dp + q, ((const v4u*)out)[q]); else store16_stream((v4u*)dp + q, ((const v4u*)out)[q]);
+        }
+      };
+      if (w.inside(slab, rb, cols, G)) {  // nothing to check
+        const S* sp[PER];
+#pragma unroll
+        for (int u = 0; u < PER; ++u) {
+          int64_t r, g;
+          w.at(slab, rb, u, r, g);
+          sp[u] = src + r * sld + g * G;
+        }
+#pragma unroll
+        for (int u = 0; u < PER; ++u) {
+          // The groups along a row are fetched one after the other, each waited for before the next is requested, and all stored at the
+          // end: reads and writes then reach memory in longer runs (512 MiB + 512 MiB f32: 6.0 TB/s with both requests in flight
+          // together, 7.4 one after the other).
+          if (ALONG > 1 && u > 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+          for (int q = 0; q < (int)(G * sizeof(S) / 16); ++q) ((v4u*)in[u])[q] = load16((const v4u*)sp[u] + q);
+        }
+#pragma unroll
+        for (int u = 0; u < PER; ++u) {
+          int64_t r, g;
+          w.at(slab, rb, u, r, g);
+          put(dst + r * dld + g * G, in[u]);
+        }
+        continue;
+      }
       bool whole[PER];
       // every load of the step is issued before the first store
 #pragma unroll
       for (int u = 0; u < PER; ++u) {
         int64_t r, g;
-        whole[u] = w.at(slab, rb, u, r, g) && vec_ok && g * G + G <= cols;
+        whole[u] = w.at(slab, rb, u, r, g) && g * G + G <= cols;
         if (whole[u]) {
 #pragma unroll
           for (int q = 0; q < (int)(G * sizeof(S) / 16); ++q) ((v4u*)in[u])[q] = load16((const v4u*)(src + r * sld + g * G) + q);
@@ -100,20 +146,11 @@ copy_window(const typename Elem<SDT>::T* src, int64_t sld, typename Elem<DDT>::T
         int64_t r, g;
         if (!w.at(slab, rb, u, r, g)) continue;
         const int64_t c0 = g * G;
-        const S* sp = src + r * sld + c0;
         D* dp = dst + r * dld + c0;
         if (whole[u]) {
-          D out[G];
-#pragma unroll
-          for (int e = 0; e < G; ++e) {
-            if constexpr (SDT == DDT) out[e] = in[u][e]; else out[e] = Elem<DDT>::store(Elem<SDT>::load(in[u][e]));
-          }
-#pragma unroll
-          for (int q = 0; q < (int)(G * sizeof(D) / 16); ++q) {
-            // a lane's two stores of a widening copy each cover half of its 32 bytes: the cache has to merge them
-            if constexpr (sizeof(D) > sizeof(S)) store16((v4u*)dp + q, ((const v4u*)out)[q]); else store16_stream((v4u*)dp + q, ((const v4u*)out)[q]);
-          }
+          put(dp, in[u]);
         } else {
+          const S* sp = src + r * sld + c0;
           for (int e = 0; e < G && c0 + e < cols; ++e) {
             if constexpr (SDT == DDT) dp[e] = sp[e]; else dp[e] = Elem<DDT>::store(Elem<SDT>::load(sp[e]));
           }
@@ -122,19 +159,18 @@ copy_window(const typename Elem<SDT>::T* src, int64_t sld, typename Elem<DDT>::T
     }
 }
 
-template <int SDT, int DDT, bool ALONG> __global__ void __launch_bounds__(256)
-copy_kernel(const typename Elem<SDT>::T* src, int64_t sld, typename Elem<DDT>::T* dst, int64_t dld, int64_t rows, int64_t cols, int vec_ok, int lanes_log2) {
-  copy_window<SDT, DDT, ALONG>(src, sld, dst, dld, rows, cols, vec_ok, lanes_log2);
+template <int SDT, int DDT, int ALONG> __global__ void __launch_bounds__(256)
+copy_kernel(const typename Elem<SDT>::T* src, int64_t sld, typename Elem<DDT>::T* dst, int64_t dld, int64_t rows, int64_t cols, int lanes_log2) {
+  copy_window<SDT, DDT, ALONG>(src, sld, dst, dld, rows, cols, lanes_log2);
 }
 
 // the same window copied once per tile of a placement: z walks the n0 x n1 tiles, each displacing both sides by its steps
-template <int SDT, int DDT, bool ALONG> __global__ void __launch_bounds__(256)
-copy_tiles_kernel(const typename Elem<SDT>::T* src, int64_t sld, typename Elem<DDT>::T* dst, int64_t dld, int64_t rows, int64_t cols, TilePlacement t, int vec_ok,
-                  int lanes_log2) {
+template <int SDT, int DDT, int ALONG> __global__ void __launch_bounds__(256)
+copy_tiles_kernel(const typename Elem<SDT>::T* src, int64_t sld, typename Elem<DDT>::T* dst, int64_t dld, int64_t rows, int64_t cols, TilePlacement t, int lanes_log2) {
   const int64_t tiles = t.n0 * t.n1;
   for (int64_t z = blockIdx.z; z < tiles; z += gridDim.z) {
     const int64_t a = z / t.n1, b = z - a * t.n1;
-    copy_window<SDT, DDT, ALONG>(src + a * t.src_step0 + b * t.src_step1, sld, dst + a * t.dst_step0 + b * t.dst_step1, dld, rows, cols, vec_ok, lanes_log2);
+    copy_window<SDT, DDT, ALONG>(src + a * t.src_step0 + b * t.src_step1, sld, dst + a * t.dst_step0 + b * t.dst_step1, dld, rows, cols, lanes_log2);
   }
 }
 
@@ -155,7 +191,7 @@ template <int KIND> __device__ __forceinline__ float wave_reduce(float v) {
 // the slices of a row read neighbouring memory at any time.
 // With gridDim.y == 1 the result goes to dst (combined with the old value unless clear), else to partial[y][row].
 template <int DT, int KIND> __global__ void __launch_bounds__(256)
-reduce_rows_kernel(const typename Elem<DT>::T* src, int64_t rows, int64_t cols, int64_t ld, int clear, typename Elem<DT>::T* dst, float* partial, int vec_ok) {
+reduce_rows_kernel(const typename Elem<DT>::T* src, int64_t rows, int64_t cols, int64_t ld, int clear, typename Elem<DT>::T* dst, float* partial) {
   typedef typename Elem<DT>::T T;
   constexpr int G = 16 / sizeof(T);
   const int64_t gpr = (cols + G - 1) / G;
@@ -165,7 +201,7 @@ reduce_rows_kernel(const typename Elem<DT>::T* src, int64_t rows, int64_t cols, 
     const T* row = src + r * ld;
     for (int64_t g = (int64_t)blockIdx.y * 256 + threadIdx.x; g < gpr; g += (int64_t)gridDim.y * 256) {
       const int64_t c0 = g * G;
-      if (vec_ok && c0 + G <= cols) {
+      if (c0 + G <= cols) {
         T in[G];
         *(v4u*)in = load16(row + c0);
 #pragma unroll
@@ -190,7 +226,7 @@ reduce_rows_kernel(const typename Elem<DT>::T* src, int64_t rows, int64_t cols, 
 // NPT groups, and combine by shuffles; a work-group holds 256 >> lanes_log2 rows and takes 4 / NPT such sets of rows per
 // step, so that every lane has four loads in flight before the first is used.
 template <int DT, int KIND, int NPT> __global__ void __launch_bounds__(256)
-reduce_short_rows_kernel(const typename Elem<DT>::T* src, int64_t rows, int64_t cols, int64_t ld, int clear, typename Elem<DT>::T* dst, int vec_ok, int lanes_log2) {
+reduce_short_rows_kernel(const typename Elem<DT>::T* src, int64_t rows, int64_t cols, int64_t ld, int clear, typename Elem<DT>::T* dst, int lanes_log2) {
   typedef typename Elem<DT>::T T;
   constexpr int G = 16 / sizeof(T), SETS = 4 / NPT;
   const int lanes = 1 << lanes_log2, lane = threadIdx.x & (lanes - 1), rows_per_set = 256 >> lanes_log2;
@@ -204,7 +240,7 @@ reduce_short_rows_kernel(const typename Elem<DT>::T* src, int64_t rows, int64_t 
 #pragma unroll
       for (int q = 0; q < NPT; ++q) {
         const int64_t c0 = (int64_t)(q * lanes + lane) * G;
-        whole[t][q] = r < rows && vec_ok && c0 + G <= cols;
+        whole[t][q] = r < rows && c0 + G <= cols;
         if (whole[t][q]) *(v4u*)in[t][q] = load16(src + r * ld + c0);
       }
     }
@@ -238,8 +274,7 @@ reduce_short_rows_kernel(const typename Elem<DT>::T* src, int64_t rows, int64_t 
 constexpr int kStripLanes = 32;  // 16 and 64 lanes measured 9 % and 15 % slower on wide views
 
 template <int DT, int KIND, int kStripFlight> __global__ void __launch_bounds__(256)
-reduce_cols_kernel(const typename Elem<DT>::T* src, int64_t rows, int64_t cols, int64_t ld, int clear, typename Elem<DT>::T* dst, float* partial, int vec_ok,
-                   int lanes_log2) {
+reduce_cols_kernel(const typename Elem<DT>::T* src, int64_t rows, int64_t cols, int64_t ld, int clear, typename Elem<DT>::T* dst, float* partial, int lanes_log2) {
   typedef typename Elem<DT>::T T;
   constexpr int G = 16 / sizeof(T);
   const int cl = threadIdx.x & ((1 << lanes_log2) - 1), rl = threadIdx.x >> lanes_log2, row_lanes = 256 >> lanes_log2;
@@ -249,7 +284,7 @@ reduce_cols_kernel(const typename Elem<DT>::T* src, int64_t rows, int64_t cols, 
 #pragma unroll
   for (int e = 0; e < G; ++e) acc[e] = Op<KIND>::id();
   if (c0 < cols) {
-    const bool whole = vec_ok && c0 + G <= cols;
+    const bool whole = c0 + G <= cols;
     for (int64_t base = (int64_t)blockIdx.y * chunk; base < rows; base += (int64_t)gridDim.y * chunk) {
       if (whole && base + chunk <= rows) {
         T in[kStripFlight][G];
@@ -326,47 +361,59 @@ reduce_finish_kernel(const float* partial, int slices, int64_t n, int clear, typ
 // at most 256; x steps along the row, y down the rows (65535 at most, work-groups loop beyond that)
 struct WalkLaunch {
   dim3 grid;
-  int lanes_log2, along;
-  WalkLaunch(int64_t rows, int64_t groups_per_row) {
+  int lanes_log2, along;  // along: groups per lane along the row, 0: eight rows per lane instead
+  WalkLaunch(int64_t rows, int64_t groups_per_row, int per_lane_along = 2) {
     lanes_log2 = 0;
     while (lanes_log2 < 8 && (int64_t(1) << lanes_log2) < groups_per_row) ++lanes_log2;
-    along = groups_per_row >= 256 * kPerLaneAlong;
-    const int kPerLane = along ? kPerLaneAlong : kPerLaneAcross;
-    const int64_t per_x = (int64_t(1) << lanes_log2) * (along ? kPerLane : 1), per_y = (int64_t)(256 >> lanes_log2) * (along ? 1 : kPerLane);
+    along = groups_per_row >= 512 ? per_lane_along : 0;
+    const int64_t per_x = (int64_t(1) << lanes_log2) * (along ? along : 1), per_y = (int64_t)(256 >> lanes_log2) * (along ? 1 : kPerLaneAcross);
     const int64_t slabs = (groups_per_row + per_x - 1) / per_x, row_blocks = (rows + per_y - 1) / per_y;
     grid = dim3((unsigned)(slabs < 1 ? 1 : (slabs > 0x7fffffff ? 0x7fffffff : slabs)), (unsigned)(row_blocks < 1 ? 1 : (row_blocks > 65535 ? 65535 : row_blocks)));
   }
 };
 
-template <int DT> hipError_t fill_t(void* dst, int64_t rows, int64_t cols, int64_t ld, double value, int vec_ok, hipStream_t s) {
+// Groups per lane of a copy along its rows.  f32 to f32, TB/s read and written, 1 / 2 / 4 groups: 16 MiB 7.2 / 5.7 / 4.8 (too few
+// work-groups), 256 MiB 6.6 / 7.2 / 6.7, 512 MiB 6.6 / 7.4 / 6.9, 768 MiB 6.5 / 6.2 / 6.9, 1 GiB 6.5 / 6.1 / 6.9, 2 GiB 6.5 / 6.0 / 6.0: more than one
+// pays until the launch has 65536 work-groups.
+int copy_groups_per_lane(int64_t rows, int64_t groups_per_row) {
+  const int64_t one = rows * ((groups_per_row + 255) / 256), two = rows * ((groups_per_row + 511) / 512), four = rows * ((groups_per_row + 1023) / 1024);
+  if (one <= 8192) return 1;
+  return two <= 65536 ? 2 : four <= 65536 ? 4 : 1;
+}
+
+template <int DT> hipError_t fill_t(void* dst, int64_t rows, int64_t cols, int64_t ld, double value, hipStream_t s) {
   typedef typename Elem<DT>::T T;
   constexpr int G = 16 / sizeof(T);
   const WalkLaunch w(rows, (cols + G - 1) / G);
-  if (w.along) hipLaunchKernelGGL((fill_kernel<DT, true>), w.grid, dim3(256), 0, s, (T*)dst, rows, cols, ld, (float)value, vec_ok, w.lanes_log2);
-  else hipLaunchKernelGGL((fill_kernel<DT, false>), w.grid, dim3(256), 0, s, (T*)dst, rows, cols, ld, (float)value, vec_ok, w.lanes_log2);
+  if (w.along) hipLaunchKernelGGL((fill_kernel<DT, 2>), w.grid, dim3(256), 0, s, (T*)dst, rows, cols, ld, (float)value, w.lanes_log2);
+  else hipLaunchKernelGGL((fill_kernel<DT, 0>), w.grid, dim3(256), 0, s, (T*)dst, rows, cols, ld, (float)value, w.lanes_log2);
   return hipGetLastError();
 }
 
-template <int SDT, int DDT> hipError_t copy_t(const void* src, int64_t sld, void* dst, int64_t dld, int64_t rows, int64_t cols, int vec_ok, hipStream_t s) {
+template <int SDT, int DDT> hipError_t copy_t(const void* src, int64_t sld, void* dst, int64_t dld, int64_t rows, int64_t cols, hipStream_t s) {
   typedef typename Elem<SDT>::T S;
   typedef typename Elem<DDT>::T D;
   constexpr int G = 16 / (sizeof(S) < sizeof(D) ? sizeof(S) : sizeof(D));
-  const WalkLaunch w(rows, (cols + G - 1) / G);
-  if (w.along) hipLaunchKernelGGL((copy_kernel<SDT, DDT, true>), w.grid, dim3(256), 0, s, (const S*)src, sld, (D*)dst, dld, rows, cols, vec_ok, w.lanes_log2);
-  else hipLaunchKernelGGL((copy_kernel<SDT, DDT, false>), w.grid, dim3(256), 0, s, (const S*)src, sld, (D*)dst, dld, rows, cols, vec_ok, w.lanes_log2);
+  const WalkLaunch w(rows, (cols + G - 1) / G, copy_groups_per_lane(rows, (cols + G - 1) / G));
+  auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, w.grid, dim3(256), 0, s, (const S*)src, sld, (D*)dst, dld, rows, cols, w.lanes_log2); };
+  switch (w.along) {
+    case 1: launch(copy_kernel<SDT, DDT, 1>); break;
+    case 2: launch(copy_kernel<SDT, DDT, 2>); break;
+    case 4: launch(copy_kernel<SDT, DDT, 4>); break;
+    default: launch(copy_kernel<SDT, DDT, 0>); break;
+  }
   return hipGetLastError();
 }
 
-template <int SDT, int DDT> hipError_t copy_tiles_t(const void* src, int64_t sld, void* dst, int64_t dld, int64_t rows, int64_t cols, const TilePlacement& t, int vec_ok,
-                                                    hipStream_t s) {
+template <int SDT, int DDT> hipError_t copy_tiles_t(const void* src, int64_t sld, void* dst, int64_t dld, int64_t rows, int64_t cols, const TilePlacement& t, hipStream_t s) {
   typedef typename Elem<SDT>::T S;
   typedef typename Elem<DDT>::T D;
   constexpr int G = 16 / (sizeof(S) < sizeof(D) ? sizeof(S) : sizeof(D));
   WalkLaunch w(rows, (cols + G - 1) / G);
   const int64_t tiles = t.n0 * t.n1;
   w.grid.z = (unsigned)(tiles > 65535 ? 65535 : tiles);
-  if (w.along) hipLaunchKernelGGL((copy_tiles_kernel<SDT, DDT, true>), w.grid, dim3(256), 0, s, (const S*)src, sld, (D*)dst, dld, rows, cols, t, vec_ok, w.lanes_log2);
-  else hipLaunchKernelGGL((copy_tiles_kernel<SDT, DDT, false>), w.grid, dim3(256), 0, s, (const S*)src, sld, (D*)dst, dld, rows, cols, t, vec_ok, w.lanes_log2);
+  if (w.along) hipLaunchKernelGGL((copy_tiles_kernel<SDT, DDT, 2>), w.grid, dim3(256), 0, s, (const S*)src, sld, (D*)dst, dld, rows, cols, t, w.lanes_log2);
+  else hipLaunchKernelGGL((copy_tiles_kernel<SDT, DDT, 0>), w.grid, dim3(256), 0, s, (const S*)src, sld, (D*)dst, dld, rows, cols, t, w.lanes_log2);
   return hipGetLastError();
 }
 
@@ -374,7 +421,7 @@ template <int SDT, int DDT> hipError_t copy_tiles_t(const void* src, int64_t sld
 constexpr int64_t kMaxGrid = 1 << 22;
 
 template <int DT, int KIND> hipError_t reduce_t(const void* src, int64_t rows, int64_t cols, int64_t ld, int dim, int clear, void* dst, float* partial,
-                                                int slices, int vec_ok, hipStream_t s) {
+                                                int slices, hipStream_t s) {
   typedef typename Elem<DT>::T T;
   constexpr int G = 16 / sizeof(T);
   const int64_t gpr = (cols + G - 1) / G;
@@ -384,12 +431,12 @@ template <int DT, int KIND> hipError_t reduce_t(const void* src, int64_t rows, i
       while (lanes_log2 < 6 && (int64_t(1) << lanes_log2) < gpr) ++lanes_log2;
       const int64_t rows_per_step = (256 >> lanes_log2) * (gpr <= 64 ? 4 : (gpr <= 128 ? 2 : 1)), blocks = (rows + rows_per_step - 1) / rows_per_step;
       const dim3 grid((unsigned)(blocks < kMaxGrid ? blocks : kMaxGrid));
-      if (gpr <= 64) hipLaunchKernelGGL((reduce_short_rows_kernel<DT, KIND, 1>), grid, dim3(256), 0, s, (const T*)src, rows, cols, ld, clear, (T*)dst, vec_ok, lanes_log2);
-      else if (gpr <= 128) hipLaunchKernelGGL((reduce_short_rows_kernel<DT, KIND, 2>), grid, dim3(256), 0, s, (const T*)src, rows, cols, ld, clear, (T*)dst, vec_ok, lanes_log2);
-      else hipLaunchKernelGGL((reduce_short_rows_kernel<DT, KIND, 4>), grid, dim3(256), 0, s, (const T*)src, rows, cols, ld, clear, (T*)dst, vec_ok, lanes_log2);
+      if (gpr <= 64) hipLaunchKernelGGL((reduce_short_rows_kernel<DT, KIND, 1>), grid, dim3(256), 0, s, (const T*)src, rows, cols, ld, clear, (T*)dst, lanes_log2);
+      else if (gpr <= 128) hipLaunchKernelGGL((reduce_short_rows_kernel<DT, KIND, 2>), grid, dim3(256), 0, s, (const T*)src, rows, cols, ld, clear, (T*)dst, lanes_log2);
+      else hipLaunchKernelGGL((reduce_short_rows_kernel<DT, KIND, 4>), grid, dim3(256), 0, s, (const T*)src, rows, cols, ld, clear, (T*)dst, lanes_log2);
     } else {
       hipLaunchKernelGGL((reduce_rows_kernel<DT, KIND>), dim3((unsigned)(rows < kMaxGrid ? rows : kMaxGrid), (unsigned)slices), dim3(256), 0, s, (const T*)src, rows, cols,
-                         ld, clear, (T*)dst, partial, vec_ok);
+                         ld, clear, (T*)dst, partial);
     }
   } else {
     int lanes_log2 = 0;
@@ -398,9 +445,9 @@ template <int DT, int KIND> hipError_t reduce_t(const void* src, int64_t rows, i
     const unsigned strips = (unsigned)((gpr + (1 << lanes_log2) - 1) >> lanes_log2);
     // a view of one strip gives at most one work-group per slice: its lanes keep more rows in flight instead
     if (strips == 1) hipLaunchKernelGGL((reduce_cols_kernel<DT, KIND, 16>), dim3(strips, (unsigned)slices), dim3(256), 0, s, (const T*)src, rows, cols, ld, clear, (T*)dst,
-                                        partial, vec_ok, lanes_log2);
+                                        partial, lanes_log2);
     else hipLaunchKernelGGL((reduce_cols_kernel<DT, KIND, 4>), dim3(strips, (unsigned)slices), dim3(256), 0, s, (const T*)src, rows, cols, ld, clear, (T*)dst, partial,
-                            vec_ok, lanes_log2);
+                            lanes_log2);
   }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || slices == 1) return e;
@@ -410,12 +457,12 @@ template <int DT, int KIND> hipError_t reduce_t(const void* src, int64_t rows, i
 }
 
 template <int DT> hipError_t reduce_k(int kind, const void* src, int64_t rows, int64_t cols, int64_t ld, int dim, int clear, void* dst, float* partial, int slices,
-                                      int vec_ok, hipStream_t s) {
+                                      hipStream_t s) {
   switch (kind) {
-    case FRISK_REDUCE_ADD: return reduce_t<DT, FRISK_REDUCE_ADD>(src, rows, cols, ld, dim, clear, dst, partial, slices, vec_ok, s);
-    case FRISK_REDUCE_MUL: return reduce_t<DT, FRISK_REDUCE_MUL>(src, rows, cols, ld, dim, clear, dst, partial, slices, vec_ok, s);
-    case FRISK_REDUCE_MIN: return reduce_t<DT, FRISK_REDUCE_MIN>(src, rows, cols, ld, dim, clear, dst, partial, slices, vec_ok, s);
-    default: return reduce_t<DT, FRISK_REDUCE_MAX>(src, rows, cols, ld, dim, clear, dst, partial, slices, vec_ok, s);
+    case FRISK_REDUCE_ADD: return reduce_t<DT, FRISK_REDUCE_ADD>(src, rows, cols, ld, dim, clear, dst, partial, slices, s);
+    case FRISK_REDUCE_MUL: return reduce_t<DT, FRISK_REDUCE_MUL>(src, rows, cols, ld, dim, clear, dst, partial, slices, s);
+    case FRISK_REDUCE_MIN: return reduce_t<DT, FRISK_REDUCE_MIN>(src, rows, cols, ld, dim, clear, dst, partial, slices, s);
+    default: return reduce_t<DT, FRISK_REDUCE_MAX>(src, rows, cols, ld, dim, clear, dst, partial, slices, s);
   }
 }
 
@@ -433,17 +480,16 @@ int reduce_slices(int dtype, int64_t rows, int64_t cols, int dim) {
   return slices;
 }
 
-hipError_t launch_fill(int dtype, void* dst, int64_t rows, int64_t cols, int64_t ld, double value, int vec_ok, hipStream_t s) {
+hipError_t launch_fill(int dtype, void* dst, int64_t rows, int64_t cols, int64_t ld, double value, hipStream_t s) {
   switch (dtype) {
-    case FRISK_F32: return fill_t<FRISK_F32>(dst, rows, cols, ld, value, vec_ok, s);
-    case FRISK_F16: return fill_t<FRISK_F16>(dst, rows, cols, ld, value, vec_ok, s);
-    default: return fill_t<FRISK_BF16>(dst, rows, cols, ld, value, vec_ok, s);
+    case FRISK_F32: return fill_t<FRISK_F32>(dst, rows, cols, ld, value, s);
+    case FRISK_F16: return fill_t<FRISK_F16>(dst, rows, cols, ld, value, s);
+    default: return fill_t<FRISK_BF16>(dst, rows, cols, ld, value, s);
   }
 }
 
-hipError_t launch_copy_tiles(int sdt, const void* src, int64_t sld, int ddt, void* dst, int64_t dld, int64_t rows, int64_t cols, const TilePlacement& t, int vec_ok,
-                             hipStream_t s) {
-#define FRISK_COPY_CASE(S, D) if (sdt == S && ddt == D) return copy_tiles_t<S, D>(src, sld, dst, dld, rows, cols, t, vec_ok, s);
+hipError_t launch_copy_tiles(int sdt, const void* src, int64_t sld, int ddt, void* dst, int64_t dld, int64_t rows, int64_t cols, const TilePlacement& t, hipStream_t s) {
+#define FRISK_COPY_CASE(S, D) if (sdt == S && ddt == D) return copy_tiles_t<S, D>(src, sld, dst, dld, rows, cols, t, s);
   FRISK_COPY_CASE(FRISK_F32, FRISK_F32) FRISK_COPY_CASE(FRISK_F32, FRISK_F16) FRISK_COPY_CASE(FRISK_F32, FRISK_BF16)
   FRISK_COPY_CASE(FRISK_F16, FRISK_F32) FRISK_COPY_CASE(FRISK_F16, FRISK_F16) FRISK_COPY_CASE(FRISK_F16, FRISK_BF16)
   FRISK_COPY_CASE(FRISK_BF16, FRISK_F32) FRISK_COPY_CASE(FRISK_BF16, FRISK_F16) FRISK_COPY_CASE(FRISK_BF16, FRISK_BF16)
@@ -451,8 +497,8 @@ hipError_t launch_copy_tiles(int sdt, const void* src, int64_t sld, int ddt, voi
   return hipErrorInvalidValue;
 }
 
-hipError_t launch_copy(int sdt, const void* src, int64_t sld, int ddt, void* dst, int64_t dld, int64_t rows, int64_t cols, int vec_ok, hipStream_t s) {
-#define FRISK_COPY_CASE(S, D) if (sdt == S && ddt == D) return copy_t<S, D>(src, sld, dst, dld, rows, cols, vec_ok, s);
+hipError_t launch_copy(int sdt, const void* src, int64_t sld, int ddt, void* dst, int64_t dld, int64_t rows, int64_t cols, hipStream_t s) {
+#define FRISK_COPY_CASE(S, D) if (sdt == S && ddt == D) return copy_t<S, D>(src, sld, dst, dld, rows, cols, s);
   FRISK_COPY_CASE(FRISK_F32, FRISK_F32) FRISK_COPY_CASE(FRISK_F32, FRISK_F16) FRISK_COPY_CASE(FRISK_F32, FRISK_BF16)
   FRISK_COPY_CASE(FRISK_F16, FRISK_F32) FRISK_COPY_CASE(FRISK_F16, FRISK_F16) FRISK_COPY_CASE(FRISK_F16, FRISK_BF16)
   FRISK_COPY_CASE(FRISK_BF16, FRISK_F32) FRISK_COPY_CASE(FRISK_BF16, FRISK_F16) FRISK_COPY_CASE(FRISK_BF16, FRISK_BF16)
@@ -461,11 +507,11 @@ hipError_t launch_copy(int sdt, const void* src, int64_t sld, int ddt, void* dst
 }
 
 hipError_t launch_reduce(int dtype, const void* src, int64_t rows, int64_t cols, int64_t ld, int dim, int kind, int clear, void* dst, float* partial, int slices,
-                         int vec_ok, hipStream_t s) {
+                         hipStream_t s) {
   switch (dtype) {
-    case FRISK_F32: return reduce_k<FRISK_F32>(kind, src, rows, cols, ld, dim, clear, dst, partial, slices, vec_ok, s);
-    case FRISK_F16: return reduce_k<FRISK_F16>(kind, src, rows, cols, ld, dim, clear, dst, partial, slices, vec_ok, s);
-    default: return reduce_k<FRISK_BF16>(kind, src, rows, cols, ld, dim, clear, dst, partial, slices, vec_ok, s);
+    case FRISK_F32: return reduce_k<FRISK_F32>(kind, src, rows, cols, ld, dim, clear, dst, partial, slices, s);
+    case FRISK_F16: return reduce_k<FRISK_F16>(kind, src, rows, cols, ld, dim, clear, dst, partial, slices, s);
+    default: return reduce_k<FRISK_BF16>(kind, src, rows, cols, ld, dim, clear, dst, partial, slices, s);
   }
 }
 
