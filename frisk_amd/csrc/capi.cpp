@@ -963,8 +963,6 @@ int frisk_hip_attention(const frisk_attention_desc* d, const void* Q, const void
   AttentionParams p;
   p.Q = Q; p.K = K; p.V = V; p.O = O; p.lse = lse;
   p.batch_heads = (int32_t)bh; p.seq_q = (int32_t)d->seq_q; p.seq_k = (int32_t)d->seq_k;
-  p.q_blocks = (int32_t)(d->seq_q / kAttnQueriesPerGroup);
-  p.xcd_remap = groups % 8 == 0 ? 1 : 0;
   p.scale_log2 = d->scale * 1.4426950408889634f;
   hipError_t e = launch_attention(d->dtype, d->k_transposed ? 1 : 0, p, (hipStream_t)stream);
   if (e != hipSuccess) return fail(FRISK_ERR_DEVICE, "attention launch failed: %s", hipGetErrorString(e));

@@ -183,3 +183,52 @@ def test_attention_sketch_shape_32_heads_4096(k_transposed):
         check(dtype, got[slot], lse[slot], ref[pick[slot]], ref_lse[pick[slot]])
     for slot in range(3, bh):
         assert np.array_equal(got[slot], got[pick[slot]]) and np.array_equal(lse[slot], lse[pick[slot]])
+
+
+SHARED_KEYS = [
+    # few work-groups: the keys are dealt to 8, 4 or 2 shares (batch*heads, seq_q, seq_k)
+    (1, 256, 256),    # 8 shares of one tile of 32 keys
+    (3, 256, 320),    # 8 shares, two of them a tile longer
+    (32, 256, 2112),  # 8 shares of 8 or 9 tiles, every CU busy
+    (40, 256, 256),   # 4 shares of one tile of 64 keys
+    (5, 2048, 448),   # 4 shares, three of them a tile longer
+    (80, 256, 128),   # 2 shares of one tile
+    (33, 512, 320),   # 2 shares of 3 and 2 tiles, no XCD remap
+    (36, 2048, 640),  # more groups than CUs
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [O.F16, O.BF16], ids=lambda d: NAMES[d])
+@pytest.mark.parametrize("k_transposed", [False, True], ids=["k_rows", "k_transposed"])
+@pytest.mark.parametrize("case", SHARED_KEYS, ids=lambda c: "bh%d_q%d_k%d" % c)
+def test_attention_with_keys_in_shares(dtype, k_transposed, case):
+    bh, sq, sk = case
+    heads = min(bh, 3)  # the oracle checks these; the other slots repeat them
+    q1, k1, v1 = make_qkv(dtype, heads, sq, sk, 128, seed=51 + sk, k_transposed=k_transposed)
+    pick = [i % heads for i in range(bh)]
+    got, lse = run_attention(dtype, q1[pick], k1[pick], v1[pick], 0.3, k_transposed)
+    ref, ref_lse = A.attention_f64(dtype, q1, k1, v1, 0.3, k_transposed)
+    check(dtype, got[:heads], lse[:heads], ref, ref_lse)
+    for slot in range(heads, bh):
+        assert np.array_equal(got[slot], got[pick[slot]]) and np.array_equal(lse[slot], lse[pick[slot]])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bh", [2, 40, 80], ids=["8_shares", "4_shares", "2_shares"])
+def test_attention_share_of_masked_keys(bh):
+    """a share whose scores are all -inf adds nothing; NaN and +inf reach the rows they belong to and no others"""
+    dtype, sq, sk, d = O.F16, 256, 512, 128
+    q, k, v = make_qkv(dtype, bh, sq, sk, d, seed=61)
+    q = np.bitwise_and(q, 0x7FFF)  # positive queries: a key of -inf scores -inf
+    masked = k.copy()
+    masked[:, 256:] = O.encode(dtype, np.array([-np.inf], dtype=np.float32))[0]
+    got, lse = run_attention(dtype, q, masked, v, 0.2)
+    ref, ref_lse = A.attention_f64(dtype, q, np.ascontiguousarray(k[:, :256]), np.ascontiguousarray(v[:, :256]), 0.2)
+    check(dtype, got, lse, ref, ref_lse)
+    q2 = q.copy()
+    q2[:, 7, 3] = O.encode(dtype, np.array([np.nan], dtype=np.float32))[0]
+    got2, lse2 = run_attention(dtype, q2, masked, v, 0.2)
+    assert np.isnan(O.decode(dtype, got2[:, 7].reshape(-1))).all() and np.isnan(lse2[:, 7]).all()
+    rest = [i for i in range(sq) if i != 7]
+    assert np.array_equal(got2[:, rest], got[:, rest]) and np.array_equal(lse2[:, rest], lse[:, rest])
