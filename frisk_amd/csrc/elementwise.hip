@@ -9,7 +9,7 @@
 // assembly over fixed registers: a step is two lane reads of the program, a jump to its handler and 8 vector instructions in
 // place, the operand picked by the register index mode.  (As a C++ switch the compiler joins the values of all cases after every
 // step by register moves: 327 vector, 300 scalar and 120 branch instructions per group of 8 columns for (x - s * c) * g + b; here
-// 136, 171 and 35.)  That body on 8192 x 8192 f16: 139 us before, 62.7 now (a plain copy: 41); log2(max(x, c) / (x + c)), bound by
+// 109, 125 and 34.)  That body on 8192 x 8192 f16: 139 us before, 54 now (a plain copy: 41); log2(max(x, c) / (x + c)), bound by
 // the vector pipe in its division, 125 -> 71.5; rows off 16-byte boundaries (4095 x 8191) 370 -> 51.
 // Operands that are the same for every row stay in registers while the lane's columns do, values of one per row stay one
 // register, and what the next group needs from memory is fetched while the current one is evaluated.  All arithmetic is
@@ -185,117 +185,121 @@ template <int DT, bool AHEAD, int DEPTH, bool UNIFORM_ROW> __global__ void __lau
 #pragma unroll
   for (int c = 0; c < 2; ++c) { code_reg[c] = prog.code[c * kChunk + (threadIdx.x & 63)]; imm_reg[c] = __builtin_bit_cast(int, prog.imm[c * kChunk + (threadIdx.x & 63)]); }
   auto type_of = [&](int k) { return DT >= 0 ? DT : p.in_dtype[k]; };
-  // where this lane is in step (rb, slab): lanes beyond the view repeat its last row or group and store nothing
-  struct Place { int64_t row; int off, valid; bool live; };
-  auto place = [&](int64_t rb_, int64_t slab_) {
-    Place q;
-    const int64_t row = rb_ * row_step + lane_row, left = groups - (slab_ << lanes_log2);
-    q.live = row < p.rows && lane_group < left;
-    q.row = row < p.rows ? row : p.rows - 1;
-    q.off = lane_group < left ? lane_group : (int)left - 1;
-    const int64_t rest = p.cols - ((slab_ << lanes_log2) + q.off) * V;
-    q.valid = rest < V ? (int)rest : V;
-    return q;
-  };
-  // element (row, first column of the group) of operand k, whose elements are of type dt
-  auto operand_at = [&](int k, int dt, bool walks, const Place& q, int64_t slab_) {
-    const int es = dt == FRISK_F32 ? 4 : 2;
-    const char* base = (const char*)p.in[k] + q.row * (p.in_row_stride[k] * es);
-    return walks ? base + (slab_ << lanes_log2) * (V * es) + (unsigned)(q.off * (V * es)) : base;
-  };
-  auto fetch = [&](int k, int dt, const Place& q, int64_t slab_, bool streamed) {
-    const char* at = operand_at(k, dt, true, q, slab_);
-    if (!ragged || q.valid >= V) return load_raw(at, dt, streamed);
-    return load_raw_partial(at, dt, q.valid);
-  };
-  auto fetch_row = [&](int k, const Place& q) {
-    const char* at = operand_at(k, p.in_dtype[k], false, q, 0);
-    return p.in_dtype[k] == FRISK_F32 ? *(const unsigned*)at : (unsigned)*(const uint16_t*)at;
-  };
   auto row_value = [&](int k, unsigned bits) {
     if (p.in_dtype[k] == FRISK_F32) return __builtin_bit_cast(float, bits);
     if (p.in_dtype[k] == FRISK_F16) return (float)__builtin_bit_cast(_Float16, (uint16_t)bits);
     return __builtin_bit_cast(float, bits << 16);
   };
+  const int64_t rb0 = blockIdx.y, row_stride = (int64_t)gridDim.y * row_step;  // rows between this lane's groups
+  if (rb0 >= row_blocks) return;
+  // A lane keeps its columns and walks down the rows, every operand's address moving on by one stride: worked out anew for every
+  // group, place and addresses made the counts above 136, 171 and 35, and 62.7 us of the 54 (a SIMD issues one scalar instruction in
+  // four cycles, so they weigh as much as the vector ones).
+  for (int64_t slab = blockIdx.x; slab < slabs; slab += gridDim.x) {
+    // lanes beyond the view repeat its last row or group and store nothing
+    const int64_t left = groups - (slab << lanes_log2);
+    const int off = lane_group < left ? lane_group : (int)left - 1;
+    const int64_t first_col = ((slab << lanes_log2) + off) * V;
+    const int valid = p.cols - first_col < V ? (int)(p.cols - first_col) : V;
+    int64_t row = rb0 * row_step + lane_row;
+    const int64_t row_in = row < p.rows ? row : p.rows - 1;
+    // element (row_in, first column of the group) of operand k, whose elements are of type dt
+    auto operand_at = [&](int k, int dt, bool walks, int64_t r) {
+      const int es = dt == FRISK_F32 ? 4 : 2;
+      const char* base = (const char*)p.in[k] + r * (p.in_row_stride[k] * es);
+      return walks ? base + (slab << lanes_log2) * (V * es) + (unsigned)(off * (V * es)) : base;
+    };
+    auto fetch_at = [&](const char* at, int dt, bool streamed) {
+      if (!ragged || valid >= V) return load_raw(at, dt, streamed);
+      return load_raw_partial(at, dt, valid);
+    };
+    auto fetch_row_at = [&](const char* at, int k) { return p.in_dtype[k] == FRISK_F32 ? *(const unsigned*)at : (unsigned)*(const uint16_t*)at; };
+    auto stride_of = [&](int k, int dt) { return row_stride * p.in_row_stride[k] * (dt == FRISK_F32 ? 4 : 2); };
+    const char *head_at = nullptr, *walk2_at = nullptr, *row0_at = nullptr, *row1_at = nullptr;
+    int64_t head_step = 0, walk2_step = 0, row0_step = 0, row1_step = 0;
+    if (prog.head >= 0) { head_at = operand_at(prog.head, type_of(prog.head), true, row_in); head_step = stride_of(prog.head, type_of(prog.head)); }
+    if constexpr (AHEAD) {
+      if (prog.walk2 >= 0) { walk2_at = operand_at(prog.walk2, type_of(prog.walk2), true, row_in); walk2_step = stride_of(prog.walk2, type_of(prog.walk2)); }
+      if (prog.row0 >= 0) { row0_at = operand_at(prog.row0, p.in_dtype[prog.row0], false, row_in); row0_step = stride_of(prog.row0, p.in_dtype[prog.row0]); }
+      if (prog.row1 >= 0) { row1_at = operand_at(prog.row1, p.in_dtype[prog.row1], false, row_in); row1_step = stride_of(prog.row1, p.in_dtype[prog.row1]); }
+    }
+    const int out_dt = DT >= 0 ? DT : p.out_dtype, out_es = out_dt == FRISK_F32 ? 4 : 2;
+    char* out_at = (char*)p.out + row_in * (p.out_ld * out_es) + (slab << lanes_log2) * (V * out_es) + (unsigned)(off * (V * out_es));
+    const int64_t out_step = row_stride * p.out_ld * out_es;
 
-  int64_t rb = blockIdx.y, slab = blockIdx.x;
-  if (rb >= row_blocks || slab >= slabs) return;
-  Place here = place(rb, slab);
-  Raw ahead{}, ahead2{};
-  unsigned row0 = 0, row1 = 0;
-  v8f col0{}, col1{};
-  auto fetch_ahead = [&](const Place& q, int64_t slab_) {
-    if (prog.head >= 0) ahead = fetch(prog.head, type_of(prog.head), q, slab_, true);
-    if constexpr (AHEAD) {
-      if (prog.walk2 >= 0) ahead2 = fetch(prog.walk2, type_of(prog.walk2), q, slab_, true);
-      if (prog.row0 >= 0) row0 = fetch_row(prog.row0, q);
-      if (prog.row1 >= 0) row1 = fetch_row(prog.row1, q);
-    }
-  };
-  auto fetch_cols = [&](const Place& q, int64_t slab_) {
-    if constexpr (AHEAD) {
-      if (prog.col0 >= 0) to_float(fetch(prog.col0, p.in_dtype[prog.col0], q, slab_, false), p.in_dtype[prog.col0], col0);
-      if (prog.col1 >= 0) to_float(fetch(prog.col1, p.in_dtype[prog.col1], q, slab_, false), p.in_dtype[prog.col1], col1);
-    }
-  };
-  fetch_ahead(here, slab);
-  fetch_cols(here, slab);
-  for (;;) {
-    int64_t next_rb = rb, next_slab = slab + gridDim.x;
-    if (next_slab >= slabs) { next_slab = blockIdx.x; next_rb += gridDim.y; }
-    const bool more = next_rb < row_blocks;
-    const Place there = place(more ? next_rb : rb, more ? next_slab : slab);
-    v8f top, s0, s1, s2, s3, s4, x, walk2;
-    asm volatile("" : "=v"(top), "=v"(s0), "=v"(x), "=v"(walk2));  // written by the program before it reads them
-    if constexpr (DEPTH > 1) asm volatile("" : "=v"(s1), "=v"(s2), "=v"(s3), "=v"(s4));
-    float row_a = 0.f, row_b = 0.f;
-    if (prog.head >= 0) to_float(ahead, type_of(prog.head), top);
-    if constexpr (AHEAD) {
-      if (prog.walk2 >= 0) to_float(ahead2, type_of(prog.walk2), walk2);
-      if (prog.row0 >= 0) row_a = row_value(prog.row0, row0);
-      if (prog.row1 >= 0) row_b = row_value(prog.row1, row1);
-    }
-    if (more) fetch_ahead(there, next_slab);
-    int pc = 0, code = code_reg[0], imm = imm_reg[0];
-    for (;;) {
-      int step;
-      if constexpr (AHEAD && DEPTH > 1)
-        asm volatile(EW_INTERPRETER : "={s50}"(step), "+{s51}"(pc), "+{v[16:23]}"(top), "+{v[24:31]}"(s0), "+{v[32:39]}"(x), "+{v[64:71]}"(s1), "+{v[72:79]}"(s2),
-                     "+{v[80:87]}"(s3), "+{v[88:95]}"(s4) : "{v12}"(code), "{v13}"(imm), "{v14}"(row_a), "{v15}"(row_b), "{v[40:47]}"(col0), "{v[48:55]}"(col1),
-                     "{v[56:63]}"(walk2) : EW_CLOBBERS);
-      else if constexpr (AHEAD)
-        asm volatile(EW_INTERPRETER : "={s50}"(step), "+{s51}"(pc), "+{v[16:23]}"(top), "+{v[24:31]}"(s0), "+{v[32:39]}"(x) : "{v12}"(code), "{v13}"(imm),
-                     "{v14}"(row_a), "{v15}"(row_b), "{v[40:47]}"(col0), "{v[48:55]}"(col1), "{v[56:63]}"(walk2) : EW_CLOBBERS);
-      else if constexpr (DEPTH > 1)
-        asm volatile(EW_INTERPRETER : "={s50}"(step), "+{s51}"(pc), "+{v[16:23]}"(top), "+{v[24:31]}"(s0), "+{v[32:39]}"(x), "+{v[64:71]}"(s1), "+{v[72:79]}"(s2),
-                     "+{v[80:87]}"(s3), "+{v[88:95]}"(s4) : "{v12}"(code), "{v13}"(imm) : EW_CLOBBERS);
-      else
-        asm volatile(EW_INTERPRETER : "={s50}"(step), "+{s51}"(pc), "+{v[16:23]}"(top), "+{v[24:31]}"(s0), "+{v[32:39]}"(x) : "{v12}"(code), "{v13}"(imm) : EW_CLOBBERS);
-      const int what = step >> 24;
-      if (what == STEP_END) break;
-      if (what == STEP_FETCH) {
-        const int k = (step >> 8) & 15;
-        if (p.in_col_stride[k]) to_float(fetch(k, p.in_dtype[k], here, slab, false), p.in_dtype[k], x);
-        else x = v8f{} + row_value(k, fetch_row(k, here));
-      } else if (what == STEP_MORE) {
-        code = code_reg[1];
-        imm = imm_reg[1];
-        pc = 0;
-      } else {
-#pragma unroll
-        for (int e = 0; e < V; ++e) top[e] = top[e] / x[e];
+    Raw ahead{}, ahead2{};
+    unsigned row0 = 0, row1 = 0;
+    v8f col0{}, col1{};
+    auto fetch_ahead = [&]() {
+      if (prog.head >= 0) ahead = fetch_at(head_at, type_of(prog.head), true);
+      if constexpr (AHEAD) {
+        if (prog.walk2 >= 0) ahead2 = fetch_at(walk2_at, type_of(prog.walk2), true);
+        if (prog.row0 >= 0) row0 = fetch_row_at(row0_at, prog.row0);
+        if (prog.row1 >= 0) row1 = fetch_row_at(row1_at, prog.row1);
       }
+    };
+    fetch_ahead();
+    if constexpr (AHEAD) {
+      if (prog.col0 >= 0) to_float(fetch_at(operand_at(prog.col0, p.in_dtype[prog.col0], true, 0), p.in_dtype[prog.col0], false), p.in_dtype[prog.col0], col0);
+      if (prog.col1 >= 0) to_float(fetch_at(operand_at(prog.col1, p.in_dtype[prog.col1], true, 0), p.in_dtype[prog.col1], false), p.in_dtype[prog.col1], col1);
     }
-    if (here.live) {
-      const int dt = DT >= 0 ? DT : p.out_dtype, es = dt == FRISK_F32 ? 4 : 2;
-      char* at = (char*)p.out + here.row * (p.out_ld * es) + (slab << lanes_log2) * (V * es) + (unsigned)(here.off * (V * es));
-      store_group(at, dt, top, here.valid);
+    for (int64_t rb = rb0;;) {
+      const int64_t next_rb = rb + gridDim.y;
+      const bool more = next_rb < row_blocks, live = row < p.rows && lane_group < left;
+      v8f top, s0, s1, s2, s3, s4, x, walk2;
+      asm volatile("" : "=v"(top), "=v"(s0), "=v"(x), "=v"(walk2));  // written by the program before it reads them
+      if constexpr (DEPTH > 1) asm volatile("" : "=v"(s1), "=v"(s2), "=v"(s3), "=v"(s4));
+      float row_a = 0.f, row_b = 0.f;
+      if (prog.head >= 0) to_float(ahead, type_of(prog.head), top);
+      if constexpr (AHEAD) {
+        if (prog.walk2 >= 0) to_float(ahead2, type_of(prog.walk2), walk2);
+        if (prog.row0 >= 0) row_a = row_value(prog.row0, row0);
+        if (prog.row1 >= 0) row_b = row_value(prog.row1, row1);
+      }
+      const int64_t here = row < p.rows ? row : p.rows - 1;
+      if (more) {
+        row += row_stride;
+        if (row < p.rows) {  // (a lane whose next row lies beyond the view fetches the present one again)
+          head_at += head_step;
+          if constexpr (AHEAD) { walk2_at += walk2_step; row0_at += row0_step; row1_at += row1_step; }
+        }
+        fetch_ahead();
+      }
+      int pc = 0, code = code_reg[0], imm = imm_reg[0];
+      for (;;) {
+        int step;
+        if constexpr (AHEAD && DEPTH > 1)
+          asm volatile(EW_INTERPRETER : "={s50}"(step), "+{s51}"(pc), "+{v[16:23]}"(top), "+{v[24:31]}"(s0), "+{v[32:39]}"(x), "+{v[64:71]}"(s1), "+{v[72:79]}"(s2),
+                       "+{v[80:87]}"(s3), "+{v[88:95]}"(s4) : "{v12}"(code), "{v13}"(imm), "{v14}"(row_a), "{v15}"(row_b), "{v[40:47]}"(col0), "{v[48:55]}"(col1),
+                       "{v[56:63]}"(walk2) : EW_CLOBBERS);
+        else if constexpr (AHEAD)
+          asm volatile(EW_INTERPRETER : "={s50}"(step), "+{s51}"(pc), "+{v[16:23]}"(top), "+{v[24:31]}"(s0), "+{v[32:39]}"(x) : "{v12}"(code), "{v13}"(imm),
+                       "{v14}"(row_a), "{v15}"(row_b), "{v[40:47]}"(col0), "{v[48:55]}"(col1), "{v[56:63]}"(walk2) : EW_CLOBBERS);
+        else if constexpr (DEPTH > 1)
+          asm volatile(EW_INTERPRETER : "={s50}"(step), "+{s51}"(pc), "+{v[16:23]}"(top), "+{v[24:31]}"(s0), "+{v[32:39]}"(x), "+{v[64:71]}"(s1), "+{v[72:79]}"(s2),
+                       "+{v[80:87]}"(s3), "+{v[88:95]}"(s4) : "{v12}"(code), "{v13}"(imm) : EW_CLOBBERS);
+        else
+          asm volatile(EW_INTERPRETER : "={s50}"(step), "+{s51}"(pc), "+{v[16:23]}"(top), "+{v[24:31]}"(s0), "+{v[32:39]}"(x) : "{v12}"(code), "{v13}"(imm) : EW_CLOBBERS);
+        const int what = step >> 24;
+        if (what == STEP_END) break;
+        if (what == STEP_FETCH) {
+          const int k = (step >> 8) & 15;
+          if (p.in_col_stride[k]) to_float(fetch_at(operand_at(k, p.in_dtype[k], true, here), p.in_dtype[k], false), p.in_dtype[k], x);
+          else x = v8f{} + row_value(k, fetch_row_at(operand_at(k, p.in_dtype[k], false, here), k));
+        } else if (what == STEP_MORE) {
+          code = code_reg[1];
+          imm = imm_reg[1];
+          pc = 0;
+        } else {
+  #pragma unroll
+          for (int e = 0; e < V; ++e) top[e] = top[e] / x[e];
+        }
+      }
+      if (live) store_group(out_at, out_dt, top, valid);
+      out_at += out_step;
+      if (!more) break;
+      rb = next_rb;
     }
-    if (!more) break;
-    if (next_slab != slab) fetch_cols(there, next_slab);
-    rb = next_rb;
-    slab = next_slab;
-    here = there;
   }
 }
 

@@ -75,3 +75,20 @@ def test_long_and_deep_programs_and_mixed_types(hip):
         for out in (O.F16, O.F32):
             for prog in (deep, long_, unfused):
                 run(hip, prog, ops, out, rows, cols)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt,rows,cols", [(O.F16, 4099, 2056), (O.F32, 4099, 2056), (O.BF16, 70001, 72), (O.F16, 70001, 71)])
+def test_lanes_that_walk_down_several_rows(hip, dt, rows, cols):
+    """more rows than the grid covers at once: two slabs of columns, and 16 lanes a row whose last row block is incomplete; operands held
+    ahead, fetched in place (more of a kind than there are slots) and mixed types"""
+    u = lambda n, t: O.uniform(n, 103, t, 0.5, 1.5)
+    other = O.F32 if dt != O.F32 else O.F16
+    ops = [(dt, "walk", u(rows * cols, 0)), (dt, "row", u(rows, 1)), (other, "row", u(rows, 2)), (dt, "row", u(rows, 3)), (dt, "col", u(cols, 4)), (dt, "col", u(cols, 5)),
+           (dt, "col", u(cols, 6)), (dt, "walk", u(rows * cols, 7))]
+    prog = [("input", 0)]
+    for k, op in zip((1, 4, 7, 2, 5, 3, 6), ("sub", "mul", "add", "max", "add", "min", "mul")):
+        prog += [("input", k), op]
+    run(hip, prog, ops, dt, rows, cols)
+    run(hip, prog, ops, dt, rows, cols, in_place=0)
+    run(hip, prog, [(other, "walk", u(rows * cols, 0))] + ops[1:], dt, rows, cols)
