@@ -190,6 +190,10 @@ __global__ void __launch_bounds__(C::NW * 64) attention_kernel(AttentionParams p
   // M phase of tile j: o += V_j^T P_j^T (unit u: key step u / DA, head_dim atom u % DA), then, if `scores`,
   // s = K_{j+1} Q^T (unit u: head_dim step u / KA, key atom u % KA).  Fragments are read two units ahead.
   auto m_phase = [&](unsigned vbase, unsigned kbase, bool scores) {
+    // the MFMAs of this wave go before the vector instructions of the wave it shares the SIMD with, which fill the slots between them
+    // (us without / with: f16 32 x 4096 x 4096 248.1 / 245.8, bf16 with K stored [128][seq_k] 237.8 / 232.2, f16 16 x 2048 x 2048 38.9 / 37.8; the
+    // softmax phase first instead: 250.8, 236.8, 39.9)
+    __builtin_amdgcn_s_setprio(1);
     unsigned ck[RK::NREG];
 #pragma unroll
     for (int r = 0; r < RK::NREG; ++r) ck[r] = rk[r] + kbase;
@@ -221,6 +225,7 @@ __global__ void __launch_bounds__(C::NW * 64) attention_kernel(AttentionParams p
         __builtin_amdgcn_sched_barrier(0);
       }
     }
+    __builtin_amdgcn_s_setprio(0);
   };
   // V phase: probabilities of the tile whose scores are in s.  Score e of the lane, e = 16 ka + r, belongs to
   // 16-key step e / 8.
