@@ -199,7 +199,7 @@ static void fill_layout(frisk_lds_layout* L, bool kcontig, int es, int fragb, in
 static int tail_split_of(const KernelEntry* k, int64_t tiles, int64_t kt, bool whole_k_tiles) {
   // the edge kernels deal any number of K tiles: their last slice may be shorter (us unsplit / split: bf16 3000x11008x4096 NT, 516
   // tiles, 248 / 212; fp16 4097x4097x4096 NT, 289 tiles, 161 / 126; 4095x4097x4001 NN with its copy to aligned rows 204 / 150)
-  const bool edge = k->edge && !k->splitk && (int64_t)k->bm * k->bn >= 256 * 256;
+  const bool edge = k->edge && !k->splitk && (int64_t)k->bm * k->bn >= 192 * 256;
   if (!edge && (!k->splitk || k->bm < 128 || k->wk > 1 || !whole_k_tiles)) return 1;
   if (tiles <= 256) return 1;
   const int64_t rest = tiles % 256;
@@ -257,6 +257,12 @@ static double estimated_cost(const KernelEntry* k, const frisk_gemm_desc* d, boo
     // 8-bit floats on the 16x16x128 atom (NT only), us against the 32x32x64 atoms: 8192^3 331 / 351, 4096^3 45.1 / 48.8, 4096x4096x512
     // 11.8 / 12.9, 4096x11008x4096 128 / 133, 6144^3 176 / 183; 3072^3 (144 tiles) 29.6 / 28.6
     if (k->atom == 16) c *= k->dtype == FRISK_E4M3 ? (tiles >= 176 ? 0.94 : 1.04) : (!k->transA && k->transB) ? 0.93 : (tiles >= 176 ? 0.96 : 0.98);
+  } else if (k->bm == 192) {
+    // three quarters of a 256x256 tile at 0.78 to 0.80 of its time.  us on 256x256 / 192x256 tiles: bf16 3000x4096x11008 NN (192 / 256
+    // tiles) 202.8 / 178.6, fp16 1999x4099x3001 NN 77.2 / 64.8, 2880x3840x2048 NT 47.8 / 38.3, 6720x5760x1024 NN 101 / 92, int8
+    // 3000x4096x4096 NN 54.8 / 43.1, 7296x4992x4096 NT 148 / 122, e4m3 the same two NT 52.3 / 42.8 and 142 / 124; where 256x256 tiles
+    // fill their rounds: fp16 3840x4096x8192 172 / 195, int8 89 / 117
+    c = k->dtype == FRISK_E4M3 ? 1.2 : 1.12;
   } else if (area >= 256 * 128) {
     c = 0.93;
   } else {
@@ -437,6 +443,9 @@ static double small_grid_cost(const KernelEntry* k, const frisk_gemm_desc* d, bo
   return t;
 }
 
+// edge kernels without a plain twin of the same tile
+static bool planners_own(const KernelEntry* k) { return k->edge && !k->splitk && k->bm == 192; }
+
 // What a launch knows beyond the descriptor: pointers off 16-byte boundaries (C: or a column-scale pointer off its vector), and
 // whether there is a workspace to use.
 struct PlanContext { bool a_off = false, b_off = false, c_off = false, no_workspace = false; };
@@ -505,6 +514,12 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
       // are left out where the plain twin fits)
       const bool whole_mn = d->M % k->bm == 0 && d->N % k->bn == 0;
       if (!k->guard && (!rows_aligned || d->K % k->bk || (k->edge ? whole_mn : !whole_mn))) continue;
+      // the 192x256 tile (an edge kernel without a plain twin) is the planner's own: a tile, wave grid, ring or atom that is asked for
+      // names the other variants
+      // (whole 256x256 tiles keep the default kernel: which one they run on is part of the planner's interface, though 144 of them
+      // leave CUs idle -- fp16 3072x3072x4096 NN 70.6 us, 62.4 on 192x256 tiles)
+      const bool whole_256 = rows_aligned && d->M % 256 == 0 && d->N % 256 == 0 && d->K % k->bk == 0;
+      if (planners_own(k) && (tile_requested || d->split_k > 1 || small || whole_256)) continue;
       // the edge kernels once more under their guarded names: K off the K tile (a whole number of chunks), and anything at all,
       // with A and B copied to aligned rows where theirs are not
       if (k->guard == 1 && k->edge && (!rows_aligned || d->K % (16 / es))) continue;
@@ -514,7 +529,8 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
       const double span_a = (double)(packed.a ? packed.lda : d->lda) * es * (d->transA ? k->bk : k->bm),
                    span_b = (double)(packed.b ? packed.ldb : d->ldb) * es * (d->transB ? k->bn : k->bk);
       if ((!k->guard || k->edge) && (span_a >= 4294967296.0 || span_b >= 4294967296.0)) continue;
-      if (k->guard && best >= 0 && !ks[best]->guard) continue;  // never a guarded kernel when a fast one fits
+      // never a guarded kernel when a fast one fits -- except those, which run at their full rate whatever their name
+      if (k->guard && !planners_own(k) && best >= 0 && !ks[best]->guard) continue;
       double cost = small && !want_split ? small_grid_cost(k, d, no_split) : estimated_cost(k, d, !want_split && !no_split && d->split_k == 0);
       // (a 32-row edge tile above 64 rows streams B once per 32 rows where the 64-row tile wastes at most as much: 130x11008x4096
       // NT 64.5 against 53.5 us)
@@ -527,7 +543,7 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
       }
       if (k->guard == 2) cost += repack_cost;
       // ties: the first listed variant is the tuned default
-      if (best < 0 || (ks[best]->guard && !k->guard) || cost < best_cost) { best = v.id; best_cost = cost; }
+      if (best < 0 || (ks[best]->guard && !k->guard && !planners_own(ks[best])) || cost < best_cost) { best = v.id; best_cost = cost; }
     }
   };
   // an explicit split_k looks among the variants with the split-K store path first; if none of them fits, the choice among

@@ -109,3 +109,17 @@ def test_tail_split_of_an_edge_kernel(hip, dtype, transA, transB, aligned):
     tiles = 16  # 17 x 16 tiles
     assert "256x256" in name and need >= 2 * tiles * 256 * 256 * 4, (name, need)
     verify(dtype, got, A, B, transA, transB)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [O.F16, O.BF16, O.I8, O.E4M3])
+@pytest.mark.parametrize("transB", [0, 1])
+def test_192_row_tiles(hip, dtype, transB):
+    """one to eight K tiles, whole and partial, M and N ending inside a tile, inside a wave's 96 rows and at their end"""
+    bk = BK[dtype]
+    for M, N, K in ((3001, 2999, bk - 24), (2976, 3072, 2 * bk + 1), (2881, 3080, 3 * bk), (2900, 2999, 3 * bk + 8), (2880, 3072, 8 * bk + 40)):
+        A = make_operand(dtype, *stored_shapes(M, N, K, 0, transB)[0], seed=86, tensor=0, scale=0.5)
+        B = make_operand(dtype, *stored_shapes(M, N, K, 0, transB)[1], seed=86, tensor=1, scale=0.5)
+        got, name, _ = launch(hip, dtype, A, B, M, N, K, 0, transB, True, ldc_extra=1)
+        assert "192x256" in name, (M, N, K, name)
+        verify(dtype, got, A, B, 0, transB)
