@@ -409,13 +409,16 @@ static double small_grid_time(const SmallGridModel& m, const KernelEntry* k, con
   const int64_t tiles = ((d->M + k->bm - 1) / k->bm) * ((d->N + k->bn - 1) / k->bn);
   const double kt = (double)((d->K + k->bk - 1) / k->bk) / split;
   const int64_t wgs = tiles * split, full = wgs / m.cap, rest = wgs % m.cap;
-  double t = m.launch, whole = kt * m.tk + m.ps, last = 0.0;
+  // one row of 64x128 tiles against a B stored [N][K] streams it 128 bytes of a row at a time: fp16 48x8192x8192 in 4 slices 37.0 us
+  // (64x32 tiles with K tiles four times as deep 28.7), 48x16384x8192 in 2 slices 64.3 (54.8)
+  const double tk = m.tk * (k->bm == 64 && k->bn == 128 && k->transB && tiles * k->bn < d->N + k->bn ? 1.4 : 1.0);
+  double t = m.launch, whole = kt * tk + m.ps, last = 0.0;
   if (m.cap == 512) {  // two work-groups per CU: the second one of any CU sets the pace of the round
     whole += kt * m.tk2;
     const double f1 = (double)std::min<int64_t>(rest, 256) / 256.0, f2 = (double)std::max<int64_t>(rest - 256, 0) / 256.0;
-    last = kt * (m.tk * (m.a + (1.0 - m.a) * f1) + (rest > 256 ? m.tk2 * (m.a2 + (1.0 - m.a2) * f2) : 0.0));
+    last = kt * (tk * (m.a + (1.0 - m.a) * f1) + (rest > 256 ? m.tk2 * (m.a2 + (1.0 - m.a2) * f2) : 0.0));
   } else {
-    last = kt * m.tk * (m.a + (1.0 - m.a) * (double)rest / m.cap);
+    last = kt * tk * (m.a + (1.0 - m.a) * (double)rest / m.cap);
   }
   t += (double)full * whole + (rest ? last : 0.0);
   if (split > 1) t += m.r0 + m.r1 * ((double)d->M * (double)d->N * split * 4.0 / 1e6);
@@ -443,8 +446,12 @@ static double small_grid_cost(const KernelEntry* k, const frisk_gemm_desc* d, bo
   return t;
 }
 
-// edge kernels without a plain twin of the same tile
-static bool planners_own(const KernelEntry* k) { return k->edge && !k->splitk && k->bm == 192; }
+// Edge kernels without a plain twin of the same tile: 192x256, and the tiles that stream B [N][K] for up to 64 rows, any number of rows
+// and any K.  Before those, rows off a multiple of 32 and K off 4 K tiles ran on 32x128 and 64x128 tiles, which fetch 128 bytes of a row of B
+// at a time, split along K.  us before / now, B from HBM: 17x8192x8192 fp16 45.9 / 24.6, int8 21.1 / 14.2, e4m3 20.5 / 13.8;
+// 48x8192x8192 37.4 / 29.5, 19.8 / 18.2, 19.4 / 17.7; 5x14336x4096 (448 tiles, ring of 2) 30.6 / 20.7, 18.5 / 13.0, 18.0 / 12.7; 24x16384x4224
+// (K a half K tile over) 33.6 / 27.8, 19.6 / 17.0, 19.1 / 16.9; 33x4096x2048 15.5 / 7.1, 7.2 / 6.8, 6.6 / 5.2; 40x11008x4096 fp16 28.5 / 28.7
+static bool planners_own(const KernelEntry* k) { return k->edge && !k->splitk && (k->bm == 192 || k->wk > 1); }
 
 // What a launch knows beyond the descriptor: pointers off 16-byte boundaries (C: or a column-scale pointer off its vector), and
 // whether there is a workspace to use.
@@ -514,12 +521,12 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
       // are left out where the plain twin fits)
       const bool whole_mn = d->M % k->bm == 0 && d->N % k->bn == 0;
       if (!k->guard && (!rows_aligned || d->K % k->bk || (k->edge ? whole_mn : !whole_mn))) continue;
-      // the 192x256 tile (an edge kernel without a plain twin) is the planner's own: a tile, wave grid, ring or atom that is asked for
-      // names the other variants
+      // the 192x256 tile and the unsplit tiles that stream B (edge kernels without a plain twin) are the planner's own: a tile, wave grid,
+      // ring or atom that is asked for names the other variants
       // (whole 256x256 tiles keep the default kernel: which one they run on is part of the planner's interface, though 144 of them
       // leave CUs idle -- fp16 3072x3072x4096 NN 70.6 us, 62.4 on 192x256 tiles)
       const bool whole_256 = rows_aligned && d->M % 256 == 0 && d->N % 256 == 0 && d->K % k->bk == 0;
-      if (planners_own(k) && (tile_requested || d->split_k > 1 || small || whole_256)) continue;
+      if (planners_own(k) && (tile_requested || d->split_k > 1 || (k->bm == 192 ? small || whole_256 : d->M > 64))) continue;
       // the edge kernels once more under their guarded names: K off the K tile (a whole number of chunks), and anything at all,
       // with A and B copied to aligned rows where theirs are not
       if (k->guard == 1 && k->edge && (!rows_aligned || d->K % (16 / es))) continue;
@@ -535,7 +542,8 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
       // (a 32-row edge tile above 64 rows streams B once per 32 rows where the 64-row tile wastes at most as much: 130x11008x4096
       // NT 64.5 against 53.5 us)
       if (k->edge && k->bm == 32 && d->M > 64 && !d->tile_m) continue;
-      if (k->edge) {
+      if (k->edge || k->guard) {
+        // (the kernels staged through registers too: one row on a 128-row tile is not a 128th of its price)
         // the models see whole tiles; rows and columns beyond M and N are work all the same (a 64-row tile on 32 rows is no
         // better than the 32-row tile that fits): the square root of the covered area over M x N, as a penalty
         const double covered = (double)((d->M + k->bm - 1) / k->bm * k->bm) * (double)((d->N + k->bn - 1) / k->bn * k->bn);

@@ -76,6 +76,11 @@ def square(bk, atom16=False, skinny_ta=(0,)):
     # 128x64 tile with K tiles twice as deep, 128x16384x4096 35.2 against 39.6 (vendor 36.0), 128x4096x16384 40.5 against 42.8
     out.append((0, 1, 64, 32, 4 * bk, 1, 1, 3, 0, 1, 4))
     out.append((0, 1, 128, 64, 2 * bk, 2, 2, 3, 0, 1, 1))
+    # ... and the three streaming kernels, unsplit, for any number of rows and any K: see planners_own in capi.cpp for what they replaced.
+    # (B stored [K][N] in 32 columns, 64 bytes of a row at a time, is no good: 48x8192x8192 52 us, on 64x128 tiles in 4 slices 33)
+    out.append(edge((0, 1, 32, 32, 4 * bk, 1, 1, 4, 0, 0, 4)))
+    out.append(edge((0, 1, 32, 32, 4 * bk, 1, 1, 2, 0, 0, 4)))
+    out.append(edge((0, 1, 64, 32, 4 * bk, 1, 1, 3, 0, 0, 4)))
     # M and N that are not multiples of the tile (K a multiple of the K tile, rows and pointers on 16-byte boundaries): the default
     # 256x256 variant and the 128x128 one with 2 + 2 tiles once more with clamped lane offsets and checked stores.  (fp16
     # 4000x4096x4096 ran 539 us on 32-row tiles and 4096x4000x4096 933 us on the guarded kernel, the vendor library 110 and 125.)

@@ -113,6 +113,25 @@ def test_tail_split_of_an_edge_kernel(hip, dtype, transA, transB, aligned):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [O.F16, O.BF16, O.I8, O.E4M3])
+@pytest.mark.parametrize("M", [1, 17, 33, 63])
+def test_tiles_that_stream_b_take_any_rows_and_any_k(hip, dtype, M):
+    """32x32 and 64x32 tiles whose waves split K: one to seven K tiles (every path through the prologue and the drain), whole and partial,
+    every work-group starting its walk over the whole ones at another of them; N ending inside a tile and inside a chunk"""
+    bk, names = 4 * BK[dtype], set()
+    cases = [(1040, bk - 56), (1037, bk + 7), (2056, 2 * bk - 24), (2056, 3 * bk), (4104, 3 * bk + 48), (4101, 4 * bk - 40), (4104, 6 * bk + 8)]
+    cases += [(8328, bk), (8328, 2 * bk + 8), (8328, 4 * bk - 8)] if M <= 32 else []  # more than 256 tiles: the ring of 2
+    for N, K in cases:
+        A = make_operand(dtype, M, K, seed=85, tensor=0, scale=0.5)
+        B = make_operand(dtype, N, K, seed=85, tensor=1, scale=0.5)
+        got, name, _ = launch(hip, dtype, A, B, M, N, K, 0, 1, True, ldc_extra=1)
+        names |= {name.split("_")[2], "s2" if "_s2" in name else "s4" if "_s4" in name else "s3"}
+        verify(dtype, got, A, B, 0, 1)
+    assert names >= ({"32x32x%d" % bk, "s2", "s4"} if M <= 32 else {"32x32x%d" % bk, "64x32x%d" % bk}), names
+    assert names <= {"32x32x%d" % bk, "64x32x%d" % bk, "s2", "s3", "s4"}, names
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [O.F16, O.BF16, O.I8, O.E4M3])
 @pytest.mark.parametrize("transB", [0, 1])
 def test_192_row_tiles(hip, dtype, transB):
     """one to eight K tiles, whole and partial, M and N ending inside a tile, inside a wave's 96 rows and at their end"""
