@@ -208,7 +208,7 @@ static int tail_split_of(const KernelEntry* k, int64_t tiles, int64_t kt, bool w
   // time, so the summing pass weighs twice as much against their slices (fp8 5120x4096x4096: 64 tiles in 4 slices of 8 K tiles
   // 92.4 us, unsplit 84, 256x128 tiles 81.4)
   const int min_slice = elem_size(k->dtype) == 1 ? 16 : 8;
-  for (int s = 8; s >= 2; s /= 2) {
+  for (int s = 8; s >= 2; s = edge ? s - 1 : s / 2) {
     const int64_t per = (kt + s - 1) / s;
     if (rest * s <= 256 && (edge ? (s - 1) * per < kt : kt % s == 0) && per >= min_slice) return s;
   }
@@ -223,8 +223,8 @@ static int tail_split_of(const KernelEntry* k, int64_t tiles, int64_t kt, bool w
 // at least 4 K tiles per slice
 static int sub_round_split(const KernelEntry* k, int64_t tiles, int64_t kt) {
   int split = 1;
-  for (int c = 2; c <= 64; c *= 2)
-    if (kt % c == 0 && kt / c >= std::max(4, k->min_k_tiles) && tiles * c <= 256) split = c;
+  for (int c = 2; c <= 64 && tiles * c <= 256; ++c)
+    if (kt % c == 0 && kt / c >= std::max(4, k->min_k_tiles)) split = c;
   return split;
 }
 
@@ -431,8 +431,11 @@ static int small_grid_split(const KernelEntry* k, const frisk_gemm_desc* d, bool
   double best_t = small_grid_time(m, k, d, 1);
   if (k->splitk && !no_split && d->split_k != 1 && m.w != 0 && d->K % k->bk == 0) {
     const int64_t tiles = ((d->M + k->bm - 1) / k->bm) * ((d->N + k->bn - 1) / k->bn), kt = d->K / k->bk;
-    for (int c = 2; c <= (k->dtype == FRISK_F32 ? 32 : 64); c *= 2)  // the sweeps behind the tables: fp32 up to 32 slices
-      if (tiles * c <= m.w && kt % c == 0 && kt / c >= std::max(m.kmin, k->min_k_tiles)) {
+    // any divisor of the K tiles (K = 5760 is 45 tiles of 128: the powers of two left it unsplit); the sweeps behind the tables: up to 64
+    // slices, fp32 32
+    const int64_t most = std::min<int64_t>({k->dtype == FRISK_F32 ? 32 : 64, tiles > 0 ? m.w / tiles : 0, kt / std::max(m.kmin, k->min_k_tiles)});
+    for (int c = 2; c <= most; ++c)
+      if (kt % c == 0) {
         const double t = small_grid_time(m, k, d, c);
         if (t < best_t) { best = c; best_t = t; }
       }
