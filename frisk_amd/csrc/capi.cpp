@@ -215,6 +215,24 @@ static int tail_split_of(const KernelEntry* k, int64_t tiles, int64_t kt, bool w
   return 1;
 }
 
+// The same for edge kernels on grids of at most half a round, whose tiles are then all split: the most slices that leave one work-group
+// per CU and enough K tiles to each (any K, unequal slices: what the split-K kernels do for whole tiles).  us unsplit / split:
+// fp16 1589x3072x9600 NN 114 / 91, 2100x2100x8000 TN 130 / 103, 1500x2816x11008 NN 131 / 90, 1001x1003x4001 NN 56.5 / 31.3, 1000x1000x4000 NT
+// 45.0 / 24.9, 600x4100x4100 TN 59.9 / 54.4, bf16 704x960x4032 TN 39.6 / 20.8, 17x4096x4096 TN 52.7 / 18.9, int8 576x1088x8064 TN 46.1 / 25.2,
+// e4m3 704x512x5760 TT 32.8 / 23.5
+static bool edge_slices_ok(const KernelEntry* k, const frisk_gemm_desc* d, int slices) {
+  const int64_t kt = (d->K + k->bk - 1) / k->bk, per = (kt + slices - 1) / slices;
+  return per >= (elem_size(k->dtype) == 1 ? 16 : 8) && (slices - 1) * per < kt;
+}
+static int edge_split_of(const KernelEntry* k, const frisk_gemm_desc* d) {
+  if (!k->edge || k->splitk || k->wk > 1 || k->bm < 128 || k->dtype == FRISK_F32) return 1;
+  const int64_t tiles = ((d->M + k->bm - 1) / k->bm) * ((d->N + k->bn - 1) / k->bn);
+  if (tiles > 128 || tiles == 0) return 1;
+  for (int s = (int)std::min<int64_t>(8, 256 / tiles); s >= 2; --s)
+    if (edge_slices_ok(k, d, s)) return s;
+  return 1;
+}
+
 // Relative time of a problem on a kernel variant, used only to rank the variants.  One wave of work-groups = one per CU
 // (256); a K tile of a 256x256 tile costs 1.5 units when every CU runs one, and less when the chip is partly idle
 // (less contention in the L2 and a higher clock): factor 0.6 + 0.4 * fill.  The constants are measured on fp16 problems
@@ -287,6 +305,8 @@ static double estimated_cost(const KernelEntry* k, const frisk_gemm_desc* d, boo
     // 1024x8192x8192 comes out even with 256x128 tiles unsplit, 123.7 against 123.9 us, and stays unsplit)
     if (cs > 1) return kt / cs * c * (0.6 + 0.4 * rest_fill * cs) * 1.08 + 5.0 + 0.07 * (double)(tiles * cs);
   }
+  if (const int cs = may_split && tiles <= 128 ? edge_split_of(k, d) : 1; cs > 1)
+    return kt / cs * c * (0.6 + 0.4 * rest_fill * cs) * 1.08 + 5.0 + 0.07 * (double)(tiles * cs) * (double)area / (256 * 256);
   double cost = (double)full * kt * c;
   if (const int ts = (k->edge && !k->splitk && !may_split) ? 1 : tail_split_of(k, tiles, (int64_t)kt, d->K % k->bk == 0); ts > 1) {
     // the last `rest` tiles as ts work-groups each, a ts-th of the K tiles apiece, plus the pass that sums them
@@ -424,8 +444,9 @@ static double small_grid_time(const SmallGridModel& m, const KernelEntry* k, con
   if (split > 1) t += m.r0 + m.r1 * ((double)d->M * (double)d->N * split * 4.0 / 1e6);
   return k->guard && !k->edge ? kStagedFactor * t : t;
 }
-// the split of a variant: among the powers of two the rule admits, the one the model makes fastest; *cost receives its time
-static int small_grid_split(const KernelEntry* k, const frisk_gemm_desc* d, bool no_split, double* cost = nullptr) {
+// the split of a variant: among those the rule admits, the one the model makes fastest; *cost receives its time.  `edges`: edge kernels may
+// be split too
+static int small_grid_split(const KernelEntry* k, const frisk_gemm_desc* d, bool no_split, bool edges, double* cost = nullptr) {
   const SmallGridModel& m = small_grid_model(k);
   int best = 1;
   double best_t = small_grid_time(m, k, d, 1);
@@ -440,12 +461,19 @@ static int small_grid_split(const KernelEntry* k, const frisk_gemm_desc* d, bool
         if (t < best_t) { best = c; best_t = t; }
       }
   }
+  // the edge kernels: slices of unequal length, whole tiles of partial sums
+  if (const int most = edges ? edge_split_of(k, d) : 1; most > 1)
+    for (int c = 2; c <= most; ++c)
+      if (edge_slices_ok(k, d, c)) {
+        const double t = small_grid_time(m, k, d, c);
+        if (t < best_t) { best = c; best_t = t; }
+      }
   if (cost) *cost = best_t;
   return best;
 }
-static double small_grid_cost(const KernelEntry* k, const frisk_gemm_desc* d, bool no_split) {
+static double small_grid_cost(const KernelEntry* k, const frisk_gemm_desc* d, bool no_split, bool edges) {
   double t = 0.0;
-  small_grid_split(k, d, no_split, &t);
+  small_grid_split(k, d, no_split, edges, &t);
   return t;
 }
 
@@ -504,6 +532,7 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
   bool policy_excluded = false;
   const bool any_layout = !list.empty(), tile_requested = d->tile_m || d->tile_n || d->tile_k || d->waves_m || d->waves_n || d->stages || d->atom;
   const bool small = small_grid(d);
+  bool split_edges = false;
   auto search = [&](bool want_split) {
     for (const Variant& v : list) {
       const KernelEntry* k = v.k;
@@ -541,7 +570,7 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
       if ((!k->guard || k->edge) && (span_a >= 4294967296.0 || span_b >= 4294967296.0)) continue;
       // never a guarded kernel when a fast one fits -- except those, which run at their full rate whatever their name
       if (k->guard && !planners_own(k) && best >= 0 && !ks[best]->guard) continue;
-      double cost = small && !want_split ? small_grid_cost(k, d, no_split) : estimated_cost(k, d, !want_split && !no_split && d->split_k == 0);
+      double cost = small && !want_split ? small_grid_cost(k, d, no_split, split_edges) : estimated_cost(k, d, !want_split && !no_split && d->split_k == 0);
       // (a 32-row edge tile above 64 rows streams B once per 32 rows where the 64-row tile wastes at most as much: 130x11008x4096
       // NT 64.5 against 53.5 us)
       if (k->edge && k->bm == 32 && d->M > 64 && !d->tile_m) continue;
@@ -562,6 +591,12 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
   const bool explicit_split = d->split_k > 1 && !no_split;
   search(explicit_split);
   if (best < 0 && explicit_split) search(false);
+  // A small grid that falls to a kernel without the split-K store path looks at split edge kernels as well.  (The sweeps behind the tables held none, and beside the
+  // split-K kernels the tables flatter them: fp16 100x4096x4096 NN 20.6 us so, 16.8 on 64x128 tiles in 4 slices.)
+  if (small && best >= 0 && !no_split && d->split_k == 0 && !ks[best]->splitk && small_grid_split(ks[best], d, no_split, false) == 1) {
+    split_edges = true;
+    search(false);
+  }
   if (d->M == 0 || d->N == 0) {  // nothing to compute
     plan->grid_x = plan->grid_y = 0;
     return FRISK_OK;
@@ -602,10 +637,13 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
   }
   if (k->edge && !k->splitk && !no_split && d->split_k == 0) {
     const int64_t edge_tiles = (int64_t)plan->grid_x * plan->grid_y;
-    if (const int ts = tail_split_of(k, edge_tiles, (d->K + k->bk - 1) / k->bk, false); ts > 1) {
+    const bool half_round = edge_tiles <= 128;
+    const int ts = !half_round ? tail_split_of(k, edge_tiles, (d->K + k->bk - 1) / k->bk, false) : small ? small_grid_split(k, d, no_split, split_edges) : edge_split_of(k, d);
+    if (ts > 1) {
+      const int64_t split_tiles = half_round ? edge_tiles : edge_tiles % 256;
       const size_t offset = (plan->workspace_bytes + 255) & ~(size_t)255;
-      plan->workspace_bytes = offset + (size_t)ts * (size_t)(edge_tiles % 256) * (size_t)k->bm * (size_t)k->bn * 4;
-      if (extras) { extras->tail_split = ts; extras->tail_tiles = (int)(edge_tiles % 256); extras->partial_offset = offset; }
+      plan->workspace_bytes = offset + (size_t)ts * (size_t)split_tiles * (size_t)k->bm * (size_t)k->bn * 4;
+      if (extras) { extras->tail_split = ts; extras->tail_tiles = (int)split_tiles; extras->partial_offset = offset; }
     }
   }
   // Split K over the grid's y dimension when the tile grid alone leaves most CUs idle (skinny problems are
@@ -619,7 +657,7 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
         return fail(FRISK_ERR_TILE, "split_k=%d leaves %lld K tiles per slice, the chosen kernel %s needs %d", d->split_k, (long long)(kt / d->split_k), k->name, k->min_k_tiles);
       split = d->split_k;
     } else if (small) {
-      split = small_grid_split(k, d, no_split);
+      split = small_grid_split(k, d, no_split, false);
     } else if (d->split_k == 0 && tiles < 256) {
       split = sub_round_split(k, tiles, kt);
     } else if (d->split_k == 0) {

@@ -142,3 +142,27 @@ def test_192_row_tiles(hip, dtype, transB):
         got, name, _ = launch(hip, dtype, A, B, M, N, K, 0, transB, True, ldc_extra=1)
         assert "192x256" in name, (M, N, K, name)
         verify(dtype, got, A, B, 0, transB)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,transA,transB,aligned,size", [
+    (O.F16, 0, 0, True, (1001, 1003, 4001)),   # 64 tiles of 128 x 128 in 4 slices
+    (O.BF16, 1, 0, True, (17, 4096, 4096)),    # one row of tiles in 8 slices
+    (O.I8, 1, 0, True, (300, 1088, 130 * 48 + 5)),  # 49 K tiles: 3 slices, the last one shorter and its last K tile partial
+    (O.E4M3, 1, 1, True, (704, 512, 5760)),
+    (O.F16, 0, 1, False, (1000, 1000, 4000 - 9)),   # behind the copies of both operands
+    (O.F16, 0, 1, True, (2500, 1664, 4040)),   # 70 tiles of 256 x 256 in 3 slices
+    (O.F16, 0, 0, True, (1500, 2816, 3016)),   # 88 tiles of 192 x 256 in 2
+])
+def test_edge_kernels_split_on_grids_of_half_a_round(hip, dtype, transA, transB, aligned, size):
+    """every tile of the grid in slices of K of unequal length, and the same problem with no workspace in one pass"""
+    M, N, K = size
+    A = make_operand(dtype, *stored_shapes(M, N, K, transA, transB)[0], seed=87, tensor=0, scale=0.5)
+    B = make_operand(dtype, *stored_shapes(M, N, K, transA, transB)[1], seed=87, tensor=1, scale=0.5)
+    for workspace in (True, False):
+        got, name, need = launch(hip, dtype, A, B, M, N, K, transA, transB, aligned, workspace=workspace, ldc_extra=1)
+        if workspace:
+            bm, bn = map(int, name.split("_")[2].split("x")[:2])
+            tiles = -(-M // bm) * -(-N // bn)
+            assert bm >= 128 and tiles <= 128 and need >= 2 * tiles * bm * bn * 4, (name, need)
+        verify(dtype, got, A, B, transA, transB)
