@@ -454,7 +454,12 @@ static int small_grid_split(const KernelEntry* k, const frisk_gemm_desc* d, bool
     const int64_t tiles = ((d->M + k->bm - 1) / k->bm) * ((d->N + k->bn - 1) / k->bn), kt = d->K / k->bk;
     // any divisor of the K tiles (K = 5760 is 45 tiles of 128: the powers of two left it unsplit); the sweeps behind the tables: up to 64
     // slices, fp32 32
-    const int64_t most = std::min<int64_t>({k->dtype == FRISK_F32 ? 32 : 64, tiles > 0 ? m.w / tiles : 0, kt / std::max(m.kmin, k->min_k_tiles)});
+    // At least 4 K tiles a slice and up to 256 work-groups, whatever range of splits a class was fitted over (`kmin`, `w`; B stored [N][K]
+    // keeps its `w`: there the unsplit tiles that stream B are as good): the model holds beyond it.  us at 16 K tiles and 128 or 256 work-groups / now: int8
+    // 40x2880x7040 NN 29.5 / 12.8, e4m3 59x7104x4608 21.7 / 14.2, fp16 37x6720x3328 23.7 / 14.5, 16x2496x4224 14.7 / 11.3, 276x1280x3520 17.5 / 12.4;
+    // 70 drawn sizes whose split changed 1.27 times faster, the worst 0.94 (3x9536x5760).  512 work-groups: 0.96 on 45.
+    const int64_t wgs = k->transB ? m.w : std::max(m.w, 256);
+    const int64_t most = std::min<int64_t>({k->dtype == FRISK_F32 ? 32 : 64, tiles > 0 ? wgs / tiles : 0, kt / std::max(std::min(m.kmin, 4), k->min_k_tiles)});
     for (int c = 2; c <= most; ++c)
       if (kt % c == 0) {
         const double t = small_grid_time(m, k, d, c);
