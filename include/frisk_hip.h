@@ -127,7 +127,7 @@ typedef struct frisk_gemm_plan {
   int32_t grid_x, grid_y;            /* work-group grid (tiles along N, tiles along M) */
   int32_t split_k;                   /* >1: partial sums go through the workspace */
   int32_t xcd_remap;                 /* 1: work-group ids are remapped so each XCD owns a compact block of tiles */
-  int32_t guarded;                   /* 1: K off the K tile, or unaligned rows or pointers */
+  int32_t guarded;                   /* 1: K off the K tile, unaligned rows or pointers, or a tile that only exists as such a kernel */
   frisk_lds_layout lds_a, lds_b;
   size_t workspace_bytes;
   double flops;                      /* 2.M.N.K */
@@ -151,7 +151,7 @@ const char* frisk_hip_last_error(void);
 int frisk_hip_plan(const frisk_gemm_desc* desc, frisk_gemm_plan* plan);
 
 /* Pure host: bytes of device workspace `frisk_hip_gemm` wants for this descriptor: split_k * M * N * 4 when the
- * plan splits K, tail_split * tail_tiles * tile_m * tile_n * 4 for a tail split, the size of the operands with padded rows
+ * plan splits K, tail_split * tail_tiles * tile_m * tile_n * 4 for a tail split (the same per slice and tile for split kernels off the tiles), the size of the operands with padded rows
  * where they are copied, else 0.  With split_k = 0 in the descriptor a launch without workspace still runs, unsplit. */
 size_t frisk_hip_workspace_bytes(const frisk_gemm_desc* desc);
 
