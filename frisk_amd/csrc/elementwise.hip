@@ -9,10 +9,10 @@
 // assembly over fixed registers: a step is two lane reads of the program, a jump to its handler and 8 vector instructions in
 // place, the operand picked by the register index mode.  (As a C++ switch the compiler joins the values of all cases after every
 // step by register moves: 327 vector, 300 scalar and 120 branch instructions per group of 8 columns for (x - s * c) * g + b; here
-// 109, 125 and 34.)  That body on 8192 x 8192 f16: 139 us before, 54 now (a plain copy: 41); log2(max(x, c) / (x + c)), bound by
+// 109, 125 and 34.)  That body on 8192 x 8192 f16: 139 us before, 51 now (a plain copy: 41); log2(max(x, c) / (x + c)), bound by
 // the vector pipe in its division, 125 -> 71.5; rows off 16-byte boundaries (4095 x 8191) 370 -> 51.
 // Operands that are the same for every row stay in registers while the lane's columns do, values of one per row stay one
-// register, and what the next group needs from memory is fetched while the current one is evaluated.  All arithmetic is
+// register, and what the next groups need from memory is fetched while the current one is evaluated.  All arithmetic is
 // fp32; the result is rounded once to the output type.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -185,15 +185,17 @@ template <int DT, bool AHEAD, int DEPTH, bool UNIFORM_ROW> __global__ void __lau
 #pragma unroll
   for (int c = 0; c < 2; ++c) { code_reg[c] = prog.code[c * kChunk + (threadIdx.x & 63)]; imm_reg[c] = __builtin_bit_cast(int, prog.imm[c * kChunk + (threadIdx.x & 63)]); }
   auto type_of = [&](int k) { return DT >= 0 ? DT : p.in_dtype[k]; };
-  auto row_value = [&](int k, unsigned bits) {
-    if (p.in_dtype[k] == FRISK_F32) return __builtin_bit_cast(float, bits);
-    if (p.in_dtype[k] == FRISK_F16) return (float)__builtin_bit_cast(_Float16, (uint16_t)bits);
+  auto row_value = [&](int dt, unsigned bits) {
+    if (dt == FRISK_F32) return __builtin_bit_cast(float, bits);
+    if (dt == FRISK_F16) return (float)__builtin_bit_cast(_Float16, (uint16_t)bits);
     return __builtin_bit_cast(float, bits << 16);
   };
+  // (named once: an operand's type read from the arguments by its number is a scalar load and a wait in every group)
+  const int row0_dt = AHEAD && prog.row0 >= 0 ? p.in_dtype[prog.row0] : FRISK_F32, row1_dt = AHEAD && prog.row1 >= 0 ? p.in_dtype[prog.row1] : FRISK_F32;
   const int64_t rb0 = blockIdx.y, row_stride = (int64_t)gridDim.y * row_step;  // rows between this lane's groups
   if (rb0 >= row_blocks) return;
   // A lane keeps its columns and walks down the rows, every operand's address moving on by one stride: worked out anew for every
-  // group, place and addresses made the counts above 136, 171 and 35, and 62.7 us of the 54 (a SIMD issues one scalar instruction in
+  // group, place and addresses made the counts above 136, 171 and 35 (203.8 us instead of 195.2 for cast, mean, that body and softmax; a SIMD issues one scalar instruction in
   // four cycles, so they weigh as much as the vector ones).
   for (int64_t slab = blockIdx.x; slab < slabs; slab += gridDim.x) {
     // lanes beyond the view repeat its last row or group and store nothing
@@ -213,57 +215,70 @@ template <int DT, bool AHEAD, int DEPTH, bool UNIFORM_ROW> __global__ void __lau
       if (!ragged || valid >= V) return load_raw(at, dt, streamed);
       return load_raw_partial(at, dt, valid);
     };
-    auto fetch_row_at = [&](const char* at, int k) { return p.in_dtype[k] == FRISK_F32 ? *(const unsigned*)at : (unsigned)*(const uint16_t*)at; };
+    auto fetch_row_at = [&](const char* at, int dt) { return dt == FRISK_F32 ? *(const unsigned*)at : (unsigned)*(const uint16_t*)at; };
     auto stride_of = [&](int k, int dt) { return row_stride * p.in_row_stride[k] * (dt == FRISK_F32 ? 4 : 2); };
     const char *head_at = nullptr, *walk2_at = nullptr, *row0_at = nullptr, *row1_at = nullptr;
     int64_t head_step = 0, walk2_step = 0, row0_step = 0, row1_step = 0;
     if (prog.head >= 0) { head_at = operand_at(prog.head, type_of(prog.head), true, row_in); head_step = stride_of(prog.head, type_of(prog.head)); }
     if constexpr (AHEAD) {
       if (prog.walk2 >= 0) { walk2_at = operand_at(prog.walk2, type_of(prog.walk2), true, row_in); walk2_step = stride_of(prog.walk2, type_of(prog.walk2)); }
-      if (prog.row0 >= 0) { row0_at = operand_at(prog.row0, p.in_dtype[prog.row0], false, row_in); row0_step = stride_of(prog.row0, p.in_dtype[prog.row0]); }
-      if (prog.row1 >= 0) { row1_at = operand_at(prog.row1, p.in_dtype[prog.row1], false, row_in); row1_step = stride_of(prog.row1, p.in_dtype[prog.row1]); }
+      if (prog.row0 >= 0) { row0_at = operand_at(prog.row0, row0_dt, false, row_in); row0_step = stride_of(prog.row0, row0_dt); }
+      if (prog.row1 >= 0) { row1_at = operand_at(prog.row1, row1_dt, false, row_in); row1_step = stride_of(prog.row1, row1_dt); }
     }
     const int out_dt = DT >= 0 ? DT : p.out_dtype, out_es = out_dt == FRISK_F32 ? 4 : 2;
     char* out_at = (char*)p.out + row_in * (p.out_ld * out_es) + (slab << lanes_log2) * (V * out_es) + (unsigned)(off * (V * out_es));
     const int64_t out_step = row_stride * p.out_ld * out_es;
 
-    Raw ahead{}, ahead2{};
-    unsigned row0 = 0, row1 = 0;
+    // what is under way from memory: the next group of 32-bit operands, the next two of 16-bit ones (16 bytes a lane and four waves a SIMD
+    // are a third of what the memory's latency asks for: one group ahead 195.2 us for the four calls of cast, mean, scale and shift, softmax on 8192 x 8192 f16, two 191.8)
+    constexpr int SETS = (DT == FRISK_F16 || DT == FRISK_BF16) && DEPTH == 1 && UNIFORM_ROW ? 2 : 1;
+    struct Held { Raw head, walk2; unsigned row0, row1; } held0{}, held1{};
     v8f col0{}, col1{};
-    auto fetch_ahead = [&]() {
-      if (prog.head >= 0) ahead = fetch_at(head_at, type_of(prog.head), true);
+    auto fetch_ahead = [&](Held& h) __attribute__((always_inline)) {
+      if (prog.head >= 0) h.head = fetch_at(head_at, type_of(prog.head), true);
       if constexpr (AHEAD) {
-        if (prog.walk2 >= 0) ahead2 = fetch_at(walk2_at, type_of(prog.walk2), true);
-        if (prog.row0 >= 0) row0 = fetch_row_at(row0_at, prog.row0);
-        if (prog.row1 >= 0) row1 = fetch_row_at(row1_at, prog.row1);
+        if (prog.walk2 >= 0) h.walk2 = fetch_at(walk2_at, type_of(prog.walk2), true);
+        if (prog.row0 >= 0) h.row0 = fetch_row_at(row0_at, row0_dt);
+        if (prog.row1 >= 0) h.row1 = fetch_row_at(row1_at, row1_dt);
       }
     };
-    fetch_ahead();
+    int64_t fetched = row;  // row of the last fetch
+    auto next_row = [&]() __attribute__((always_inline)) {
+      fetched += row_stride;
+      if (fetched < p.rows) {  // (a lane whose next row lies beyond the view fetches the present one again)
+        head_at += head_step;
+        if constexpr (AHEAD) { walk2_at += walk2_step; row0_at += row0_step; row1_at += row1_step; }
+      }
+    };
+    fetch_ahead(held0);
+    if constexpr (SETS == 2) {
+      if (rb0 + gridDim.y < row_blocks) {
+        next_row();
+        fetch_ahead(held1);
+      }
+    }
     if constexpr (AHEAD) {
       if (prog.col0 >= 0) to_float(fetch_at(operand_at(prog.col0, p.in_dtype[prog.col0], true, 0), p.in_dtype[prog.col0], false), p.in_dtype[prog.col0], col0);
       if (prog.col1 >= 0) to_float(fetch_at(operand_at(prog.col1, p.in_dtype[prog.col1], true, 0), p.in_dtype[prog.col1], false), p.in_dtype[prog.col1], col1);
     }
-    for (int64_t rb = rb0;;) {
-      const int64_t next_rb = rb + gridDim.y;
-      const bool more = next_rb < row_blocks, live = row < p.rows && lane_group < left;
+    int64_t rb = rb0;
+    // one group, whose operands are in h; true: it was the last one
+    auto group = [&](Held& h) __attribute__((always_inline)) {
+      const bool live = row < p.rows && lane_group < left;
       v8f top, s0, s1, s2, s3, s4, x, walk2;
       asm volatile("" : "=v"(top), "=v"(s0), "=v"(x), "=v"(walk2));  // written by the program before it reads them
       if constexpr (DEPTH > 1) asm volatile("" : "=v"(s1), "=v"(s2), "=v"(s3), "=v"(s4));
       float row_a = 0.f, row_b = 0.f;
-      if (prog.head >= 0) to_float(ahead, type_of(prog.head), top);
+      if (prog.head >= 0) to_float(h.head, type_of(prog.head), top);
       if constexpr (AHEAD) {
-        if (prog.walk2 >= 0) to_float(ahead2, type_of(prog.walk2), walk2);
-        if (prog.row0 >= 0) row_a = row_value(prog.row0, row0);
-        if (prog.row1 >= 0) row_b = row_value(prog.row1, row1);
+        if (prog.walk2 >= 0) to_float(h.walk2, type_of(prog.walk2), walk2);
+        if (prog.row0 >= 0) row_a = row_value(row0_dt, h.row0);
+        if (prog.row1 >= 0) row_b = row_value(row1_dt, h.row1);
       }
       const int64_t here = row < p.rows ? row : p.rows - 1;
-      if (more) {
-        row += row_stride;
-        if (row < p.rows) {  // (a lane whose next row lies beyond the view fetches the present one again)
-          head_at += head_step;
-          if constexpr (AHEAD) { walk2_at += walk2_step; row0_at += row0_step; row1_at += row1_step; }
-        }
-        fetch_ahead();
+      if (rb + SETS * (int64_t)gridDim.y < row_blocks) {
+        next_row();
+        fetch_ahead(h);
       }
       int pc = 0, code = code_reg[0], imm = imm_reg[0];
       for (;;) {
@@ -285,7 +300,7 @@ template <int DT, bool AHEAD, int DEPTH, bool UNIFORM_ROW> __global__ void __lau
         if (what == STEP_FETCH) {
           const int k = (step >> 8) & 15;
           if (p.in_col_stride[k]) to_float(fetch_at(operand_at(k, p.in_dtype[k], true, here), p.in_dtype[k], false), p.in_dtype[k], x);
-          else x = v8f{} + row_value(k, fetch_row_at(operand_at(k, p.in_dtype[k], false, here), k));
+          else x = v8f{} + row_value(p.in_dtype[k], fetch_row_at(operand_at(k, p.in_dtype[k], false, here), p.in_dtype[k]));
         } else if (what == STEP_MORE) {
           code = code_reg[1];
           imm = imm_reg[1];
@@ -297,8 +312,13 @@ template <int DT, bool AHEAD, int DEPTH, bool UNIFORM_ROW> __global__ void __lau
       }
       if (live) store_group(out_at, out_dt, top, valid);
       out_at += out_step;
-      if (!more) break;
-      rb = next_rb;
+      row += row_stride;
+      rb += gridDim.y;
+      return rb >= row_blocks;
+    };
+    for (;;) {
+      if (group(held0)) break;
+      if constexpr (SETS == 2) { if (group(held1)) break; }
     }
   }
 }
