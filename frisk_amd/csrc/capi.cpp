@@ -758,15 +758,17 @@ int frisk_hip_gemm(const frisk_gemm_desc* desc, const void* A, const void* B, vo
   const uintptr_t es = (uintptr_t)elem_size(desc->dtype_ab), os = (uintptr_t)elem_size(desc->dtype_out);
   if (((uintptr_t)A | (uintptr_t)B) & (es - 1) || (uintptr_t)C & (os - 1) || (((uintptr_t)scaleA | (uintptr_t)scaleB) & 3))
     return fail(FRISK_ERR_ALIGNMENT, "pointers must be aligned to their element size");
-  if (plan.workspace_bytes > 0 && (!workspace || workspace_bytes < plan.workspace_bytes)) {
-    // an explicit split_k needs its workspace; the planner's own choice degrades to a single pass without one
+  const bool ws_aligned = ((uintptr_t)workspace & 15) == 0;
+  if (plan.workspace_bytes > 0 && (!workspace || workspace_bytes < plan.workspace_bytes || (!ws_aligned && desc->split_k <= 1))) {
+    // an explicit split_k needs its workspace; the planner's own choice degrades to a single pass without one it can use, be it
+    // missing, too small or off 16-byte boundaries: a caller cannot know which sizes the planner splits
     if (desc->split_k > 1) return fail(FRISK_ERR_WORKSPACE, "split_k=%d needs %zu bytes of workspace", desc->split_k, plan.workspace_bytes);
     ctx.no_workspace = true;
     extras = LaunchExtras{};
     st = make_plan(desc, &plan, false, ctx, &extras);
     if (st != FRISK_OK) return st;
   }
-  if (plan.workspace_bytes > 0 && ((uintptr_t)workspace & 15)) return fail(FRISK_ERR_ALIGNMENT, "workspace must be 16-byte aligned");
+  if (plan.workspace_bytes > 0 && !ws_aligned) return fail(FRISK_ERR_ALIGNMENT, "workspace must be 16-byte aligned");
   if (!device_ok()) return fail(FRISK_ERR_DEVICE, "no gfx950 device is current");
 
   GemmParams p;

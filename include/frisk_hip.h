@@ -157,7 +157,8 @@ size_t frisk_hip_workspace_bytes(const frisk_gemm_desc* desc);
 
 /* Launch on `stream` (a hipStream_t, may be NULL for the default stream).
  * A, B, C, scaleA, scaleB, workspace are device pointers.  scaleA/scaleB are
- * fp32: M and N entries for ROW_COL_SCALE, one entry each for TENSOR_SCALE. */
+ * fp32: M and N entries for ROW_COL_SCALE, one entry each for TENSOR_SCALE.
+ * A workspace that is too small or not 16-byte aligned is an error with split_k > 1 and not used otherwise. */
 int frisk_hip_gemm(const frisk_gemm_desc* desc, const void* A, const void* B, void* C, const float* scaleA,
                    const float* scaleB, void* workspace, size_t workspace_bytes, void* stream);
 

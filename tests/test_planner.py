@@ -394,3 +394,17 @@ def test_tail_splits_the_planner_chooses_can_exceed_the_static_workspace():
             assert p.workspace_bytes == p.tail_split * p.tail_tiles * 256 * 256 * 4
             over += p.workspace_bytes > static
     assert over >= 8
+
+
+@pytest.mark.skipif(os.path.exists("/dev/kfd"), reason="passes addresses that are not device memory")
+@pytest.mark.parametrize("M,N,K,split", [(256, 4096, 4096, 0), (1589, 3072, 9600, 0), (3000, 11008, 4096, 0), (1999, 4099, 3001, 0), (256, 4096, 4096, 2)])
+def test_unaligned_workspace_is_refused_for_an_explicit_split_only(M, N, K, split):
+    """split-K, split edge tiles, tail split, operand copies: the planner's own use of the workspace is no reason to refuse a call,
+    which without a GPU ends at the device check"""
+    base = 1 << 32
+    d = R.make_desc(R.F16, M, N, K, transB=True, split_k=split)
+    need = R.plan(d).workspace_bytes
+    assert need > 0
+    with pytest.raises(R.FriskHipError) as e:
+        R.gemm(d, base, base * 2, base * 3, workspace_ptr=base * 4 + 4, workspace_bytes=need)
+    assert R.STATUS_NAMES[e.value.status] == ("ERR_ALIGNMENT" if split else "ERR_DEVICE")
