@@ -458,8 +458,12 @@ static int small_grid_split(const KernelEntry* k, const frisk_gemm_desc* d, bool
     // keeps its `w`: there the unsplit tiles that stream B are as good): the model holds beyond it.  us at 16 K tiles and 128 or 256 work-groups / now: int8
     // 40x2880x7040 NN 29.5 / 12.8, e4m3 59x7104x4608 21.7 / 14.2, fp16 37x6720x3328 23.7 / 14.5, 16x2496x4224 14.7 / 11.3, 276x1280x3520 17.5 / 12.4;
     // 70 drawn sizes whose split changed 1.27 times faster, the worst 0.94 (3x9536x5760).  512 work-groups: 0.96 on 45.
-    const int64_t wgs = k->transB ? m.w : std::max(m.w, 256);
-    const int64_t most = std::min<int64_t>({k->dtype == FRISK_F32 ? 32 : 64, tiles > 0 ? wgs / tiles : 0, kt / std::max(std::min(m.kmin, 4), k->min_k_tiles)});
+    // A descriptor that names a tile stays within the fitted range: the unsplit and the split kernel of one tile are different kernels, and
+    // which of the two a tile names is not to move with the model (e4m3 512x512x2048 on 256x256 tiles of the 16x16x128 atom: unsplit).
+    const bool named = d->tile_m || d->tile_n || d->tile_k;
+    const int64_t wgs = k->transB || named ? m.w : std::max(m.w, 256);
+    const int kmin = std::max(named ? m.kmin : std::min(m.kmin, 4), k->min_k_tiles);
+    const int64_t most = std::min<int64_t>({k->dtype == FRISK_F32 ? 32 : 64, tiles > 0 ? wgs / tiles : 0, kt / kmin});
     for (int c = 2; c <= most; ++c)
       if (kt % c == 0) {
         const double t = small_grid_time(m, k, d, c);

@@ -408,3 +408,10 @@ def test_unaligned_workspace_is_refused_for_an_explicit_split_only(M, N, K, spli
     with pytest.raises(R.FriskHipError) as e:
         R.gemm(d, base, base * 2, base * 3, workspace_ptr=base * 4 + 4, workspace_bytes=need)
     assert R.STATUS_NAMES[e.value.status] == ("ERR_ALIGNMENT" if split else "ERR_DEVICE")
+
+
+def test_named_tile_keeps_its_unsplit_kernel_within_the_fitted_range():
+    """16 K tiles on 4 tiles of 256x256: one slice of the shortest length the tables were fitted over"""
+    d = R.make_desc(R.E4M3, 512, 512, 2048, dtype_out=R.BF16, transB=1, epilogue=R.EPI_TENSOR_SCALE, tile=(256, 256, 128), atom=16)
+    p = R.plan(d)
+    assert (p.split_k, p.workspace_bytes) == (1, 0) and R.kernel_names()[p.kernel_id].endswith("_a16")
