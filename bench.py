@@ -254,7 +254,7 @@ def main():
     C8 = torch.empty(M, N, device=dev, dtype=torch.float16)
     d8 = R.make_desc(R.I8, M, N, K, dtype_out=R.F16, epilogue=R.EPI_ROW_COL_SCALE)
     t8 = time_launches(torch, gemm_launcher(d8, (A8.data_ptr(), B8.data_ptr(), C8.data_ptr(), sA.data_ptr(), sB.data_ptr())), a.steps, a.warmup, stream)
-    legs = {"int8_4096": mfma_leg("W8A8 int8 4096^3 NN, int32 accumulate, per-row/per-column fp32 scales, fp16 out (configs[3])", "i8", flops, t8,
+    legs = {"int8_4096": mfma_leg("W8A8 int8 4096^3 NN, int32 accumulate, per-row/per-column fp32 scales, fp16 out", "i8", flops, t8,
                                   {"kernel": R.kernel_names()[R.plan(d8).kernel_id]})}
     vendor = {}
 
@@ -323,7 +323,7 @@ def main():
             legs[key]["sustained_peak"] = sustained_peak(ceiling, dk)
             legs[key]["frac_of_sustained"] = round(legs[key]["achieved"] / legs[key]["sustained_peak"], 4)
 
-        # configs[0]: fp32 1024^3 built through the IR builder, lowered by frisk_ffi.runtime, launched through the C ABI
+        # fp32 1024^3 built through the IR builder, lowered by frisk_ffi.runtime, launched through the C ABI
         import frisk_amd  # noqa: F401  (puts the builder package on the path)
         import frisk as F
         M1 = 1024
@@ -335,7 +335,7 @@ def main():
         p1 = [A1.data_ptr(), B1.data_ptr(), C1.data_ptr()]
         t1 = time_launches(torch, lambda: F.runtime.launch(kern, p1, cs), a.steps, a.warmup, stream)
         legs["fp32_1024_builder"] = mfma_leg("fp32 1024^3 NN, U[-1,1], built with the IR builder (128x128x32 tiles as in the design sketch) and launched by "
-                                             "frisk_ffi.runtime, which matches the program and lets the planner pick the kernel (configs[0]); the time "
+                                             "frisk_ffi.runtime, which matches the program and lets the planner pick the kernel; the time "
                                              "includes that host work per launch", "f32", 2.0 * M1 ** 3, t1)
         d1 = R.make_desc(R.F32, M1, M1, M1)
         t1c = time_launches(torch, gemm_launcher(d1, (A1.data_ptr(), B1.data_ptr(), C1.data_ptr(), None, None)), a.steps, a.warmup, stream)
@@ -345,7 +345,7 @@ def main():
         vendor["fp32_1024"] = vendor_leg(torch, "torch.matmul(A, B, out=C), fp32 1024^3 NN (allow_tf32 = %s)" % torch.backends.cuda.matmul.allow_tf32,
                                          lambda: torch.matmul(A1, B1, out=C1v), 2.0 * M1 ** 3, a.steps, a.warmup, stream, t1c["mean_ms"])
 
-        # bf16 8192^3 NT; configs[4], square part: fp8 e4m3 8192^3 NT with per-tensor scales, bf16 out
+        # bf16 8192^3 NT; square part of the fp8 pair: fp8 e4m3 8192^3 NT with per-tensor scales, bf16 out
         Mb = 8192
         big_steps = max(5, min(a.steps, 40))
         Ab = (torch.randn(Mb, Mb, device=dev, generator=g) * 0.02).bfloat16()
@@ -353,7 +353,7 @@ def main():
         Cb = torch.empty(Mb, Mb, device=dev, dtype=torch.bfloat16)
         db = R.make_desc(R.BF16, Mb, Mb, Mb, dtype_out=R.BF16, transB=True)
         tb = time_launches(torch, gemm_launcher(db, (Ab.data_ptr(), Bb.data_ptr(), Cb.data_ptr(), None, None)), big_steps, 3, stream)
-        legs["bf16_8192_nt"] = mfma_leg("bf16 8192^3 NT, N(0,1)*0.02, fp32 accumulate, bf16 out (configs[2])", "bf16", 2.0 * Mb ** 3, tb,
+        legs["bf16_8192_nt"] = mfma_leg("bf16 8192^3 NT, N(0,1)*0.02, fp32 accumulate, bf16 out", "bf16", 2.0 * Mb ** 3, tb,
                                         {"kernel": R.kernel_names()[R.plan(db).kernel_id], "steps": big_steps,
                                          "sustained_peak": sustained_peak(ceiling, "bf16")})
         legs["bf16_8192_nt"]["frac_of_sustained"] = round(legs["bf16_8192_nt"]["achieved"] / legs["bf16_8192_nt"]["sustained_peak"], 4)
@@ -366,7 +366,7 @@ def main():
         one = torch.full((1,), 0.01, device=dev)
         d8f = R.make_desc(R.E4M3, Mb, Mb, Mb, dtype_out=R.BF16, transB=True, epilogue=R.EPI_TENSOR_SCALE)
         t8f = time_launches(torch, gemm_launcher(d8f, (A8f.data_ptr(), B8f.data_ptr(), Cb.data_ptr(), one.data_ptr(), one.data_ptr())), big_steps, 3, stream)
-        legs["fp8_8192_nt"] = mfma_leg("fp8 e4m3 8192^3 NT, N(0,1) scaled to the e4m3 range, per-tensor fp32 scales, bf16 out (configs[4], square part)",
+        legs["fp8_8192_nt"] = mfma_leg("fp8 e4m3 8192^3 NT, N(0,1) scaled to the e4m3 range, per-tensor fp32 scales, bf16 out (square part)",
                                        "e4m3", 2.0 * Mb ** 3, t8f, {"kernel": R.kernel_names()[R.plan(d8f).kernel_id], "steps": big_steps,
                                                                     "sustained_peak": sustained_peak(ceiling, "e4m3")})
         legs["fp8_8192_nt"]["frac_of_sustained"] = round(legs["fp8_8192_nt"]["achieved"] / legs["fp8_8192_nt"]["sustained_peak"], 4)
@@ -399,7 +399,7 @@ def main():
         legs["fp8_skinny_32x8192x8192"] = {"bound": "hbm", "achieved": round(sk_gbs, 1), "peak": 8000.0, "unit": "GB/s", "frac": round(sk_gbs / 8000.0, 4),
                                            "kernel_ms": round(tsk["mean_ms"], 5), "kernel_ms_median": round(tsk["median_ms"], 5),
                                            "kernel_ms_min": round(tsk["min_ms"], 5), "kernel": R.kernel_names()[pf.kernel_id], "split_k": pf.split_k,
-                                           "workload": "fp8 e4m3 M=32 N=K=8192 NT, per-tensor scales, bf16 out (configs[4], decode part); algorithmic bytes "
+                                           "workload": "fp8 e4m3 M=32 N=K=8192 NT, per-tensor scales, bf16 out (decode part); algorithmic bytes "
                                                        "|A|+|B|+|C|+scales per launch, B rotating over 6 buffers"}
         vk_turn = [0]
 
