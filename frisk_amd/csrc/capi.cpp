@@ -767,10 +767,13 @@ int frisk_hip_gemm(const frisk_gemm_desc* desc, const void* A, const void* B, vo
     // an explicit split_k needs its workspace; the planner's own choice degrades to a single pass without one it can use, be it
     // missing, too small or off 16-byte boundaries: a caller cannot know which sizes the planner splits
     if (desc->split_k > 1) return fail(FRISK_ERR_WORKSPACE, "split_k=%d needs %zu bytes of workspace", desc->split_k, plan.workspace_bytes);
+    const size_t wanted = plan.workspace_bytes;
     ctx.no_workspace = true;
     extras = LaunchExtras{};
     st = make_plan(desc, &plan, false, ctx, &extras);
-    if (st != FRISK_OK) return st;
+    // a tile or wave policy that the caller named and that only kernels without staging through registers have: they want the copies
+    if (st != FRISK_OK)
+      return fail(FRISK_ERR_WORKSPACE, "rows or pointers off 16-byte boundaries: the tile or wave policy asked for runs on aligned copies of A or B, which need %zu bytes of 16-byte aligned workspace", wanted);
   }
   if (plan.workspace_bytes > 0 && !ws_aligned) return fail(FRISK_ERR_ALIGNMENT, "workspace must be 16-byte aligned");
   if (!device_ok()) return fail(FRISK_ERR_DEVICE, "no gfx950 device is current");

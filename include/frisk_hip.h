@@ -152,7 +152,9 @@ int frisk_hip_plan(const frisk_gemm_desc* desc, frisk_gemm_plan* plan);
 
 /* Pure host: bytes of device workspace `frisk_hip_gemm` wants for this descriptor: split_k * M * N * 4 when the
  * plan splits K, tail_split * tail_tiles * tile_m * tile_n * 4 for a tail split (the same per slice and tile for split kernels off the tiles), the size of the operands with padded rows
- * where they are copied, else 0.  With split_k = 0 in the descriptor a launch without workspace still runs, unsplit. */
+ * where they are copied, else 0.  With split_k = 0 in the descriptor a launch without workspace still runs, unsplit -- unless the descriptor names a
+ * tile, wave grid, ring, atom or wave policy which, for rows or pointers off 16-byte boundaries, only the kernels that work on the copies have:
+ * then it is FRISK_ERR_WORKSPACE. */
 size_t frisk_hip_workspace_bytes(const frisk_gemm_desc* desc);
 
 /* Launch on `stream` (a hipStream_t, may be NULL for the default stream).

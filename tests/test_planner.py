@@ -415,3 +415,29 @@ def test_named_tile_keeps_its_unsplit_kernel_within_the_fitted_range():
     d = R.make_desc(R.E4M3, 512, 512, 2048, dtype_out=R.BF16, transB=1, epilogue=R.EPI_TENSOR_SCALE, tile=(256, 256, 128), atom=16)
     p = R.plan(d)
     assert (p.split_k, p.workspace_bytes) == (1, 0) and R.kernel_names()[p.kernel_id].endswith("_a16")
+
+
+@pytest.mark.skipif(os.path.exists("/dev/kfd"), reason="passes addresses that are not device memory")
+@pytest.mark.parametrize("kw", [dict(tile=(256, 256, 64)), dict(policy=R.POLICY_FULL_ROW), dict(policy=R.POLICY_FULL_COL)], ids=["tile", "full_row", "full_col"])
+def test_a_plan_that_needs_copies_says_so_at_the_launch(kw):
+    """odd rows and a tile or wave policy that no kernel staging through registers has: the plan stands, and a launch without the workspace it
+    names is refused for the workspace, not for the tile"""
+    base = 1 << 32
+    M, N, K = (1001, 1003, 1001) if "tile" in kw else (31, 1003, 1001)
+    d = R.make_desc(R.F16, M, N, K, transB=True, **kw)
+    need = R.plan(d).workspace_bytes
+    assert need >= 2 * (M + N) * 1008 and R.workspace_bytes(d) == need
+
+    def status(launch, *ws):
+        with pytest.raises(R.FriskHipError) as e:
+            launch(d, base, base * 2, base * 3, **dict(zip(("workspace_ptr", "workspace_bytes"), ws)))
+        return R.STATUS_NAMES[e.value.status], str(e.value)
+
+    for ws in ((), (base * 4, need - 1), (base * 4 + 4, need)):
+        what, message = status(R.gemm, *ws)
+        assert what == "ERR_WORKSPACE" and str(need) in message, (ws, what, message)
+    assert status(R.gemm, base * 4, need)[0] == "ERR_DEVICE"  # everything in order but the GPU
+    assert status(R.gemm_static_ws)[0] == "ERR_DEVICE"
+    if "tile" in kw:  # copies larger than the static array
+        d = R.make_desc(R.F16, 4001, 4003, 4001, transB=True, **kw)
+        assert status(R.gemm_static_ws)[0] == "ERR_WORKSPACE"
