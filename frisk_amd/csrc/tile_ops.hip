@@ -27,7 +27,6 @@ template <> struct Elem<FRISK_BF16> { typedef __bf16 T; static __device__ float 
 // 2^lanes_log2 lanes of a work-group lie along a row, the remaining 256 >> lanes_log2 across rows, work-groups step
 // along the row in x and down the rows in y.  Every lane handles several groups per step: ALONG (1, 2 or 4) neighbours along the row
 // (4 KiB apart) where the row is long enough to give them work, or (ALONG 0) the same columns of eight rows.
-constexpr int kPerLaneAcross = 8;
 
 template <int ALONG> struct Walk {
   static constexpr int PER = ALONG ? ALONG : kPerLaneAcross;
@@ -357,36 +356,13 @@ reduce_finish_kernel(const float* partial, int slices, int64_t n, int clear, typ
   }
 }
 
-// grid and lane split of the division-free walk: lanes along a row = the power of two that covers the row's groups,
-// at most 256; x steps along the row, y down the rows (65535 at most, work-groups loop beyond that)
-struct WalkLaunch {
-  dim3 grid;
-  int lanes_log2, along;  // along: groups per lane along the row, 0: eight rows per lane instead
-  WalkLaunch(int64_t rows, int64_t groups_per_row, int per_lane_along = 2) {
-    lanes_log2 = 0;
-    while (lanes_log2 < 8 && (int64_t(1) << lanes_log2) < groups_per_row) ++lanes_log2;
-    along = groups_per_row >= 512 ? per_lane_along : 0;
-    const int64_t per_x = (int64_t(1) << lanes_log2) * (along ? along : 1), per_y = (int64_t)(256 >> lanes_log2) * (along ? 1 : kPerLaneAcross);
-    const int64_t slabs = (groups_per_row + per_x - 1) / per_x, row_blocks = (rows + per_y - 1) / per_y;
-    grid = dim3((unsigned)(slabs < 1 ? 1 : (slabs > 0x7fffffff ? 0x7fffffff : slabs)), (unsigned)(row_blocks < 1 ? 1 : (row_blocks > 65535 ? 65535 : row_blocks)));
-  }
-};
-
-// Groups per lane of a copy along its rows.  f32 to f32, TB/s read and written, 1 / 2 / 4 groups: 16 MiB 7.2 / 5.7 / 4.8 (too few
-// work-groups), 256 MiB 6.6 / 7.2 / 6.7, 512 MiB 6.6 / 7.4 / 6.9, 768 MiB 6.5 / 6.2 / 6.9, 1 GiB 6.5 / 6.1 / 6.9, 2 GiB 6.5 / 6.0 / 6.0: more than one
-// pays until the launch has 65536 work-groups.
-int copy_groups_per_lane(int64_t rows, int64_t groups_per_row) {
-  const int64_t one = rows * ((groups_per_row + 255) / 256), two = rows * ((groups_per_row + 511) / 512), four = rows * ((groups_per_row + 1023) / 1024);
-  if (one <= 8192) return 1;
-  return two <= 65536 ? 2 : four <= 65536 ? 4 : 1;
-}
-
 template <int DT> hipError_t fill_t(void* dst, int64_t rows, int64_t cols, int64_t ld, double value, hipStream_t s) {
   typedef typename Elem<DT>::T T;
   constexpr int G = 16 / sizeof(T);
-  const WalkLaunch w(rows, (cols + G - 1) / G);
-  if (w.along) hipLaunchKernelGGL((fill_kernel<DT, 2>), w.grid, dim3(256), 0, s, (T*)dst, rows, cols, ld, (float)value, w.lanes_log2);
-  else hipLaunchKernelGGL((fill_kernel<DT, 0>), w.grid, dim3(256), 0, s, (T*)dst, rows, cols, ld, (float)value, w.lanes_log2);
+  const WalkGrid w = walk_grid(rows, (cols + G - 1) / G);
+  const dim3 grid(w.x, w.y);
+  if (w.along) hipLaunchKernelGGL((fill_kernel<DT, 2>), grid, dim3(256), 0, s, (T*)dst, rows, cols, ld, (float)value, w.lanes_log2);
+  else hipLaunchKernelGGL((fill_kernel<DT, 0>), grid, dim3(256), 0, s, (T*)dst, rows, cols, ld, (float)value, w.lanes_log2);
   return hipGetLastError();
 }
 
@@ -394,8 +370,8 @@ template <int SDT, int DDT> hipError_t copy_t(const void* src, int64_t sld, void
   typedef typename Elem<SDT>::T S;
   typedef typename Elem<DDT>::T D;
   constexpr int G = 16 / (sizeof(S) < sizeof(D) ? sizeof(S) : sizeof(D));
-  const WalkLaunch w(rows, (cols + G - 1) / G, copy_groups_per_lane(rows, (cols + G - 1) / G));
-  auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, w.grid, dim3(256), 0, s, (const S*)src, sld, (D*)dst, dld, rows, cols, w.lanes_log2); };
+  const WalkGrid w = walk_grid(rows, (cols + G - 1) / G, copy_groups_per_lane(rows, (cols + G - 1) / G));
+  auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(w.x, w.y), dim3(256), 0, s, (const S*)src, sld, (D*)dst, dld, rows, cols, w.lanes_log2); };
   switch (w.along) {
     case 1: launch(copy_kernel<SDT, DDT, 1>); break;
     case 2: launch(copy_kernel<SDT, DDT, 2>); break;
@@ -409,11 +385,11 @@ template <int SDT, int DDT> hipError_t copy_tiles_t(const void* src, int64_t sld
   typedef typename Elem<SDT>::T S;
   typedef typename Elem<DDT>::T D;
   constexpr int G = 16 / (sizeof(S) < sizeof(D) ? sizeof(S) : sizeof(D));
-  WalkLaunch w(rows, (cols + G - 1) / G);
+  const WalkGrid w = walk_grid(rows, (cols + G - 1) / G);
   const int64_t tiles = t.n0 * t.n1;
-  w.grid.z = (unsigned)(tiles > 65535 ? 65535 : tiles);
-  if (w.along) hipLaunchKernelGGL((copy_tiles_kernel<SDT, DDT, 2>), w.grid, dim3(256), 0, s, (const S*)src, sld, (D*)dst, dld, rows, cols, t, w.lanes_log2);
-  else hipLaunchKernelGGL((copy_tiles_kernel<SDT, DDT, 0>), w.grid, dim3(256), 0, s, (const S*)src, sld, (D*)dst, dld, rows, cols, t, w.lanes_log2);
+  const dim3 grid(w.x, w.y, (unsigned)(tiles > 65535 ? 65535 : tiles));
+  if (w.along) hipLaunchKernelGGL((copy_tiles_kernel<SDT, DDT, 2>), grid, dim3(256), 0, s, (const S*)src, sld, (D*)dst, dld, rows, cols, t, w.lanes_log2);
+  else hipLaunchKernelGGL((copy_tiles_kernel<SDT, DDT, 0>), grid, dim3(256), 0, s, (const S*)src, sld, (D*)dst, dld, rows, cols, t, w.lanes_log2);
   return hipGetLastError();
 }
 

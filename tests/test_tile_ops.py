@@ -4,6 +4,9 @@ and the HIP kernels against the oracle through the C ABI (GPU).
 Bars: fill and same-type copy bit-exact; converting copies bit-exact (one rounding, the oracle's codec); min / max
 bit-exact; add / mul within 1e-3 (f16, bf16: the result's own rounding dominates) or 1e-5 (f32) of the float64 value,
 relative to max(|r|, rms(R))."""
+import os
+import subprocess
+
 import numpy as np
 import pytest
 
@@ -131,6 +134,26 @@ def test_copy_gpu(hip, sdt, ddt):
         view = got[shift:].reshape(rows, dld)
         assert np.array_equal(view[:, :cols], T.copy(sdt, vals, ddt)), (rows, cols, pad, shift)
         assert np.array_equal(view[:, cols:], dst0[shift:].reshape(rows, dld)[:, cols:]) and np.array_equal(got[:shift], dst0[:shift])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("sdt,ddt", [(O.F32, O.F32), (O.F16, O.F16), (O.F32, O.F16), (O.BF16, O.F32)], ids=lambda d: NAMES[d])
+@pytest.mark.parametrize("rows,groups", [(4100, 520), (40000, 520), (65540, 512)], ids=["2_along", "4_along", "1_along_and_more_rows_than_the_grid"])
+def test_copies_with_several_groups_per_lane(hip, sdt, ddt, rows, groups):
+    """Views large enough for two and four groups per lane along the rows (more than 8192 work-groups of 256 groups), and for one again: rows that
+    end inside a slab and inside a group, padded, starting on any element.  Compared on the device, the bytes outside the view too."""
+    import torch
+    types = {O.F32: torch.float32, O.F16: torch.float16, O.BF16: torch.bfloat16}
+    es = {O.F32: 4, O.F16: 2, O.BF16: 2}
+    G = 16 // min(es[sdt], es[ddt])
+    cols, shift = groups * G + 3, 1
+    sld, dld = cols + 2, cols + 5
+    src = torch.randn(shift + rows * sld, device="cuda", dtype=types[sdt], generator=torch.Generator(device="cuda").manual_seed(71))
+    dst = torch.full((shift + rows * dld,), 7.0, device="cuda", dtype=types[ddt])
+    want = dst.clone()
+    want.as_strided((rows, cols), (dld, 1), shift).copy_(src.as_strided((rows, cols), (sld, 1), shift))
+    hip.copy(sdt, src.data_ptr() + shift * es[sdt], sld, ddt, dst.data_ptr() + shift * es[ddt], dld, rows, cols, torch.cuda.current_stream().cuda_stream)
+    assert torch.equal(dst, want)
 
 
 def _close(dt, got, ref64):
@@ -409,3 +432,35 @@ def test_copy_tiles_gpu(hip):
                 sr, sc, dr, dc = so // sld, so % sld, do // dld, do % dld
                 want[dr:dr + tr, dc:dc + tc] = conv[sr:sr + tr, sc:sc + tc]
         assert np.array_equal(_host(dy, O.NP_STORAGE[ddt]).reshape(dst_rows, dld), want), (sdt, ddt, tr, tc)
+
+
+def test_grids_of_fill_and_copy_fit_a_launch(tmp_path):
+    """the grid arithmetic of csrc/tile_ops.h on the host: fewer than 2^32 lanes in x for views of up to 2^36 groups of 16 bytes (a dense view is
+    one row), 65535 work-groups in y, and steps that cover the view with work-groups that loop"""
+    src = tmp_path / "grids.cpp"
+    src.write_text("""
+#include <cstdio>
+#include "tile_ops.h"
+int main() {
+  using namespace frisk;
+  long long rows, groups;
+  while (scanf("%lld %lld", &rows, &groups) == 2)
+    for (int per : {2, copy_groups_per_lane(rows, groups)}) {
+      const WalkGrid g = walk_grid(rows, groups, per);
+      printf("%lld %lld %d %u %u %d %d\\n", rows, groups, per, g.x, g.y, g.lanes_log2, g.along);
+    }
+}
+""")
+    exe = tmp_path / "grids"
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    subprocess.run([os.environ.get("CXX", "g++"), "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", "-I" + os.path.join(root, "include"),
+                    "-I" + os.path.join(root, "frisk_amd", "csrc"), str(src), "-o", str(exe)], check=True)
+    views = [(1, 1 << e) for e in range(0, 37)] + [(1 << r, 1 << c) for r in range(1, 31, 3) for c in range(0, 28, 3)] + [(70001, 600), (3, 511), (5000, 513)]
+    out = subprocess.run([str(exe)], input="\n".join("%d %d" % v for v in views), capture_output=True, text=True, check=True).stdout.split("\n")
+    assert len(out) == 2 * len(views) + 1
+    for line in out[:-1]:
+        rows, groups, per, x, y, lanes_log2, along = map(int, line.split())
+        assert 1 <= x * 256 < 1 << 32 and 1 <= y <= 65535, line
+        assert along in (0, per) and (along > 0) == (groups >= 512) and 0 <= lanes_log2 <= 8
+        slabs, blocks = -(-groups // ((1 << lanes_log2) * max(along, 1))), -(-rows // ((256 >> lanes_log2) * (1 if along else 8)))
+        assert x == min(slabs, 1 << 23) and y == min(blocks, 65535), line
