@@ -232,3 +232,37 @@ def test_attention_share_of_masked_keys(bh):
     assert np.isnan(O.decode(dtype, got2[:, 7].reshape(-1))).all() and np.isnan(lse2[:, 7]).all()
     rest = [i for i in range(sq) if i != 7]
     assert np.array_equal(got2[:, rest], got[:, rest]) and np.array_equal(lse2[:, rest], lse[:, rest])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bh", [2, 40, 80], ids=["8_shares", "4_shares", "2_shares"])
+@pytest.mark.parametrize("visible", [64, 448], ids=["most_keys", "last_tile"])
+def test_attention_keys_masked_by_the_lowest_value(bh, visible):
+    """Keys whose first component is the lowest bf16, against queries that are 1 there: their scores times the scale lie within a tenth of the
+    lowest fp32, and whole shares of the keys hold nothing else"""
+    dtype, sq, sk = O.BF16, 256, 512
+    q, k, v = make_qkv(dtype, bh, sq, sk, 128, seed=62)
+    q[:, :, 0] = O.encode(dtype, np.array([1.0], np.float32))[0]
+    k[:, :, 0] = O.encode(dtype, np.array([0.0], np.float32))[0]
+    k[:, visible:, 0] = 0xFF7F  # -3.39e38; times 0.65 log2(e): -3.18e38
+    got, lse = run_attention(dtype, q, k, v, 0.65)
+    heads = min(bh, 2)
+    ref, ref_lse = A.attention_f64(dtype, q[:heads], k[:heads], v[:heads], 0.65)
+    check(dtype, got[:heads], lse[:heads], ref, ref_lse)
+    assert np.isfinite(O.decode(dtype, got.reshape(-1))).all() and np.isfinite(lse).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bh", [2, 40, 80], ids=["8_shares", "4_shares", "2_shares"])
+def test_attention_infinite_scores_stay_in_their_rows(bh):
+    """a query of +inf scores +inf and -inf: its row is NaN, whichever share its largest score lies in; the other rows of its wave only see
+    their exponent references move"""
+    dtype, sq, sk = O.F16, 256, 512
+    q, k, v = make_qkv(dtype, bh, sq, sk, 128, seed=63)
+    ref, ref_lse = A.attention_f64(dtype, q[:2], k[:2], v[:2], 0.2)
+    q[:, 9, 5] = O.encode(dtype, np.array([np.inf], np.float32))[0]
+    got, lse = run_attention(dtype, q, k, v, 0.2)
+    assert np.isnan(O.decode(dtype, got[:, 9].reshape(-1))).all() and np.isnan(lse[:, 9]).all()
+    rest = [i for i in range(sq) if i != 9]
+    assert np.isfinite(O.decode(dtype, got[:, rest].reshape(-1))).all() and np.isfinite(lse[:, rest]).all()
+    check(dtype, np.ascontiguousarray(got[:2, rest]), lse[:2, rest], ref[:, rest], ref_lse[:, rest])

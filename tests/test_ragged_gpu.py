@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 
 import oracle as O
-from helpers import DEFAULT_OUT, TOL, from_dev, make_operand, stored_shapes, to_dev
+from helpers import DEFAULT_OUT, TOL, from_dev, make_operand, run_gemm, stored_shapes, to_dev
 
 BK = {O.F32: 32, O.F16: 64, O.BF16: 64, O.I8: 128, O.E4M3: 128}
 ES = {O.F32: 4, O.F16: 2, O.BF16: 2, O.I8: 1, O.E4M3: 1}
@@ -166,3 +166,37 @@ def test_edge_kernels_split_on_grids_of_half_a_round(hip, dtype, transA, transB,
             tiles = -(-M // bm) * -(-N // bn)
             assert bm >= 128 and tiles <= 128 and need >= 2 * tiles * bm * bn * 4, (name, need)
         verify(dtype, got, A, B, transA, transB)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,tail", [(500, 1501, False), (500, 1503, False), (16 * 256 + 3, 15 * 256 + 17, True)])
+def test_summed_edge_tiles_apply_scales_and_accumulate(hip, M, N, tail):
+    """the second kernel of split edge tiles at ragged M and N: column scales of exactly N entries with N ending inside a quad of columns, rows of
+    C off 16-byte boundaries, the tensor scale and the old values of C; int8 bit for bit"""
+    K8, K16 = 8048, 4024 if not tail else 2008
+
+    def split(*a, **kw):
+        p = hip.plan(hip.make_desc(*a, transB=True, **kw))
+        tiles = p.grid_x * p.grid_y % 256 if tail else p.grid_x * p.grid_y
+        assert "_guard" in hip.kernel_names()[p.kernel_id] and p.workspace_bytes >= 2 * tiles * p.tile_m * p.tile_n * 4, (hip.kernel_names()[p.kernel_id], p.workspace_bytes)
+
+    Ai, Bi = make_operand(O.I8, M, K8, 88, 0), make_operand(O.I8, N, K8, 88, 1)
+    sA, sB = O.uniform(M, 88, 2, 0.001, 0.02), O.uniform(N, 88, 3, 0.001, 0.02)
+    acc = O.gemm_i32(Ai, Bi, 0, 1)
+    split(O.I8, M, N, K8, dtype_out=O.F16, epilogue=hip.EPI_ROW_COL_SCALE)
+    got = run_gemm(hip, O.I8, Ai, Bi, 0, 1, O.F16, M, N, K8, epilogue=hip.EPI_ROW_COL_SCALE, sA=sA, sB=sB, pad_c=0)
+    assert np.array_equal(got, O.epilogue_rowcol_f16(acc, sA, sB))
+    C0 = (np.arange(M * N, dtype=np.int64).reshape(M, N) % 91 - 45).astype(np.int32)
+    assert np.array_equal(run_gemm(hip, O.I8, Ai, Bi, 0, 1, O.I32, M, N, K8, C_init=C0, clear_accum=False), acc + C0)
+    Ah, Bh = make_operand(O.F16, M, K16, 89, 0, scale=0.5), make_operand(O.F16, N, K16, 89, 1, scale=0.5)
+    Cf = O.uniform(M * N, 89, 2, -1.0, 1.0).reshape(M, N).astype(np.float32)
+    split(O.F16, M, N, K16, dtype_out=O.F32, clear_accum=False)
+    got = run_gemm(hip, O.F16, Ah, Bh, 0, 1, O.F32, M, N, K16, C_init=Cf, clear_accum=False)
+    r = O.compare(O.F32, np.ascontiguousarray(got), O.gemm_f64(O.F16, Ah, Bh, False, True) + Cf.astype(np.float64))
+    assert r["nonfinite"] == 0 and r["max_rel"] <= TOL[O.F32] and r["fro_rel"] <= TOL[O.F32], r
+    if not tail:
+        A8, B8 = make_operand(O.E4M3, M, K8, 90, 0, scale=0.5), make_operand(O.E4M3, N, K8, 90, 1, scale=0.5)
+        split(O.E4M3, M, N, K8, dtype_out=O.BF16, epilogue=hip.EPI_TENSOR_SCALE)
+        got = run_gemm(hip, O.E4M3, A8, B8, 0, 1, O.BF16, M, N, K8, epilogue=hip.EPI_TENSOR_SCALE, sA=[0.25], sB=[0.02])
+        r = O.compare(O.BF16, np.ascontiguousarray(got), O.epilogue_tensor(O.gemm_f64(O.E4M3, A8, B8, False, True), np.float32(0.25), np.float32(0.02)))
+        assert r["nonfinite"] == 0 and r["max_rel"] <= TOL[O.BF16] and r["fro_rel"] <= TOL[O.BF16], r
