@@ -9,8 +9,8 @@
 // assembly over fixed registers: a step is two lane reads of the program, a jump to its handler and 8 vector instructions in
 // place, the operand picked by the register index mode.  (As a C++ switch the compiler joins the values of all cases after every
 // step by register moves: 327 vector, 300 scalar and 120 branch instructions per group of 8 columns for (x - s * c) * g + b; here
-// 109, 125 and 34.)  That body on 8192 x 8192 f16: 139 us before, 51 now (a plain copy: 41); log2(max(x, c) / (x + c)), bound by
-// the vector pipe in its division, 125 -> 71.5; rows off 16-byte boundaries (4095 x 8191) 370 -> 51.
+// 109, 125 and 34.)  That body on 8192 x 8192 f16: 137 us before, 51 now (a plain copy: 41); log2(max(x, c) / (x + c)), bound by
+// the vector pipe in its division, 123 -> 69.5; x + y 80 -> 71; rows off 16-byte boundaries (4095 x 8191) 369 -> 46.
 // Operands that are the same for every row stay in registers while the lane's columns do, values of one per row stay one
 // register, and what the next groups need from memory is fetched while the current one is evaluated.  All arithmetic is
 // fp32; the result is rounded once to the output type.
@@ -41,10 +41,26 @@ constexpr int kChunk = 64;  // steps in one register of a wave, one per lane; ST
 struct EwSteps {
   int code[2 * kChunk];
   float imm[2 * kChunk];
+  int n;                  // steps
   int depth;              // most values below the top at any time
   int head, walk2;        // operands fetched a group ahead: the one the program starts with, and another that walks the rows (-1: none)
   int col0, col1;         // operands that are the same for every row, kept in registers while the columns stay
   int row0, row1;         // operands of one value per row, fetched a group ahead
+};
+// An operand as the kernel addresses it, resolved on the host (an operand looked up by its number is a chain of dependent scalar loads).
+struct EwOperand {
+  const char* at;     // nullptr: none
+  int64_t row_bytes;  // to the next row
+  int dt, walks;      // walks: one element per column
+};
+struct EwArgs {
+  int64_t rows, cols, out_row_bytes;
+  char* out;
+  int out_dt, n_steps;
+  EwOperand head, walk2, row0, row1, col0, col1;
+  EwOperand in[FRISK_EW_MAX_INPUTS];  // for STEP_FETCH, by number
+  int code[2 * kChunk];
+  float imm[2 * kChunk];
 };
 
 // ---- the interpreter loop.  EACH: one instruction per column.  Handlers lie 256 bytes apart, in the order of Step; NEXT fetches
@@ -104,14 +120,29 @@ __device__ __forceinline__ Raw load_raw(const char* at, int dt, bool streamed) {
   }
   return r;
 }
-// the first `valid` (1 to 7) of 8 elements
-__device__ __forceinline__ Raw load_raw_partial(const char* at, int dt, int valid) {
+// The first `valid` (1 to 7) of 8 elements.  TOGETHER: without branches, the last one again in place of those beyond it, so that all are under way
+// together: what a small view waits for (300 x 77 f16: x g + b 4.7 -> 3.9 us); the kernels for long rows keep the branches, which cost them fewer
+// registers (8192 x 8192 f16, (x - s c) g + b: 51.5 us, 53.2 without).
+template <bool TOGETHER> __device__ __forceinline__ Raw load_raw_partial(const char* at, int dt, int valid) {
   unsigned w[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+  if constexpr (TOGETHER) {
+    if (dt == FRISK_F32) {
 #pragma unroll
-  for (int e = 0; e < V; ++e) {
-    if (e >= valid) continue;
-    if (dt == FRISK_F32) w[e] = ((const unsigned*)at)[e];
-    else w[e / 2] |= (unsigned)((const uint16_t*)at)[e] << (16 * (e & 1));
+      for (int e = 0; e < V; ++e) w[e] = ((const unsigned*)at)[e < valid ? e : valid - 1];
+    } else {
+      unsigned h[V];
+#pragma unroll
+      for (int e = 0; e < V; ++e) h[e] = ((const uint16_t*)at)[e < valid ? e : valid - 1];
+#pragma unroll
+      for (int e = 0; e < V; ++e) w[e / 2] |= h[e] << (16 * (e & 1));
+    }
+  } else {
+#pragma unroll
+    for (int e = 0; e < V; ++e) {
+      if (e >= valid) continue;
+      if (dt == FRISK_F32) w[e] = ((const unsigned*)at)[e];
+      else w[e / 2] |= (unsigned)((const uint16_t*)at)[e] << (16 * (e & 1));
+    }
   }
   return Raw{v4u{w[0], w[1], w[2], w[3]}, v4u{w[4], w[5], w[6], w[7]}};
 }
@@ -170,10 +201,17 @@ __device__ __forceinline__ void store_group(char* at, int dt, const v8f& r, int 
   }
 }
 
-// DT: element type of the operands that walk the rows and of the output (-1: mixed, read from the arguments).  AHEAD: the operands
-// named in EwSteps beside `head` are held or fetched ahead (44 more registers for 32-bit operands, 32 for 16-bit ones).  DEPTH: values
-// below the top the program needs.  UNIFORM_ROW: a wave's lanes lie in one row (rows of at least 64 groups).
-template <int DT, bool AHEAD, int DEPTH, bool UNIFORM_ROW> __global__ void __launch_bounds__(256) elementwise_kernel(EwParams p, EwSteps prog, int lanes_log2) {
+// DT: element type of the operands that walk the rows and of the output (-1: mixed, read from the arguments).  HELD: which operands beside
+// `head` are held or fetched ahead: none; the second one that walks the rows; that one and the broadcast ones (44 more registers for 32-bit
+// operands, 32 for 16-bit ones, and 1500 instructions in front of the first step instead of 650: x + y of 1024 x 4096 f16 7.4 us with them,
+// 6.5 without, f32 11.3 and 9.9, 100000 x 24 f16 5.6 and 4.5, 8192 x 8192 f16 74.4 and 71).  DEPTH: values below the top the program needs.
+// UNIFORM_ROW: a wave's lanes lie in one row (rows of at least 64 groups).
+enum Held { HELD_NONE, HELD_WALK, HELD_ALL };
+// Kernels that hold all of them run four waves a SIMD where their registers allow it ((x - s c) g + b of 100000 x 24 f16: 136 registers and three
+// waves 8.6 us, 7.4 with four).
+constexpr bool four_waves(int dt, int held, int depth, bool uniform_row) { return held == HELD_ALL && depth == 1 && !(dt == FRISK_F32 && !uniform_row); }
+template <int DT, int HELD, int DEPTH, bool UNIFORM_ROW> __global__ void __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(four_waves(DT, HELD, DEPTH, UNIFORM_ROW) ? 4 : 1, four_waves(DT, HELD, DEPTH, UNIFORM_ROW) ? 4 : 8))) elementwise_kernel(EwArgs p, int lanes_log2) {
   const int lanes = 1 << lanes_log2, row_step = 256 >> lanes_log2;
   const int lane_group = threadIdx.x & (lanes - 1);
   int lane_row = threadIdx.x >> lanes_log2;
@@ -181,17 +219,17 @@ template <int DT, bool AHEAD, int DEPTH, bool UNIFORM_ROW> __global__ void __lau
   const int64_t groups = (p.cols + V - 1) / V, slabs = (groups + lanes - 1) >> lanes_log2, row_blocks = (p.rows + row_step - 1) / row_step;
   const bool ragged = p.cols % V != 0;
   // step i of a chunk of the program in lane i: a lane read instead of a dependent scalar load
-  int code_reg[2], imm_reg[2];
-#pragma unroll
-  for (int c = 0; c < 2; ++c) { code_reg[c] = prog.code[c * kChunk + (threadIdx.x & 63)]; imm_reg[c] = __builtin_bit_cast(int, prog.imm[c * kChunk + (threadIdx.x & 63)]); }
-  auto type_of = [&](int k) { return DT >= 0 ? DT : p.in_dtype[k]; };
+  int code_reg[2] = {p.code[threadIdx.x & 63], 0}, imm_reg[2] = {__builtin_bit_cast(int, p.imm[threadIdx.x & 63]), 0};
+  if (p.n_steps > kChunk) {
+    code_reg[1] = p.code[kChunk + (threadIdx.x & 63)];
+    imm_reg[1] = __builtin_bit_cast(int, p.imm[kChunk + (threadIdx.x & 63)]);
+  }
+  auto type_of = [&](const EwOperand& k) { return DT >= 0 ? DT : k.dt; };
   auto row_value = [&](int dt, unsigned bits) {
     if (dt == FRISK_F32) return __builtin_bit_cast(float, bits);
     if (dt == FRISK_F16) return (float)__builtin_bit_cast(_Float16, (uint16_t)bits);
     return __builtin_bit_cast(float, bits << 16);
   };
-  // (named once: an operand's type read from the arguments by its number is a scalar load and a wait in every group)
-  const int row0_dt = AHEAD && prog.row0 >= 0 ? p.in_dtype[prog.row0] : FRISK_F32, row1_dt = AHEAD && prog.row1 >= 0 ? p.in_dtype[prog.row1] : FRISK_F32;
   const int64_t rb0 = blockIdx.y, row_stride = (int64_t)gridDim.y * row_step;  // rows between this lane's groups
   if (rb0 >= row_blocks) return;
   // A lane keeps its columns and walks down the rows, every operand's address moving on by one stride: worked out anew for every
@@ -205,41 +243,44 @@ template <int DT, bool AHEAD, int DEPTH, bool UNIFORM_ROW> __global__ void __lau
     const int valid = p.cols - first_col < V ? (int)(p.cols - first_col) : V;
     int64_t row = rb0 * row_step + lane_row;
     const int64_t row_in = row < p.rows ? row : p.rows - 1;
-    // element (row_in, first column of the group) of operand k, whose elements are of type dt
-    auto operand_at = [&](int k, int dt, bool walks, int64_t r) {
+    // element (r, first column of the group) of an operand whose elements are of type dt
+    auto operand_at = [&](const EwOperand& k, int dt, bool walks, int64_t r) {
       const int es = dt == FRISK_F32 ? 4 : 2;
-      const char* base = (const char*)p.in[k] + r * (p.in_row_stride[k] * es);
+      const char* base = k.at + r * k.row_bytes;
       return walks ? base + (slab << lanes_log2) * (V * es) + (unsigned)(off * (V * es)) : base;
     };
     auto fetch_at = [&](const char* at, int dt, bool streamed) {
       if (!ragged || valid >= V) return load_raw(at, dt, streamed);
-      return load_raw_partial(at, dt, valid);
+      return load_raw_partial<!UNIFORM_ROW && HELD != HELD_ALL>(at, dt, valid);
     };
     auto fetch_row_at = [&](const char* at, int dt) { return dt == FRISK_F32 ? *(const unsigned*)at : (unsigned)*(const uint16_t*)at; };
-    auto stride_of = [&](int k, int dt) { return row_stride * p.in_row_stride[k] * (dt == FRISK_F32 ? 4 : 2); };
     const char *head_at = nullptr, *walk2_at = nullptr, *row0_at = nullptr, *row1_at = nullptr;
     int64_t head_step = 0, walk2_step = 0, row0_step = 0, row1_step = 0;
-    if (prog.head >= 0) { head_at = operand_at(prog.head, type_of(prog.head), true, row_in); head_step = stride_of(prog.head, type_of(prog.head)); }
-    if constexpr (AHEAD) {
-      if (prog.walk2 >= 0) { walk2_at = operand_at(prog.walk2, type_of(prog.walk2), true, row_in); walk2_step = stride_of(prog.walk2, type_of(prog.walk2)); }
-      if (prog.row0 >= 0) { row0_at = operand_at(prog.row0, row0_dt, false, row_in); row0_step = stride_of(prog.row0, row0_dt); }
-      if (prog.row1 >= 0) { row1_at = operand_at(prog.row1, row1_dt, false, row_in); row1_step = stride_of(prog.row1, row1_dt); }
+    if (p.head.at) { head_at = operand_at(p.head, type_of(p.head), true, row_in); head_step = row_stride * p.head.row_bytes; }
+    if constexpr (HELD >= HELD_WALK) {
+      if (p.walk2.at) { walk2_at = operand_at(p.walk2, type_of(p.walk2), true, row_in); walk2_step = row_stride * p.walk2.row_bytes; }
     }
-    const int out_dt = DT >= 0 ? DT : p.out_dtype, out_es = out_dt == FRISK_F32 ? 4 : 2;
-    char* out_at = (char*)p.out + row_in * (p.out_ld * out_es) + (slab << lanes_log2) * (V * out_es) + (unsigned)(off * (V * out_es));
-    const int64_t out_step = row_stride * p.out_ld * out_es;
+    if constexpr (HELD == HELD_ALL) {
+      if (p.row0.at) { row0_at = operand_at(p.row0, p.row0.dt, false, row_in); row0_step = row_stride * p.row0.row_bytes; }
+      if (p.row1.at) { row1_at = operand_at(p.row1, p.row1.dt, false, row_in); row1_step = row_stride * p.row1.row_bytes; }
+    }
+    const int out_dt = DT >= 0 ? DT : p.out_dt, out_es = out_dt == FRISK_F32 ? 4 : 2;
+    char* out_at = p.out + row_in * p.out_row_bytes + (slab << lanes_log2) * (V * out_es) + (unsigned)(off * (V * out_es));
+    const int64_t out_step = row_stride * p.out_row_bytes;
 
     // what is under way from memory: the next group of 32-bit operands, the next two of 16-bit ones (16 bytes a lane and four waves a SIMD
     // are a third of what the memory's latency asks for: one group ahead 195.2 us for the four calls of cast, mean, scale and shift, softmax on 8192 x 8192 f16, two 191.8)
     constexpr int SETS = (DT == FRISK_F16 || DT == FRISK_BF16) && DEPTH == 1 && UNIFORM_ROW ? 2 : 1;
-    struct Held { Raw head, walk2; unsigned row0, row1; } held0{}, held1{};
+    struct Ahead { Raw head, walk2; unsigned row0, row1; } held0{}, held1{};
     v8f col0{}, col1{};
-    auto fetch_ahead = [&](Held& h) __attribute__((always_inline)) {
-      if (prog.head >= 0) h.head = fetch_at(head_at, type_of(prog.head), true);
-      if constexpr (AHEAD) {
-        if (prog.walk2 >= 0) h.walk2 = fetch_at(walk2_at, type_of(prog.walk2), true);
-        if (prog.row0 >= 0) h.row0 = fetch_row_at(row0_at, row0_dt);
-        if (prog.row1 >= 0) h.row1 = fetch_row_at(row1_at, row1_dt);
+    auto fetch_ahead = [&](Ahead& h) __attribute__((always_inline)) {
+      if (p.head.at) h.head = fetch_at(head_at, type_of(p.head), true);
+      if constexpr (HELD >= HELD_WALK) {
+        if (p.walk2.at) h.walk2 = fetch_at(walk2_at, type_of(p.walk2), true);
+      }
+      if constexpr (HELD == HELD_ALL) {
+        if (p.row0.at) h.row0 = fetch_row_at(row0_at, p.row0.dt);
+        if (p.row1.at) h.row1 = fetch_row_at(row1_at, p.row1.dt);
       }
     };
     int64_t fetched = row;  // row of the last fetch
@@ -247,7 +288,8 @@ template <int DT, bool AHEAD, int DEPTH, bool UNIFORM_ROW> __global__ void __lau
       fetched += row_stride;
       if (fetched < p.rows) {  // (a lane whose next row lies beyond the view fetches the present one again)
         head_at += head_step;
-        if constexpr (AHEAD) { walk2_at += walk2_step; row0_at += row0_step; row1_at += row1_step; }
+        if constexpr (HELD >= HELD_WALK) walk2_at += walk2_step;
+        if constexpr (HELD == HELD_ALL) { row0_at += row0_step; row1_at += row1_step; }
       }
     };
     fetch_ahead(held0);
@@ -257,23 +299,25 @@ template <int DT, bool AHEAD, int DEPTH, bool UNIFORM_ROW> __global__ void __lau
         fetch_ahead(held1);
       }
     }
-    if constexpr (AHEAD) {
-      if (prog.col0 >= 0) to_float(fetch_at(operand_at(prog.col0, p.in_dtype[prog.col0], true, 0), p.in_dtype[prog.col0], false), p.in_dtype[prog.col0], col0);
-      if (prog.col1 >= 0) to_float(fetch_at(operand_at(prog.col1, p.in_dtype[prog.col1], true, 0), p.in_dtype[prog.col1], false), p.in_dtype[prog.col1], col1);
+    if constexpr (HELD == HELD_ALL) {
+      if (p.col0.at) to_float(fetch_at(operand_at(p.col0, p.col0.dt, true, 0), p.col0.dt, false), p.col0.dt, col0);
+      if (p.col1.at) to_float(fetch_at(operand_at(p.col1, p.col1.dt, true, 0), p.col1.dt, false), p.col1.dt, col1);
     }
     int64_t rb = rb0;
     // one group, whose operands are in h; true: it was the last one
-    auto group = [&](Held& h) __attribute__((always_inline)) {
+    auto group = [&](Ahead& h) __attribute__((always_inline)) {
       const bool live = row < p.rows && lane_group < left;
       v8f top, s0, s1, s2, s3, s4, x, walk2;
       asm volatile("" : "=v"(top), "=v"(s0), "=v"(x), "=v"(walk2));  // written by the program before it reads them
       if constexpr (DEPTH > 1) asm volatile("" : "=v"(s1), "=v"(s2), "=v"(s3), "=v"(s4));
       float row_a = 0.f, row_b = 0.f;
-      if (prog.head >= 0) to_float(h.head, type_of(prog.head), top);
-      if constexpr (AHEAD) {
-        if (prog.walk2 >= 0) to_float(h.walk2, type_of(prog.walk2), walk2);
-        if (prog.row0 >= 0) row_a = row_value(row0_dt, h.row0);
-        if (prog.row1 >= 0) row_b = row_value(row1_dt, h.row1);
+      if (p.head.at) to_float(h.head, type_of(p.head), top);
+      if constexpr (HELD >= HELD_WALK) {
+        if (p.walk2.at) to_float(h.walk2, type_of(p.walk2), walk2);
+      }
+      if constexpr (HELD == HELD_ALL) {
+        if (p.row0.at) row_a = row_value(p.row0.dt, h.row0);
+        if (p.row1.at) row_b = row_value(p.row1.dt, h.row1);
       }
       const int64_t here = row < p.rows ? row : p.rows - 1;
       if (rb + SETS * (int64_t)gridDim.y < row_blocks) {
@@ -283,24 +327,28 @@ template <int DT, bool AHEAD, int DEPTH, bool UNIFORM_ROW> __global__ void __lau
       int pc = 0, code = code_reg[0], imm = imm_reg[0];
       for (;;) {
         int step;
-        if constexpr (AHEAD && DEPTH > 1)
-          asm volatile(EW_INTERPRETER : "={s50}"(step), "+{s51}"(pc), "+{v[16:23]}"(top), "+{v[24:31]}"(s0), "+{v[32:39]}"(x), "+{v[64:71]}"(s1), "+{v[72:79]}"(s2),
-                       "+{v[80:87]}"(s3), "+{v[88:95]}"(s4) : "{v12}"(code), "{v13}"(imm), "{v14}"(row_a), "{v15}"(row_b), "{v[40:47]}"(col0), "{v[48:55]}"(col1),
-                       "{v[56:63]}"(walk2) : EW_CLOBBERS);
-        else if constexpr (AHEAD)
-          asm volatile(EW_INTERPRETER : "={s50}"(step), "+{s51}"(pc), "+{v[16:23]}"(top), "+{v[24:31]}"(s0), "+{v[32:39]}"(x) : "{v12}"(code), "{v13}"(imm),
-                       "{v14}"(row_a), "{v15}"(row_b), "{v[40:47]}"(col0), "{v[48:55]}"(col1), "{v[56:63]}"(walk2) : EW_CLOBBERS);
-        else if constexpr (DEPTH > 1)
-          asm volatile(EW_INTERPRETER : "={s50}"(step), "+{s51}"(pc), "+{v[16:23]}"(top), "+{v[24:31]}"(s0), "+{v[32:39]}"(x), "+{v[64:71]}"(s1), "+{v[72:79]}"(s2),
-                       "+{v[80:87]}"(s3), "+{v[88:95]}"(s4) : "{v12}"(code), "{v13}"(imm) : EW_CLOBBERS);
-        else
-          asm volatile(EW_INTERPRETER : "={s50}"(step), "+{s51}"(pc), "+{v[16:23]}"(top), "+{v[24:31]}"(s0), "+{v[32:39]}"(x) : "{v12}"(code), "{v13}"(imm) : EW_CLOBBERS);
+#define EW_RUN(MORE_OUT, IN)                                                                                                                   \
+  asm volatile(EW_INTERPRETER : "={s50}"(step), "+{s51}"(pc), "+{v[16:23]}"(top), "+{v[24:31]}"(s0), "+{v[32:39]}"(x) MORE_OUT                 \
+               : "{v12}"(code), "{v13}"(imm) IN : EW_CLOBBERS)
+#define EW_DEEP , "+{v[64:71]}"(s1), "+{v[72:79]}"(s2), "+{v[80:87]}"(s3), "+{v[88:95]}"(s4)
+#define EW_WALK2 , "{v[56:63]}"(walk2)
+#define EW_BROADCAST , "{v14}"(row_a), "{v15}"(row_b), "{v[40:47]}"(col0), "{v[48:55]}"(col1)
+        if constexpr (HELD == HELD_ALL && DEPTH > 1) EW_RUN(EW_DEEP, EW_BROADCAST EW_WALK2);
+        else if constexpr (HELD == HELD_ALL) EW_RUN(, EW_BROADCAST EW_WALK2);
+        else if constexpr (HELD == HELD_WALK && DEPTH > 1) EW_RUN(EW_DEEP, EW_WALK2);
+        else if constexpr (HELD == HELD_WALK) EW_RUN(, EW_WALK2);
+        else if constexpr (DEPTH > 1) EW_RUN(EW_DEEP, );
+        else EW_RUN(, );
+#undef EW_RUN
+#undef EW_DEEP
+#undef EW_WALK2
+#undef EW_BROADCAST
         const int what = step >> 24;
         if (what == STEP_END) break;
         if (what == STEP_FETCH) {
-          const int k = (step >> 8) & 15;
-          if (p.in_col_stride[k]) to_float(fetch_at(operand_at(k, p.in_dtype[k], true, here), p.in_dtype[k], false), p.in_dtype[k], x);
-          else x = v8f{} + row_value(p.in_dtype[k], fetch_row_at(operand_at(k, p.in_dtype[k], false, here), p.in_dtype[k]));
+          const EwOperand& k = p.in[(step >> 8) & 15];
+          if (k.walks) to_float(fetch_at(operand_at(k, k.dt, true, here), k.dt, false), k.dt, x);
+          else x = v8f{} + row_value(k.dt, fetch_row_at(operand_at(k, k.dt, false, here), k.dt));
         } else if (what == STEP_MORE) {
           code = code_reg[1];
           imm = imm_reg[1];
@@ -323,8 +371,8 @@ template <int DT, bool AHEAD, int DEPTH, bool UNIFORM_ROW> __global__ void __lau
   }
 }
 
-// The postfix program as steps.  `ahead`: inputs may be held in slots (else each mention is fetched where it stands).
-EwSteps steps_of(const EwParams& p, bool ahead) {
+// The postfix program as steps.  `held`: which inputs may be held in slots (each mention of the others is fetched where it stands).
+EwSteps steps_of(const EwParams& p, int held) {
   EwSteps s{};
   s.head = s.walk2 = s.col0 = s.col1 = s.row0 = s.row1 = -1;
   int n = 0, below = -1;  // steps so far, values below the top
@@ -339,6 +387,11 @@ EwSteps steps_of(const EwParams& p, bool ahead) {
   const int by_row[6] = {STEP_ADDR, STEP_SUBR, STEP_MULR, STEP_DIVR, STEP_MAXR, STEP_MINR};
   const int from_below[6] = {STEP_ADDV, STEP_RSUBV, STEP_MULV, STEP_RDIVV, STEP_MAXV, STEP_MINV};  // the value below is the left operand
   bool seen[FRISK_EW_MAX_INPUTS] = {};
+  // with no second operand that moves with the rows, the place of one serves an operand that is the same for every row
+  bool col_as_walk2 = held == HELD_WALK;
+  for (int i = 1; i < p.n_ops; ++i)
+    if (p.op[i] == FRISK_EW_INPUT && p.in_col_stride[p.arg[i]] && (p.in_row_stride[p.arg[i]] || p.in_dtype[p.arg[i]] != p.out_dtype) && p.arg[i] != (p.op[0] == FRISK_EW_INPUT ? p.arg[0] : -1))
+      col_as_walk2 = false;
   for (int i = 0; i < p.n_ops; ++i) {
     const int op = p.op[i];
     if (op == FRISK_EW_INPUT || op == FRISK_EW_CONST) {
@@ -346,11 +399,11 @@ EwSteps steps_of(const EwParams& p, bool ahead) {
       const bool walks = p.in_col_stride[k] != 0;
       if (op == FRISK_EW_INPUT && !seen[k]) {
         seen[k] = true;
+        const bool same_every_row = p.in_row_stride[k] == 0 && p.rows > 1;
         if (i == 0 && walks) s.head = k;
-        else if (!ahead) {}
-        else if (!walks) { if (s.row0 < 0) s.row0 = k; else if (s.row1 < 0) s.row1 = k; }
-        else if (p.in_row_stride[k] == 0 && p.rows > 1) { if (s.col0 < 0) s.col0 = k; else if (s.col1 < 0) s.col1 = k; }
-        else if (s.walk2 < 0) s.walk2 = k;
+        else if (held == HELD_ALL && !walks) { if (s.row0 < 0) s.row0 = k; else if (s.row1 < 0) s.row1 = k; }
+        else if (held == HELD_ALL && same_every_row) { if (s.col0 < 0) s.col0 = k; else if (s.col1 < 0) s.col1 = k; }
+        else if (held != HELD_NONE && walks && s.walk2 < 0 && (!same_every_row || col_as_walk2)) s.walk2 = k;
       }
       const bool fused = next >= FRISK_EW_ADD && next <= FRISK_EW_MIN;  // pushed only to be the right operand of the next step
       if (!fused && ++below > 0) emit(STEP_SAVE, slot_below(below));
@@ -373,48 +426,85 @@ EwSteps steps_of(const EwParams& p, bool ahead) {
     }
   }
   emit(STEP_END);
+  s.n = n;
   return s;
 }
 // two postfix steps make at most four steps (a value saved, fetched, loaded and combined from below)
 static_assert(2 * FRISK_EW_MAX_OPS + 2 <= 2 * kChunk, "a program fits into two chunks");
 
-template <int DT, bool AHEAD> void launch_typed(const dim3& grid, const EwParams& p, const EwSteps& prog, int lanes_log2, hipStream_t s) {
-#define FRISK_EW_LAUNCH(DEPTH)                                                                                                         \
-  if (lanes_log2 >= 6) hipLaunchKernelGGL((elementwise_kernel<DT, AHEAD, DEPTH, true>), grid, dim3(256), 0, s, p, prog, lanes_log2);   \
-  else hipLaunchKernelGGL((elementwise_kernel<DT, AHEAD, DEPTH, false>), grid, dim3(256), 0, s, p, prog, lanes_log2);
-  if (prog.depth <= 1) { FRISK_EW_LAUNCH(1) } else { FRISK_EW_LAUNCH(5) }
+template <int DT, int HELD> void launch_typed(const dim3& grid, const EwArgs& a, int depth, int lanes_log2, hipStream_t s) {
+#define FRISK_EW_LAUNCH(DEPTH)                                                                                                 \
+  if (lanes_log2 >= 6) hipLaunchKernelGGL((elementwise_kernel<DT, HELD, DEPTH, true>), grid, dim3(256), 0, s, a, lanes_log2); \
+  else hipLaunchKernelGGL((elementwise_kernel<DT, HELD, DEPTH, false>), grid, dim3(256), 0, s, a, lanes_log2);
+  if (depth <= 1) { FRISK_EW_LAUNCH(1) } else { FRISK_EW_LAUNCH(5) }
 #undef FRISK_EW_LAUNCH
+}
+template <int DT> void launch_held(int held, const dim3& grid, const EwArgs& a, int depth, int lanes_log2, hipStream_t s) {
+  if (held == HELD_ALL) launch_typed<DT, HELD_ALL>(grid, a, depth, lanes_log2, s);
+  else if (held == HELD_WALK) launch_typed<DT, HELD_WALK>(grid, a, depth, lanes_log2, s);
+  else launch_typed<DT, HELD_NONE>(grid, a, depth, lanes_log2, s);
 }
 
 }  // namespace
 
-hipError_t launch_elementwise(const EwParams& p, hipStream_t s) {
-  // one type for everything that moves with the rows: the kernels for it; mixed types: the one that looks at each operand's type,
-  // which holds nothing ahead but the first operand
-  EwSteps prog = steps_of(p, true);
-  int dt = p.out_dtype;
-  bool ahead = prog.walk2 >= 0 || prog.col0 >= 0 || prog.row0 >= 0;
-  if ((prog.head >= 0 && p.in_dtype[prog.head] != dt) || (prog.walk2 >= 0 && p.in_dtype[prog.walk2] != dt)) {
-    dt = -1;
-    ahead = false;
-    prog = steps_of(p, false);
+hipError_t launch_elementwise(const EwParams& given, hipStream_t s) {
+  EwParams p = given;
+  // A dense view is one row, down which no lane walks and fetches ahead.  A 16-bit one that gives every lane more than one group is folded to
+  // rows of one group a lane (8192 x 8192 f16: log2(max(x, c) / (x + c)) 73.6 -> 69.5 us, x * y + z 95.7 -> 95.4; f32, of which one group less
+  // is under way, lost: 117 -> 119).
+  constexpr int64_t kFold = 256 * V, kCap = 256 * 16;
+  bool half = p.out_dtype != FRISK_F32;
+  for (int k = 0; k < FRISK_EW_MAX_INPUTS; ++k) half = half && (p.in_col_stride[k] == 0 || p.in_dtype[k] == p.out_dtype);
+  if (p.rows == 1 && half && p.cols % kFold == 0 && p.cols / kFold > kCap) {
+    p.rows = p.cols / kFold;
+    p.cols = p.out_ld = kFold;
+    for (int k = 0; k < FRISK_EW_MAX_INPUTS; ++k) p.in_row_stride[k] = p.in_col_stride[k] ? kFold : 0;
   }
   const int64_t groups = (p.cols + V - 1) / V;
   int lanes_log2 = 0;
   while (lanes_log2 < 8 && ((int64_t)1 << lanes_log2) < groups) ++lanes_log2;
   const int64_t lanes = (int64_t)1 << lanes_log2, row_step = 256 >> lanes_log2;
   // enough work-groups to fill the chip several times over, every lane walking its row / column strides beyond that
-  int64_t gx = (groups + lanes - 1) / lanes, gy = (p.rows + row_step - 1) / row_step;
-  const int64_t cap = 256 * 16;
-  if (gx > cap) gx = cap;
-  if (gx * gy > cap) gy = (cap + gx - 1) / gx;
+  const int64_t row_blocks = (p.rows + row_step - 1) / row_step;
+  int64_t gx = (groups + lanes - 1) / lanes, gy = row_blocks;
+  if (gx > kCap) gx = kCap;
+  if (gx * gy > kCap) gy = (kCap + gx - 1) / gx;
   if (gy > 65535) gy = 65535;
+  // Holding the broadcast operands pays where a lane walks down several rows, not where its one group waits for them to be set up (us held / not:
+  // x + b of 1024 x 4096 f16 7.6 / 5.8, f32 9.2 / 8.0, 300 x 77 f16 4.5 / 3.7; (x - s c) g + b of 100000 x 24 f16 8.6 / 6.9)
+  const int most = (row_blocks + gy - 1) / gy >= 2 ? HELD_ALL : HELD_WALK;
+  // one type for everything that moves with the rows: the kernels for it; mixed types: the one that looks at each operand's type,
+  // which holds nothing ahead but the first operand
+  EwSteps prog = steps_of(p, most);
+  int dt = p.out_dtype;
+  int held = prog.col0 >= 0 || prog.row0 >= 0 ? HELD_ALL : prog.walk2 >= 0 ? HELD_WALK : HELD_NONE;
+  // f32 with three groups a lane and more: the larger kernel's four waves a SIMD stream better than five of the smaller one (us, four / five:
+  // x + y of 8192 x 8192 142 / 147, 20000 x 2048 87.6 / 90.5, 4095 x 8191 72.0 / 73.3; 4096 x 4096, two groups a lane, 38.7 / 37.3)
+  if (dt == FRISK_F32 && held == HELD_WALK && ((groups + lanes - 1) / lanes) * row_blocks >= 3 * gx * gy) held = HELD_ALL;
+  if ((prog.head >= 0 && p.in_dtype[prog.head] != dt) || (prog.walk2 >= 0 && p.in_dtype[prog.walk2] != dt)) {
+    dt = -1;
+    held = HELD_NONE;
+    prog = steps_of(p, HELD_NONE);
+  }
+  EwArgs a{};
+  a.rows = p.rows; a.cols = p.cols;
+  a.out = (char*)p.out; a.out_dt = p.out_dtype; a.out_row_bytes = p.out_ld * (p.out_dtype == FRISK_F32 ? 4 : 2);
+  auto operand = [&](int k) {
+    if (k < 0) return EwOperand{};
+    return EwOperand{(const char*)p.in[k], p.in_row_stride[k] * (p.in_dtype[k] == FRISK_F32 ? 4 : 2), p.in_dtype[k], p.in_col_stride[k]};
+  };
+  for (int k = 0; k < FRISK_EW_MAX_INPUTS; ++k) a.in[k] = operand(k);
+  a.head = operand(prog.head); a.walk2 = operand(prog.walk2);
+  a.row0 = operand(prog.row0); a.row1 = operand(prog.row1); a.col0 = operand(prog.col0); a.col1 = operand(prog.col1);
+  a.n_steps = prog.n;
+  __builtin_memcpy(a.code, prog.code, sizeof a.code);
+  __builtin_memcpy(a.imm, prog.imm, sizeof a.imm);
   const dim3 grid((unsigned)gx, (unsigned)gy);
   switch (dt) {
-    case FRISK_F32: if (ahead) launch_typed<FRISK_F32, true>(grid, p, prog, lanes_log2, s); else launch_typed<FRISK_F32, false>(grid, p, prog, lanes_log2, s); break;
-    case FRISK_F16: if (ahead) launch_typed<FRISK_F16, true>(grid, p, prog, lanes_log2, s); else launch_typed<FRISK_F16, false>(grid, p, prog, lanes_log2, s); break;
-    case FRISK_BF16: if (ahead) launch_typed<FRISK_BF16, true>(grid, p, prog, lanes_log2, s); else launch_typed<FRISK_BF16, false>(grid, p, prog, lanes_log2, s); break;
-    default: launch_typed<-1, false>(grid, p, prog, lanes_log2, s); break;
+    case FRISK_F32: launch_held<FRISK_F32>(held, grid, a, prog.depth, lanes_log2, s); break;
+    case FRISK_F16: launch_held<FRISK_F16>(held, grid, a, prog.depth, lanes_log2, s); break;
+    case FRISK_BF16: launch_held<FRISK_BF16>(held, grid, a, prog.depth, lanes_log2, s); break;
+    default: launch_typed<-1, HELD_NONE>(grid, a, prog.depth, lanes_log2, s); break;
   }
   return hipGetLastError();
 }

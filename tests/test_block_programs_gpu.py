@@ -92,3 +92,45 @@ def test_lanes_that_walk_down_several_rows(hip, dt, rows, cols):
     run(hip, prog, ops, dt, rows, cols)
     run(hip, prog, ops, dt, rows, cols, in_place=0)
     run(hip, prog, [(other, "walk", u(rows * cols, 0))] + ops[1:], dt, rows, cols)
+
+
+def on_device(hip, prog, dt, rows, cols, kinds, want, ld=None, in_place=False):
+    """operands of `kinds` (walk, row, col, one) drawn on the device; `want` computes the reference from them in float64"""
+    import torch
+    t = {O.F32: torch.float32, O.F16: torch.float16, O.BF16: torch.bfloat16}[dt]
+    ld = ld or cols
+    g = torch.Generator(device="cuda").manual_seed(104)
+    draw = lambda *shape: (torch.rand(*shape, device="cuda", generator=g) * 1.5 + 0.5).to(t)
+    shape = {"walk": (rows, ld), "row": (rows, 1), "col": (1, cols), "one": (1, 1)}
+    stride = {"walk": (dt, ld, 1), "row": (dt, 1, 0), "col": (dt, 0, 1), "one": (dt, 0, 0)}
+    ops = [draw(*shape[k]) for k in kinds]
+    ref = want(*[o.double()[:, :cols] for o in ops]).expand(rows, cols).clone()
+    out = ops[0] if in_place else torch.full((rows, ld), 7.0, device="cuda", dtype=t)
+    beyond = out[:, cols:].clone()
+    hip.elementwise(hip.make_elementwise_desc(prog, [stride[k] for k in kinds], dt, rows, cols, out_ld=ld), [o.data_ptr() for o in ops], out.data_ptr(),
+                    torch.cuda.current_stream().cuda_stream)
+    err = ((out[:, :cols].double() - ref).abs() / ref.abs().clamp(min=1.0)).max().item()
+    assert err <= TOL[dt] and torch.equal(out[:, cols:], beyond), (prog, rows, cols, err)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", [O.F32, O.F16, O.BF16])
+@pytest.mark.parametrize("rows,cols", [(8200, 520), (2051, 2059)])
+def test_broadcast_operands_held_while_a_lane_walks_down(hip, dt, rows, cols):
+    """every operation on an operand held for the rows a lane walks: one value per row, per column, and one in all (the smaller views above hold none)"""
+    import torch
+    does = {"add": torch.add, "sub": torch.sub, "mul": torch.mul, "div": torch.div, "max": torch.maximum, "min": torch.minimum}
+    for op in BINARY:
+        for kind in ("row", "col", "one"):
+            on_device(hip, [("input", 0), ("input", 1), op], dt, rows, cols, ["walk", kind], does[op], ld=cols + 1)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", [O.F32, O.F16, O.BF16])
+@pytest.mark.parametrize("rows,cols", [(1, 4097 * 2048), (1, 4097 * 2048 - 8), (3073, 8192), (4096, 2048)], ids=["folded", "one_row", "three_groups_a_lane", "one_group_a_lane"])
+def test_dense_views_of_several_groups_a_lane(hip, dt, rows, cols):
+    """dense views just above and below the sizes at which 16-bit ones are folded and f32 ones change kernel; in place too"""
+    gated = [("input", 0), ("input", 1), "mul", ("input", 2), "add"]
+    on_device(hip, gated, dt, rows, cols, ["walk", "walk", "walk"], lambda x, y, z: x * y + z)
+    on_device(hip, [("input", 0), ("input", 1), "add"], dt, rows, cols, ["walk", "walk"], lambda x, y: x + y, in_place=True)
+    on_device(hip, [("input", 0), ("const", 1.0), "add", "log2"], dt, rows, cols, ["walk"], lambda x: (x + 1).log2(), in_place=True)
