@@ -103,6 +103,8 @@ struct EwArgs {
   EW_HANDLER(EW_EACH("v_exp_f32 v[16+\\e], v[16+\\e]") "s_nop 0\n")                                                     \
   EW_HANDLER(EW_EACH("v_log_f32 v[16+\\e], v[16+\\e]") "s_nop 0\n")                                                     \
   ".Lew_out%=:\n"
+// (M0, which the index mode writes, is a reserved register that the compiler refuses among the clobbers: these kernels must have no other use of it,
+// as tests/test_asm_hazards.py checks in their listing)
 #define EW_CLOBBERS "s48", "s49", "s52", "s54", "s55", "s56", "scc"
 
 typedef float v8f __attribute__((ext_vector_type(8)));

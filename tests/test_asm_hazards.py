@@ -128,3 +128,31 @@ def test_attention_kernel_has_no_use_of_m0_besides_its_transfers(tmp_path):
     listing = out.read_text()
     assert listing.count("global_load_lds_dwordx4") >= 4 * 16 and listing.count("v_mfma_f32_32x32x16") >= 4 * 32  # four kernels (f16 / bf16, two K layouts)
     assert foreign_m0_uses(listing) == [] and "scratch_" not in listing
+
+
+def test_the_interpreter_of_block_bodies_declares_every_scalar_register_it_writes():
+    """csrc/elementwise.hip runs its steps in inline assembly: what its scalar instructions write must be an output or a clobber, else the
+    compiler may keep a value there (M0, a reserved register, cannot be declared: the listing is checked below)"""
+    source = open(os.path.join(CSRC, "elementwise.hip")).read()
+    text = source[source.index("#define EW_EACH"):source.index("#define EW_CLOBBERS")].replace("\\n", "\n")
+    written = set("s%s" % r for r in re.findall(r"\bv_readlane_b32 s(\d+)", text))
+    for lo, hi in re.findall(r"\bs_getpc_b64 s\[(\d+):(\d+)\]", text):
+        written.update("s%d" % r for r in range(int(lo), int(hi) + 1))
+    written.update(re.findall(r"\bs_(?:add|addc|addk|lshr|lshl|mov|and|or|sub|subb)\w* (s\d+)", text))
+    assert {"s48", "s49", "s50", "s51", "s52", "s54", "s55", "s56"} <= written
+    clobbers = set(re.findall(r'"(\w+)"', re.search(r"#define EW_CLOBBERS (.*)", source).group(1)))
+    outputs = set(re.findall(r'"[=+]\{(s\d+)\}"', source))
+    assert written <= clobbers | outputs, written - clobbers - outputs
+
+
+@pytest.mark.skipif(not (os.path.exists(HIPCC) or shutil.which("hipcc")), reason="needs hipcc to produce the ISA listing")
+def test_kernels_of_block_bodies_have_no_use_of_m0_besides_the_index_mode(tmp_path):
+    out = tmp_path / "elementwise.s"
+    cmd = [HIPCC if os.path.exists(HIPCC) else "hipcc", "--offload-arch=gfx950", "-O3", "-std=c++17", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+           "-I" + os.path.join(ROOT, "include"), "-I" + CSRC, "-Wno-unused-command-line-argument", "--cuda-device-only", "-S", os.path.join(CSRC, "elementwise.hip"), "-o", str(out)]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-2000:]
+    listing = out.read_text()
+    assert listing.count("s_set_gpr_idx_on") > 28 * 10 and foreign_m0_uses(listing) == [] and "scratch_" not in listing
+    # instructions that read M0 without naming it
+    assert not re.search(r"^\s+(s_movrel|v_movrel|s_sendmsg|ds_gws|ds_append|ds_consume|buffer_load\w* .* lds|global_load_lds)", listing, re.M)
