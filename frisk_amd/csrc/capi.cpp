@@ -193,15 +193,19 @@ static void fill_layout(frisk_lds_layout* L, bool kcontig, int es, int fragb, in
   (void)nw;
 }
 
+// Workspace a plan may use: any (what frisk_hip_plan reports), a limit (splits of K of as many slices as fit; a tail split fits or is dropped), or
+// none.
+static constexpr size_t kAnyWorkspace = ~(size_t)0;
+
 // Tail split: a grid of a little more than a whole number of rounds of 256 tiles leaves most CUs idle in its last round.
 // With a kernel that has the split-K store path, the last tiles % 256 tiles (at most half a round) are computed by 2, 4 or
 // 8 work-groups each, every one taking an equal share of the K tiles (at least 4).  Returns that count, 1 for no split.
-static int tail_split_of(const KernelEntry* k, int64_t tiles, int64_t kt, bool whole_k_tiles) {
+static int tail_split_of(const KernelEntry* k, int64_t tiles, int64_t kt, bool whole_k_tiles, size_t workspace) {
   // the edge kernels deal any number of K tiles: their last slice may be shorter (us unsplit / split: bf16 3000x11008x4096 NT, 516
   // tiles, 248 / 212; fp16 4097x4097x4096 NT, 289 tiles, 161 / 126; 4095x4097x4001 NN with its copy to aligned rows 204 / 150)
   const bool edge = k->edge && !k->splitk && (int64_t)k->bm * k->bn >= 192 * 256;
   if (!edge && (!k->splitk || k->bm < 128 || k->wk > 1 || !whole_k_tiles)) return 1;
-  if (tiles <= 256) return 1;
+  if (tiles <= 256 || workspace == 0) return 1;
   const int64_t rest = tiles % 256;
   if (rest == 0 || rest > 128) return 1;
   // shallower slices do not repay the second launch (measured); the 8-bit kernels run a K tile of twice the depth in the same
@@ -210,7 +214,7 @@ static int tail_split_of(const KernelEntry* k, int64_t tiles, int64_t kt, bool w
   const int min_slice = elem_size(k->dtype) == 1 ? 16 : 8;
   for (int s = 8; s >= 2; s = edge ? s - 1 : s / 2) {
     const int64_t per = (kt + s - 1) / s;
-    if (rest * s <= 256 && (edge ? (s - 1) * per < kt : kt % s == 0) && per >= min_slice) return s;
+    if (rest * s <= 256 && (edge ? (s - 1) * per < kt : kt % s == 0) && per >= min_slice) return (size_t)(s * rest) * k->bm * k->bn * 4 <= workspace ? s : 1;
   }
   return 1;
 }
@@ -224,12 +228,12 @@ static bool edge_slices_ok(const KernelEntry* k, const frisk_gemm_desc* d, int s
   const int64_t kt = (d->K + k->bk - 1) / k->bk, per = (kt + slices - 1) / slices;
   return per >= (elem_size(k->dtype) == 1 ? 16 : 8) && (slices - 1) * per < kt;
 }
-static int edge_split_of(const KernelEntry* k, const frisk_gemm_desc* d) {
+static int edge_split_of(const KernelEntry* k, const frisk_gemm_desc* d, size_t workspace) {
   if (!k->edge || k->splitk || k->wk > 1 || k->bm < 128 || k->dtype == FRISK_F32) return 1;
   const int64_t tiles = ((d->M + k->bm - 1) / k->bm) * ((d->N + k->bn - 1) / k->bn);
   if (tiles > 128 || tiles == 0) return 1;
   for (int s = (int)std::min<int64_t>(8, 256 / tiles); s >= 2; --s)
-    if (edge_slices_ok(k, d, s)) return s;
+    if (edge_slices_ok(k, d, s) && (size_t)(s * tiles) * k->bm * k->bn * 4 <= workspace) return s;
   return 1;
 }
 
@@ -239,10 +243,10 @@ static int edge_split_of(const KernelEntry* k, const frisk_gemm_desc* d) {
 // between 1024^3 and 8192^3 and carry over to the 8-bit types, whose K tiles hold the same number of bytes.
 // the split the planner gives a grid below one round of a variant with the split-K store path: up to one work-group per CU,
 // at least 4 K tiles per slice
-static int sub_round_split(const KernelEntry* k, int64_t tiles, int64_t kt) {
+static int sub_round_split(const KernelEntry* k, const frisk_gemm_desc* d, int64_t tiles, int64_t kt, size_t workspace) {
   int split = 1;
   for (int c = 2; c <= 64 && tiles * c <= 256; ++c)
-    if (kt % c == 0 && kt / c >= std::max(4, k->min_k_tiles)) split = c;
+    if (kt % c == 0 && kt / c >= std::max(4, k->min_k_tiles) && (size_t)c * (size_t)d->M * (size_t)d->N * 4 <= workspace) split = c;
   return split;
 }
 
@@ -250,7 +254,7 @@ static int sub_round_split(const KernelEntry* k, int64_t tiles, int64_t kt) {
 // registers against copy + LDS transfers on 128x128 tiles: 4095x4097x4001 304 / 227, 1999x4099x3001 154 / 100, 1001x999x1003 31 / 21)
 static constexpr double kStagedFactor = 1.6;
 
-static double estimated_cost(const KernelEntry* k, const frisk_gemm_desc* d, bool may_split = false) {
+static double estimated_cost(const KernelEntry* k, const frisk_gemm_desc* d, bool may_split, size_t workspace) {
   const int64_t tiles = ((d->M + k->bm - 1) / k->bm) * ((d->N + k->bn - 1) / k->bn);
   const double kt = (double)((d->K + k->bk - 1) / k->bk);
   double c;  // cost of one K tile with the chip full
@@ -300,15 +304,15 @@ static double estimated_cost(const KernelEntry* k, const frisk_gemm_desc* d, boo
   if (may_split && k->splitk && k->bm >= 128 && tiles < 256 && d->K % k->bk == 0) {
     // below one round with a deep K the planner splits K over the idle CUs (2048x4096x16384 fp16: 128 tiles of 256x256 in 2
     // slices 209.5 us, 256 tiles of 256x128 unsplit 243.6): the slices' K tiles at the fill they reach, plus the summing pass
-    const int cs = sub_round_split(k, tiles, (int64_t)kt);
+    const int cs = sub_round_split(k, d, tiles, (int64_t)kt, workspace);
     // (measured: the slices' loops 8 % above the per-K-tile rate of a long loop, the pass at 256 KiB per tile and slice in 0.07 us;
     // 1024x8192x8192 comes out even with 256x128 tiles unsplit, 123.7 against 123.9 us, and stays unsplit)
     if (cs > 1) return kt / cs * c * (0.6 + 0.4 * rest_fill * cs) * 1.08 + 5.0 + 0.07 * (double)(tiles * cs);
   }
-  if (const int cs = may_split && tiles <= 128 ? edge_split_of(k, d) : 1; cs > 1)
+  if (const int cs = may_split && tiles <= 128 ? edge_split_of(k, d, workspace) : 1; cs > 1)
     return kt / cs * c * (0.6 + 0.4 * rest_fill * cs) * 1.08 + 5.0 + 0.07 * (double)(tiles * cs) * (double)area / (256 * 256);
   double cost = (double)full * kt * c;
-  if (const int ts = (k->edge && !k->splitk && !may_split) ? 1 : tail_split_of(k, tiles, (int64_t)kt, d->K % k->bk == 0); ts > 1) {
+  if (const int ts = (k->edge && !k->splitk && !may_split) ? 1 : tail_split_of(k, tiles, (int64_t)kt, d->K % k->bk == 0, k->edge || workspace ? workspace : kAnyWorkspace); ts > 1) {
     // the last `rest` tiles as ts work-groups each, a ts-th of the K tiles apiece, plus the pass that sums them
     // (a dependent launch, and rest * ts tiles of 32-bit partial sums to read)
     return cost + kt / ts * c * (0.6 + 0.4 * rest_fill * ts) + 5.0 + 0.04 * (double)(rest * ts);
@@ -446,11 +450,11 @@ static double small_grid_time(const SmallGridModel& m, const KernelEntry* k, con
 }
 // the split of a variant: among those the rule admits, the one the model makes fastest; *cost receives its time.  `edges`: edge kernels may
 // be split too
-static int small_grid_split(const KernelEntry* k, const frisk_gemm_desc* d, bool no_split, bool edges, double* cost = nullptr) {
+static int small_grid_split(const KernelEntry* k, const frisk_gemm_desc* d, size_t workspace, bool edges, double* cost = nullptr) {
   const SmallGridModel& m = small_grid_model(k);
   int best = 1;
   double best_t = small_grid_time(m, k, d, 1);
-  if (k->splitk && !no_split && d->split_k != 1 && m.w != 0 && d->K % k->bk == 0) {
+  if (k->splitk && workspace && d->split_k != 1 && m.w != 0 && d->K % k->bk == 0) {
     const int64_t tiles = ((d->M + k->bm - 1) / k->bm) * ((d->N + k->bn - 1) / k->bn), kt = d->K / k->bk;
     // any divisor of the K tiles (K = 5760 is 45 tiles of 128: the powers of two left it unsplit); the sweeps behind the tables: up to 64
     // slices, fp32 32
@@ -465,13 +469,13 @@ static int small_grid_split(const KernelEntry* k, const frisk_gemm_desc* d, bool
     const int kmin = std::max(named ? m.kmin : std::min(m.kmin, 4), k->min_k_tiles);
     const int64_t most = std::min<int64_t>({k->dtype == FRISK_F32 ? 32 : 64, tiles > 0 ? wgs / tiles : 0, kt / kmin});
     for (int c = 2; c <= most; ++c)
-      if (kt % c == 0) {
+      if (kt % c == 0 && (size_t)c * (size_t)d->M * (size_t)d->N * 4 <= workspace) {
         const double t = small_grid_time(m, k, d, c);
         if (t < best_t) { best = c; best_t = t; }
       }
   }
   // the edge kernels: slices of unequal length, whole tiles of partial sums
-  if (const int most = edges ? edge_split_of(k, d) : 1; most > 1)
+  if (const int most = edges ? edge_split_of(k, d, workspace) : 1; most > 1)
     for (int c = 2; c <= most; ++c)
       if (edge_slices_ok(k, d, c)) {
         const double t = small_grid_time(m, k, d, c);
@@ -480,9 +484,9 @@ static int small_grid_split(const KernelEntry* k, const frisk_gemm_desc* d, bool
   if (cost) *cost = best_t;
   return best;
 }
-static double small_grid_cost(const KernelEntry* k, const frisk_gemm_desc* d, bool no_split, bool edges) {
+static double small_grid_cost(const KernelEntry* k, const frisk_gemm_desc* d, size_t workspace, bool edges) {
   double t = 0.0;
-  small_grid_split(k, d, no_split, edges, &t);
+  small_grid_split(k, d, workspace, edges, &t);
   return t;
 }
 
@@ -494,8 +498,8 @@ static double small_grid_cost(const KernelEntry* k, const frisk_gemm_desc* d, bo
 static bool planners_own(const KernelEntry* k) { return k->edge && !k->splitk && (k->bm == 192 || k->wk > 1); }
 
 // What a launch knows beyond the descriptor: pointers off 16-byte boundaries (C: or a column-scale pointer off its vector), and
-// whether there is a workspace to use.
-struct PlanContext { bool a_off = false, b_off = false, c_off = false, no_workspace = false; };
+// how much workspace there is to use.
+struct PlanContext { bool a_off = false, b_off = false, c_off = false; size_t workspace = kAnyWorkspace; };
 // Operands that are copied to aligned rows in the workspace before the product runs, and where they go.
 struct Repack { bool a = false, b = false; int64_t lda = 0, ldb = 0; size_t b_offset = 0, bytes = 0; };
 // What a launch needs of a plan beyond the public structure: the copies, and the tail split of an edge kernel (whose slices may
@@ -515,7 +519,7 @@ static Repack repack_of(const frisk_gemm_desc* d, bool a, bool b) {
 }
 
 static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_model, const PlanContext& ctx = {}, LaunchExtras* extras = nullptr) {
-  const bool no_split = ctx.no_workspace;
+  const bool no_split = ctx.workspace == 0;
   int st = validate(d);
   if (st != FRISK_OK) return st;
   if (!plan) return fail(FRISK_ERR_NULL, "plan is null");
@@ -542,6 +546,11 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
   const bool any_layout = !list.empty(), tile_requested = d->tile_m || d->tile_n || d->tile_k || d->waves_m || d->waves_n || d->stages || d->atom;
   const bool small = small_grid(d);
   bool split_edges = false;
+  // what the partial sums of a kernel may take of the workspace: all of it, or what lies behind the copies it works on
+  auto left_for_sums = [&](const KernelEntry* k) {
+    const size_t copies = k->guard == 2 && packed.bytes ? (packed.bytes + 255) & ~(size_t)255 : 0;
+    return ctx.workspace == kAnyWorkspace ? kAnyWorkspace : ctx.workspace > copies ? ctx.workspace - copies : 0;
+  };
   auto search = [&](bool want_split) {
     for (const Variant& v : list) {
       const KernelEntry* k = v.k;
@@ -571,7 +580,7 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
       // the edge kernels once more under their guarded names: K off the K tile (a whole number of chunks), and anything at all,
       // with A and B copied to aligned rows where theirs are not
       if (k->guard == 1 && k->edge && (!rows_aligned || d->K % (16 / es))) continue;
-      if (k->guard == 2 && packed.bytes && (no_split || d->split_k != 0)) continue;
+      if (k->guard == 2 && packed.bytes && (packed.bytes > ctx.workspace || d->split_k != 0)) continue;
       // ... and address a tile's chunks by 32-bit lane offsets from its first row: the stored rows of one tile must span
       // less than 4 GiB
       const double span_a = (double)(packed.a ? packed.lda : d->lda) * es * (d->transA ? k->bk : k->bm),
@@ -579,7 +588,8 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
       if ((!k->guard || k->edge) && (span_a >= 4294967296.0 || span_b >= 4294967296.0)) continue;
       // never a guarded kernel when a fast one fits -- except those, which run at their full rate whatever their name
       if (k->guard && !planners_own(k) && best >= 0 && !ks[best]->guard) continue;
-      double cost = small && !want_split ? small_grid_cost(k, d, no_split, split_edges) : estimated_cost(k, d, !want_split && !no_split && d->split_k == 0);
+      const size_t left = left_for_sums(k);
+      double cost = small && !want_split ? small_grid_cost(k, d, left, split_edges) : estimated_cost(k, d, !want_split && left > 0 && d->split_k == 0, left);
       // (a 32-row edge tile above 64 rows streams B once per 32 rows where the 64-row tile wastes at most as much: 130x11008x4096
       // NT 64.5 against 53.5 us)
       if (k->edge && k->bm == 32 && d->M > 64 && !d->tile_m) continue;
@@ -602,7 +612,7 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
   if (best < 0 && explicit_split) search(false);
   // A small grid that falls to a kernel without the split-K store path looks at split edge kernels as well.  (The sweeps behind the tables held none, and beside the
   // split-K kernels the tables flatter them: fp16 100x4096x4096 NN 20.6 us so, 16.8 on 64x128 tiles in 4 slices.)
-  if (small && best >= 0 && !no_split && d->split_k == 0 && !ks[best]->splitk && small_grid_split(ks[best], d, no_split, false) == 1) {
+  if (small && best >= 0 && !no_split && d->split_k == 0 && !ks[best]->splitk && small_grid_split(ks[best], d, left_for_sums(ks[best]), false) == 1) {
     split_edges = true;
     search(false);
   }
@@ -647,7 +657,8 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
   if (k->edge && !k->splitk && !no_split && d->split_k == 0) {
     const int64_t edge_tiles = (int64_t)plan->grid_x * plan->grid_y;
     const bool half_round = edge_tiles <= 128;
-    const int ts = !half_round ? tail_split_of(k, edge_tiles, (d->K + k->bk - 1) / k->bk, false) : small ? small_grid_split(k, d, no_split, split_edges) : edge_split_of(k, d);
+    const size_t left = left_for_sums(k);
+    const int ts = !half_round ? tail_split_of(k, edge_tiles, (d->K + k->bk - 1) / k->bk, false, left) : small ? small_grid_split(k, d, left, split_edges) : edge_split_of(k, d, left);
     if (ts > 1) {
       const int64_t split_tiles = half_round ? edge_tiles : edge_tiles % 256;
       const size_t offset = (plan->workspace_bytes + 255) & ~(size_t)255;
@@ -666,11 +677,11 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
         return fail(FRISK_ERR_TILE, "split_k=%d leaves %lld K tiles per slice, the chosen kernel %s needs %d", d->split_k, (long long)(kt / d->split_k), k->name, k->min_k_tiles);
       split = d->split_k;
     } else if (small) {
-      split = small_grid_split(k, d, no_split, false);
+      split = small_grid_split(k, d, ctx.workspace, false);
     } else if (d->split_k == 0 && tiles < 256) {
-      split = sub_round_split(k, tiles, kt);
+      split = sub_round_split(k, d, tiles, kt, ctx.workspace);
     } else if (d->split_k == 0) {
-      const int ts = tail_split_of(k, tiles, kt, true);
+      const int ts = tail_split_of(k, tiles, kt, true, ctx.workspace);
       if (ts > 1) {
         plan->tail_split = ts;
         plan->tail_tiles = (int)(tiles % 256);
@@ -764,11 +775,11 @@ int frisk_hip_gemm(const frisk_gemm_desc* desc, const void* A, const void* B, vo
     return fail(FRISK_ERR_ALIGNMENT, "pointers must be aligned to their element size");
   const bool ws_aligned = ((uintptr_t)workspace & 15) == 0;
   if (plan.workspace_bytes > 0 && (!workspace || workspace_bytes < plan.workspace_bytes || (!ws_aligned && desc->split_k <= 1))) {
-    // an explicit split_k needs its workspace; the planner's own choice degrades to a single pass without one it can use, be it
-    // missing, too small or off 16-byte boundaries: a caller cannot know which sizes the planner splits
+    // an explicit split_k needs its workspace; the planner's own choice takes the splits that fit the one there is, and one pass without one it can
+    // use, be it missing or off 16-byte boundaries: a caller cannot know which sizes the planner splits
     if (desc->split_k > 1) return fail(FRISK_ERR_WORKSPACE, "split_k=%d needs %zu bytes of workspace", desc->split_k, plan.workspace_bytes);
     const size_t wanted = plan.workspace_bytes;
-    ctx.no_workspace = true;
+    ctx.workspace = workspace && ws_aligned ? workspace_bytes : 0;
     extras = LaunchExtras{};
     st = make_plan(desc, &plan, false, ctx, &extras);
     // a tile or wave policy that the caller named and that only kernels without staging through registers have: they want the copies
@@ -831,14 +842,17 @@ int frisk_hip_gemm_static_ws(const frisk_gemm_desc* desc, const void* A, const v
   frisk_gemm_plan plan;
   int st = make_plan(desc, &plan, false);
   if (st != FRISK_OK) return st;
-  // What does not fit the array: an explicit split_k is refused (the caller asked for exactly that split); a split the
-  // planner chose by itself (tail splits of large grids reach 64 MiB) is dropped, and the launch runs as one pass, which
-  // is what frisk_hip_gemm does for the same descriptor without a workspace.
+  // What does not fit the array: an explicit split_k is refused (the caller asked for exactly that split), and so is a named tile that runs on copies
+  // larger than it; of the splits the planner chooses by itself it takes those that fit (a split of K of fewer slices; no tail split: those of
+  // large grids reach 64 MiB).
   if (plan.workspace_bytes > (size_t)FRISK_HIP_STATIC_WS_BYTES) {
     if (desc->split_k > 1)
       return fail(FRISK_ERR_WORKSPACE, "split_k=%d needs %zu bytes of partial sums, the static workspace holds %zu: pass a smaller split_k, or use frisk_hip_gemm with a workspace",
                   desc->split_k, plan.workspace_bytes, (size_t)FRISK_HIP_STATIC_WS_BYTES);
-    return frisk_hip_gemm(desc, A, B, C, scaleA, scaleB, nullptr, 0, stream);
+    PlanContext limited;
+    limited.workspace = FRISK_HIP_STATIC_WS_BYTES;
+    st = make_plan(desc, &plan, false, limited);
+    if (st != FRISK_OK || plan.workspace_bytes == 0) return frisk_hip_gemm(desc, A, B, C, scaleA, scaleB, nullptr, 0, stream);
   }
   void* ws = nullptr;
   if (plan.workspace_bytes > 0) {

@@ -160,20 +160,26 @@ size_t frisk_hip_workspace_bytes(const frisk_gemm_desc* desc);
 /* Launch on `stream` (a hipStream_t, may be NULL for the default stream).
  * A, B, C, scaleA, scaleB, workspace are device pointers.  scaleA/scaleB are
  * fp32: M and N entries for ROW_COL_SCALE, one entry each for TENSOR_SCALE.
- * A workspace that is too small or not 16-byte aligned is an error with split_k > 1 and not used otherwise. */
+ * With split_k > 1 a workspace that is too small or not 16-byte aligned is an error.  Otherwise one off 16-byte boundaries is not used, and of one that
+ * is smaller than frisk_hip_workspace_bytes says what fits it: a split of K of fewer slices, copies without a split, or nothing. */
 int frisk_hip_gemm(const frisk_gemm_desc* desc, const void* A, const void* B, void* C, const float* scaleA,
                    const float* scaleB, void* workspace, size_t workspace_bytes, void* stream);
 
 /* frisk_hip_gemm for callers that cannot allocate device memory (code under HIP graph capture, tight serving loops,
- * harnesses that forbid hipMalloc) and therefore have no workspace to pass.  No counterpart in the reference.  The
- * partial sums of a split-K or tail-split plan go to a fixed array of FRISK_HIP_STATIC_WS_BYTES that lives in the
+ * harnesses that forbid hipMalloc) and therefore have no workspace to pass.  No counterpart in the reference.  What
+ * frisk_hip_gemm keeps in its workspace -- the partial sums of split plans, and copies of operands whose rows or
+ * pointers lie off 16-byte boundaries -- goes to a fixed array of FRISK_HIP_STATIC_WS_BYTES that lives in the
  * library's device image (one copy per GPU, held until the process ends); neither this call nor anything it calls
  * allocates or frees.  (The HIP runtime places a device image on a GPU when it is first used there, which takes device
- * memory once: call frisk_hip_init() on each GPU beforehand and that has happened before the first launch.)  Same planner, kernels and results as frisk_hip_gemm with a large enough workspace, with two
- * exceptions for plans that need more than the array holds: an explicit split_k > 1 in the descriptor is refused with
- * FRISK_ERR_WORKSPACE, and a split the planner chose itself (split_k = 0: the tail split of a large grid can want
- * 64 MiB) is dropped, the launch running as a single pass exactly as frisk_hip_gemm does without a workspace.  All calls on one GPU share the array: calls that may overlap on that GPU (different streams,
- * different host threads) race on it and must be serialised by the caller; calls on one stream are ordered. */
+ * memory once: call frisk_hip_init() on each GPU beforehand and that has happened before the first launch.)  Same
+ * planner, kernels and results as frisk_hip_gemm with a workspace of that size: an explicit split_k > 1 that needs
+ * more is refused with FRISK_ERR_WORKSPACE, and so is a named tile that runs on copies larger than the array; of a
+ * split the planner chooses itself (split_k = 0) as many slices are made as fit, and a tail split that does not fit
+ * (that of a large grid can want 64 MiB) is dropped.  All calls on one GPU share the array: calls that may overlap on
+ * that GPU (different streams, different host threads) race on it and must be serialised by the caller; calls on one
+ * stream are ordered.  A call uses the array exactly if frisk_hip_workspace_bytes of its descriptor is not 0 --
+ * which sizes those are changes with the planner -- so a caller that cannot serialise asks, or passes split_k = 1:
+ * such a call never does. */
 #define FRISK_HIP_STATIC_WS_BYTES (32u << 20)
 size_t frisk_hip_static_workspace_bytes(void);
 int frisk_hip_gemm_static_ws(const frisk_gemm_desc* desc, const void* A, const void* B, void* C, const float* scaleA,

@@ -433,7 +433,7 @@ def test_a_plan_that_needs_copies_says_so_at_the_launch(kw):
             launch(d, base, base * 2, base * 3, **dict(zip(("workspace_ptr", "workspace_bytes"), ws)))
         return R.STATUS_NAMES[e.value.status], str(e.value)
 
-    for ws in ((), (base * 4, need - 1), (base * 4 + 4, need)):
+    for ws in ((), (base * 4, 2 * (M + N) * 1008 - 1), (base * 4 + 4, need)):  # (one that holds the copies but not the sums of a split will do)
         what, message = status(R.gemm, *ws)
         assert what == "ERR_WORKSPACE" and str(need) in message, (ws, what, message)
     assert status(R.gemm, base * 4, need)[0] == "ERR_DEVICE"  # everything in order but the GPU

@@ -101,3 +101,30 @@ def test_static_workspace_refuses_what_does_not_fit(hip):
     with pytest.raises(hip.FriskHipError) as e:
         hip.gemm_static_ws(d, 256, 256, 256, None, None, None)  # refused before any pointer is looked at
     assert e.value.status == hip.ERR_WORKSPACE and "static workspace" in str(e.value)
+
+
+@pytest.mark.parametrize("dtype,M,N,K,transA,transB", [(O.F32, 416, 2048, 11904, 0, 1), (O.F16, 256, 5888, 16000, 1, 0)])
+def test_split_of_more_slices_than_the_array_holds_runs_with_fewer(hip, dtype, M, N, K, transA, transB):
+    """the split the planner likes best wants 39 and 57 MiB: the call runs the best split that fits, not one pass"""
+    import torch
+    d = hip.make_desc(dtype, M, N, K, transA=bool(transA), transB=bool(transB))
+    p = hip.plan(d)
+    assert p.split_k > 1 and p.workspace_bytes > hip.static_workspace_bytes()
+    g = torch.Generator(device="cuda").manual_seed(53)
+    t = {O.F32: torch.float32, O.F16: torch.float16}[dtype]
+    A = torch.randn((K, M) if transA else (M, K), device="cuda", generator=g).to(t)
+    B = torch.randn((N, K) if transB else (K, N), device="cuda", generator=g).to(t)
+    stream, out = torch.cuda.current_stream().cuda_stream, []
+    ws = torch.empty(hip.static_workspace_bytes(), dtype=torch.uint8, device="cuda")
+    for run in (lambda C: hip.gemm_static_ws(d, A.data_ptr(), B.data_ptr(), C.data_ptr(), None, None, stream),
+                lambda C: hip.gemm(d, A.data_ptr(), B.data_ptr(), C.data_ptr(), None, None, ws.data_ptr(), ws.numel(), stream),
+                lambda C: hip.gemm(d, A.data_ptr(), B.data_ptr(), C.data_ptr(), None, None, None, 0, stream)):
+        C = torch.zeros(M, N, device="cuda", dtype=t)
+        run(C)
+        out.append(C)
+    static, with_32_mib, one_pass = out
+    assert torch.equal(static, with_32_mib)
+    assert not torch.equal(static, one_pass), "ran as one pass"  # the slices' sums round in another order
+    exact = (A.t() if transA else A).double() @ (B.t() if transB else B).double()
+    tol = 1e-4 if dtype == O.F32 else 1e-2
+    assert float((static.double() - exact).norm() / exact.norm()) <= tol
