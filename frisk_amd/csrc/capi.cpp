@@ -254,7 +254,7 @@ static int sub_round_split(const KernelEntry* k, const frisk_gemm_desc* d, int64
 // registers against copy + LDS transfers on 128x128 tiles: 4095x4097x4001 304 / 227, 1999x4099x3001 154 / 100, 1001x999x1003 31 / 21)
 static constexpr double kStagedFactor = 1.6;
 
-static double estimated_cost(const KernelEntry* k, const frisk_gemm_desc* d, bool may_split, size_t workspace) {
+static double estimated_cost(const KernelEntry* k, const frisk_gemm_desc* d, bool may_split, bool split_edges, size_t workspace) {
   const int64_t tiles = ((d->M + k->bm - 1) / k->bm) * ((d->N + k->bn - 1) / k->bn);
   const double kt = (double)((d->K + k->bk - 1) / k->bk);
   double c;  // cost of one K tile with the chip full
@@ -309,20 +309,27 @@ static double estimated_cost(const KernelEntry* k, const frisk_gemm_desc* d, boo
     // 1024x8192x8192 comes out even with 256x128 tiles unsplit, 123.7 against 123.9 us, and stays unsplit)
     if (cs > 1) return kt / cs * c * (0.6 + 0.4 * rest_fill * cs) * 1.08 + 5.0 + 0.07 * (double)(tiles * cs);
   }
-  if (const int cs = may_split && tiles <= 128 ? edge_split_of(k, d, workspace) : 1; cs > 1)
-    return kt / cs * c * (0.6 + 0.4 * rest_fill * cs) * 1.08 + 5.0 + 0.07 * (double)(tiles * cs) * (double)area / (256 * 256);
   double cost = (double)full * kt * c;
-  if (const int ts = (k->edge && !k->splitk && !may_split) ? 1 : tail_split_of(k, tiles, (int64_t)kt, d->K % k->bk == 0, k->edge || workspace ? workspace : kAnyWorkspace); ts > 1) {
-    // the last `rest` tiles as ts work-groups each, a ts-th of the K tiles apiece, plus the pass that sums them
-    // (a dependent launch, and rest * ts tiles of 32-bit partial sums to read)
-    return cost + kt / ts * c * (0.6 + 0.4 * rest_fill * ts) + 5.0 + 0.04 * (double)(rest * ts);
-  }
   if (rest) {
     if (k->bm == 32)  // the skinny kernels are bound by streaming B and need the parallelism: idle CUs are lost bandwidth
       cost += full ? kt * c : kt * c / std::max(rest_fill, 0.25);
     else
       cost += kt * c * (0.6 + 0.4 * rest_fill);
   }
+  // the last `rest` tiles as ts work-groups each, a ts-th of the K tiles apiece, plus the pass that sums them
+  // (a dependent launch, and rest * ts tiles of 32-bit partial sums to read)
+  auto tail_cost = [&](int ts) { return (double)full * kt * c + kt / ts * c * (0.6 + 0.4 * rest_fill * ts) + 5.0 + 0.04 * (double)(rest * ts); };
+  if (k->edge && !k->splitk) {
+    if (!may_split || !split_edges) return cost;
+    // at most what one pass costs; but rows that end off a K tile slow a pass of many K tiles more than this knows (bf16 4099x3857x1976 TN, us in
+    // one pass / split: 88.8 / 74.9; at K = 1984 89.6 / 77.3)
+    const double one_pass = d->K % k->bk == 0 ? cost : INFINITY;
+    if (const int cs = tiles <= 128 ? edge_split_of(k, d, workspace) : 1; cs > 1)
+      return std::min(one_pass, kt / cs * c * (0.6 + 0.4 * rest_fill * cs) * 1.08 + 5.0 + 0.07 * (double)(tiles * cs) * (double)area / (256 * 256));
+    const int ts = tail_split_of(k, tiles, (int64_t)kt, false, workspace);
+    return ts > 1 ? std::min(one_pass, tail_cost(ts)) : cost;
+  }
+  if (const int ts = tail_split_of(k, tiles, (int64_t)kt, d->K % k->bk == 0, workspace ? workspace : kAnyWorkspace); ts > 1) return tail_cost(ts);
   return cost;
 }
 
@@ -497,6 +504,33 @@ static double small_grid_cost(const KernelEntry* k, const frisk_gemm_desc* d, si
 // (K a half K tile over) 33.6 / 27.8, 19.6 / 17.0, 19.1 / 16.9; 33x4096x2048 15.5 / 7.1, 7.2 / 6.8, 6.6 / 5.2; 40x11008x4096 fp16 28.5 / 28.7
 static bool planners_own(const KernelEntry* k) { return k->edge && !k->splitk && (k->bm == 192 || k->wk > 1); }
 
+// What rounds of large tiles take, in microseconds: start + whole rounds of `cap` work-groups x (round + K tiles x tk) + a last one at round + K tiles x
+// tk x (part + (1 - part) x fill).  `round` is what a round costs beside its K loop (first transfers, stores): 3 us for two 128x128 tiles a CU, 9 for
+// a 256x256 one, which is why the larger tiles need a deep K.  Fitted to 1100 problems of 257 to 2200 tiles of 128x128, K 256 to 8192, operands in
+// rotation (standard deviation 3 to 8 %).
+struct RoundModel { int cap; float start, round, tk, part; };
+static const RoundModel* round_model(const KernelEntry* k) {
+  static const RoundModel edge[2][3] = {{{512, 2.8f, 2.8f, 0.95f, 0.38f}, {256, 0.8f, 7.3f, 1.00f, 0.64f}, {256, 1.1f, 8.7f, 1.33f, 0.61f}},    // 16-bit: 128x128, 192x256, 256x256
+                                        {{512, 3.1f, 3.25f, 1.00f, 0.46f}, {256, 1.5f, 9.0f, 1.00f, 0.63f}, {256, 1.7f, 11.6f, 1.31f, 0.59f}}};  // 8-bit
+  static const RoundModel plain[2][3] = {{{512, 1.3f, 2.3f, 1.02f, 0.33f}, {256, 1.8f, 1.7f, 0.53f, 0.60f}, {256, 2.2f, 2.6f, 0.91f, 0.56f}},   // 128x128 in rings of 2 and 3, 256x128 and 128x256
+                                         {{512, 1.7f, 1.1f, 1.04f, 0.46f}, {256, 1.8f, 1.7f, 0.53f, 0.62f}, {256, 2.4f, 2.4f, 0.85f, 0.50f}}};
+  const int es = elem_size(k->dtype), area = k->bm * k->bn;
+  if (es == 4 || k->bm < 128 || k->bn < 128 || k->wk > 1 || k->wm * k->wn != 4) return nullptr;
+  if (k->edge && !k->splitk) return &edge[es == 1][area == 128 * 128 ? 0 : k->bm == 192 ? 1 : 2];
+  if (k->edge || k->guard || area == 256 * 256) return nullptr;
+  return &plain[es == 1][area == 128 * 128 ? (k->stages >= 3 ? 1 : 0) : 2];
+}
+// `slices` > 1: every tile (up to half a round of them) or those behind the whole rounds split along K, and the pass that sums them
+static double round_time(const RoundModel& m, const KernelEntry* k, const frisk_gemm_desc* d, int slices) {
+  const int64_t tiles = ((d->M + k->bm - 1) / k->bm) * ((d->N + k->bn - 1) / k->bn), kt = (d->K + k->bk - 1) / k->bk;
+  const int64_t split = slices <= 1 ? 0 : tiles <= 128 ? tiles : tiles % 256, plain = tiles - split, full = plain / m.cap, last = plain % m.cap + split * slices;
+  const double k_last = split ? (double)((kt + slices - 1) / slices) : (double)kt;
+  double t = m.start + (double)full * (m.round + (double)kt * m.tk);
+  if (last) t += m.round + k_last * m.tk * (m.part + (1.0 - m.part) * (double)last / m.cap);
+  if (split) t += 3.5 + 0.25 * (double)(split * slices) * k->bm * k->bn * 4.0 / 1e6;
+  return t;
+}
+
 // What a launch knows beyond the descriptor: pointers off 16-byte boundaries (C: or a column-scale pointer off its vector), and
 // how much workspace there is to use.
 struct PlanContext { bool a_off = false, b_off = false, c_off = false; size_t workspace = kAnyWorkspace; };
@@ -545,7 +579,7 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
   bool policy_excluded = false;
   const bool any_layout = !list.empty(), tile_requested = d->tile_m || d->tile_n || d->tile_k || d->waves_m || d->waves_n || d->stages || d->atom;
   const bool small = small_grid(d);
-  bool split_edges = false;
+  bool split_edges = false, settled = false;  // settled: without the 192x256 tile and without splits of edge tiles
   // what the partial sums of a kernel may take of the workspace: all of it, or what lies behind the copies it works on
   auto left_for_sums = [&](const KernelEntry* k) {
     const size_t copies = k->guard == 2 && packed.bytes ? (packed.bytes + 255) & ~(size_t)255 : 0;
@@ -576,7 +610,7 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
       // (whole 256x256 tiles keep the default kernel: which one they run on is part of the planner's interface, though 144 of them
       // leave CUs idle -- fp16 3072x3072x4096 NN 70.6 us, 62.4 on 192x256 tiles)
       const bool whole_256 = rows_aligned && d->M % 256 == 0 && d->N % 256 == 0 && d->K % k->bk == 0;
-      if (planners_own(k) && (tile_requested || d->split_k > 1 || (k->bm == 192 ? small || whole_256 : d->M > 64))) continue;
+      if (planners_own(k) && (tile_requested || d->split_k > 1 || (k->bm == 192 ? small || whole_256 || settled : d->M > 64))) continue;
       // the edge kernels once more under their guarded names: K off the K tile (a whole number of chunks), and anything at all,
       // with A and B copied to aligned rows where theirs are not
       if (k->guard == 1 && k->edge && (!rows_aligned || d->K % (16 / es))) continue;
@@ -589,7 +623,7 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
       // never a guarded kernel when a fast one fits -- except those, which run at their full rate whatever their name
       if (k->guard && !planners_own(k) && best >= 0 && !ks[best]->guard) continue;
       const size_t left = left_for_sums(k);
-      double cost = small && !want_split ? small_grid_cost(k, d, left, split_edges) : estimated_cost(k, d, !want_split && left > 0 && d->split_k == 0, left);
+      double cost = small && !want_split ? small_grid_cost(k, d, left, split_edges) : estimated_cost(k, d, !want_split && left > 0 && d->split_k == 0, !settled, left);
       // (a 32-row edge tile above 64 rows streams B once per 32 rows where the 64-row tile wastes at most as much: 130x11008x4096
       // NT 64.5 against 53.5 us)
       if (k->edge && k->bm == 32 && d->M > 64 && !d->tile_m) continue;
@@ -610,11 +644,45 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
   const bool explicit_split = d->split_k > 1 && !no_split;
   search(explicit_split);
   if (best < 0 && explicit_split) search(false);
-  // A small grid that falls to a kernel without the split-K store path looks at split edge kernels as well.  (The sweeps behind the tables held none, and beside the
-  // split-K kernels the tables flatter them: fp16 100x4096x4096 NN 20.6 us so, 16.8 on 64x128 tiles in 4 slices.)
-  if (small && best >= 0 && !no_split && d->split_k == 0 && !ks[best]->splitk && small_grid_split(ks[best], d, left_for_sums(ks[best]), false) == 1) {
+  // A small grid that falls to a kernel without the split-K store path looks at split edge kernels as well, where K is deep enough to split at
+  // all.  (The sweeps behind the tables held none, and beside the split-K kernels the tables flatter them: fp16 100x4096x4096 NN 20.6 us so, 16.8 on 64x128 tiles in 4 slices.)
+  if (small && best >= 0 && !no_split && d->split_k == 0 && es < 4 && d->K > (es == 1 ? 16 * 128 : 8 * 64) && !ks[best]->splitk && small_grid_split(ks[best], d, left_for_sums(ks[best]), false) == 1) {
     split_edges = true;
     search(false);
+  }
+  // slices of the chosen kernel where it is an edge kernel: of its tiles on grids of up to half a round, of the last ones beyond
+  auto edge_slices = [&]() {
+    const KernelEntry* k = ks[best];
+    if (!k->edge || k->splitk || no_split || d->split_k != 0 || settled) return 1;
+    const int64_t tiles = ((d->M + k->bm - 1) / k->bm) * ((d->N + k->bn - 1) / k->bn);
+    const size_t left = left_for_sums(k);
+    return tiles > 128 ? tail_split_of(k, tiles, (d->K + k->bk - 1) / k->bk, false, left) : small ? small_grid_split(k, d, left, split_edges) : edge_split_of(k, d, left);
+  };
+  // The 192x256 tile and split edge tiles against what a problem of whole K tiles and aligned rows runs on otherwise, 128x128 and 256x256 tiles in one
+  // pass at their full rate: the costs above come out a few per cent apart there, closer than they are accurate, so the model of rounds must see a
+  // gain too, of 4 % where the tile is another one.  us in one pass / so: bf16 2496x1664x3584 NN (260 tiles of 128x128) 39.8 / 44.1,
+  // fp16 1500x2816x3008 NN 34.3 / 39.9, int8 1728x4480x640 NN 13.0 / 15.5, 6464x960x2560 NN 24.2 / 28.0.  Of 301 other
+  // problems of 257 to 2200 tiles 144 were slower by 3 % and more on the route of the costs alone and 1 (int8 5952x1024x8192 NT, 59.2 / 61.9) with this
+  // rule, which keeps 111 of 135 gains beyond 3 % (of those it leaves, f16 1856x4288x4736 NT, 82 / 69, is the largest).
+  if (best >= 0 && rows_aligned && d->K % ks[best]->bk == 0 && round_model(ks[best])) {
+    const int fresh = best, slices = edge_slices();
+    if (slices > 1 || ks[fresh]->bm == 192) {
+      const bool edges_were_split = split_edges;
+      const double fresh_time = round_time(*round_model(ks[fresh]), ks[fresh], d, slices);
+      best = -1;
+      settled = true;
+      split_edges = false;
+      search(false);
+      const KernelEntry* k = best >= 0 ? ks[best] : nullptr;
+      const RoundModel* m = k ? round_model(k) : nullptr;
+      const bool own_split = k && k->splitk && (small ? small_grid_split(k, d, left_for_sums(k), false) : 1) > 1;
+      const bool same_tile = k && k->bm == ks[fresh]->bm && k->bn == ks[fresh]->bn;
+      if (!m || own_split || fresh_time < (same_tile ? 0.99 : 0.96) * round_time(*m, k, d, 1)) {
+        best = fresh;
+        settled = false;
+        split_edges = edges_were_split;
+      }
+    }
   }
   if (d->M == 0 || d->N == 0) {  // nothing to compute
     plan->grid_x = plan->grid_y = 0;
@@ -654,17 +722,11 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
     plan->workspace_bytes = packed.bytes;
     if (extras) extras->repack = packed;
   }
-  if (k->edge && !k->splitk && !no_split && d->split_k == 0) {
-    const int64_t edge_tiles = (int64_t)plan->grid_x * plan->grid_y;
-    const bool half_round = edge_tiles <= 128;
-    const size_t left = left_for_sums(k);
-    const int ts = !half_round ? tail_split_of(k, edge_tiles, (d->K + k->bk - 1) / k->bk, false, left) : small ? small_grid_split(k, d, left, split_edges) : edge_split_of(k, d, left);
-    if (ts > 1) {
-      const int64_t split_tiles = half_round ? edge_tiles : edge_tiles % 256;
-      const size_t offset = (plan->workspace_bytes + 255) & ~(size_t)255;
-      plan->workspace_bytes = offset + (size_t)ts * (size_t)split_tiles * (size_t)k->bm * (size_t)k->bn * 4;
-      if (extras) { extras->tail_split = ts; extras->tail_tiles = (int)split_tiles; extras->partial_offset = offset; }
-    }
+  if (const int ts = edge_slices(); ts > 1) {
+    const int64_t edge_tiles = (int64_t)plan->grid_x * plan->grid_y, split_tiles = edge_tiles <= 128 ? edge_tiles : edge_tiles % 256;
+    const size_t offset = (plan->workspace_bytes + 255) & ~(size_t)255;
+    plan->workspace_bytes = offset + (size_t)ts * (size_t)split_tiles * (size_t)k->bm * (size_t)k->bn * 4;
+    if (extras) { extras->tail_split = ts; extras->tail_tiles = (int)split_tiles; extras->partial_offset = offset; }
   }
   // Split K over the grid's y dimension when the tile grid alone leaves most CUs idle (skinny problems are
   // bound by streaming the large operand, which needs many work-groups in flight).  Slices hold whole K tiles.

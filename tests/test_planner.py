@@ -441,3 +441,22 @@ def test_a_plan_that_needs_copies_says_so_at_the_launch(kw):
     if "tile" in kw:  # copies larger than the static array
         d = R.make_desc(R.F16, 4001, 4003, 4001, transB=True, **kw)
         assert status(R.gemm_static_ws)[0] == "ERR_WORKSPACE"
+
+
+def _route(dt, M, N, K, lay="NN", **kw):
+    p = R.plan(R.make_desc(dt, M, N, K, transA=lay[0] == "T", transB=lay[1] == "T", **{"dtype_out": {R.I8: R.I32, R.E4M3: R.F32}.get(dt), **kw}))
+    return R.kernel_names()[p.kernel_id], p
+
+
+@pytest.mark.parametrize("dt,M,N,K,lay", [(R.BF16, 2496, 1664, 3584, "NN"), (R.F16, 1500, 2816, 3008, "NN"), (R.I8, 1728, 4480, 640, "NN"), (R.F16, 3256, 2128, 320, "NT"),
+                                          (R.F16, 5568, 2176, 7168, "NN")])
+def test_one_pass_where_it_is_the_faster_route(dt, M, N, K, lay):
+    """257 and more tiles of 128x128, aligned rows, whole K tiles: neither 192x256 tiles nor splits of edge tiles, which took 10 to 20 % longer"""
+    name, p = _route(dt, M, N, K, lay)
+    assert name.endswith("_edge") and "192x256" not in name and (p.workspace_bytes, p.split_k) == (0, 1), (name, p.workspace_bytes)
+
+
+@pytest.mark.parametrize("dt,M,N,K,lay", [(R.F16, 1589, 3072, 9600, "NN"), (R.F16, 2100, 2100, 8000, "TN"), (R.F16, 1500, 2816, 11008, "NN"), (R.BF16, 704, 960, 4032, "TN"),
+                                          (R.I8, 576, 1088, 8064, "TN"), (R.E4M3, 704, 512, 5760, "TT")])
+def test_deep_edge_tiles_stay_split(dt, M, N, K, lay):
+    assert _route(dt, M, N, K, lay)[1].workspace_bytes > 0
