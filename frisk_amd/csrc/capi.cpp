@@ -440,9 +440,12 @@ static double small_grid_time(const SmallGridModel& m, const KernelEntry* k, con
   const int64_t tiles = ((d->M + k->bm - 1) / k->bm) * ((d->N + k->bn - 1) / k->bn);
   const double kt = (double)((d->K + k->bk - 1) / k->bk) / split;
   const int64_t wgs = tiles * split, full = wgs / m.cap, rest = wgs % m.cap;
-  // one row of 64x128 tiles against a B stored [N][K] streams it 128 bytes of a row at a time: fp16 48x8192x8192 in 4 slices 37.0 us
-  // (64x32 tiles with K tiles four times as deep 28.7), 48x16384x8192 in 2 slices 64.3 (54.8)
-  const double tk = m.tk * (k->bm == 64 && k->bn == 128 && k->transB && tiles * k->bn < d->N + k->bn ? 1.4 : 1.0);
+  // One row of 64x128 tiles against a B stored [N][K] streams it 128 bytes of a row at a time, which is slow where its rows are a multiple of 16 KiB
+  // apart and little slower elsewhere.  us on them / on 64x32 tiles, whose K tiles are four times as deep: fp16 48x8192x8192 37.0 / 28.7,
+  // 48x16384x8192 64.3 / 54.8; but 49x10368x3712 18.6 / 23.8, 51x10112x2688 14.2 / 19.4, 35x14400x3968 26 / 32 (B from the last-level cache)
+  const bool one_row = k->bm == 64 && k->bn == 128 && k->transB && tiles * k->bn < d->N + k->bn;
+  const bool far_rows = d->K * elem_size(k->dtype) % 16384 == 0;
+  const double tk = m.tk * (!one_row ? 1.0 : far_rows ? 1.4 : split == 1 ? 1.05 : 1.0);
   double t = m.launch, whole = kt * tk + m.ps, last = 0.0;
   if (m.cap == 512) {  // two work-groups per CU: the second one of any CU sets the pace of the round
     whole += kt * m.tk2;
@@ -452,6 +455,9 @@ static double small_grid_time(const SmallGridModel& m, const KernelEntry* k, con
     last = kt * tk * (m.a + (1.0 - m.a) * (double)rest / m.cap);
   }
   t += (double)full * whole + (rest ? last : 0.0);
+  // (64x32 tiles beyond one round, which the sweep behind the table held few of, take 10 % longer than their rounds add up to: with both rules 12 of 1048
+  // drawn problems of 1 to 64 rows are more than 8 % slower than on 64x128 and 32x128 tiles, 134 before)
+  if (k->bm == 64 && k->wk > 1 && k->dtype != FRISK_F32 && wgs > 256 && !far_rows) t *= 1.1;
   if (split > 1) t += m.r0 + m.r1 * ((double)d->M * (double)d->N * split * 4.0 / 1e6);
   return k->guard && !k->edge ? kStagedFactor * t : t;
 }

@@ -460,3 +460,10 @@ def test_one_pass_where_it_is_the_faster_route(dt, M, N, K, lay):
                                           (R.I8, 576, 1088, 8064, "TN"), (R.E4M3, 704, 512, 5760, "TT")])
 def test_deep_edge_tiles_stay_split(dt, M, N, K, lay):
     assert _route(dt, M, N, K, lay)[1].workspace_bytes > 0
+
+
+@pytest.mark.parametrize("dt,M,N,K,tile", [(R.F16, 49, 10368, 3712, "64x128"), (R.F16, 51, 10112, 2688, "64x128"), (R.F16, 35, 14400, 3968, "64x128"), (R.F16, 33, 16384, 2048, "64x128"),
+                                           (R.E4M3, 59, 15744, 4992, "64x128"), (R.F16, 48, 8192, 8192, "64x32"), (R.F16, 48, 16384, 8192, "64x32")])
+def test_tiles_of_33_to_64_rows_on_weights_stored_by_columns(dt, M, N, K, tile):
+    """64x32 tiles only where the rows of the weights lie multiples of 16 KiB apart (or fewer of them fill the chip)"""
+    assert ("_nt_%sx" % tile) in _route(dt, M, N, K, "NT")[0]
