@@ -481,10 +481,10 @@ static int small_grid_split(const KernelEntry* k, const frisk_gemm_desc* d, size
     const int64_t wgs = k->transB || named ? m.w : std::max(m.w, 256);
     const int kmin = std::max(named ? m.kmin : std::min(m.kmin, 4), k->min_k_tiles);
     const int64_t most = std::min<int64_t>({k->dtype == FRISK_F32 ? 32 : 64, tiles > 0 ? wgs / tiles : 0, kt / kmin});
-    // fp32: a split within the range that the table was fitted over (powers of two) gives way to one of more slices for 12 % of modelled time: the bare model
-    // takes some to more and shorter slices that are slower.  us in 4 slices / in what it takes: 60x2752x1152 NT 12.2 / 13.3 (9), 88x1536x1152
-    // 11.5 / 12.7 (9), 107x1408x2176 15.9 / 17.4 (17), 411x384x2944 18.3 / 20.2 (23), 456x448x1280 12.8 / 13.9 (8).  Of 250 drawn problems 7 are more than 3 %
-    // slower than in that range, 19 by the bare model, at the same time on average
+    // fp32: a split within the range that the table was fitted over (powers of two) gives way to one of more slices of at most 10 K tiles for 12 % of modelled
+    // time: the bare model takes some to shorter slices that are slower.  us in 4 slices / in what it takes: 60x2752x1152 NT 12.2 / 13.3 (9), 88x1536x1152
+    // 11.5 / 12.7 (9), 107x1408x2176 15.9 / 17.4 (17), 411x384x2944 18.3 / 20.2 (23), 456x448x1280 12.8 / 13.9 (8); longer slices gain as modelled:
+    // 592x1280x7296 NT 114.9 in 2, 99.9 in 6, 975x384x8064 67.5 in 4, 60.3 in 21
     int fitted = 1;
     double fitted_t = INFINITY;
     for (int c = 2; c <= most; ++c)
@@ -493,7 +493,7 @@ static int small_grid_split(const KernelEntry* k, const frisk_gemm_desc* d, size
         if (t < best_t) { best = c; best_t = t; }
         if (k->dtype == FRISK_F32 && !(c & (c - 1)) && kt / c >= m.kmin && tiles * c <= m.w && t < fitted_t) { fitted = c; fitted_t = t; }
       }
-    if (best > fitted && fitted > 1 && fitted_t < 1.12 * best_t) { best = fitted; best_t = fitted_t; }
+    if (best > fitted && fitted > 1 && kt / best <= 10 && fitted_t < 1.12 * best_t) { best = fitted; best_t = fitted_t; }
   }
   // the edge kernels: slices of unequal length, whole tiles of partial sums
   if (const int most = edges ? edge_split_of(k, d, workspace) : 1; most > 1)

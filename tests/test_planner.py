@@ -470,7 +470,8 @@ def test_tiles_of_33_to_64_rows_on_weights_stored_by_columns(dt, M, N, K, tile):
 
 
 @pytest.mark.parametrize("M,N,K,lay,slices", [(60, 2752, 1152, "NT", 4), (88, 1536, 1152, "NT", 4), (107, 1408, 2176, "NT", 4), (411, 384, 2944, "NT", 4), (456, 448, 1280, "NT", 4),
-                                              (52, 192, 896, "NT", 7), (72, 192, 768, "NT", 6), (256, 512, 2400, "NN", 15)])
+                                              (52, 192, 896, "NT", 7), (72, 192, 768, "NT", 6), (256, 512, 2400, "NN", 15), (592, 1280, 7296, "NT", 6),
+                                              (975, 384, 8064, "NN", 21), (416, 2048, 11904, "NT", 12)])
 def test_slices_of_fp32_small_grids(M, N, K, lay, slices):
-    """more slices than the fitted range holds only for a clear gain, and where nothing in that range will do"""
+    """more and shorter slices than the fitted range holds only for a clear gain, and where nothing in that range will do"""
     assert _route(R.F32, M, N, K, lay)[1].split_k == slices
