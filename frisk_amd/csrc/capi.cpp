@@ -590,8 +590,16 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
   const auto& list = variants(d->dtype_ab, d->transA != 0, d->transB != 0);
   int best = -1;
   double best_cost = 0.0;
+  const bool tile_requested = d->tile_m || d->tile_n || d->tile_k || d->waves_m || d->waves_n || d->stages || d->atom;
+  // The kernels staged through registers take any rows in one launch, 1.4 us per K tile of 128 bytes behind those that work on copies (8-bit 2.2, fp32 0.7), so
+  // with few K tiles the launch that makes the copies costs more than it saves.  us staged / on copies: fp32 28x24x26 NN 4.8 / 7.5, 69x16x17 4.9 / 7.2,
+  // 78x18x35 TN 5.9 / 7.0, bf16 16x25x21 NT 6.9 / 7.6; but int8 24x884x344 TN 10.6 / 8.4,
+  // fp32 123x9x168 NN 9.7 / 7.7
+  const double staged_rounds = std::max(1.0, (double)((d->M + 127) / 128) * (double)((d->N + 127) / 128) / 512.0);
+  const bool copies_lose = packed.bytes && !tile_requested && d->policy == FRISK_POLICY_SQUARE &&
+                           staged_rounds * (double)(((int64_t)d->K * es + 127) / 128) * (es == 4 ? 0.72 : es == 2 ? 1.4 : 2.2) < 3.5 + (double)packed.bytes / 2.2e6;
   bool policy_excluded = false;
-  const bool any_layout = !list.empty(), tile_requested = d->tile_m || d->tile_n || d->tile_k || d->waves_m || d->waves_n || d->stages || d->atom;
+  const bool any_layout = !list.empty();
   const bool small = small_grid(d);
   bool split_edges = false, settled = false;  // settled: without the 192x256 tile and without splits of edge tiles
   // what the partial sums of a kernel may take of the workspace: all of it, or what lies behind the copies it works on
@@ -628,7 +636,7 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
       // the edge kernels once more under their guarded names: K off the K tile (a whole number of chunks), and anything at all,
       // with A and B copied to aligned rows where theirs are not
       if (k->guard == 1 && k->edge && (!rows_aligned || d->K % (16 / es))) continue;
-      if (k->guard == 2 && packed.bytes && (packed.bytes > ctx.workspace || d->split_k != 0)) continue;
+      if (k->guard == 2 && packed.bytes && (packed.bytes > ctx.workspace || d->split_k != 0 || copies_lose)) continue;
       // ... and address a tile's chunks by 32-bit lane offsets from its first row: the stored rows of one tile must span
       // less than 4 GiB
       const double span_a = (double)(packed.a ? packed.lda : d->lda) * es * (d->transA ? k->bk : k->bm),
@@ -659,7 +667,8 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
   search(explicit_split);
   if (best < 0 && explicit_split) search(false);
   // A small grid that falls to a kernel without the split-K store path looks at split edge kernels as well, where K is deep enough to split at
-  // all.  (The sweeps behind the tables held none, and beside the split-K kernels the tables flatter them: fp16 100x4096x4096 NN 20.6 us so, 16.8 on 64x128 tiles in 4 slices.)
+  // all.  (The sweeps behind the tables held none, and beside the split-K kernels the tables flatter them: fp16 100x4096x4096 NN 20.6 us so, 16.8 on
+  // 64x128 tiles in 4 slices.)
   if (small && best >= 0 && !no_split && d->split_k == 0 && es < 4 && d->K > (es == 1 ? 16 * 128 : 8 * 64) && !ks[best]->splitk && small_grid_split(ks[best], d, left_for_sums(ks[best]), false) == 1) {
     split_edges = true;
     search(false);

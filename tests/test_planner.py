@@ -475,3 +475,11 @@ def test_tiles_of_33_to_64_rows_on_weights_stored_by_columns(dt, M, N, K, tile):
 def test_slices_of_fp32_small_grids(M, N, K, lay, slices):
     """more and shorter slices than the fitted range holds only for a clear gain, and where nothing in that range will do"""
     assert _route(R.F32, M, N, K, lay)[1].split_k == slices
+
+
+@pytest.mark.parametrize("dt,M,N,K,lay,copies", [(R.F32, 28, 24, 26, "NN", 0), (R.F32, 69, 16, 17, "NN", 0), (R.BF16, 16, 25, 21, "NT", 0), (R.F16, 22, 19, 50, "NT", 0), (R.E4M3, 15, 17, 33, "NN", 0),
+                                                 (R.I8, 24, 884, 344, "TN", 1), (R.F32, 123, 9, 168, "NN", 1), (R.F16, 1001, 1003, 1005, "NN", 1)])
+def test_copies_of_rows_off_16_bytes_are_for_more_than_a_few_k_tiles(dt, M, N, K, lay, copies):
+    """a launch for the copies costs more than staging a few K tiles through registers, at any workspace"""
+    name, p = _route(dt, M, N, K, lay)
+    assert (p.workspace_bytes > 0) == bool(copies) and bool(re.search(r"_s\dx\d(_a16)?_guard", name)) == bool(copies), name
