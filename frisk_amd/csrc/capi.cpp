@@ -198,8 +198,9 @@ static void fill_layout(frisk_lds_layout* L, bool kcontig, int es, int fragb, in
 static constexpr size_t kAnyWorkspace = ~(size_t)0;
 
 // Tail split: a grid of a little more than a whole number of rounds of 256 tiles leaves most CUs idle in its last round.
-// With a kernel that has the split-K store path, the last tiles % 256 tiles (at most half a round) are computed by 2, 4 or
-// 8 work-groups each, every one taking an equal share of the K tiles (at least 4).  Returns that count, 1 for no split.
+// The last tiles % 256 tiles (at most half a round) are then computed by several work-groups each: with a kernel that has the split-K store path by 2, 4
+// or 8 with an equal share of the K tiles apiece, with a large edge kernel by any 2 to 8, whose last share may be shorter.  Returns that count, 1 for no
+// split.
 static int tail_split_of(const KernelEntry* k, int64_t tiles, int64_t kt, bool whole_k_tiles, size_t workspace) {
   // the edge kernels deal any number of K tiles: their last slice may be shorter (us unsplit / split: bf16 3000x11008x4096 NT, 516
   // tiles, 248 / 212; fp16 4097x4097x4096 NT, 289 tiles, 161 / 126; 4095x4097x4001 NN with its copy to aligned rows 204 / 150)
@@ -237,10 +238,6 @@ static int edge_split_of(const KernelEntry* k, const frisk_gemm_desc* d, size_t 
   return 1;
 }
 
-// Relative time of a problem on a kernel variant, used only to rank the variants.  One wave of work-groups = one per CU
-// (256); a K tile of a 256x256 tile costs 1.5 units when every CU runs one, and less when the chip is partly idle
-// (less contention in the L2 and a higher clock): factor 0.6 + 0.4 * fill.  The constants are measured on fp16 problems
-// between 1024^3 and 8192^3 and carry over to the 8-bit types, whose K tiles hold the same number of bytes.
 // the split the planner gives a grid below one round of a variant with the split-K store path: up to one work-group per CU,
 // at least 4 K tiles per slice
 static int sub_round_split(const KernelEntry* k, const frisk_gemm_desc* d, int64_t tiles, int64_t kt, size_t workspace) {
@@ -254,6 +251,10 @@ static int sub_round_split(const KernelEntry* k, const frisk_gemm_desc* d, int64
 // registers against copy + LDS transfers on 128x128 tiles: 4095x4097x4001 304 / 227, 1999x4099x3001 154 / 100, 1001x999x1003 31 / 21)
 static constexpr double kStagedFactor = 1.6;
 
+// Relative time of a problem on a kernel variant, used only to rank the variants.  One wave of work-groups = one per CU
+// (256); a K tile of a 256x256 tile costs 1.5 units when every CU runs one, and less when the chip is partly idle
+// (less contention in the L2 and a higher clock): factor 0.6 + 0.4 * fill.  The constants are measured on fp16 problems
+// between 1024^3 and 8192^3 and carry over to the 8-bit types, whose K tiles hold the same number of bytes.
 static double estimated_cost(const KernelEntry* k, const frisk_gemm_desc* d, bool may_split, bool split_edges, size_t workspace) {
   const int64_t tiles = ((d->M + k->bm - 1) / k->bm) * ((d->N + k->bn - 1) / k->bn);
   const double kt = (double)((d->K + k->bk - 1) / k->bk);
@@ -337,8 +338,8 @@ static double estimated_cost(const KernelEntry* k, const frisk_gemm_desc* d, boo
 // work-group per tile, so the choice is a (variant, split of K) pair.  Measured per element type over 81 skinny shapes (M 32 ..
 // 2048, N and K 1024 .. 28672) and 90 squarish ones (sides 768 .. 2048, K 1024 .. 8192), both layouts of B, every variant at
 // every split 1 .. 32, B taken in turn from as many copies as fill 400 MiB so that it streams from HBM as the weights of a model
-// do (with one B of at most 128 MiB the last-level cache serves it: 26.5 instead of 38 us at fp16 64x8192x8192).  A variant's splits are the powers of two that keep tiles x split within `w` work-groups and `kmin` K
-// tiles per slice; variants and splits are compared by a time model fitted to the sweep, in microseconds:
+// do (with one B of at most 128 MiB the last-level cache serves it: 26.5 instead of 38 us at fp16 64x8192x8192).  The sweep's splits of a
+// variant were the powers of two that keep tiles x split within `w` work-groups and `kmin` K tiles per slice (small_grid_split goes beyond them); variants and splits are compared by a time model fitted to the sweep, in microseconds:
 //   launch + whole rounds x (K tiles x tk + ps) + a last round at K tiles x tk x (a + (1 - a) x fill) + the summing pass
 //   (r0 + r1 x megabytes of partial sums) when split;
 // variants of which a CU holds two work-groups (`cap` 512) pay tk2 per K tile more once any CU holds its second one:

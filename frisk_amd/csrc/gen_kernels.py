@@ -81,7 +81,7 @@ def square(bk, atom16=False, skinny_ta=(0,)):
     out.append(edge((0, 1, 32, 32, 4 * bk, 1, 1, 4, 0, 0, 4)))
     out.append(edge((0, 1, 32, 32, 4 * bk, 1, 1, 2, 0, 0, 4)))
     out.append(edge((0, 1, 64, 32, 4 * bk, 1, 1, 3, 0, 0, 4)))
-    # M and N that are not multiples of the tile (K a multiple of the K tile, rows and pointers on 16-byte boundaries): the default
+    # M and N that are not multiples of the tile, and any K (rows of A and B on 16-byte boundaries, or copied there first): the default
     # 256x256 variant and the 128x128 one with 2 + 2 tiles once more with clamped lane offsets and checked stores.  (fp16
     # 4000x4096x4096 ran 539 us on 32-row tiles and 4096x4000x4096 933 us on the guarded kernel, the vendor library 110 and 125.)
     for ta in (0, 1):

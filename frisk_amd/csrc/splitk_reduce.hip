@@ -84,7 +84,7 @@ template <bool INT_ACC> __global__ void __launch_bounds__(256) tail_reduce_kerne
     if (m >= p.M || n >= p.N) continue;
     int isum[4] = {0, 0, 0, 0};
     float fsum[4] = {0.f, 0.f, 0.f, 0.f};
-    r_v4i v[8];  // a tail has 2, 4 or 8 slices: all fetched before the first addition, added in slice order
+    r_v4i v[8];  // at most 8 slices: all fetched before the first addition, added in slice order
 #pragma unroll
     for (int z = 0; z < 8; ++z)
       if (z < p.tail_split) v[z] = *(const r_v4i*)((const char*)p.partial + (((size_t)z * p.tail_tiles + t) * tile_elems + (size_t)r * BN + c) * 4);
