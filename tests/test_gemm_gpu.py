@@ -735,3 +735,15 @@ def test_config_fp8_skinny_decode(hip):
     ref = O.epilogue_tensor(O.gemm_f64(O.E4M3, A, B, False, True), sA, sB)
     r = check(O.E4M3, O.BF16, got, ref)
     note(f"fp8 skinny 32x8192x8192 NT split_k={p.split_k}: {r}")
+
+
+@pytest.mark.parametrize("dtype", [O.F16, O.E4M3])
+def test_rows_of_64x32_tiles_walk_k_in_step(hip, dtype):
+    """in a grid of several rows of tiles every work-group walks K from its first tile (their operands meet in the L2): equal rows of A give equal
+    bits in every row of tiles, which sums taken in another order do not"""
+    K, N = 7 * 4 * BK[dtype], 96
+    A = make_operand(dtype, 64, K, seed=5, tensor=0, scale=0.5)
+    B = make_operand(dtype, N, K, seed=5, tensor=1, scale=0.5)
+    got = run_gemm(hip, dtype, np.concatenate([A, A, A]), B, 0, 1, O.F32, 192, N, K, tile=(64, 32, 4 * BK[dtype]), split_k=1)
+    assert np.array_equal(got[:64].view(np.uint32), got[64:128].view(np.uint32)) and np.array_equal(got[:64].view(np.uint32), got[128:].view(np.uint32))
+    check(dtype, O.F32, got[:64], O.gemm_f64(dtype, A, B, 0, 1))
