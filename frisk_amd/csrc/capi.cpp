@@ -463,8 +463,13 @@ static double small_grid_time(const SmallGridModel& m, const KernelEntry* k, con
   return k->guard && !k->edge ? kStagedFactor * t : t;
 }
 // the split of a variant: among those the rule admits, the one the model makes fastest; *cost receives its time.  `edges`: edge kernels may
-// be split too
-static int small_grid_split(const KernelEntry* k, const frisk_gemm_desc* d, size_t workspace, bool edges, double* cost = nullptr) {
+// be split too.  `table_range`: only splits of the range that the table was fitted over
+static bool in_table_range(const KernelEntry* k, const frisk_gemm_desc* d, int split) {
+  const SmallGridModel& m = small_grid_model(k);
+  const int64_t tiles = ((d->M + k->bm - 1) / k->bm) * ((d->N + k->bn - 1) / k->bn);
+  return split == 1 || (!(split & (split - 1)) && d->K / k->bk / split >= m.kmin && tiles * split <= m.w);
+}
+static int small_grid_split(const KernelEntry* k, const frisk_gemm_desc* d, size_t workspace, bool edges, bool table_range, double* cost = nullptr) {
   const SmallGridModel& m = small_grid_model(k);
   int best = 1;
   double best_t = small_grid_time(m, k, d, 1);
@@ -489,10 +494,10 @@ static int small_grid_split(const KernelEntry* k, const frisk_gemm_desc* d, size
     int fitted = 1;
     double fitted_t = INFINITY;
     for (int c = 2; c <= most; ++c)
-      if (kt % c == 0 && (size_t)c * (size_t)d->M * (size_t)d->N * 4 <= workspace) {
+      if (kt % c == 0 && (size_t)c * (size_t)d->M * (size_t)d->N * 4 <= workspace && (!table_range || in_table_range(k, d, c))) {
         const double t = small_grid_time(m, k, d, c);
         if (t < best_t) { best = c; best_t = t; }
-        if (k->dtype == FRISK_F32 && !(c & (c - 1)) && kt / c >= m.kmin && tiles * c <= m.w && t < fitted_t) { fitted = c; fitted_t = t; }
+        if (k->dtype == FRISK_F32 && in_table_range(k, d, c) && t < fitted_t) { fitted = c; fitted_t = t; }
       }
     if (best > fitted && fitted > 1 && kt / best <= 10 && fitted_t < 1.12 * best_t) { best = fitted; best_t = fitted_t; }
   }
@@ -506,9 +511,43 @@ static int small_grid_split(const KernelEntry* k, const frisk_gemm_desc* d, size
   if (cost) *cost = best_t;
   return best;
 }
-static double small_grid_cost(const KernelEntry* k, const frisk_gemm_desc* d, size_t workspace, bool edges) {
+static double small_grid_cost(const KernelEntry* k, const frisk_gemm_desc* d, size_t workspace, bool edges, bool table_range) {
   double t = 0.0;
-  small_grid_split(k, d, workspace, edges, &t);
+  small_grid_split(k, d, workspace, edges, table_range, &t);
+  return t;
+}
+
+// Beyond the range of the table (other splits than those of its sweep, kernels that the sweep did not hold) its times are off by a factor of each variant's
+// own, and a split costs more by the slice than it knows, since the summing pass waits for its slices.  This is the time with both put right, for the choice
+// between a route beyond the range and the best one within it; 16- and 8-bit types.  Over 64 rows whole x the table's in one pass, scale x the table's
+// + split + slice x (slices - 1) in slices, fitted to 4600 problems of M and N from 128 and 512, K 1024 to 16384, operands in rotation (deviation of a variant's times 4 to 9 %, 5 to
+// 14 without).
+static double refined_time(const KernelEntry* k, const frisk_gemm_desc* d, int split) {
+  struct Fit { float whole, scale, split, slice; };
+  static const Fit fits[2][14] = {  // in the order of kSmallGrid
+      {{1.02f, 1.0f, 0.0f, 0.0f}, {1.1f, 1.035f, -2.6f, 0.155f}, {1.0f, 1.0f, 0.0f, 0.0f}, {1.0f, 1.0f, 0.0f, 0.0f}, {1.0f, 1.15f, -3.7f, 0.04f}, {1.0f, 1.15f, -3.7f, 0.04f},  // 16-bit
+       {1.0f, 1.0f, 0.0f, 0.0f}, {0.94f, 0.754f, 0.25f, 0.18f}, {0.94f, 0.754f, 0.25f, 0.18f}, {0.85f, 0.85f, 0.0f, 0.18f}, {0.85f, 0.85f, 0.0f, 0.18f},
+       {0.92f, 0.897f, -2.54f, 0.199f}, {0.97f, 0.943f, -0.69f, 0.086f}, {1.02f, 1.061f, -2.07f, 0.188f}},
+      {{1.17f, 1.0f, 0.0f, 0.0f}, {0.99f, 0.97f, -1.79f, 0.161f}, {1.0f, 1.0f, 0.0f, 0.0f}, {1.0f, 1.0f, 0.0f, 0.0f}, {1.0f, 1.0f, 0.0f, 0.1f}, {1.0f, 1.0f, 0.0f, 0.1f},  // 8-bit
+       {1.0f, 1.0f, 0.0f, 0.0f}, {0.85f, 0.829f, -0.53f, 0.183f}, {0.85f, 0.829f, -0.53f, 0.183f}, {0.888f, 0.888f, 0.0f, 0.18f}, {0.888f, 0.888f, 0.0f, 0.18f},
+       {0.95f, 0.924f, -1.89f, 0.189f}, {0.99f, 0.95f, 0.0f, 0.1f}, {1.01f, 1.0f, -1.17f, 0.153f}},
+  };
+  const int es = elem_size(k->dtype);
+  double t = small_grid_time(small_grid_model(k), k, d, split);
+  if (d->M > 64) {
+    const Fit& f = fits[es == 1][small_grid_class(k)];
+    return split > 1 ? f.scale * t + f.split + f.slice * (split - 1) : f.whole * t;
+  }
+  const int64_t wgs = ((d->M + k->bm - 1) / k->bm) * ((d->N + k->bn - 1) / k->bn) * split, kt = (d->K + k->bk - 1) / k->bk;
+  if (es == 2 && k->bm == 64) {
+    // fp16 62x4672x7424 NT 26.1 us on 64x32 tiles, 23.6 on 64x128 tiles in 4 slices; bf16 49x3648x5888 NN 18.1 on 32x128 tiles, 14.2 on 64x128 ones
+    if (k->wk > 1 && d->K > 4096 && d->K * es % 16384) t *= 1.15;
+    if (k->bn == 128 && !k->transB && split > 1 && split < 8) t *= 0.93;
+  } else if (es == 1 && k->bm == 32) {
+    // 32x32 tiles beyond one round, a K tile of 512, where K ends inside one of a few: int8 32x9216x2688 NT 9.1 us, on 32x128 tiles 8.1; 5x14528x2688
+    // 9.6 / 8.8; but e4m3 7x13504x3712 12.0 / 14.2, 2x15808x3200 11.5 / 13.3
+    if (k->bn == 32 && wgs > 256 && d->K % k->bk && kt <= 6) t *= 1.17;
+  }
   return t;
 }
 
@@ -603,6 +642,7 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
   const bool any_layout = !list.empty();
   const bool small = small_grid(d);
   bool split_edges = false, settled = false;  // settled: without the 192x256 tile and without splits of edge tiles
+  bool table_range = false;                    // small grids: the kernels and splits that their table was fitted over
   // what the partial sums of a kernel may take of the workspace: all of it, or what lies behind the copies it works on
   auto left_for_sums = [&](const KernelEntry* k) {
     const size_t copies = k->guard == 2 && packed.bytes ? (packed.bytes + 255) & ~(size_t)255 : 0;
@@ -633,7 +673,7 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
       // (whole 256x256 tiles keep the default kernel: which one they run on is part of the planner's interface, though 144 of them
       // leave CUs idle -- fp16 3072x3072x4096 NN 70.6 us, 62.4 on 192x256 tiles)
       const bool whole_256 = rows_aligned && d->M % 256 == 0 && d->N % 256 == 0 && d->K % k->bk == 0;
-      if (planners_own(k) && (tile_requested || d->split_k > 1 || (k->bm == 192 ? small || whole_256 || settled : d->M > 64))) continue;
+      if (planners_own(k) && (tile_requested || table_range || d->split_k > 1 || (k->bm == 192 ? small || whole_256 || settled : d->M > 64))) continue;
       // the edge kernels once more under their guarded names: K off the K tile (a whole number of chunks), and anything at all,
       // with A and B copied to aligned rows where theirs are not
       if (k->guard == 1 && k->edge && (!rows_aligned || d->K % (16 / es))) continue;
@@ -646,7 +686,7 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
       // never a guarded kernel when a fast one fits -- except those, which run at their full rate whatever their name
       if (k->guard && !planners_own(k) && best >= 0 && !ks[best]->guard) continue;
       const size_t left = left_for_sums(k);
-      double cost = small && !want_split ? small_grid_cost(k, d, left, split_edges) : estimated_cost(k, d, !want_split && left > 0 && d->split_k == 0, !settled, left);
+      double cost = small && !want_split ? small_grid_cost(k, d, left, split_edges, table_range) : estimated_cost(k, d, !want_split && left > 0 && d->split_k == 0, !settled, left);
       // (a 32-row edge tile above 64 rows streams B once per 32 rows where the 64-row tile wastes at most as much: 130x11008x4096
       // NT 64.5 against 53.5 us)
       if (k->edge && k->bm == 32 && d->M > 64 && !d->tile_m) continue;
@@ -670,7 +710,7 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
   // A small grid that falls to a kernel without the split-K store path looks at split edge kernels as well, where K is deep enough to split at
   // all.  (The sweeps behind the tables held none, and beside the split-K kernels the tables flatter them: fp16 100x4096x4096 NN 20.6 us so, 16.8 on
   // 64x128 tiles in 4 slices.)
-  if (small && best >= 0 && !no_split && d->split_k == 0 && es < 4 && d->K > (es == 1 ? 16 * 128 : 8 * 64) && !ks[best]->splitk && small_grid_split(ks[best], d, left_for_sums(ks[best]), false) == 1) {
+  if (small && best >= 0 && !no_split && d->split_k == 0 && es < 4 && d->K > (es == 1 ? 16 * 128 : 8 * 64) && !ks[best]->splitk && small_grid_split(ks[best], d, left_for_sums(ks[best]), false, false) == 1) {
     split_edges = true;
     search(false);
   }
@@ -680,8 +720,30 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
     if (!k->edge || k->splitk || no_split || d->split_k != 0 || settled) return 1;
     const int64_t tiles = ((d->M + k->bm - 1) / k->bm) * ((d->N + k->bn - 1) / k->bn);
     const size_t left = left_for_sums(k);
-    return tiles > 128 ? tail_split_of(k, tiles, (d->K + k->bk - 1) / k->bk, false, left) : small ? small_grid_split(k, d, left, split_edges) : edge_split_of(k, d, left);
+    return tiles > 128 ? tail_split_of(k, tiles, (d->K + k->bk - 1) / k->bk, false, left) : small ? small_grid_split(k, d, left, split_edges, false) : edge_split_of(k, d, left);
   };
+  // A small grid whose route lies beyond the range of its table keeps it unless the refined times see the best route within the range ahead, over 64 rows by
+  // 3 %.  The routes that this changes are 5 % faster up to 64 rows (165 drawn problems, 4 of them slower by 3 % or more); over 64 rows, of 127, 8 % faster
+  // with operands that the last-level cache holds and 2 % slower with operands from memory.  us within / beyond: fp16 1024x1024x6272 NT 23.0 in 2
+  // slices of 64x128 tiles, 31.0 in 7 of 256x256; 384x256x5888 NT 11.1 / 14.4, 128x1024x4864 NN 11.7 / 14.9, int8 640x128x14848 NT 13.0 / 16.6,
+  // 32x9216x2688 NT 8.1 / 9.1.
+  if (small && best >= 0 && es < 4 && rows_aligned && !tile_requested && d->split_k <= 1) {
+    const KernelEntry* k = ks[best];
+    const int fresh = best, split = k->splitk && d->K % k->bk == 0 ? small_grid_split(k, d, left_for_sums(k), false, false) : 1;
+    if (planners_own(k) ? edge_slices() == 1 : k->splitk && !in_table_range(k, d, split)) {
+      const bool edges_were_split = split_edges;
+      best = -1;
+      table_range = true;
+      split_edges = false;
+      search(false);
+      const KernelEntry* in = best >= 0 ? ks[best] : nullptr;
+      if (!in || in->guard || refined_time(k, d, split) * (d->M > 64 ? 0.97 : 1.0) < refined_time(in, d, small_grid_split(in, d, left_for_sums(in), false, true))) {
+        best = fresh;
+        table_range = false;
+        split_edges = edges_were_split;
+      }
+    }
+  }
   // The 192x256 tile and split edge tiles against what a problem of whole K tiles and aligned rows runs on otherwise, 128x128 and 256x256 tiles in one
   // pass at their full rate: the costs above come out a few per cent apart there, closer than they are accurate, so the model of rounds must see a
   // gain too, of 4 % where the tile is another one.  us in one pass / so: bf16 2496x1664x3584 NN (260 tiles of 128x128) 39.8 / 44.1,
@@ -699,7 +761,7 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
       search(false);
       const KernelEntry* k = best >= 0 ? ks[best] : nullptr;
       const RoundModel* m = k ? round_model(k) : nullptr;
-      const bool own_split = k && k->splitk && (small ? small_grid_split(k, d, left_for_sums(k), false) : 1) > 1;
+      const bool own_split = k && k->splitk && (small ? small_grid_split(k, d, left_for_sums(k), false, table_range) : 1) > 1;
       const bool same_tile = k && k->bm == ks[fresh]->bm && k->bn == ks[fresh]->bn;
       if (!m || own_split || fresh_time < (same_tile ? 0.99 : 0.96) * round_time(*m, k, d, 1)) {
         best = fresh;
@@ -763,7 +825,7 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
         return fail(FRISK_ERR_TILE, "split_k=%d leaves %lld K tiles per slice, the chosen kernel %s needs %d", d->split_k, (long long)(kt / d->split_k), k->name, k->min_k_tiles);
       split = d->split_k;
     } else if (small) {
-      split = small_grid_split(k, d, ctx.workspace, false);
+      split = small_grid_split(k, d, ctx.workspace, false, table_range);
     } else if (d->split_k == 0 && tiles < 256) {
       split = sub_round_split(k, d, tiles, kt, ctx.workspace);
     } else if (d->split_k == 0) {
