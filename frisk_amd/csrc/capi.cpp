@@ -763,7 +763,10 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
       const RoundModel* m = k ? round_model(k) : nullptr;
       const bool own_split = k && k->splitk && (small ? small_grid_split(k, d, left_for_sums(k), false, table_range) : 1) > 1;
       const bool same_tile = k && k->bm == ks[fresh]->bm && k->bn == ks[fresh]->bn;
-      if (!m || own_split || fresh_time < (same_tile ? 0.99 : 0.96) * round_time(*m, k, d, 1)) {
+      // one round of two 128x128 tiles a CU beats a partial one of unsplit 192x256 tiles, which has more to do on each CU than the model knows (us: bf16
+      // 2624x3008x7680 NN 119.9 / 140.3, 1536x5312x7424 116.5 / 133.1, fp16 1920x4224x5120 87.6 / 93.7; 11 of 11 drawn problems slower by 3 to 15 %)
+      const bool one_round = m && m->cap == 512 && slices == 1 && (((d->M + 127) / 128) * ((d->N + 127) / 128) <= 512);
+      if (!m || own_split || (!one_round && fresh_time < (same_tile ? 0.99 : 0.96) * round_time(*m, k, d, 1))) {
         best = fresh;
         settled = false;
         split_edges = edges_were_split;

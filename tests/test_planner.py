@@ -449,7 +449,7 @@ def _route(dt, M, N, K, lay="NN", **kw):
 
 
 @pytest.mark.parametrize("dt,M,N,K,lay", [(R.BF16, 2496, 1664, 3584, "NN"), (R.F16, 1500, 2816, 3008, "NN"), (R.I8, 1728, 4480, 640, "NN"), (R.F16, 3256, 2128, 320, "NT"),
-                                          (R.F16, 5568, 2176, 7168, "NN")])
+                                          (R.F16, 5568, 2176, 7168, "NN"), (R.BF16, 2624, 3008, 7680, "NN"), (R.BF16, 1536, 5312, 7424, "NN"), (R.F16, 2112, 3776, 5504, "NT")])
 def test_one_pass_where_it_is_the_faster_route(dt, M, N, K, lay):
     """257 and more tiles of 128x128, aligned rows, whole K tiles: neither 192x256 tiles nor splits of edge tiles, which took 10 to 20 % longer"""
     name, p = _route(dt, M, N, K, lay)
