@@ -463,16 +463,16 @@ static double small_grid_time(const SmallGridModel& m, const KernelEntry* k, con
   return k->guard && !k->edge ? kStagedFactor * t : t;
 }
 // the split of a variant: among those the rule admits, the one the model makes fastest; *cost receives its time.  `edges`: edge kernels may
-// be split too.  `table_range`: only splits of the range that the table was fitted over
+// be split too.  `table_range`: only splits of the range that the table was fitted over; *range_cost receives the time of the best of those
 static bool in_table_range(const KernelEntry* k, const frisk_gemm_desc* d, int split) {
   const SmallGridModel& m = small_grid_model(k);
   const int64_t tiles = ((d->M + k->bm - 1) / k->bm) * ((d->N + k->bn - 1) / k->bn);
   return split == 1 || (!(split & (split - 1)) && d->K / k->bk / split >= m.kmin && tiles * split <= m.w);
 }
-static int small_grid_split(const KernelEntry* k, const frisk_gemm_desc* d, size_t workspace, bool edges, bool table_range, double* cost = nullptr) {
+static int small_grid_split(const KernelEntry* k, const frisk_gemm_desc* d, size_t workspace, bool edges, bool table_range, double* cost = nullptr, double* range_cost = nullptr) {
   const SmallGridModel& m = small_grid_model(k);
   int best = 1;
-  double best_t = small_grid_time(m, k, d, 1);
+  double best_t = small_grid_time(m, k, d, 1), range_t = best_t;
   if (k->splitk && workspace && d->split_k != 1 && m.w != 0 && d->K % k->bk == 0) {
     const int64_t tiles = ((d->M + k->bm - 1) / k->bm) * ((d->N + k->bn - 1) / k->bn), kt = d->K / k->bk;
     // any divisor of the K tiles (K = 5760 is 45 tiles of 128: the powers of two left it unsplit); the sweeps behind the tables: up to 64
@@ -497,6 +497,7 @@ static int small_grid_split(const KernelEntry* k, const frisk_gemm_desc* d, size
       if (kt % c == 0 && (size_t)c * (size_t)d->M * (size_t)d->N * 4 <= workspace && (!table_range || in_table_range(k, d, c))) {
         const double t = small_grid_time(m, k, d, c);
         if (t < best_t) { best = c; best_t = t; }
+        if (range_cost && t < range_t && in_table_range(k, d, c)) range_t = t;
         if (k->dtype == FRISK_F32 && in_table_range(k, d, c) && t < fitted_t) { fitted = c; fitted_t = t; }
       }
     if (best > fitted && fitted > 1 && kt / best <= 10 && fitted_t < 1.12 * best_t) { best = fitted; best_t = fitted_t; }
@@ -509,12 +510,8 @@ static int small_grid_split(const KernelEntry* k, const frisk_gemm_desc* d, size
         if (t < best_t) { best = c; best_t = t; }
       }
   if (cost) *cost = best_t;
+  if (range_cost) *range_cost = range_t;
   return best;
-}
-static double small_grid_cost(const KernelEntry* k, const frisk_gemm_desc* d, size_t workspace, bool edges, bool table_range) {
-  double t = 0.0;
-  small_grid_split(k, d, workspace, edges, table_range, &t);
-  return t;
 }
 
 // Beyond the range of the table (other splits than those of its sweep, kernels that the sweep did not hold) its times are off by a factor of each variant's
@@ -642,7 +639,11 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
   const bool any_layout = !list.empty();
   const bool small = small_grid(d);
   bool split_edges = false, settled = false;  // settled: without the 192x256 tile and without splits of edge tiles
-  bool table_range = false;                    // small grids: the kernels and splits that their table was fitted over
+  // small grids: the best of the kernels and splits that their table was fitted over, found beside the best of all
+  const bool want_range = small && es < 4 && rows_aligned && !tile_requested && d->split_k <= 1;
+  int best_in = -1;
+  double best_in_cost = 0.0;
+  bool table_range = false;  // that one is taken
   // what the partial sums of a kernel may take of the workspace: all of it, or what lies behind the copies it works on
   auto left_for_sums = [&](const KernelEntry* k) {
     const size_t copies = k->guard == 2 && packed.bytes ? (packed.bytes + 255) & ~(size_t)255 : 0;
@@ -673,7 +674,7 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
       // (whole 256x256 tiles keep the default kernel: which one they run on is part of the planner's interface, though 144 of them
       // leave CUs idle -- fp16 3072x3072x4096 NN 70.6 us, 62.4 on 192x256 tiles)
       const bool whole_256 = rows_aligned && d->M % 256 == 0 && d->N % 256 == 0 && d->K % k->bk == 0;
-      if (planners_own(k) && (tile_requested || table_range || d->split_k > 1 || (k->bm == 192 ? small || whole_256 || settled : d->M > 64))) continue;
+      if (planners_own(k) && (tile_requested || d->split_k > 1 || (k->bm == 192 ? small || whole_256 || settled : d->M > 64))) continue;
       // the edge kernels once more under their guarded names: K off the K tile (a whole number of chunks), and anything at all,
       // with A and B copied to aligned rows where theirs are not
       if (k->guard == 1 && k->edge && (!rows_aligned || d->K % (16 / es))) continue;
@@ -686,7 +687,9 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
       // never a guarded kernel when a fast one fits -- except those, which run at their full rate whatever their name
       if (k->guard && !planners_own(k) && best >= 0 && !ks[best]->guard) continue;
       const size_t left = left_for_sums(k);
-      double cost = small && !want_split ? small_grid_cost(k, d, left, split_edges, table_range) : estimated_cost(k, d, !want_split && left > 0 && d->split_k == 0, !settled, left);
+      double cost = 0.0, range_cost = 0.0;
+      if (small && !want_split) small_grid_split(k, d, left, split_edges, false, &cost, want_range ? &range_cost : nullptr);
+      else cost = estimated_cost(k, d, !want_split && left > 0 && d->split_k == 0, !settled, left);
       // (a 32-row edge tile above 64 rows streams B once per 32 rows where the 64-row tile wastes at most as much: 130x11008x4096
       // NT 64.5 against 53.5 us)
       if (k->edge && k->bm == 32 && d->M > 64 && !d->tile_m) continue;
@@ -695,11 +698,14 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
         // the models see whole tiles; rows and columns beyond M and N are work all the same (a 64-row tile on 32 rows is no
         // better than the 32-row tile that fits): the square root of the covered area over M x N, as a penalty
         const double covered = (double)((d->M + k->bm - 1) / k->bm * k->bm) * (double)((d->N + k->bn - 1) / k->bn * k->bn);
-        cost *= std::sqrt(covered / ((double)d->M * (double)d->N));
+        const double waste = std::sqrt(covered / ((double)d->M * (double)d->N));
+        cost *= waste;
+        range_cost *= waste;
       }
       if (k->guard == 2) cost += repack_cost;
       // ties: the first listed variant is the tuned default
       if (best < 0 || (ks[best]->guard && !k->guard && !planners_own(ks[best])) || cost < best_cost) { best = v.id; best_cost = cost; }
+      if (want_range && !k->guard && !planners_own(k) && (best_in < 0 || range_cost < best_in_cost)) { best_in = v.id; best_in_cost = range_cost; }
     }
   };
   // an explicit split_k looks among the variants with the split-K store path first; if none of them fits, the choice among
@@ -727,21 +733,14 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
   // with operands that the last-level cache holds and 2 % slower with operands from memory.  us within / beyond: fp16 1024x1024x6272 NT 23.0 in 2
   // slices of 64x128 tiles, 31.0 in 7 of 256x256; 384x256x5888 NT 11.1 / 14.4, 128x1024x4864 NN 11.7 / 14.9, int8 640x128x14848 NT 13.0 / 16.6,
   // 32x9216x2688 NT 8.1 / 9.1.
-  if (small && best >= 0 && es < 4 && rows_aligned && !tile_requested && d->split_k <= 1) {
-    const KernelEntry* k = ks[best];
-    const int fresh = best, split = k->splitk && d->K % k->bk == 0 ? small_grid_split(k, d, left_for_sums(k), false, false) : 1;
-    if (planners_own(k) ? edge_slices() == 1 : k->splitk && !in_table_range(k, d, split)) {
-      const bool edges_were_split = split_edges;
-      best = -1;
+  if (best >= 0 && best_in >= 0) {
+    const KernelEntry *k = ks[best], *in = ks[best_in];
+    const int split = k->splitk && d->K % k->bk == 0 ? small_grid_split(k, d, left_for_sums(k), false, false) : 1;
+    if ((planners_own(k) ? edge_slices() == 1 : k->splitk && !in_table_range(k, d, split)) &&
+        refined_time(k, d, split) * (d->M > 64 ? 0.97 : 1.0) >= refined_time(in, d, small_grid_split(in, d, left_for_sums(in), false, true))) {
+      best = best_in;
       table_range = true;
       split_edges = false;
-      search(false);
-      const KernelEntry* in = best >= 0 ? ks[best] : nullptr;
-      if (!in || in->guard || refined_time(k, d, split) * (d->M > 64 ? 0.97 : 1.0) < refined_time(in, d, small_grid_split(in, d, left_for_sums(in), false, true))) {
-        best = fresh;
-        table_range = false;
-        split_edges = edges_were_split;
-      }
     }
   }
   // The 192x256 tile and split edge tiles against what a problem of whole K tiles and aligned rows runs on otherwise, 128x128 and 256x256 tiles in one
