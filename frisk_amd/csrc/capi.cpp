@@ -671,8 +671,8 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
       if (!k->guard && (!rows_aligned || d->K % k->bk || (k->edge ? whole_mn : !whole_mn))) continue;
       // the 192x256 tile and the unsplit tiles that stream B (edge kernels without a plain twin) are the planner's own: a tile, wave grid,
       // ring or atom that is asked for names the other variants
-      // (whole 256x256 tiles keep the default kernel: which one they run on is part of the planner's interface, though 144 of them
-      // leave CUs idle -- fp16 3072x3072x4096 NN 70.6 us, 62.4 on 192x256 tiles)
+      // (whole 256x256 tiles keep the default kernel: which one the square sizes run on is part of the planner's interface.  That costs time where they
+      // leave CUs idle -- fp16 3072x3072x4096 NN, 144 of them, 70.6 us, 62.4 on 192x256 tiles -- and holds for every multiple of 256)
       const bool whole_256 = rows_aligned && d->M % 256 == 0 && d->N % 256 == 0 && d->K % k->bk == 0;
       if (planners_own(k) && (tile_requested || d->split_k > 1 || (k->bm == 192 ? small || whole_256 || settled : d->M > 64))) continue;
       // the edge kernels once more under their guarded names: K off the K tile (a whole number of chunks), and anything at all,
