@@ -714,9 +714,9 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
   search(explicit_split);
   if (best < 0 && explicit_split) search(false);
   // A small grid that falls to a kernel without the split-K store path looks at split edge kernels as well, where K is deep enough to split at
-  // all and M fills half of their 128 rows.  (The sweeps behind the tables held none, and beside the split-K kernels the tables flatter them: fp16 100x4096x4096 NN 20.6 us so, 16.8 on
+  // all and the kernel is not one of those that stream B for up to 64 rows.  (The sweeps behind the tables held none, and beside the split-K kernels the tables flatter them: fp16 100x4096x4096 NN 20.6 us so, 16.8 on
   // 64x128 tiles in 4 slices.)
-  if (small && d->M > 64 && best >= 0 && !no_split && d->split_k == 0 && es < 4 && d->K > (es == 1 ? 16 * 128 : 8 * 64) && !ks[best]->splitk && small_grid_split(ks[best], d, left_for_sums(ks[best]), false, false) == 1) {
+  if (small && best >= 0 && !planners_own(ks[best]) && !no_split && d->split_k == 0 && es < 4 && d->K > (es == 1 ? 16 * 128 : 8 * 64) && !ks[best]->splitk && small_grid_split(ks[best], d, left_for_sums(ks[best]), false, false) == 1) {
     split_edges = true;
     search(false);
   }
