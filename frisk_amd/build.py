@@ -28,7 +28,9 @@ COMMON = [
     "-I" + os.path.join(ROOT, "include"), "-I" + CSRC,
     "-Wno-unused-command-line-argument",
 ]
-SOURCES = ["kernels_f16.hip", "kernels_f16_2.hip", "kernels_bf16.hip", "kernels_bf16_2.hip", "kernels_i8.hip", "kernels_i8_2.hip", "kernels_e4m3.hip", "kernels_e4m3_2.hip", "kernels_f32.hip", "kernels_f32_2.hip", "splitk_reduce.hip", "repack.hip", "tile_ops.hip", "elementwise.hip", "softmax.hip", "attention.hip", "capi.cpp"]
+# (the longest units first)
+SOURCES = ["kernels_%s%s.hip" % (t, "" if part == 1 else "_%d" % part) for part in (1, 2, 3, 4) for t in ("f16", "bf16", "i8", "e4m3", "f32") if t != "f32" or part < 3]
+SOURCES += ["splitk_reduce.hip", "repack.hip", "tile_ops.hip", "elementwise.hip", "softmax.hip", "attention.hip", "capi.cpp"]
 
 
 def _compile(src):

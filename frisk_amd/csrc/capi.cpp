@@ -56,16 +56,25 @@ static int fail(int status, const char* fmt, ...) {
 static const std::vector<const KernelEntry*>& kernels() {
   static const std::vector<const KernelEntry*> all = [] {
     std::vector<const KernelEntry*> v;
-    for (int i = 0; i < kNumKernelsF16; ++i) v.push_back(&kKernelsF16[i]);
-    for (int i = 0; i < kNumKernelsF16_2; ++i) v.push_back(&kKernelsF16_2[i]);
-    for (int i = 0; i < kNumKernelsBF16; ++i) v.push_back(&kKernelsBF16[i]);
-    for (int i = 0; i < kNumKernelsBF16_2; ++i) v.push_back(&kKernelsBF16_2[i]);
-    for (int i = 0; i < kNumKernelsI8; ++i) v.push_back(&kKernelsI8[i]);
-    for (int i = 0; i < kNumKernelsI8_2; ++i) v.push_back(&kKernelsI8_2[i]);
-    for (int i = 0; i < kNumKernelsE4M3; ++i) v.push_back(&kKernelsE4M3[i]);
-    for (int i = 0; i < kNumKernelsE4M3_2; ++i) v.push_back(&kKernelsE4M3_2[i]);
-    for (int i = 0; i < kNumKernelsF32; ++i) v.push_back(&kKernelsF32[i]);
-    for (int i = 0; i < kNumKernelsF32_2; ++i) v.push_back(&kKernelsF32_2[i]);
+    auto add = [&](const KernelEntry* table, int n) { for (int i = 0; i < n; ++i) v.push_back(&table[i]); };
+    add(kKernelsF16, kNumKernelsF16);
+    add(kKernelsF16_2, kNumKernelsF16_2);
+    add(kKernelsF16_3, kNumKernelsF16_3);
+    add(kKernelsF16_4, kNumKernelsF16_4);
+    add(kKernelsBF16, kNumKernelsBF16);
+    add(kKernelsBF16_2, kNumKernelsBF16_2);
+    add(kKernelsBF16_3, kNumKernelsBF16_3);
+    add(kKernelsBF16_4, kNumKernelsBF16_4);
+    add(kKernelsI8, kNumKernelsI8);
+    add(kKernelsI8_2, kNumKernelsI8_2);
+    add(kKernelsI8_3, kNumKernelsI8_3);
+    add(kKernelsI8_4, kNumKernelsI8_4);
+    add(kKernelsE4M3, kNumKernelsE4M3);
+    add(kKernelsE4M3_2, kNumKernelsE4M3_2);
+    add(kKernelsE4M3_3, kNumKernelsE4M3_3);
+    add(kKernelsE4M3_4, kNumKernelsE4M3_4);
+    add(kKernelsF32, kNumKernelsF32);
+    add(kKernelsF32_2, kNumKernelsF32_2);
     return v;
   }();
   return all;
@@ -118,16 +127,23 @@ static void wave_partition(int policy, int64_t M, int64_t N, int num_waves, int 
   *wn = (int)std::max<int64_t>(1, n_w);
 }
 
+// Kernels that the search over the variants leaves out, and no descriptor can name: the planner goes over to them from the kernel that the search has
+// found (`follow_up` in make_plan).
+static bool is_follow_up(const KernelEntry* k) {
+  if (k->dtype == FRISK_F32) return k->bm == 32 && k->bn == 32 && !k->splitk;
+  return (k->bm == 64 && k->bn == 64) || (k->bm == 128 && k->bn == 128 && k->edge && k->stages == 3);
+}
+
 // The compiled variants of one element type and pair of layouts, in table order, with what the planner would otherwise work out
 // for each of them on every call: which wave policies their wave grid satisfies (computeWarpPartition gives it for their tile and
 // wave count).  A launch of a 128x128x128 product spent 0.75 of its 3.9 us of host time walking the whole table.
-struct Variant { const KernelEntry* k; int id; bool policy[3]; };
+struct Variant { const KernelEntry* k; int id; bool policy[3]; bool follow_up; };
 static const std::vector<Variant>& variants(int dtype, bool transA, bool transB) {
   static const std::vector<std::vector<Variant>> all = [] {
     std::vector<std::vector<Variant>> v(6 * 4);
     const auto& ks = kernels();
     for (size_t i = 0; i < ks.size(); ++i) {
-      Variant x{ks[i], (int)i, {}};
+      Variant x{ks[i], (int)i, {}, is_follow_up(ks[i])};
       for (int policy = 0; policy < 3; ++policy) {
         int wm = 0, wn = 0;
         wave_partition(policy, x.k->bm, x.k->bn, x.k->wm * x.k->wn, x.k->atom, x.k->atom, &wm, &wn);
@@ -603,6 +619,60 @@ static Repack repack_of(const frisk_gemm_desc* d, bool a, bool b) {
   return r;
 }
 
+// The 128x128 edge tile with 3 + 3 tiles of LDS, which takes over the launch of the one with 2 + 2 as it is, slices included.
+static bool same_edge_tile(const KernelEntry* k) { return k->bm == 128 && k->bn == 128 && k->edge && k->stages == 3; }
+
+// The kernel (its index) that runs a problem in place of `k`, which the search has found with `split` slices of K or `slices` of its edge tiles: -1, that
+// one stays.  A CU fetches at most 100 bytes a nanosecond into LDS whatever the tile and however many tiles are under way (41 bytes a cycle; a
+// loop of nothing but transfers), so where every CU has one work-group at most, the time goes with (rows + columns) x K of the tile.
+static int follow_up(const std::vector<Variant>& list, const KernelEntry* k, const frisk_gemm_desc* d, bool rows_aligned, int split, int slices, const Repack& packed) {
+  const int es = elem_size(k->dtype);
+  const bool staged = k->guard && !k->edge;  // through registers
+  if (staged || split > 1) return -1;
+  auto tiles_of = [&](int bm, int bn) { return ((d->M + bm - 1) / bm) * ((d->N + bn - 1) / bn); };
+  // the variant of a tile for this problem: the plain kernel where it fits, else the edge kernel, named for what it takes (an incumbent that
+  // works on copies of its operands hands them on)
+  auto variant = [&](int bm, int bn, int stages) {
+    const KernelEntry *plain = nullptr, *edge[3] = {};
+    int id = -1, edge_id[3] = {-1, -1, -1};
+    for (const Variant& v : list)
+      if (v.follow_up && v.k->bm == bm && v.k->bn == bn && v.k->stages == stages) {
+        if (v.k->edge) { edge[v.k->guard] = v.k; edge_id[v.k->guard] = v.id; }
+        else { plain = v.k; id = v.id; }
+      }
+    const KernelEntry* x = edge[0] ? edge[0] : plain;
+    if (!x) return -1;
+    const double span_a = (double)(packed.a ? packed.lda : d->lda) * es * (d->transA ? x->bk : x->bm), span_b = (double)(packed.b ? packed.ldb : d->ldb) * es * (d->transB ? x->bn : x->bk);
+    if (span_a >= 4294967296.0 || span_b >= 4294967296.0) return -1;
+    const bool whole_k = d->K % x->bk == 0;
+    if (rows_aligned && whole_k && d->M % bm == 0 && d->N % bn == 0) return id;
+    if (!edge[0]) return -1;
+    return rows_aligned && whole_k ? edge_id[0] : rows_aligned && d->K % (16 / es) == 0 ? edge_id[1] : k->guard == 2 ? edge_id[2] : -1;
+  };
+  if (k->dtype == FRISK_F32) {
+    // 32x32 tiles, the four waves splitting K, on up to 512 work-groups (two a CU): a 64x64 tile keeps its CU's matrix pipe busy and a quarter of
+    // as many leave most CUs without one.  us, operands in the last-level cache, on 64x64 or 32x128 tiles / so: 128x1280x1024 NN 18.9 / 9.1,
+    // 896x256x1792 30.8 / 14.1, 128x384x896 16.3 / 7.6, 256x2048x1408 (512) 24.9 / 17.8; off the tiles 323x130x437 NT 13.8 / 10.0, 8-row problems of 4000 to
+    // 9000 columns half the time; but 512x1152x512 (576) 11.2 / 12.4, 1280x640x768 (800) 16.2 / 19.7, and in a second round on fewer than two K
+    // tiles of 128 296x856x160 (270) 6.2 / 7.2
+    return k->wk == 1 && d->K >= (tiles_of(32, 32) <= 256 ? 128 : 256) && tiles_of(32, 32) <= 512 ? variant(32, 32, 2) : -1;
+  }
+  // (up to 64 rows and 256 tiles of 64x64, 1024x1024 for one, stay on the kernels that the planner has always named for them: fp16 1024^3 NN 7.8 us, 6.7 on 64x64)
+  if (d->M <= 64) return -1;
+  const int64_t k_bytes = d->K * es;
+  const bool edge128 = k->edge && !k->splitk && k->bm == 128 && k->bn == 128;
+  // 64x64 tiles in a single round, in place of 128x128 edge tiles, split or not, and of unsplit 64x128 tiles.  us, operands in the last-level cache:
+  // fp16 525x1136x1480 NT 19.1 / 9.6, 558x296x1200 16.1 / 7.1, 852x824x1840 NN 19.8 / 11.8, 1229x608x3960 22.9 / 18.7, 768x1152x2048 12.0 / 9.3,
+  // e4m3 1408x576x2208 NT 18.7 / 8.2; in place of 64x128 tiles not for less than 1 KiB of K, 906x312x320 NT 5.0 / 5.2; with more than 7.5 KiB the slices have caught up, 494x1144x3768 NN 20.9 / 18.7
+  if (tiles_of(64, 64) < 256 && k_bytes <= 7680 && (edge128 || (k->bm == 64 && k->bn == 128 && k_bytes >= 1024)))
+    if (const int id = variant(64, 64, 3); id >= 0) return id;
+  // 128x128 edge tiles with 3 + 3 tiles of LDS where no CU has two work-groups.  us with 2 + 2 / 3 + 3: fp16 3916x632x2592 NT 32.4 / 24.4, 512x1392x1368 TN
+  // 18.3 / 13.5, 558x296x1200 16.1 / 12.2, e4m3 2304x1664x4048 NN 28.1 / 21.9; under 12 K tiles the longer prologue costs up to 4 %
+  if (edge128 && tiles_of(128, 128) * (tiles_of(128, 128) <= 128 ? slices : 1) <= 256 && (d->K + k->bk - 1) / k->bk >= 12 && !(tiles_of(128, 128) > 128 && slices > 1))
+    return variant(128, 128, 3);
+  return -1;
+}
+
 static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_model, const PlanContext& ctx = {}, LaunchExtras* extras = nullptr) {
   const bool no_split = ctx.workspace == 0;
   int st = validate(d);
@@ -652,6 +722,7 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
   auto search = [&](bool want_split) {
     for (const Variant& v : list) {
       const KernelEntry* k = v.k;
+      if (v.follow_up) continue;
       if (d->tile_m && d->tile_m != k->bm) continue;
       if (d->tile_n && d->tile_n != k->bn) continue;
       if (d->tile_k && d->tile_k != k->bk) continue;
@@ -772,6 +843,13 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
       }
     }
   }
+  // Slices of the edge kernel that the search has found, and of K on a small grid; then the kernels that only follow up on one of the search.
+  const int found_slices = best >= 0 ? edge_slices() : 1;
+  int found_split = 1;
+  if (best >= 0 && small && ks[best]->splitk && !no_split && d->K % ks[best]->bk == 0) found_split = small_grid_split(ks[best], d, ctx.workspace, false, table_range);
+  const bool follows = best >= 0 && !tile_requested && d->split_k <= 1 && d->policy == FRISK_POLICY_SQUARE;
+  if (const int next = follows ? follow_up(list, ks[best], d, rows_aligned, found_split, found_slices, packed) : -1; next >= 0) best = next;
+  const bool one_pass = best >= 0 && is_follow_up(ks[best]) && !same_edge_tile(ks[best]);
   if (d->M == 0 || d->N == 0) {  // nothing to compute
     plan->grid_x = plan->grid_y = 0;
     return FRISK_OK;
@@ -810,7 +888,7 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
     plan->workspace_bytes = packed.bytes;
     if (extras) extras->repack = packed;
   }
-  if (const int ts = edge_slices(); ts > 1) {
+  if (const int ts = one_pass ? 1 : found_slices; ts > 1) {
     const int64_t edge_tiles = (int64_t)plan->grid_x * plan->grid_y, split_tiles = edge_tiles <= 128 ? edge_tiles : edge_tiles % 256;
     const size_t offset = (plan->workspace_bytes + 255) & ~(size_t)255;
     plan->workspace_bytes = offset + (size_t)ts * (size_t)split_tiles * (size_t)k->bm * (size_t)k->bn * 4;
@@ -827,7 +905,7 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
         return fail(FRISK_ERR_TILE, "split_k=%d leaves %lld K tiles per slice, the chosen kernel %s needs %d", d->split_k, (long long)(kt / d->split_k), k->name, k->min_k_tiles);
       split = d->split_k;
     } else if (small) {
-      split = small_grid_split(k, d, ctx.workspace, false, table_range);
+      split = found_split;
     } else if (d->split_k == 0 && tiles < 256) {
       split = sub_round_split(k, d, tiles, kt, ctx.workspace);
     } else if (d->split_k == 0) {
@@ -959,8 +1037,9 @@ int frisk_hip_gemm(const frisk_gemm_desc* desc, const void* A, const void* B, vo
   p.tail_kt = tail_split > 1 ? (p.kt_per_slice + tail_split - 1) / tail_split : 0;
   p.tile_m = k->bm; p.tile_n = k->bn;
   // 64x32 tiles in more than one row share their rows of A and B through the L2, which work-groups at different K tiles do not: us rotated / not, 400 problems
-  // of 65 to 2048 rows, operands in the last-level cache: 8.6 % slower on average, 1024x512x6400 fp16 28.2 / 17.0; from memory 2.8 % faster
-  p.k_rotate = k->bm == 32 || p.tiles_m == 1;
+  // of 65 to 2048 rows, operands in the last-level cache: 8.6 % slower on average, 1024x512x6400 fp16 28.2 / 17.0; from memory 2.8 % faster.  The fp32 tiles of
+  // 32x32 that follow up on larger ones likewise (94 problems, 3.5 % slower rotated, 710x693x3944 73 / 61)
+  p.k_rotate = (k->bm == 32 && !is_follow_up(k)) || p.tiles_m == 1;
   hipError_t e = hipSuccess;
   if (repack.bytes) {
     RepackParams r;

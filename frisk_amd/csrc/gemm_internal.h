@@ -80,23 +80,39 @@ struct RepackParams {
 };
 hipError_t launch_repack(const RepackParams& p, hipStream_t stream);
 
-// defined in kernels_*.hip (two tables per element type: kernels_<type>.hip and kernels_<type>_2.hip)
+// defined in kernels_*.hip (several tables per element type)
 extern const KernelEntry kKernelsF16[];
 extern const int kNumKernelsF16;
 extern const KernelEntry kKernelsF16_2[];
 extern const int kNumKernelsF16_2;
+extern const KernelEntry kKernelsF16_3[];
+extern const int kNumKernelsF16_3;
+extern const KernelEntry kKernelsF16_4[];
+extern const int kNumKernelsF16_4;
 extern const KernelEntry kKernelsBF16[];
 extern const int kNumKernelsBF16;
 extern const KernelEntry kKernelsBF16_2[];
 extern const int kNumKernelsBF16_2;
+extern const KernelEntry kKernelsBF16_3[];
+extern const int kNumKernelsBF16_3;
+extern const KernelEntry kKernelsBF16_4[];
+extern const int kNumKernelsBF16_4;
 extern const KernelEntry kKernelsI8[];
 extern const int kNumKernelsI8;
 extern const KernelEntry kKernelsI8_2[];
 extern const int kNumKernelsI8_2;
+extern const KernelEntry kKernelsI8_3[];
+extern const int kNumKernelsI8_3;
+extern const KernelEntry kKernelsI8_4[];
+extern const int kNumKernelsI8_4;
 extern const KernelEntry kKernelsE4M3[];
 extern const int kNumKernelsE4M3;
 extern const KernelEntry kKernelsE4M3_2[];
 extern const int kNumKernelsE4M3_2;
+extern const KernelEntry kKernelsE4M3_3[];
+extern const int kNumKernelsE4M3_3;
+extern const KernelEntry kKernelsE4M3_4[];
+extern const int kNumKernelsE4M3_4;
 extern const KernelEntry kKernelsF32[];
 extern const int kNumKernelsF32;
 extern const KernelEntry kKernelsF32_2[];

@@ -100,6 +100,14 @@ def square(bk, atom16=False, skinny_ta=(0,)):
     for ta in (0, 1):
         for tb in (0, 1):
             out.append((ta, tb, 128, 128, bk, 2, 2, 2, 1, 0, 1))
+    # Few tiles, one work-group per CU (`follow_up` in capi.cpp): the 128x128 edge tile with 3 + 3 tiles, and 64x64 tiles whose K tile two sets of
+    # four waves share, where A is stored [M][K] (8-bit types: B [N][K] too, transposed rows of 64 bytes are too short)
+    for ta in (0, 1):
+        for tb in (0, 1):
+            out.append(edge((ta, tb, 128, 128, bk, 2, 2, 3, 0, 0, 1, 3)))
+    for tb in (0, 1) if bk == 64 else (1,):
+        out.append((0, tb, 64, 64, 2 * bk, 2, 2, 3, 0, 0, 2))
+        out.append(edge((0, tb, 64, 64, 2 * bk, 2, 2, 3, 0, 0, 2)))
     return out
 
 VARIANTS = {
@@ -126,7 +134,9 @@ VARIANTS = {
             + [(0, 1, 32, 32, 128, 1, 1, 4, 0, 1, 4), (0, 1, 32, 32, 128, 1, 1, 2, 0, 1, 4), (0, 1, 64, 32, 128, 1, 1, 3, 0, 1, 4)]
             + [edge((ta, tb, bm, bm, 32, 2, 2, 2, 0, 0, 1)) for bm in (128, 64) for ta in (0, 1) for tb in (0, 1)]
             + [edge((0, tb, 32, 128, 32, 1, 4, 3, 0, 1, 1)) for tb in (0, 1)] + [edge((0, tb, 64, 64, 32, 2, 2, 3, 0, 1, 1)) for tb in (0, 1)]
-            + [(ta, tb, 64, 64, 32, 2, 2, 2, 1, 0, 1) for ta in (0, 1) for tb in (0, 1)]),
+            + [(ta, tb, 64, 64, 32, 2, 2, 2, 1, 0, 1) for ta in (0, 1) for tb in (0, 1)]
+            # 32x32 tiles, the four waves splitting K, where 64x64 ones leave CUs idle and K is not split (`follow_up` in capi.cpp)
+            + [(0, 0, 32, 32, 128, 1, 1, 2, 0, 0, 4)] + [edge((ta, tb, 32, 32, 128, 1, 1, 2, 0, 0, 4)) for ta in (0, 1) for tb in (0, 1)]),
 }
 
 def cfg_of(enum, v):
@@ -134,15 +144,17 @@ def cfg_of(enum, v):
     return f"GemmCfg<{enum}, {ta}, {tb}, {bm}, {bn}, {bk}, {wm}, {wn}, {st}, {'true' if gd else 'false'}, {'true' if sk else 'false'}, {wk}, {sb}" + (f", {at}, true>" if eg else (f", {at}>" if at != 32 else ">"))
 
 HERE = os.path.dirname(os.path.abspath(__file__))
-# A type's variants go into two translation units of about equal size (kernels_<type>.hip, kernels_<type>_2.hip), each with a
+# A type's variants go into a few translation units of about equal size (kernels_<type>.hip, kernels_<type>_2.hip, ...), each with a
 # table of its own: the units compile in parallel, and the longest of them sets the time of a build.  The planner walks the
-# first table, then the second, so the order of the list above is the order it sees.
+# tables in their order, so the order of the list above is the order it sees.
 written = []
 for tag, (enum, suffix, variants) in VARIANTS.items():
-    half = (len(variants) + 1) // 2
-    for part, chunk in ((1, variants[:half]), (2, variants[half:])):
-        ext = "" if part == 1 else "_2"
-        lines = [f"// {enum} kernel instantiations, part {part} of 2.  Generated by gen_kernels.py; do not edit by hand.",
+    parts = 2 if tag == "f32" else 4
+    size = (len(variants) + parts - 1) // parts
+    for part in range(1, parts + 1):
+        chunk = variants[(part - 1) * size:part * size]
+        ext = "" if part == 1 else f"_{part}"
+        lines = [f"// {enum} kernel instantiations, part {part} of {parts}.  Generated by gen_kernels.py; do not edit by hand.",
                  '#include "gemm_kernel.hip.inc"', "namespace frisk {"]
         for v in chunk:
             lines.append(f"template __global__ void gemm_kernel<{cfg_of(enum, v)}>(GemmParams);")

@@ -1,6 +1,8 @@
 """Problems off the tiles on the device: a K that is no multiple of the K tile on the edge kernels, rows off 16-byte boundaries staged
 through registers (no workspace) and copied to aligned rows first (workspace).  Operands end with their last element, and the
 bytes around C are checked for stray writes."""
+import re
+
 import numpy as np
 import pytest
 
@@ -200,3 +202,37 @@ def test_summed_edge_tiles_apply_scales_and_accumulate(hip, M, N, tail):
         got = run_gemm(hip, O.E4M3, A8, B8, 0, 1, O.BF16, M, N, K8, epilogue=hip.EPI_TENSOR_SCALE, sA=[0.25], sB=[0.02])
         r = O.compare(O.BF16, np.ascontiguousarray(got), O.epilogue_tensor(O.gemm_f64(O.E4M3, A8, B8, False, True), np.float32(0.25), np.float32(0.02)))
         assert r["nonfinite"] == 0 and r["max_rel"] <= TOL[O.BF16] and r["fro_rel"] <= TOL[O.BF16], r
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,transA,transB,tile", [(O.F16, 0, 0, "64x64"), (O.F16, 0, 1, "64x64"), (O.BF16, 0, 0, "64x64"), (O.BF16, 0, 1, "64x64"), (O.I8, 0, 1, "64x64"), (O.E4M3, 0, 1, "64x64"),
+                                                      (O.F16, 1, 1, "128x128"), (O.BF16, 1, 0, "128x128"), (O.I8, 0, 0, "128x128"), (O.E4M3, 1, 0, "128x128"), (O.E4M3, 0, 0, "128x128"),
+                                                      (O.F32, 0, 0, "32x32"), (O.F32, 0, 1, "32x32"), (O.F32, 1, 0, "32x32"), (O.F32, 1, 1, "32x32")])
+def test_tiles_that_follow_up_on_few_larger_ones(hip, dtype, transA, transB, tile):
+    """64x64 and 32x32 tiles whose waves share a K tile and the 128x128 edge tile in a ring of 3: one to seven K tiles, whole and partial; M and N
+    at the end of a tile, one beyond it, and inside a chunk; rows on 16-byte boundaries and copied there; accumulation into C"""
+    per = {"64x64": 128, "128x128": 64, "32x32": 128}[tile] * (1 if tile == "32x32" else 2 // ES[dtype])  # the K tile
+    tiles = {"64x64": (1, 2, 3, 4, 7), "128x128": (13, 14, 16), "32x32": (1, 2, 3, 5)}[tile]
+    ms = {"64x64": (128, 129, 255), "128x128": (130, 257, 383), "32x32": (96, 97, 127)}[tile]
+    seen, cases = set(), []
+    for n in tiles:
+        for M, N, K in ((ms[0], 256, n * per), (ms[1], 200, n * per - 16), (ms[2], 333, n * per + 9)):
+            cases += [(M, N, K, True), (M, N, K, False)]
+    if tile == "64x64":  # whole tiles
+        cases += [(576, 576, 4 * per, True), (960, 704, 8 * per, True)]
+    for i, (M, N, K, aligned) in enumerate(cases):
+        A = make_operand(dtype, *stored_shapes(M, N, K, transA, transB)[0], seed=91 + i, tensor=0, scale=0.5)
+        B = make_operand(dtype, *stored_shapes(M, N, K, transA, transB)[1], seed=91 + i, tensor=1, scale=0.5)
+        got, name, _ = launch(hip, dtype, A, B, M, N, K, transA, transB, aligned, ldc_extra=0 if M % 32 == 0 and aligned else 1)
+        verify(dtype, got, A, B, transA, transB)
+        if "_%sx" % tile in name and ("_s3" in name or tile == "32x32"):
+            seen |= {-(-K // per), "plain" if re.search("_s[23]$", name) else "partial K" if K % per else "whole K", "aligned" if aligned else "copied"}
+    assert seen >= set(tiles[1:]) | {"partial K", "aligned", "copied"} | ({"plain"} if tile == "64x64" or (tile == "32x32" and not transA and not transB) else set()), seen
+    M, N, K = ms[1], 264, tiles[-1] * per - 16
+    A = make_operand(dtype, *stored_shapes(M, N, K, transA, transB)[0], seed=99, tensor=0, scale=0.5)
+    B = make_operand(dtype, *stored_shapes(M, N, K, transA, transB)[1], seed=99, tensor=1, scale=0.5)
+    if dtype != O.I8:
+        C0 = O.uniform(M * N, 99, 2, -1.0, 1.0).reshape(M, N).astype(np.float32)
+        got = run_gemm(hip, dtype, A, B, transA, transB, O.F32, M, N, K, C_init=C0, clear_accum=False)
+        r = O.compare(O.F32, np.ascontiguousarray(got), O.gemm_f64(dtype, A, B, transA, transB) + C0.astype(np.float64))
+        assert r["nonfinite"] == 0 and r["max_rel"] <= TOL[O.F32] and r["fro_rel"] <= TOL[O.F32], r
