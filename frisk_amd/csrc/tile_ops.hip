@@ -198,17 +198,24 @@ reduce_rows_kernel(const typename Elem<DT>::T* src, int64_t rows, int64_t cols, 
   for (int64_t r = blockIdx.x; r < rows; r += gridDim.x) {
     float acc = Op<KIND>::id();
     const T* row = src + r * ld;
-    for (int64_t g = (int64_t)blockIdx.y * 256 + threadIdx.x; g < gpr; g += (int64_t)gridDim.y * 256) {
-      const int64_t c0 = g * G;
-      if (c0 + G <= cols) {
-        T in[G];
-        *(v4u*)in = load16(row + c0);
+    // four groups of a lane under way together, combined in their order (one after the other 98 x 12807 bf16 took 6.2 us, 8192 x 8192 f16 22.9)
+    const int64_t whole = cols / G, step = (int64_t)gridDim.y * 256;
+    int64_t g = (int64_t)blockIdx.y * 256 + threadIdx.x;
+    for (; g < whole; g += 4 * step) {
+      T in[4][G];
 #pragma unroll
-        for (int e = 0; e < G; ++e) acc = Op<KIND>::f(acc, Elem<DT>::load(in[e]));
-      } else {
-        for (int e = 0; e < G && c0 + e < cols; ++e) acc = Op<KIND>::f(acc, Elem<DT>::load(row[c0 + e]));
+      for (int u = 0; u < 4; ++u)
+        if (g + u * step < whole) *(v4u*)in[u] = load16(row + (g + u * step) * G);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        if (g + u * step >= whole) continue;
+#pragma unroll
+        for (int e = 0; e < G; ++e) acc = Op<KIND>::f(acc, Elem<DT>::load(in[u][e]));
       }
     }
+    // the row's last group, if it is not whole, is the last one of its lane (slices are a power of two)
+    if (whole < gpr && (whole & (step - 1)) == (int64_t)blockIdx.y * 256 + threadIdx.x)
+      for (int64_t c = whole * G; c < cols; ++c) acc = Op<KIND>::f(acc, Elem<DT>::load(row[c]));
     acc = wave_reduce<KIND>(acc);
     if ((threadIdx.x & 63) == 0) wsum[threadIdx.x >> 6] = acc;
     __syncthreads();
@@ -328,6 +335,65 @@ reduce_cols_kernel(const typename Elem<DT>::T* src, int64_t rows, int64_t cols, 
   }
 }
 
+// along dim 0 in one launch, for views that would otherwise be split down the rows but have few enough of them (cols_in_one_launch): 1024 lanes on
+// a strip of 8 x 16 bytes (or fewer, of a narrower view), eight rows under way per lane.  The row lanes of a wave combine by shuffles, the waves in
+// LDS.  What it saves is the launch that combines the slices: us in two launches / so, f16 309 x 3904 6.9 / 4.1, 256 x 1024 7.0 / 4.1, 1259 x 1728 7.6 /
+// 6.3, f32 309 x 3904 7.4 / 4.3.  A work-group walks its strip at some 40 bytes a nanosecond (1024 lanes, of which all wait, then all add), so from
+// 2000 rows on the slices are ahead again (f16 2000 x 1984 7.9 / 8.3, 3000 x 1024 8.6 / 13.3), and so they are where there is more than one strip for
+// every CU (1000 x 65536 25.2 / 27.7).
+template <int DT, int KIND> __global__ void __launch_bounds__(1024)
+reduce_tall_kernel(const typename Elem<DT>::T* src, int64_t rows, int64_t cols, int64_t ld, int clear, typename Elem<DT>::T* dst, int lanes_log2) {
+  typedef typename Elem<DT>::T T;
+  constexpr int G = 16 / sizeof(T), FLIGHT = 8;
+  const int lanes = 1 << lanes_log2, cl = threadIdx.x & (lanes - 1), rl = threadIdx.x >> lanes_log2, row_lanes = 1024 >> lanes_log2;
+  const int64_t c0 = (((int64_t)blockIdx.x << lanes_log2) + cl) * G;
+  float acc[G];
+#pragma unroll
+  for (int e = 0; e < G; ++e) acc[e] = Op<KIND>::id();
+  if (c0 + G <= cols) {
+    for (int64_t r = rl; r < rows; r += FLIGHT * row_lanes) {
+      T in[FLIGHT][G];
+#pragma unroll
+      for (int u = 0; u < FLIGHT; ++u)
+        if (r + u * row_lanes < rows) *(v4u*)in[u] = load16(src + (r + u * row_lanes) * ld + c0);
+#pragma unroll
+      for (int u = 0; u < FLIGHT; ++u) {
+        if (r + u * row_lanes >= rows) continue;
+#pragma unroll
+        for (int e = 0; e < G; ++e) acc[e] = Op<KIND>::f(acc[e], Elem<DT>::load(in[u][e]));
+      }
+    }
+  } else if (c0 < cols) {
+    for (int64_t r = rl; r < rows; r += row_lanes) {
+#pragma unroll
+      for (int e = 0; e < G; ++e)
+        if (c0 + e < cols) acc[e] = Op<KIND>::f(acc[e], Elem<DT>::load(src[r * ld + c0 + e]));
+    }
+  }
+  for (int off = 32; off >= lanes; off >>= 1) {
+#pragma unroll
+    for (int e = 0; e < G; ++e) acc[e] = Op<KIND>::f(acc[e], __shfl_xor(acc[e], off, 64));
+  }
+  __shared__ float red[16][8 * G];  // [wave][column of the strip]
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  if (lane < lanes) {
+#pragma unroll
+    for (int e = 0; e < G; ++e) red[wave][lane * G + e] = acc[e];
+  }
+  __syncthreads();
+  const int64_t c = ((int64_t)blockIdx.x << lanes_log2) * G + threadIdx.x;
+  if ((int)threadIdx.x >= lanes * G || c >= cols) return;
+  float part[16];  // in pairs: in a row the 16 came out 1.2 times as far from the exact sum as the slices did
+#pragma unroll
+  for (int w = 0; w < 16; ++w) part[w] = red[w][threadIdx.x];
+#pragma unroll
+  for (int half = 8; half >= 1; half >>= 1)
+#pragma unroll
+    for (int w = 0; w < half; ++w) part[w] = Op<KIND>::f(part[w], part[w + half]);
+  const float v = part[0];
+  dst[c] = Elem<DT>::store(clear ? v : Op<KIND>::f(Elem<DT>::load(dst[c]), v));
+}
+
 // second pass of a split reduction: out[i] = kind over s of partial[s][i] (combined with dst unless clear).  64 outputs x 4
 // slice lanes per work-group: a lane combines every fourth slice with four loads in flight, so that 256 slices cost 16
 // memory round trips instead of 256.
@@ -396,6 +462,22 @@ template <int SDT, int DDT> hipError_t copy_tiles_t(const void* src, int64_t sld
 // a launch may hold fewer than 2^32 lanes: grids are capped and work-groups loop
 constexpr int64_t kMaxGrid = 1 << 22;
 
+// (`gpr`: groups of 16 bytes in a row)
+bool cols_in_one_launch(int64_t rows, int64_t gpr) { return rows <= 1536 && gpr <= 256 * 8; }
+
+// slices of the reduced extent that give the launch enough work-groups
+int split_of(int dtype, int64_t rows, int64_t cols, int dim) {
+  // Split the reduced extent so that about 1024 work-groups exist, each still reducing at least 16 KiB.
+  const int es = dtype == FRISK_F32 ? 4 : 2;
+  const int G = 16 / es;
+  const int64_t groups = dim == 1 ? rows : (cols + kStripLanes * G - 1) / (kStripLanes * G);
+  const int64_t strip_bytes = cols * es < kStripLanes * 16 ? cols * es : kStripLanes * 16;
+  const int64_t extent_bytes = dim == 1 ? cols * es : rows * strip_bytes;  // bytes one work-group would walk unsplit
+  int slices = 1;
+  while (groups * slices < 1024 && extent_bytes / (slices * 2) >= 16384 && slices < 256) slices *= 2;
+  return slices;
+}
+
 template <int DT, int KIND> hipError_t reduce_t(const void* src, int64_t rows, int64_t cols, int64_t ld, int dim, int clear, void* dst, float* partial,
                                                 int slices, hipStream_t s) {
   typedef typename Elem<DT>::T T;
@@ -414,6 +496,11 @@ template <int DT, int KIND> hipError_t reduce_t(const void* src, int64_t rows, i
       hipLaunchKernelGGL((reduce_rows_kernel<DT, KIND>), dim3((unsigned)(rows < kMaxGrid ? rows : kMaxGrid), (unsigned)slices), dim3(256), 0, s, (const T*)src, rows, cols,
                          ld, clear, (T*)dst, partial);
     }
+  } else if (slices == 1 && split_of(DT, rows, cols, dim) > 1 && cols_in_one_launch(rows, gpr)) {
+    int lanes_log2 = 0;
+    while (lanes_log2 < 3 && (int64_t(1) << lanes_log2) < gpr) ++lanes_log2;
+    hipLaunchKernelGGL((reduce_tall_kernel<DT, KIND>), dim3((unsigned)((gpr + (1 << lanes_log2) - 1) >> lanes_log2)), dim3(1024), 0, s, (const T*)src, rows, cols, ld, clear,
+                       (T*)dst, lanes_log2);
   } else {
     int lanes_log2 = 0;
     while ((1 << lanes_log2) < kStripLanes && (int64_t(1) << lanes_log2) < gpr) ++lanes_log2;
@@ -445,15 +532,8 @@ template <int DT> hipError_t reduce_k(int kind, const void* src, int64_t rows, i
 }  // namespace
 
 int reduce_slices(int dtype, int64_t rows, int64_t cols, int dim) {
-  // Split the reduced extent so that about 1024 work-groups exist, each still reducing at least 16 KiB.
-  const int es = dtype == FRISK_F32 ? 4 : 2;
-  const int G = 16 / es;
-  const int64_t groups = dim == 1 ? rows : (cols + kStripLanes * G - 1) / (kStripLanes * G);
-  const int64_t strip_bytes = cols * es < kStripLanes * 16 ? cols * es : kStripLanes * 16;
-  const int64_t extent_bytes = dim == 1 ? cols * es : rows * strip_bytes;  // bytes one work-group would walk unsplit
-  int slices = 1;
-  while (groups * slices < 1024 && extent_bytes / (slices * 2) >= 16384 && slices < 256) slices *= 2;
-  return slices;
+  const int64_t gpr = (cols * (dtype == FRISK_F32 ? 4 : 2) + 15) / 16;
+  return dim == 0 && cols_in_one_launch(rows, gpr) ? 1 : split_of(dtype, rows, cols, dim);
 }
 
 hipError_t launch_fill(int dtype, void* dst, int64_t rows, int64_t cols, int64_t ld, double value, hipStream_t s) {

@@ -1,10 +1,11 @@
-"""The passes beside the products at the edges of their loops: the sums of split-K slices and of split edge tiles."""
-or in one launch, and the last group of a row in block bodies."""
+"""The passes beside the products at the edges of their loops: the sums of split-K slices, reductions whose loads are under way several at a time
+or in one launch."""
 import numpy as np
 import pytest
 
 import oracle as O
 from helpers import make_operand, run_gemm
+from oracle import tile_ops as T
 
 
 @pytest.mark.gpu
@@ -29,3 +30,34 @@ def test_the_sum_of_split_edge_tiles_is_exact(hip, columns):
     M, N, K = 193, 128 * columns - 5, 128 * 16 * 8
     A, B = make_operand(O.I8, M, K, 62, 0), make_operand(O.I8, K, N, 62, 1)
     assert np.array_equal(run_gemm(hip, O.I8, A, B, 0, 0, O.I32, M, N, K), O.gemm_i32(A, B))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", [O.F32, O.F16, O.BF16])
+@pytest.mark.parametrize("rows,cols,dim", [
+    (129, 8, 0), (1023, 40, 0), (1024, 65, 0), (1025, 500, 0), (1535, 9, 0), (1536, 64, 0), (1537, 64, 0), (1200, 16384, 0), (1200, 16385, 0), (1500, 3, 0),  # one launch, and beyond it
+    (3, 2049, 1), (3, 4096, 1), (2, 8191, 1), (2, 8192, 1), (5, 8193, 1), (3, 10248, 1), (2, 40000, 1), (1, 65543, 1)])                                        # 1 to 5 groups a lane, slices
+def test_reductions_with_several_loads_under_way(hip, dt, rows, cols, dim):
+    import torch
+    ld, st = cols + 3, O.NP_STORAGE[dt]
+    vals = O.encode(dt, O.normal(rows * cols, 63, 0, 1.0)).reshape(rows, cols)
+    src = np.zeros((rows, ld), st)
+    src[:, :cols] = vals
+    x = torch.from_numpy(src.view(np.uint8).reshape(-1).copy()).cuda()
+    kept = rows if dim == 1 else cols
+    old = O.encode(dt, O.normal(kept, 63, 1, 0.5))
+    need = hip.reduce_workspace_bytes(dt, rows, cols, dim)
+    ws = torch.full((max(need, 4),), 0xFF, dtype=torch.uint8, device="cuda")
+    for kind, clear in (("max", True), ("min", False), ("add", True), ("add", False)):
+        d = torch.from_numpy(old.view(np.uint8).reshape(-1).copy()).cuda()
+        hip.reduce(dt, x.data_ptr(), rows, cols, ld, dim, kind, clear, d.data_ptr(), ws.data_ptr() if need else None, need, torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        got = d.cpu().numpy().view(st)
+        if kind != "add":
+            assert np.array_equal(got, T.reduce(dt, vals, dim, kind, None if clear else old)), (kind, clear)
+            continue
+        want = T.reduce_f64(dt, vals, dim, kind, None if clear else old).astype(np.float64).reshape(-1)
+        # one rounding to the element type of |sum| <= sum of |x|, and fp32 sums of at most 64 + 10 additions in a row each
+        size = np.abs(O.decode(dt, vals).astype(np.float64)).sum(axis=dim).reshape(-1) + np.abs(O.decode(dt, old).astype(np.float64))
+        bound = {O.F32: 2.0 ** -24, O.F16: 2.0 ** -11, O.BF16: 2.0 ** -8}[dt] * np.abs(want) + 2.0 ** -24 * 80 * size
+        assert np.all(np.abs(O.decode(dt, got).astype(np.float64) - want) <= bound)
