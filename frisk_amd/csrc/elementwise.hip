@@ -10,7 +10,7 @@
 // place, the operand picked by the register index mode.  (As a C++ switch the compiler joins the values of all cases after every
 // step by register moves: 327 vector, 300 scalar and 120 branch instructions per group of 8 columns for (x - s * c) * g + b; here
 // 109, 125 and 34.)  That body on 8192 x 8192 f16: 137 us before, 51 now (a plain copy: 41); log2(max(x, c) / (x + c)), bound by
-// the vector pipe in its division, 123 -> 69.5; x + y 80 -> 71; rows off 16-byte boundaries (4095 x 8191) 369 -> 46.
+// the vector pipe in its division, 123 -> 69.5; x + y 80 -> 65; rows off 16-byte boundaries (4095 x 8191) 369 -> 29.
 // Operands that are the same for every row stay in registers while the lane's columns do, values of one per row stay one
 // register, and what the next groups need from memory is fetched while the current one is evaluated.  All arithmetic is
 // fp32; the result is rounded once to the output type.
@@ -122,29 +122,19 @@ __device__ __forceinline__ Raw load_raw(const char* at, int dt, bool streamed) {
   }
   return r;
 }
-// The first `valid` (1 to 7) of 8 elements.  TOGETHER: without branches, the last one again in place of those beyond it, so that all are under way
-// together: what a small view waits for (300 x 77 f16: x g + b 4.7 -> 3.9 us); the kernels for long rows keep the branches, which cost them fewer
-// registers (8192 x 8192 f16, (x - s c) g + b: 51.5 us, 53.2 without).
-template <bool TOGETHER> __device__ __forceinline__ Raw load_raw_partial(const char* at, int dt, int valid) {
+// The first `valid` (1 to 7) of 8 elements, of a row that has no more: without branches, the last one again in place of those beyond it, so that all
+// are under way together
+__device__ __forceinline__ Raw load_raw_narrow(const char* at, int dt, int valid) {
   unsigned w[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-  if constexpr (TOGETHER) {
-    if (dt == FRISK_F32) {
+  if (dt == FRISK_F32) {
 #pragma unroll
-      for (int e = 0; e < V; ++e) w[e] = ((const unsigned*)at)[e < valid ? e : valid - 1];
-    } else {
-      unsigned h[V];
-#pragma unroll
-      for (int e = 0; e < V; ++e) h[e] = ((const uint16_t*)at)[e < valid ? e : valid - 1];
-#pragma unroll
-      for (int e = 0; e < V; ++e) w[e / 2] |= h[e] << (16 * (e & 1));
-    }
+    for (int e = 0; e < V; ++e) w[e] = ((const unsigned*)at)[e < valid ? e : valid - 1];
   } else {
+    unsigned h[V];
 #pragma unroll
-    for (int e = 0; e < V; ++e) {
-      if (e >= valid) continue;
-      if (dt == FRISK_F32) w[e] = ((const unsigned*)at)[e];
-      else w[e / 2] |= (unsigned)((const uint16_t*)at)[e] << (16 * (e & 1));
-    }
+    for (int e = 0; e < V; ++e) h[e] = ((const uint16_t*)at)[e < valid ? e : valid - 1];
+#pragma unroll
+    for (int e = 0; e < V; ++e) w[e / 2] |= h[e] << (16 * (e & 1));
   }
   return Raw{v4u{w[0], w[1], w[2], w[3]}, v4u{w[4], w[5], w[6], w[7]}};
 }
@@ -171,8 +161,9 @@ __device__ __forceinline__ float load_one(const char* at, int dt) {
   if (dt == FRISK_F16) return (float)*(const _Float16*)at;
   return (float)*(const __bf16*)at;
 }
-__device__ __forceinline__ void store_group(char* at, int dt, const v8f& r, int valid) {
-  if (valid >= V) {
+// columns first .. last - 1 of a group that starts at `at`
+__device__ __forceinline__ void store_group(char* at, int dt, const v8f& r, int first, int last) {
+  if (first == 0 && last == V) {
     if (dt == FRISK_F32) {
       v4u a, b;
 #pragma unroll
@@ -196,7 +187,7 @@ __device__ __forceinline__ void store_group(char* at, int dt, const v8f& r, int 
   }
 #pragma unroll
   for (int e = 0; e < V; ++e) {
-    if (e >= valid) continue;
+    if (e < first || e >= last) continue;
     if (dt == FRISK_F32) ((float*)at)[e] = r[e];
     else if (dt == FRISK_F16) ((_Float16*)at)[e] = (_Float16)r[e];
     else ((__bf16*)at)[e] = (__bf16)r[e];
@@ -207,19 +198,21 @@ __device__ __forceinline__ void store_group(char* at, int dt, const v8f& r, int 
 // `head` are held or fetched ahead: none; the second one that walks the rows; that one and the broadcast ones (44 more registers for 32-bit
 // operands, 32 for 16-bit ones, and 1500 instructions in front of the first step instead of 650: x + y of 1024 x 4096 f16 7.4 us with them,
 // 6.5 without, f32 11.3 and 9.9, 100000 x 24 f16 5.6 and 4.5, 8192 x 8192 f16 74.4 and 71).  DEPTH: values below the top the program needs.
-// UNIFORM_ROW: a wave's lanes lie in one row (rows of at least 64 groups).
+// ROWS: a wave's lanes lie in several rows, in one (rows of at least 64 groups), or in one each, of less than a group (as a case of the first, its loads
+// cost that one 0.4 us in 4.8 of 6304 x 136 f16).
+enum Rows { ROWS_SHARED, ROWS_UNIFORM, ROWS_NARROW };
 enum Held { HELD_NONE, HELD_WALK, HELD_ALL };
 // Kernels that hold all of them run four waves a SIMD where their registers allow it ((x - s c) g + b of 100000 x 24 f16: 136 registers and three
 // waves 8.6 us, 7.4 with four).
 constexpr bool four_waves(int dt, int held, int depth, bool uniform_row) { return held == HELD_ALL && depth == 1 && !(dt == FRISK_F32 && !uniform_row); }
-template <int DT, int HELD, int DEPTH, bool UNIFORM_ROW> __global__ void __launch_bounds__(256)
-__attribute__((amdgpu_waves_per_eu(four_waves(DT, HELD, DEPTH, UNIFORM_ROW) ? 4 : 1, four_waves(DT, HELD, DEPTH, UNIFORM_ROW) ? 4 : 8))) elementwise_kernel(EwArgs p, int lanes_log2) {
+template <int DT, int HELD, int DEPTH, int ROWS> __global__ void __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(four_waves(DT, HELD, DEPTH, ROWS == ROWS_UNIFORM) ? 4 : 1, four_waves(DT, HELD, DEPTH, ROWS == ROWS_UNIFORM) ? 4 : 8))) elementwise_kernel(EwArgs p, int lanes_log2) {
   const int lanes = 1 << lanes_log2, row_step = 256 >> lanes_log2;
   const int lane_group = threadIdx.x & (lanes - 1);
   int lane_row = threadIdx.x >> lanes_log2;
-  if constexpr (UNIFORM_ROW) lane_row = __builtin_amdgcn_readfirstlane(lane_row);
+  if constexpr (ROWS == ROWS_UNIFORM) lane_row = __builtin_amdgcn_readfirstlane(lane_row);
   const int64_t groups = (p.cols + V - 1) / V, slabs = (groups + lanes - 1) >> lanes_log2, row_blocks = (p.rows + row_step - 1) / row_step;
-  const bool ragged = p.cols % V != 0;
+  constexpr bool narrow = ROWS == ROWS_NARROW;
   // step i of a chunk of the program in lane i: a lane read instead of a dependent scalar load
   int code_reg[2] = {p.code[threadIdx.x & 63], 0}, imm_reg[2] = {__builtin_bit_cast(int, p.imm[threadIdx.x & 63]), 0};
   if (p.n_steps > kChunk) {
@@ -241,19 +234,23 @@ __attribute__((amdgpu_waves_per_eu(four_waves(DT, HELD, DEPTH, UNIFORM_ROW) ? 4 
     // lanes beyond the view repeat its last row or group and store nothing
     const int64_t left = groups - (slab << lanes_log2);
     const int off = lane_group < left ? lane_group : (int)left - 1;
-    const int64_t first_col = ((slab << lanes_log2) + off) * V;
-    const int valid = p.cols - first_col < V ? (int)(p.cols - first_col) : V;
+    // A row's last group, where it is not whole, is evaluated together with the columns before it that fill it up: every load is then 16 bytes of
+    // the row.  The lane stores columns `mine` and up of its 8, the others being the neighbour's (whose store may have come first where the
+    // output is an operand too).  Fetched element by element behind branches, that group held up every row: (x - s c) g + b of 4095 x 8191 bf16 47.6 us, 32.3 so,
+    // 16000 x 3999 f16 99.0 and 61.0, 6330 x 669 17.7 and 11.9.
+    const int64_t past = ((slab << lanes_log2) + off + 1) * V - p.cols;
+    const int mine = past > 0 && !narrow ? (int)past : 0, last = narrow ? (int)p.cols : V, lane_col = off * V - mine;
     int64_t row = rb0 * row_step + lane_row;
     const int64_t row_in = row < p.rows ? row : p.rows - 1;
     // element (r, first column of the group) of an operand whose elements are of type dt
     auto operand_at = [&](const EwOperand& k, int dt, bool walks, int64_t r) {
       const int es = dt == FRISK_F32 ? 4 : 2;
       const char* base = k.at + r * k.row_bytes;
-      return walks ? base + (slab << lanes_log2) * (V * es) + (unsigned)(off * (V * es)) : base;
+      return walks ? base + (slab << lanes_log2) * (V * es) + lane_col * es : base;
     };
     auto fetch_at = [&](const char* at, int dt, bool streamed) {
-      if (!ragged || valid >= V) return load_raw(at, dt, streamed);
-      return load_raw_partial<!UNIFORM_ROW && HELD != HELD_ALL>(at, dt, valid);
+      if constexpr (narrow) return load_raw_narrow(at, dt, last);
+      else return load_raw(at, dt, streamed);
     };
     auto fetch_row_at = [&](const char* at, int dt) { return dt == FRISK_F32 ? *(const unsigned*)at : (unsigned)*(const uint16_t*)at; };
     const char *head_at = nullptr, *walk2_at = nullptr, *row0_at = nullptr, *row1_at = nullptr;
@@ -267,12 +264,12 @@ __attribute__((amdgpu_waves_per_eu(four_waves(DT, HELD, DEPTH, UNIFORM_ROW) ? 4 
       if (p.row1.at) { row1_at = operand_at(p.row1, p.row1.dt, false, row_in); row1_step = row_stride * p.row1.row_bytes; }
     }
     const int out_dt = DT >= 0 ? DT : p.out_dt, out_es = out_dt == FRISK_F32 ? 4 : 2;
-    char* out_at = p.out + row_in * p.out_row_bytes + (slab << lanes_log2) * (V * out_es) + (unsigned)(off * (V * out_es));
+    char* out_at = p.out + row_in * p.out_row_bytes + (slab << lanes_log2) * (V * out_es) + lane_col * out_es;
     const int64_t out_step = row_stride * p.out_row_bytes;
 
     // what is under way from memory: the next group of 32-bit operands, the next two of 16-bit ones (16 bytes a lane and four waves a SIMD
     // are a third of what the memory's latency asks for: one group ahead 195.2 us for the four calls of cast, mean, scale and shift, softmax on 8192 x 8192 f16, two 191.8)
-    constexpr int SETS = (DT == FRISK_F16 || DT == FRISK_BF16) && DEPTH == 1 && UNIFORM_ROW ? 2 : 1;
+    constexpr int SETS = (DT == FRISK_F16 || DT == FRISK_BF16) && DEPTH == 1 && ROWS == ROWS_UNIFORM ? 2 : 1;
     struct Ahead { Raw head, walk2; unsigned row0, row1; } held0{}, held1{};
     v8f col0{}, col1{};
     auto fetch_ahead = [&](Ahead& h) __attribute__((always_inline)) {
@@ -360,7 +357,7 @@ __attribute__((amdgpu_waves_per_eu(four_waves(DT, HELD, DEPTH, UNIFORM_ROW) ? 4 
           for (int e = 0; e < V; ++e) top[e] = top[e] / x[e];
         }
       }
-      if (live) store_group(out_at, out_dt, top, valid);
+      if (live) store_group(out_at, out_dt, top, mine, last);
       out_at += out_step;
       row += row_stride;
       rb += gridDim.y;
@@ -435,9 +432,10 @@ EwSteps steps_of(const EwParams& p, int held) {
 static_assert(2 * FRISK_EW_MAX_OPS + 2 <= 2 * kChunk, "a program fits into two chunks");
 
 template <int DT, int HELD> void launch_typed(const dim3& grid, const EwArgs& a, int depth, int lanes_log2, hipStream_t s) {
-#define FRISK_EW_LAUNCH(DEPTH)                                                                                                 \
-  if (lanes_log2 >= 6) hipLaunchKernelGGL((elementwise_kernel<DT, HELD, DEPTH, true>), grid, dim3(256), 0, s, a, lanes_log2); \
-  else hipLaunchKernelGGL((elementwise_kernel<DT, HELD, DEPTH, false>), grid, dim3(256), 0, s, a, lanes_log2);
+#define FRISK_EW_LAUNCH(DEPTH)                                                                                                                   \
+  if (a.cols < V) hipLaunchKernelGGL((elementwise_kernel<DT, HELD, DEPTH, ROWS_NARROW>), grid, dim3(256), 0, s, a, lanes_log2);                 \
+  else if (lanes_log2 >= 6) hipLaunchKernelGGL((elementwise_kernel<DT, HELD, DEPTH, ROWS_UNIFORM>), grid, dim3(256), 0, s, a, lanes_log2);      \
+  else hipLaunchKernelGGL((elementwise_kernel<DT, HELD, DEPTH, ROWS_SHARED>), grid, dim3(256), 0, s, a, lanes_log2);
   if (depth <= 1) { FRISK_EW_LAUNCH(1) } else { FRISK_EW_LAUNCH(5) }
 #undef FRISK_EW_LAUNCH
 }
@@ -454,7 +452,7 @@ hipError_t launch_elementwise(const EwParams& given, hipStream_t s) {
   // A dense view is one row, down which no lane walks and fetches ahead.  A 16-bit one that gives every lane more than one group is folded to
   // rows of one group a lane (8192 x 8192 f16: log2(max(x, c) / (x + c)) 73.6 -> 69.5 us, x * y + z 95.7 -> 95.4; f32, of which one group less
   // is under way, lost: 117 -> 119).
-  constexpr int64_t kFold = 256 * V, kCap = 256 * 16;
+  constexpr int64_t kFold = 256 * V, kCap = 256 * 16, kHeldCap = 256 * 4;
   bool half = p.out_dtype != FRISK_F32;
   for (int k = 0; k < FRISK_EW_MAX_INPUTS; ++k) half = half && (p.in_col_stride[k] == 0 || p.in_dtype[k] == p.out_dtype);
   if (p.rows == 1 && half && p.cols % kFold == 0 && p.cols / kFold > kCap) {
@@ -466,20 +464,31 @@ hipError_t launch_elementwise(const EwParams& given, hipStream_t s) {
   int lanes_log2 = 0;
   while (lanes_log2 < 8 && ((int64_t)1 << lanes_log2) < groups) ++lanes_log2;
   const int64_t lanes = (int64_t)1 << lanes_log2, row_step = 256 >> lanes_log2;
-  // enough work-groups to fill the chip several times over, every lane walking its row / column strides beyond that
+  // Enough work-groups to fill the chip several times over, every lane walking its row / column strides beyond that: 16 per CU; of the kernels that
+  // hold more than the first operand 4 per CU, a single round of those with broadcast operands (four waves a SIMD), so that what stands in front of the
+  // first group (up to 1000 instructions) is paid once per lane.  us with 16 / 4 per CU: (x - s c) g + b of 8192 x 8192 f16 54.8 / 51.6, 3000 x 4096 16.7 /
+  // 11.5, 6330 x 669 11.9 / 8.8, 4095 x 8191 bf16 32.3 / 28.5, 4000 x 4096 f32 28.1 / 26.0; x + y of 8192 x 8192 f16 69 / 64, 16000 x 3999 63.1 / 60.2; but
+  // exp2(x) c of 16000 x 3999 44.7 / 48.1, and f32, with one group a lane under way, where 16 per CU still leave eight rows to a lane (8192 x 8192 101.8 /
+  // 106.5; 20000 x 2048 61.7 / 61.0).
   const int64_t row_blocks = (p.rows + row_step - 1) / row_step;
-  int64_t gx = (groups + lanes - 1) / lanes, gy = row_blocks;
-  if (gx > kCap) gx = kCap;
-  if (gx * gy > kCap) gy = (kCap + gx - 1) / gx;
-  if (gy > 65535) gy = 65535;
-  // Holding the broadcast operands pays where a lane walks down several rows, not where its one group waits for them to be set up (us held / not:
-  // x + b of 1024 x 4096 f16 7.6 / 5.8, f32 9.2 / 8.0, 300 x 77 f16 4.5 / 3.7; (x - s c) g + b of 100000 x 24 f16 8.6 / 6.9)
+  int64_t gx = 0, gy = 0;
+  auto set_grid = [&](int64_t cap) {
+    gx = (groups + lanes - 1) / lanes;
+    gy = row_blocks;
+    if (gx > cap) gx = cap;
+    if (gx * gy > cap) gy = (cap + gx - 1) / gx;
+    if (gy > 65535) gy = 65535;
+  };
+  // Holding the broadcast operands pays where a lane walks down two rows or more, not where its one group waits for them to be set up (us held / not,
+  // two rows a lane: (x - s c) g + b of 1024 x 4096 f16 6.8 / 8.3, f32 9.4 / 10.3, 100000 x 24 f16 5.8 / 6.6, x + b of 1024 x 4096 f32 8.5 / 8.0)
+  set_grid(kHeldCap);
   const int most = (row_blocks + gy - 1) / gy >= 2 ? HELD_ALL : HELD_WALK;
   // one type for everything that moves with the rows: the kernels for it; mixed types: the one that looks at each operand's type,
   // which holds nothing ahead but the first operand
   EwSteps prog = steps_of(p, most);
   int dt = p.out_dtype;
   int held = prog.col0 >= 0 || prog.row0 >= 0 ? HELD_ALL : prog.walk2 >= 0 ? HELD_WALK : HELD_NONE;
+  if (held == HELD_NONE || (dt == FRISK_F32 && ((groups + lanes - 1) / lanes) * row_blocks >= 8 * kCap)) set_grid(kCap);
   // f32 with three groups a lane and more: the larger kernel's four waves a SIMD stream better than five of the smaller one (us, four / five:
   // x + y of 8192 x 8192 142 / 147, 20000 x 2048 87.6 / 90.5, 4095 x 8191 72.0 / 73.3; 4096 x 4096, two groups a lane, 38.7 / 37.3)
   if (dt == FRISK_F32 && held == HELD_WALK && ((groups + lanes - 1) / lanes) * row_blocks >= 3 * gx * gy) held = HELD_ALL;
@@ -487,6 +496,7 @@ hipError_t launch_elementwise(const EwParams& given, hipStream_t s) {
     dt = -1;
     held = HELD_NONE;
     prog = steps_of(p, HELD_NONE);
+    set_grid(kCap);
   }
   EwArgs a{};
   a.rows = p.rows; a.cols = p.cols;

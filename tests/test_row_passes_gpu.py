@@ -1,5 +1,5 @@
 """The passes beside the products at the edges of their loops: the sums of split-K slices, reductions whose loads are under way several at a time
-or in one launch."""
+or in one launch, and the last group of a row in block bodies."""
 import numpy as np
 import pytest
 
@@ -61,3 +61,32 @@ def test_reductions_with_several_loads_under_way(hip, dt, rows, cols, dim):
         size = np.abs(O.decode(dt, vals).astype(np.float64)).sum(axis=dim).reshape(-1) + np.abs(O.decode(dt, old).astype(np.float64))
         bound = {O.F32: 2.0 ** -24, O.F16: 2.0 ** -11, O.BF16: 2.0 ** -8}[dt] * np.abs(want) + 2.0 ** -24 * 80 * size
         assert np.all(np.abs(O.decode(dt, got).astype(np.float64) - want) <= bound)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt,tdt", [(O.F32, "float32"), (O.F16, "float16"), (O.BF16, "bfloat16")])
+@pytest.mark.parametrize("rows", [1, 5, 2600])
+def test_the_last_group_of_a_row(hip, dt, tdt, rows):
+    """rows of a whole number of groups of 8 columns and of 1 to 7 columns more, shorter than a group, than a wave, than a work-group and longer; into
+    another matrix and into its own operand.  Every operation rounds to fp32 once, as torch's do: the same bits."""
+    import torch
+    tdt = getattr(torch, tdt)
+    g = torch.Generator(device="cuda").manual_seed(5)
+    stream = torch.cuda.current_stream().cuda_stream
+    for cols in (1, 5, 7, 8, 9, 12, 15, 17, 127, 131, 511, 513, 518, 2047, 2054) + ((20003,) if rows < 100 else ()):
+        ld = cols + 1
+        x, z = (torch.randn(rows, ld, device="cuda", generator=g).to(tdt) for _ in range(2))
+        r, c = torch.randn(rows, device="cuda", generator=g).to(tdt), torch.randn(cols, device="cuda", generator=g).to(tdt)
+        body = [("input", 0), ("input", 1), "sub", ("input", 2), "mul", ("input", 3), "add"]
+        for operands, program, want in (
+                ([x, r, c, z], body, (x.float()[:, :cols] - r.float()[:, None]) * c.float() + z.float()[:, :cols]),
+                ([x, z], [("input", 0), ("input", 1), "add"], x.float()[:, :cols] + z.float()[:, :cols]),
+                ([x], [("input", 0), ("const", 0.75), "mul"], x.float()[:, :cols] * 0.75)):
+            strides = [(dt, ld, 1) if t is x or t is z else (dt, 1, 0) if t is r else (dt, 0, 1) for t in operands]
+            desc = hip.make_elementwise_desc(program, strides, dt, rows, cols, out_ld=ld)
+            for out in (torch.full_like(x, 3.0), x.clone()):
+                beside = out[:, cols:].clone()
+                ins = [out if t is x and bool((out == x).all()) else t for t in operands]
+                hip.elementwise(desc, [t.data_ptr() for t in ins], out.data_ptr(), stream)
+                torch.cuda.synchronize()
+                assert torch.equal(out[:, :cols], want.to(tdt)) and torch.equal(out[:, cols:], beside), (rows, cols, len(operands))
