@@ -7,6 +7,8 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <memory>
+#include <new>
 #include <string>
 #include <vector>
 
@@ -254,12 +256,21 @@ static int edge_split_of(const KernelEntry* k, const frisk_gemm_desc* d, size_t 
   return 1;
 }
 
+// Slices of K are whole K tiles, of unequal length where their number does not divide the K tiles: all as long as the first but the last, which gets
+// what is left, at least what the kernel's loop is written for.  (Divisors alone left a
+// prime number of K tiles, or twice one, in few slices or one: us so / now, fp16 4x576x6784 NN 17.4 / 9.6, 21x5952x7808 32.8 / 21.4, bf16 3x6848x6016 25.3 / 18.7,
+// 198x896x7552 22.0 / 15.5, int8 3x2240x6784 16.5 / 10.3, e4m3 58x2240x7552 19.2 / 11.9.)
+static bool slices_ok(const KernelEntry* k, int64_t kt, int slices) {
+  const int64_t per = (kt + slices - 1) / slices, last = kt - (slices - 1) * per;
+  return last >= std::max(1, slices > 1 ? k->min_k_tiles : 1);
+}
+
 // the split the planner gives a grid below one round of a variant with the split-K store path: up to one work-group per CU,
 // at least 4 K tiles per slice
 static int sub_round_split(const KernelEntry* k, const frisk_gemm_desc* d, int64_t tiles, int64_t kt, size_t workspace) {
   int split = 1;
   for (int c = 2; c <= 64 && tiles * c <= 256; ++c)
-    if (kt % c == 0 && kt / c >= std::max(4, k->min_k_tiles) && (size_t)c * (size_t)d->M * (size_t)d->N * 4 <= workspace) split = c;
+    if (slices_ok(k, kt, c) && (kt + c - 1) / c >= std::max(4, k->min_k_tiles) && (size_t)c * (size_t)d->M * (size_t)d->N * 4 <= workspace) split = c;
   return split;
 }
 
@@ -324,7 +335,7 @@ static double estimated_cost(const KernelEntry* k, const frisk_gemm_desc* d, boo
     const int cs = sub_round_split(k, d, tiles, (int64_t)kt, workspace);
     // (measured: the slices' loops 8 % above the per-K-tile rate of a long loop, the pass at 256 KiB per tile and slice in 0.07 us;
     // 1024x8192x8192 comes out even with 256x128 tiles unsplit, 123.7 against 123.9 us, and stays unsplit)
-    if (cs > 1) return kt / cs * c * (0.6 + 0.4 * rest_fill * cs) * 1.08 + 5.0 + 0.07 * (double)(tiles * cs);
+    if (cs > 1) return (double)(((int64_t)kt + cs - 1) / cs) * c * (0.6 + 0.4 * rest_fill * cs) * 1.08 + 5.0 + 0.07 * (double)(tiles * cs);
   }
   double cost = (double)full * kt * c;
   if (rest) {
@@ -455,7 +466,7 @@ static const SmallGridModel& small_grid_model(const KernelEntry* k) {
 }
 static double small_grid_time(const SmallGridModel& m, const KernelEntry* k, const frisk_gemm_desc* d, int split) {
   const int64_t tiles = ((d->M + k->bm - 1) / k->bm) * ((d->N + k->bn - 1) / k->bn);
-  const double kt = (double)((d->K + k->bk - 1) / k->bk) / split;
+  const double kt = (double)(((d->K + k->bk - 1) / k->bk + split - 1) / split);  // of the longest slice
   const int64_t wgs = tiles * split, full = wgs / m.cap, rest = wgs % m.cap;
   // One row of 64x128 tiles against a B stored [N][K] streams it 128 bytes of a row at a time, which is slow where its rows are a multiple of 16 KiB
   // apart and little slower elsewhere.  us on them / on 64x32 tiles, whose K tiles are four times as deep: fp16 48x8192x8192 37.0 / 28.7,
@@ -483,7 +494,7 @@ static double small_grid_time(const SmallGridModel& m, const KernelEntry* k, con
 static bool in_table_range(const KernelEntry* k, const frisk_gemm_desc* d, int split) {
   const SmallGridModel& m = small_grid_model(k);
   const int64_t tiles = ((d->M + k->bm - 1) / k->bm) * ((d->N + k->bn - 1) / k->bn);
-  return split == 1 || (!(split & (split - 1)) && d->K / k->bk / split >= m.kmin && tiles * split <= m.w);
+  return split == 1 || (!(split & (split - 1)) && d->K / k->bk % split == 0 && d->K / k->bk / split >= m.kmin && tiles * split <= m.w);
 }
 static int small_grid_split(const KernelEntry* k, const frisk_gemm_desc* d, size_t workspace, bool edges, bool table_range, double* cost = nullptr, double* range_cost = nullptr) {
   const SmallGridModel& m = small_grid_model(k);
@@ -507,15 +518,22 @@ static int small_grid_split(const KernelEntry* k, const frisk_gemm_desc* d, size
     // time: the bare model takes some to shorter slices that are slower.  us in 4 slices / in what it takes: 60x2752x1152 NT 12.2 / 13.3 (9), 88x1536x1152
     // 11.5 / 12.7 (9), 107x1408x2176 15.9 / 17.4 (17), 411x384x2944 18.3 / 20.2 (23), 456x448x1280 12.8 / 13.9 (8); longer slices gain as modelled:
     // 592x1280x7296 NT 114.9 in 2, 99.9 in 6, 975x384x8064 67.5 in 4, 60.3 in 21
-    int fitted = 1;
-    double fitted_t = INFINITY;
+    int fitted = 1, uneven = 1;
+    double fitted_t = INFINITY, uneven_t = INFINITY;
     for (int c = 2; c <= most; ++c)
-      if (kt % c == 0 && (size_t)c * (size_t)d->M * (size_t)d->N * 4 <= workspace && (!table_range || in_table_range(k, d, c))) {
+      if (slices_ok(k, kt, c) && (kt % c == 0 || (k->dtype != FRISK_F32 && !named)) && (size_t)c * (size_t)d->M * (size_t)d->N * 4 <= workspace && (!table_range || in_table_range(k, d, c))) {
         const double t = small_grid_time(m, k, d, c);
+        if (kt % c) {
+          if (t < uneven_t) { uneven = c; uneven_t = t; }
+          continue;
+        }
         if (t < best_t) { best = c; best_t = t; }
         if (range_cost && t < range_t && in_table_range(k, d, c)) range_t = t;
         if (k->dtype == FRISK_F32 && in_table_range(k, d, c) && t < fitted_t) { fitted = c; fitted_t = t; }
       }
+    // slices of unequal length for 10 % of modelled time and what the model leaves out, 0.15 us a slice and 1 us for a second launch where there was
+    // none: us without / with them, fp16 96x768x6528 NN 11.1 in 6 slices, 11.8 in 13, e4m3 6x576x3712 8.8 in one, 9.9 in 6
+    if (uneven_t + 0.15 * (uneven - best) + (best == 1 ? 1.0 : 0.0) < 0.9 * best_t) { best = uneven; best_t = uneven_t; }
     if (best > fitted && fitted > 1 && kt / best <= 10 && fitted_t < 1.12 * best_t) { best = fitted; best_t = fitted_t; }
   }
   // the edge kernels: slices of unequal length, whole tiles of partial sums
@@ -603,9 +621,9 @@ static double round_time(const RoundModel& m, const KernelEntry* k, const frisk_
 struct PlanContext { bool a_off = false, b_off = false, c_off = false; size_t workspace = kAnyWorkspace; };
 // Operands that are copied to aligned rows in the workspace before the product runs, and where they go.
 struct Repack { bool a = false, b = false; int64_t lda = 0, ldb = 0; size_t b_offset = 0, bytes = 0; };
-// What a launch needs of a plan beyond the public structure: the copies, and the tail split of an edge kernel (whose slices may
-// differ in length), its partial sums behind the copies in the workspace.
-struct LaunchExtras { Repack repack; int tail_split = 1, tail_tiles = 0; size_t partial_offset = 0; };
+// What a launch needs of a plan beyond the public structure: the copies, the splits whose slices differ in length (of K, where the structure says 1, and the
+// tail split of an edge kernel, its partial sums behind the copies in the workspace).
+struct LaunchExtras { Repack repack; int split_k = 1; int tail_split = 1, tail_tiles = 0; size_t partial_offset = 0; };
 
 static Repack repack_of(const frisk_gemm_desc* d, bool a, bool b) {
   Repack r;
@@ -802,13 +820,13 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
   // A small grid whose route lies beyond the range of its table keeps it unless the refined times see the best route within the range ahead, over 64 rows by
   // 3 %.  The routes that this changes are 5 % faster up to 64 rows (165 drawn problems, 4 of them slower by 3 % or more); over 64 rows, of 127, 8 % faster
   // with operands that the last-level cache holds and 2 % slower with operands from memory.  us within / beyond: fp16 1024x1024x6272 NT 23.0 in 2
-  // slices of 64x128 tiles, 31.0 in 7 of 256x256; 384x256x5888 NT 11.1 / 14.4, 128x1024x4864 NN 11.7 / 14.9, int8 640x128x14848 NT 13.0 / 16.6,
+  // slices of 64x128 tiles, 31.0 in 7 of 256x256 (and 25.6 in 3 of 128x128 where slices of unequal length did not have to gain a fifth); 384x256x5888 NT 11.1 / 14.4, 128x1024x4864 NN 11.7 / 14.9, int8 640x128x14848 NT 13.0 / 16.6,
   // 32x9216x2688 NT 8.1 / 9.1.
   if (best >= 0 && best_in >= 0) {
     const KernelEntry *k = ks[best], *in = ks[best_in];
     const int split = k->splitk && d->K % k->bk == 0 ? small_grid_split(k, d, left_for_sums(k), false, false) : 1;
     if ((planners_own(k) ? edge_slices() == 1 : k->splitk && !in_table_range(k, d, split)) &&
-        refined_time(k, d, split) * (d->M > 64 ? 0.97 : 1.0) >= refined_time(in, d, small_grid_split(in, d, left_for_sums(in), false, true))) {
+        refined_time(k, d, split) * (d->K / k->bk % split ? 1.2 : d->M > 64 ? 0.97 : 1.0) >= refined_time(in, d, small_grid_split(in, d, left_for_sums(in), false, true))) {
       best = best_in;
       table_range = true;
       split_edges = false;
@@ -919,9 +937,36 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
   } else if (d->split_k > 1 && !no_split) {
     return fail(FRISK_ERR_TILE, "split_k=%d: the chosen kernel %s has no split-K path", d->split_k, k->name);
   }
-  plan->split_k = split;
+  plan->split_k = kt % split ? 1 : split;
+  if (extras) extras->split_k = split;
   if (split > 1) plan->workspace_bytes = (size_t)split * (size_t)d->M * (size_t)d->N * 4;
   if (plan->tail_split <= 1) { plan->tail_split = 1; plan->tail_tiles = 0; }
+  return FRISK_OK;
+}
+
+// make_plan without the model of the LDS layouts, for the calls that launch.  A program's few descriptors come round again and again, and walking the
+// variants takes 0.9 us (128x128x128) to 4 (a few rows against a large B, with all their splits) of a call that takes 7 to 8 through Python; a plan
+// depends on nothing but the descriptor's values and the context, so each thread keeps those of the last descriptors that it has met: kept by value, in
+// kKeptPlans places of 0.5 KiB, refused descriptors not at all.  us a call through Python before / now:
+// 128x128x128 fp16 8.0 / 7.5 in a row, 18.7 / 18.0 waited for.
+constexpr unsigned kKeptPlans = 64;  // a power of two
+static int planned(const frisk_gemm_desc* d, frisk_gemm_plan* plan, const PlanContext& ctx, LaunchExtras* extras) {
+  struct Kept { frisk_gemm_desc desc; PlanContext ctx; frisk_gemm_plan plan; LaunchExtras extras; bool used = false; };
+  static thread_local std::unique_ptr<Kept[]> kept(new (std::nothrow) Kept[kKeptPlans]);
+  if (!d || !kept) return make_plan(d, plan, false, ctx, extras);
+  uint64_t h = (uint64_t)d->M * 0x9e3779b97f4a7c15ull ^ (uint64_t)d->N * 0xc2b2ae3d27d4eb4full ^ (uint64_t)d->K * 0x165667b19e3779f9ull;
+  h ^= (uint64_t)ctx.workspace * 0xd6e8feb86659fd93ull + (uint64_t)((d->dtype_ab * 4 + d->transA * 2 + d->transB) * 16 + d->epilogue * 4 + (d->clear_accum ? 1 : 0));
+  Kept& k = kept[(h * 0x9e3779b97f4a7c15ull) >> 58];
+  static_assert(kKeptPlans == 64, "the place is the top six bits of the product");
+  const bool same = k.used && std::memcmp(&k.desc, d, sizeof *d) == 0 && k.ctx.a_off == ctx.a_off && k.ctx.b_off == ctx.b_off && k.ctx.c_off == ctx.c_off && k.ctx.workspace == ctx.workspace;
+  if (!same) {
+    LaunchExtras fresh;
+    frisk_gemm_plan p;
+    if (int st = make_plan(d, &p, false, ctx, &fresh); st != FRISK_OK) { *plan = p; return st; }
+    k = Kept{*d, ctx, p, fresh, true};
+  }
+  *plan = k.plan;
+  if (extras) *extras = k.extras;
   return FRISK_OK;
 }
 
@@ -981,7 +1026,7 @@ int frisk_hip_plan(const frisk_gemm_desc* desc, frisk_gemm_plan* plan) { return 
 
 size_t frisk_hip_workspace_bytes(const frisk_gemm_desc* desc) {
   frisk_gemm_plan plan;
-  if (make_plan(desc, &plan, false) != FRISK_OK) return 0;
+  if (planned(desc, &plan, {}, nullptr) != FRISK_OK) return 0;
   return plan.workspace_bytes;
 }
 
@@ -993,7 +1038,7 @@ int frisk_hip_gemm(const frisk_gemm_desc* desc, const void* A, const void* B, vo
   ctx.a_off = (uintptr_t)A & 15;
   ctx.b_off = (uintptr_t)B & 15;
   ctx.c_off = ((uintptr_t)C & 15) || (desc && desc->epilogue == FRISK_EPI_ROW_COL_SCALE && ((uintptr_t)scaleB & 15));
-  int st = make_plan(desc, &plan, false, ctx, &extras);
+  int st = planned(desc, &plan, ctx, &extras);
   if (st != FRISK_OK) return st;
   if (desc->M == 0 || desc->N == 0) return FRISK_OK;
   if (!A || !B || !C) return fail(FRISK_ERR_NULL, "A, B and C must be device pointers");
@@ -1008,8 +1053,7 @@ int frisk_hip_gemm(const frisk_gemm_desc* desc, const void* A, const void* B, vo
     if (desc->split_k > 1) return fail(FRISK_ERR_WORKSPACE, "split_k=%d needs %zu bytes of workspace", desc->split_k, plan.workspace_bytes);
     const size_t wanted = plan.workspace_bytes;
     ctx.workspace = workspace && ws_aligned ? workspace_bytes : 0;
-    extras = LaunchExtras{};
-    st = make_plan(desc, &plan, false, ctx, &extras);
+    st = planned(desc, &plan, ctx, &extras);
     // a tile or wave policy that the caller named and that only kernels without staging through registers have: they want the copies
     if (st != FRISK_OK)
       return fail(FRISK_ERR_WORKSPACE, "rows or pointers off 16-byte boundaries: the tile or wave policy asked for runs on aligned copies of A or B, which need %zu bytes of 16-byte aligned workspace", wanted);
@@ -1026,11 +1070,11 @@ int frisk_hip_gemm(const frisk_gemm_desc* desc, const void* A, const void* B, vo
   p.xcd_remap = plan.xcd_remap;
   p.epilogue = desc->epilogue; p.dtype_out = desc->dtype_out; p.accumulate = desc->clear_accum ? 0 : 1;
   const KernelEntry* k = kernels()[plan.kernel_id];
-  p.split_k = plan.split_k;
-  p.kt_per_slice = (int)((desc->K + k->bk - 1) / k->bk) / plan.split_k;
+  p.split_k = extras.split_k;
+  p.kt_per_slice = (int)(((desc->K + k->bk - 1) / k->bk + p.split_k - 1) / p.split_k);
   const Repack& repack = extras.repack;
   const int tail_split = std::max(plan.tail_split, extras.tail_split);
-  p.partial = plan.split_k > 1 || tail_split > 1 ? (char*)workspace + extras.partial_offset : nullptr;
+  p.partial = p.split_k > 1 || tail_split > 1 ? (char*)workspace + extras.partial_offset : nullptr;
   p.tail_split = tail_split;
   p.tail_tiles = extras.tail_split > 1 ? extras.tail_tiles : plan.tail_tiles;
   p.tail_from = p.tiles_m * p.tiles_n - p.tail_tiles;
@@ -1055,7 +1099,7 @@ int frisk_hip_gemm(const frisk_gemm_desc* desc, const void* A, const void* B, vo
   }
   e = k->launch(p, (hipStream_t)stream);
   if (e != hipSuccess) return fail(FRISK_ERR_DEVICE, "launch of %s failed: %s", k->name, hipGetErrorString(e));
-  if (plan.split_k > 1) {
+  if (p.split_k > 1) {
     e = launch_splitk_reduce(p, desc->dtype_acc == FRISK_I32, (hipStream_t)stream);
     if (e != hipSuccess) return fail(FRISK_ERR_DEVICE, "launch of the split-K reduction failed: %s", hipGetErrorString(e));
   }
@@ -1071,7 +1115,7 @@ size_t frisk_hip_static_workspace_bytes(void) { return (size_t)FRISK_HIP_STATIC_
 int frisk_hip_gemm_static_ws(const frisk_gemm_desc* desc, const void* A, const void* B, void* C, const float* scaleA, const float* scaleB,
                              void* stream) {
   frisk_gemm_plan plan;
-  int st = make_plan(desc, &plan, false);
+  int st = planned(desc, &plan, {}, nullptr);
   if (st != FRISK_OK) return st;
   // What does not fit the array: an explicit split_k is refused (the caller asked for exactly that split), and so is a named tile that runs on copies
   // larger than it; of the splits the planner chooses by itself it takes those that fit (a split of K of fewer slices; no tail split: those of
@@ -1082,7 +1126,7 @@ int frisk_hip_gemm_static_ws(const frisk_gemm_desc* desc, const void* A, const v
                   desc->split_k, plan.workspace_bytes, (size_t)FRISK_HIP_STATIC_WS_BYTES);
     PlanContext limited;
     limited.workspace = FRISK_HIP_STATIC_WS_BYTES;
-    st = make_plan(desc, &plan, false, limited);
+    st = planned(desc, &plan, limited, nullptr);
     if (st != FRISK_OK || plan.workspace_bytes == 0) return frisk_hip_gemm(desc, A, B, C, scaleA, scaleB, nullptr, 0, stream);
   }
   void* ws = nullptr;

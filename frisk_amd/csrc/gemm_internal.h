@@ -17,7 +17,7 @@ struct GemmParams {
   int tiles_m, tiles_n;
   int group_m, xcd_remap;
   int epilogue, dtype_out, accumulate;
-  // K range of a work-group: blockIdx.y walks `split_k` slices of `kt_per_slice` K tiles each.  With more than one
+  // K range of a work-group: blockIdx.y walks `split_k` slices of `kt_per_slice` K tiles each, the last of them possibly fewer.  With more than one
   // slice the kernel writes raw 32-bit accumulators to partial[slice][M][N] and a second kernel sums the slices.
   int split_k, kt_per_slice;
   void* partial;

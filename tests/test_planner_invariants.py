@@ -78,3 +78,54 @@ def test_every_plan_is_a_kernel_that_may_run_on_the_problem(seed):
             assert p.split_k == 1 and p.tail_split == 1 and p.workspace_bytes == 0, what
     # the walk reached every kind of kernel
     assert {"", "_edge", "_splitk", "_splitk_edge", "_guard", "_guard_chunks"} <= seen, seen
+
+
+def test_kept_plans_are_those_of_their_descriptor():
+    """workspace_bytes looks its plan up among those that the thread keeps, plan() works it out anew: the same for more descriptors than are kept, met
+    in any order and from several threads"""
+    import random
+    import threading
+    rng = random.Random(17)
+    dts = [rng.choice([R.F16, R.BF16, R.I8, R.E4M3, R.F32]) for _ in range(300)]
+    descs = [R.make_desc(dt, rng.randrange(1, 700), rng.randrange(1, 700) * rng.choice([1, 8]), rng.randrange(1, 9000),
+                         dtype_out=OUT[dt], transA=rng.random() < 0.5, transB=rng.random() < 0.5, clear_accum=rng.random() < 0.5) for dt in dts]
+    want = [R.plan(d).workspace_bytes for d in descs]
+    assert len(set(want)) > 50
+
+    def walk(seed, wrong):
+        order = random.Random(seed).choices(range(len(descs)), k=2000)
+        wrong.extend(i for i in order if R.workspace_bytes(descs[i]) != want[i])
+
+    wrong = []
+    threads = [threading.Thread(target=walk, args=(s, wrong)) for s in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    walk(9, wrong)
+    assert not wrong
+
+
+def test_slices_of_unequal_length_leave_the_last_one_its_k_tiles():
+    """a split in slices of unequal length, which the plan reports by its workspace alone: every slice holds K tiles, the last one at least as many as the
+    kernel's loop is written for (16x16x128 atoms: four); a split that the caller names still has to divide them"""
+    uneven = 0
+    for dt in (R.F16, R.I8, R.E4M3):
+        for tb in (0, 1):
+            for M, N in ((4, 576), (58, 2240), (200, 896), (512, 512), (2048, 2048), (2304, 1280)):
+                for K in range(2048, 9000, 128):
+                    d = R.make_desc(dt, M, N, K, transB=tb, dtype_out={R.F16: R.F16, R.I8: R.F16, R.E4M3: R.BF16}[dt],
+                                    epilogue={R.F16: R.EPI_NONE, R.I8: R.EPI_ROW_COL_SCALE, R.E4M3: R.EPI_TENSOR_SCALE}[dt])
+                    p = R.plan(d)
+                    if p.split_k > 1 or p.tail_split > 1 or not p.workspace_bytes or "_splitk" not in R.kernel_names()[p.kernel_id]:
+                        continue
+                    kt, slices = K // p.tile_k, p.workspace_bytes // (M * N * 4)
+                    per = -(-kt // slices)
+                    last = kt - (slices - 1) * per
+                    assert K % p.tile_k == 0 and p.workspace_bytes == slices * M * N * 4 and slices > 1, (dt, M, N, K)
+                    assert (4 if dt == R.E4M3 and p.mfma_m == 16 else 1) <= last < per, (dt, M, N, K, slices)
+                    assert R.plan(R.make_desc(dt, M, N, K, transB=tb, dtype_out=d.dtype_out, epilogue=d.epilogue, split_k=1)).workspace_bytes == 0
+                    uneven += 1
+    assert uneven > 50
+    with pytest.raises(R.FriskHipError):
+        R.plan(R.make_desc(R.F16, 256, 256, 64 * 7, split_k=2))

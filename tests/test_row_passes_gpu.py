@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 
 import oracle as O
-from helpers import make_operand, run_gemm
+from helpers import TOL, make_operand, run_gemm
 from oracle import tile_ops as T
 
 
@@ -90,3 +90,26 @@ def test_the_last_group_of_a_row(hip, dt, tdt, rows):
                 hip.elementwise(desc, [t.data_ptr() for t in ins], out.data_ptr(), stream)
                 torch.cuda.synchronize()
                 assert torch.equal(out[:, :cols], want.to(tdt)) and torch.equal(out[:, cols:], beside), (rows, cols, len(operands))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,transA,transB", [(O.F16, 0, 0), (O.F16, 1, 0), (O.BF16, 0, 1), (O.I8, 0, 0), (O.I8, 0, 1), (O.E4M3, 0, 0), (O.E4M3, 0, 1)])
+def test_slices_of_unequal_length(hip, dtype, transA, transB):
+    """numbers of K tiles that no number of slices divides, a few rows to a few hundred, off the tiles and on them: the last slice is the shorter one"""
+    bk, seen = {O.F16: 64, O.BF16: 64, O.I8: 128, O.E4M3: 128}[dtype], 0
+    for M, N, tiles in ((4, 576, 53), (32, 512, 59), (58, 2240, 59), (64, 1024, 53), (128, 512, 31), (198, 896, 59), (256, 768, 43)):
+        if (transA and M % 32) or (transB and M <= 64):
+            continue
+        K = bk * tiles * (2 if transB else 1)
+        p = hip.plan(hip.make_desc(dtype, M, N, K, transA=transA, transB=transB, dtype_out={O.I8: O.I32, O.E4M3: O.BF16}.get(dtype, dtype)))
+        seen += p.split_k == 1 and p.tail_split == 1 and p.workspace_bytes > 0 and "_splitk" in hip.kernel_names()[p.kernel_id]
+        A = make_operand(dtype, *((K, M) if transA else (M, K)), 64, 0, scale=0.5)
+        B = make_operand(dtype, *((N, K) if transB else (K, N)), 64, 1, scale=0.5)
+        out = {O.I8: O.I32, O.E4M3: O.BF16}.get(dtype, dtype)
+        got = run_gemm(hip, dtype, A, B, transA, transB, out, M, N, K)
+        if dtype == O.I8:
+            assert np.array_equal(got, O.gemm_i32(A, B, transA, transB)), (M, N, K)
+        else:
+            r = O.compare(out, np.ascontiguousarray(got), O.gemm_f64(dtype, A, B, transA, transB))
+            assert r["nonfinite"] == 0 and r["max_rel"] <= TOL[dtype] and r["fro_rel"] <= TOL[dtype], (M, N, K, r)
+    assert seen
