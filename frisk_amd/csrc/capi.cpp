@@ -133,7 +133,7 @@ static void wave_partition(int policy, int64_t M, int64_t N, int num_waves, int 
 // found (`follow_up` in make_plan).
 static bool is_follow_up(const KernelEntry* k) {
   if (k->dtype == FRISK_F32) return k->bm == 32 && k->bn == 32 && !k->splitk;
-  return (k->bm == 64 && k->bn == 64) || (k->bm == 128 && k->bn == 128 && k->edge && k->stages == 3);
+  return (k->bm == 64 && k->bn == 64) || k->bm == 160 || k->bm == 224 || (k->bm == 128 && k->bn == 128 && k->edge && k->stages == 3);
 }
 
 // The compiled variants of one element type and pair of layouts, in table order, with what the planner would otherwise work out
@@ -318,6 +318,9 @@ static double estimated_cost(const KernelEntry* k, const frisk_gemm_desc* d, boo
   } else {
     // 3 + 3 tiles when the grid is one wave, 2 + 2 (two work-groups per CU) beyond
     c = k->stages >= 3 ? (tiles <= 256 ? 0.46 : 0.55) : (tiles <= 256 ? 0.55 : 0.52);
+    // 128x64 tiles with a K tile twice as deep: as many MFMAs a K tile as 128x128, 1.5 times its transfers.  us on 128x64 / what it runs on instead: fp16
+    // 3072x1792x1536 NT 32.8 / 21.9, 3200x1920x4352 85.9 / 53.5, 896x6592x6016 117 / 81
+    if (k->bm == 128 && k->bn == 64) c *= 1.5;
   }
   if (k->guard && !k->edge) c *= kStagedFactor;
   if (k->bm == 32 && k->wk > 1) {
@@ -605,8 +608,17 @@ static const RoundModel* round_model(const KernelEntry* k) {
   if (k->edge || k->guard || area == 256 * 256) return nullptr;
   return &plain[es == 1][area == 128 * 128 ? (k->stages >= 3 ? 1 : 0) : 2];
 }
+// The same for the tiles that only `other_tile` takes, and for 256x256 in whole tiles.
+static const RoundModel* tile_model(const KernelEntry* k) {
+  static const RoundModel more[2][3] = {{{256, 1.0f, 6.0f, 0.875f, 0.66f}, {256, 1.0f, 8.0f, 1.165f, 0.62f}, {256, 1.1f, 8.2f, 1.33f, 0.61f}},    // 16-bit: 160x256, 224x256, 256x256
+                                        {{256, 1.5f, 7.5f, 0.875f, 0.66f}, {256, 1.6f, 10.3f, 1.15f, 0.61f}, {256, 1.7f, 11.1f, 1.31f, 0.59f}}};  // 8-bit
+  const int es = elem_size(k->dtype);
+  if (es == 4 || k->wm * k->wn * k->wk != 4 || k->bn != 256) return round_model(k);
+  if (k->edge && (k->bm == 160 || k->bm == 224)) return &more[es == 1][k->bm == 224];
+  return !k->edge && !k->guard && k->bm == 256 ? &more[es == 1][2] : round_model(k);
+}
 // `slices` > 1: every tile (up to half a round of them) or those behind the whole rounds split along K, and the pass that sums them
-static double round_time(const RoundModel& m, const KernelEntry* k, const frisk_gemm_desc* d, int slices) {
+static double round_time(RoundModel m, const KernelEntry* k, const frisk_gemm_desc* d, int slices) {
   const int64_t tiles = ((d->M + k->bm - 1) / k->bm) * ((d->N + k->bn - 1) / k->bn), kt = (d->K + k->bk - 1) / k->bk;
   const int64_t split = slices <= 1 ? 0 : tiles <= 128 ? tiles : tiles % 256, plain = tiles - split, full = plain / m.cap, last = plain % m.cap + split * slices;
   const double k_last = split ? (double)((kt + slices - 1) / slices) : (double)kt;
@@ -689,6 +701,40 @@ static int follow_up(const std::vector<Variant>& list, const KernelEntry* k, con
   if (edge128 && tiles_of(128, 128) * (tiles_of(128, 128) <= 128 ? slices : 1) <= 256 && (d->K + k->bk - 1) / k->bk >= 12 && !(tiles_of(128, 128) > 128 && slices > 1))
     return variant(128, 128, 3);
   return -1;
+}
+
+// The edge tile (its index) that takes a problem of more than 256 tiles of 128x128 over from `k`, which the search has found and
+// which runs it in one pass: the one whose rounds the model sees through 3 % sooner, -1 where there is none.  The search's costs know nothing of what a round pays beside
+// its K loop, nor of bytes of C: a 256x256 tile of 4-byte C with old values is 512 KiB, 19 us of a round whatever the K.  us before / now, operands
+// in rotation: fp16 1596x3540x778 NN 24.4 on 192x256 / 18.8 on 128x128, 6656x1664x361 TN into fp32 sums 34.8 on 256x256 / 26.6 on 128x128; 2156x3328x6528 NN
+// 102.8 on 128x128 / 86.7 on 160x256, 3325x2420x2483 NT 56.6 on 128x128 / 49.1 on 160x256, 2368x5376x5376 NT 111.6 on 256x256 / 105.1 on 224x256.  Of 600 problems drawn
+// over the four types 150 or so change over, 15 % faster, one of them slower (int8 4288x7424x640 NT, 38.1 / 39.7).  The 160- and 224-row tiles from 12 K tiles on (their longer
+// prologue; with fewer the smaller tiles are as good).
+static int other_tile(const std::vector<Variant>& list, const KernelEntry* k, const frisk_gemm_desc* d, bool rows_aligned, const Repack& packed) {
+  const int es = elem_size(k->dtype), os = elem_size(d->dtype_out);
+  const bool whole_k = d->K % k->bk == 0;
+  const double more_bytes = os - 2 + (d->clear_accum ? 0 : os);  // of C, by the element, beyond those of the models' fits
+  auto time = [&](const KernelEntry* x, const RoundModel* m) {
+    RoundModel with_c = *m;
+    with_c.round += (float)(more_bytes * (m->cap == 512 ? 0.92 : 3.2 * x->bm * x->bn / 65536.0));
+    return round_time(with_c, x, d, 1);
+  };
+  const RoundModel* now = k->guard && !k->edge ? nullptr : tile_model(k);
+  if (!now || d->K <= k->bk) return -1;  // (a single K tile has no loop to model)
+  double best_time = 0.97 * time(k, now);
+  int best = -1;
+  for (const Variant& v : list) {
+    const KernelEntry* x = v.k;
+    const RoundModel* m = x != k && x->edge && !x->splitk && x->stages == 2 ? tile_model(x) : nullptr;
+    if (!m || x->guard != (rows_aligned && whole_k ? 0 : rows_aligned && d->K % (16 / es) == 0 ? 1 : 2) || (x->guard == 2 && k->guard != 2)) continue;
+    if ((x->bm == 128 || x->bm == 256) && x->guard == 0 && d->M % x->bm == 0 && d->N % x->bn == 0) continue;  // the plain twin was there to be found
+    if ((x->bm == 160 || x->bm == 224) && (d->K + x->bk - 1) / x->bk < 12) continue;
+    if ((d->K + x->bk - 1) / x->bk < x->min_k_tiles) continue;
+    const double span_a = (double)(packed.a ? packed.lda : d->lda) * es * (d->transA ? x->bk : x->bm), span_b = (double)(packed.b ? packed.ldb : d->ldb) * es * (d->transB ? x->bn : x->bk);
+    if (span_a >= 4294967296.0 || span_b >= 4294967296.0) continue;
+    if (const double t = time(x, m); t < best_time) { best = v.id; best_time = t; }
+  }
+  return best;
 }
 
 static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_model, const PlanContext& ctx = {}, LaunchExtras* extras = nullptr) {
@@ -866,8 +912,18 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
   int found_split = 1;
   if (best >= 0 && small && ks[best]->splitk && !no_split && d->K % ks[best]->bk == 0) found_split = small_grid_split(ks[best], d, ctx.workspace, false, table_range);
   const bool follows = best >= 0 && !tile_requested && d->split_k <= 1 && d->policy == FRISK_POLICY_SQUARE;
-  if (const int next = follows ? follow_up(list, ks[best], d, rows_aligned, found_split, found_slices, packed) : -1; next >= 0) best = next;
-  const bool one_pass = best >= 0 && is_follow_up(ks[best]) && !same_edge_tile(ks[best]);
+  int next = follows ? follow_up(list, ks[best], d, rows_aligned, found_split, found_slices, packed) : -1;
+  if (follows && next < 0 && !small && es < 4 && !(rows_aligned && d->M % 256 == 0 && d->N % 256 == 0 && d->K % ks[best]->bk == 0)) {
+    // (what is split along K stays as it is: the models of split and unsplit grids are not close enough, fp16 1563x3054x3567 NT 51.0 us on 192x256 tiles in
+    // 2 slices, 59.0 on 128x128 ones)
+    const KernelEntry* k = ks[best];
+    const int64_t tiles = ((d->M + k->bm - 1) / k->bm) * ((d->N + k->bn - 1) / k->bn), kt = d->K / k->bk;
+    const bool splits = k->splitk && !no_split && d->split_k == 0 && d->K % k->bk == 0;
+    if (found_slices == 1 && (!splits || (tiles < 256 ? sub_round_split(k, d, tiles, kt, ctx.workspace) : tail_split_of(k, tiles, kt, true, ctx.workspace)) == 1))
+      next = other_tile(list, k, d, rows_aligned, packed);
+  }
+  if (next >= 0) best = next;
+  const bool one_pass = next >= 0 && !same_edge_tile(ks[best]);
   if (d->M == 0 || d->N == 0) {  // nothing to compute
     plan->grid_x = plan->grid_y = 0;
     return FRISK_OK;

@@ -91,6 +91,12 @@ def square(bk, atom16=False, skinny_ta=(0,)):
     # 192x256 tiles (A stored [M][K]; 96-row waves), an edge kernel only: where rounds of 256x256 tiles come out uneven
     for tb in (0, 1):
         out.append(edge((0, tb, 192, 256, bk, 2, 2, 2, 0, 0, 1, 3) + ((16,) if atom16 else ())))
+    # ... and 160x256 and 224x256 ones (80- and 112-row waves of 16-row atoms), to which only `follow_up` goes over: more sizes of tile, fewer CUs left idle in
+    # the last round
+    if atom16:
+        for tb in (0, 1):
+            for bm in (160, 224):
+                out.append(edge((0, tb, bm, 256, bk, 2, 2, 2, 0, 0, 1, 3, 16)))
     # ... and the 32x128 and 64x128 tiles with the split-K store path likewise: a number of rows that is no multiple of 32 against
     # a large B (fp16 48x8192x8192: 68 us on 128x128 edge tiles, the vendor library 27-35)
     for tb in (0, 1):

@@ -500,3 +500,21 @@ def test_small_grids_stay_within_the_range_of_their_table(dt, M, N, K, lay, tile
 def test_splits_beyond_that_range_stay_where_they_gain(dt, M, N, K, lay, beyond):
     name, p = _route(dt, M, N, K, lay)
     assert p.split_k == beyond, (name, p.split_k)
+
+
+@pytest.mark.parametrize("dt,M,N,K,lay,kw,tile", [
+    (R.F16, 1596, 3540, 778, "NN", dict(lda=784, ldb=3544, ldc=3544), "128x128"),  # few K tiles: 128x128, two a CU, instead of 192x256
+    (R.F16, 6656, 1664, 361, "TN", dict(dtype_out=R.F32, clear_accum=False, ldc=1664), "128x128"),  # 4-byte C with old values instead of 256x256
+    (R.F16, 2156, 3328, 6528, "NN", {}, "160x256"), (R.F16, 1792, 5120, 7552, "NT", {}, "256x256"),
+    (R.BF16, 3584, 4095, 896, "NN", dict(ldb=4096, ldc=4096), "224x256"), (R.I8, 2400, 3584, 1536, "NT", {}, "160x256"),
+    (R.E4M3, 2400, 3584, 1536, "NT", {}, None), (R.F16, 2400, 3584, 704, "NN", {}, None), (R.F16, 2400, 3584, 1024, "TN", {}, None)])
+def test_tile_of_problems_beyond_small_grids(dt, M, N, K, lay, kw, tile):
+    """160- and 224-row tiles from 12 K tiles on, where A is stored along K, in 16-bit types and int8"""
+    name, p = _route(dt, M, N, K, lay, **kw)
+    assert (tile or "x") in name and (tile or ("160x256" not in name and "224x256" not in name)) and p.split_k == 1, name
+    for rows in (160, 224):  # no descriptor names them
+        with pytest.raises(RuntimeError, match="tile"):
+            R.plan(R.make_desc(dt, M, N, K, transA=lay[0] == "T", transB=lay[1] == "T", tile=(rows, 256, 64 if dt in (R.F16, R.BF16) else 128),
+                               dtype_out={R.I8: R.I32, R.E4M3: R.F32}.get(dt)))
+    for base in ((768, 1792, 5632), (896, 6592, 6016), (3200, 1920, 4352)):
+        assert "_128x64x" not in _route(R.F16, *base, "NT")[0]

@@ -147,6 +147,40 @@ def test_192_row_tiles(hip, dtype, transB):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [O.F16, O.BF16, O.I8])
+@pytest.mark.parametrize("transB", [0, 1])
+def test_160_and_224_row_tiles(hip, dtype, transB):
+    """whole tiles, M and N ending inside a tile, inside a wave's 80 and 112 rows and inside an atom; whole K tiles and partial ones of a chunk and of an element"""
+    bk = BK[dtype]
+    for M, N, K, tile in ((2400, 3584, 12 * bk, "160x256"), (2399, 3583, 12 * bk + 1, "160x256"), (2321, 3592, 15 * bk + 8, "160x256"), (3584, 4095, 14 * bk, "224x256"),
+                          (3473, 3900, 13 * bk + 3, "224x256")):
+        A = make_operand(dtype, *stored_shapes(M, N, K, 0, transB)[0], seed=91, tensor=0, scale=0.5)
+        B = make_operand(dtype, *stored_shapes(M, N, K, 0, transB)[1], seed=91, tensor=1, scale=0.5)
+        got, name, need = launch(hip, dtype, A, B, M, N, K, 0, transB, True, ldc_extra=int(M != 2400))
+        assert tile in name and need == 0, (M, N, K, name, need)
+        verify(dtype, got, A, B, 0, transB)
+
+
+@pytest.mark.gpu
+def test_160_row_tiles_apply_scales_and_accumulate(hip):
+    """int8 with per-row and per-column scales (bit for bit) and into old int32 values, fp16 into old fp32 ones; rows off 16-byte boundaries behind copies"""
+    M, N, K8, K16 = 2399, 3581, 1537, 772
+    Ai, Bi = make_operand(O.I8, M, K8, 92, 0), make_operand(O.I8, N, K8, 92, 1)
+    sA, sB = O.uniform(M, 92, 2, 0.001, 0.02), O.uniform(N, 92, 3, 0.001, 0.02)
+    acc = O.gemm_i32(Ai, Bi, 0, 1)
+    got = run_gemm(hip, O.I8, Ai, Bi, 0, 1, O.F16, M, N, K8, epilogue=hip.EPI_ROW_COL_SCALE, sA=sA, sB=sB, pad_c=0)
+    assert np.array_equal(got, O.epilogue_rowcol_f16(acc, sA, sB))
+    C0 = (np.arange(M * N, dtype=np.int64).reshape(M, N) % 91 - 45).astype(np.int32)
+    assert np.array_equal(run_gemm(hip, O.I8, Ai, Bi, 0, 1, O.I32, M, N, K8, C_init=C0, clear_accum=False), acc + C0)
+    Ah, Bh = make_operand(O.F16, M, K16, 93, 0, scale=0.5), make_operand(O.F16, K16, N, 93, 1, scale=0.5)
+    Cf = O.uniform(M * N, 93, 2, -1.0, 1.0).reshape(M, N).astype(np.float32)
+    assert "160x256" in hip.kernel_names()[hip.plan(hip.make_desc(O.F16, M, N, K16, dtype_out=O.F16)).kernel_id]
+    got = run_gemm(hip, O.F16, Ah, Bh, 0, 0, O.F32, M, N, K16, C_init=Cf, clear_accum=False)
+    r = O.compare(O.F32, np.ascontiguousarray(got), O.gemm_f64(O.F16, Ah, Bh) + Cf.astype(np.float64))
+    assert r["nonfinite"] == 0 and r["max_rel"] <= TOL[O.F32] and r["fro_rel"] <= TOL[O.F32], r
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtype,transA,transB,aligned,size", [
     (O.F16, 0, 0, True, (1001, 1003, 4001)),   # 64 tiles of 128 x 128 in 4 slices
     (O.BF16, 1, 0, True, (17, 4096, 4096)),    # one row of tiles in 8 slices
