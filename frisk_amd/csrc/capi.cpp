@@ -322,7 +322,7 @@ static double estimated_cost(const KernelEntry* k, const frisk_gemm_desc* d, boo
     // 3072x1792x1536 NT 32.8 / 21.9, 3200x1920x4352 85.9 / 53.5, 896x6592x6016 117 / 81
     if (k->bm == 128 && k->bn == 64) c *= 1.5;
   }
-  if (k->guard && !k->edge) c *= kStagedFactor;
+  if (k->guard && !k->edge && k->dtype == FRISK_F32) c *= kStagedFactor;  // (the other types: make_plan, at its search)
   if (k->bm == 32 && k->wk > 1) {
     // The 32x32 kernel streams B.  With a ring of 4 tiles one work-group fills a CU: whole rounds of 256, each paying its
     // own start (measured 14.8 us for 256 tiles, 35.8 for 512).  With a ring of 2 two work-groups share a CU: slower alone
@@ -838,6 +838,13 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
         range_cost *= waste;
       }
       if (k->guard == 2) cost += repack_cost;
+      // What staging through registers costs beyond the model of its tile: 0.3 us a K tile of 128 bytes where both operands are stored along K, else 1.0
+      // (8-bit 0.75), fitted to 330 problems of 1 to 25 K tiles.  (As a factor of 1.6 alone it kept problems of many K tiles from the copies.  Of 400 drawn
+      // problems with rows off 16 bytes 248 change over, 25 % faster, 11 of them slower by 3 to 12 %, one by 25.  us staged / on copies: e4m3
+      // 2410x865x1222 TN 24.8 / 18.1, fp16 1524x1901x861 NN 29.7 / 21.3, 6720x832x1337 NN 44.0 / 30.8; but int8 445x2933x150 NN 10.3 / 11.6,
+      // 355x3775x872 NT 15.1 / 16.9, which stay staged)
+      if (k->guard == 1 && !k->edge && es < 4)
+        cost += staged_rounds * (double)(((int64_t)d->K * es + 127) / 128) * (!d->transA && d->transB ? 0.32 : es == 2 ? 1.0 : 0.75);
       // ties: the first listed variant is the tuned default
       if (best < 0 || (ks[best]->guard && !k->guard && !planners_own(ks[best])) || cost < best_cost) { best = v.id; best_cost = cost; }
       if (want_range && !k->guard && !planners_own(k) && (best_in < 0 || range_cost < best_in_cost)) { best_in = v.id; best_in_cost = range_cost; }

@@ -518,3 +518,14 @@ def test_tile_of_problems_beyond_small_grids(dt, M, N, K, lay, kw, tile):
                                dtype_out={R.I8: R.I32, R.E4M3: R.F32}.get(dt)))
     for base in ((768, 1792, 5632), (896, 6592, 6016), (3200, 1920, 4352)):
         assert "_128x64x" not in _route(R.F16, *base, "NT")[0]
+
+
+@pytest.mark.parametrize("dt,M,N,K,lay,copies", [(R.E4M3, 2410, 865, 1222, "TN", True), (R.F16, 1524, 1901, 861, "NN", True), (R.BF16, 6720, 832, 1337, "NN", True),
+                                                 (R.I8, 445, 2933, 150, "NN", False), (R.I8, 355, 3775, 872, "NT", False), (R.F16, 157, 23, 32, "TT", False)])
+def test_rows_off_16_bytes_are_copied_where_k_is_deep_enough(dt, M, N, K, lay, copies):
+    """staged through registers in one launch with few K tiles; without a workspace always"""
+    es = 1 if dt in (R.I8, R.E4M3) else 2
+    name, p = _route(dt, M, N, K, lay)
+    sizes = [rows * (-(-cols * es // 16) * 16) for rows, cols in ((K, M) if lay[0] == "T" else (M, K), (N, K) if lay[1] == "T" else (K, N)) if cols * es % 16]
+    assert name.endswith("_s2_guard") == (not copies) and p.split_k == 1, name
+    assert p.workspace_bytes >= sum(sizes) if copies else p.workspace_bytes == 0, (p.workspace_bytes, sizes)
