@@ -842,7 +842,7 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
       // (8-bit 0.75), fitted to 330 problems of 1 to 25 K tiles.  (As a factor of 1.6 alone it kept problems of many K tiles from the copies.  Of 400 drawn
       // problems with rows off 16 bytes 248 change over, 25 % faster, 11 of them slower by 3 to 12 %, one by 25.  us staged / on copies: e4m3
       // 2410x865x1222 TN 24.8 / 18.1, fp16 1524x1901x861 NN 29.7 / 21.3, 6720x832x1337 NN 44.0 / 30.8; but int8 445x2933x150 NN 10.3 / 11.6,
-      // 355x3775x872 NT 15.1 / 16.9, which stay staged)
+      // 464x2236x198 NT 8.8 / 11.7, which stay staged)
       if (k->guard == 1 && !k->edge && es < 4)
         cost += staged_rounds * (double)(((int64_t)d->K * es + 127) / 128) * (!d->transA && d->transB ? 0.32 : es == 2 ? 1.0 : 0.75);
       // ties: the first listed variant is the tuned default
