@@ -666,7 +666,7 @@ static int follow_up(const std::vector<Variant>& list, const KernelEntry* k, con
     const KernelEntry *plain = nullptr, *edge[3] = {};
     int id = -1, edge_id[3] = {-1, -1, -1};
     for (const Variant& v : list)
-      if (v.follow_up && v.k->bm == bm && v.k->bn == bn && v.k->stages == stages) {
+      if ((v.follow_up || (bm == 128 && !v.k->edge && !v.k->guard && !v.k->splitk)) && v.k->bm == bm && v.k->bn == bn && v.k->stages == stages) {
         if (v.k->edge) { edge[v.k->guard] = v.k; edge_id[v.k->guard] = v.id; }
         else { plain = v.k; id = v.id; }
       }
@@ -696,6 +696,11 @@ static int follow_up(const std::vector<Variant>& list, const KernelEntry* k, con
   // e4m3 1408x576x2208 NT 18.7 / 8.2; in place of 64x128 tiles not for less than 1 KiB of K, 906x312x320 NT 5.0 / 5.2; with more than 7.5 KiB the slices have caught up, 494x1144x3768 NN 20.9 / 18.7
   if (tiles_of(64, 64) < 256 && k_bytes <= 7680 && (edge128 || (k->bm == 64 && k->bn == 128 && k_bytes >= 1024)))
     if (const int id = variant(64, 64, 3); id >= 0) return id;
+  // 128x128 tiles with 3 + 3 tiles of LDS in a single round, one on each CU, in place of unsplit 64x128 ones of which some CUs hold two: a third less to transfer.  us
+  // on 64x128 / so: fp16 363x8512x2176 NT 25.2 / 20.8, 1206x3072x1280 NN 17.6 / 15.9, bf16 1108x3008x1792 NT 20.2 / 18.1, 5952x640x7296 NN 82.5 / 73.1.  Of 79 drawn 16-bit
+  // problems all are faster, by 18 %, and all of 48 8-bit ones of 2 KiB of K and more, by 20 % (of 37 with less 14 are slower, int8 1856x1152x1024 NT by 17 %)
+  if (k->bm == 64 && k->bn == 128 && (es == 2 || k_bytes >= 2048) && tiles_of(64, 128) > 256 && tiles_of(128, 128) <= 256)
+    if (const int id = variant(128, 128, 3); id >= 0) return id;
   // 128x128 edge tiles with 3 + 3 tiles of LDS where no CU has two work-groups.  us with 2 + 2 / 3 + 3: fp16 3916x632x2592 NT 32.4 / 24.4, 512x1392x1368 TN
   // 18.3 / 13.5, 558x296x1200 16.1 / 12.2, e4m3 2304x1664x4048 NN 28.1 / 21.9; under 12 K tiles the longer prologue costs up to 4 %
   if (edge128 && tiles_of(128, 128) * (tiles_of(128, 128) <= 128 ? slices : 1) <= 256 && (d->K + k->bk - 1) / k->bk >= 12 && !(tiles_of(128, 128) > 128 && slices > 1))

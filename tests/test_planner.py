@@ -529,3 +529,12 @@ def test_rows_off_16_bytes_are_copied_where_k_is_deep_enough(dt, M, N, K, lay, c
     sizes = [rows * (-(-cols * es // 16) * 16) for rows, cols in ((K, M) if lay[0] == "T" else (M, K), (N, K) if lay[1] == "T" else (K, N)) if cols * es % 16]
     assert name.endswith("_s2_guard") == (not copies) and p.split_k == 1, name
     assert p.workspace_bytes >= sum(sizes) if copies else p.workspace_bytes == 0, (p.workspace_bytes, sizes)
+
+
+@pytest.mark.parametrize("dt,M,N,K,lay,tile", [(R.F16, 363, 8512, 2176, "NT", "128x128x64_w2x2_s3_edge"), (R.BF16, 5952, 640, 7296, "NN", "128x128x64_w2x2_s3_edge"), (R.F16, 1280, 2560, 512, "TN", "128x128x64_w2x2_s3"),
+                                               (R.I8, 528, 5440, 2048, "NT", "128x128x128_w2x2_s3_edge"), (R.I8, 448, 8192, 1920, "NT", "64x128x128_w2x2_s3_splitk"),
+                                               (R.F16, 1600, 1280, 3456, "TT", "64x128x64_w2x2_s3_splitk")])
+def test_a_single_round_of_128_row_tiles_before_two_64_row_ones_a_cu(dt, M, N, K, lay, tile):
+    """more than 256 tiles of 64x128 and at most 256 of 128x128, 8-bit types from 2 KiB of K on"""
+    name, p = _route(dt, M, N, K, lay)
+    assert name.endswith(tile) and (p.split_k, p.workspace_bytes) == (1, 0), (name, p.workspace_bytes)
