@@ -658,7 +658,7 @@ static bool same_edge_tile(const KernelEntry* k) { return k->bm == 128 && k->bn 
 static int follow_up(const std::vector<Variant>& list, const KernelEntry* k, const frisk_gemm_desc* d, bool rows_aligned, int split, int slices, const Repack& packed) {
   const int es = elem_size(k->dtype);
   const bool staged = k->guard && !k->edge;  // through registers
-  if (staged || split > 1) return -1;
+  if (staged || (split > 1 && (d->M > 64 || k->dtype == FRISK_F32))) return -1;
   auto tiles_of = [&](int bm, int bn) { return ((d->M + bm - 1) / bm) * ((d->N + bn - 1) / bn); };
   // the variant of a tile for this problem: the plain kernel where it fits, else the edge kernel, named for what it takes (an incumbent that
   // works on copies of its operands hands them on)
@@ -687,9 +687,21 @@ static int follow_up(const std::vector<Variant>& list, const KernelEntry* k, con
     // tiles of 128 296x856x160 (270) 6.2 / 7.2
     return k->wk == 1 && d->K >= (tiles_of(32, 32) <= 256 ? 128 : 256) && tiles_of(32, 32) <= 512 ? variant(32, 32, 2) : -1;
   }
-  // (up to 64 rows and 256 tiles of 64x64, 1024x1024 for one, stay on the kernels that the planner has always named for them: fp16 1024^3 NN 7.8 us, 6.7 on 64x64)
-  if (d->M <= 64) return -1;
   const int64_t k_bytes = d->K * es;
+  if (d->M <= 64) {
+    // 64x64 tiles for up to 64 rows where they are one round that fills half the CUs and more, with 256 bytes of a row of B at a time and three tiles under way on
+    // each.  In place of unsplit 32x128 and 64x128 tiles; of 32x128 ones in 2 slices on B [K][N], for the second launch that goes; and below 32 rows on B [N][K] of
+    // two 32x32 work-groups a CU (16-bit from 9 rows on, 8-bit up to 6000 of K: elsewhere as many are slower).  us, B from memory, before / so: bf16 5x11584x2304
+    // NN 17.9 / 12.3, 58x9536x3584 NN 22.1 / 15.9, 12x15296x6400 NN 41 / 32, fp16 13x10432x3456 NT 19.5 / 17.4, e4m3 1x9856x2944 NT 12.2 / 9.6; but fp16
+    // 6x14016x7808 NT 40.0 / 45, 24x15552x8192 NT (rows 16 KiB apart) 35 / 44, 10752x6144 NN in 3 slices 29.7 / 37.  Of 280 drawn problems 93 change over,
+    // 13 % faster, none of them slower by 3 % and more.
+    const int64_t wgs = tiles_of(64, 64);
+    if (wgs <= 128 || wgs > 256 || (d->transB && d->M >= 32) || k_bytes < 2048) return -1;  // (measured from 2 KiB of K on)
+    const bool two_a_cu = k->bm == 32 && k->bn == 32 && k->stages == 2;
+    const bool so = k->bn == 128 ? split == 1 || (split == 2 && !d->transB && k->bm == 32 && wgs > 170)
+                                 : two_a_cu && split == 1 && (es == 2 ? d->M > 8 && d->K * es % 16384 : d->K < 6000 && d->K % 4096);
+    return so ? variant(64, 64, 3) : -1;
+  }
   const bool edge128 = k->edge && !k->splitk && k->bm == 128 && k->bn == 128;
   // 64x64 tiles in a single round, in place of 128x128 edge tiles, split or not, and of unsplit 64x128 tiles.  us, operands in the last-level cache:
   // fp16 525x1136x1480 NT 19.1 / 9.6, 558x296x1200 16.1 / 7.1, 852x824x1840 NN 19.8 / 11.8, 1229x608x3960 22.9 / 18.7, 768x1152x2048 12.0 / 9.3,

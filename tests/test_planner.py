@@ -538,3 +538,12 @@ def test_a_single_round_of_128_row_tiles_before_two_64_row_ones_a_cu(dt, M, N, K
     """more than 256 tiles of 64x128 and at most 256 of 128x128, 8-bit types from 2 KiB of K on"""
     name, p = _route(dt, M, N, K, lay)
     assert name.endswith(tile) and (p.split_k, p.workspace_bytes) == (1, 0), (name, p.workspace_bytes)
+
+
+@pytest.mark.parametrize("dt,M,N,K,lay,tile", [(R.BF16, 5, 11584, 2304, "NN", "64x64"), (R.F16, 58, 9536, 3584, "NN", "64x64"), (R.F16, 12, 15296, 6400, "NN", "64x64"), (R.F16, 13, 10432, 3456, "NT", "64x64"),
+                                               (R.E4M3, 1, 9856, 2944, "NT", "64x64"), (R.I8, 14, 8704, 5376, "NT", "64x64"), (R.F16, 6, 14016, 7808, "NT", "32x32"), (R.F16, 24, 15552, 8192, "NT", "32x32"),
+                                               (R.BF16, 36, 10752, 6144, "NN", "64x128"), (R.I8, 9, 13568, 6528, "NT", "32x32"), (R.F16, 12, 8128, 2304, "NN", "x128"), (R.BF16, 12, 16448, 2304, "NN", "x128")])
+def test_few_rows_on_64_column_tiles_in_one_round(dt, M, N, K, lay, tile):
+    """129 to 256 tiles of 64x64, and the kernels and sizes beside them that keep their own"""
+    name, p = _route(dt, M, N, K, lay)
+    assert tile in name.split("_w")[0] and (tile != "64x64" or (p.split_k, p.workspace_bytes) == (1, 0)), (name, p.split_k, p.workspace_bytes)

@@ -147,6 +147,19 @@ def test_192_row_tiles(hip, dtype, transB):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype,transB", [(O.F16, 0), (O.BF16, 0), (O.F16, 1), (O.I8, 1), (O.E4M3, 1)])
+def test_few_rows_on_64_column_tiles(hip, dtype, transB):
+    """a few rows to 64 of them (B stored along K: below 32), N ending inside a tile, eight to eleven K tiles of 256 bytes, whole and partial"""
+    bk, few = 2 * BK[dtype], 9 if transB and dtype == O.F16 else 1
+    for M, N, K in ((few, 8256, 8 * bk), (17, 9544, 8 * bk + 32), (31, 16320, 9 * bk), (12 if transB else 64, 12296, 10 * bk), (16 if transB else 33, 8264, 11 * bk - 64)):
+        A = make_operand(dtype, M, K, seed=94, tensor=0, scale=0.5)
+        B = make_operand(dtype, *stored_shapes(M, N, K, 0, transB)[1], seed=94, tensor=1, scale=0.5)
+        got, name, need = launch(hip, dtype, A, B, M, N, K, 0, transB, True)
+        assert "64x64x" in name and need == 0, (M, N, K, name, need)
+        verify(dtype, got, A, B, 0, transB)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [O.F16, O.BF16, O.I8])
 @pytest.mark.parametrize("transB", [0, 1])
 def test_160_and_224_row_tiles(hip, dtype, transB):
