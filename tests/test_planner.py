@@ -547,3 +547,12 @@ def test_few_rows_on_64_column_tiles_in_one_round(dt, M, N, K, lay, tile):
     """129 to 256 tiles of 64x64, and the kernels and sizes beside them that keep their own"""
     name, p = _route(dt, M, N, K, lay)
     assert tile in name.split("_w")[0] and (tile != "64x64" or (p.split_k, p.workspace_bytes) == (1, 0)), (name, p.split_k, p.workspace_bytes)
+
+
+@pytest.mark.parametrize("dt,M,N,K,lay,tile", [(R.F16, 832, 1216, 6144, "NN", "64x64"), (R.BF16, 960, 1088, 8704, "NN", "64x64"), (R.F16, 928, 896, 4480, "NT", "64x64"), (R.E4M3, 332, 1920, 6656, "NT", "64x64"),
+                                               (R.F16, 192, 2880, 3072, "NN", "64x64"), (R.F16, 68, 6656, 8576, "NN", "64x128"), (R.F16, 416, 1408, 8064, "NN", "64x128"), (R.F16, 1024, 1024, 4096, "NN", "x"),
+                                               (R.I8, 332, 1920, 6656, "NN", "64x128")])
+def test_64x64_tiles_in_place_of_few_slices_of_64x128_ones(dt, M, N, K, lay, tile):
+    """129 to 255 tiles of 64x64, A stored along K (8-bit types: B too)"""
+    name, p = _route(dt, M, N, K, lay)
+    assert tile in name.split("_w")[0] and (tile != "64x64" or (p.split_k, p.workspace_bytes) == (1, 0)), (name, p.split_k, p.workspace_bytes)
