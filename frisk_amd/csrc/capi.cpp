@@ -862,13 +862,16 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
         range_cost *= waste;
       }
       if (k->guard == 2) cost += repack_cost;
-      // What staging through registers costs beyond the model of its tile: 0.3 us a K tile of 128 bytes where both operands are stored along K, else 1.0
-      // (8-bit 0.75), fitted to 330 problems of 1 to 25 K tiles.  (As a factor of 1.6 alone it kept problems of many K tiles from the copies.  Of 400 drawn
-      // problems with rows off 16 bytes 248 change over, 25 % faster, 11 of them slower by 3 to 12 %, one by 25.  us staged / on copies: e4m3
-      // 2410x865x1222 TN 24.8 / 18.1, fp16 1524x1901x861 NN 29.7 / 21.3, 6720x832x1337 NN 44.0 / 30.8; but int8 445x2933x150 NN 10.3 / 11.6,
-      // 464x2236x198 NT 8.8 / 11.7, which stay staged)
-      if (k->guard == 1 && !k->edge && es < 4)
-        cost += staged_rounds * (double)(((int64_t)d->K * es + 127) / 128) * (!d->transA && d->transB ? 0.32 : es == 2 ? 1.0 : 0.75);
+      // What staging through registers costs beyond the model of its tile, a K tile of 128 bytes: on small grids 0.3 us where both operands are stored along K,
+      // else 1.0 (8-bit 0.75); on larger ones, whose CUs hold two, 0.55, 1.0, 1.2 (int8) and 1.9 (8-bit float).  Fitted to 330 and 75 problems.  (As a factor of
+      // 1.6 alone it kept problems of many K tiles from the copies.  Of 400 drawn problems with rows off 16 bytes 248 change over, 25 % faster, 11 of them slower by
+      // 3 to 12 %, one by 25.  us staged / on copies: e4m3 2410x865x1222 TN 24.8 / 18.1, 2511x2241x536 TT 26.7 / 17.2, fp16 1524x1901x861 NN 29.7 / 21.3,
+      // 6720x832x1337 NN 44.0 / 30.8, bf16 2321x2172x1978 NT 50.7 / 38.4; but int8 445x2933x150 NN 10.3 / 11.6, 464x2236x198 NT 8.8 / 11.7, which stay staged)
+      if (k->guard == 1 && !k->edge && es < 4) {
+        const bool along_k = !d->transA && d->transB;
+        const double rate = along_k ? (small ? 0.32 : 0.55) : es == 2 ? 1.0 : small ? 0.75 : k->dtype == FRISK_I8 ? 1.2 : 1.9;
+        cost += staged_rounds * (double)(((int64_t)d->K * es + 127) / 128) * rate;
+      }
       // ties: the first listed variant is the tuned default
       if (best < 0 || (ks[best]->guard && !k->guard && !planners_own(ks[best])) || cost < best_cost) { best = v.id; best_cost = cost; }
       if (want_range && !k->guard && !planners_own(k) && (best_in < 0 || range_cost < best_in_cost)) { best_in = v.id; best_in_cost = range_cost; }

@@ -520,7 +520,7 @@ def test_tile_of_problems_beyond_small_grids(dt, M, N, K, lay, kw, tile):
         assert "_128x64x" not in _route(R.F16, *base, "NT")[0]
 
 
-@pytest.mark.parametrize("dt,M,N,K,lay,copies", [(R.E4M3, 2410, 865, 1222, "TN", True), (R.F16, 1524, 1901, 861, "NN", True), (R.BF16, 6720, 832, 1337, "NN", True),
+@pytest.mark.parametrize("dt,M,N,K,lay,copies", [(R.E4M3, 2410, 865, 1222, "TN", True), (R.E4M3, 2511, 2241, 536, "TT", True), (R.BF16, 2321, 2172, 1978, "NT", True), (R.F16, 1524, 1901, 861, "NN", True), (R.BF16, 6720, 832, 1337, "NN", True),
                                                  (R.I8, 445, 2933, 150, "NN", False), (R.I8, 464, 2236, 198, "NT", False), (R.F16, 157, 23, 32, "TT", False)])
 def test_rows_off_16_bytes_are_copied_where_k_is_deep_enough(dt, M, N, K, lay, copies):
     """staged through registers in one launch with few K tiles; without a workspace always"""
