@@ -767,6 +767,7 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
   if (st != FRISK_OK) return st;
   if (!plan) return fail(FRISK_ERR_NULL, "plan is null");
   std::memset(plan, 0, sizeof *plan);
+  if (extras) *extras = LaunchExtras{};  // (a call that plans once more for the workspace it has hands in those of its first plan)
   plan->kernel_id = -1;
   const int es = elem_size(d->dtype_ab), os = elem_size(d->dtype_out);
   plan->flops = 2.0 * (double)d->M * (double)d->N * (double)d->K;

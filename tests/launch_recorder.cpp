@@ -1,0 +1,84 @@
+// What the library would launch, on a machine without a GPU: the calls of the HIP runtime that the library makes are defined here, in the executable, where the
+// loader finds them first, and print what they are asked for instead.  Pointers are made up; nothing reads them.
+//
+//   launch_recorder gemm keep|nokeep <dtype> <M> <N> <K> <transA> <transB> <workspace bytes>
+//   launch_recorder block <dtype> <rows> <cols> <operands: m = rows x cols, r = one value a row, c = one a column>
+#include <dlfcn.h>
+#include <hip/hip_runtime_api.h>
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <new>
+#include <string>
+#include "frisk_hip.h"
+
+static bool g_keep = true;
+
+extern "C" {
+static struct { dim3 grid, block; size_t lds; hipStream_t stream; } g_pushed;
+hipError_t __hipPushCallConfiguration(dim3 grid, dim3 block, size_t lds, hipStream_t stream) { g_pushed = {grid, block, lds, stream}; return hipSuccess; }
+hipError_t __hipPopCallConfiguration(dim3* grid, dim3* block, size_t* lds, hipStream_t* stream) {
+  *grid = g_pushed.grid; *block = g_pushed.block; *lds = g_pushed.lds; *stream = g_pushed.stream;
+  return hipSuccess;
+}
+hipError_t hipLaunchKernel(const void* kernel, dim3 grid, dim3 block, void**, size_t, hipStream_t) {
+  Dl_info info{};
+  dladdr(kernel, &info);
+  std::printf("launch %s %u %u %u %u\n", info.dli_sname ? info.dli_sname : "?", grid.x, grid.y, grid.z, block.x);
+  return hipSuccess;
+}
+hipError_t hipGetDevice(int* device) { *device = 0; return hipSuccess; }
+hipError_t hipGetDevicePropertiesR0600(hipDeviceProp_tR0600* p, int) { std::memset(p, 0, sizeof *p); std::strcpy(p->gcnArchName, "gfx950"); return hipSuccess; }
+hipError_t hipFuncSetAttribute(const void*, hipFuncAttribute, int) { return hipSuccess; }
+hipError_t hipGetLastError() { return hipSuccess; }
+}
+// the storage of the plans that a thread keeps
+void* operator new[](size_t n, const std::nothrow_t&) noexcept { return g_keep ? std::malloc(n) : nullptr; }
+void operator delete[](void* p) noexcept { std::free(p); }
+
+static void* at(int i) { return (void*)((size_t)1 << (32 + i)); }
+
+static int gemm(char** arg) {
+  g_keep = !std::strcmp(arg[0], "keep");
+  frisk_gemm_desc d{};
+  d.abi_version = FRISK_HIP_ABI_VERSION;
+  d.dtype_ab = std::atoi(arg[1]);
+  d.dtype_acc = d.dtype_ab == FRISK_I8 ? FRISK_I32 : FRISK_F32;
+  d.dtype_out = d.dtype_ab == FRISK_I8 ? FRISK_I32 : d.dtype_ab == FRISK_E4M3 ? FRISK_BF16 : d.dtype_ab;
+  d.M = std::atoll(arg[2]); d.N = std::atoll(arg[3]); d.K = std::atoll(arg[4]);
+  d.transA = std::atoi(arg[5]); d.transB = std::atoi(arg[6]);
+  d.lda = d.transA ? d.M : d.K; d.ldb = d.transB ? d.K : d.N; d.ldc = d.N;
+  d.clear_accum = 1;
+  const size_t bytes = (size_t)std::atoll(arg[7]);
+  const int st = frisk_hip_gemm(&d, at(0), at(1), at(2), nullptr, nullptr, bytes ? at(3) : nullptr, bytes, nullptr);
+  std::printf("status %d\n", st);
+  return 0;
+}
+
+static int block(char** arg) {
+  frisk_elementwise_desc d{};
+  const std::string operands = arg[3];
+  d.abi_version = FRISK_HIP_ABI_VERSION;
+  d.out_dtype = std::atoi(arg[0]);
+  d.rows = std::atoll(arg[1]); d.cols = d.out_ld = std::atoll(arg[2]);
+  d.n_inputs = (int)operands.size();
+  const void* in[FRISK_EW_MAX_INPUTS] = {};
+  for (int k = 0; k < d.n_inputs; ++k) {  // x, then + or * the next operand
+    in[k] = at(k);
+    d.in_dtype[k] = d.out_dtype;
+    d.in_row_stride[k] = operands[k] == 'm' ? d.cols : operands[k] == 'r';
+    d.in_col_stride[k] = operands[k] != 'r';
+    d.op[d.n_ops] = FRISK_EW_INPUT;
+    d.arg[d.n_ops++] = k;
+    if (k) d.op[d.n_ops++] = k & 1 ? FRISK_EW_ADD : FRISK_EW_MUL;
+  }
+  std::printf("status %d\n", frisk_hip_elementwise(&d, in, at(8), nullptr));
+  return 0;
+}
+
+int main(int argc, char** argv) {
+  const std::string what = argc > 1 ? argv[1] : "";
+  if (what == "gemm" && argc == 10) return gemm(argv + 2);
+  if (what == "block" && argc == 6) return block(argv + 2);
+  return 2;
+}

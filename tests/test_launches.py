@@ -1,0 +1,40 @@
+"""What a call launches, recorded on the CPU: an executable whose own definitions of the HIP runtime's calls come before the runtime's prints them."""
+import os
+import subprocess
+
+import pytest
+
+from frisk_amd import runtime as R
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+
+
+@pytest.fixture(scope="module")
+def recorded(tmp_path_factory):
+    exe = str(tmp_path_factory.mktemp("launches") / "launch_recorder")
+    rocm, lib = os.environ.get("ROCM_PATH", "/opt/rocm"), os.path.dirname(R.LIB_PATH)
+    subprocess.run([os.environ.get("CXX", "g++"), "-O1", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-I" + os.path.join(rocm, "include"), "-I" + os.path.join(ROOT, "include"),
+                    os.path.join(HERE, "launch_recorder.cpp"), "-o", exe, "-L" + lib, "-lfrisk_hip", "-L" + os.path.join(rocm, "lib"), "-lamdhip64", "-ldl",
+                    "-Wl,-rpath," + lib, "-Wl,-rpath," + os.path.join(rocm, "lib")], check=True)
+
+    def run(*args):
+        """(status, [(kernel, grid x, grid y, lanes)])"""
+        out = subprocess.run([exe] + [str(a) for a in args], check=True, capture_output=True, text=True).stdout.split("\n")
+        launches = [l.split()[1:] for l in out if l.startswith("launch ")]
+        return int([l for l in out if l.startswith("status ")][0].split()[1]), [(n, int(x), int(y), int(lanes)) for n, x, y, _, lanes in launches]
+    return run
+
+
+@pytest.mark.parametrize("keep", ["keep", "nokeep"])
+@pytest.mark.parametrize("dt,M,N,K,transA,transB", [(R.F16, 1999, 4099, 3001, 0, 0), (R.F16, 1589, 3072, 9600, 0, 0), (R.F16, 4, 576, 6784, 0, 0), (R.I8, 58, 2240, 7680, 0, 0)])
+def test_a_call_without_workspace_uses_none_of_the_plan_that_needs_one(recorded, dt, M, N, K, transA, transB, keep):
+    """copies, split edge tiles, slices of K: planned again without a workspace, nothing of the first plan is left, also where the thread has no storage for the
+    plans it keeps"""
+    need = R.workspace_bytes(R.make_desc(dt, M, N, K, transA=transA, transB=transB, dtype_out=R.I32 if dt == R.I8 else None))
+    assert need > 0
+    status, with_it = recorded("gemm", keep, dt, M, N, K, transA, transB, need)
+    assert status == 0 and len(with_it) >= 2
+    for too_small in (0, 16):
+        status, launches = recorded("gemm", keep, dt, M, N, K, transA, transB, too_small)
+        assert status == 0 and len(launches) == 1 and "gemm_kernel" in launches[0][0] and launches[0][2] == 1, launches
