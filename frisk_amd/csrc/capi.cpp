@@ -633,9 +633,9 @@ static double round_time(RoundModel m, const KernelEntry* k, const frisk_gemm_de
 struct PlanContext { bool a_off = false, b_off = false, c_off = false; size_t workspace = kAnyWorkspace; };
 // Operands that are copied to aligned rows in the workspace before the product runs, and where they go.
 struct Repack { bool a = false, b = false; int64_t lda = 0, ldb = 0; size_t b_offset = 0, bytes = 0; };
-// What a launch needs of a plan beyond the public structure: the copies, the splits whose slices differ in length (of K, where the structure says 1, and the
-// tail split of an edge kernel, its partial sums behind the copies in the workspace).
-struct LaunchExtras { Repack repack; int split_k = 1; int tail_split = 1, tail_tiles = 0; size_t partial_offset = 0; };
+// What a launch needs of a plan beyond the public structure: the copies, and the tail split of an edge kernel (whose slices may
+// differ in length), its partial sums behind the copies in the workspace.
+struct LaunchExtras { Repack repack; int tail_split = 1, tail_tiles = 0; size_t partial_offset = 0; };
 
 static Repack repack_of(const frisk_gemm_desc* d, bool a, bool b) {
   Repack r;
@@ -1028,8 +1028,7 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
   } else if (d->split_k > 1 && !no_split) {
     return fail(FRISK_ERR_TILE, "split_k=%d: the chosen kernel %s has no split-K path", d->split_k, k->name);
   }
-  plan->split_k = kt % split ? 1 : split;
-  if (extras) extras->split_k = split;
+  plan->split_k = split;
   if (split > 1) plan->workspace_bytes = (size_t)split * (size_t)d->M * (size_t)d->N * 4;
   if (plan->tail_split <= 1) { plan->tail_split = 1; plan->tail_tiles = 0; }
   return FRISK_OK;
@@ -1161,7 +1160,7 @@ int frisk_hip_gemm(const frisk_gemm_desc* desc, const void* A, const void* B, vo
   p.xcd_remap = plan.xcd_remap;
   p.epilogue = desc->epilogue; p.dtype_out = desc->dtype_out; p.accumulate = desc->clear_accum ? 0 : 1;
   const KernelEntry* k = kernels()[plan.kernel_id];
-  p.split_k = extras.split_k;
+  p.split_k = plan.split_k;
   p.kt_per_slice = (int)(((desc->K + k->bk - 1) / k->bk + p.split_k - 1) / p.split_k);
   const Repack& repack = extras.repack;
   const int tail_split = std::max(plan.tail_split, extras.tail_split);

@@ -125,7 +125,8 @@ typedef struct frisk_gemm_plan {
   int32_t stages, stages_b;          /* LDS ring depth for tiles of A and of B */
   int32_t lds_bytes;                 /* total, <= 163840 */
   int32_t grid_x, grid_y;            /* work-group grid (tiles along N, tiles along M) */
-  int32_t split_k;                   /* >1: partial sums go through the workspace */
+  int32_t split_k;                   /* >1: slices of K, whose partial sums go through the workspace: ceil(K tiles / split_k) K tiles
+                                        each, and what is left, at least one, for the last (a split the descriptor names divides them) */
   int32_t xcd_remap;                 /* 1: work-group ids are remapped so each XCD owns a compact block of tiles */
   int32_t guarded;                   /* 1: K off the K tile, unaligned rows or pointers, or a tile that only exists as such a kernel */
   frisk_lds_layout lds_a, lds_b;

@@ -67,13 +67,17 @@ def test_every_plan_is_a_kernel_that_may_run_on_the_problem(seed):
             assert rows_aligned and K % (16 // es) == 0, what
         assert bool(p.guarded) == (guard is not None), what
         if p.split_k > 1:
-            assert splitk and K % bk == 0 and (K // bk) % p.split_k == 0 and p.workspace_bytes == p.split_k * M * N * 4, what
-            assert split in (0, p.split_k), what
+            # slices of equal length but the last, which holds at least one K tile; those of a split that the descriptor names divide the K tiles
+            per = -(-(K // bk) // p.split_k)
+            assert splitk and K % bk == 0 and (p.split_k - 1) * per < K // bk and p.workspace_bytes == p.split_k * M * N * 4, what
+            assert split in (0, p.split_k) and (split == 0 or (K // bk) % split == 0), what
         else:
             assert p.split_k == 1, what
         if p.tail_split > 1:
             assert splitk and not edge and p.tail_tiles == (p.grid_x * p.grid_y) % 256 and (K // bk) % p.tail_split == 0, what
             assert p.workspace_bytes == p.tail_split * p.tail_tiles * bm * bn * 4, what
+        if splitk and p.workspace_bytes:
+            assert p.split_k > 1 or p.tail_split > 1, what
         if split == 1:
             assert p.split_k == 1 and p.tail_split == 1 and p.workspace_bytes == 0, what
     # the walk reached every kind of kernel
@@ -107,8 +111,8 @@ def test_kept_plans_are_those_of_their_descriptor():
 
 
 def test_slices_of_unequal_length_leave_the_last_one_its_k_tiles():
-    """a split in slices of unequal length, which the plan reports by its workspace alone: every slice holds K tiles, the last one at least as many as the
-    kernel's loop is written for (16x16x128 atoms: four); a split that the caller names still has to divide them"""
+    """a split in slices of unequal length: the plan says how many, every slice holds K tiles, the last one at least as many as the kernel's loop is
+    written for (16x16x128 atoms: four); a split that the caller names still has to divide them"""
     uneven = 0
     for dt in (R.F16, R.I8, R.E4M3):
         for tb in (0, 1):
@@ -117,12 +121,12 @@ def test_slices_of_unequal_length_leave_the_last_one_its_k_tiles():
                     d = R.make_desc(dt, M, N, K, transB=tb, dtype_out={R.F16: R.F16, R.I8: R.F16, R.E4M3: R.BF16}[dt],
                                     epilogue={R.F16: R.EPI_NONE, R.I8: R.EPI_ROW_COL_SCALE, R.E4M3: R.EPI_TENSOR_SCALE}[dt])
                     p = R.plan(d)
-                    if p.split_k > 1 or p.tail_split > 1 or not p.workspace_bytes or "_splitk" not in R.kernel_names()[p.kernel_id]:
+                    kt, slices = K // p.tile_k, p.split_k
+                    if kt % slices == 0:
                         continue
-                    kt, slices = K // p.tile_k, p.workspace_bytes // (M * N * 4)
                     per = -(-kt // slices)
                     last = kt - (slices - 1) * per
-                    assert K % p.tile_k == 0 and p.workspace_bytes == slices * M * N * 4 and slices > 1, (dt, M, N, K)
+                    assert K % p.tile_k == 0 and p.workspace_bytes == slices * M * N * 4 and slices > 1 and p.tail_split == 1, (dt, M, N, K)
                     assert (4 if dt == R.E4M3 and p.mfma_m == 16 else 1) <= last < per, (dt, M, N, K, slices)
                     assert R.plan(R.make_desc(dt, M, N, K, transB=tb, dtype_out=d.dtype_out, epilogue=d.epilogue, split_k=1)).workspace_bytes == 0
                     uneven += 1
