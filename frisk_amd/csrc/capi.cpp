@@ -1044,8 +1044,11 @@ static int planned(const frisk_gemm_desc* d, frisk_gemm_plan* plan, const PlanCo
   struct Kept { frisk_gemm_desc desc; PlanContext ctx; frisk_gemm_plan plan; LaunchExtras extras; bool used = false; };
   static thread_local std::unique_ptr<Kept[]> kept(new (std::nothrow) Kept[kKeptPlans]);
   if (!d || !kept) return make_plan(d, plan, false, ctx, extras);
+  // (one shape on two leading dimensions, output types or pointer alignments in turn are two places)
   uint64_t h = (uint64_t)d->M * 0x9e3779b97f4a7c15ull ^ (uint64_t)d->N * 0xc2b2ae3d27d4eb4full ^ (uint64_t)d->K * 0x165667b19e3779f9ull;
   h ^= (uint64_t)ctx.workspace * 0xd6e8feb86659fd93ull + (uint64_t)((d->dtype_ab * 4 + d->transA * 2 + d->transB) * 16 + d->epilogue * 4 + (d->clear_accum ? 1 : 0));
+  h += (uint64_t)d->lda * 0xa0761d6478bd642full ^ (uint64_t)d->ldb * 0xe7037ed1a0b428dbull ^ (uint64_t)d->ldc * 0x8ebc6af09c88c6e3ull;
+  h += (uint64_t)(d->dtype_out * 8 + ctx.a_off * 4 + ctx.b_off * 2 + ctx.c_off) * 0x589965cc75374cc3ull;
   Kept& k = kept[(h * 0x9e3779b97f4a7c15ull) >> 58];
   static_assert(kKeptPlans == 64, "the place is the top six bits of the product");
   const bool same = k.used && std::memcmp(&k.desc, d, sizeof *d) == 0 && k.ctx.a_off == ctx.a_off && k.ctx.b_off == ctx.b_off && k.ctx.c_off == ctx.c_off && k.ctx.workspace == ctx.workspace;

@@ -2,9 +2,12 @@
 // loader finds them first, and print what they are asked for instead.  Pointers are made up; nothing reads them.
 //
 //   launch_recorder gemm keep|nokeep <dtype> <M> <N> <K> <transA> <transB> <workspace bytes>
+//   launch_recorder kept
 //   launch_recorder block <dtype> <rows> <cols> <operands: m = rows x cols, r = one value a row, c = one a column>
 #include <dlfcn.h>
 #include <hip/hip_runtime_api.h>
+#include <algorithm>
+#include <chrono>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -12,7 +15,7 @@
 #include <string>
 #include "frisk_hip.h"
 
-static bool g_keep = true;
+static bool g_keep = true, g_quiet = false;
 
 extern "C" {
 static struct { dim3 grid, block; size_t lds; hipStream_t stream; } g_pushed;
@@ -22,6 +25,7 @@ hipError_t __hipPopCallConfiguration(dim3* grid, dim3* block, size_t* lds, hipSt
   return hipSuccess;
 }
 hipError_t hipLaunchKernel(const void* kernel, dim3 grid, dim3 block, void**, size_t, hipStream_t) {
+  if (g_quiet) return hipSuccess;
   Dl_info info{};
   dladdr(kernel, &info);
   std::printf("launch %s %u %u %u %u\n", info.dli_sname ? info.dli_sname : "?", grid.x, grid.y, grid.z, block.x);
@@ -55,6 +59,47 @@ static int gemm(char** arg) {
   return 0;
 }
 
+// nanoseconds of a call, the least of many rounds: one call over and over; the same shape in turn on two leading dimensions, output types and pointer alignments,
+// the median of seven shapes (two plans in 64 places may still meet); a shape that comes round too late to be kept
+static int kept() {
+  g_quiet = true;
+  frisk_gemm_desc base{};
+  base.abi_version = FRISK_HIP_ABI_VERSION;
+  base.dtype_ab = FRISK_F16; base.dtype_acc = FRISK_F32; base.dtype_out = FRISK_F16;
+  base.M = 48; base.N = 4096; base.K = 4096;
+  base.lda = base.K; base.ldb = base.ldc = base.N;
+  base.clear_accum = 1;
+  auto least = [](auto call) {
+    double best = 1e9;
+    for (int round = 0; round < 40; ++round) {
+      const auto t0 = std::chrono::steady_clock::now();
+      for (int i = 0; i < 200; ++i) call(i);
+      best = std::min(best, std::chrono::duration<double, std::nano>(std::chrono::steady_clock::now() - t0).count() / 200);
+    }
+    return best;
+  };
+  auto pair = [&](const char* what, auto change, size_t off) {
+    double ns[7];
+    for (int k = 0; k < 7; ++k) {
+      frisk_gemm_desc one = base, other = base;
+      one.M = other.M = 41 + k;
+      change(other);
+      ns[k] = least([&](int i) { frisk_hip_gemm(i & 1 ? &other : &one, (char*)at(0) + (i & 1 ? off : 0), at(1), at(2), nullptr, nullptr, nullptr, 0, nullptr); });
+    }
+    std::sort(ns, ns + 7);
+    std::printf("%s %.1f\n", what, ns[3]);
+  };
+  pair("again", [](frisk_gemm_desc&) {}, 0);
+  pair("lda", [](frisk_gemm_desc& d) { d.lda += 8; }, 0);
+  pair("ldb", [](frisk_gemm_desc& d) { d.ldb += 8; }, 0);
+  pair("ldc", [](frisk_gemm_desc& d) { d.ldc += 8; }, 0);
+  pair("dtype_out", [](frisk_gemm_desc& d) { d.dtype_out = FRISK_F32; }, 0);
+  pair("alignment", [](frisk_gemm_desc&) {}, 2);
+  int n = 0;
+  std::printf("new %.1f\n", least([&](int) { frisk_gemm_desc d = base; d.M = 33 + n++ % 32; d.N += 64 * (n % 97); d.ldb = d.ldc = d.N; frisk_hip_gemm(&d, at(0), at(1), at(2), nullptr, nullptr, nullptr, 0, nullptr); }));
+  return 0;
+}
+
 static int block(char** arg) {
   frisk_elementwise_desc d{};
   const std::string operands = arg[3];
@@ -79,6 +124,7 @@ static int block(char** arg) {
 int main(int argc, char** argv) {
   const std::string what = argc > 1 ? argv[1] : "";
   if (what == "gemm" && argc == 10) return gemm(argv + 2);
+  if (what == "kept") return kept();
   if (what == "block" && argc == 6) return block(argv + 2);
   return 2;
 }
