@@ -1055,7 +1055,7 @@ static int planned(const frisk_gemm_desc* d, frisk_gemm_plan* plan, const PlanCo
   if (!same) {
     LaunchExtras fresh;
     frisk_gemm_plan p;
-    if (int st = make_plan(d, &p, false, ctx, &fresh); st != FRISK_OK) { *plan = p; return st; }
+    if (int st = make_plan(d, &p, false, ctx, &fresh); st != FRISK_OK) return st;  // (p may not have been written)
     k = Kept{*d, ctx, p, fresh, true};
   }
   *plan = k.plan;
