@@ -684,7 +684,7 @@ static int follow_up(const std::vector<Variant>& list, const KernelEntry* k, con
     // as many leave most CUs without one.  us, operands in the last-level cache, on 64x64 or 32x128 tiles / so: 128x1280x1024 NN 18.9 / 9.1,
     // 896x256x1792 30.8 / 14.1, 128x384x896 16.3 / 7.6, 256x2048x1408 (512) 24.9 / 17.8; off the tiles 323x130x437 NT 13.8 / 10.0, 8-row problems of 4000 to
     // 9000 columns half the time; but 512x1152x512 (576) 11.2 / 12.4, 1280x640x768 (800) 16.2 / 19.7, and in a second round on fewer than two K
-    // tiles of 128 296x856x160 (270) 6.2 / 7.2
+    // tiles of 128 296x856x160 (270) 6.2 / 7.2; whole tiles under A [K][M] 256x256x512 TN 10.5 / 6.0, 512x512x512 TT 11.4 / 6.7, 1024x512x256 7.6 / 6.6
     return k->wk == 1 && d->K >= (tiles_of(32, 32) <= 256 ? 128 : 256) && tiles_of(32, 32) <= 512 ? variant(32, 32, 2) : -1;
   }
   const int64_t k_bytes = d->K * es;

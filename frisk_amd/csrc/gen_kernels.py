@@ -142,7 +142,8 @@ VARIANTS = {
             + [edge((0, tb, 32, 128, 32, 1, 4, 3, 0, 1, 1)) for tb in (0, 1)] + [edge((0, tb, 64, 64, 32, 2, 2, 3, 0, 1, 1)) for tb in (0, 1)]
             + [(ta, tb, 64, 64, 32, 2, 2, 2, 1, 0, 1) for ta in (0, 1) for tb in (0, 1)]
             # 32x32 tiles, the four waves splitting K, where 64x64 ones leave CUs idle and K is not split (`follow_up` in capi.cpp)
-            + [(0, 0, 32, 32, 128, 1, 1, 2, 0, 0, 4)] + [edge((ta, tb, 32, 32, 128, 1, 1, 2, 0, 0, 4)) for ta in (0, 1) for tb in (0, 1)]),
+            # (plain ones where the search has none of that tile, which it has for B [N][K] under A [M][K])
+            + [(ta, tb, 32, 32, 128, 1, 1, 2, 0, 0, 4) for ta, tb in ((0, 0), (1, 0), (1, 1))] + [edge((ta, tb, 32, 32, 128, 1, 1, 2, 0, 0, 4)) for ta in (0, 1) for tb in (0, 1)]),
 }
 
 def cfg_of(enum, v):

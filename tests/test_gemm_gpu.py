@@ -494,6 +494,23 @@ def test_fp32_small_grids_split_k(hip, transA, transB):
         check(O.F32, O.F32, run_gemm(hip, O.F32, A, B, transA, transB, O.F32, M, N, K, C_init=C0, clear_accum=False), ref + C0)
 
 
+@pytest.mark.parametrize("transA", [0, 1])
+@pytest.mark.parametrize("M,N,K", [(32, 32, 128), (64, 96, 384), (256, 256, 512), (512, 480, 640), (1024, 512, 256)])
+def test_fp32_whole_32_row_tiles(hip, M, N, K, transA):
+    """whole tiles of the 32x32 kernel whose four waves split K, from a single one to more than one a CU, of one to five K tiles; both layouts of B under A
+    [K][M], into C and onto it"""
+    for transB in (0, 1) if transA else (0,):
+        sa, sb = stored_shapes(M, N, K, transA, transB)
+        A, B = make_operand(O.F32, *sa, seed=67, tensor=0, scale=0.5), make_operand(O.F32, *sb, seed=67, tensor=1, scale=0.5)
+        ref = O.gemm_f64(O.F32, A, B, transA, transB)
+        name = hip.kernel_names()[hip.plan(hip.make_desc(O.F32, M, N, K, transA=transA, transB=transB)).kernel_id]
+        assert name.endswith("_32x32x128_w1x1x4_s2"), name
+        note(f"case fp32 whole 32x32 tA={transA} tB={transB} {M}x{N}x{K}")
+        check(O.F32, O.F32, run_gemm(hip, O.F32, A, B, transA, transB, O.F32, M, N, K), ref)
+        C0 = O.uniform(M * N, 67, 2, -1.0, 1.0).reshape(M, N).astype(np.float32)
+        check(O.F32, O.F32, run_gemm(hip, O.F32, A, B, transA, transB, O.F32, M, N, K, C_init=C0, clear_accum=False), ref + C0)
+
+
 @pytest.mark.parametrize("dtype", [O.F16, O.BF16, O.I8, O.E4M3, O.F32])
 @pytest.mark.parametrize("transA,transB", [(0, 0), (0, 1), (1, 0), (1, 1)])
 def test_edge_kernels_take_any_m_and_n(hip, dtype, transA, transB):

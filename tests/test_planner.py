@@ -556,3 +556,12 @@ def test_64x64_tiles_in_place_of_few_slices_of_64x128_ones(dt, M, N, K, lay, til
     """129 to 255 tiles of 64x64, A stored along K (8-bit types: B too)"""
     name, p = _route(dt, M, N, K, lay)
     assert tile in name.split("_w")[0] and (tile != "64x64" or (p.split_k, p.workspace_bytes) == (1, 0)), (name, p.split_k, p.workspace_bytes)
+
+
+@pytest.mark.parametrize("lay", ["NN", "NT", "TN", "TT"])
+@pytest.mark.parametrize("M,N,K", [(128, 128, 512), (256, 256, 512), (512, 256, 384), (384, 384, 512), (512, 512, 512)])
+def test_fp32_whole_tiles_take_the_32_row_tiles_that_ragged_ones_take(M, N, K, lay):
+    """64x64 tiles would leave most CUs without one, in every layout"""
+    for rows in (M, M + 4):
+        name, p = _route(R.F32, rows, N, K, lay)
+        assert "_32x32x128_" in name and p.split_k == 1 and p.workspace_bytes == 0, (rows, name)
