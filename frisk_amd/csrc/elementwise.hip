@@ -469,14 +469,15 @@ hipError_t launch_elementwise(const EwParams& given, hipStream_t s) {
   // first group (up to 1000 instructions) is paid once per lane.  us with 16 / 4 per CU: (x - s c) g + b of 8192 x 8192 f16 54.8 / 51.6, 3000 x 4096 16.7 /
   // 11.5, 6330 x 669 11.9 / 8.8, 4095 x 8191 bf16 32.3 / 28.5, 4000 x 4096 f32 28.1 / 26.0; x + y of 8192 x 8192 f16 69 / 64, 16000 x 3999 63.1 / 60.2; but
   // exp2(x) c of 16000 x 3999 44.7 / 48.1, and f32, with one group a lane under way, where 16 per CU still leave eight rows to a lane (8192 x 8192 101.8 /
-  // 106.5; 20000 x 2048 61.7 / 61.0).
+  // 106.5; 20000 x 2048 61.7 / 61.0).  Never more than the cap, where a row's slabs do not divide it: the few above a single round ran as a second one
+  // (1026 instead of 1020, x + b of 3000 x 11008 f16 29.3 us, 23.3 so, (x - s c) g + b 35.2 and 25.9, f32 66.4 and 59.1; 10000 x 5000 f16 54.7 and 40.1).
   const int64_t row_blocks = (p.rows + row_step - 1) / row_step;
   int64_t gx = 0, gy = 0;
   auto set_grid = [&](int64_t cap) {
     gx = (groups + lanes - 1) / lanes;
     gy = row_blocks;
     if (gx > cap) gx = cap;
-    if (gx * gy > cap) gy = (cap + gx - 1) / gx;
+    if (gx * gy > cap) gy = cap / gx;
     if (gy > 65535) gy = 65535;
   };
   // Holding the broadcast operands pays where a lane walks down two rows or more, not where its one group waits for them to be set up (us held / not,

@@ -47,3 +47,13 @@ def test_kept_plans_tell_leading_dimensions_types_and_alignments_apart(recorded)
     ns = recorded("kept")
     for what in ("lda", "ldb", "ldc", "dtype_out", "alignment"):
         assert ns[what] < (ns["again"] * ns["new"]) ** 0.5, ns
+
+
+@pytest.mark.parametrize("dt", [R.F16, R.BF16, R.F32])
+@pytest.mark.parametrize("cols", [2048, 4097, 5000, 11008, 20000, 16384])
+def test_block_bodies_with_held_operands_are_one_round_of_work_groups(recorded, dt, cols):
+    """as many work-groups as the chip holds at once, 4 a CU, also where a row's slabs of 2048 columns do not divide their number: a few more would run alone"""
+    for operands in ("mc", "mr", "mrc", "mcc"):
+        status, launches = recorded("block", dt, 6000 // -(-cols // 2048), cols, operands)
+        (_, x, y, lanes), = launches
+        assert status == 0 and lanes == 256 and x == -(-cols // 2048) and 1024 - x < x * y <= 1024, (operands, x, y)
