@@ -467,9 +467,12 @@ hipError_t launch_elementwise(const EwParams& given, hipStream_t s) {
   // Enough work-groups to fill the chip several times over, every lane walking its row / column strides beyond that: 16 per CU; of the kernels that
   // hold more than the first operand 4 per CU, a single round of those with broadcast operands (four waves a SIMD), so that what stands in front of the
   // first group (up to 1000 instructions) is paid once per lane.  us with 16 / 4 per CU: (x - s c) g + b of 8192 x 8192 f16 54.8 / 51.6, 3000 x 4096 16.7 /
-  // 11.5, 6330 x 669 11.9 / 8.8, 4095 x 8191 bf16 32.3 / 28.5, 4000 x 4096 f32 28.1 / 26.0; x + y of 8192 x 8192 f16 69 / 64, 16000 x 3999 63.1 / 60.2; but
-  // exp2(x) c of 16000 x 3999 44.7 / 48.1, and f32, with one group a lane under way, where 16 per CU still leave eight rows to a lane (8192 x 8192 101.8 /
-  // 106.5; 20000 x 2048 61.7 / 61.0).  Never more than the cap, where a row's slabs do not divide it: the few above a single round ran as a second one
+  // 11.5, 6330 x 669 11.9 / 8.8, 4095 x 8191 bf16 32.3 / 28.5, 4000 x 4096 f32 28.1 / 26.0; x + y of 8192 x 8192 f16 69 / 64; but exp2(x) c of 16000 x
+  // 3999, which holds no more than the first operand, 44.7 / 48.1.  f32, of which a lane has one group under way, goes back to 16 per CU where the set-up weighs little:
+  // from 12 groups a lane (on 4 per CU) with operands of one value a column held, from 7 with those of one value a row alone, from 5 with a second operand
+  // that walks the rows.  us with 16 / 4 per CU: (x - s c) g + b of 4096 x 4096 26.5 / 25.5, 4000 x 3000 30.3 / 27.9, but 4095 x 8191 60.4 / 60.9, 20000 x 2048
+  // 65.3 / 67.0, 10000 x 5000 85.4 / 88.1, 1000000 x 24 49.0 / 51.0; x s 2000 x 5000 16.9 / 15.3, 4000 x 3000 25.8 / 27.2; x g + y 2048 x 4096 21.8 / 20.1, 20000 x 300
+  // 20.4 / 18.4, but 3000 x 4096 30.1 / 31.0, 20000 x 2048 90.7 / 93.4; x + y 2048 x 4096 20.3 / 20.6, 4096 x 4096 38.4 / 39.2.  Never more than the cap, where a row's slabs do not divide it: the few above a single round ran as a second one
   // (1026 instead of 1020, x + b of 3000 x 11008 f16 29.3 us, 23.3 so, (x - s c) g + b 35.2 and 25.9, f32 66.4 and 59.1; 10000 x 5000 f16 54.7 and 40.1).
   const int64_t row_blocks = (p.rows + row_step - 1) / row_step;
   int64_t gx = 0, gy = 0;
@@ -481,18 +484,22 @@ hipError_t launch_elementwise(const EwParams& given, hipStream_t s) {
     if (gy > 65535) gy = 65535;
   };
   // Holding the broadcast operands pays where a lane walks down two rows or more, not where its one group waits for them to be set up (us held / not,
-  // two rows a lane: (x - s c) g + b of 1024 x 4096 f16 6.8 / 8.3, f32 9.4 / 10.3, 100000 x 24 f16 5.8 / 6.6, x + b of 1024 x 4096 f32 8.5 / 8.0)
+  // two rows a lane: (x - s c) g + b of 1024 x 4096 f16 6.8 / 8.3, f32 10.3 / 11.6, 100000 x 24 f16 5.8 / 6.6).  For two rows of f32 it does not pay for a single operand of
+  // one value a column, nor in rows shorter than a wave: x + b of 1024 x 4096 9.3 / 8.9, 100000 x 24 8.2 / 7.0, x g + b 8.8 / 8.0.
   set_grid(kHeldCap);
   const int most = (row_blocks + gy - 1) / gy >= 2 ? HELD_ALL : HELD_WALK;
   // one type for everything that moves with the rows: the kernels for it; mixed types: the one that looks at each operand's type,
   // which holds nothing ahead but the first operand
   EwSteps prog = steps_of(p, most);
   int dt = p.out_dtype;
+  const bool f32 = dt == FRISK_F32;
+  const int64_t steps = ((groups + lanes - 1) / lanes) * row_blocks;  // work-groups of one group a lane
+  if (f32 && most == HELD_ALL && steps <= 2 * kHeldCap && (lanes_log2 < 6 || (prog.col0 >= 0 && prog.col1 < 0 && prog.row0 < 0))) prog = steps_of(p, HELD_WALK);
   int held = prog.col0 >= 0 || prog.row0 >= 0 ? HELD_ALL : prog.walk2 >= 0 ? HELD_WALK : HELD_NONE;
-  if (held == HELD_NONE || (dt == FRISK_F32 && ((groups + lanes - 1) / lanes) * row_blocks >= 8 * kCap)) set_grid(kCap);
-  // f32 with three groups a lane and more: the larger kernel's four waves a SIMD stream better than five of the smaller one (us, four / five:
-  // x + y of 8192 x 8192 142 / 147, 20000 x 2048 87.6 / 90.5, 4095 x 8191 72.0 / 73.3; 4096 x 4096, two groups a lane, 38.7 / 37.3)
-  if (dt == FRISK_F32 && held == HELD_WALK && ((groups + lanes - 1) / lanes) * row_blocks >= 3 * gx * gy) held = HELD_ALL;
+  if (held == HELD_NONE || (f32 && steps > (prog.walk2 >= 0 ? 5 : prog.col0 < 0 ? 7 : 12) * kHeldCap)) set_grid(kCap);
+  // f32 with more than three groups a lane on 16 per CU: the larger kernel's four waves a SIMD stream better than five of the smaller one (us, four / five: x + y of
+  // 8192 x 8192 144.4 / 149.1, 20000 x 2048 88.1 / 90.4, 4095 x 8191 72.9 / 74.8; with two, 4096 x 4096 39.6 / 38.4, 3000 x 4096 29.9 / 29.2)
+  if (f32 && held == HELD_WALK && steps > 3 * kCap) held = HELD_ALL;
   if ((prog.head >= 0 && p.in_dtype[prog.head] != dt) || (prog.walk2 >= 0 && p.in_dtype[prog.walk2] != dt)) {
     dt = -1;
     held = HELD_NONE;
