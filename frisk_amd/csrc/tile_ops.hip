@@ -346,7 +346,12 @@ reduce_tall_kernel(const typename Elem<DT>::T* src, int64_t rows, int64_t cols, 
   typedef typename Elem<DT>::T T;
   constexpr int G = 16 / sizeof(T), FLIGHT = 8;
   const int lanes = 1 << lanes_log2, cl = threadIdx.x & (lanes - 1), rl = threadIdx.x >> lanes_log2, row_lanes = 1024 >> lanes_log2;
-  const int64_t c0 = (((int64_t)blockIdx.x << lanes_log2) + cl) * G;
+  // A row's last group, where it is not whole, is read with the columns before it that fill it up, which are another lane's: every load is 16 bytes of the
+  // row and eight are under way.  (Element by element, a row after the other, it held up the call: f16 1435 x 1495 25.0 us, 10.5 so,
+  // 970 x 8671 19.0 and 8.9.)
+  const int64_t first = (((int64_t)blockIdx.x << lanes_log2) + cl) * G;
+  const int before = first < cols && first + G > cols && cols >= G ? (int)(first + G - cols) : 0;
+  const int64_t c0 = first - before;
   float acc[G];
 #pragma unroll
   for (int e = 0; e < G; ++e) acc[e] = Op<KIND>::id();
@@ -363,7 +368,7 @@ reduce_tall_kernel(const typename Elem<DT>::T* src, int64_t rows, int64_t cols, 
         for (int e = 0; e < G; ++e) acc[e] = Op<KIND>::f(acc[e], Elem<DT>::load(in[u][e]));
       }
     }
-  } else if (c0 < cols) {
+  } else if (c0 < cols) {  // the only group of a row that has no more
     for (int64_t r = rl; r < rows; r += row_lanes) {
 #pragma unroll
       for (int e = 0; e < G; ++e)
@@ -378,7 +383,8 @@ reduce_tall_kernel(const typename Elem<DT>::T* src, int64_t rows, int64_t cols, 
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   if (lane < lanes) {
 #pragma unroll
-    for (int e = 0; e < G; ++e) red[wave][lane * G + e] = acc[e];
+    for (int e = 0; e < G; ++e)
+      if (e >= before) red[wave][lane * G + e - before] = acc[e];
   }
   __syncthreads();
   const int64_t c = ((int64_t)blockIdx.x << lanes_log2) * G + threadIdx.x;

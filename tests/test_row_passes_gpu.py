@@ -64,6 +64,30 @@ def test_reductions_with_several_loads_under_way(hip, dt, rows, cols, dim):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dt", [O.F32, O.F16, O.BF16])
+@pytest.mark.parametrize("pitch", ["dense", "lines", "odd"])
+def test_the_last_group_of_columns_reduced_in_one_launch(hip, dt, pitch):
+    """a last group of 1 to all but one columns, alone in its strip, with others and behind whole strips, of rows that start on 128-byte lines or anywhere; what
+    lies between the rows is no number.  Whole numbers whose sums every type holds: the same bits in any order."""
+    import torch
+    es, G = O.NP_STORAGE[dt]().itemsize, 16 // O.NP_STORAGE[dt]().itemsize
+    tdt = {O.F32: torch.float32, O.F16: torch.float16, O.BF16: torch.bfloat16}[dt]
+    g = torch.Generator(device="cuda").manual_seed(6)
+    for rows in (120, 1152, 1153, 1536):
+        for cols in [G - 1, G, 2 * G + 1] + [8 * G * k + r for k in (1, 3) for r in (0, 1, G - 1, G + 2, 8 * G - 1)]:
+            ld = {"dense": cols, "lines": -(-cols * es // 128) * 128 // es, "odd": cols + 1 + (cols & 1)}[pitch]
+            x = torch.full((rows, ld), float("nan"), device="cuda", dtype=tdt)
+            x[:, :cols] = (torch.rand(rows, cols, device="cuda", generator=g) < 0.06).to(tdt) * (2 * torch.randint(0, 2, (rows, cols), device="cuda", generator=g) - 1).to(tdt)
+            need = hip.reduce_workspace_bytes(dt, rows, cols, 0)
+            ws = torch.full((max(need, 4),), 0xFF, dtype=torch.uint8, device="cuda")
+            for with_ws in (True, False):
+                d = torch.full((cols + 1,), 7.0, device="cuda", dtype=tdt)
+                hip.reduce(dt, x.data_ptr(), rows, cols, ld, 0, "add", True, d.data_ptr(), ws.data_ptr() if need and with_ws else None, need if with_ws else 0, torch.cuda.current_stream().cuda_stream)
+                torch.cuda.synchronize()
+                assert torch.equal(d[:cols].float(), x[:, :cols].float().sum(0)) and float(d[cols]) == 7.0, (rows, cols, ld, with_ws)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("dt,tdt", [(O.F32, "float32"), (O.F16, "float16"), (O.BF16, "bfloat16")])
 @pytest.mark.parametrize("rows", [1, 5, 2600])
 def test_the_last_group_of_a_row(hip, dt, tdt, rows):
