@@ -340,7 +340,8 @@ reduce_cols_kernel(const typename Elem<DT>::T* src, int64_t rows, int64_t cols, 
 // LDS.  What it saves is the launch that combines the slices: us in two launches / so, f16 309 x 3904 6.9 / 4.1, 256 x 1024 7.0 / 4.1, 1259 x 1728 7.6 /
 // 6.3, f32 309 x 3904 7.4 / 4.3.  A work-group walks its strip at some 40 bytes a nanosecond (1024 lanes, of which all wait, then all add), so from
 // 2000 rows on the slices are ahead again (f16 2000 x 1984 7.9 / 8.3, 3000 x 1024 8.6 / 13.3), and so they are where there is more than one strip for
-// every CU (1000 x 65536 25.2 / 27.7).
+// every CU (1000 x 65536 25.2 / 27.7).  Rows that do not start on 128-byte lines, of which a strip takes two each, leave the range from 1152 on unless they are short (f32 1452 x
+// 460 7.1 / 9.2, f16 1379 x 2120 7.9 / 9.7, 1228 x 1544 11 % slower; but 970 x 8671 12.3 / 8.9, 1354 x 56 10.6 / 5.4, and on lines 1434 x 7414 13.4 / 8.1).
 template <int DT, int KIND> __global__ void __launch_bounds__(1024)
 reduce_tall_kernel(const typename Elem<DT>::T* src, int64_t rows, int64_t cols, int64_t ld, int clear, typename Elem<DT>::T* dst, int lanes_log2) {
   typedef typename Elem<DT>::T T;
@@ -468,8 +469,11 @@ template <int SDT, int DDT> hipError_t copy_tiles_t(const void* src, int64_t sld
 // a launch may hold fewer than 2^32 lanes: grids are capped and work-groups loop
 constexpr int64_t kMaxGrid = 1 << 22;
 
-// (`gpr`: groups of 16 bytes in a row)
-bool cols_in_one_launch(int64_t rows, int64_t gpr) { return rows <= 1536 && gpr <= 256 * 8; }
+// `on_lines`: every row starts on a 128-byte boundary.  Where they don't, a strip of 128 bytes takes two lines of every row, and the slices are ahead sooner (lines
+// at reduce_tall_kernel).
+bool cols_in_one_launch(int64_t rows, int64_t row_bytes, bool on_lines) {
+  return rows <= (on_lines || row_bytes <= 256 ? 1536 : 1152) && row_bytes <= 256 * 128;
+}
 
 // slices of the reduced extent that give the launch enough work-groups
 int split_of(int dtype, int64_t rows, int64_t cols, int dim) {
@@ -489,6 +493,10 @@ template <int DT, int KIND> hipError_t reduce_t(const void* src, int64_t rows, i
   typedef typename Elem<DT>::T T;
   constexpr int G = 16 / sizeof(T);
   const int64_t gpr = (cols + G - 1) / G;
+  // (without slices the one launch takes every view of its range)
+  const bool tall = dim == 0 && split_of(DT, rows, cols, dim) > 1 &&
+                    cols_in_one_launch(rows, cols * (int64_t)sizeof(T), slices == 1 || ((uintptr_t)src % 128 == 0 && ld * sizeof(T) % 128 == 0));
+  if (tall) slices = 1;
   if (dim == 1) {
     if (gpr <= 256 && slices == 1) {
       int lanes_log2 = 0;
@@ -502,7 +510,7 @@ template <int DT, int KIND> hipError_t reduce_t(const void* src, int64_t rows, i
       hipLaunchKernelGGL((reduce_rows_kernel<DT, KIND>), dim3((unsigned)(rows < kMaxGrid ? rows : kMaxGrid), (unsigned)slices), dim3(256), 0, s, (const T*)src, rows, cols,
                          ld, clear, (T*)dst, partial);
     }
-  } else if (slices == 1 && split_of(DT, rows, cols, dim) > 1 && cols_in_one_launch(rows, gpr)) {
+  } else if (tall) {
     int lanes_log2 = 0;
     while (lanes_log2 < 3 && (int64_t(1) << lanes_log2) < gpr) ++lanes_log2;
     hipLaunchKernelGGL((reduce_tall_kernel<DT, KIND>), dim3((unsigned)((gpr + (1 << lanes_log2) - 1) >> lanes_log2)), dim3(1024), 0, s, (const T*)src, rows, cols, ld, clear,
@@ -537,9 +545,9 @@ template <int DT> hipError_t reduce_k(int kind, const void* src, int64_t rows, i
 
 }  // namespace
 
+// (where the one launch depends on the rows' pitch, the slices' sums have their place all the same)
 int reduce_slices(int dtype, int64_t rows, int64_t cols, int dim) {
-  const int64_t gpr = (cols * (dtype == FRISK_F32 ? 4 : 2) + 15) / 16;
-  return dim == 0 && cols_in_one_launch(rows, gpr) ? 1 : split_of(dtype, rows, cols, dim);
+  return dim == 0 && cols_in_one_launch(rows, cols * (dtype == FRISK_F32 ? 4 : 2), false) ? 1 : split_of(dtype, rows, cols, dim);
 }
 
 hipError_t launch_fill(int dtype, void* dst, int64_t rows, int64_t cols, int64_t ld, double value, hipStream_t s) {

@@ -4,6 +4,7 @@
 //   launch_recorder gemm keep|nokeep <dtype> <M> <N> <K> <transA> <transB> <workspace bytes>
 //   launch_recorder kept
 //   launch_recorder block <dtype> <rows> <cols> <operands: m = rows x cols, r = one value a row, c = one a column>
+//   launch_recorder reduce <dtype> <rows> <cols> <leading dimension> <dim> <bytes from the source to a 256-byte boundary> <workspace: 1 what the library asks for, 0 none>
 #include <dlfcn.h>
 #include <hip/hip_runtime_api.h>
 #include <algorithm>
@@ -121,10 +122,19 @@ static int block(char** arg) {
   return 0;
 }
 
+static int reduce(char** arg) {
+  const int dtype = std::atoi(arg[0]), dim = std::atoi(arg[4]);
+  const int64_t rows = std::atoll(arg[1]), cols = std::atoll(arg[2]);
+  const size_t bytes = std::atoi(arg[6]) ? frisk_hip_reduce_workspace_bytes(dtype, rows, cols, dim) : 0;
+  std::printf("status %d\n", frisk_hip_reduce(dtype, (char*)at(0) + std::atoi(arg[5]), rows, cols, std::atoll(arg[3]), dim, FRISK_REDUCE_ADD, 1, at(1), bytes ? at(3) : nullptr, bytes, nullptr));
+  return 0;
+}
+
 int main(int argc, char** argv) {
   const std::string what = argc > 1 ? argv[1] : "";
   if (what == "gemm" && argc == 10) return gemm(argv + 2);
   if (what == "kept") return kept();
+  if (what == "reduce" && argc == 9) return reduce(argv + 2);
   if (what == "block" && argc == 6) return block(argv + 2);
   return 2;
 }

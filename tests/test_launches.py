@@ -68,3 +68,15 @@ def test_grids_of_f32_block_bodies(recorded, rows, cols, operands, groups):
     status, launches = recorded("block", R.F32, rows, cols, operands)
     (_, x, y, _), = launches
     assert status == 0 and groups - x < x * y <= groups, (x, y)
+
+
+@pytest.mark.parametrize("dt,rows,cols,ld,off,one", [
+    (R.F16, 1152, 1495, 1495, 0, True), (R.F16, 1153, 1495, 1495, 0, False), (R.F16, 1435, 1495, 1536, 0, True), (R.F16, 1435, 1495, 1536, 16, False),  # rows anywhere, on 128-byte lines, off by a chunk
+    (R.F16, 1536, 128, 131, 0, True), (R.F16, 1536, 129, 131, 0, False), (R.F32, 1452, 460, 460, 0, False), (R.F32, 1452, 480, 480, 0, True),            # 256 bytes of a row and more
+    (R.BF16, 1537, 1536, 1536, 0, False), (R.BF16, 1000, 16384, 16385, 0, True), (R.BF16, 1000, 16385, 16385, 0, False)])
+def test_column_reductions_in_one_launch_or_in_slices(recorded, dt, rows, cols, ld, off, one):
+    """work-groups of 1024 lanes up to 1152 rows, on 128-byte lines or of 256 bytes at most up to 1536, else slices and their sums; without a workspace always one launch"""
+    status, launches = recorded("reduce", dt, rows, cols, ld, 0, off, 1)
+    assert status == 0 and [lanes for _, _, _, lanes in launches] == ([1024] if one else [256, 256]), launches
+    status, launches = recorded("reduce", dt, rows, cols, ld, 0, off, 0)
+    assert status == 0 and [lanes for _, _, _, lanes in launches] == [1024 if rows <= 1536 and cols < 16385 else 256], launches
