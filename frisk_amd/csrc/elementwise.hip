@@ -483,20 +483,28 @@ hipError_t launch_elementwise(const EwParams& given, hipStream_t s) {
     if (gx * gy > cap) gy = cap / gx;
     if (gy > 65535) gy = 65535;
   };
-  // Holding the broadcast operands pays where a lane walks down two rows or more, not where its one group waits for them to be set up (us held / not,
-  // two rows a lane: (x - s c) g + b of 1024 x 4096 f16 6.8 / 8.3, f32 10.3 / 11.6, 100000 x 24 f16 5.8 / 6.6).  For two rows of f32 it does not pay for a single operand of
-  // one value a column, nor in rows shorter than a wave: x + b of 1024 x 4096 9.3 / 8.9, 100000 x 24 8.2 / 7.0, x g + b 8.8 / 8.0.
-  set_grid(kHeldCap);
-  const int most = (row_blocks + gy - 1) / gy >= 2 ? HELD_ALL : HELD_WALK;
+  // Holding the broadcast operands pays where a lane walks down two rows or more, not where its one group waits for them to be set up, and the kernels that hold none fit
+  // five work-groups on a CU: up to 5 / 4 of the smaller grid is a round of one group a lane.  us on 4 per CU, held / one group a lane, 1.004, 1.1, 1.25 and 1.5 times that grid: f16 x + b
+  // of 2048 columns 4.9 / 4.0, 5.0 / 4.2, 5.0 / 4.3, 5.1 / 5.3, (x - s c) g + b 5.7 / 5.6, 5.8 / 5.8, 5.9 / 5.9, 5.9 / 7.7, x y + z 5.9 / 5.2, 6.1 / 5.3, 6.4 / 5.6, 7.6 / 8.3, f32 x g + b
+  // 6.8 / 6.4, 7.4 / 7.0, 7.9 / 7.7, 8.8 / 9.3; Alone, without a second operand that walks the rows, 6 / 4 for one operand of one value a row (x s 4.8 / 4.2, 4.8 / 4.3, 4.9 / 4.5, 5.0 / 4.8, twice the grid 5.5 / 6.2), twice the grid for one of one value a column
+  // in f32 or in rows shorter than a wave (x + b f16 of 24 columns 5.2 / 4.9, f32 of 4096 9.3 / 9.5, 1.75 times 9.0 / 8.9).  f32 with operands of one value a row in longer rows holds them at once (x s 6.1 / 6.3).
+  const EwSteps all = steps_of(p, HELD_ALL);
+  const bool f32 = p.out_dtype == FRISK_F32, short_rows = lanes_log2 < 6;
+  const int columns = (all.col0 >= 0) + (all.col1 >= 0), per_row = (all.row0 >= 0) + (all.row1 >= 0);
+  int quarters = 5;  // of kHeldCap work-groups
+  if (f32 && per_row && !short_rows) quarters = 4;
+  else if (all.walk2 < 0 && columns == 1 && !per_row && (f32 || short_rows)) quarters = 8;
+  else if (all.walk2 < 0 && per_row == 1 && !columns) quarters = 6;
+  const int64_t steps = ((groups + lanes - 1) / lanes) * row_blocks;  // work-groups of one group a lane
+  const bool few = 4 * steps <= quarters * kHeldCap;
   // one type for everything that moves with the rows: the kernels for it; mixed types: the one that looks at each operand's type,
   // which holds nothing ahead but the first operand
-  EwSteps prog = steps_of(p, most);
+  EwSteps prog = few ? steps_of(p, HELD_WALK) : all;
   int dt = p.out_dtype;
-  const bool f32 = dt == FRISK_F32;
-  const int64_t steps = ((groups + lanes - 1) / lanes) * row_blocks;  // work-groups of one group a lane
-  if (f32 && most == HELD_ALL && steps <= 2 * kHeldCap && (lanes_log2 < 6 || (prog.col0 >= 0 && prog.col1 < 0 && prog.row0 < 0))) prog = steps_of(p, HELD_WALK);
   int held = prog.col0 >= 0 || prog.row0 >= 0 ? HELD_ALL : prog.walk2 >= 0 ? HELD_WALK : HELD_NONE;
-  if (held == HELD_NONE || (f32 && steps > (prog.walk2 >= 0 ? 5 : prog.col0 < 0 ? 7 : 12) * kHeldCap)) set_grid(kCap);
+// (16-bit ones too, beside a second operand that walks long rows and from 28 groups a lane on: x g + y of 8192 x 8192 f16 59.9 with 16 per CU, 63.8 with 4; 24 groups, 6144 x 8192, 58.7 / 56.0)
+  const bool deep = f32 ? steps > (prog.walk2 >= 0 ? 5 : prog.col0 < 0 ? 7 : 12) * kHeldCap : prog.walk2 >= 0 && held == HELD_ALL && lanes_log2 == 8 && steps > 28 * kHeldCap;
+  set_grid(held == HELD_NONE || few || deep ? kCap : kHeldCap);
   // f32 with more than three groups a lane on 16 per CU: the larger kernel's four waves a SIMD stream better than five of the smaller one (us, four / five: x + y of
   // 8192 x 8192 144.4 / 149.1, 20000 x 2048 88.1 / 90.4, 4095 x 8191 72.9 / 74.8; with two, 4096 x 4096 39.6 / 38.4, 3000 x 4096 29.9 / 29.2)
   if (f32 && held == HELD_WALK && steps > 3 * kCap) held = HELD_ALL;

@@ -59,12 +59,24 @@ def test_block_bodies_with_held_operands_are_one_round_of_work_groups(recorded, 
         assert status == 0 and lanes == 256 and x == -(-cols // 2048) and 1024 - x < x * y <= 1024, (operands, x, y)
 
 
+@pytest.mark.parametrize("dt,rows,cols,operands,groups", [
+    (R.F16, 7, 300000, "mc", 1029), (R.BF16, 640, 4096, "mrcc", 1280), (R.F16, 641, 4096, "mrcc", 1024), (R.F32, 640, 4096, "mmc", 1280),    # five work-groups a CU in one round
+    (R.F16, 768, 4096, "mr", 1536), (R.F16, 769, 4096, "mr", 1024), (R.F32, 513, 4096, "mr", 1024), (R.F32, 1024, 4096, "mc", 2048),          # one broadcast operand
+    (R.F16, 131072, 24, "mc", 2048), (R.F16, 100000, 24, "mcm", 1024),
+    (R.F16, 7168, 8192, "mcm", 1024), (R.F16, 7169, 8192, "mcm", 4096), (R.F16, 7169, 8192, "mcc", 1024)])                                    # a second operand that walks long rows
+def test_grids_of_block_bodies_with_few_or_many_groups_a_lane(recorded, dt, rows, cols, operands, groups):
+    """one group a lane where the kernels that hold no broadcast operand take all of them at once; 16 work-groups a CU again from 28 groups a lane beside a second walking operand"""
+    status, launches = recorded("block", dt, rows, cols, operands)
+    (_, x, y, _), = launches
+    assert status == 0 and groups - x < x * y <= groups, (x, y)
+
+
 @pytest.mark.parametrize("rows,cols,operands,groups", [
     (2048, 4096, "mm", 1024), (3000, 4096, "mm", 4096), (4096, 4096, "mm", 4096), (4096, 4096, "mcm", 4096), (20000, 300, "mcm", 1024),  # a second operand that walks the rows
     (1500, 7000, "mr", 1024), (4096, 4096, "mr", 4096), (4096, 4096, "mrcc", 1024), (6200, 4096, "mrcc", 4096),                        # held operands alone
-    (100000, 24, "mr", 1563), (200000, 24, "mrc", 1024)])                                                                             # rows shorter than a wave
+    (200000, 24, "mrc", 1024)])                                                                                                                                       # rows shorter than a wave
 def test_grids_of_f32_block_bodies(recorded, rows, cols, operands, groups):
-    """4 work-groups a CU up to 5, 7 or 12 groups a lane, 16 beyond; of two rows a lane one each where nothing is held"""
+    """4 work-groups a CU up to 5, 7 or 12 groups a lane, 16 beyond"""
     status, launches = recorded("block", R.F32, rows, cols, operands)
     (_, x, y, _), = launches
     assert status == 0 and groups - x < x * y <= groups, (x, y)
