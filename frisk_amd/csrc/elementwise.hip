@@ -488,11 +488,15 @@ hipError_t launch_elementwise(const EwParams& given, hipStream_t s) {
   // of 2048 columns 4.9 / 4.0, 5.0 / 4.2, 5.0 / 4.3, 5.1 / 5.3, (x - s c) g + b 5.7 / 5.6, 5.8 / 5.8, 5.9 / 5.9, 5.9 / 7.7, x y + z 5.9 / 5.2, 6.1 / 5.3, 6.4 / 5.6, 7.6 / 8.3, f32 x g + b
   // 6.8 / 6.4, 7.4 / 7.0, 7.9 / 7.7, 8.8 / 9.3; Alone, without a second operand that walks the rows, 6 / 4 for one operand of one value a row (x s 4.8 / 4.2, 4.8 / 4.3, 4.9 / 4.5, 5.0 / 4.8, twice the grid 5.5 / 6.2), twice the grid for one of one value a column
   // in f32 or in rows shorter than a wave (x + b f16 of 24 columns 5.2 / 4.9, f32 of 4096 9.3 / 9.5, 1.75 times 9.0 / 8.9).  f32 with operands of one value a row in longer rows holds them at once (x s 6.1 / 6.3).
+  // f32 in rows shorter than a wave, whose lanes each look for a column's value, holds none up to 5 times the grid beside a second operand that walks the rows, up to 12 times where there are one or two and
+  // up to twice with more: us held on 4 per CU / not held on 16, 2, 4 and 8 times, 24 columns: x + b 9.9 / 8.1, 16.6 / 14.9, 28.0 / 23.3, x s 9.8 / 8.9, 16.3 / 15.3, 27.9 / 26.0, x g + b 10.7 / 9.3,
+  // 17.5 / 16.9, 28.4 / 27.2, x g + y 11.6 / 11.3, 20.1 / 19.1, 34.7 / 33.7 (held on 16 33.7), (x - s c) g + b 11.5 / 10.7, 18.6 / 19.8, 30.2 / 32.7; 12 times, held on 16 / not, x g + b 39.0 / 37.8, 16 times 46.8 / 47.3.
   const EwSteps all = steps_of(p, HELD_ALL);
   const bool f32 = p.out_dtype == FRISK_F32, short_rows = lanes_log2 < 6;
   const int columns = (all.col0 >= 0) + (all.col1 >= 0), per_row = (all.row0 >= 0) + (all.row1 >= 0);
   int quarters = 5;  // of kHeldCap work-groups
-  if (f32 && per_row && !short_rows) quarters = 4;
+  if (f32 && short_rows && columns + per_row) quarters = all.walk2 >= 0 ? 20 : columns + per_row <= 2 ? 48 : 8;
+  else if (f32 && per_row) quarters = 4;
   else if (all.walk2 < 0 && columns == 1 && !per_row && (f32 || short_rows)) quarters = 8;
   else if (all.walk2 < 0 && per_row == 1 && !columns) quarters = 6;
   const int64_t steps = ((groups + lanes - 1) / lanes) * row_blocks;  // work-groups of one group a lane

@@ -74,9 +74,9 @@ def test_grids_of_block_bodies_with_few_or_many_groups_a_lane(recorded, dt, rows
 @pytest.mark.parametrize("rows,cols,operands,groups", [
     (2048, 4096, "mm", 1024), (3000, 4096, "mm", 4096), (4096, 4096, "mm", 4096), (4096, 4096, "mcm", 4096), (20000, 300, "mcm", 1024),  # a second operand that walks the rows
     (1500, 7000, "mr", 1024), (4096, 4096, "mr", 4096), (4096, 4096, "mrcc", 1024), (6200, 4096, "mrcc", 4096),                        # held operands alone
-    (200000, 24, "mrc", 1024)])                                                                                                                                       # rows shorter than a wave
+    (100000, 24, "mr", 1563), (200000, 24, "mrc", 3125), (800000, 24, "mrc", 4096), (200000, 24, "mrcc", 1024), (120000, 24, "mrcc", 1875), (350000, 24, "mcm", 4096)])  # rows shorter than a wave
 def test_grids_of_f32_block_bodies(recorded, rows, cols, operands, groups):
-    """4 work-groups a CU up to 5, 7 or 12 groups a lane, 16 beyond"""
+    """4 work-groups a CU up to 5, 7 or 12 groups a lane, 16 beyond; in rows shorter than a wave 16 where nothing is held"""
     status, launches = recorded("block", R.F32, rows, cols, operands)
     (_, x, y, _), = launches
     assert status == 0 and groups - x < x * y <= groups, (x, y)
