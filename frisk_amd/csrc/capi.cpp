@@ -791,9 +791,15 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
   // with few K tiles the launch that makes the copies costs more than it saves.  us staged / on copies: fp32 28x24x26 NN 4.8 / 7.5, 69x16x17 4.9 / 7.2,
   // 78x18x35 TN 5.9 / 7.0, bf16 16x25x21 NT 6.9 / 7.6; but int8 24x884x344 TN 10.6 / 8.4,
   // fp32 123x9x168 NN 9.7 / 7.7
-  const double staged_rounds = std::max(1.0, (double)((d->M + 127) / 128) * (double)((d->N + 127) / 128) / 512.0);
+  const int64_t k_tiles = ((int64_t)d->K * es + 127) / 128, tiles128 = ((d->M + 127) / 128) * ((d->N + 127) / 128), tiles64 = ((d->M + 63) / 64) * ((d->N + 63) / 64);
+  const double staged_rounds = std::max(1.0, (double)tiles128 / 512.0);
+  // Two more cases of grids of at most 256 tiles of 128x128.  8-bit problems of two K tiles (all layouts but TN, where A comes in rows of M and B in rows of N and both are turned on the way to
+  // LDS; us staged / on copies: int8 76x529x162 NN 9.3 / 10.7, e4m3 158x1761x133 NN 9.4 / 10.7, 73x294x179 TT 9.3 / 10.4, NN 6 % and TT 9 % on average, TN 6 % faster on copies; three K
+  // tiles NN 9.3 / 8.5).  Operands stored along K, which staging through registers costs least, beyond the 64x64 tiles and short of the ring of 3 that `follow_up` has for copies: 4
+  // to 11 K tiles 5 % on average, e4m3 525x3807x542 13.2 / 14.5, int8 1482x2240x730 14.1 / 15.9, bf16 943x2739x586 17.4 / 18.8; with 12 and more, or in 64x64 tiles, copies gain 4 to 50 %.
+  const bool staged_ahead = es < 4 && tiles128 <= 256 && (!d->transA && d->transB ? k_tiles < 12 && tiles64 >= 256 : es == 1 && k_tiles <= 2 && !(d->transA && !d->transB));
   const bool copies_lose = packed.bytes && !tile_requested && d->policy == FRISK_POLICY_SQUARE &&
-                           staged_rounds * (double)(((int64_t)d->K * es + 127) / 128) * (es == 4 ? 0.72 : es == 2 ? 1.4 : 2.2) < 3.5 + (double)packed.bytes / 2.2e6;
+                           (staged_ahead || staged_rounds * (double)k_tiles * (es == 4 ? 0.72 : es == 2 ? 1.4 : 2.2) < 3.5 + (double)packed.bytes / 2.2e6);
   bool policy_excluded = false;
   const bool any_layout = !list.empty();
   const bool small = small_grid(d);
@@ -865,13 +871,13 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
       if (k->guard == 2) cost += repack_cost;
       // What staging through registers costs beyond the model of its tile, a K tile of 128 bytes: on small grids 0.3 us where both operands are stored along K,
       // else 1.0 (8-bit 0.75); on larger ones, whose CUs hold two, 0.55, 1.0, 1.2 (int8) and 1.9 (8-bit float).  Fitted to 330 and 75 problems.  (As a factor of
-      // 1.6 alone it kept problems of many K tiles from the copies.  Of 400 drawn problems with rows off 16 bytes 248 change over, 25 % faster, 11 of them slower by
-      // 3 to 12 %, one by 25.  us staged / on copies: e4m3 2410x865x1222 TN 24.8 / 18.1, 2511x2241x536 TT 26.7 / 17.2, fp16 1524x1901x861 NN 29.7 / 21.3,
+      // 1.6 alone it kept problems of many K tiles from the copies.  Of 400 drawn problems with rows off 16 bytes 248 change over, 25 % faster.  The few that were slower, by
+      // 3 to 25 %, `staged_ahead` leaves as they were.  us staged / on copies: e4m3 2410x865x1222 TN 24.8 / 18.1, 2511x2241x536 TT 26.7 / 17.2, fp16 1524x1901x861 NN 29.7 / 21.3,
       // 6720x832x1337 NN 44.0 / 30.8, bf16 2321x2172x1978 NT 50.7 / 38.4; but int8 445x2933x150 NN 10.3 / 11.6, 464x2236x198 NT 8.8 / 11.7, which stay staged)
       if (k->guard == 1 && !k->edge && es < 4) {
         const bool along_k = !d->transA && d->transB;
         const double rate = along_k ? (small ? 0.32 : 0.55) : es == 2 ? 1.0 : small ? 0.75 : k->dtype == FRISK_I8 ? 1.2 : 1.9;
-        cost += staged_rounds * (double)(((int64_t)d->K * es + 127) / 128) * rate;
+        cost += staged_rounds * (double)k_tiles * rate;
       }
       // ties: the first listed variant is the tuned default
       if (best < 0 || (ks[best]->guard && !k->guard && !planners_own(ks[best])) || cost < best_cost) { best = v.id; best_cost = cost; }

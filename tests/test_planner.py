@@ -565,3 +565,13 @@ def test_fp32_whole_tiles_take_the_32_row_tiles_that_ragged_ones_take(M, N, K, l
     for rows in (M, M + 4):
         name, p = _route(R.F32, rows, N, K, lay)
         assert "_32x32x128_" in name and p.split_k == 1 and p.workspace_bytes == 0, (rows, name)
+
+
+@pytest.mark.parametrize("dt,M,N,K,lay,copies", [
+    (R.I8, 76, 529, 162, "NN", False), (R.E4M3, 73, 294, 179, "TT", False), (R.I8, 394, 75, 204, "TN", True), (R.I8, 158, 1761, 257, "NN", True), (R.E4M3, 3252, 2942, 142, "NN", True),  # two K tiles
+    (R.E4M3, 525, 3807, 542, "NT", False), (R.I8, 1482, 2240, 730, "NT", False), (R.BF16, 943, 2739, 586, "NT", False), (R.F16, 1039, 1384, 703, "NT", False),                   # stored along K
+    (R.F16, 1039, 1384, 705, "NT", True), (R.E4M3, 1039, 1384, 1409, "NT", True), (R.BF16, 943, 929, 586, "NT", True), (R.F16, 1039, 1384, 595, "NN", True)])
+def test_rows_off_16_bytes_stay_staged_where_copies_gain_nothing(dt, M, N, K, lay, copies):
+    """8-bit types with two K tiles, and operands stored along K of fewer than 12 in 256 tiles of 64x64 and more, on at most 256 tiles of 128x128"""
+    name, p = _route(dt, M, N, K, lay)
+    assert name.endswith("_s2_guard") == (not copies) and (p.workspace_bytes > 0) == copies, (name, p.workspace_bytes)
