@@ -730,10 +730,13 @@ static int follow_up(const std::vector<Variant>& list, const KernelEntry* k, con
 // The edge tile (its index) that takes a problem of more than 256 tiles of 128x128 over from `k`, which the search has found and
 // which runs it in one pass: the one whose rounds the model sees through 3 % sooner, -1 where there is none.  The search's costs know nothing of what a round pays beside
 // its K loop, nor of bytes of C: a 256x256 tile of 4-byte C with old values is 512 KiB, 19 us of a round whatever the K.  us before / now, operands
-// in rotation: fp16 1596x3540x778 NN 24.4 on 192x256 / 18.8 on 128x128, 6656x1664x361 TN into fp32 sums 34.8 on 256x256 / 26.6 on 128x128; 2156x3328x6528 NN
-// 102.8 on 128x128 / 86.7 on 160x256, 3325x2420x2483 NT 56.6 on 128x128 / 49.1 on 160x256, 2368x5376x5376 NT 111.6 on 256x256 / 105.1 on 224x256.  Of 600 problems drawn
+// from memory: fp16 1596x3540x778 NN 24.4 on 192x256 / 18.8 on 128x128, 6656x1664x361 TN into fp32 sums 34.8 on 256x256 / 26.6 on 128x128; 3325x2420x2483 NT 56.6 on
+// 128x128 / 49.1 on 160x256, 2368x5376x5376 NT 111.6 on 256x256 / 105.1 on 224x256.  Of 600 problems drawn
 // over the four types 150 or so change over, 15 % faster, one of them slower (int8 4288x7424x640 NT, 38.1 / 39.7).  The 160- and 224-row tiles from 12 K tiles on (their longer
 // prologue; with fewer the smaller tiles are as good).
+// Where the 128x128 tiles are one round, two a CU, which hides a wait for memory that one 160x256 tile cannot, what is gained hangs on where the operands come from: of 99 drawn 16-bit
+// problems 160x256 tiles are 10 % faster with both in the last-level cache (2156x3328x6528 NN 102.2 / 89.9), 5 % with A there and B from memory (101.2 / 94.8) and 3 % slower, NN 6 %, with both from
+// memory (101.1 / 108.2).  int8, of 12, 5, 4 and -6 % (960x6144x4096 NT 29.4 / 31.0, 34.4 / 34.8, 35.7 / 39.3), stays on 128x128.
 static int other_tile(const std::vector<Variant>& list, const KernelEntry* k, const frisk_gemm_desc* d, bool rows_aligned, const Repack& packed) {
   const int es = elem_size(k->dtype), os = elem_size(d->dtype_out);
   const bool whole_k = d->K % k->bk == 0;
@@ -745,6 +748,7 @@ static int other_tile(const std::vector<Variant>& list, const KernelEntry* k, co
   };
   const RoundModel* now = k->guard && !k->edge ? nullptr : tile_model(k);
   if (!now || d->K <= k->bk) return -1;  // (a single K tile has no loop to model)
+  const bool two_a_cu = now->cap == 512 && ((d->M + 127) / 128) * ((d->N + 127) / 128) <= 512;  // a single round of 128x128 tiles
   double best_time = 0.97 * time(k, now);
   int best = -1;
   for (const Variant& v : list) {
@@ -752,7 +756,7 @@ static int other_tile(const std::vector<Variant>& list, const KernelEntry* k, co
     const RoundModel* m = x != k && x->edge && !x->splitk && x->stages == 2 ? tile_model(x) : nullptr;
     if (!m || x->guard != (rows_aligned && whole_k ? 0 : rows_aligned && d->K % (16 / es) == 0 ? 1 : 2) || (x->guard == 2 && k->guard != 2)) continue;
     if ((x->bm == 128 || x->bm == 256) && x->guard == 0 && d->M % x->bm == 0 && d->N % x->bn == 0) continue;  // the plain twin was there to be found
-    if ((x->bm == 160 || x->bm == 224) && (d->K + x->bk - 1) / x->bk < 12) continue;
+    if ((x->bm == 160 || x->bm == 224) && ((d->K + x->bk - 1) / x->bk < 12 || (es == 1 && two_a_cu))) continue;
     if ((d->K + x->bk - 1) / x->bk < x->min_k_tiles) continue;
     const double span_a = (double)(packed.a ? packed.lda : d->lda) * es * (d->transA ? x->bk : x->bm), span_b = (double)(packed.b ? packed.ldb : d->ldb) * es * (d->transB ? x->bn : x->bk);
     if (span_a >= 4294967296.0 || span_b >= 4294967296.0) continue;

@@ -575,3 +575,9 @@ def test_rows_off_16_bytes_stay_staged_where_copies_gain_nothing(dt, M, N, K, la
     """8-bit types with two K tiles, and operands stored along K of fewer than 12 in 256 tiles of 64x64 and more, on at most 256 tiles of 128x128"""
     name, p = _route(dt, M, N, K, lay)
     assert name.endswith("_s2_guard") == (not copies) and (p.workspace_bytes > 0) == copies, (name, p.workspace_bytes)
+
+
+@pytest.mark.parametrize("dt,M,N,K,lay,tile", [(R.I8, 960, 6144, 4096, "NT", "128x128"), (R.I8, 3904, 1792, 3328, "NT", "128x128"), (R.I8, 1664, 4544, 3968, "NN", "128x128"), (R.F16, 1999, 4096, 3008, "NN", "160x256"),
+                                               (R.BF16, 1384, 11008, 2240, "NT", "160x256"), (R.I8, 2400, 3584, 1536, "NT", "160x256")])
+def test_int8_keeps_a_single_round_of_two_128_row_tiles_a_cu(dt, M, N, K, lay, tile):
+    assert "_%sx" % tile in _route(dt, M, N, K, lay)[0]
