@@ -705,14 +705,15 @@ static int follow_up(const std::vector<Variant>& list, const KernelEntry* k, con
   const bool edge128 = k->edge && !k->splitk && k->bm == 128 && k->bn == 128;
   // 64x64 tiles in a single round, in place of 128x128 edge tiles, split or not, and of unsplit 64x128 tiles.  us, operands in the last-level cache:
   // fp16 525x1136x1480 NT 19.1 / 9.6, 558x296x1200 16.1 / 7.1, 852x824x1840 NN 19.8 / 11.8, 1229x608x3960 22.9 / 18.7, 768x1152x2048 12.0 / 9.3,
-  // e4m3 1408x576x2208 NT 18.7 / 8.2; in place of 64x128 tiles not for less than 1 KiB of K, 906x312x320 NT 5.0 / 5.2; with more than 7.5 KiB the slices have caught up, 494x1144x3768 NN 20.9 / 18.7
+  // e4m3 1408x576x2208 NT 18.7 / 8.2; in place of 64x128 tiles not for less than 1 KiB of K, 906x312x320 NT 5.0 / 5.2; with more than 7.5 KiB the slices have caught up, B [K][N] more than 7: from
+  // memory 239x183x3823 NN 21.3 in 8 slices / 25.1, 107x688x3480 19.8 / 22.7 (6 to 7 KiB 4 % faster, and NT 9 %)
   // ... and of 64x128 tiles whatever the K where they are unsplit, and where they are split into 2 slices (B [K][N]: up to 12 KiB of K) or 16-bit ones into
   // 3 (up to 7 KiB), for the second launch that goes: fp16 832x1216x6144 NN 29.6 / 22.2, 1088x832x4864 NT 19.5 / 17.7, 876x1088x5120 NN 22.0 / 19.7; in 2 slices
   // 928x896x4480 NT 23 % faster, e4m3 332x1920x6656 NT 16 %; but fp16 68x6656x8576 NN in 2 slices 17 % slower, 416x1408x8064 NN in 3 12 %.  Of 120 drawn problems
   // 67 change over, 13 % faster, one of them slower, by 3 %.
   const bool tall = k->bm == 64 && k->bn == 128;
   const bool sliced = tiles_of(64, 64) > 128 && (split == 2 ? d->transB || k_bytes <= 12288 : split == 3 && es == 2 && k_bytes <= 7168);
-  if (tiles_of(64, 64) < 256 && ((edge128 && k_bytes <= 7680) || (tall && (split == 1 ? k_bytes >= 1024 : sliced))))
+  if (tiles_of(64, 64) < 256 && ((edge128 && k_bytes <= (d->transB ? 7680 : 7168)) || (tall && (split == 1 ? k_bytes >= 1024 : sliced))))
     if (const int id = variant(64, 64, 3); id >= 0) return id;
   if (split > 1) return -1;
   // 128x128 tiles with 3 + 3 tiles of LDS in a single round, one on each CU, in place of unsplit 64x128 ones of which some CUs hold two: a third less to transfer.  us

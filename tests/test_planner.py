@@ -581,3 +581,10 @@ def test_rows_off_16_bytes_stay_staged_where_copies_gain_nothing(dt, M, N, K, la
                                                (R.BF16, 1384, 11008, 2240, "NT", "160x256"), (R.I8, 2400, 3584, 1536, "NT", "160x256")])
 def test_int8_keeps_a_single_round_of_two_128_row_tiles_a_cu(dt, M, N, K, lay, tile):
     assert "_%sx" % tile in _route(dt, M, N, K, lay)[0]
+
+
+@pytest.mark.parametrize("dt,M,N,K,lay,tile", [(R.F16, 408, 1026, 3664, "NN", "128x128"), (R.BF16, 97, 173, 3810, "NN", "128x128"), (R.F16, 408, 1026, 3584, "NN", "64x64"), (R.F16, 97, 173, 3810, "NT", "64x64"),
+                                               (R.BF16, 97, 173, 3848, "NT", "128x128")])
+def test_64x64_tiles_leave_deep_k_to_slices_of_128x128_ones(dt, M, N, K, lay, tile):
+    """up to 7 KiB of K where B is stored by columns, 7.5 KiB where it is stored along K"""
+    assert "_%sx" % tile in _route(dt, M, N, K, lay)[0]
