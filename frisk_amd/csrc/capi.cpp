@@ -691,15 +691,15 @@ static int follow_up(const std::vector<Variant>& list, const KernelEntry* k, con
   if (d->M <= 64) {
     // 64x64 tiles for up to 64 rows where they are one round that fills half the CUs and more, with 256 bytes of a row of B at a time and three tiles under way on
     // each.  In place of unsplit 32x128 and 64x128 tiles; of 32x128 ones in 2 slices on B [K][N], for the second launch that goes; and below 32 rows on B [N][K] of
-    // two 32x32 work-groups a CU (16-bit from 9 rows on, 8-bit up to 6000 of K: elsewhere as many are slower).  us, B from memory, before / so: bf16 5x11584x2304
+    // two 32x32 work-groups a CU (16-bit from 9 rows on and not where rows of B are a multiple of 4 KiB apart, 8-bit up to 6000 of K: elsewhere as many are slower).  us, B from memory, before / so: bf16 5x11584x2304
     // NN 17.9 / 12.3, 58x9536x3584 NN 22.1 / 15.9, 12x15296x6400 NN 41 / 32, fp16 13x10432x3456 NT 19.5 / 17.4, e4m3 1x9856x2944 NT 12.2 / 9.6; but fp16
-    // 6x14016x7808 NT 40.0 / 45, 24x15552x8192 NT (rows 16 KiB apart) 35 / 44, 10752x6144 NN in 3 slices 29.7 / 37.  Of 280 drawn problems 93 change over,
+    // 6x14016x7808 NT 40.0 / 45, 24x15552x8192 NT (rows 16 KiB apart) 35 / 44, bf16 19x15424x4096 NT (8 KiB) 20 % slower, 21x12736x6144 (12 KiB) 12 %, 10752x6144 NN in 3 slices 29.7 / 37.  Of 280 drawn problems 93 change over,
     // 13 % faster, none of them slower by 3 % and more.
     const int64_t wgs = tiles_of(64, 64);
     if (wgs <= 128 || wgs > 256 || (d->transB && d->M >= 32) || k_bytes < 2048) return -1;  // (measured from 2 KiB of K on)
     const bool two_a_cu = k->bm == 32 && k->bn == 32 && k->stages == 2;
     const bool so = k->bn == 128 ? split == 1 || (split == 2 && !d->transB && k->bm == 32 && wgs > 170)
-                                 : two_a_cu && split == 1 && (es == 2 ? d->M > 8 && d->K * es % 16384 : d->K < 6000 && d->K % 4096);
+                                 : two_a_cu && split == 1 && (es == 2 ? d->M > 8 && d->ldb * es % 4096 : d->K < 6000 && d->K % 4096);
     return so ? variant(64, 64, 3) : -1;
   }
   const bool edge128 = k->edge && !k->splitk && k->bm == 128 && k->bn == 128;

@@ -588,3 +588,10 @@ def test_int8_keeps_a_single_round_of_two_128_row_tiles_a_cu(dt, M, N, K, lay, t
 def test_64x64_tiles_leave_deep_k_to_slices_of_128x128_ones(dt, M, N, K, lay, tile):
     """up to 7 KiB of K where B is stored by columns, 7.5 KiB where it is stored along K"""
     assert "_%sx" % tile in _route(dt, M, N, K, lay)[0]
+
+
+@pytest.mark.parametrize("dt,M,N,K,tile", [(R.BF16, 19, 15424, 4096, "32x32"), (R.F16, 10, 14144, 4096, "32x32"), (R.BF16, 21, 12736, 6144, "32x32"), (R.BF16, 11, 11712, 2048, "32x32"), (R.BF16, 19, 15424, 4224, "64x64"),
+                                           (R.E4M3, 7, 15424, 4096, "32x32"), (R.E4M3, 7, 15424, 2048, "64x64")])
+def test_few_rows_on_weights_whose_rows_lie_a_multiple_of_4_kib_apart(dt, M, N, K, tile):
+    """16-bit weights stored along K stay on the 32x32 tiles that fetch 512 bytes of a row at a time"""
+    assert "_%sx" % tile in _route(dt, M, N, K, "NT")[0]
