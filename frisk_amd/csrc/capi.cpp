@@ -792,7 +792,7 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
   int best = -1;
   double best_cost = 0.0;
   const bool tile_requested = d->tile_m || d->tile_n || d->tile_k || d->waves_m || d->waves_n || d->stages || d->atom;
-  // The kernels staged through registers take any rows in one launch, 1.4 us per K tile of 128 bytes behind those that work on copies (8-bit 2.2, fp32 0.7), so
+  // The kernels staged through registers take any rows in one launch, 1.4 us per K tile of 128 bytes behind those that work on copies (TT 1.25, 8-bit 2.2, fp32 0.7), so
   // with few K tiles the launch that makes the copies costs more than it saves.  us staged / on copies: fp32 28x24x26 NN 4.8 / 7.5, 69x16x17 4.9 / 7.2,
   // 78x18x35 TN 5.9 / 7.0, bf16 16x25x21 NT 6.9 / 7.6; but int8 24x884x344 TN 10.6 / 8.4,
   // fp32 123x9x168 NN 9.7 / 7.7
@@ -804,7 +804,7 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
   // to 11 K tiles 5 % on average, e4m3 525x3807x542 13.2 / 14.5, int8 1482x2240x730 14.1 / 15.9, bf16 943x2739x586 17.4 / 18.8; with 12 and more, or in 64x64 tiles, copies gain 4 to 50 %.
   const bool staged_ahead = es < 4 && tiles128 <= 256 && (!d->transA && d->transB ? k_tiles < 12 && tiles64 >= 256 : es == 1 && k_tiles <= 2 && !(d->transA && !d->transB));
   const bool copies_lose = packed.bytes && !tile_requested && d->policy == FRISK_POLICY_SQUARE &&
-                           (staged_ahead || staged_rounds * (double)k_tiles * (es == 4 ? 0.72 : es == 2 ? 1.4 : 2.2) < 3.5 + (double)packed.bytes / 2.2e6);
+                           (staged_ahead || staged_rounds * (double)k_tiles * (es == 4 ? 0.72 : es == 1 ? 2.2 : d->transA && d->transB ? 1.25 : 1.4) < 3.5 + (double)packed.bytes / 2.2e6);
   bool policy_excluded = false;
   const bool any_layout = !list.empty();
   const bool small = small_grid(d);

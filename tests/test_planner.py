@@ -595,3 +595,9 @@ def test_64x64_tiles_leave_deep_k_to_slices_of_128x128_ones(dt, M, N, K, lay, ti
 def test_few_rows_on_weights_whose_rows_lie_a_multiple_of_4_kib_apart(dt, M, N, K, tile):
     """16-bit weights stored along K stay on the 32x32 tiles that fetch 512 bytes of a row at a time"""
     assert "_%sx" % tile in _route(dt, M, N, K, "NT")[0]
+
+
+@pytest.mark.parametrize("dt,M,N,K,lay,copies", [(R.BF16, 2540, 407, 171, "TT", False), (R.BF16, 2178, 889, 188, "TT", False), (R.F16, 304, 913, 162, "TT", True), (R.BF16, 2540, 407, 171, "NN", True), (R.BF16, 2540, 407, 235, "TT", True)])
+def test_three_k_tiles_under_a_and_b_both_transposed_stay_staged_where_there_is_much_to_copy(dt, M, N, K, lay, copies):
+    name, p = _route(dt, M, N, K, lay)
+    assert name.endswith("_s2_guard") == (not copies) and (p.workspace_bytes > 0) == copies, (name, p.workspace_bytes)
