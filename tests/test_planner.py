@@ -601,9 +601,3 @@ def test_few_rows_on_weights_whose_rows_lie_a_multiple_of_4_kib_apart(dt, M, N, 
 def test_three_k_tiles_under_a_and_b_both_transposed_stay_staged_where_there_is_much_to_copy(dt, M, N, K, lay, copies):
     name, p = _route(dt, M, N, K, lay)
     assert name.endswith("_s2_guard") == (not copies) and (p.workspace_bytes > 0) == copies, (name, p.workspace_bytes)
-
-
-@pytest.mark.parametrize("dt,M,N,K,lay,tile", [(R.BF16, 2880, 2304, 6528, "NN", "128x128"), (R.F16, 1901, 3392, 6400, "NN", "128x128"), (R.BF16, 2880, 2304, 6528, "NT", "x256"), (R.BF16, 2398, 3072, 2240, "NN", "160x256")])
-def test_large_operands_keep_a_single_round_of_two_128_row_tiles_a_cu(dt, M, N, K, lay, tile):
-    """more than 64 MiB of operands and result, which a program hardly finds in the last-level cache"""
-    assert "%sx" % tile in _route(dt, M, N, K, lay)[0]
