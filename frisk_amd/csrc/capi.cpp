@@ -737,7 +737,8 @@ static int follow_up(const std::vector<Variant>& list, const KernelEntry* k, con
 // prologue; with fewer the smaller tiles are as good).
 // Where the 128x128 tiles are one round, two a CU, which hides a wait for memory that one 160x256 tile cannot, what is gained hangs on where the operands come from: of 99 drawn 16-bit
 // problems 160x256 tiles are 10 % faster with both in the last-level cache (2156x3328x6528 NN 102.2 / 89.9), 5 % with A there and B from memory (101.2 / 94.8) and 3 % slower, NN 6 %, with both from
-// memory (101.1 / 108.2).  int8, of 12, 5, 4 and -6 % (960x6144x4096 NT 29.4 / 31.0, 34.4 / 34.8, 35.7 / 39.3), stays on 128x128.
+// memory (101.1 / 108.2).  int8, of 87, 3, 2 and -6 % (960x6144x4096
+// NT 29.4 / 31.0, 34.4 / 34.8, 35.7 / 39.3) and e4m3, on 192x256 tiles 5 to 11 % slower wherever they come from, stay on 128x128.
 static int other_tile(const std::vector<Variant>& list, const KernelEntry* k, const frisk_gemm_desc* d, bool rows_aligned, const Repack& packed) {
   const int es = elem_size(k->dtype), os = elem_size(d->dtype_out);
   const bool whole_k = d->K % k->bk == 0;
@@ -757,7 +758,8 @@ static int other_tile(const std::vector<Variant>& list, const KernelEntry* k, co
     const RoundModel* m = x != k && x->edge && !x->splitk && x->stages == 2 ? tile_model(x) : nullptr;
     if (!m || x->guard != (rows_aligned && whole_k ? 0 : rows_aligned && d->K % (16 / es) == 0 ? 1 : 2) || (x->guard == 2 && k->guard != 2)) continue;
     if ((x->bm == 128 || x->bm == 256) && x->guard == 0 && d->M % x->bm == 0 && d->N % x->bn == 0) continue;  // the plain twin was there to be found
-    if ((x->bm == 160 || x->bm == 224) && ((d->K + x->bk - 1) / x->bk < 12 || (es == 1 && two_a_cu))) continue;
+    if (es == 1 && two_a_cu && x->bm != 128) continue;
+    if ((x->bm == 160 || x->bm == 224) && (d->K + x->bk - 1) / x->bk < 12) continue;
     if ((d->K + x->bk - 1) / x->bk < x->min_k_tiles) continue;
     const double span_a = (double)(packed.a ? packed.lda : d->lda) * es * (d->transA ? x->bk : x->bm), span_b = (double)(packed.b ? packed.ldb : d->ldb) * es * (d->transB ? x->bn : x->bk);
     if (span_a >= 4294967296.0 || span_b >= 4294967296.0) continue;

@@ -578,8 +578,9 @@ def test_rows_off_16_bytes_stay_staged_where_copies_gain_nothing(dt, M, N, K, la
 
 
 @pytest.mark.parametrize("dt,M,N,K,lay,tile", [(R.I8, 960, 6144, 4096, "NT", "128x128"), (R.I8, 3904, 1792, 3328, "NT", "128x128"), (R.I8, 1664, 4544, 3968, "NN", "128x128"), (R.F16, 1999, 4096, 3008, "NN", "160x256"),
+                                               (R.E4M3, 960, 7936, 5632, "NT", "128x128"), (R.I8, 1856, 4352, 6528, "NN", "128x128"),
                                                (R.BF16, 1384, 11008, 2240, "NT", "160x256"), (R.I8, 2400, 3584, 1536, "NT", "160x256")])
-def test_int8_keeps_a_single_round_of_two_128_row_tiles_a_cu(dt, M, N, K, lay, tile):
+def test_8_bit_types_keep_a_single_round_of_two_128_row_tiles_a_cu(dt, M, N, K, lay, tile):
     assert "_%sx" % tile in _route(dt, M, N, K, lay)[0]
 
 
