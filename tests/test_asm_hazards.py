@@ -3,6 +3,7 @@ wait states an MFMA needs around them.  This test compiles a few of those kernel
 checks the two patterns that would be wrong: a vector instruction writing a register that an MFMA reads within the next
 few instructions (accumulator initialisation right before the first MFMA), and a vector instruction reading an MFMA
 result too soon after it (before the drain the kernel issues ahead of the epilogue)."""
+import concurrent.futures
 import os
 import re
 import shutil
@@ -14,16 +15,18 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 CSRC = os.path.join(ROOT, "frisk_amd", "csrc")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
-SOURCE = """
-#include "gemm_kernel.hip.inc"
-namespace frisk {
-template __global__ void gemm_kernel<GemmCfg<FRISK_F16, 0, 1, 256, 256, 64, 2, 2, 2, false, false, 1, 3, 16>>(GemmParams);
-template __global__ void gemm_kernel<GemmCfg<FRISK_F16, 0, 0, 256, 256, 64, 2, 2, 2, false, true, 1, 3, 16>>(GemmParams);
-template __global__ void gemm_kernel<GemmCfg<FRISK_BF16, 1, 1, 256, 256, 64, 2, 2, 2, false, false, 1, 3, 16>>(GemmParams);
-template __global__ void gemm_kernel<GemmCfg<FRISK_I8, 1, 0, 256, 256, 128, 2, 2, 2, false, false, 1, 3, 16>>(GemmParams);
-template __global__ void gemm_kernel<GemmCfg<FRISK_E4M3, 0, 1, 256, 256, 128, 2, 2, 2, false, false, 1, 3, 16>>(GemmParams);
-}
-"""
+KERNELS = [
+    "template __global__ void gemm_kernel<GemmCfg<FRISK_F16, 0, 1, 256, 256, 64, 2, 2, 2, false, false, 1, 3, 16>>(GemmParams);",
+    "template __global__ void gemm_kernel<GemmCfg<FRISK_F16, 0, 0, 256, 256, 64, 2, 2, 2, false, true, 1, 3, 16>>(GemmParams);",
+    "template __global__ void gemm_kernel<GemmCfg<FRISK_BF16, 1, 1, 256, 256, 64, 2, 2, 2, false, false, 1, 3, 16>>(GemmParams);",
+    "template __global__ void gemm_kernel<GemmCfg<FRISK_I8, 1, 0, 256, 256, 128, 2, 2, 2, false, false, 1, 3, 16>>(GemmParams);",
+    "template __global__ void gemm_kernel<GemmCfg<FRISK_E4M3, 0, 1, 256, 256, 128, 2, 2, 2, false, false, 1, 3, 16>>(GemmParams);",
+    "template __global__ void gemm_kernel<GemmCfg<FRISK_F16, 0, 0, 160, 256, 64, 2, 2, 2, false, false, 1, 3, 16, true>>(GemmParams);",
+    "template __global__ void gemm_kernel<GemmCfg<FRISK_BF16, 0, 1, 192, 256, 64, 2, 2, 2, false, false, 1, 3, 16, true>>(GemmParams);",
+    "template __global__ void gemm_kernel<GemmCfg<FRISK_BF16, 0, 0, 224, 256, 64, 2, 2, 2, false, false, 1, 3, 16, true>>(GemmParams);",
+    "template __global__ void gemm_kernel<GemmCfg<FRISK_I8, 0, 1, 160, 256, 128, 2, 2, 2, false, false, 1, 3, 16, true>>(GemmParams);",
+    "template __global__ void gemm_kernel<GemmCfg<FRISK_I8, 0, 0, 224, 256, 128, 2, 2, 2, false, false, 1, 3, 16, true>>(GemmParams);",
+]
 
 
 def _registers(text):
@@ -101,14 +104,17 @@ def test_scanner_sees_both_patterns():
 
 @pytest.mark.skipif(not (os.path.exists(HIPCC) or shutil.which("hipcc")), reason="needs hipcc to produce the ISA listing")
 def test_inline_assembly_mfma_kernels_keep_their_wait_states(tmp_path):
-    src = tmp_path / "atoms16.hip"
-    src.write_text(SOURCE)
-    out = tmp_path / "atoms16.s"
-    cmd = [HIPCC if os.path.exists(HIPCC) else "hipcc", "--offload-arch=gfx950", "-O3", "-std=c++17", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
-           "-I" + os.path.join(ROOT, "include"), "-I" + CSRC, "-Wno-unused-command-line-argument", "--cuda-device-only", "-S", str(src), "-o", str(out)]
-    r = subprocess.run(cmd, capture_output=True, text=True)
-    assert r.returncode == 0, r.stderr[-2000:]
-    listing = out.read_text()
+    def compiled(i, kernel):  # (a unit each, side by side: one kernel takes half a minute)
+        src, out = tmp_path / ("atoms16_%d.hip" % i), tmp_path / ("atoms16_%d.s" % i)
+        src.write_text('#include "gemm_kernel.hip.inc"\nnamespace frisk {\n%s\n}\n' % kernel)
+        cmd = [HIPCC if os.path.exists(HIPCC) else "hipcc", "--offload-arch=gfx950", "-O3", "-std=c++17", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+               "-I" + os.path.join(ROOT, "include"), "-I" + CSRC, "-Wno-unused-command-line-argument", "--cuda-device-only", "-S", str(src), "-o", str(out)]
+        r = subprocess.run(cmd, capture_output=True, text=True)
+        assert r.returncode == 0, r.stderr[-2000:]
+        return out.read_text()
+
+    with concurrent.futures.ThreadPoolExecutor(min(8, os.cpu_count() or 1)) as pool:
+        listing = "\n".join(pool.map(compiled, range(len(KERNELS)), KERNELS))
     assert listing.count("v_mfma_f32_16x16x32_f16") > 300 and "v_mfma_i32_16x16x64_i8" in listing and "v_mfma_f32_16x16x32_bf16" in listing
     assert listing.count("v_mfma_f32_16x16x128_f8f6f4") >= 64 * 7 and "scratch_" not in listing  # seven tile bodies, no spills
     bad = hazards(listing)

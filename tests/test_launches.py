@@ -42,6 +42,15 @@ def test_a_call_without_workspace_uses_none_of_the_plan_that_needs_one(recorded,
         assert status == 0 and len(launches) == 1 and "gemm_kernel" in launches[0][0] and launches[0][2] == 1, launches
 
 
+@pytest.mark.parametrize("dt,M,N,K,transA,transB", [(R.E4M3, 2410, 865, 1222, 1, 0), (R.E4M3, 2511, 2241, 536, 1, 1), (R.BF16, 2321, 2172, 1978, 0, 1), (R.F16, 1524, 1901, 861, 0, 0),
+                                                    (R.I8, 445, 2933, 150, 0, 0), (R.F16, 157, 23, 32, 1, 1)])
+def test_rows_off_16_bytes_are_staged_through_registers_without_a_workspace(recorded, dt, M, N, K, transA, transB):
+    """the 128x128 kernel whose flag for it (the first of two after the wave grid and the ring) is set"""
+    status, launches = recorded("gemm", "keep", dt, M, N, K, transA, transB, 0)
+    (name, *_), = launches
+    assert status == 0 and "gemm_kernel" in name and "ELi128ELi128E" in name and "ELi2ELi2ELi2ELb1ELb0E" in name, name
+
+
 def test_kept_plans_tell_leading_dimensions_types_and_alignments_apart(recorded):
     """one shape in turn on two of them finds both plans kept: nearer to the time of a repeated call (0.06 us) than to that of a new one (2 us)"""
     ns = recorded("kept")

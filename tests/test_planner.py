@@ -523,7 +523,7 @@ def test_tile_of_problems_beyond_small_grids(dt, M, N, K, lay, kw, tile):
 @pytest.mark.parametrize("dt,M,N,K,lay,copies", [(R.E4M3, 2410, 865, 1222, "TN", True), (R.E4M3, 2511, 2241, 536, "TT", True), (R.BF16, 2321, 2172, 1978, "NT", True), (R.F16, 1524, 1901, 861, "NN", True), (R.BF16, 6720, 832, 1337, "NN", True),
                                                  (R.I8, 445, 2933, 150, "NN", False), (R.I8, 464, 2236, 198, "NT", False), (R.F16, 157, 23, 32, "TT", False)])
 def test_rows_off_16_bytes_are_copied_where_k_is_deep_enough(dt, M, N, K, lay, copies):
-    """staged through registers in one launch with few K tiles; without a workspace always"""
+    """staged through registers in one launch with few K tiles (without a workspace always: tests of recorded launches)"""
     es = 1 if dt in (R.I8, R.E4M3) else 2
     name, p = _route(dt, M, N, K, lay)
     sizes = [rows * (-(-cols * es // 16) * 16) for rows, cols in ((K, M) if lay[0] == "T" else (M, K), (N, K) if lay[1] == "T" else (K, N)) if cols * es % 16]

@@ -24,10 +24,15 @@ def test_the_sum_of_any_number_of_slices_is_exact(hip, split):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("columns", [64, 42, 32, 25, 21, 18, 16])
-def test_the_sum_of_split_edge_tiles_is_exact(hip, columns):
-    """two rows of 128x128 edge tiles over K tiles enough for 2 to 8 slices, in place of as many work-groups as there are CUs"""
-    M, N, K = 193, 128 * columns - 5, 128 * 16 * 8
+@pytest.mark.parametrize("M,N,K,tile,slices", [
+    (193, 123, 4608, 128, 2), (193, 123, 6144, 128, 3), (193, 128 * 32 - 5, 16384, 128, 4), (193, 128 * 25 - 5, 16384, 128, 5), (193, 128 * 21 - 5, 16384, 128, 6),
+    (193, 128 * 18 - 5, 16384, 128, 7), (193, 128 * 16 - 5, 16384, 128, 8), (513, 6651, 4608, 192, 2), (513, 6651, 8192, 192, 3), (193, 128 * 64 - 5, 16384, 256, 7),
+    (193, 128 * 42 - 5, 16384, 256, 8)])
+def test_the_sum_of_split_edge_tiles_is_exact(hip, M, N, K, tile, slices):
+    """2 to 8 slices of edge tiles, in place of as many work-groups as there are CUs; B's rows are copied to aligned ones first, the sums lie behind them"""
+    p = hip.plan(hip.make_desc(O.I8, M, N, K, dtype_out=O.I32))
+    copies = -(-K * (-(-N // 16) * 16) // 256) * 256
+    assert p.tile_m == tile and p.workspace_bytes - copies == slices * p.grid_x * p.grid_y * p.tile_m * p.tile_n * 4
     A, B = make_operand(O.I8, M, K, 62, 0), make_operand(O.I8, K, N, 62, 1)
     assert np.array_equal(run_gemm(hip, O.I8, A, B, 0, 0, O.I32, M, N, K), O.gemm_i32(A, B))
 
