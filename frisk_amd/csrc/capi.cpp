@@ -130,7 +130,7 @@ static void wave_partition(int policy, int64_t M, int64_t N, int num_waves, int 
 }
 
 // Kernels that the search over the variants leaves out, and no descriptor can name: the planner goes over to them from the kernel that the search has
-// found (`follow_up` in make_plan).
+// found (`follow_up` and `other_tile`).
 static bool is_follow_up(const KernelEntry* k) {
   if (k->dtype == FRISK_F32) return k->bm == 32 && k->bn == 32 && !k->splitk;
   return (k->bm == 64 && k->bn == 64) || k->bm == 160 || k->bm == 224 || (k->bm == 128 && k->bn == 128 && k->edge && k->stages == 3);
@@ -653,8 +653,9 @@ static Repack repack_of(const frisk_gemm_desc* d, bool a, bool b) {
 static bool same_edge_tile(const KernelEntry* k) { return k->bm == 128 && k->bn == 128 && k->edge && k->stages == 3; }
 
 // The kernel (its index) that runs a problem in place of `k`, which the search has found with `split` slices of K or `slices` of its edge tiles: -1, that
-// one stays.  A CU fetches at most 100 bytes a nanosecond into LDS whatever the tile and however many tiles are under way (41 bytes a cycle; a
-// loop of nothing but transfers), so where every CU has one work-group at most, the time goes with (rows + columns) x K of the tile.
+// one stays.  Where every CU has one work-group at most, the bytes that it fetches, (rows + columns) x K, are a first measure of the time: fp16 tiles of one round reach, in bytes a
+// nanosecond and CU from the last-level cache / from memory, 85 / 55 (64x64 NT), 74 / 46 (NN), 80 / 53 (64x128 NT), 67 / 61 (128x128 in a ring of 3) and 51 / 49 (256x256, bound by its
+// MFMAs).  No more than that: where each rule below ends is the edge of a sweep over drawn problems, timed on both sides, not a consequence of these rates.
 static int follow_up(const std::vector<Variant>& list, const KernelEntry* k, const frisk_gemm_desc* d, bool rows_aligned, int split, int slices, const Repack& packed) {
   const int es = elem_size(k->dtype);
   const bool staged = k->guard && !k->edge;  // through registers
@@ -681,7 +682,7 @@ static int follow_up(const std::vector<Variant>& list, const KernelEntry* k, con
   };
   if (k->dtype == FRISK_F32) {
     // 32x32 tiles, the four waves splitting K, on up to 512 work-groups (two a CU): a 64x64 tile keeps its CU's matrix pipe busy and a quarter of
-    // as many leave most CUs without one.  us, operands in the last-level cache, on 64x64 or 32x128 tiles / so: 128x1280x1024 NN 18.9 / 9.1,
+    // as many leave most CUs without one.  us, operands in the last-level cache and no workspace (with one these are split along K), on 64x64 or 32x128 tiles / so: 128x1280x1024 NN 18.9 / 9.1,
     // 896x256x1792 30.8 / 14.1, 128x384x896 16.3 / 7.6, 256x2048x1408 (512) 24.9 / 17.8; off the tiles 323x130x437 NT 13.8 / 10.0, 8-row problems of 4000 to
     // 9000 columns half the time; but 512x1152x512 (576) 11.2 / 12.4, 1280x640x768 (800) 16.2 / 19.7, and in a second round on fewer than two K
     // tiles of 128 296x856x160 (270) 6.2 / 7.2; whole tiles under A [K][M] 256x256x512 TN 10.5 / 6.0, 512x512x512 TT 11.4 / 6.7, 1024x512x256 7.6 / 6.6
@@ -718,7 +719,8 @@ static int follow_up(const std::vector<Variant>& list, const KernelEntry* k, con
   if (split > 1) return -1;
   // 128x128 tiles with 3 + 3 tiles of LDS in a single round, one on each CU, in place of unsplit 64x128 ones of which some CUs hold two: a third less to transfer.  us
   // on 64x128 / so: fp16 363x8512x2176 NT 25.2 / 20.8, 1206x3072x1280 NN 17.6 / 15.9, bf16 1108x3008x1792 NT 20.2 / 18.1, 5952x640x7296 NN 82.5 / 73.1.  Of 79 drawn 16-bit
-  // problems all are faster, by 18 %, and all of 48 8-bit ones of 2 KiB of K and more, by 20 % (of 37 with less 14 are slower, int8 1856x1152x1024 NT by 17 %)
+  // problems all are faster, by 18 %, and all of 48 8-bit ones of 2 KiB of K and more, by 20 % (of 37 with less 14 are slower, int8 1856x1152x1024 NT by 17 %).  Of 243 more,
+  // from memory, 11 are slower, by 3 to 7 % (bf16 2752x1024x896 NT 11.5 / 12.4)
   if (k->bm == 64 && k->bn == 128 && (es == 2 || k_bytes >= 2048) && tiles_of(64, 128) > 256 && tiles_of(128, 128) <= 256)
     if (const int id = variant(128, 128, 3); id >= 0) return id;
   // 128x128 edge tiles with 3 + 3 tiles of LDS where no CU has two work-groups.  us with 2 + 2 / 3 + 3: fp16 3916x632x2592 NT 32.4 / 24.4, 512x1392x1368 TN

@@ -9,8 +9,8 @@
 // assembly over fixed registers: a step is two lane reads of the program, a jump to its handler and 8 vector instructions in
 // place, the operand picked by the register index mode.  (As a C++ switch the compiler joins the values of all cases after every
 // step by register moves: 327 vector, 300 scalar and 120 branch instructions per group of 8 columns for (x - s * c) * g + b; here
-// 109, 125 and 34.)  That body on 8192 x 8192 f16: 137 us before, 51 now (a plain copy: 41); log2(max(x, c) / (x + c)), bound by
-// the vector pipe in its division, 123 -> 69.5; x + y 80 -> 65; rows off 16-byte boundaries (4095 x 8191) 369 -> 29.
+// 109, 125 and 34.)  That body on 8192 x 8192 f16: 137 us before, 46 to 51 now (a plain copy: 41); log2(max(x, c) / (x + c)), bound by
+// the vector pipe in its division, 123 -> 69.5; x + y 80 -> 58; rows off 16-byte boundaries (4095 x 8191) 369 -> 29.
 // Operands that are the same for every row stay in registers while the lane's columns do, values of one per row stay one
 // register, and what the next groups need from memory is fetched while the current one is evaluated.  All arithmetic is
 // fp32; the result is rounded once to the output type.

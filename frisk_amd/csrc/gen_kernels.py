@@ -91,7 +91,7 @@ def square(bk, atom16=False, skinny_ta=(0,)):
     # 192x256 tiles (A stored [M][K]; 96-row waves), an edge kernel only: where rounds of 256x256 tiles come out uneven
     for tb in (0, 1):
         out.append(edge((0, tb, 192, 256, bk, 2, 2, 2, 0, 0, 1, 3) + ((16,) if atom16 else ())))
-    # ... and 160x256 and 224x256 ones (80- and 112-row waves of 16-row atoms), to which only `follow_up` goes over: more sizes of tile, fewer CUs left idle in
+    # ... and 160x256 and 224x256 ones (80- and 112-row waves of 16-row atoms), to which only `other_tile` in capi.cpp goes over: more sizes of tile, fewer CUs left idle in
     # the last round
     if atom16:
         for tb in (0, 1):

@@ -255,7 +255,8 @@ int frisk_hip_copy_tiles(int src_dtype, const void* src, int64_t src_ld, int dst
  * `dim` (0: over rows, dst has cols entries; 1: over columns, dst has rows entries) with `kind`.  Arithmetic
  * in fp32, result rounded to dtype.  clear = 1: dst := reduction; clear = 0: dst := kind(dst, reduction).
  * min / max ignore NaN operands (maxnum / minnum).  Long reductions are split over work-groups through
- * `workspace` (frisk_hip_reduce_workspace_bytes; 0 for most shapes). */
+ * `workspace` (frisk_hip_reduce_workspace_bytes; 0 for most shapes; asked for by sizes alone, so a launch whose leading
+ * dimension suits it better may leave the workspace unused). */
 size_t frisk_hip_reduce_workspace_bytes(int dtype, int64_t rows, int64_t cols, int dim);
 int frisk_hip_reduce(int dtype, const void* src, int64_t rows, int64_t cols, int64_t ld, int dim, int kind, int clear, void* dst,
                      void* workspace, size_t workspace_bytes, void* stream);
