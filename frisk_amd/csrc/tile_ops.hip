@@ -186,41 +186,51 @@ template <int KIND> __device__ __forceinline__ float wave_reduce(float v) {
   return v;
 }
 
-// along dim 1: work-group (x = row, y = column slice) reduces every gridDim.y-th run of 256 16-byte groups of one row, so that
+// along dim 1: work-group (x = row, y = column slice) reduces every gridDim.y-th run of THREADS 16-byte groups of one row, so that
 // the slices of a row read neighbouring memory at any time.
 // With gridDim.y == 1 the result goes to dst (combined with the old value unless clear), else to partial[y][row].
-template <int DT, int KIND> __global__ void __launch_bounds__(256)
+// A row's last group, where it is not whole, is fetched with the elements before it that fill it up, which are left out: every load is 16 bytes of the row and
+// those of a lane are under way together (element by element behind the others: us so / now, f16 2490 x 2453 6.7 / 4.5, 10069 x 4946 19.7 / 16.0, 2490 x 4453 8.9 / 5.9, f32
+// 5531 x 1315 8.8 / 6.6).  512 lanes from 1025 groups on (f32 4000 x 8192 20.4 / 19.7, f16 4426 x 15161 27.7 / 26.8); views that the last-level cache may hold are read
+// through the caches (2490 x 4453 6.2 past them, 5.9 so; 10069 x 4946 16.0 past them, 16.8).
+template <int DT, int KIND, int THREADS, bool STREAMED> __global__ void __launch_bounds__(THREADS)
 reduce_rows_kernel(const typename Elem<DT>::T* src, int64_t rows, int64_t cols, int64_t ld, int clear, typename Elem<DT>::T* dst, float* partial) {
   typedef typename Elem<DT>::T T;
-  constexpr int G = 16 / sizeof(T);
-  const int64_t gpr = (cols + G - 1) / G;
-  __shared__ float wsum[4];
+  constexpr int G = 16 / sizeof(T), FLIGHT = 4;
+  const int64_t gpr = (cols + G - 1) / G, whole = cols / G, step = (int64_t)gridDim.y * THREADS;
+  const int twice = (int)(gpr * G - cols);
+  __shared__ float wsum[THREADS / 64];
   for (int64_t r = blockIdx.x; r < rows; r += gridDim.x) {
     float acc = Op<KIND>::id();
     const T* row = src + r * ld;
     // four groups of a lane under way together, combined in their order (one after the other 98 x 12807 bf16 took 6.2 us, 8192 x 8192 f16 22.9)
-    const int64_t whole = cols / G, step = (int64_t)gridDim.y * 256;
-    int64_t g = (int64_t)blockIdx.y * 256 + threadIdx.x;
-    for (; g < whole; g += 4 * step) {
-      T in[4][G];
+    for (int64_t g = (int64_t)blockIdx.y * THREADS + threadIdx.x; g < gpr; g += FLIGHT * step) {
+      T in[FLIGHT][G];
 #pragma unroll
-      for (int u = 0; u < 4; ++u)
-        if (g + u * step < whole) *(v4u*)in[u] = load16(row + (g + u * step) * G);
+      for (int u = 0; u < FLIGHT; ++u) {
+        const int64_t at = g + u * step < whole ? (g + u * step) * G : cols - G;
+        if (g + u * step >= gpr) continue;
+        if constexpr (STREAMED) *(v4u*)in[u] = load16(row + at);
+        else *(v4u*)in[u] = *(const v4u_any*)(row + at);
+      }
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        if (g + u * step >= whole) continue;
+      for (int u = 0; u < FLIGHT; ++u) {
+        if (g + u * step < whole) {
 #pragma unroll
-        for (int e = 0; e < G; ++e) acc = Op<KIND>::f(acc, Elem<DT>::load(in[u][e]));
+          for (int e = 0; e < G; ++e) acc = Op<KIND>::f(acc, Elem<DT>::load(in[u][e]));
+        } else if (g + u * step < gpr) {
+#pragma unroll
+          for (int e = 0; e < G; ++e)
+            if (e >= twice) acc = Op<KIND>::f(acc, Elem<DT>::load(in[u][e]));
+        }
       }
     }
-    // the row's last group, if it is not whole, is the last one of its lane (slices are a power of two)
-    if (whole < gpr && (whole & (step - 1)) == (int64_t)blockIdx.y * 256 + threadIdx.x)
-      for (int64_t c = whole * G; c < cols; ++c) acc = Op<KIND>::f(acc, Elem<DT>::load(row[c]));
     acc = wave_reduce<KIND>(acc);
     if ((threadIdx.x & 63) == 0) wsum[threadIdx.x >> 6] = acc;
     __syncthreads();
     if (threadIdx.x == 0) {
       float v = Op<KIND>::f(Op<KIND>::f(wsum[0], wsum[1]), Op<KIND>::f(wsum[2], wsum[3]));
+      if constexpr (THREADS == 512) v = Op<KIND>::f(v, Op<KIND>::f(Op<KIND>::f(wsum[4], wsum[5]), Op<KIND>::f(wsum[6], wsum[7])));
       if (gridDim.y > 1) partial[(int64_t)blockIdx.y * rows + r] = v;
       else dst[r] = Elem<DT>::store(clear ? v : Op<KIND>::f(Elem<DT>::load(dst[r]), v));
     }
@@ -239,15 +249,19 @@ reduce_short_rows_kernel(const typename Elem<DT>::T* src, int64_t rows, int64_t 
   const int64_t blocks = (rows + rows_per_set * SETS - 1) / (rows_per_set * SETS);
   for (int64_t rb = blockIdx.x; rb < blocks; rb += gridDim.x) {
     T in[SETS][NPT][G];
-    bool whole[SETS][NPT];
+    const bool narrow = cols < G;  // rows of less than a group go element by element
 #pragma unroll
     for (int t = 0; t < SETS; ++t) {
       const int64_t r = (rb * SETS + t) * rows_per_set + (threadIdx.x >> lanes_log2);
 #pragma unroll
       for (int q = 0; q < NPT; ++q) {
         const int64_t c0 = (int64_t)(q * lanes + lane) * G;
-        whole[t][q] = r < rows && c0 + G <= cols;
-        if (whole[t][q]) *(v4u*)in[t][q] = load16(src + r * ld + c0);
+        if (r >= rows || c0 >= cols) continue;
+        // (a last group that is not whole with the elements before it that fill it up)
+        if (!narrow) *(v4u*)in[t][q] = load16(src + r * ld + (c0 + G <= cols ? c0 : cols - G));
+        else
+#pragma unroll
+          for (int e = 0; e < G; ++e) in[t][q][e] = src[r * ld + (e < cols ? e : 0)];
       }
     }
 #pragma unroll
@@ -258,11 +272,14 @@ reduce_short_rows_kernel(const typename Elem<DT>::T* src, int64_t rows, int64_t 
 #pragma unroll
       for (int q = 0; q < NPT; ++q) {
         const int64_t c0 = (int64_t)(q * lanes + lane) * G;
-        if (whole[t][q]) {
+        if (live && c0 + G <= cols) {
 #pragma unroll
           for (int e = 0; e < G; ++e) acc = Op<KIND>::f(acc, Elem<DT>::load(in[t][q][e]));
-        } else if (live) {
-          for (int e = 0; e < G && c0 + e < cols; ++e) acc = Op<KIND>::f(acc, Elem<DT>::load(src[r * ld + c0 + e]));
+        } else if (live && c0 < cols) {
+          const int lo = narrow ? 0 : (int)(c0 + G - cols), hi = narrow ? (int)cols : G;
+#pragma unroll
+          for (int e = 0; e < G; ++e)
+            if (e >= lo && e < hi) acc = Op<KIND>::f(acc, Elem<DT>::load(in[t][q][e]));
         }
       }
       for (int off = lanes >> 1; off >= 1; off >>= 1) acc = Op<KIND>::f(acc, __shfl_xor(acc, off, 64));
@@ -496,7 +513,8 @@ template <int DT, int KIND> hipError_t reduce_t(const void* src, int64_t rows, i
   // (without slices the one launch takes every view of its range)
   const bool tall = dim == 0 && split_of(DT, rows, cols, dim) > 1 &&
                     cols_in_one_launch(rows, cols * (int64_t)sizeof(T), slices == 1 || ((uintptr_t)src % 128 == 0 && ld * sizeof(T) % 128 == 0));
-  if (tall) slices = 1;
+  // rows of up to 64 KiB in one launch, however few (us in slices and a second launch / so, f32 394 x 9229 7.4 / 4.8, 64 x 16000 7.8 / 4.6)
+  if (tall || (dim == 1 && gpr <= 4096)) slices = 1;
   if (dim == 1) {
     if (gpr <= 256 && slices == 1) {
       int lanes_log2 = 0;
@@ -507,8 +525,12 @@ template <int DT, int KIND> hipError_t reduce_t(const void* src, int64_t rows, i
       else if (gpr <= 128) hipLaunchKernelGGL((reduce_short_rows_kernel<DT, KIND, 2>), grid, dim3(256), 0, s, (const T*)src, rows, cols, ld, clear, (T*)dst, lanes_log2);
       else hipLaunchKernelGGL((reduce_short_rows_kernel<DT, KIND, 4>), grid, dim3(256), 0, s, (const T*)src, rows, cols, ld, clear, (T*)dst, lanes_log2);
     } else {
-      hipLaunchKernelGGL((reduce_rows_kernel<DT, KIND>), dim3((unsigned)(rows < kMaxGrid ? rows : kMaxGrid), (unsigned)slices), dim3(256), 0, s, (const T*)src, rows, cols,
-                         ld, clear, (T*)dst, partial);
+      const dim3 grid((unsigned)(rows < kMaxGrid ? rows : kMaxGrid), (unsigned)slices);
+      const bool streamed = rows * cols * (int64_t)sizeof(T) > (int64_t)64 << 20;
+      auto launch = [&](auto kernel, int threads) { hipLaunchKernelGGL(kernel, grid, dim3(threads), 0, s, (const T*)src, rows, cols, ld, clear, (T*)dst, partial); };
+      if (gpr > 1024) { if (streamed) launch(reduce_rows_kernel<DT, KIND, 512, true>, 512); else launch(reduce_rows_kernel<DT, KIND, 512, false>, 512); }
+      else if (streamed) launch(reduce_rows_kernel<DT, KIND, 256, true>, 256);
+      else launch(reduce_rows_kernel<DT, KIND, 256, false>, 256);
     }
   } else if (tall) {
     int lanes_log2 = 0;

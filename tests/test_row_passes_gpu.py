@@ -142,3 +142,27 @@ def test_slices_of_unequal_length(hip, dtype, transA, transB):
             r = O.compare(out, np.ascontiguousarray(got), O.gemm_f64(dtype, A, B, transA, transB))
             assert r["nonfinite"] == 0 and r["max_rel"] <= TOL[dtype] and r["fro_rel"] <= TOL[dtype], (M, N, K, r)
     assert seen
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt,tdt", [(O.F32, "float32"), (O.F16, "float16"), (O.BF16, "bfloat16")])
+def test_the_last_group_of_a_row_reduced(hip, dt, tdt):
+    """rows shared by lanes of a wave, of 256 and 512 lanes and of several work-groups, with a last group of 1 to all but one elements; what lies between the rows is no
+    number.  Whole numbers whose sums every type holds: the same bits in any order."""
+    import torch
+    tdt = getattr(torch, tdt)
+    G = 16 // torch.empty(0, dtype=tdt).element_size()
+    g = torch.Generator(device="cuda").manual_seed(7)
+    stream = torch.cuda.current_stream().cuda_stream
+    for cols in (1, G - 1, G, G + 1, 63 * G + 1, 64 * G - 1, 128 * G + 1, 256 * G - 1, 256 * G + 1, 1024 * G - 1, 1024 * G + 3, 2049 * G, 4096 * G - 1, 4096 * G + 1, 9000 * G + 5):
+        for rows in (1, 3, 700 if cols < 300 * G else 5) + ((16600,) if cols in (256 * G + 1, 1024 * G + 3) and G == 4 else ()):
+            x = torch.full((rows, cols + 1), float("nan"), device="cuda", dtype=tdt)
+            x[:, :cols] = (torch.rand(rows, cols, device="cuda", generator=g) < 0.06).to(tdt) * (2 * torch.randint(0, 2, (rows, cols), device="cuda", generator=g) - 1).to(tdt)
+            need = hip.reduce_workspace_bytes(dt, rows, cols, 1)
+            ws = torch.full((max(need, 4),), 0xFF, dtype=torch.uint8, device="cuda")
+            for kind, clear in (("add", True), ("add", False), ("max", True)):
+                d = torch.full((rows + 1,), 7.0, device="cuda", dtype=tdt)
+                hip.reduce(dt, x.data_ptr(), rows, cols, cols + 1, 1, kind, clear, d.data_ptr(), ws.data_ptr() if need else None, need, stream)
+                torch.cuda.synchronize()
+                want = x[:, :cols].float().sum(1) + (0 if clear else 7.0) if kind == "add" else x[:, :cols].float().amax(1)
+                assert torch.equal(d[:rows].float(), want) and float(d[rows]) == 7.0, (rows, cols, kind, clear)
