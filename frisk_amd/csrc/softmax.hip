@@ -2,11 +2,10 @@
 // @online_softmax (tmp/ir.mlir:21-66): per row, chunks of 1024 go through frisk.copy, frisk.reduce max, a frisk.block
 // of exp2(x * cst - max * cst), frisk.reduce sum and a running log-sum (:33-57), then a second sweep writes
 // exp2(x * cst - lse) (:58-68).  Here rows of up to 256 groups of 16 bytes (2048 f16) are shared by 1 to 64 lanes of one
-// wave and combined by shuffles; longer rows get a work-group of 256 lanes each.  Rows of up to 64 elements per lane are
+// wave and combined by shuffles; longer rows get a work-group of 256 or 512 lanes each.  Rows of up to 4096 groups (32768 f16, 16384 f32) are
 // read once and held in registers (maximum, exponentials, sum, scaling: one read and one write of HBM per element);
 // longer rows take the sketch's two sweeps with a running maximum and sum per lane, the second sweep re-reading x.
-// A lane moves 16 bytes at a time, wherever the rows start; only a row's last group, when it is not whole, is walked element by
-// element (4095 x 8191 f16: 55.5 us while rows off 16-byte boundaries went element by element, 31.5 now).
+// A lane moves 16 bytes at a time, wherever the rows start.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include "tile_ops.h"
@@ -39,14 +38,14 @@ template <int DT, bool STREAMED> __device__ __forceinline__ void load_group(cons
     for (int e = 0; e < G; ++e) v[e] = e < left ? SElem<DT>::load(x[g * G + e]) * c : -INFINITY;
   }
 }
-template <int DT, bool WHOLE = false> __device__ __forceinline__ void store_group(typename SElem<DT>::T* y, int64_t g, int64_t cols, const float (&v)[16 / sizeof(typename SElem<DT>::T)]) {
+template <int DT> __device__ __forceinline__ void store_group(typename SElem<DT>::T* y, int64_t g, int64_t cols, const float (&v)[16 / sizeof(typename SElem<DT>::T)]) {
   typedef typename SElem<DT>::T T;
   constexpr int G = 16 / (int)sizeof(T);
   const int64_t left = cols - g * G;
   T out[G];
 #pragma unroll
   for (int e = 0; e < G; ++e) out[e] = SElem<DT>::store(v[e]);
-  if (WHOLE || left >= G) __builtin_nontemporal_store(*(const v4u*)out, (v4u_any*)(y + g * G));
+  if (left >= G) __builtin_nontemporal_store(*(const v4u*)out, (v4u_any*)(y + g * G));
   else {
 #pragma unroll
     for (int e = 0; e < G; ++e)
@@ -90,9 +89,89 @@ __device__ __forceinline__ MaxSum block_merge(MaxSum v, float* lds) {
   return r;
 }
 
-// Longer rows, a work-group each.  NPT > 0: the row fits in NPT 16-byte groups per lane and is kept in registers.  NPT == 0: two sweeps.
-// WHOLE: the row is a whole number of groups (the code for a last one that is not costs 8 % where no row needs it).
-template <int DT, int NPT, bool WHOLE>
+// the maximum (SUM false) or the sum of a value of every lane of the work-group; `lds`: a float per wave that nothing else has touched since the last barrier
+template <bool SUM, int THREADS> __device__ __forceinline__ float block_all(float v, float* lds) {
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) {
+    const float o = __shfl_xor(v, off);
+    v = SUM ? v + o : fmaxf(v, o);
+  }
+  if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = v;
+  __syncthreads();
+  float r = lds[0];
+#pragma unroll
+  for (int w = 1; w < THREADS / 64; ++w) r = SUM ? r + lds[w] : fmaxf(r, lds[w]);
+  return r;
+}
+
+// Rows of 257 to 4096 groups, a work-group each, NPT groups a lane in registers.  A row's last group, where it is not whole, is read and written together with the
+// elements before it that fill it up (which enter the sum as their own lane's): every access is 16 bytes of the row and all loads of a row are under way
+// together.  Fetched element by element behind the others, that group held up every row by a memory latency: us before / now, f16 10069 x 4946 49.5 / 33.7,
+// 2490 x 2453 11.8 / 6.9, 870 x 16370 20.0 / 10.4 (with 512 lanes: 12.5 with 256), f32 5531 x 1315 17.6 / 10.6, 394 x 9229 (two launches before) 11.9 / 6.9;
+// rows that are whole groups gain by the shorter reductions, f16 8192 x 8192 47.3 / 43.5, which a plain copy takes 39 for.
+// STREAMED, for views that the last-level cache does not hold beside their result: the loads pass the caches by (8192 x 8192 f16 43.5, 45.0 without; but 870 x 16370
+// 10.4 without, 11.9 with), and where rows start off 16-byte boundaries the groups start at the first boundary, what lies before it being a group that overlaps
+// like the last one: stores that cross lines half way cost memory traffic (4426 x 15161 f16 54.9 at the rows' starts, 47.5 so; out of the cache 7.1 either way, 545 x 12163).
+template <int DT, int NPT, int THREADS, bool STREAMED>
+__global__ void __launch_bounds__(THREADS) softmax_held_rows_kernel(const typename SElem<DT>::T* src, int64_t sld, typename SElem<DT>::T* dst, int64_t dld, int64_t rows,
+                                                                    int cols, float c, float* lse) {
+  typedef typename SElem<DT>::T T;
+  constexpr int G = 16 / (int)sizeof(T);
+  __shared__ float lds[2][THREADS / 64];  // one row's sum is read before the next row's maximum has passed its barrier
+  for (int64_t r = blockIdx.x; r < rows; r += gridDim.x) {
+    const T* x = src + r * sld;
+    T* y = dst + r * dld;
+    // groups 0 .. full - 1 from element `head` on, then the one that ends with the row, then the one it starts with
+    const int head = STREAMED ? (int)((0 - (uintptr_t)y) & 15) / (int)sizeof(T) : 0;
+    const int full = (cols - head) / G, body = head + full * G, tail = cols - body, groups = full + (tail > 0) + (head > 0);
+    T in[NPT][G];
+    int at[NPT];
+#pragma unroll
+    for (int q = 0; q < NPT; ++q) {
+      const int g = q * THREADS + (int)threadIdx.x;
+      at[q] = g < full ? head + g * G : (tail > 0 && g == full ? cols - G : 0);
+      if (g < groups) {
+        if constexpr (STREAMED) *(v4u*)in[q] = __builtin_nontemporal_load((const v4u_any*)(x + at[q]));
+        else *(v4u*)in[q] = *(const v4u_any*)(x + at[q]);
+      }
+    }
+    float v[NPT][G], mx = -INFINITY;
+#pragma unroll
+    for (int q = 0; q < NPT; ++q)
+#pragma unroll
+      for (int e = 0; e < G; ++e) {
+        v[q][e] = q * THREADS + (int)threadIdx.x < groups ? SElem<DT>::load(in[q][e]) * c : -INFINITY;
+        mx = fmaxf(mx, v[q][e]);
+      }
+    const float top = block_all<false, THREADS>(mx, lds[0]);
+    float sum = 0.f;
+#pragma unroll
+    for (int q = 0; q < NPT; ++q) {
+      const int g = q * THREADS + (int)threadIdx.x;
+      // which elements of the group are its own
+      const bool last = tail > 0 && g == full;
+      const int lo = last ? G - tail : 0, hi = g < full || last ? G : head;
+#pragma unroll
+      for (int e = 0; e < G; ++e) {
+        v[q][e] = __builtin_amdgcn_exp2f(v[q][e] - top);
+        sum += g < groups && e >= lo && e < hi ? v[q][e] : 0.f;
+      }
+    }
+    const float all = block_all<true, THREADS>(sum, lds[1]);
+    const float inv = 1.f / all;
+#pragma unroll
+    for (int q = 0; q < NPT; ++q) {
+      T out[G];
+#pragma unroll
+      for (int e = 0; e < G; ++e) out[e] = SElem<DT>::store(v[q][e] * inv);
+      if (q * THREADS + (int)threadIdx.x < groups) __builtin_nontemporal_store(*(const v4u*)out, (v4u_any*)(y + at[q]));
+    }
+    if (lse && threadIdx.x == 0) lse[r] = top + __builtin_amdgcn_logf(all);
+  }
+}
+
+// Rows beyond that, a work-group each: two sweeps.
+template <int DT>
 __global__ void __launch_bounds__(256) softmax_rows_kernel(const typename SElem<DT>::T* src, int64_t sld, typename SElem<DT>::T* dst, int64_t dld, int64_t rows,
                                                            int64_t cols, float c, float* lse) {
   typedef typename SElem<DT>::T T;
@@ -102,66 +181,23 @@ __global__ void __launch_bounds__(256) softmax_rows_kernel(const typename SElem<
   for (int64_t r = blockIdx.x; r < rows; r += gridDim.x) {
     const T* x = src + r * sld;
     T* y = dst + r * dld;
-    if constexpr (NPT > 0) {
-      float v[NPT][G];
-      // every whole group is requested before the first is used; the row's last group, if it is not whole, comes behind them
-      T in[NPT][G];
+    MaxSum acc = {-INFINITY, 0.f};
+    for (int64_t g = threadIdx.x; g < groups; g += 256) {
+      float v[G];
+      load_group<DT, false>(x, g, cols, c, v);
 #pragma unroll
-      for (int q = 0; q < NPT; ++q) {
-        const int64_t g = (int64_t)q * 256 + threadIdx.x;
-        if (g * G + G <= cols) *(v4u*)in[q] = __builtin_nontemporal_load((const v4u_any*)(x + g * G));
-      }
-      float mx = -INFINITY;
-#pragma unroll
-      for (int q = 0; q < NPT; ++q) {
-        const int64_t g = (int64_t)q * 256 + threadIdx.x;
-#pragma unroll
-        for (int e = 0; e < G; ++e) v[q][e] = -INFINITY;
-        if (g * G + G <= cols) {
-#pragma unroll
-          for (int e = 0; e < G; ++e) v[q][e] = SElem<DT>::load(in[q][e]) * c;
-        } else if (!WHOLE && g < groups) load_group<DT, true>(x, g, cols, c, v[q]);
-#pragma unroll
-        for (int e = 0; e < G; ++e) mx = fmaxf(mx, v[q][e]);
-      }
-      const MaxSum top = block_merge(MaxSum{mx, 1.f}, lds);  // only the maximum is used here
-      float sum = 0.f;
-#pragma unroll
-      for (int q = 0; q < NPT; ++q)
-#pragma unroll
-        for (int e = 0; e < G; ++e) {
-          v[q][e] = __builtin_amdgcn_exp2f(v[q][e] - top.m);
-          sum += v[q][e];
-        }
-      const MaxSum all = block_merge(MaxSum{0.f, sum}, lds);  // equal maxima: the sums add
-      const float inv = 1.f / all.l;
-#pragma unroll
-      for (int q = 0; q < NPT; ++q) {
-        const int64_t g = (int64_t)q * 256 + threadIdx.x;
-#pragma unroll
-        for (int e = 0; e < G; ++e) v[q][e] *= inv;
-        if (g < groups) store_group<DT, WHOLE>(y, g, cols, v[q]);
-      }
-      if (lse && threadIdx.x == 0) lse[r] = top.m + __builtin_amdgcn_logf(all.l);
-    } else {
-      MaxSum acc = {-INFINITY, 0.f};
-      for (int64_t g = threadIdx.x; g < groups; g += 256) {
-        float v[G];
-        load_group<DT, false>(x, g, cols, c, v);
-#pragma unroll
-        for (int e = 0; e < G; ++e) acc.add(v[e]);
-      }
-      const MaxSum all = block_merge(acc, lds);
-      const float ref = all.m + __builtin_amdgcn_logf(all.l);  // log2 of the denominator
-      for (int64_t g = threadIdx.x; g < groups; g += 256) {
-        float v[G];
-        load_group<DT, false>(x, g, cols, c, v);
-#pragma unroll
-        for (int e = 0; e < G; ++e) v[e] = __builtin_amdgcn_exp2f(v[e] - ref);
-        store_group<DT>(y, g, cols, v);
-      }
-      if (lse && threadIdx.x == 0) lse[r] = ref;
+      for (int e = 0; e < G; ++e) acc.add(v[e]);
     }
+    const MaxSum all = block_merge(acc, lds);
+    const float ref = all.m + __builtin_amdgcn_logf(all.l);  // log2 of the denominator
+    for (int64_t g = threadIdx.x; g < groups; g += 256) {
+      float v[G];
+      load_group<DT, false>(x, g, cols, c, v);
+#pragma unroll
+      for (int e = 0; e < G; ++e) v[e] = __builtin_amdgcn_exp2f(v[e] - ref);
+      store_group<DT>(y, g, cols, v);
+    }
+    if (lse && threadIdx.x == 0) lse[r] = ref;
   }
 }
 
@@ -180,25 +216,34 @@ __global__ void __launch_bounds__(256) softmax_short_rows_kernel(const typename 
     const T* x = src + r * sld;
     T* y = dst + r * dld;
     float v[NPT][G];
-    bool whole[NPT];
     T in[NPT][G];
+    // a last group that is not whole is read and written with the elements before it, `twice` of them, which are another lane's; a row of less
+    // than a group goes element by element
+    const bool narrow = cols < G;
+    int64_t at[NPT];
+    int twice[NPT];
+    bool inside[NPT];
 #pragma unroll
     for (int q = 0; q < NPT; ++q) {
       const int64_t c0 = (int64_t)(q * lanes + lane) * G;
-      whole[q] = live && c0 + G <= cols;
-      if (whole[q]) *(v4u*)in[q] = __builtin_nontemporal_load((const v4u_any*)(x + c0));
+      inside[q] = live && c0 < cols;
+      twice[q] = !narrow && c0 + G > cols ? (int)(c0 + G - cols) : 0;
+      at[q] = c0 - twice[q];
+      if (inside[q]) {
+        if (!narrow) *(v4u*)in[q] = __builtin_nontemporal_load((const v4u_any*)(x + at[q]));
+        else
+#pragma unroll
+          for (int e = 0; e < G; ++e) in[q][e] = x[e < cols ? e : 0];
+      }
     }
     float mx = -INFINITY;
 #pragma unroll
-    for (int q = 0; q < NPT; ++q) {
-      const int64_t c0 = (int64_t)(q * lanes + lane) * G;
+    for (int q = 0; q < NPT; ++q)
 #pragma unroll
       for (int e = 0; e < G; ++e) {
-        if (whole[q]) v[q][e] = SElem<DT>::load(in[q][e]) * c;
-        else v[q][e] = live && c0 + e < cols ? SElem<DT>::load(x[c0 + e]) * c : -INFINITY;
+        v[q][e] = inside[q] && (!narrow || e < cols) ? SElem<DT>::load(in[q][e]) * c : -INFINITY;
         mx = fmaxf(mx, v[q][e]);
       }
-    }
     for (int off = lanes >> 1; off >= 1; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
     float sum = 0.f;
 #pragma unroll
@@ -206,23 +251,21 @@ __global__ void __launch_bounds__(256) softmax_short_rows_kernel(const typename 
 #pragma unroll
       for (int e = 0; e < G; ++e) {
         v[q][e] = __builtin_amdgcn_exp2f(v[q][e] - mx);
-        sum += v[q][e];
+        sum += e >= twice[q] ? v[q][e] : 0.f;
       }
     for (int off = lanes >> 1; off >= 1; off >>= 1) sum += __shfl_xor(sum, off, 64);
     const float inv = 1.f / sum;
 #pragma unroll
     for (int q = 0; q < NPT; ++q) {
-      const int64_t c0 = (int64_t)(q * lanes + lane) * G;
-      if (whole[q]) {
-        T out[G];
+      if (!inside[q]) continue;
+      T out[G];
 #pragma unroll
-        for (int e = 0; e < G; ++e) out[e] = SElem<DT>::store(v[q][e] * inv);
-        __builtin_nontemporal_store(*(const v4u*)out, (v4u_any*)(y + c0));
-      } else if (live) {
+      for (int e = 0; e < G; ++e) out[e] = SElem<DT>::store(v[q][e] * inv);
+      if (!narrow) __builtin_nontemporal_store(*(const v4u*)out, (v4u_any*)(y + at[q]));
+      else
 #pragma unroll
         for (int e = 0; e < G; ++e)
-          if (c0 + e < cols) y[c0 + e] = SElem<DT>::store(v[q][e] * inv);
-      }
+          if (e < cols) y[e] = out[e];
     }
     if (lse && live && lane == 0) lse[r] = mx + __builtin_amdgcn_logf(sum);
   }
@@ -278,16 +321,20 @@ __global__ void __launch_bounds__(256) softmax_split_write_kernel(const typename
   if (lse && blockIdx.y == 0 && threadIdx.x == 0) lse[blockIdx.x] = ref;
 }
 
+// groups of a row that a work-group holds, and bytes of a view from which on its rows stream past the caches (with the result they are most of the 256 MiB of
+// the last-level cache)
+constexpr int64_t kHeldGroups = 4096, kStreamedBytes = (int64_t)112 << 20;
+
 template <int DT> hipError_t launch_typed(const void* src, int64_t sld, void* dst, int64_t dld, int64_t rows, int64_t cols, float c, float* lse, float* partial,
                                           int slices, hipStream_t s) {
   typedef typename SElem<DT>::T T;
   constexpr int G = 16 / (int)sizeof(T);
   const unsigned grid = (unsigned)(rows < 256 * 64 ? rows : 256 * 64);
-  const int64_t per_pass = 256 * (int64_t)G;
   const T* x = (const T*)src;
   T* y = (T*)dst;
   const int64_t groups = (cols + G - 1) / G;
-  if (slices > 1) {
+  // (rows that a work-group can hold stay whole, in one launch, however few they are: f32 64 x 16000 10.6 us in slices, 5.5 whole)
+  if (slices > 1 && groups > kHeldGroups) {
     const dim3 sgrid((unsigned)rows, (unsigned)slices);
     hipLaunchKernelGGL((softmax_split_stats_kernel<DT>), sgrid, dim3(256), 0, s, x, sld, cols, c, partial);
     hipLaunchKernelGGL((softmax_split_write_kernel<DT>), sgrid, dim3(256), 0, s, x, sld, y, dld, cols, c, lse, (const float*)partial);
@@ -303,21 +350,29 @@ template <int DT> hipError_t launch_typed(const void* src, int64_t sld, void* ds
     else hipLaunchKernelGGL((softmax_short_rows_kernel<DT, 4>), sgrid, dim3(256), 0, s, x, sld, y, dld, rows, cols, c, lse, lanes_log2);
     return hipGetLastError();
   }
-#define FRISK_SOFTMAX_ROWS(NPT)                                                                                                                         \
-  if (cols % G == 0) hipLaunchKernelGGL((softmax_rows_kernel<DT, NPT, true>), dim3(grid), dim3(256), 0, s, x, sld, y, dld, rows, cols, c, lse);           \
-  else hipLaunchKernelGGL((softmax_rows_kernel<DT, NPT, false>), dim3(grid), dim3(256), 0, s, x, sld, y, dld, rows, cols, c, lse);
-  if (cols <= 2 * per_pass) { FRISK_SOFTMAX_ROWS(2) }
-  else if (cols <= 4 * per_pass) { FRISK_SOFTMAX_ROWS(4) }
-  else if (cols <= 8 * per_pass) { FRISK_SOFTMAX_ROWS(8) }
-  else hipLaunchKernelGGL((softmax_rows_kernel<DT, 0, false>), dim3(grid), dim3(256), 0, s, x, sld, y, dld, rows, cols, c, lse);
-#undef FRISK_SOFTMAX_ROWS
+  if (groups <= kHeldGroups) {
+    const bool streamed = rows * cols * (int64_t)sizeof(T) > kStreamedBytes;
+    const int64_t most = groups + (streamed && (((uintptr_t)y | dld * sizeof(T)) & 15) ? 1 : 0);  // a row that starts off a boundary may have a group more
+    auto launch = [&](auto kernel, int threads) { hipLaunchKernelGGL(kernel, dim3(grid), dim3(threads), 0, s, x, sld, y, dld, rows, (int)cols, c, lse); };
+#define FRISK_SOFTMAX_HELD(NPT, THREADS) \
+  if (most <= NPT * THREADS) { if (streamed) launch(softmax_held_rows_kernel<DT, NPT, THREADS, true>, THREADS); else launch(softmax_held_rows_kernel<DT, NPT, THREADS, false>, THREADS); }
+    FRISK_SOFTMAX_HELD(2, 256)
+    else FRISK_SOFTMAX_HELD(3, 256)
+    else FRISK_SOFTMAX_HELD(2, 512)
+    else FRISK_SOFTMAX_HELD(3, 512)
+    else FRISK_SOFTMAX_HELD(4, 512)
+    else FRISK_SOFTMAX_HELD(6, 512)
+    else FRISK_SOFTMAX_HELD(9, 512)
+#undef FRISK_SOFTMAX_HELD
+  } else hipLaunchKernelGGL((softmax_rows_kernel<DT>), dim3(grid), dim3(256), 0, s, x, sld, y, dld, rows, cols, c, lse);
   return hipGetLastError();
 }
 
 }  // namespace
 
 int softmax_slices(int dtype, int64_t rows, int64_t cols) {
-  // Fewer than 1024 rows of at least 32 KiB: split each so that about 1024 work-groups exist, each with at least 16 KiB.
+  // Fewer than 1024 rows of at least 32 KiB: split each so that about 1024 work-groups exist, each with at least 16 KiB (the rows among them that a
+  // work-group can hold are not, and leave their workspace unused).
   const int64_t row_bytes = cols * (dtype == FRISK_F32 ? 4 : 2);
   int slices = 1;
   while (rows * slices < 1024 && row_bytes / (slices * 2) >= 16384 && slices < 256) slices *= 2;

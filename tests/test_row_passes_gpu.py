@@ -166,3 +166,34 @@ def test_the_last_group_of_a_row_reduced(hip, dt, tdt):
                 torch.cuda.synchronize()
                 want = x[:, :cols].float().sum(1) + (0 if clear else 7.0) if kind == "add" else x[:, :cols].float().amax(1)
                 assert torch.equal(d[:rows].float(), want) and float(d[rows]) == 7.0, (rows, cols, kind, clear)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt,tdt,tol", [(O.F32, "float32", 2e-5), (O.F16, "float16", 2e-3), (O.BF16, "bfloat16", 8e-3)])
+def test_softmax_of_rows_held_in_registers(hip, dt, tdt, tol):
+    """rows at the edges of what a number of groups per lane holds, starting on any element, in matrices that the caches are read through and past (from 112 MiB on, where the
+    first group is a part too); what lies between the rows is no number and stays as it is.  Bar: that of the other softmax tests."""
+    import torch
+    tdt = getattr(torch, tdt)
+    es = torch.empty(0, dtype=tdt).element_size()
+    G = 16 // es
+    g = torch.Generator(device="cuda").manual_seed(8)
+    stream = torch.cuda.current_stream().cuda_stream
+    edges = [G * k + r for k in (256, 512, 768, 1024, 1536, 2048, 3072, 4096) for r in (-1, 0, 1)]
+    many = [(-(-(112 << 20) // (cols * es)) + 1, cols) for cols in (256 * G + 1, 512 * G, 512 * G - 1, 4096 * G - 1, 4096 * G)]
+    for rows, cols in [(3, c) for c in edges + [1, G - 1, G + 1, 64 * G + 3, 129 * G - 1]] + many:
+        for ld, shift in ((cols + 1, 0), (cols + 3, 1), (-(-cols // G) * G + G, G - 1)) if rows == 3 else ((cols + 1, 1),):
+            base = torch.full((shift + rows * ld,), float("nan"), device="cuda", dtype=tdt)
+            x = base[shift:].view(rows, ld)
+            x[:, :cols] = (torch.randn(rows, cols, device="cuda", generator=g) * 3).to(tdt)
+            out = torch.full_like(base, 5.0)
+            y, lse = out[shift:].view(rows, ld), torch.full((rows,), float("nan"), device="cuda")
+            hip.softmax(dt, x.data_ptr(), ld, y.data_ptr(), ld, rows, cols, 1.25, lse.data_ptr(), stream)
+            torch.cuda.synchronize()
+            z = x[:, :cols].double() * (1.25 * 0.6931471805599453)
+            want, want_lse = torch.softmax(z, 1), torch.logsumexp(z, 1) / 0.6931471805599453
+            scale = torch.maximum(want, want.square().mean().sqrt())
+            assert bool(((y[:, :cols].double() - want).abs() <= tol * scale + (2.0 ** -25 if dt == O.F16 else 0)).all()), (rows, cols, ld, shift)
+            assert float((lse.double() - want_lse).abs().max()) <= 1e-4 * max(1.0, float(want_lse.abs().max())), (rows, cols, ld, shift)
+            assert bool((y[:, cols:] == 5.0).all()) and bool((out[:shift] == 5.0).all()), (rows, cols, ld, shift)
+            del z, want, scale
