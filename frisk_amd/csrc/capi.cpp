@@ -1123,7 +1123,8 @@ const char* frisk_hip_last_error(void) { return g_last_error.c_str(); }
 int frisk_hip_init(void) {
   if (!device_ok()) return fail(FRISK_ERR_DEVICE, "no gfx950 device is current");
   for (const KernelEntry* k : kernels())
-    if (hipError_t e = k->prepare(); e != hipSuccess) return fail(FRISK_ERR_DEVICE, "preparing %s failed: %s", k->name, hipGetErrorString(e));
+    for (auto prepare : {k->prepare, k->prepare_old_c})
+      if (hipError_t e = prepare ? prepare() : hipSuccess; e != hipSuccess) return fail(FRISK_ERR_DEVICE, "preparing %s failed: %s", k->name, hipGetErrorString(e));
   if (hipError_t e = prepare_attention(); e != hipSuccess) return fail(FRISK_ERR_DEVICE, "preparing the attention kernels failed: %s", hipGetErrorString(e));
   void* ws = nullptr;
   if (hipError_t e = scratch_of_current_device(&ws); e != hipSuccess) return fail(FRISK_ERR_DEVICE, "resolving the static workspace failed: %s", hipGetErrorString(e));
@@ -1205,7 +1206,8 @@ int frisk_hip_gemm(const frisk_gemm_desc* desc, const void* A, const void* B, vo
     e = launch_repack(r, (hipStream_t)stream);
     if (e != hipSuccess) return fail(FRISK_ERR_DEVICE, "launch of the copy to aligned rows failed: %s", hipGetErrorString(e));
   }
-  e = k->launch(p, (hipStream_t)stream);
+  const bool old_c = k->launch_old_c && p.accumulate && p.dtype_out == FRISK_F32 && p.epilogue == FRISK_EPI_NONE;
+  e = (old_c ? k->launch_old_c : k->launch)(p, (hipStream_t)stream);
   if (e != hipSuccess) return fail(FRISK_ERR_DEVICE, "launch of %s failed: %s", k->name, hipGetErrorString(e));
   if (p.split_k > 1) {
     e = launch_splitk_reduce(p, desc->dtype_acc == FRISK_I32, (hipStream_t)stream);

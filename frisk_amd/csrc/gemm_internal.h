@@ -66,6 +66,9 @@ struct KernelEntry {
   int min_k_tiles;  // fewest K tiles the kernel's loop is written for
   hipError_t (*launch)(const GemmParams&, hipStream_t);
   hipError_t (*prepare)();  // one-time, non-stream set-up of the kernel function (dynamic LDS limit)
+  // the same for a kernel of the same tile that accumulates into a float32 C without scales, in place of `launch` there (nullptr: none)
+  hipError_t (*launch_old_c)(const GemmParams&, hipStream_t) = nullptr;
+  hipError_t (*prepare_old_c)() = nullptr;
 };
 
 // sums the split-K slices and applies the epilogue (splitk_reduce.hip)

@@ -150,6 +150,13 @@ def cfg_of(enum, v):
     ta, tb, bm, bn, bk, wm, wn, st, gd, sk, wk, sb, at, eg = full(v)
     return f"GemmCfg<{enum}, {ta}, {tb}, {bm}, {bn}, {bk}, {wm}, {wn}, {st}, {'true' if gd else 'false'}, {'true' if sk else 'false'}, {wk}, {sb}" + (f", {at}, true>" if eg else (f", {at}>" if at != 32 else ">"))
 
+def old_c_cfg_of(enum, v):
+    """the kernel that accumulates into a float32 C in place of variant v's, if it has one: 128x128 tiles under A stored [K][M] and B [K][N], the layouts of a weight gradient"""
+    ta, tb, bm, bn, bk, wm, wn, st, gd, sk, wk, sb, at, eg = full(v)
+    if enum not in ("FRISK_F16", "FRISK_BF16") or (ta, tb, bm, bn, gd, sk) != (1, 0, 128, 128, 0, 0):
+        return None
+    return f"GemmCfg<{enum}, 1, 0, 128, 128, {bk}, {wm}, {wn}, {st}, false, false, 1, {sb}, 32, {'true' if eg else 'false'}, true>"
+
 HERE = os.path.dirname(os.path.abspath(__file__))
 # A type's variants go into a few translation units of about equal size (kernels_<type>.hip, kernels_<type>_2.hip, ...), each with a
 # table of its own: the units compile in parallel, and the longest of them sets the time of a build.  The planner walks the
@@ -165,11 +172,14 @@ for tag, (enum, suffix, variants) in VARIANTS.items():
                  '#include "gemm_kernel.hip.inc"', "namespace frisk {"]
         for v in chunk:
             lines.append(f"template __global__ void gemm_kernel<{cfg_of(enum, v)}>(GemmParams);")
+            if old_c_cfg_of(enum, v):
+                lines.append(f"template __global__ void gemm_kernel<{old_c_cfg_of(enum, v)}>(GemmParams);")
         lines.append("#ifndef __HIP_DEVICE_COMPILE__")
         lines.append(f"const KernelEntry kKernels{suffix}{ext}[] = {{")
         for v in chunk:
             ta, tb, bm, bn, bk, wm, wn, st, gd, sk, wk, sb, at, eg = full(v)
             cfg = cfg_of(enum, v)
+            old = f", &launch_gemm<{old_c_cfg_of(enum, v)}>, &prepare_gemm<{old_c_cfg_of(enum, v)}>" if old_c_cfg_of(enum, v) else ""
             waves = f"w{wm}x{wn}" + (f"x{wk}" if wk > 1 else "")
             # An edge kernel also takes a K that is no multiple of the K tile and a C of any alignment.  The table names it once per use:
             # `_edge` (only M or N off the tile), `_guard_chunks` (K off the K tile too, everything on 16-byte boundaries and K a whole number of
@@ -177,7 +187,7 @@ for tag, (enum, suffix, variants) in VARIANTS.items():
             for gd, eg, what in (((0, 1, "_edge"), (1, 1, "_guard_chunks"), (2, 1, "_guard")) if eg and not sk else ((gd, eg, "_guard" if gd else "_splitk" * bool(sk) + "_edge" * bool(eg)),)):
                 stages = f"s{st}" + (f"x{sb}" if sb != st or gd == 2 else "")
                 name = f"{tag}_{'t' if ta else 'n'}{'t' if tb else 'n'}_{bm}x{bn}x{bk}_{waves}_{stages}" + (f"_a{at}" if at != 32 else "") + what
-                lines.append(f'    {{"{name}", {enum}, {ta}, {tb}, {bm}, {bn}, {bk}, {wm}, {wn}, {st}, {sb}, {wk}, {gd}, {sk}, {at}, {eg}, {cfg}::LDS_BYTES, {cfg}::MIN_K_TILES, &launch_gemm<{cfg}>, &prepare_gemm<{cfg}>}},')
+                lines.append(f'    {{"{name}", {enum}, {ta}, {tb}, {bm}, {bn}, {bk}, {wm}, {wn}, {st}, {sb}, {wk}, {gd}, {sk}, {at}, {eg}, {cfg}::LDS_BYTES, {cfg}::MIN_K_TILES, &launch_gemm<{cfg}>, &prepare_gemm<{cfg}>{old}}},')
         lines.append("};")
         lines.append(f"const int kNumKernels{suffix}{ext} = sizeof(kKernels{suffix}{ext}) / sizeof(kKernels{suffix}{ext}[0]);")
         lines.append("#endif")

@@ -50,3 +50,22 @@ def test_whole_tiles_of_an_edge_kernel_beside_the_others(hip, dtype, transA, tra
                 if dtype != O.F32 and M > 256:
                     for tile in (128, 256):
                         check(hip, dtype, transA, transB, M, N, K, out, epilogue, False, N + 3, 1, tile=(tile, tile, 0))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [O.F16, O.BF16])
+@pytest.mark.parametrize("stages", [2, 3])
+def test_old_values_fetched_beside_the_k_tiles(hip, dtype, stages):
+    """A weight gradient on 128x128 tiles into float32: from one K tile, whose old values come at once, over four and two pieces a K tile to loops that go on behind them, whole and
+    with a partial last tile; wave tiles inside C and beyond it"""
+    for tiles in (1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 12, 19):
+        for K in (tiles * 64, tiles * 64 - 8, tiles * 64 - 3):
+            if K % 64 == 0:
+                check(hip, dtype, 1, 0, 256, 128, K, O.F32, hip.EPI_NONE, False, 128, 0, tile=(128, 128, 0), stages=stages)
+            if stages == 2:
+                check(hip, dtype, 1, 0, 200, 320, K, O.F32, hip.EPI_NONE, False, 323, 1, tile=(128, 128, 0), stages=2)
+            else:  # (the planner's own choice: no descriptor names the ring of 3 off the tile)
+                check(hip, dtype, 1, 0, 2600, 1027, K, O.F32, hip.EPI_NONE, False, 1030, 1)
+    p = hip.plan(hip.make_desc(dtype, 2600, 1027, 715, dtype_out=O.F32, transA=True, clear_accum=False))
+    assert (p.tile_m, p.tile_n, p.stages) == (128, 128, 3)
+    check(hip, dtype, 1, 0, 2304, 1289, 712, O.F32, hip.EPI_NONE, False, 1289, 0)
