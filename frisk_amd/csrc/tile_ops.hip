@@ -192,36 +192,42 @@ template <int KIND> __device__ __forceinline__ float wave_reduce(float v) {
 // A row's last group, where it is not whole, is fetched with the elements before it that fill it up, which are left out: every load is 16 bytes of the row and
 // those of a lane are under way together (element by element behind the others: us so / now, f16 2490 x 2453 6.7 / 4.5, 10069 x 4946 19.7 / 16.0, 2490 x 4453 8.9 / 5.9, f32
 // 5531 x 1315 8.8 / 6.6).  512 lanes from 1025 groups on (f32 4000 x 8192 20.4 / 19.7, f16 4426 x 15161 27.7 / 26.8); views that the last-level cache may hold are read
-// through the caches (2490 x 4453 6.2 past them, 5.9 so; 10069 x 4946 16.0 past them, 16.8).
+// through the caches (2490 x 4453 6.2 past them, 5.9 so; 10069 x 4946 16.0 past them, 16.8).  Past them, groups that straddle 128-byte lines are fetched twice: where rows start
+// off 16-byte boundaries the groups start at the first one, what lies before it being a group that overlaps like the last (bf16 6199 x 10825 30.7 at the rows' starts, 25.7 so).
 template <int DT, int KIND, int THREADS, bool STREAMED> __global__ void __launch_bounds__(THREADS)
 reduce_rows_kernel(const typename Elem<DT>::T* src, int64_t rows, int64_t cols, int64_t ld, int clear, typename Elem<DT>::T* dst, float* partial) {
   typedef typename Elem<DT>::T T;
   constexpr int G = 16 / sizeof(T), FLIGHT = 4;
-  const int64_t gpr = (cols + G - 1) / G, whole = cols / G, step = (int64_t)gridDim.y * THREADS;
-  const int twice = (int)(gpr * G - cols);
+  const int64_t step = (int64_t)gridDim.y * THREADS;
   __shared__ float wsum[THREADS / 64];
   for (int64_t r = blockIdx.x; r < rows; r += gridDim.x) {
     float acc = Op<KIND>::id();
     const T* row = src + r * ld;
+    // groups 0 .. full - 1 from element `head` on, then the one that ends with the row, then the one it starts with
+    const int64_t head = STREAMED ? ((0 - (uintptr_t)row) & 15) / sizeof(T) : 0, full = (cols - head) / G, tail = cols - head - full * G;
+    const int64_t groups = full + (tail > 0) + (STREAMED && head > 0);
     // four groups of a lane under way together, combined in their order (one after the other 98 x 12807 bf16 took 6.2 us, 8192 x 8192 f16 22.9)
-    for (int64_t g = (int64_t)blockIdx.y * THREADS + threadIdx.x; g < gpr; g += FLIGHT * step) {
+    for (int64_t g = (int64_t)blockIdx.y * THREADS + threadIdx.x; g < groups; g += FLIGHT * step) {
       T in[FLIGHT][G];
 #pragma unroll
       for (int u = 0; u < FLIGHT; ++u) {
-        const int64_t at = g + u * step < whole ? (g + u * step) * G : cols - G;
-        if (g + u * step >= gpr) continue;
+        const int64_t k = g + u * step, at = k < full ? head + k * G : (!STREAMED || (tail > 0 && k == full) ? cols - G : 0);
+        if (k >= groups) continue;
         if constexpr (STREAMED) *(v4u*)in[u] = load16(row + at);
         else *(v4u*)in[u] = *(const v4u_any*)(row + at);
       }
 #pragma unroll
       for (int u = 0; u < FLIGHT; ++u) {
-        if (g + u * step < whole) {
+        const int64_t k = g + u * step;
+        if (k < full) {
 #pragma unroll
           for (int e = 0; e < G; ++e) acc = Op<KIND>::f(acc, Elem<DT>::load(in[u][e]));
-        } else if (g + u * step < gpr) {
+        } else if (k < groups) {
+          const bool last = !STREAMED || (tail > 0 && k == full);
+          const int lo = last ? G - (int)tail : 0, hi = last ? G : (int)head;  // its own elements
 #pragma unroll
           for (int e = 0; e < G; ++e)
-            if (e >= twice) acc = Op<KIND>::f(acc, Elem<DT>::load(in[u][e]));
+            if (e >= lo && e < hi) acc = Op<KIND>::f(acc, Elem<DT>::load(in[u][e]));
         }
       }
     }
