@@ -9,7 +9,7 @@
 // assembly over fixed registers: a step is two lane reads of the program, a jump to its handler and 8 vector instructions in
 // place, the operand picked by the register index mode.  (As a C++ switch the compiler joins the values of all cases after every
 // step by register moves: 327 vector, 300 scalar and 120 branch instructions per group of 8 columns for (x - s * c) * g + b; here
-// 109, 125 and 34.)  That body on 8192 x 8192 f16: 137 us before, 46 to 51 now (a plain copy: 41); log2(max(x, c) / (x + c)), bound by
+// 109, 125 and 34.)  That body on 8192 x 8192 f16: 137 us before, 45 now (a plain copy: 39); log2(max(x, c) / (x + c)), bound by
 // the vector pipe in its division, 123 -> 69.5; x + y 80 -> 58; rows off 16-byte boundaries (4095 x 8191) 369 -> 29.
 // Operands that are the same for every row stay in registers while the lane's columns do, values of one per row stay one
 // register, and what the next groups need from memory is fetched while the current one is evaluated.  All arithmetic is
@@ -38,6 +38,11 @@ enum Step {
 };
 constexpr int kSlotS0 = 0, kSlotX = 8, kSlotCol0 = 16, kSlotCol1 = 24, kSlotWalk2 = 32, kSlotS1 = 40;
 constexpr int kChunk = 64;  // steps in one register of a wave, one per lane; STEP_MORE goes on to the second register
+// What an operand of one value per row goes through before the steps see it: value * mul + add, one operation with a constant (or none) whose other part changes
+// nothing, so that it rounds once as that operation does.  Done on a row's value it is one instruction a group; as steps on eight columns a lane, with the value
+// below the top kept meanwhile, it was four steps in place of one: (x - s c) g + b of 8192 x 8192 f16 48.7 us as steps, 45.1 so, bf16
+// 3077 x 3724 12.1 / 10.9, 12208 x 658 12.4 / 10.8, 6199 x 10825 54.5 / 51.9; f32, which memory bounds, even.
+struct RowScale { float mul = 1.f, add = -0.f; };
 struct EwSteps {
   int code[2 * kChunk];
   float imm[2 * kChunk];
@@ -46,6 +51,7 @@ struct EwSteps {
   int head, walk2;        // operands fetched a group ahead: the one the program starts with, and another that walks the rows (-1: none)
   int col0, col1;         // operands that are the same for every row, kept in registers while the columns stay
   int row0, row1;         // operands of one value per row, fetched a group ahead
+  RowScale scale0, scale1;
 };
 // An operand as the kernel addresses it, resolved on the host (an operand looked up by its number is a chain of dependent scalar loads).
 struct EwOperand {
@@ -58,6 +64,7 @@ struct EwArgs {
   char* out;
   int out_dt, n_steps;
   EwOperand head, walk2, row0, row1, col0, col1;
+  RowScale scale0, scale1;
   EwOperand in[FRISK_EW_MAX_INPUTS];  // for STEP_FETCH, by number
   int code[2 * kChunk];
   float imm[2 * kChunk];
@@ -315,8 +322,8 @@ __attribute__((amdgpu_waves_per_eu(four_waves(DT, HELD, DEPTH, ROWS == ROWS_UNIF
         if (p.walk2.at) to_float(h.walk2, type_of(p.walk2), walk2);
       }
       if constexpr (HELD == HELD_ALL) {
-        if (p.row0.at) row_a = row_value(p.row0.dt, h.row0);
-        if (p.row1.at) row_b = row_value(p.row1.dt, h.row1);
+        if (p.row0.at) row_a = __builtin_fmaf(row_value(p.row0.dt, h.row0), p.scale0.mul, p.scale0.add);
+        if (p.row1.at) row_b = __builtin_fmaf(row_value(p.row1.dt, h.row1), p.scale1.mul, p.scale1.add);
       }
       const int64_t here = row < p.rows ? row : p.rows - 1;
       if (rb + SETS * (int64_t)gridDim.y < row_blocks) {
@@ -391,8 +398,39 @@ EwSteps steps_of(const EwParams& p, int held) {
   for (int i = 1; i < p.n_ops; ++i)
     if (p.op[i] == FRISK_EW_INPUT && p.in_col_stride[p.arg[i]] && (p.in_row_stride[p.arg[i]] || p.in_dtype[p.arg[i]] != p.out_dtype) && p.arg[i] != (p.op[0] == FRISK_EW_INPUT ? p.arg[0] : -1))
       col_as_walk2 = false;
+  int mentions[FRISK_EW_MAX_INPUTS] = {};
+  for (int i = 0; i < p.n_ops; ++i)
+    if (p.op[i] == FRISK_EW_INPUT) ++mentions[p.arg[i]];
+  // steps i, i + 1 and i + 2 combine the only mention of an operand of one value per row, which a slot can hold, with a constant
+  auto scaled_row = [&](int i, RowScale& scale) {
+    if (held != HELD_ALL || i + 2 >= p.n_ops || (s.row0 >= 0 && s.row1 >= 0)) return -1;
+    const bool value_first = p.op[i] == FRISK_EW_INPUT;
+    if (p.op[value_first ? i : i + 1] != FRISK_EW_INPUT || p.op[value_first ? i + 1 : i] != FRISK_EW_CONST) return -1;
+    const int k = p.arg[value_first ? i : i + 1];
+    const float c = p.imm[value_first ? i + 1 : i];
+    if (p.in_col_stride[k] != 0 || mentions[k] != 1) return -1;
+    switch (p.op[i + 2]) {
+      case FRISK_EW_ADD: scale.add = c; return k;
+      case FRISK_EW_SUB: scale.mul = value_first ? 1.f : -1.f; scale.add = value_first ? -c : c; return k;
+      case FRISK_EW_MUL: scale.mul = c; return k;
+      default: return -1;
+    }
+  };
   for (int i = 0; i < p.n_ops; ++i) {
     const int op = p.op[i];
+    RowScale scale;
+    if (const int k = scaled_row(i, scale); k >= 0) {
+      const bool first = s.row0 < 0;
+      (first ? s.row0 : s.row1) = k;
+      (first ? s.scale0 : s.scale1) = scale;
+      const int next = i + 3 < p.n_ops ? p.op[i + 3] : -1;
+      const bool fused = next >= FRISK_EW_ADD && next <= FRISK_EW_MIN;
+      if (!fused && ++below > 0) emit(STEP_SAVE, slot_below(below));
+      if (below > s.depth) s.depth = below;
+      emit(fused ? by_row[next - FRISK_EW_ADD] : STEP_LOADR, !first);
+      i += 2 + fused;
+      continue;
+    }
     if (op == FRISK_EW_INPUT || op == FRISK_EW_CONST) {
       const int k = op == FRISK_EW_INPUT ? p.arg[i] : 0, next = i + 1 < p.n_ops ? p.op[i + 1] : -1;
       const bool walks = p.in_col_stride[k] != 0;
@@ -528,6 +566,7 @@ hipError_t launch_elementwise(const EwParams& given, hipStream_t s) {
   for (int k = 0; k < FRISK_EW_MAX_INPUTS; ++k) a.in[k] = operand(k);
   a.head = operand(prog.head); a.walk2 = operand(prog.walk2);
   a.row0 = operand(prog.row0); a.row1 = operand(prog.row1); a.col0 = operand(prog.col0); a.col1 = operand(prog.col1);
+  a.scale0 = prog.scale0; a.scale1 = prog.scale1;
   a.n_steps = prog.n;
   __builtin_memcpy(a.code, prog.code, sizeof a.code);
   __builtin_memcpy(a.imm, prog.imm, sizeof a.imm);

@@ -134,3 +134,36 @@ def test_dense_views_of_several_groups_a_lane(hip, dt, rows, cols):
     on_device(hip, gated, dt, rows, cols, ["walk", "walk", "walk"], lambda x, y, z: x * y + z)
     on_device(hip, [("input", 0), ("input", 1), "add"], dt, rows, cols, ["walk", "walk"], lambda x, y: x + y, in_place=True)
     on_device(hip, [("input", 0), ("const", 1.0), "add", "log2"], dt, rows, cols, ["walk"], lambda x: (x + 1).log2(), in_place=True)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt,tdt", [(O.F32, "float32"), (O.F16, "float16"), (O.BF16, "bfloat16")])
+@pytest.mark.parametrize("rows,cols", [(3, 40), (4100, 520), (6200, 259)])
+def test_a_value_of_the_row_combined_with_a_constant(hip, dt, tdt, rows, cols):
+    """either way round, once and for both slots, as a right operand, before everything else and with the operand mentioned again; zeros of either sign and infinities among the
+    values.  One rounding to fp32 per operation, as torch's do: the same bits."""
+    import torch
+    tdt, g = getattr(torch, tdt), torch.Generator(device="cuda").manual_seed(9)
+    x = torch.randn(rows, cols, device="cuda", generator=g).to(tdt)
+    r, s = (torch.randn(rows, device="cuda", generator=g).to(tdt) for _ in range(2))
+    col = (torch.rand(cols, device="cuda", generator=g) + 0.5).to(tdt)
+    r[0], r[1], r[2] = 0.0, -0.0, float("inf")
+    X, Rv, Sv, Cv = x.float(), r.float()[:, None], s.float()[:, None], col.float()
+    does = {"add": torch.add, "sub": torch.sub, "mul": torch.mul}
+    programs = []
+    for name, f in does.items():
+        for c in (0.75, -3.0):
+            k = torch.tensor(c, device="cuda")
+            programs += [([("input", 0), ("input", 1), ("const", c), name, "sub", ("input", 3), "mul"], (X - f(Rv, k)) * Cv),
+                         ([("input", 0), ("const", c), ("input", 1), name, "max"], torch.maximum(X, f(k, Rv))),
+                         ([("input", 1), ("const", c), name, ("input", 0), "add"], f(Rv, k) + X),
+                         ([("input", 0), ("input", 1), ("const", c), name, "neg", "add"], X + (-f(Rv, k))),
+                         ([("input", 0), ("input", 1), ("const", c), name, "add", ("const", 2.0), ("input", 2), name, "mul"], (X + f(Rv, k)) * f(torch.tensor(2.0, device="cuda"), Sv)),
+                         ([("input", 0), ("input", 2), ("const", c), name, "add", ("input", 2), "mul"], (X + f(Sv, k)) * Sv),
+                         ([("input", 0), ("input", 2), ("const", c), "div", "add"], X + Sv / k)]
+    for program, want in programs:
+        desc = hip.make_elementwise_desc(program, [(dt, cols, 1), (dt, 1, 0), (dt, 1, 0), (dt, 0, 1)], dt, rows, cols)
+        out = torch.full_like(x, 7.0)
+        hip.elementwise(desc, [t.data_ptr() for t in (x, r, s, col)], out.data_ptr(), torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        assert torch.equal(out, want.to(tdt)), program
