@@ -1,6 +1,6 @@
 """Builds libfrisk_hip.so (HIP kernels + C ABI) for gfx950, in-tree.
 
-    python -m frisk_amd.build          # rebuild everything (HIP library, the device-check library, frisk_ffi extension)
+    python -m frisk_amd.build          # rebuild everything (HIP library, the device-check library, the frisk_ffi and frisk_launch extensions)
     python -m frisk_amd.build --if-missing
 
 hipcc cross-compiles without a GPU; the resulting library is loaded from
@@ -96,6 +96,21 @@ def build_ffi(verbose=True):
     return out
 
 
+def build_launch(verbose=True):
+    """the `frisk_launch` CPython extension (the calls of runtime.py that launch kernels), host code only"""
+    import sysconfig
+
+    out = os.path.join(HERE, "frisk_launch" + sysconfig.get_config_var("EXT_SUFFIX"))
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-shared", "-fPIC", "-fvisibility=hidden", "-I" + sysconfig.get_paths()["include"], "-I" + os.path.join(ROOT, "include"),
+           os.path.join(FFI_DIR, "launch.cpp"), "-o", out]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("building frisk_launch failed:\n" + r.stderr)
+    if verbose:
+        print("built", out)
+    return out
+
+
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--if-missing", action="store_true")
@@ -107,6 +122,7 @@ def main():
     build(a.j)
     build_hwcheck()
     build_ffi()
+    build_launch()
 
 
 if __name__ == "__main__":

@@ -174,15 +174,17 @@ struct AffineExpr {
   AffineExpr ceil_div(const AffineExpr& o) const { return binary(ExprKind::CeilDiv, *this, o); }
   AffineExpr mod(const AffineExpr& o) const { return binary(ExprKind::Mod, *this, o); }
 
-  int64_t eval(const std::vector<int64_t>& dims, const std::vector<int64_t>& syms) const {
-    switch (kind()) {
-      case ExprKind::Constant: return impl->value;
-      case ExprKind::DimId: return dims.at((size_t)impl->value);
-      case ExprKind::SymbolId: return syms.at((size_t)impl->value);
+  int64_t eval(const std::vector<int64_t>& dims, const std::vector<int64_t>& syms) const { return eval(impl.get(), dims, syms); }
+  static int64_t eval(const AffineExprImpl* e, const std::vector<int64_t>& dims, const std::vector<int64_t>& syms) {
+    if (!e) throw std::invalid_argument("cannot evaluate a null affine expression");
+    switch (e->kind) {
+      case ExprKind::Constant: return e->value;
+      case ExprKind::DimId: return dims.at((size_t)e->value);
+      case ExprKind::SymbolId: return syms.at((size_t)e->value);
       default: break;
     }
-    int64_t a = AffineExpr(impl->lhs).eval(dims, syms), b = AffineExpr(impl->rhs).eval(dims, syms);
-    switch (kind()) {
+    const int64_t a = eval(e->lhs.get(), dims, syms), b = eval(e->rhs.get(), dims, syms);
+    switch (e->kind) {
       case ExprKind::Add: return a + b;
       case ExprKind::Mul: return a * b;
       case ExprKind::Mod: return a - floordiv(a, b) * b;
@@ -961,22 +963,21 @@ inline CopyOrigin copy_origin(const Operation* cp, bool dst_side, Value by, Valu
     else if (k && v == k) which[(size_t)i] = 2;
     else throw std::invalid_argument("not a tiled GEMM kernel: a copy is indexed by something other than the grid indices and the K induction variable");
   }
-  auto at = [&](int64_t vby, int64_t vbx, int64_t vk) {
-    const int64_t val[3] = {vby, vbx, vk};
-    std::vector<int64_t> dims, syms;
-    for (int i = 0; i < count; ++i) (i < map.num_dims() ? dims : syms).push_back(val[which[(size_t)i]]);
-    std::vector<int64_t> out;
-    for (int r = 0; r < map.num_results(); ++r) out.push_back(map.impl->results[(size_t)r].eval(dims, syms));
-    return out;
-  };
+  // the map at five points, whose inputs and results take no storage of their own (with it the ten vectors of a copy's side were a quarter of the match)
+  static const int64_t points[5][3] = {{0, 0, 0}, {1, 0, 0}, {0, 1, 0}, {0, 0, 1}, {2, 3, 5}};
+  const size_t results = (size_t)map.num_results();
+  std::vector<int64_t> dims((size_t)map.num_dims()), syms((size_t)(count - map.num_dims()));
   CopyOrigin o;
-  o.c0 = at(0, 0, 0);
-  const std::vector<int64_t> m1 = at(1, 0, 0), n1 = at(0, 1, 0), k1 = at(0, 0, 1), probe = at(2, 3, 5);
-  for (size_t r = 0; r < o.c0.size(); ++r) {
-    o.cm.push_back(m1[r] - o.c0[r]);
-    o.cn.push_back(n1[r] - o.c0[r]);
-    o.ck.push_back(k1[r] - o.c0[r]);
-    if (probe[r] != o.c0[r] + 2 * o.cm[r] + 3 * o.cn[r] + 5 * o.ck[r]) throw std::invalid_argument("not a tiled GEMM kernel: a copy's index map is not linear in the grid and K indices");
+  o.c0.resize(results); o.cm.resize(results); o.cn.resize(results); o.ck.resize(results);
+  std::vector<int64_t>* const at[4] = {&o.c0, &o.cm, &o.cn, &o.ck};
+  for (int t = 0; t < 5; ++t) {
+    for (int i = 0; i < count; ++i) (i < map.num_dims() ? dims[(size_t)i] : syms[(size_t)(i - map.num_dims())]) = points[t][which[(size_t)i]];
+    for (size_t r = 0; r < results; ++r) {
+      const int64_t v = map.impl->results[r].eval(dims, syms);
+      if (t == 0) o.c0[r] = v;
+      else if (t < 4) (*at[t])[r] = v - o.c0[r];
+      else if (v != o.c0[r] + 2 * o.cm[r] + 3 * o.cn[r] + 5 * o.ck[r]) throw std::invalid_argument("not a tiled GEMM kernel: a copy's index map is not linear in the grid and K indices");
+    }
   }
   return o;
 }

@@ -1,4 +1,4 @@
-"""ctypes binding of libfrisk_hip.so (include/frisk_hip.h).
+"""ctypes binding of libfrisk_hip.so (include/frisk_hip.h); the calls that launch kernels go through the extension frisk_launch.
 
 This is the thin host layer the builder front end and the benchmarks use to
 reach the HIP kernels.  It never falls back to another implementation: if the
@@ -79,6 +79,7 @@ class FriskHipError(RuntimeError):
 
 
 _lib = None
+_native = None  # frisk_launch: the calls that launch kernels, without ctypes' conversion of their arguments
 
 EXPORTS = ["frisk_hip_init", "frisk_hip_abi_version", "frisk_hip_last_error", "frisk_hip_plan", "frisk_hip_workspace_bytes",
            "frisk_hip_gemm", "frisk_hip_lds_access_cycles", "frisk_hip_lds_search", "frisk_hip_lds_search_atom", "frisk_hip_lds_offset", "frisk_hip_wave_partition",
@@ -89,7 +90,7 @@ EXPORTS = ["frisk_hip_init", "frisk_hip_abi_version", "frisk_hip_last_error", "f
 
 def lib():
     """Loads libfrisk_hip.so; raises if it has not been built (python -m frisk_amd.build)."""
-    global _lib
+    global _lib, _native
     if _lib is not None:
         return _lib
     if not os.path.exists(LIB_PATH):
@@ -132,8 +133,19 @@ def lib():
     L.frisk_hip_reduce.argtypes = [ctypes.c_int, vp, i64, i64, i64, ctypes.c_int, ctypes.c_int, ctypes.c_int, vp, vp, ctypes.c_size_t, vp]
     if L.frisk_hip_abi_version() != ABI_VERSION:
         raise ImportError("libfrisk_hip.so has ABI %d, binding expects %d" % (L.frisk_hip_abi_version(), ABI_VERSION))
-    _lib = L
+    try:
+        from . import frisk_launch
+    except ImportError as e:
+        raise ImportError("frisk_launch is not built: run `python -m frisk_amd.build`") from e
+    frisk_launch.bind(GemmDesc, ElementwiseDesc, AttentionDesc, *[ctypes.cast(getattr(L, "frisk_hip_" + f), ctypes.c_void_p).value
+                                                                  for f in ("gemm", "fill", "copy", "reduce", "elementwise", "softmax", "attention")])
+    _native, _lib = frisk_launch, L
     return L
+
+
+def _bound():
+    lib()
+    return _native
 
 
 def _check(status):
@@ -180,8 +192,12 @@ def workspace_bytes(desc):
 
 def gemm(desc, A_ptr, B_ptr, C_ptr, scaleA_ptr=None, scaleB_ptr=None, workspace_ptr=None, workspace_bytes=0, stream=None):
     """Asynchronous launch on `stream` (a raw hipStream_t value or None). Pointers are raw device addresses."""
-    _check(lib().frisk_hip_gemm(ctypes.byref(desc), A_ptr, B_ptr, C_ptr, scaleA_ptr, scaleB_ptr, workspace_ptr,
-                                workspace_bytes, stream))
+    # (None: arguments that only ctypes takes; the other launches alike)
+    status = (_native or _bound()).gemm(desc, A_ptr, B_ptr, C_ptr, scaleA_ptr, scaleB_ptr, workspace_ptr, workspace_bytes, stream)
+    if status is None:
+        status = lib().frisk_hip_gemm(ctypes.byref(desc), A_ptr, B_ptr, C_ptr, scaleA_ptr, scaleB_ptr, workspace_ptr, workspace_bytes, stream)
+    if status:
+        _check(status)
 
 
 def static_workspace_bytes():
@@ -200,12 +216,20 @@ REDUCE_KINDS = {"add": 0, "sum": 0, "mul": 1, "min": 2, "max": 3}
 
 def fill(dtype, dst_ptr, rows, cols, ld, value, stream=None):
     """frisk.fill on a rank-2 view of device memory (asynchronous on `stream`)"""
-    _check(lib().frisk_hip_fill(dtype, dst_ptr, rows, cols, ld, float(value), stream))
+    status = (_native or _bound()).fill(dtype, dst_ptr, rows, cols, ld, float(value), stream)
+    if status is None:
+        status = lib().frisk_hip_fill(dtype, dst_ptr, rows, cols, ld, float(value), stream)
+    if status:
+        _check(status)
 
 
 def copy(src_dtype, src_ptr, src_ld, dst_dtype, dst_ptr, dst_ld, rows, cols, stream=None):
     """frisk.copy of a rows x cols window, converting between f32 / f16 / bf16 when the types differ"""
-    _check(lib().frisk_hip_copy(src_dtype, src_ptr, src_ld, dst_dtype, dst_ptr, dst_ld, rows, cols, stream))
+    status = (_native or _bound()).copy(src_dtype, src_ptr, src_ld, dst_dtype, dst_ptr, dst_ld, rows, cols, stream)
+    if status is None:
+        status = lib().frisk_hip_copy(src_dtype, src_ptr, src_ld, dst_dtype, dst_ptr, dst_ld, rows, cols, stream)
+    if status:
+        _check(status)
 
 
 def copy_tiles(src_dtype, src_ptr, src_ld, dst_dtype, dst_ptr, dst_ld, tile_rows, tile_cols, n0, src_step0, dst_step0, n1=1, src_step1=0, dst_step1=0, stream=None):
@@ -237,8 +261,12 @@ def make_elementwise_desc(program, inputs, out_dtype, rows, cols, out_ld=None):
 
 def elementwise(desc, input_ptrs, out_ptr, stream=None):
     """frisk.block body as one interpreted kernel: out = program(inputs) for every point (asynchronous on `stream`)"""
-    arr = (ctypes.c_void_p * max(1, len(input_ptrs)))(*input_ptrs)
-    _check(lib().frisk_hip_elementwise(ctypes.byref(desc), arr, out_ptr, stream))
+    status = (_native or _bound()).elementwise(desc, input_ptrs, out_ptr, stream)
+    if status is None:
+        arr = (ctypes.c_void_p * max(1, len(input_ptrs)))(*input_ptrs)
+        status = lib().frisk_hip_elementwise(ctypes.byref(desc), arr, out_ptr, stream)
+    if status:
+        _check(status)
 
 
 def reduce_workspace_bytes(dtype, rows, cols, dim):
@@ -248,7 +276,12 @@ def reduce_workspace_bytes(dtype, rows, cols, dim):
 def reduce(dtype, src_ptr, rows, cols, ld, dim, kind, clear, dst_ptr, workspace_ptr=None, workspace_bytes=0, stream=None):
     """frisk.reduce along `dim` with kind "add" | "mul" | "min" | "max" (or its enum value)"""
     k = REDUCE_KINDS[kind] if isinstance(kind, str) else kind
-    _check(lib().frisk_hip_reduce(dtype, src_ptr, rows, cols, ld, dim, k, int(bool(clear)), dst_ptr, workspace_ptr, workspace_bytes, stream))
+    clear = 1 if clear else 0
+    status = (_native or _bound()).reduce(dtype, src_ptr, rows, cols, ld, dim, k, clear, dst_ptr, workspace_ptr, workspace_bytes, stream)
+    if status is None:
+        status = lib().frisk_hip_reduce(dtype, src_ptr, rows, cols, ld, dim, k, clear, dst_ptr, workspace_ptr, workspace_bytes, stream)
+    if status:
+        _check(status)
 
 
 def softmax_workspace_bytes(dtype, rows, cols):
@@ -259,7 +292,11 @@ def softmax(dtype, src_ptr, src_ld, dst_ptr, dst_ld, rows, cols, scale_log2=1.44
             workspace_bytes=0):
     """row softmax in base 2: dst = 2^(scale_log2 * src) / row sum; the default scale makes it the natural softmax.
     A workspace of softmax_workspace_bytes lets a few very long rows be split over several work-groups each."""
-    _check(lib().frisk_hip_softmax(dtype, src_ptr, src_ld, dst_ptr, dst_ld, rows, cols, scale_log2, lse_ptr, workspace_ptr, workspace_bytes, stream))
+    status = (_native or _bound()).softmax(dtype, src_ptr, src_ld, dst_ptr, dst_ld, rows, cols, scale_log2, lse_ptr, workspace_ptr, workspace_bytes, stream)
+    if status is None:
+        status = lib().frisk_hip_softmax(dtype, src_ptr, src_ld, dst_ptr, dst_ld, rows, cols, scale_log2, lse_ptr, workspace_ptr, workspace_bytes, stream)
+    if status:
+        _check(status)
 
 
 def make_attention_desc(dtype, batch, heads, seq_q, seq_k, head_dim=128, scale=None, k_transposed=False):
@@ -274,7 +311,11 @@ def make_attention_desc(dtype, batch, heads, seq_q, seq_k, head_dim=128, scale=N
 
 def attention(desc, Q_ptr, K_ptr, V_ptr, O_ptr, lse_ptr=None, stream=None):
     """fused softmax(scale * Q K^T) V (asynchronous on `stream`); lse_ptr optionally receives the row log-sum-exp"""
-    _check(lib().frisk_hip_attention(ctypes.byref(desc), Q_ptr, K_ptr, V_ptr, O_ptr, lse_ptr, stream))
+    status = (_native or _bound()).attention(desc, Q_ptr, K_ptr, V_ptr, O_ptr, lse_ptr, stream)
+    if status is None:
+        status = lib().frisk_hip_attention(ctypes.byref(desc), Q_ptr, K_ptr, V_ptr, O_ptr, lse_ptr, stream)
+    if status:
+        _check(status)
 
 
 def wave_partition(policy, tile_m, tile_n, num_waves):
