@@ -1002,7 +1002,12 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
   plan->guarded = k->guard != 0;
   // (grids that are no multiple of 8 too, their last few ids staying in place; us in launch order / regrouped: bf16 3000x11008x4096 NT,
   // 516 tiles, 208.5 / 198.2; bf16 7168x6912x4096 TN, 756 tiles, 274.5 / 264.5; single rounds even)
-  plan->xcd_remap = (int64_t)plan->grid_x * plan->grid_y >= 8;
+  // One row of tiles against B [K][N] whose rows lie a multiple of 2 KiB apart stays in launch order: its tiles share A alone, which every L2 gets either way, and neighbouring
+  // columns on one XCD are the same few of its L2's channels in every row.  us regrouped / in launch order, B from memory: fp16 48x8192x8192 32.8 / 31.4, 1x8192x8192 30.8 / 29.2, bf16 16x8192x5120
+  // 22.4 / 20.8, 48x12288x8192 45.7 / 44.7, int8 16x8192x2048 7.9 / 7.4, e4m3 8x12288x2048 10.1 / 9.6; 100 problems with N a multiple of 1024 or 2048 1.02 times as fast, none slower by 3 %.
+  // Elsewhere 8-bit rows end inside lines that neighbouring tiles share (e4m3 5x5184x4096 10.2 / 11.1); B [N][K] 16x8192x2048 8.7 / 11.0.
+  const bool columns = plan->grid_y == 1 && !d->transB && d->ldb * es % 2048 == 0;
+  plan->xcd_remap = (int64_t)plan->grid_x * plan->grid_y >= 8 && !columns;
   if (with_model) {  // for the caller of frisk_hip_plan: no launch looks at the LDS layouts
     fill_layout(&plan->lds_a, !d->transA, es, frag_bytes(d->dtype_ab), k->bm, k->bk, k->wm * k->wn * k->wk, k->atom);
     fill_layout(&plan->lds_b, d->transB != 0, es, frag_bytes(d->dtype_ab), k->bn, k->bk, k->wm * k->wn * k->wk, k->atom);
