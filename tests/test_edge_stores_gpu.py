@@ -40,9 +40,10 @@ def check(hip, dtype, transA, transB, M, N, K, out, epilogue, clear, ldc, shift,
 @pytest.mark.parametrize("dtype", [O.F32, O.F16, O.BF16, O.I8, O.E4M3])
 @pytest.mark.parametrize("transA,transB", [(0, 0), (0, 1), (1, 0), (1, 1)])
 def test_whole_tiles_of_an_edge_kernel_beside_the_others(hip, dtype, transA, transB):
-    """M and N of whole tiles under a partial K tile (no store to check), one short of and one beyond them; C packed, in odd rows and off its first 16-byte boundary"""
+    """M and N of whole tiles under a partial K tile (nothing to check), one short of and one beyond them, 1 to 12 columns of a wave's tile; C packed, in odd rows and off its first 16-byte
+    boundary"""
     K = {O.F32: 3 * 32 + 4, O.F16: 3 * 64 + 8, O.BF16: 3 * 64 + 8, O.I8: 3 * 128 + 16, O.E4M3: 4 * 128 + 16}[dtype]
-    for M, N in ((512, 512), (511, 513), (257, 640), (130, 384), (96, 257)):
+    for M, N in ((512, 512), (511, 513), (257, 640), (130, 384), (96, 257), (300, 131), (77, 521), (260, 268)):
         for out in OUTS[dtype]:
             for epilogue in (hip.EPI_NONE, hip.EPI_ROW_COL_SCALE, hip.EPI_TENSOR_SCALE)[:1 if out == O.I32 else 3]:
                 for clear, ldc, shift in ((True, N, 0), (True, N + 3, 1), (False, N, 0), (False, N + 3, 1)):
