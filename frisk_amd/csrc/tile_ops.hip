@@ -494,8 +494,11 @@ constexpr int64_t kMaxGrid = 1 << 22;
 
 // `on_lines`: every row starts on a 128-byte boundary.  Where they don't, a strip of 128 bytes takes two lines of every row, and the slices are ahead sooner (lines
 // at reduce_tall_kernel).
+// Long rows on lines, which give most CUs a strip, stay in it longer: us in slices / in one launch, bf16 2000 x 7168 10.8 / 10.7, 2000 x 8192 11.4 / 10.8, 2500 x 8192
+// 12.5 / 13.3, 2500 x 11008 15.2 / 13.7, 3000 x 11008 17.9 / 15.6, 3000 x 16384 21.1 / 20.2, f32 3000 x 7168 18.3 / 17.5; 4096 x 12288 bf16 20.6 / 21.6.
 bool cols_in_one_launch(int64_t rows, int64_t row_bytes, bool on_lines) {
-  return rows <= (on_lines || row_bytes <= 256 ? 1536 : 1152) && row_bytes <= 256 * 128;
+  const int64_t most = !on_lines && row_bytes > 256 ? 1152 : !on_lines || row_bytes < 14 << 10 ? 1536 : row_bytes < 20 << 10 ? 2048 : 3072;
+  return rows <= most && row_bytes <= 256 * 128;
 }
 
 // slices of the reduced extent that give the launch enough work-groups

@@ -197,3 +197,26 @@ def test_softmax_of_rows_held_in_registers(hip, dt, tdt, tol):
             assert float((lse.double() - want_lse).abs().max()) <= 1e-4 * max(1.0, float(want_lse.abs().max())), (rows, cols, ld, shift)
             assert bool((y[:, cols:] == 5.0).all()) and bool((out[:shift] == 5.0).all()), (rows, cols, ld, shift)
             del z, want, scale
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt,tdt", [(O.F32, "float32"), (O.F16, "float16"), (O.BF16, "bfloat16")])
+def test_columns_of_long_rows_in_one_launch_and_beyond(hip, dt, tdt):
+    """both sides of the numbers of rows up to which rows of 14 and 20 KiB on 128-byte lines are summed in one launch; the same rows off lines and without a workspace.  Whole numbers
+    whose sums every type holds"""
+    import torch
+    tdt = getattr(torch, tdt)
+    es = torch.empty(0, dtype=tdt).element_size()
+    g = torch.Generator(device="cuda").manual_seed(10)
+    for kib, rows in ((14, 2048), (14, 2049), (20, 3072), (20, 3073)):
+        for cols in (kib * 1024 // es, kib * 1024 // es - 64, kib * 1024 // es + 3):
+            for ld in (-(-cols * es // 128) * 128 // es, cols + 1 + (cols & 1)):
+                x = torch.full((rows, ld), float("nan"), device="cuda", dtype=tdt)
+                x[:, :cols] = ((torch.rand(rows, cols, device="cuda", generator=g) < 0.03).float() * (2 * torch.randint(0, 2, (rows, cols), device="cuda", generator=g) - 1).float()).to(tdt)
+                need = hip.reduce_workspace_bytes(dt, rows, cols, 0)
+                ws = torch.full((max(need, 4),), 0xFF, dtype=torch.uint8, device="cuda")
+                for with_ws in (True, False):
+                    d = torch.full((cols + 1,), 7.0, device="cuda", dtype=tdt)
+                    hip.reduce(dt, x.data_ptr(), rows, cols, ld, 0, "add", False, d.data_ptr(), ws.data_ptr() if with_ws else None, need if with_ws else 0, torch.cuda.current_stream().cuda_stream)
+                    torch.cuda.synchronize()
+                    assert torch.equal(d[:cols].float(), x[:, :cols].float().sum(0) + 7) and float(d[cols]) == 7.0, (rows, cols, ld, with_ws)
