@@ -129,6 +129,19 @@ __device__ __forceinline__ Raw load_raw(const char* at, int dt, bool streamed) {
   }
   return r;
 }
+// the same of two halves of 4 columns, the second one `apart` columns behind the first
+__device__ __forceinline__ Raw load_halves(const char* at, int dt, int64_t apart, bool streamed) {
+  typedef unsigned v2u_any __attribute__((ext_vector_type(2), aligned(2)));
+  Raw r;
+  if (dt == FRISK_F32) {
+    r.a = streamed ? __builtin_nontemporal_load((const v4u_any*)at) : *(const v4u_any*)at;
+    r.b = streamed ? __builtin_nontemporal_load((const v4u_any*)(at + apart * 4)) : *(const v4u_any*)(at + apart * 4);
+  } else {
+    const v2u_any lo = *(const v2u_any*)at, hi = *(const v2u_any*)(at + apart * 2);
+    r.a = v4u{lo[0], lo[1], hi[0], hi[1]};
+  }
+  return r;
+}
 // The first `valid` (1 to 7) of 8 elements, of a row that has no more: without branches, the last one again in place of those beyond it, so that all
 // are under way together
 __device__ __forceinline__ Raw load_raw_narrow(const char* at, int dt, int valid) {
@@ -201,6 +214,21 @@ __device__ __forceinline__ void store_group(char* at, int dt, const v8f& r, int 
   }
 }
 
+template <bool V> struct StreamedTag { static constexpr bool value = V; };
+// half a group of 32-bit columns from `first` (0 to 4) on
+template <bool STREAMED> __device__ __forceinline__ void store_half(char* at, const v8f& r, int half, int first) {
+  v4u w;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) { const float x = r[4 * half + e]; w[e] = __builtin_bit_cast(unsigned, x); }
+  if (first == 0) {
+    if constexpr (STREAMED) __builtin_nontemporal_store(w, (v4u_any*)at); else *(v4u_any*)at = w;
+    return;
+  }
+#pragma unroll
+  for (int e = 1; e < 4; ++e)
+    if (e >= first) ((unsigned*)at)[e] = w[e];
+}
+
 // DT: element type of the operands that walk the rows and of the output (-1: mixed, read from the arguments).  HELD: which operands beside
 // `head` are held or fetched ahead: none; the second one that walks the rows; that one and the broadcast ones (44 more registers for 32-bit
 // operands, 32 for 16-bit ones, and 1500 instructions in front of the first step instead of 650: x + y of 1024 x 4096 f16 7.4 us with them,
@@ -220,6 +248,11 @@ __attribute__((amdgpu_waves_per_eu(four_waves(DT, HELD, DEPTH, ROWS == ROWS_UNIF
   if constexpr (ROWS == ROWS_UNIFORM) lane_row = __builtin_amdgcn_readfirstlane(lane_row);
   const int64_t groups = (p.cols + V - 1) / V, slabs = (groups + lanes - 1) >> lanes_log2, row_blocks = (p.rows + row_step - 1) / row_step;
   constexpr bool narrow = ROWS == ROWS_NARROW;
+  // HALVES: a lane's 8 columns of 32-bit operands are 4 and 4, a slab's lanes side by side in either half, so that every access of a wave is one run of memory.  (With a
+  // lane's two accesses side by side each takes half of every line, and stores past the caches, which halves allow, would write lines twice.  us side by side / so, f32: (x - s c) g + b of
+  // 4096 x 4096 29.1 / 23.0, 2875 x 5713 30.3 / 25.5, 20000 x 300 15.3 / 11.6, 8192 x 8192 104.2 / 100.3, exp2(x) c of 4095 x 8191 50.4 / 42.0, x + y of 1500 x 2000 8.8 / 7.5; halves with stores through
+  // the caches 26.9, 28.8, 14.2.)
+  constexpr bool HALVES = DT == FRISK_F32 && !narrow;
   // step i of a chunk of the program in lane i: a lane read instead of a dependent scalar load
   int code_reg[2] = {p.code[threadIdx.x & 63], 0}, imm_reg[2] = {__builtin_bit_cast(int, p.imm[threadIdx.x & 63]), 0};
   if (p.n_steps > kChunk) {
@@ -246,7 +279,13 @@ __attribute__((amdgpu_waves_per_eu(four_waves(DT, HELD, DEPTH, ROWS == ROWS_UNIF
     // output is an operand too).  Fetched element by element behind branches, that group held up every row: (x - s c) g + b of 4095 x 8191 bf16 47.6 us, 32.3 so,
     // 16000 x 3999 f16 99.0 and 61.0, 6330 x 669 17.7 and 11.9.
     const int64_t past = ((slab << lanes_log2) + off + 1) * V - p.cols;
-    const int mine = past > 0 && !narrow ? (int)past : 0, last = narrow ? (int)p.cols : V, lane_col = off * V - mine;
+    const int mine = past > 0 && !narrow ? (int)past : 0, last = narrow ? (int)p.cols : V;
+    // HALVES: columns that the slab has, where the lane's halves start, and the columns of either that are another lane's (4: all)
+    const int64_t rest = p.cols - (slab << lanes_log2) * V;
+    const int col_a = lane_group * 4, col_b = (lanes + lane_group) * 4;
+    const int64_t at_a = col_a + 4 <= rest ? col_a : rest - 4, at_b = col_b + 4 <= rest ? col_b : rest - 4, apart = at_b - at_a;
+    const int mine_a = col_a - at_a < 4 ? (int)(col_a - at_a) : 4, mine_b = col_b - at_b < 4 ? (int)(col_b - at_b) : 4;
+    const int64_t lane_col = HALVES ? at_a : off * V - mine;
     int64_t row = rb0 * row_step + lane_row;
     const int64_t row_in = row < p.rows ? row : p.rows - 1;
     // element (r, first column of the group) of an operand whose elements are of type dt
@@ -257,6 +296,7 @@ __attribute__((amdgpu_waves_per_eu(four_waves(DT, HELD, DEPTH, ROWS == ROWS_UNIF
     };
     auto fetch_at = [&](const char* at, int dt, bool streamed) {
       if constexpr (narrow) return load_raw_narrow(at, dt, last);
+      else if constexpr (HALVES) return load_halves(at, dt, apart, streamed);
       else return load_raw(at, dt, streamed);
     };
     auto fetch_row_at = [&](const char* at, int dt) { return dt == FRISK_F32 ? *(const unsigned*)at : (unsigned)*(const uint16_t*)at; };
@@ -364,7 +404,23 @@ __attribute__((amdgpu_waves_per_eu(four_waves(DT, HELD, DEPTH, ROWS == ROWS_UNIF
           for (int e = 0; e < V; ++e) top[e] = top[e] / x[e];
         }
       }
-      if (live) store_group(out_at, out_dt, top, mine, last);
+      if constexpr (HALVES) {
+        auto store = [&](auto streamed) __attribute__((always_inline)) {
+          if (mine_a < 4) store_half<decltype(streamed)::value>(out_at, top, 0, mine_a);
+          if (mine_b < 4) store_half<decltype(streamed)::value>(out_at + apart * 4, top, 1, mine_b);
+        };
+        // past the caches, but for rows of up to 32 columns, whose halves are parts of lines
+        if (row < p.rows) {
+          if constexpr (ROWS == ROWS_UNIFORM) store(StreamedTag<true>{});
+          else if (lanes_log2 >= 3) {
+            asm volatile("");  // (these keep the compiler from making one store of the two, which is then not streamed)
+            store(StreamedTag<true>{});
+          } else {
+            store(StreamedTag<false>{});
+            asm volatile("");
+          }
+        }
+      } else if (live) store_group(out_at, out_dt, top, mine, last);
       out_at += out_step;
       row += row_stride;
       rb += gridDim.y;
@@ -546,10 +602,8 @@ hipError_t launch_elementwise(const EwParams& given, hipStream_t s) {
   int held = prog.col0 >= 0 || prog.row0 >= 0 ? HELD_ALL : prog.walk2 >= 0 ? HELD_WALK : HELD_NONE;
 // (16-bit ones too, beside a second operand that walks long rows and from 28 groups a lane on: x g + y of 8192 x 8192 f16 59.9 with 16 per CU, 63.8 with 4; 24 groups, 6144 x 8192, 58.7 / 56.0)
   const bool deep = f32 ? steps > (prog.walk2 >= 0 ? 5 : prog.col0 < 0 ? 7 : 12) * kHeldCap : prog.walk2 >= 0 && held == HELD_ALL && lanes_log2 == 8 && steps > 28 * kHeldCap;
-  set_grid(held == HELD_NONE || few || deep ? kCap : kHeldCap);
-  // f32 with more than three groups a lane on 16 per CU: the larger kernel's four waves a SIMD stream better than five of the smaller one (us, four / five: x + y of
-  // 8192 x 8192 144.4 / 149.1, 20000 x 2048 88.1 / 90.4, 4095 x 8191 72.9 / 74.8; with two, 4096 x 4096 39.6 / 38.4, 3000 x 4096 29.9 / 29.2)
-  if (f32 && held == HELD_WALK && steps > 3 * kCap) held = HELD_ALL;
+  // (f32 with two operands that walk long rows on 64 per CU: us on 16 / 64, x + y of 8192 x 8192 143.6 / 139.8, x g + y 145.2 / 141.2, 10000 x 5000 115.6 / 106.8; rows of 24 columns 60.3 / 69.7)
+  set_grid(held == HELD_NONE || few || deep ? (f32 && prog.walk2 >= 0 && deep && !short_rows ? kCap * 4 : kCap) : kHeldCap);
   if ((prog.head >= 0 && p.in_dtype[prog.head] != dt) || (prog.walk2 >= 0 && p.in_dtype[prog.walk2] != dt)) {
     dt = -1;
     held = HELD_NONE;

@@ -167,3 +167,30 @@ def test_a_value_of_the_row_combined_with_a_constant(hip, dt, tdt, rows, cols):
         hip.elementwise(desc, [t.data_ptr() for t in (x, r, s, col)], out.data_ptr(), torch.cuda.current_stream().cuda_stream)
         torch.cuda.synchronize()
         assert torch.equal(out, want.to(tdt)), program
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [3, 1100, 5000])
+def test_halves_of_a_lanes_columns_with_operands_of_other_types(hip, rows):
+    """32-bit rows of 8 columns to more than a slab of 2048 beside f16 and bf16 operands of one value per column and per row, held and fetched in place; packed and one element
+    apart, into another matrix and in place.  One rounding to fp32 per operation, as torch's do: the same bits."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(12)
+    stream = torch.cuda.current_stream().cuda_stream
+    for cols in (8, 9, 11, 12, 13, 31, 33, 35, 36, 64, 67, 259, 511, 512, 513, 1026) + ((2047, 2048, 2049, 2051, 2052, 4101) if rows < 5000 else ()):
+        for ld in (cols, cols + 1):
+            x = torch.randn(rows, ld, device="cuda", generator=g)
+            c1, c2 = torch.randn(cols, device="cuda", generator=g).half(), torch.randn(cols, device="cuda", generator=g).bfloat16()
+            r1, c3 = torch.randn(rows, device="cuda", generator=g).half(), torch.randn(cols, device="cuda", generator=g)
+            X = x[:, :cols]
+            for program, want in (
+                    ([("input", 0), ("input", 1), "mul", ("input", 2), "add"], X * c1.float() + c2.float()),
+                    ([("input", 0), ("input", 3), "sub", ("input", 1), "mul", ("input", 2), "add", ("input", 4), "max"], torch.maximum((X - r1.float()[:, None]) * c1.float() + c2.float(), c3)),
+                    ([("input", 0), ("const", 2.5), "mul"], X * 2.5)):
+                desc = hip.make_elementwise_desc(program, [(O.F32, ld, 1), (O.F16, 0, 1), (O.BF16, 0, 1), (O.F16, 1, 0), (O.F32, 0, 1)], O.F32, rows, cols, out_ld=ld)
+                for out in (torch.full_like(x, 3.0), x.clone()):
+                    beside = out[:, cols:].clone()
+                    first = out if bool((out == x).all()) else x
+                    hip.elementwise(desc, [t.data_ptr() for t in (first, c1, c2, r1, c3)], out.data_ptr(), stream)
+                    torch.cuda.synchronize()
+                    assert torch.equal(out[:, :cols], want) and torch.equal(out[:, cols:], beside), (rows, cols, ld, len(program))
