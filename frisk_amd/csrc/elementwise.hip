@@ -602,8 +602,9 @@ hipError_t launch_elementwise(const EwParams& given, hipStream_t s) {
   int held = prog.col0 >= 0 || prog.row0 >= 0 ? HELD_ALL : prog.walk2 >= 0 ? HELD_WALK : HELD_NONE;
 // (16-bit ones too, beside a second operand that walks long rows and from 28 groups a lane on: x g + y of 8192 x 8192 f16 59.9 with 16 per CU, 63.8 with 4; 24 groups, 6144 x 8192, 58.7 / 56.0)
   const bool deep = f32 ? steps > (prog.walk2 >= 0 ? 5 : prog.col0 < 0 ? 7 : 12) * kHeldCap : prog.walk2 >= 0 && held == HELD_ALL && lanes_log2 == 8 && steps > 28 * kHeldCap;
-  // (f32 with two operands that walk long rows on 64 per CU: us on 16 / 64, x + y of 8192 x 8192 143.6 / 139.8, x g + y 145.2 / 141.2, 10000 x 5000 115.6 / 106.8; rows of 24 columns 60.3 / 69.7)
-  set_grid(held == HELD_NONE || few || deep ? (f32 && prog.walk2 >= 0 && deep && !short_rows ? kCap * 4 : kCap) : kHeldCap);
+  // (f32 with two operands that walk long rows on 64 per CU: us on 16 / 64, x + y of 8192 x 8192 143.6 / 139.8, x g + y 145.2 / 141.2, 10000 x 5000 115.6 / 106.8, 4096 x 8192 70.4 / 67.9, 3000 x 8192 52.1 / 51.4, even below;
+  // rows of 24 columns 60.3 / 69.7)
+  set_grid(held == HELD_NONE || few || deep ? (f32 && prog.walk2 >= 0 && !short_rows && 2 * steps > 5 * kCap ? kCap * 4 : kCap) : kHeldCap);
   if ((prog.head >= 0 && p.in_dtype[prog.head] != dt) || (prog.walk2 >= 0 && p.in_dtype[prog.walk2] != dt)) {
     dt = -1;
     held = HELD_NONE;
