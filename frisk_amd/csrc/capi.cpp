@@ -730,6 +730,27 @@ static int follow_up(const std::vector<Variant>& list, const KernelEntry* k, con
   return -1;
 }
 
+// 256x256 edge tiles in slices of K (their index), for 16-bit problems of half a round to one of 128x128 tiles that run unsplit on those, one a CU, or on 64x128 tiles, where K is
+// deep; -1 elsewhere.  Such a CU takes 256 rows and columns a K tile from the last-level cache, 0.5 us at the 60 to 70 bytes a nanosecond that it pulls, however many others
+// are idle; a 256x256 tile takes half of that for the same work, and its slices fill the grid.  They cost a pass over 40 to 66 MB of partial sums, 15 to 20 us, so
+// it takes more than 100 K tiles and five slices, 128 where there are four.  us before / so, operands from memory: fp16 1696x1280x7360 NN 67.8 / 51.2, 2114x1152x10752 NT 95.6 / 69.7, 1777x1024x13376 NT (64x128)
+// 90.4 / 60.5, 1137x2880x11968 NT (4 slices) 110.7 / 87.3, bf16 2669x1256x6720 NN 70.8 / 60.4, 454x4951x16128 NT 137.2 / 81.2; what keeps its tile: 5312 of K
+// 1173x2944 NN 51.6 / 55.9, 6080 954x3008 52.2 / 56.3; three slices 2095x1856x9472 NN 83.7 / 92.5, 559x5504x6784 62.1 / 67.5; four under 8192 of K 802x3904x6912 NT 61.3 / 65.7, 2369x1472x8000 67.5 / 71.0, 7424
+// 2148x1635 70.3 / 69.2.  8-bit types stay: 10240 of
+// K int8 2828x896 NN 48.5 / 49.2.  Of 430 drawn problems half change over, 24 % faster, one of them
+// slower (bf16 764x4032x8192 NT 68.2 / 70.4).
+static int deep_tile(const std::vector<Variant>& list, const KernelEntry* k, const frisk_gemm_desc* d, bool rows_aligned, size_t workspace) {
+  const int64_t tiles = ((d->M + 127) / 128) * ((d->N + 127) / 128);
+  if (elem_size(k->dtype) != 2 || k->guard || !rows_aligned || k->bn != 128 || k->stages != 3 || k->wk > 1 || tiles < 100 || tiles > 256 || d->K < 6600 || d->M <= 256 || d->N <= 256) return -1;
+  for (const Variant& v : list) {
+    const KernelEntry* x = v.k;
+    if (!x->edge || x->guard || x->splitk || x->bm != 256 || x->bn != 256 || (d->M % 256 == 0 && d->N % 256 == 0) || d->K % x->bk) continue;
+    if ((double)d->lda * 2 * (d->transA ? x->bk : x->bm) >= 4294967296.0 || (double)d->ldb * 2 * (d->transB ? x->bn : x->bk) >= 4294967296.0) continue;
+    if (const int slices = edge_split_of(x, d, workspace); slices >= (d->K < 8192 ? 5 : 4)) return v.id;
+  }
+  return -1;
+}
+
 // The edge tile (its index) that takes a problem of more than 256 tiles of 128x128 over from `k`, which the search has found and
 // which runs it in one pass: the one whose rounds the model sees through 3 % sooner, -1 where there is none.  The search's costs know nothing of what a round pays beside
 // its K loop, nor of bytes of C: a 256x256 tile of 4-byte C with old values is 512 KiB, 19 us of a round whatever the K.  us before / now, operands
@@ -958,7 +979,7 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
     }
   }
   // Slices of the edge kernel that the search has found, and of K on a small grid; then the kernels that only follow up on one of the search.
-  const int found_slices = best >= 0 ? edge_slices() : 1;
+  int found_slices = best >= 0 ? edge_slices() : 1;
   int found_split = 1;
   if (best >= 0 && small && ks[best]->splitk && !no_split && d->K % ks[best]->bk == 0) found_split = small_grid_split(ks[best], d, ctx.workspace, false, table_range);
   const bool follows = best >= 0 && !tile_requested && d->split_k <= 1 && d->policy == FRISK_POLICY_SQUARE;
@@ -972,6 +993,12 @@ static int make_plan(const frisk_gemm_desc* d, frisk_gemm_plan* plan, bool with_
     if (found_slices == 1 && (!splits || (tiles < 256 ? sub_round_split(k, d, tiles, kt, ctx.workspace) : tail_split_of(k, tiles, kt, true, ctx.workspace)) == 1))
       next = other_tile(list, k, d, rows_aligned, packed);
   }
+  if (follows && d->split_k == 0 && !no_split && found_slices == 1 && found_split == 1)
+    if (const int id = deep_tile(list, ks[next >= 0 ? next : best], d, rows_aligned, left_for_sums(ks[best])); id >= 0) {
+      best = id;
+      next = -1;
+      found_slices = edge_split_of(ks[id], d, left_for_sums(ks[id]));
+    }
   if (next >= 0) best = next;
   const bool one_pass = next >= 0 && !same_edge_tile(ks[best]);
   if (d->M == 0 || d->N == 0) {  // nothing to compute

@@ -1,0 +1,72 @@
+"""Deep 16-bit products of one round of 128x128 tiles, which run on 256x256 edge tiles in slices of K: which ones, and what they give."""
+import pytest
+
+import oracle as O
+from frisk_amd import runtime as R
+
+# (M, N, K, slices of the 256x256 tiles that `workspace_bytes` is for; 0: another tile)
+ROUTES = [(1777, 1216, 7040, 7), (2043, 1144, 9024, 6), (1213, 2370, 9984, 5), (2669, 1256, 6656, 0), (2560, 1025, 6656, 5), (1137, 2880, 11968, 4), (600, 5214, 8192, 4), (600, 5214, 8128, 0),
+          (1777, 1216, 6592, 0), (1512, 2624, 10368, 0), (2095, 1856, 9472, 0), (250, 6400, 9024, 0), (2048, 2048, 8192, 0), (3000, 4096, 8192, 0), (700, 1216, 9024, 0)]
+
+
+def routed(p):
+    return "256x256x64_w2x2_s2x3_a16_edge" in R.kernel_names()[p.kernel_id]
+
+
+@pytest.mark.parametrize("dtype", [O.F16, O.BF16])
+@pytest.mark.parametrize("transB", [0, 1])
+@pytest.mark.parametrize("M,N,K,slices", ROUTES)
+def test_which_problems(dtype, transB, M, N, K, slices):
+    ld = (N + 7) // 8 * 8
+    d = R.make_desc(dtype, M, N, K, transB=transB, ldb=K if transB else ld, ldc=ld)
+    p = R.plan(d)
+    where = (R.kernel_names()[p.kernel_id], p.workspace_bytes)
+    if slices:
+        assert routed(p) and p.workspace_bytes == slices * p.grid_x * p.grid_y * 256 * 256 * 4 == R.workspace_bytes(d), where
+    else:
+        assert not routed(p) or p.workspace_bytes == 0 or M * N > 256 * 128 * 128, where
+
+
+@pytest.mark.parametrize("change", [dict(tile=(128, 128, 0)), dict(split_k=1), dict(policy=R.POLICY_FULL_ROW)])
+def test_what_a_descriptor_asks_for_stays(change):
+    """a tile, a number of slices or a wave policy that the descriptor names"""
+    try:
+        p = R.plan(R.make_desc(O.F16, 1777, 1216, 7040, **change))
+    except R.FriskHipError:
+        return  # (no kernel under that wave policy)
+    assert not routed(p) or change.get("split_k") != 1 and "tile" not in change
+
+
+@pytest.mark.parametrize("dtype", [O.I8, O.E4M3, O.F32])
+def test_other_types_stay(dtype):
+    p = R.plan(R.make_desc(dtype, 1777, 1216, 14080 if dtype != O.F32 else 3520, dtype_out={O.I8: O.I32, O.E4M3: O.BF16}.get(dtype)))
+    assert "256x256" not in R.kernel_names()[p.kernel_id] or dtype == O.F32
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [O.F16, O.BF16])
+@pytest.mark.parametrize("transA,transB", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_their_results(hip, dtype, transA, transB):
+    """whole numbers, exact in any order: C off its tiles and packed, old values, scales, 16- and 32-bit C"""
+    from test_edge_stores_gpu import check
+    for M, N, K in ((1216, 1416, 6656), (1336, 1736, 7104), (2208, 904, 9024)):
+        for out in (dtype, O.F32):
+            check(hip, dtype, transA, transB, M, N, K, out, hip.EPI_NONE, False, (N + 7) // 8 * 8 + 8, 0)
+            check(hip, dtype, transA, transB, M, N, K, out, hip.EPI_ROW_COL_SCALE, True, N, 0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("share", [0, 3, 4, 7])
+def test_with_less_workspace(hip, share):
+    """slices that the workspace does not hold fall away; below four another tile takes the problem"""
+    import torch
+    M, N, K = 1777, 1216, 7040
+    g = torch.Generator(device="cuda").manual_seed(share)
+    A, B = (torch.randint(-2, 3, s, device="cuda", generator=g).half() for s in ((M, K), (K, N)))
+    C = torch.full((M, N), 7.0, device="cuda")
+    d = hip.make_desc(O.F16, M, N, K, dtype_out=O.F32)
+    need = share * 35 * 256 * 256 * 4
+    ws = torch.empty(max(need, 16), dtype=torch.uint8, device="cuda")
+    hip.gemm(d, A.data_ptr(), B.data_ptr(), C.data_ptr(), None, None, ws.data_ptr() if need else None, need, torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    assert torch.equal(C, A.float() @ B.float())
