@@ -730,18 +730,18 @@ static int follow_up(const std::vector<Variant>& list, const KernelEntry* k, con
   return -1;
 }
 
-// 256x256 edge tiles in slices of K (their index), for 16-bit problems of half a round to one of 128x128 tiles that run unsplit on those, one a CU, or on 64x128 tiles, where K is
-// deep; -1 elsewhere.  Such a CU takes 256 rows and columns a K tile from the last-level cache, 0.5 us at the 60 to 70 bytes a nanosecond that it pulls, however many others
-// are idle; a 256x256 tile takes half of that for the same work, and its slices fill the grid.  They cost a pass over 40 to 66 MB of partial sums, 15 to 20 us, so
-// it takes more than 100 K tiles and five slices, 128 where there are four.  us before / so, operands from memory: fp16 1696x1280x7360 NN 67.8 / 51.2, 2114x1152x10752 NT 95.6 / 69.7, 1777x1024x13376 NT (64x128)
-// 90.4 / 60.5, 1137x2880x11968 NT (4 slices) 110.7 / 87.3, bf16 2669x1256x6720 NN 70.8 / 60.4, 454x4951x16128 NT 137.2 / 81.2; what keeps its tile: 5312 of K
-// 1173x2944 NN 51.6 / 55.9, 6080 954x3008 52.2 / 56.3; three slices 2095x1856x9472 NN 83.7 / 92.5, 559x5504x6784 62.1 / 67.5; four under 8192 of K 802x3904x6912 NT 61.3 / 65.7, 2369x1472x8000 67.5 / 71.0, 7424
-// 2148x1635 70.3 / 69.2.  8-bit types stay: 10240 of
-// K int8 2828x896 NN 48.5 / 49.2.  Of 430 drawn problems half change over, 24 % faster, one of them
-// slower (bf16 764x4032x8192 NT 68.2 / 70.4).
+// 256x256 edge tiles in slices of K (their index), for 16-bit problems of a quarter of a round to one of 128x128 tiles that run unsplit on those, one a CU, or on 64x128 tiles, where K
+// is deep; -1 elsewhere.  Such a CU takes 192 or 256 rows and columns a K tile from the last-level cache, 0.5 us at the 60 to 70 bytes a nanosecond that it pulls, however many
+// others are idle; a 256x256 tile takes half of that for the same work, and its slices fill the grid.  They cost a pass over 40 to 66 MB of partial sums, 15 to 20 us, so
+// it takes more than 100 K tiles and five slices, 128 where there are four, 88 up to 100 tiles of 128x128.  us before / so, operands from memory: fp16 1696x1280x7360 NN 67.8 / 51.2,
+// 2114x1152x10752 NT 95.6 / 69.7, 1777x1024x13376 NT (64x128) 90.4 / 60.5, 370x2696x10240 NT 71.9 / 42.9, 511x2264x6272 NN 49.5 / 36.9, 1137x2880x11968 NT (4 slices) 110.7 / 87.3, bf16
+// 2669x1256x6720 NN 70.8 / 60.4, 454x4951x16128 NT 137.2 / 81.2; what keeps its tile: of 100 tiles at most 808x1773x4416 NN 32.3 / 36.2, of more
+// 1173x2944x5312 NN 51.6 / 55.9, 954x3008x6080 52.2 / 56.3, 2877x632x5952 NT 41.7 / 45.2; three slices 2095x1856x9472 NN 83.7 / 92.5; four under 8192 of K 802x3904x6912 NT
+// 61.3 / 65.7, 2369x1472x8000 67.5 / 71.0, 2148x1635x7424 70.3 / 69.2.  8-bit types stay: 10240 of K int8 2828x896 NN 48.5 / 49.2.  Of 680 drawn problems 270 change over, 27 % faster,
+// one of them slower (bf16 764x4032x8192 NT 68.2 / 70.4).  Error against 64 bits, fp32 C of 1137x2880x11968: 6.9e-7 in one chain, 3.5e-7 in four.
 static int deep_tile(const std::vector<Variant>& list, const KernelEntry* k, const frisk_gemm_desc* d, bool rows_aligned, size_t workspace) {
   const int64_t tiles = ((d->M + 127) / 128) * ((d->N + 127) / 128);
-  if (elem_size(k->dtype) != 2 || k->guard || !rows_aligned || k->bn != 128 || k->stages != 3 || k->wk > 1 || tiles < 100 || tiles > 256 || d->K < 6600 || d->M <= 256 || d->N <= 256) return -1;
+  if (elem_size(k->dtype) != 2 || k->guard || !rows_aligned || k->bn != 128 || k->stages != 3 || k->wk > 1 || tiles < 64 || tiles > 256 || d->K < (tiles <= 100 ? 5600 : 6600) || d->M <= 256 || d->N <= 256) return -1;
   for (const Variant& v : list) {
     const KernelEntry* x = v.k;
     if (!x->edge || x->guard || x->splitk || x->bm != 256 || x->bn != 256 || (d->M % 256 == 0 && d->N % 256 == 0) || d->K % x->bk) continue;

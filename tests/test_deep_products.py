@@ -5,7 +5,7 @@ import oracle as O
 from frisk_amd import runtime as R
 
 # (M, N, K, slices of the 256x256 tiles that `workspace_bytes` is for; 0: another tile)
-ROUTES = [(1777, 1216, 7040, 7), (2043, 1144, 9024, 6), (1213, 2370, 9984, 5), (2669, 1256, 6656, 0), (2560, 1025, 6656, 5), (1137, 2880, 11968, 4), (600, 5214, 8192, 4), (600, 5214, 8128, 0),
+ROUTES = [(1777, 1216, 7040, 7), (2043, 1144, 9024, 6), (1213, 2370, 9984, 5), (2669, 1256, 6656, 0), (2560, 1025, 6656, 5), (1137, 2880, 11968, 4), (511, 2264, 5632, 8), (511, 2264, 5568, 0), (600, 5214, 8192, 4), (600, 5214, 8128, 0),
           (1777, 1216, 6592, 0), (1512, 2624, 10368, 0), (2095, 1856, 9472, 0), (250, 6400, 9024, 0), (2048, 2048, 8192, 0), (3000, 4096, 8192, 0), (700, 1216, 9024, 0)]
 
 
