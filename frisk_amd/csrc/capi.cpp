@@ -739,18 +739,20 @@ static int follow_up(const std::vector<Variant>& list, const KernelEntry* k, con
 // tiles at most 808x1773x4416 NN 32.3 / 36.2, of more 954x3008x6080 52.2 / 56.3, 2877x632x5952 NT 41.7 / 45.2; three slices 2095x1856x9472 NN 83.7 / 92.5; four under 8192 of K
 // 802x3904x6912 NT 61.3 / 65.7, 2148x1635x7424 70.3 / 69.2; int8 3090x512x11008 NN 39.8 / 41.4, e4m3 944x3472x9728 NT (4) 40.3 / 49.5.  Of 960 drawn problems 400 change over, 28 % faster, one of them
 // slower (bf16 764x4032x8192 NT 68.2 / 70.4).
-// Beyond 256 of them, on edge tiles in one pass, which are a round that is not full or two: 2 or 3 slices.  us before / so: fp16 1019x5408x6912 NT 117.3 / 84.9, bf16 995x5616x8192 NN 140.4 / 98.5,
+// Beyond 256 of them, on edge tiles in one pass, which are a round that is not full or two: 2 or 3 slices of up to 112 tiles (above, where smaller tiles nearly fill their
+// round, 7 % on average are left).  us before / so: fp16 1019x5408x6912 NT 117.3 / 84.9, bf16 995x5616x8192 NN 140.4 / 98.5,
 // 1012x4640x5248 NT (3) 86.3 / 60.2, 2736x2320x7296 NT 106.8 / 98.5, int8 1921x2848x12800 NN 109.3 / 85.4, e4m3 2624x1760x7424 NN (3) 62.2 / 51.0; under the lines below bf16 1347x4288x5120 NN 72.8 / 77.0, int8
 // 1336x3680x6912 NT 49.7 / 55.2, 3022x2176x11392 NN 83.5 / 87.0, e4m3 1114x4304x6144 NT (3) 45.0 / 49.6.  Of 350 drawn problems 90 change over, 11 % faster, none of them slower by 2 %.
 // Error against 64 bits, fp32 C of fp16 1137x2880x11968: 6.9e-7 in one chain, 3.5e-7 in four.
 static int deep_tile(const std::vector<Variant>& list, const KernelEntry* k, const frisk_gemm_desc* d, bool rows_aligned, size_t workspace) {
   const int64_t tiles = ((d->M + 127) / 128) * ((d->N + 127) / 128);
+  const int64_t tiles256 = ((d->M + 255) / 256) * ((d->N + 255) / 256);
   const int es = elem_size(k->dtype);
   if (es == 4 || k->guard || !rows_aligned || k->wk > 1 || tiles < 64 || tiles > 512 || d->M <= 256 || d->N <= 256) return -1;
   if (tiles > 256 ? !k->edge || k->splitk : k->bn != 128 || k->stages != 3) return -1;
   auto deep = [&](int slices) {
     const bool along_n = !d->transA && !d->transB;
-    if (tiles > 256) return slices >= 2 && d->K >= (es == 2 ? (slices == 2 ? 5632 : 4352) : slices == 2 ? 12032 : along_n ? 6400 : 8576);
+    if (tiles > 256) return slices >= 2 && tiles256 <= 112 && d->K >= (es == 2 ? (slices == 2 ? 5632 : 4352) : slices == 2 ? 12032 : along_n ? 6400 : 8576);
     if (es == 2) return slices >= 4 && d->K >= (slices == 4 ? 8192 : tiles <= 100 ? 5600 : 6600);
     return slices >= 4 && d->K >= (slices == 4 ? 16384 : along_n ? 11264 : 12288);
   };
