@@ -731,18 +731,17 @@ static int follow_up(const std::vector<Variant>& list, const KernelEntry* k, con
 }
 
 // 256x256 edge tiles in slices of K (their index), for 16- and 8-bit problems of a quarter of a round to two of 128x128 tiles whose K is deep and whose tiles are not split otherwise; -1 elsewhere.
-// Up to 256 tiles of 128x128, on those, one a CU, or on 64x128 tiles: such a CU takes 192 or 256 rows and columns a K tile from the last-level cache, 0.5 us at the 60 to 70 bytes a
-// nanosecond that it pulls, however many others are idle; a 256x256 tile takes half of that for the same work, and its slices fill the grid.  They cost a pass over 40 to 66 MB of
-// partial sums, 15 to 20 us, so it takes more than 100 K tiles and five slices, 128 where there are four, 88 up to 100 tiles of 128x128; 8-bit types, whose partial sums are twice as
-// much beside their operands, about as many.  us before / so, operands from memory: fp16 1696x1280x7360 NN 67.8 / 51.2, 2114x1152x10752 NT 95.6 / 69.7, 370x2696x10240 NT 71.9 / 42.9, 511x2264x6272
-// NN 49.5 / 36.9, 1137x2880x11968 NT (4 slices) 110.7 / 87.3, bf16 454x4951x16128 NT 137.2 / 81.2, int8 1249x1520x12544 NN 57.8 / 45.3, e4m3 1410x1024x12928 NT 39.7 / 37.1; what keeps its tile: of 100
-// tiles at most 808x1773x4416 NN 32.3 / 36.2, of more 954x3008x6080 52.2 / 56.3, 2877x632x5952 NT 41.7 / 45.2; three slices 2095x1856x9472 NN 83.7 / 92.5; four under 8192 of K
-// 802x3904x6912 NT 61.3 / 65.7, 2148x1635x7424 70.3 / 69.2; int8 3090x512x11008 NN 39.8 / 41.4, e4m3 944x3472x9728 NT (4) 40.3 / 49.5.  Of 960 drawn problems 400 change over, 28 % faster, one of them
-// slower (bf16 764x4032x8192 NT 68.2 / 70.4).
+// Up to 256 tiles of 128x128, on those, one a CU, or on 64x128 tiles: such a CU takes 192 or 256 rows and columns a K tile, 0.5 us at the 60 to 70 bytes a nanosecond that it
+// pulls from the last-level cache, however many others are idle; a 256x256 tile takes half of that for the same work, and its slices fill the grid.  They cost a pass over 40 to 66 MB of
+// partial sums, 15 to 20 us, so it takes four slices and 117 K tiles and more, 164 in place of 64x128 tiles, two of which on a CU hide more; 8-bit types, whose partial sums are twice as much beside
+// their operands, 114 and 129.  The lines are where operands from the last-level cache gain too; from memory gains begin at three quarters of that K.  us before / so, from memory:
+// bf16 2043x1144x9024 NN 90.6 / 58.9, fp16 2114x1152x10752 NT 95.6 / 69.7, 1777x1024x13376 NT (64x128) 90.4 / 60.5, 1137x2880x11968 NT (4 slices) 110.7 / 87.3, bf16 454x4951x16128 NT 137.2 / 81.2, e4m3 1883x720x17920
+// NN 77.4 / 43.2; from the cache bf16 2880x768x13184 TN into fp32 sums 118.7 / 75.6, 768x3456x7424 TN 1.02 times as fast, 1152x2432x6720 NT 56.0 / 59.1, fp16 832x2176x9408 TN (64x128) 51.0 / 57.6, e4m3
+// 1856x1344x13312 NT 43.4 / 50.2, int8 1600x1152x16128 NN (64x128) 42.6 / 50.9; three slices 2095x1856x9472 NN 83.7 / 92.5.
 // Beyond 256 of them, on edge tiles in one pass, which are a round that is not full or two: 2 or 3 slices of up to 112 tiles (above, where smaller tiles nearly fill their
-// round, 7 % on average are left).  us before / so: fp16 1019x5408x6912 NT 117.3 / 84.9, bf16 995x5616x8192 NN 140.4 / 98.5,
-// 1012x4640x5248 NT (3) 86.3 / 60.2, 2736x2320x7296 NT 106.8 / 98.5, int8 1921x2848x12800 NN 109.3 / 85.4, e4m3 2624x1760x7424 NN (3) 62.2 / 51.0; under the lines below bf16 1347x4288x5120 NN 72.8 / 77.0, int8
-// 1336x3680x6912 NT 49.7 / 55.2, 3022x2176x11392 NN 83.5 / 87.0, e4m3 1114x4304x6144 NT (3) 45.0 / 49.6.  Of 350 drawn problems 90 change over, 11 % faster, none of them slower by 2 %.
+// round, 7 % on average are left).  us before / so, from memory: fp16 1019x5408x6912 NT 117.3 / 84.9, bf16 995x5616x8192 NN 140.4 / 98.5,
+// 1012x4640x5248 NT (3) 86.3 / 60.2, 2736x2320x7296 NT 106.8 / 98.5, int8 1921x2848x12800 NN 109.3 / 85.4, from the cache 1.00 to 1.28 times as fast; under the lines below bf16 1347x4288x5120 NN 72.8 / 77.0, int8
+// 1336x3680x6912 NT 49.7 / 55.2, 3022x2176x11392 NN 83.5 / 87.0, 1472x3328x6528 NN (3, cache) 42.8 / 51.3.
 // Error against 64 bits, fp32 C of fp16 1137x2880x11968: 6.9e-7 in one chain, 3.5e-7 in four.
 static int deep_tile(const std::vector<Variant>& list, const KernelEntry* k, const frisk_gemm_desc* d, bool rows_aligned, size_t workspace) {
   const int64_t tiles = ((d->M + 127) / 128) * ((d->N + 127) / 128);
@@ -751,10 +750,8 @@ static int deep_tile(const std::vector<Variant>& list, const KernelEntry* k, con
   if (es == 4 || k->guard || !rows_aligned || k->wk > 1 || tiles < 64 || tiles > 512 || d->M <= 256 || d->N <= 256) return -1;
   if (tiles > 256 ? !k->edge || k->splitk : k->bn != 128 || k->stages != 3) return -1;
   auto deep = [&](int slices) {
-    const bool along_n = !d->transA && !d->transB;
-    if (tiles > 256) return slices >= 2 && tiles256 <= 112 && d->K >= (es == 2 ? (slices == 2 ? 5632 : 4352) : slices == 2 ? 12032 : along_n ? 6400 : 8576);
-    if (es == 2) return slices >= 4 && d->K >= (slices == 4 ? 8192 : tiles <= 100 ? 5600 : 6600);
-    return slices >= 4 && d->K >= (slices == 4 ? 16384 : along_n ? 11264 : 12288);
+    if (tiles > 256) return slices >= 2 && tiles256 <= 112 && d->K >= (es == 2 ? (slices == 2 ? 6144 : 4352) : slices == 2 ? 12032 : 8576);
+    return slices >= 4 && d->K >= (es == 2 ? (k->bm == 64 ? 10496 : slices == 4 ? 8192 : 7488) : k->bm == 64 ? 16512 : slices == 4 ? 16384 : 14592);
   };
   for (const Variant& v : list) {
     const KernelEntry* x = v.k;

@@ -5,8 +5,9 @@ import oracle as O
 from frisk_amd import runtime as R
 
 # (M, N, K, slices of the 256x256 tiles that `workspace_bytes` is for; 0: another tile)
-ROUTES = [(1777, 1216, 7040, 7), (2043, 1144, 9024, 6), (1213, 2370, 9984, 5), (2669, 1256, 6656, 0), (2560, 1025, 6656, 5), (1137, 2880, 11968, 4), (511, 2264, 5632, 8), (511, 2264, 5568, 0), (600, 5214, 8192, 4), (600, 5214, 8128, 0),
-          (1777, 1216, 6592, 0), (1512, 2624, 10368, 0), (2095, 1856, 9472, 0), (250, 6400, 9024, 0), (2048, 2048, 8192, 0), (3000, 4096, 8192, 0), (1019, 5408, 6912, 2), (1347, 4288, 5568, 0), (1012, 4640, 4352, 3), (1012, 4640, 4288, 0), (700, 1216, 9024, 0)]
+ROUTES = [(1777, 1216, 7488, 7), (2043, 1144, 9024, 6), (1213, 2370, 9984, 5), (2669, 1256, 7424, 0), (2560, 1025, 7488, 5), (1137, 2880, 11968, 4), (511, 2264, 10496, 8), (511, 2264, 10432, 0),
+          (600, 5214, 8192, 4), (600, 5214, 8128, 0), (1777, 1216, 7424, 0), (1512, 2624, 10368, 0), (2095, 1856, 9472, 0), (250, 6400, 9024, 0), (2048, 2048, 8192, 0), (3000, 4096, 8192, 0),
+          (1019, 5408, 6912, 2), (1347, 4288, 6080, 0), (1012, 4640, 4352, 3), (1012, 4640, 4288, 0), (700, 1216, 9024, 0)]
 
 
 def routed(p):
@@ -28,11 +29,11 @@ def test_which_problems(dtype, transB, M, N, K, slices):
 
 
 @pytest.mark.parametrize("dtype", [O.I8, O.E4M3])
-@pytest.mark.parametrize("M,N,K,nn,nt", [(1249, 1520, 12544, 1, 1), (1249, 1520, 12160, 1, 0), (1249, 1520, 11136, 0, 0), (944, 3472, 16384, 1, 1), (1921, 2848, 12032, 1, 1),
-                                         (1921, 2848, 11904, 0, 0), (1196, 4320, 8576, 1, 1), (1201, 3360, 8448, 1, 0), (2624, 1760, 6272, 0, 0)])
-def test_which_problems_of_8_bit_types(dtype, M, N, K, nn, nt):
-    for transB, sliced in ((0, nn), (1, nt)):
-        p = R.plan(R.make_desc(dtype, M, N, K, transB=transB, dtype_out={O.I8: O.I32, O.E4M3: O.BF16}[dtype]))
+@pytest.mark.parametrize("M,N,K,sliced", [(1249, 1520, 16512, 1), (1152, 2368, 14592, 1), (1152, 2368, 14464, 0), (944, 3472, 16384, 1), (1921, 2848, 12032, 1), (1921, 2848, 11904, 0), (1196, 4320, 8576, 1)])
+def test_which_problems_of_8_bit_types(dtype, M, N, K, sliced):
+    for transB in (0, 1):
+        ld = (N + 15) // 16 * 16
+        p = R.plan(R.make_desc(dtype, M, N, K, transB=transB, ldb=K if transB else ld, ldc=ld, dtype_out={O.I8: O.I32, O.E4M3: O.BF16}[dtype]))
         assert sliced == (p.tile_m == p.tile_n == 256 and p.workspace_bytes > 0), (transB, R.kernel_names()[p.kernel_id], p.workspace_bytes)
 
 
@@ -40,7 +41,7 @@ def test_which_problems_of_8_bit_types(dtype, M, N, K, nn, nt):
 def test_what_a_descriptor_asks_for_stays(change):
     """a tile, a number of slices or a wave policy that the descriptor names"""
     try:
-        p = R.plan(R.make_desc(O.F16, 1777, 1216, 7040, **change))
+        p = R.plan(R.make_desc(O.F16, 1777, 1216, 7488, **change))
     except R.FriskHipError:
         return  # (no kernel under that wave policy)
     assert not routed(p) or change.get("split_k") != 1 and "tile" not in change
@@ -52,7 +53,7 @@ def test_what_a_descriptor_asks_for_stays(change):
 def test_their_results(hip, dtype, transA, transB):
     """whole numbers, exact in any order: C off its tiles and packed, old values, scales, 16- and 32-bit C"""
     from test_edge_stores_gpu import check
-    for M, N, K in ((1216, 1416, 6656), (1336, 1736, 7104), (2208, 904, 9024), (512, 2264, 5632), (1016, 4640, 4352), (1016, 5408, 6912)):
+    for M, N, K in ((1216, 1416, 7488), (1336, 1736, 8192), (2208, 904, 9024), (512, 2264, 10496), (1016, 4640, 4352), (1016, 5408, 6912)):
         for out in (dtype, O.F32):
             check(hip, dtype, transA, transB, M, N, K, out, hip.EPI_NONE, False, (N + 7) // 8 * 8 + 8, 0)
             check(hip, dtype, transA, transB, M, N, K, out, hip.EPI_ROW_COL_SCALE, True, N, 0)
@@ -63,7 +64,7 @@ def test_their_results(hip, dtype, transA, transB):
 @pytest.mark.parametrize("transB", [0, 1])
 def test_their_results_in_8_bit_types(hip, dtype, transB):
     from test_edge_stores_gpu import check
-    for M, N, K in ((1249, 1520, 12544), (944, 3472, 16384), (2624, 1760, 8576), (1921, 2848, 12032)):
+    for M, N, K in ((1249, 1520, 16512), (944, 3472, 16384), (2624, 1760, 8576), (1921, 2848, 12032)):
         for out in ((O.I32, O.F32) if dtype == O.I8 else (O.BF16, O.F32)):
             check(hip, dtype, 0, transB, M, N, K, out, hip.EPI_NONE, False, (N + 15) // 8 * 8, 0)
 
@@ -73,7 +74,7 @@ def test_their_results_in_8_bit_types(hip, dtype, transB):
 def test_with_less_workspace(hip, share):
     """slices that the workspace does not hold fall away; below four another tile takes the problem"""
     import torch
-    M, N, K = 1777, 1216, 7040
+    M, N, K = 1777, 1216, 7488
     g = torch.Generator(device="cuda").manual_seed(share)
     A, B = (torch.randint(-2, 3, s, device="cuda", generator=g).half() for s in ((M, K), (K, N)))
     C = torch.full((M, N), 7.0, device="cuda")
