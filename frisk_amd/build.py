@@ -1,7 +1,7 @@
 """Builds libfrisk_hip.so (HIP kernels + C ABI) for gfx950, in-tree.
 
     python -m frisk_amd.build          # rebuild everything (HIP library, the device-check library, the frisk_ffi and frisk_launch extensions)
-    python -m frisk_amd.build --if-missing
+    python -m frisk_amd.build --if-missing   # what is not there yet, the extensions for this interpreter
 
 hipcc cross-compiles without a GPU; the resulting library is loaded from
 frisk_amd/lib/ by frisk_amd.runtime.
@@ -11,6 +11,7 @@ import concurrent.futures
 import os
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
@@ -76,15 +77,16 @@ def build_hwcheck(verbose=True):
 
 
 FFI_DIR = os.path.join(HERE, "ffi")
+EXT_SUFFIX = sysconfig.get_config_var("EXT_SUFFIX")  # (of the interpreter that imports them)
+FFI_EXT = os.path.join(HERE, "frisk", "frisk_ffi" + EXT_SUFFIX)
+LAUNCH_EXT = os.path.join(HERE, "frisk_launch" + EXT_SUFFIX)
 FFI_SOURCES = ["ffi.cpp", "ir.cpp", "runtime.cpp"]
 
 
 def build_ffi(verbose=True):
     """the `frisk_ffi` CPython extension (IR builder + runtime), host code only"""
-    import sysconfig
-
     import pybind11
-    out = os.path.join(HERE, "frisk", "frisk_ffi" + sysconfig.get_config_var("EXT_SUFFIX"))
+    out = FFI_EXT
     cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-shared", "-fPIC", "-fvisibility=hidden",
            "-I" + pybind11.get_include(), "-I" + sysconfig.get_paths()["include"], "-I" + os.path.join(ROOT, "include")]
     cmd += [os.path.join(FFI_DIR, f) for f in FFI_SOURCES] + ["-o", out, "-ldl"]
@@ -98,9 +100,7 @@ def build_ffi(verbose=True):
 
 def build_launch(verbose=True):
     """the `frisk_launch` CPython extension (the calls of runtime.py that launch kernels), host code only"""
-    import sysconfig
-
-    out = os.path.join(HERE, "frisk_launch" + sysconfig.get_config_var("EXT_SUFFIX"))
+    out = LAUNCH_EXT
     cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-shared", "-fPIC", "-fvisibility=hidden", "-I" + sysconfig.get_paths()["include"], "-I" + os.path.join(ROOT, "include"),
            os.path.join(FFI_DIR, "launch.cpp"), "-o", out]
     r = subprocess.run(cmd, capture_output=True, text=True)
@@ -116,13 +116,11 @@ def main():
     ap.add_argument("--if-missing", action="store_true")
     ap.add_argument("-j", type=int, default=None)
     a = ap.parse_args()
-    if a.if_missing and os.path.exists(LIB):
-        print("present", LIB)
-        return
-    build(a.j)
-    build_hwcheck()
-    build_ffi()
-    build_launch()
+    for path, make in ((LIB, lambda: build(a.j)), (HWCHECK_LIB, build_hwcheck), (FFI_EXT, build_ffi), (LAUNCH_EXT, build_launch)):
+        if a.if_missing and os.path.exists(path):
+            print("present", path)
+        else:
+            make()
 
 
 if __name__ == "__main__":
