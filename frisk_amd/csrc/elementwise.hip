@@ -41,7 +41,8 @@ constexpr int kChunk = 64;  // steps in one register of a wave, one per lane; ST
 // What an operand of one value per row goes through before the steps see it: value * mul + add, one operation with a constant (or none) whose other part changes
 // nothing, so that it rounds once as that operation does.  Done on a row's value it is one instruction a group; as steps on eight columns a lane, with the value
 // below the top kept meanwhile, it was four steps in place of one: (x - s c) g + b of 8192 x 8192 f16 48.7 us as steps, 45.1 so, bf16
-// 3077 x 3724 12.1 / 10.9, 12208 x 658 12.4 / 10.8, 6199 x 10825 54.5 / 51.9; f32, which memory bounds, even.
+// 3077 x 3724 12.1 / 10.9, 12208 x 658 12.4 / 10.8, 6199 x 10825 54.5 / 51.9; f32, which memory bounds, even.  Programs without such a constant run on kernels without the multiply-add
+// (HELD_ALL): under it they were 1 to 2 % slower, f16 100000 x 24 x g + y 6.9 us, 6.2 without, x s 6.0 / 5.6, 3168 x 2891 (x - s) g + b 13.65 / 13.3, x g + b 12.93 / 12.69, 4096 x 4096 15.15 / 14.95.
 struct RowScale { float mul = 1.f, add = -0.f; };
 struct EwSteps {
   int code[2 * kChunk];
@@ -52,6 +53,7 @@ struct EwSteps {
   int col0, col1;         // operands that are the same for every row, kept in registers while the columns stay
   int row0, row1;         // operands of one value per row, fetched a group ahead
   RowScale scale0, scale1;
+  bool scaled;            // either of them meets a constant
 };
 // An operand as the kernel addresses it, resolved on the host (an operand looked up by its number is a chain of dependent scalar loads).
 struct EwOperand {
@@ -64,10 +66,10 @@ struct EwArgs {
   char* out;
   int out_dt, n_steps;
   EwOperand head, walk2, row0, row1, col0, col1;
-  RowScale scale0, scale1;
   EwOperand in[FRISK_EW_MAX_INPUTS];  // for STEP_FETCH, by number
   int code[2 * kChunk];
   float imm[2 * kChunk];
+  RowScale scale0, scale1;  // HELD_SCALED
 };
 
 // ---- the interpreter loop.  EACH: one instruction per column.  Handlers lie 256 bytes apart, in the order of Step; NEXT fetches
@@ -230,16 +232,16 @@ template <bool STREAMED> __device__ __forceinline__ void store_half(char* at, co
 }
 
 // DT: element type of the operands that walk the rows and of the output (-1: mixed, read from the arguments).  HELD: which operands beside
-// `head` are held or fetched ahead: none; the second one that walks the rows; that one and the broadcast ones (44 more registers for 32-bit
+// `head` are held or fetched ahead: none; the second one that walks the rows; that one and the broadcast ones, whose values of the row may meet constants first (HELD_SCALED) (44 more registers for 32-bit
 // operands, 32 for 16-bit ones, and 1500 instructions in front of the first step instead of 650: x + y of 1024 x 4096 f16 7.4 us with them,
 // 6.5 without, f32 11.3 and 9.9, 100000 x 24 f16 5.6 and 4.5, 8192 x 8192 f16 74.4 and 71).  DEPTH: values below the top the program needs.
 // ROWS: a wave's lanes lie in several rows, in one (rows of at least 64 groups), or in one each, of less than a group (as a case of the first, its loads
 // cost that one 0.4 us in 4.8 of 6304 x 136 f16).
 enum Rows { ROWS_SHARED, ROWS_UNIFORM, ROWS_NARROW };
-enum Held { HELD_NONE, HELD_WALK, HELD_ALL };
+enum Held { HELD_NONE, HELD_WALK, HELD_ALL, HELD_SCALED };
 // Kernels that hold all of them run four waves a SIMD where their registers allow it ((x - s c) g + b of 100000 x 24 f16: 136 registers and three
 // waves 8.6 us, 7.4 with four).
-constexpr bool four_waves(int dt, int held, int depth, bool uniform_row) { return held == HELD_ALL && depth == 1 && !(dt == FRISK_F32 && !uniform_row); }
+constexpr bool four_waves(int dt, int held, int depth, bool uniform_row) { return held >= HELD_ALL && depth == 1 && !(dt == FRISK_F32 && !uniform_row); }
 template <int DT, int HELD, int DEPTH, int ROWS> __global__ void __launch_bounds__(256)
 __attribute__((amdgpu_waves_per_eu(four_waves(DT, HELD, DEPTH, ROWS == ROWS_UNIFORM) ? 4 : 1, four_waves(DT, HELD, DEPTH, ROWS == ROWS_UNIFORM) ? 4 : 8))) elementwise_kernel(EwArgs p, int lanes_log2) {
   const int lanes = 1 << lanes_log2, row_step = 256 >> lanes_log2;
@@ -310,7 +312,7 @@ __attribute__((amdgpu_waves_per_eu(four_waves(DT, HELD, DEPTH, ROWS == ROWS_UNIF
     if constexpr (HELD >= HELD_WALK) {
       if (p.walk2.at) { walk2_at = operand_at(p.walk2, type_of(p.walk2), true, row_in); walk2_step = row_stride * p.walk2.row_bytes; }
     }
-    if constexpr (HELD == HELD_ALL) {
+    if constexpr (HELD >= HELD_ALL) {
       if (p.row0.at) { row0_at = operand_at(p.row0, p.row0.dt, false, row_in); row0_step = row_stride * p.row0.row_bytes; }
       if (p.row1.at) { row1_at = operand_at(p.row1, p.row1.dt, false, row_in); row1_step = row_stride * p.row1.row_bytes; }
     }
@@ -328,7 +330,7 @@ __attribute__((amdgpu_waves_per_eu(four_waves(DT, HELD, DEPTH, ROWS == ROWS_UNIF
       if constexpr (HELD >= HELD_WALK) {
         if (p.walk2.at) h.walk2 = fetch_at(walk2_at, type_of(p.walk2), true);
       }
-      if constexpr (HELD == HELD_ALL) {
+      if constexpr (HELD >= HELD_ALL) {
         if (p.row0.at) h.row0 = fetch_row_at(row0_at, p.row0.dt);
         if (p.row1.at) h.row1 = fetch_row_at(row1_at, p.row1.dt);
       }
@@ -339,7 +341,7 @@ __attribute__((amdgpu_waves_per_eu(four_waves(DT, HELD, DEPTH, ROWS == ROWS_UNIF
       if (fetched < p.rows) {  // (a lane whose next row lies beyond the view fetches the present one again)
         head_at += head_step;
         if constexpr (HELD >= HELD_WALK) walk2_at += walk2_step;
-        if constexpr (HELD == HELD_ALL) { row0_at += row0_step; row1_at += row1_step; }
+        if constexpr (HELD >= HELD_ALL) { row0_at += row0_step; row1_at += row1_step; }
       }
     };
     fetch_ahead(held0);
@@ -349,7 +351,7 @@ __attribute__((amdgpu_waves_per_eu(four_waves(DT, HELD, DEPTH, ROWS == ROWS_UNIF
         fetch_ahead(held1);
       }
     }
-    if constexpr (HELD == HELD_ALL) {
+    if constexpr (HELD >= HELD_ALL) {
       if (p.col0.at) to_float(fetch_at(operand_at(p.col0, p.col0.dt, true, 0), p.col0.dt, false), p.col0.dt, col0);
       if (p.col1.at) to_float(fetch_at(operand_at(p.col1, p.col1.dt, true, 0), p.col1.dt, false), p.col1.dt, col1);
     }
@@ -365,9 +367,13 @@ __attribute__((amdgpu_waves_per_eu(four_waves(DT, HELD, DEPTH, ROWS == ROWS_UNIF
       if constexpr (HELD >= HELD_WALK) {
         if (p.walk2.at) to_float(h.walk2, type_of(p.walk2), walk2);
       }
-      if constexpr (HELD == HELD_ALL) {
-        if (p.row0.at) row_a = __builtin_fmaf(row_value(p.row0.dt, h.row0), p.scale0.mul, p.scale0.add);
-        if (p.row1.at) row_b = __builtin_fmaf(row_value(p.row1.dt, h.row1), p.scale1.mul, p.scale1.add);
+      if constexpr (HELD >= HELD_ALL) {
+        if (p.row0.at) row_a = row_value(p.row0.dt, h.row0);
+        if (p.row1.at) row_b = row_value(p.row1.dt, h.row1);
+      }
+      if constexpr (HELD == HELD_SCALED) {
+        row_a = __builtin_fmaf(row_a, p.scale0.mul, p.scale0.add);
+        row_b = __builtin_fmaf(row_b, p.scale1.mul, p.scale1.add);
       }
       const int64_t here = row < p.rows ? row : p.rows - 1;
       if (rb + SETS * (int64_t)gridDim.y < row_blocks) {
@@ -383,8 +389,8 @@ __attribute__((amdgpu_waves_per_eu(four_waves(DT, HELD, DEPTH, ROWS == ROWS_UNIF
 #define EW_DEEP , "+{v[64:71]}"(s1), "+{v[72:79]}"(s2), "+{v[80:87]}"(s3), "+{v[88:95]}"(s4)
 #define EW_WALK2 , "{v[56:63]}"(walk2)
 #define EW_BROADCAST , "{v14}"(row_a), "{v15}"(row_b), "{v[40:47]}"(col0), "{v[48:55]}"(col1)
-        if constexpr (HELD == HELD_ALL && DEPTH > 1) EW_RUN(EW_DEEP, EW_BROADCAST EW_WALK2);
-        else if constexpr (HELD == HELD_ALL) EW_RUN(, EW_BROADCAST EW_WALK2);
+        if constexpr (HELD >= HELD_ALL && DEPTH > 1) EW_RUN(EW_DEEP, EW_BROADCAST EW_WALK2);
+        else if constexpr (HELD >= HELD_ALL) EW_RUN(, EW_BROADCAST EW_WALK2);
         else if constexpr (HELD == HELD_WALK && DEPTH > 1) EW_RUN(EW_DEEP, EW_WALK2);
         else if constexpr (HELD == HELD_WALK) EW_RUN(, EW_WALK2);
         else if constexpr (DEPTH > 1) EW_RUN(EW_DEEP, );
@@ -483,6 +489,7 @@ EwSteps steps_of(const EwParams& p, int held) {
       const bool first = s.row0 < 0;
       (first ? s.row0 : s.row1) = k;
       (first ? s.scale0 : s.scale1) = scale;
+      s.scaled = true;
       const int next = i + 3 < p.n_ops ? p.op[i + 3] : -1;
       const bool fused = next >= FRISK_EW_ADD && next <= FRISK_EW_MIN;
       if (!fused && ++below > 0) emit(STEP_SAVE, slot_below(below));
@@ -537,8 +544,9 @@ template <int DT, int HELD> void launch_typed(const dim3& grid, const EwArgs& a,
   if (depth <= 1) { FRISK_EW_LAUNCH(1) } else { FRISK_EW_LAUNCH(5) }
 #undef FRISK_EW_LAUNCH
 }
-template <int DT> void launch_held(int held, const dim3& grid, const EwArgs& a, int depth, int lanes_log2, hipStream_t s) {
-  if (held == HELD_ALL) launch_typed<DT, HELD_ALL>(grid, a, depth, lanes_log2, s);
+template <int DT> void launch_held(int held, bool scaled, const dim3& grid, const EwArgs& a, int depth, int lanes_log2, hipStream_t s) {
+  if (held == HELD_ALL && scaled) launch_typed<DT, HELD_SCALED>(grid, a, depth, lanes_log2, s);
+  else if (held == HELD_ALL) launch_typed<DT, HELD_ALL>(grid, a, depth, lanes_log2, s);
   else if (held == HELD_WALK) launch_typed<DT, HELD_WALK>(grid, a, depth, lanes_log2, s);
   else launch_typed<DT, HELD_NONE>(grid, a, depth, lanes_log2, s);
 }
@@ -631,9 +639,9 @@ hipError_t launch_elementwise(const EwParams& given, hipStream_t s) {
   __builtin_memcpy(a.imm, prog.imm, sizeof a.imm);
   const dim3 grid((unsigned)gx, (unsigned)gy);
   switch (dt) {
-    case FRISK_F32: launch_held<FRISK_F32>(held, grid, a, prog.depth, lanes_log2, s); break;
-    case FRISK_F16: launch_held<FRISK_F16>(held, grid, a, prog.depth, lanes_log2, s); break;
-    case FRISK_BF16: launch_held<FRISK_BF16>(held, grid, a, prog.depth, lanes_log2, s); break;
+    case FRISK_F32: launch_held<FRISK_F32>(held, prog.scaled, grid, a, prog.depth, lanes_log2, s); break;
+    case FRISK_F16: launch_held<FRISK_F16>(held, prog.scaled, grid, a, prog.depth, lanes_log2, s); break;
+    case FRISK_BF16: launch_held<FRISK_BF16>(held, prog.scaled, grid, a, prog.depth, lanes_log2, s); break;
     default: launch_typed<-1, HELD_NONE>(grid, a, prog.depth, lanes_log2, s); break;
   }
   return hipGetLastError();

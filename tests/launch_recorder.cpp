@@ -3,20 +3,25 @@
 //
 //   launch_recorder gemm keep|nokeep <dtype> <M> <N> <K> <transA> <transB> <workspace bytes>
 //   launch_recorder kept
-//   launch_recorder block <dtype> <rows> <cols> <operands: m = rows x cols, r = one value a row, c = one a column>
+//   launch_recorder block <dtype> <rows> <cols> <operands: m = rows x cols, r = one value a row, s = that times a constant, c = one a column>
 //   launch_recorder reduce <dtype> <rows> <cols> <leading dimension> <dim> <bytes from the source to a 256-byte boundary> <workspace: 1 what the library asks for, 0 none>
-#include <dlfcn.h>
 #include <hip/hip_runtime_api.h>
 #include <algorithm>
 #include <chrono>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <map>
 #include <new>
 #include <string>
 #include "frisk_hip.h"
 
 static bool g_keep = true, g_quiet = false;
+
+static std::map<const void*, std::string>& kernel_names() {
+  static auto* names = new std::map<const void*, std::string>;
+  return *names;
+}
 
 extern "C" {
 static struct { dim3 grid, block; size_t lds; hipStream_t stream; } g_pushed;
@@ -27,11 +32,12 @@ hipError_t __hipPopCallConfiguration(dim3* grid, dim3* block, size_t* lds, hipSt
 }
 hipError_t hipLaunchKernel(const void* kernel, dim3 grid, dim3 block, void**, size_t, hipStream_t) {
   if (g_quiet) return hipSuccess;
-  Dl_info info{};
-  dladdr(kernel, &info);
-  std::printf("launch %s %u %u %u %u\n", info.dli_sname ? info.dli_sname : "?", grid.x, grid.y, grid.z, block.x);
+  const auto name = kernel_names().find(kernel);
+  std::printf("launch %s %u %u %u %u\n", name != kernel_names().end() ? name->second.c_str() : "?", grid.x, grid.y, grid.z, block.x);
   return hipSuccess;
 }
+// (called as the library is loaded: kernels of anonymous namespaces have no name that dladdr finds)
+void __hipRegisterFunction(void**, const void* host, char*, const char* name, unsigned, void*, void*, dim3*, dim3*, int*) { kernel_names()[host] = name; }
 hipError_t hipGetDevice(int* device) { *device = 0; return hipSuccess; }
 hipError_t hipGetDevicePropertiesR0600(hipDeviceProp_tR0600* p, int) { std::memset(p, 0, sizeof *p); std::strcpy(p->gcnArchName, "gfx950"); return hipSuccess; }
 hipError_t hipFuncSetAttribute(const void*, hipFuncAttribute, int) { return hipSuccess; }
@@ -112,10 +118,16 @@ static int block(char** arg) {
   for (int k = 0; k < d.n_inputs; ++k) {  // x, then + or * the next operand
     in[k] = at(k);
     d.in_dtype[k] = d.out_dtype;
-    d.in_row_stride[k] = operands[k] == 'm' ? d.cols : operands[k] == 'r';
-    d.in_col_stride[k] = operands[k] != 'r';
+    const bool of_row = operands[k] == 'r' || operands[k] == 's';
+    d.in_row_stride[k] = operands[k] == 'm' ? d.cols : of_row;
+    d.in_col_stride[k] = !of_row;
     d.op[d.n_ops] = FRISK_EW_INPUT;
     d.arg[d.n_ops++] = k;
+    if (operands[k] == 's') {
+      d.op[d.n_ops] = FRISK_EW_CONST;
+      d.imm[d.n_ops++] = 0.5f;
+      d.op[d.n_ops++] = FRISK_EW_MUL;
+    }
     if (k) d.op[d.n_ops++] = k & 1 ? FRISK_EW_ADD : FRISK_EW_MUL;
   }
   std::printf("status %d\n", frisk_hip_elementwise(&d, in, at(8), nullptr));
