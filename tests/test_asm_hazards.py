@@ -162,3 +162,14 @@ def test_kernels_of_block_bodies_have_no_use_of_m0_besides_the_index_mode(tmp_pa
     assert listing.count("s_set_gpr_idx_on") > 28 * 10 and foreign_m0_uses(listing) == [] and "scratch_" not in listing
     # instructions that read M0 without naming it
     assert not re.search(r"^\s+(s_movrel|v_movrel|s_sendmsg|ds_gws|ds_append|ds_consume|buffer_load\w* .* lds|global_load_lds)", listing, re.M)
+
+
+@pytest.mark.skipif(not (os.path.exists(HIPCC) or shutil.which("hipcc")), reason="needs hipcc to produce the ISA listing")
+def test_what_stands_in_front_of_a_16_bit_body(tmp_path):
+    """the 16-bit kernels that hold all operands place their columns in 32 bits: 1780 instructions in all, 1801 with the 64 that the halves of 32-bit rows ask for"""
+    out = tmp_path / "elementwise.s"
+    cmd = [HIPCC if os.path.exists(HIPCC) else "hipcc", "--offload-arch=gfx950", "-O3", "-std=c++17", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+           "-I" + os.path.join(ROOT, "include"), "-I" + CSRC, "-Wno-unused-command-line-argument", "--cuda-device-only", "-S", os.path.join(CSRC, "elementwise.hip"), "-o", str(out)]
+    assert subprocess.run(cmd, capture_output=True).returncode == 0
+    body = re.search(r"^_ZN5frisk\S*elementwise_kernelILi1ELi2ELi1ELi1E\S*:.*?\n(.*?)s_endpgm", out.read_text(), re.S | re.M).group(1)
+    assert 1000 < len(re.findall(r"^\s+(?:[sv]|global|flat|ds|scratch)_", body, re.M)) <= 1790
