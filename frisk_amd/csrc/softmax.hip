@@ -333,8 +333,7 @@ template <int DT> hipError_t launch_typed(const void* src, int64_t sld, void* ds
   const T* x = (const T*)src;
   T* y = (T*)dst;
   const int64_t groups = (cols + G - 1) / G;
-  // (rows that a work-group can hold stay whole, in one launch, however few they are: f32 64 x 16000 10.6 us in slices, 5.5 whole)
-  if (slices > 1 && groups > kHeldGroups) {
+  if (slices > 1) {
     const dim3 sgrid((unsigned)rows, (unsigned)slices);
     hipLaunchKernelGGL((softmax_split_stats_kernel<DT>), sgrid, dim3(256), 0, s, x, sld, cols, c, partial);
     hipLaunchKernelGGL((softmax_split_write_kernel<DT>), sgrid, dim3(256), 0, s, x, sld, y, dld, cols, c, lse, (const float*)partial);
@@ -371,9 +370,10 @@ template <int DT> hipError_t launch_typed(const void* src, int64_t sld, void* ds
 }  // namespace
 
 int softmax_slices(int dtype, int64_t rows, int64_t cols) {
-  // Fewer than 1024 rows of at least 32 KiB: split each so that about 1024 work-groups exist, each with at least 16 KiB (the rows among them that a
-  // work-group can hold are not, and leave their workspace unused).
+  // Fewer than 1024 rows that a work-group cannot hold: split each so that about 1024 work-groups exist, each with at least 16 KiB.  (The others stay whole, in one launch, however few
+  // they are: f32 64 x 16000 10.6 us in slices, 5.5 whole.)
   const int64_t row_bytes = cols * (dtype == FRISK_F32 ? 4 : 2);
+  if (row_bytes <= kHeldGroups * 16) return 1;
   int slices = 1;
   while (rows * slices < 1024 && row_bytes / (slices * 2) >= 16384 && slices < 256) slices *= 2;
   return slices;

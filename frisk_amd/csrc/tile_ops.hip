@@ -503,8 +503,10 @@ bool cols_in_one_launch(int64_t rows, int64_t row_bytes, bool on_lines) {
 
 // slices of the reduced extent that give the launch enough work-groups
 int split_of(int dtype, int64_t rows, int64_t cols, int dim) {
-  // Split the reduced extent so that about 1024 work-groups exist, each still reducing at least 16 KiB.
+  // Split the reduced extent so that about 1024 work-groups exist, each still reducing at least 16 KiB.  Rows of up to 64 KiB stay whole, however few (us in slices and a second launch / in
+  // one, f32 394 x 9229 7.4 / 4.8, 64 x 16000 7.8 / 4.6).
   const int es = dtype == FRISK_F32 ? 4 : 2;
+  if (dim == 1 && cols * es <= 65536) return 1;
   const int G = 16 / es;
   const int64_t groups = dim == 1 ? rows : (cols + kStripLanes * G - 1) / (kStripLanes * G);
   const int64_t strip_bytes = cols * es < kStripLanes * 16 ? cols * es : kStripLanes * 16;
@@ -522,8 +524,7 @@ template <int DT, int KIND> hipError_t reduce_t(const void* src, int64_t rows, i
   // (without slices the one launch takes every view of its range)
   const bool tall = dim == 0 && split_of(DT, rows, cols, dim) > 1 &&
                     cols_in_one_launch(rows, cols * (int64_t)sizeof(T), slices == 1 || ((uintptr_t)src % 128 == 0 && ld * sizeof(T) % 128 == 0));
-  // rows of up to 64 KiB in one launch, however few (us in slices and a second launch / so, f32 394 x 9229 7.4 / 4.8, 64 x 16000 7.8 / 4.6)
-  if (tall || (dim == 1 && gpr <= 4096)) slices = 1;
+  if (tall) slices = 1;
   if (dim == 1) {
     if (gpr <= 256 && slices == 1) {
       int lanes_log2 = 0;

@@ -83,6 +83,17 @@ def test_tile_op_status_codes_before_any_launch():
     assert R.reduce_workspace_bytes(R.F16, 4, 1 << 22, 1) % (4 * 4) == 0 and R.reduce_workspace_bytes(R.F16, 4, 1 << 22, 1) > 0
 
 
+@pytest.mark.parametrize("dt", FLOATS, ids=[NAMES[d] for d in FLOATS])
+def test_rows_that_run_whole_ask_for_no_workspace(dt):
+    """up to 64 KiB a row: reductions along dim 1 and softmax are one launch, however few the rows"""
+    from frisk_amd import runtime as R
+    most = 65536 // (4 if dt == O.F32 else 2)
+    for rows in (1, 5, 300, 1023, 1024):
+        for cols in (1, most // 2, most // 2 + 1, most - 1, most):
+            assert R.softmax_workspace_bytes(dt, rows, cols) == 0 == R.reduce_workspace_bytes(dt, rows, cols, 1), (rows, cols)
+        assert (R.softmax_workspace_bytes(dt, rows, most + 1) > 0) == (R.reduce_workspace_bytes(dt, rows, most + 1, 1) > 0) == (rows < 1024), rows
+
+
 # ------------------------------------------------------------------ HIP kernels against the oracle (GPU)
 def _dev(arr):
     import torch
@@ -238,11 +249,12 @@ def test_softmax_status_codes_before_any_launch():
     assert status(R.F16, p + 1, 8, p, 8, 4, 8) == R.ERR_ALIGNMENT
     assert status(R.F16, p, 8, p, 8, 4, 8, float("inf")) == R.ERR_ARGUMENT
     R.softmax(R.F16, None, 8, None, 8, 0, 8)                          # nothing to do
-    # pure host: only fewer than 1024 rows of at least 32 KiB ask for a workspace, 8 bytes per row and slice
+    # pure host: only fewer than 1024 rows of more than 64 KiB ask for a workspace, 8 bytes per row and slice
     assert R.softmax_workspace_bytes(R.F16, 8, 1 << 24) == 8 * 128 * 8 and R.softmax_workspace_bytes(R.F16, 128, 1 << 20) == 128 * 8 * 8
     assert R.softmax_workspace_bytes(R.F16, 2000, 1 << 20) == 0 and R.softmax_workspace_bytes(R.F32, 4, 4096) == 0 and R.softmax_workspace_bytes(R.I8, 4, 1 << 20) == 0
 
 
+HELD = 4096 * 16  # bytes of a row up to which a work-group holds it whole
 SOFTMAX_VIEWS = [(1, 1, 0, 0), (3, 8, 0, 0), (7, 1000, 0, 0), (5, 1003, 3, 1), (64, 2048, 8, 0), (16, 4096, 0, 0), (9, 8192, 0, 0), (4, 16384, 0, 0),
                  (3, 16392, 0, 0), (2, 70000, 0, 0), (300, 40, 0, 0),
                  # rows shared by 1 ... 64 lanes of a wave with 1, 2 and 4 groups per lane, whole and partial last groups
@@ -274,7 +286,7 @@ def test_softmax_gpu(hip, dt):
             ref, lse = T.softmax_f64(dt, vals, cst)
             scale = np.maximum(np.abs(ref), np.sqrt(np.mean(ref * ref)))
             ws_bytes = hip.softmax_workspace_bytes(dt, rows, cols)
-            assert (ws_bytes > 0) == (cols * es >= 32768), (rows, cols)     # only a few very long rows are split
+            assert (ws_bytes > 0) == (cols * es > HELD), (rows, cols)     # only a few very long rows are split
             ws = torch.full((max(ws_bytes, 4),), 0xFF, dtype=torch.uint8, device="cuda")
             dS = _dev(src)
             for use_ws in ((False, True) if ws_bytes else (False,)):
