@@ -259,15 +259,15 @@ SOFTMAX_VIEWS = [(1, 1, 0, 0), (3, 8, 0, 0), (7, 1000, 0, 0), (5, 1003, 3, 1), (
                  (3, 16392, 0, 0), (2, 70000, 0, 0), (300, 40, 0, 0),
                  # rows shared by 1 ... 64 lanes of a wave with 1, 2 and 4 groups per lane, whole and partial last groups
                  (513, 8, 0, 0), (1000, 24, 0, 0), (999, 100, 4, 0), (130, 600, 0, 0), (77, 1500, 4, 0), (50, 1003, 5, 0), (31, 2040, 8, 0),
-                 # long rows split over work-groups through the workspace: aligned, odd, padded
+                 # long rows split over work-groups through the workspace: aligned, odd, padded (f16 and bf16 rows of 32768 are held whole)
                  (3, 300000, 0, 0), (2, 100003, 5, 1), (40, 32768, 8, 0)]
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dt", FLOATS, ids=[NAMES[d] for d in FLOATS])
 def test_softmax_gpu(hip, dt):
-    """every path: rows shared by the lanes of a wave, a work-group per row with the row in registers (2, 4, 8 groups per
-    lane), two sweeps (long rows), long rows split over work-groups (with a workspace), element by element (odd views);
+    """every path: rows shared by the lanes of a wave, a work-group per row with the row in registers (up to 4096 groups of 16 bytes),
+    two sweeps (longer rows), those split over work-groups (with a workspace), rows of less than a group element by element;
     bar: each element within 2e-3 (f16), 8e-3 (bf16), 2e-5 (f32) of the float64 value relative to max(|r|, rms), rows sum
     to one within that, log-sum within 1e-4"""
     import torch
@@ -309,9 +309,9 @@ def test_softmax_gpu(hip, dt):
     torch.cuda.synchronize()
     g = O.decode(dt, _host(d, st)).astype(np.float64).reshape(4, 512)
     assert np.all(g[:, 17] == 0.0) and np.allclose(g.sum(axis=1), 1.0, atol=64 * tol)
-    # the same on the streaming paths, whose running (maximum, sum) meets the mask first: masked columns incl. column 0 in a
-    # row of two sweeps (over 16384 elements per row), an odd-length long row (element by element) and a row split over work-groups
-    for rows, cols, use_ws in ((3, 20480, False), (2, 18001, False), (2, 65536, True)):
+    # the same on the streaming paths, whose running (maximum, sum) meets the mask first: masked columns incl. column 0 in
+    # rows of two sweeps, whole groups and not, and a row split over work-groups; and in rows held in registers (f32: two sweeps too)
+    for rows, cols, use_ws in sorted({(3, HELD // es + 4096, False), (2, HELD // es + 1617, False), (3, 20480, False), (2, 18001, False), (2, 65536, True)}):
         vals = O.encode(dt, O.normal(rows * cols, 45, 0, 1.0)).reshape(rows, cols)
         masked = [0, 1, 7, cols // 2, cols - 1]
         vals[:, masked] = O.encode(dt, np.array([-np.inf], dtype=np.float32))[0]
