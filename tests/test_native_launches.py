@@ -47,3 +47,53 @@ def test_what_the_extension_does_not_take_goes_by_ctypes():
             f(*args)
     with pytest.raises(TypeError):
         R.elementwise(R.make_elementwise_desc([("input", 0), "neg"], [(R.F32, 8, 1)], R.F32, 2, 8), ["x"], P)
+
+
+P2, P3, P4, P5, P6, P7, STREAM = (P * k for k in range(2, 9))
+
+
+def calls():
+    """every launch with integer pointers, all arguments different: what the wrapper hands on"""
+    gemm, body = R.make_desc(R.F16, 8, 8, 8, lda=3), R.make_elementwise_desc([("input", 0), ("input", 1), "add"], [(R.F32, 8, 1), (R.F32, 8, 1)], R.F32, 2, 8)
+    att = R.make_attention_desc(R.F16, 1, 1, 256, 64, 96)
+    return {"gemm": (gemm, P, P2, P3, P4, P5, P6, 77, STREAM), "fill": (R.F32, P, 2, 5, 4, 1.5, STREAM), "copy": (R.F32, P, 6, R.F16, P2, 9, 3, 7, STREAM),
+            "reduce": (R.BF16, P, 4, 6, 5, 1, 3, 1, P2, P3, 78, STREAM), "elementwise": (body, [P, P2], None, STREAM), "softmax": (R.F16, P, 3, P2, 8, 2, 4, 2.5, P3, P4, 79, STREAM),
+            "attention": (att, P, P2, P3, P4, P5, STREAM)}
+
+
+@pytest.mark.parametrize("name", sorted(calls()))
+def test_the_extension_carries_the_calls(name):
+    """the library's status comes back through the extension (these are refused), not the None that sends a call by ctypes; what only ctypes takes is left to it"""
+    f, args = getattr(R._bound(), name), calls()[name]
+    status = f(*args)
+    assert type(status) is int and status != 0, status
+    assert f(*args[:-1], ctypes.c_void_p(STREAM)) is None and f(*args[:-1]) is None
+
+
+def test_arguments_in_the_order_of_the_c_interface():
+    """functions that note what they are called with, in the library's place"""
+    native, L = R._bound(), R.lib()
+    names = ("gemm", "fill", "copy", "reduce", "elementwise", "softmax", "attention")
+    vp, i64, i32, size = ctypes.c_void_p, ctypes.c_int64, ctypes.c_int, ctypes.c_size_t
+    types = {"gemm": (vp,) * 7 + (size, vp), "fill": (i32, vp, i64, i64, i64, ctypes.c_double, vp), "copy": (i32, vp, i64, i32, vp, i64, i64, i64, vp),
+             "reduce": (i32, vp, i64, i64, i64, i32, i32, i32, vp, vp, size, vp), "elementwise": (vp, ctypes.POINTER(vp), vp, vp),
+             "softmax": (i32, vp, i64, vp, i64, i64, i64, ctypes.c_float, vp, vp, size, vp), "attention": (vp,) * 7}
+    bind = lambda at: native.bind(R.GemmDesc, R.ElementwiseDesc, R.AttentionDesc, *at)
+    seen = {}
+
+    def stub(name):
+        def record(*args):
+            seen[name] = [tuple(a[:2]) if name == "elementwise" and i == 1 else a for i, a in enumerate(args)]
+            return 40 + names.index(name)
+        return ctypes.CFUNCTYPE(i32, *types[name])(record)
+    stubs = [stub(n) for n in names]
+    try:
+        bind([ctypes.cast(s, vp).value for s in stubs])
+        for i, name in enumerate(names):
+            args = calls()[name]
+            assert getattr(native, name)(*args) == 40 + i
+            want = [ctypes.addressof(a) if isinstance(a, ctypes.Structure) else tuple(a) if isinstance(a, list) else a for a in args]
+            assert seen[name] == want, name
+    finally:
+        bind([ctypes.cast(getattr(L, "frisk_hip_" + n), vp).value for n in names])
+    assert "lda=3" in refused(R.gemm, R.make_desc(R.F16, 8, 8, 8, lda=3), P, P, P)
