@@ -43,6 +43,14 @@ def test_a_call_without_workspace_uses_none_of_the_plan_that_needs_one(recorded,
         assert status == 0 and len(launches) == 1 and "gemm_kernel" in launches[0][0] and launches[0][2] == 1, launches
 
 
+@pytest.mark.parametrize("slices,tile", [(7, "ELi256ELi256E"), (5, "ELi256ELi256E"), (4, None), (3, None), (0, None)])
+def test_slices_of_a_deep_product_that_the_workspace_does_not_hold_fall_away(recorded, slices, tile):
+    """35 tiles of 256x256 under 117 K tiles: five slices and more; below that line another tile takes the product"""
+    status, launches = recorded("gemm", "keep", R.F16, 1777, 1216, 7488, 0, 0, slices * 35 * 256 * 256 * 4)
+    assert status == 0 and ("ELi256ELi256E" in launches[0][0]) == bool(tile), launches
+    assert not tile or (launches[0][1] == 35 * slices and "tail_reduce_kernel" in launches[1][0]), launches
+
+
 @pytest.mark.parametrize("dt,M,N,K,transA,transB", [(R.E4M3, 2410, 865, 1222, 1, 0), (R.E4M3, 2511, 2241, 536, 1, 1), (R.BF16, 2321, 2172, 1978, 0, 1), (R.F16, 1524, 1901, 861, 0, 0),
                                                     (R.I8, 445, 2933, 150, 0, 0), (R.F16, 157, 23, 32, 1, 1)])
 def test_rows_off_16_bytes_are_staged_through_registers_without_a_workspace(recorded, dt, M, N, K, transA, transB):
