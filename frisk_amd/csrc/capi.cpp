@@ -732,26 +732,37 @@ static int follow_up(const std::vector<Variant>& list, const KernelEntry* k, con
 
 // 256x256 edge tiles in slices of K (their index), for 16- and 8-bit problems of a quarter of a round to two of 128x128 tiles whose K is deep and whose tiles are not split otherwise; -1 elsewhere.
 // Up to 256 tiles of 128x128, on those, one a CU, or on 64x128 tiles: such a CU takes 192 or 256 rows and columns a K tile, 0.5 us at the 60 to 70 bytes a nanosecond that it
-// pulls from the last-level cache, however many others are idle; a 256x256 tile takes half of that for the same work, and its slices fill the grid.  They cost a pass over 40 to 66 MB of
-// partial sums, 15 to 20 us, so it takes four slices and 117 K tiles and more, 164 in place of 64x128 tiles, two of which on a CU hide more; 8-bit types, whose partial sums are twice as much beside
-// their operands, 114 and 129.  The lines are where operands from the last-level cache gain too; from memory gains begin at three quarters of that K.  us before / so, from memory:
-// bf16 2043x1144x9024 NN 90.6 / 58.9, fp16 2114x1152x10752 NT 95.6 / 69.7, 1777x1024x13376 NT (64x128) 90.4 / 60.5, 1137x2880x11968 NT (4 slices) 110.7 / 87.3, bf16 454x4951x16128 NT 137.2 / 81.2, e4m3 1883x720x17920
-// NN 77.4 / 43.2; from the cache bf16 2880x768x13184 TN into fp32 sums 118.7 / 75.6, 768x3456x7424 TN 1.02 times as fast, 1152x2432x6720 NT 56.0 / 59.1, fp16 832x2176x9408 TN (64x128) 51.0 / 57.6, e4m3
-// 1856x1344x13312 NT 43.4 / 50.2, int8 1600x1152x16128 NN (64x128) 42.6 / 50.9; three slices 2095x1856x9472 NN 83.7 / 92.5.
+// pulls from the last-level cache, however many others are idle; a 256x256 tile takes half of that for the same work, and its slices fill the grid.  They cost 40 to 66 MB of
+// partial sums: the pass that adds them takes 9 to 13 us, and with the writing and what a slice pays beside its K tiles a call spends 25 to 30 us that do not grow with K (19 of 144 work-groups).
 // Beyond 256 of them, on edge tiles in one pass, which are a round that is not full or two: 2 or 3 slices of up to 112 tiles (above, where smaller tiles nearly fill their
-// round, 7 % on average are left).  us before / so, from memory: fp16 1019x5408x6912 NT 117.3 / 84.9, bf16 995x5616x8192 NN 140.4 / 98.5,
-// 1012x4640x5248 NT (3) 86.3 / 60.2, 2736x2320x7296 NT 106.8 / 98.5, int8 1921x2848x12800 NN 109.3 / 85.4, from the cache 1.00 to 1.28 times as fast; under the lines below bf16 1347x4288x5120 NN 72.8 / 77.0, int8
-// 1336x3680x6912 NT 49.7 / 55.2, 3022x2176x11392 NN 83.5 / 87.0, 1472x3328x6528 NN (3, cache) 42.8 / 51.3.
+// round, 7 % on average are left).  us before / so, from memory: bf16 2043x1144x9024 NN 90.6 / 58.9, fp16 2114x1152x10752 NT 95.6 / 69.7, 1777x1024x13376 NT (64x128) 90.4 / 60.5, 1137x2880x11968 NT (4
+// slices) 110.7 / 87.3, bf16 454x4951x16128 NT 137.2 / 81.2, e4m3 1883x720x17920 NN 77.4 / 43.2, fp16 1019x5408x6912 NT 117.3 / 84.9, bf16 995x5616x8192 NN 140.4 / 98.5, 1012x4640x5248 NT (3) 86.3 / 60.2,
+// int8 1921x2848x12800 NN 109.3 / 85.4.
+// Problems whose M and N are multiples of 256 are not here: they have split-K kernels of their own (2048x1280x8192 runs in 4 slices).
 // Error against 64 bits, fp32 C of fp16 1137x2880x11968: 6.9e-7 in one chain, 3.5e-7 in four.
+//
+// The least K of 16- and 8-bit types: where operands from memory, or the weights alone, gain (0.97 to 1.00 in a few of 150 measured at a line).  With both operands in the last-level cache, as in a
+// call repeated on the same buffers, a product at its line runs at 0.82 to 1.35 times its former speed, at 1.3 times that K at 0.92 to 1.42.  At the lines (and beyond), all from memory / the weights alone / all
+// from the cache, three to seven shapes in two layouts:
+struct DeepLine { int64_t k16, k8, k8_nk; };  // k8_nk: of 8-bit types against B [N][K]
+static constexpr DeepLine kDeepLines[] = {
+    {7488, 14592, 14592},   // five slices and more in place of 128x128 tiles: 16-bit 1.16 to 1.31, cache 0.93 to 1.09, then 0.98 to 1.15; 8-bit 1.17 to 1.38, cache 0.87 to 1.08, 0.94 to 1.13
+    {8192, 16384, 18432},   // four: 16-bit 1.01 to 1.20 / 0.98 to 1.12 / 0.89 to 1.04, at 9472 1.07 to 1.29 / 1.06 to 1.21 / 0.94 to 1.09; 8-bit NN 1.23 to 1.35 / 1.21 to 1.28 / 0.94 to 1.09; e4m3 NT at 16384
+                            // 0.97 to 1.08 / 0.96 to 1.03 / 0.84 to 0.89 (944x3472 62.5 us before, 65.1 so), at 18432 1.07 to 1.20 / 1.08 to 1.18 / 0.87 to 0.92
+    {10496, 16512, 16512},  // four and more in place of 64x128 tiles, two of which on a CU hide more: 16-bit 1.20 to 1.62 / 1.18 to 1.29 / 0.92 to 1.24; 8-bit 1.10 to 1.67 / 0.97 to 1.50 / 0.82 to 1.35
+    {4352, 8576, 8576},     // three beyond 256 tiles: 16-bit 1.03 to 1.32 / 1.03 to 1.11 / 0.92 to 0.98, at 4992 1.12 to 1.38 / 1.12 to 1.15 / 1.00 to 1.02; 8-bit 1.09 to 1.38, cache 0.92 to 1.11
+    {6144, 12032, 12032},   // two: 16-bit 1.02 to 1.35, cache 0.98 to 1.05; 8-bit 1.05 to 1.44, cache 0.93 to 1.17
+};
 static int deep_tile(const std::vector<Variant>& list, const KernelEntry* k, const frisk_gemm_desc* d, bool rows_aligned, size_t workspace) {
   const int64_t tiles = ((d->M + 127) / 128) * ((d->N + 127) / 128);
   const int64_t tiles256 = ((d->M + 255) / 256) * ((d->N + 255) / 256);
   const int es = elem_size(k->dtype);
   if (es == 4 || k->guard || !rows_aligned || k->wk > 1 || tiles < 64 || tiles > 512 || d->M <= 256 || d->N <= 256) return -1;
-  if (tiles > 256 ? !k->edge || k->splitk : k->bn != 128 || k->stages != 3) return -1;
+  if (tiles > 256 ? !k->edge || k->splitk || tiles256 > 112 : k->bn != 128 || k->stages != 3) return -1;
   auto deep = [&](int slices) {
-    if (tiles > 256) return slices >= 2 && tiles256 <= 112 && d->K >= (es == 2 ? (slices == 2 ? 6144 : 4352) : slices == 2 ? 12032 : 8576);
-    return slices >= 4 && d->K >= (es == 2 ? (k->bm == 64 ? 10496 : slices == 4 ? 8192 : 7488) : k->bm == 64 ? 16512 : slices == 4 ? 16384 : 14592);
+    if (slices < (tiles > 256 ? 2 : 4)) return false;
+    const DeepLine& line = kDeepLines[tiles > 256 ? (slices == 2 ? 4 : 3) : k->bm == 64 ? 2 : slices == 4 ? 1 : 0];
+    return d->K >= (es == 2 ? line.k16 : d->transB ? line.k8_nk : line.k8);
   };
   for (const Variant& v : list) {
     const KernelEntry* x = v.k;

@@ -28,8 +28,19 @@ def test_which_problems(dtype, transB, M, N, K, slices):
         assert not routed(p) or p.workspace_bytes == 0, where  # (whole grids of 256x256 tiles may be the planner's choice in one pass)
 
 
+@pytest.mark.parametrize("dtype,M,N,K,slices", [(O.E4M3, 944, 3472, 16384, (4, 0)), (O.E4M3, 944, 3472, 16256, (0, 0)), (O.E4M3, 944, 3472, 18304, (4, 0)), (O.E4M3, 944, 3472, 18432, (4, 4)),
+                                                (O.I8, 1333, 2200, 16256, (0, 0)), (O.I8, 1333, 2200, 18304, (4, 0)), (O.I8, 1333, 2200, 18432, (4, 4))])
+def test_four_slices_of_8_bit_types_by_the_layout_of_B(dtype, M, N, K, slices):
+    """against B [N][K], which the 128x128 tiles read faster, two K tiles in seven later: at 16384 it was slower from memory too"""
+    for transB in (0, 1):
+        ld = (N + 15) // 16 * 16
+        p = R.plan(R.make_desc(dtype, M, N, K, transB=transB, ldb=K if transB else ld, ldc=ld, dtype_out={O.I8: O.I32, O.E4M3: O.BF16}[dtype]))
+        got = p.workspace_bytes // (p.grid_x * p.grid_y * 256 * 256 * 4) if p.tile_m == p.tile_n == 256 else 0
+        assert got == slices[transB], (transB, R.kernel_names()[p.kernel_id], p.workspace_bytes)
+
+
 @pytest.mark.parametrize("dtype", [O.I8, O.E4M3])
-@pytest.mark.parametrize("M,N,K,sliced", [(1249, 1520, 16512, 1), (1152, 2368, 14592, 1), (1152, 2368, 14464, 0), (944, 3472, 16384, 1), (1921, 2848, 12032, 1), (1921, 2848, 11904, 0), (1196, 4320, 8576, 1)])
+@pytest.mark.parametrize("M,N,K,sliced", [(1249, 1520, 16512, 1), (1152, 2368, 14592, 1), (1152, 2368, 14464, 0), (944, 3472, 18432, 1), (1921, 2848, 12032, 1), (1921, 2848, 11904, 0), (1196, 4320, 8576, 1)])
 def test_which_problems_of_8_bit_types(dtype, M, N, K, sliced):
     for transB in (0, 1):
         ld = (N + 15) // 16 * 16
@@ -68,7 +79,7 @@ def test_their_results(hip, dtype, transA, transB):
 @pytest.mark.parametrize("transB", [0, 1])
 def test_their_results_in_8_bit_types(hip, dtype, transB):
     from test_edge_stores_gpu import check
-    for M, N, K in ((1249, 1520, 16512), (944, 3472, 16384), (1200, 4320, 8576), (1921, 2848, 12032)):
+    for M, N, K in ((1249, 1520, 16512), (944, 3472, 18432), (1200, 4320, 8576), (1921, 2848, 12032)):
         for out in ((O.I32, O.F32) if dtype == O.I8 else (O.BF16, O.F32)):
             p = hip.plan(hip.make_desc(dtype, M, N, K, dtype_out=out, transB=transB, ldc=(N + 15) // 8 * 8, clear_accum=False))
             assert p.tile_m == p.tile_n == 256 and p.workspace_bytes, (M, N, K, out)
