@@ -189,47 +189,49 @@ template <int KIND> __device__ __forceinline__ float wave_reduce(float v) {
 // along dim 1: work-group (x = row, y = column slice) reduces every gridDim.y-th run of THREADS 16-byte groups of one row, so that
 // the slices of a row read neighbouring memory at any time.
 // With gridDim.y == 1 the result goes to dst (combined with the old value unless clear), else to partial[y][row].
-// A row's last group, where it is not whole, is fetched with the elements before it that fill it up, which are left out: every load is 16 bytes of the row and
-// those of a lane are under way together (element by element behind the others: us so / now, f16 2490 x 2453 6.7 / 4.5, 10069 x 4946 19.7 / 16.0, 2490 x 4453 8.9 / 5.9, f32
-// 5531 x 1315 8.8 / 6.6).  512 lanes from 1025 groups on (f32 4000 x 8192 20.4 / 19.7, f16 4426 x 15161 27.7 / 26.8); views that the last-level cache may hold are read
-// through the caches (2490 x 4453 6.2 past them, 5.9 so; 10069 x 4946 16.0 past them, 16.8).  Past them, groups that straddle 128-byte lines are fetched twice: where rows start
-// off 16-byte boundaries the groups start at the first one, what lies before it being a group that overlaps like the last (bf16 6199 x 10825 30.7 at the rows' starts, 25.7 so).
-template <int DT, int KIND, int THREADS, bool STREAMED> __global__ void __launch_bounds__(THREADS)
+// A row's last group, where it is not whole, is fetched first, with the elements before it that fill it up, which are left out: every load is 16 bytes of the row, those of a lane are under way
+// together, and the loop over the whole groups knows nothing of it.  us element by element behind the loop / as a group of the loop / so, from memory: f16 3000 x 4095 9.7 / 7.3 / 7.3, 2490 x 2453
+// 7.0 / 5.4 / 5.1, 10069 x 4946 20.2 / 18.4 / 16.1, f32 5531 x 1315 10.0 / 7.8 / 7.6; rows of whole groups, f16 2177 x 8944 8.4 / 9.8 / 8.4, 4096 x 8192 11.5 / 12.4 / 11.6.
+// LOADS: rows on 16-byte boundaries are read past the caches (through them f16 4096 x 8192 from the last-level cache 11.2, 9.4 so, f32 3000 x 4096 8.8 / 6.8); off them, groups that straddle 128-byte lines would
+// be fetched twice: through the caches in views that the last-level cache may hold (f16 2490 x 4453 out of it 5.14 past them, 4.96 so; f32 5531 x 1315 6.5 / 6.3), and beyond, past them with the groups starting at a row's first
+// boundary, what lies before it being a group that overlaps like the last (bf16 6199 x 10825 27.4 at the rows' starts, 21.3 so).
+enum RowLoads { LOADS_CACHED, LOADS_PAST, LOADS_FROM_BOUNDARY };
+template <int DT, int KIND, int THREADS, int LOADS> __global__ void __launch_bounds__(THREADS)
 reduce_rows_kernel(const typename Elem<DT>::T* src, int64_t rows, int64_t cols, int64_t ld, int clear, typename Elem<DT>::T* dst, float* partial) {
   typedef typename Elem<DT>::T T;
   constexpr int G = 16 / sizeof(T), FLIGHT = 4;
-  const int64_t step = (int64_t)gridDim.y * THREADS;
+  const int64_t step = (int64_t)gridDim.y * THREADS, me = (int64_t)blockIdx.y * THREADS + threadIdx.x;
+  auto load = [](const T* at) {
+    if constexpr (LOADS == LOADS_CACHED) return *(const v4u_any*)at;
+    else return load16(at);
+  };
   __shared__ float wsum[THREADS / 64];
   for (int64_t r = blockIdx.x; r < rows; r += gridDim.x) {
     float acc = Op<KIND>::id();
     const T* row = src + r * ld;
-    // groups 0 .. full - 1 from element `head` on, then the one that ends with the row, then the one it starts with
-    const int64_t head = STREAMED ? ((0 - (uintptr_t)row) & 15) / sizeof(T) : 0, full = (cols - head) / G, tail = cols - head - full * G;
-    const int64_t groups = full + (tail > 0) + (STREAMED && head > 0);
+    // groups 0 .. full - 1 from element `head` on, then the one that ends with the row, then the one it starts with: the last ones of their lanes (slices are a power of two)
+    const int64_t head = LOADS == LOADS_FROM_BOUNDARY ? ((0 - (uintptr_t)row) & 15) / sizeof(T) : 0, full = (cols - head) / G, tail = cols - head - full * G;
+    const bool ends = tail > 0 && (full & (step - 1)) == me, starts = head > 0 && ((full + (tail > 0)) & (step - 1)) == me;
+    T edge[G];
+    if (ends || starts) *(v4u*)edge = load(row + (ends ? cols - G : 0));
     // four groups of a lane under way together, combined in their order (one after the other 98 x 12807 bf16 took 6.2 us, 8192 x 8192 f16 22.9)
-    for (int64_t g = (int64_t)blockIdx.y * THREADS + threadIdx.x; g < groups; g += FLIGHT * step) {
+    for (int64_t g = me; g < full; g += FLIGHT * step) {
       T in[FLIGHT][G];
 #pragma unroll
-      for (int u = 0; u < FLIGHT; ++u) {
-        const int64_t k = g + u * step, at = k < full ? head + k * G : (!STREAMED || (tail > 0 && k == full) ? cols - G : 0);
-        if (k >= groups) continue;
-        if constexpr (STREAMED) *(v4u*)in[u] = load16(row + at);
-        else *(v4u*)in[u] = *(const v4u_any*)(row + at);
-      }
+      for (int u = 0; u < FLIGHT; ++u)
+        if (g + u * step < full) *(v4u*)in[u] = load(row + head + (g + u * step) * G);
 #pragma unroll
       for (int u = 0; u < FLIGHT; ++u) {
-        const int64_t k = g + u * step;
-        if (k < full) {
+        if (g + u * step >= full) continue;
 #pragma unroll
-          for (int e = 0; e < G; ++e) acc = Op<KIND>::f(acc, Elem<DT>::load(in[u][e]));
-        } else if (k < groups) {
-          const bool last = !STREAMED || (tail > 0 && k == full);
-          const int lo = last ? G - (int)tail : 0, hi = last ? G : (int)head;  // its own elements
-#pragma unroll
-          for (int e = 0; e < G; ++e)
-            if (e >= lo && e < hi) acc = Op<KIND>::f(acc, Elem<DT>::load(in[u][e]));
-        }
+        for (int e = 0; e < G; ++e) acc = Op<KIND>::f(acc, Elem<DT>::load(in[u][e]));
       }
+    }
+    if (ends || starts) {
+      const int lo = ends ? G - (int)tail : 0, hi = ends ? G : (int)head;  // its own elements
+#pragma unroll
+      for (int e = 0; e < G; ++e)
+        if (e >= lo && e < hi) acc = Op<KIND>::f(acc, Elem<DT>::load(edge[e]));
     }
     acc = wave_reduce<KIND>(acc);
     if ((threadIdx.x & 63) == 0) wsum[threadIdx.x >> 6] = acc;
@@ -247,7 +249,11 @@ reduce_rows_kernel(const typename Elem<DT>::T* src, int64_t rows, int64_t cols, 
 // along dim 1, rows of at most 256 groups of 16 bytes: 2^lanes_log2 <= 64 lanes of one wave share a row, each taking up to
 // NPT groups, and combine by shuffles; a work-group holds 256 >> lanes_log2 rows and takes 4 / NPT such sets of rows per
 // step, so that every lane has four loads in flight before the first is used.
-template <int DT, int KIND, int NPT> __global__ void __launch_bounds__(256)
+// TAIL: rows of whole groups (with the code for another last group f16 20000 x 1000 10.5 us out of the last-level cache, 9.2 so, bf16 5878 x 864 5.8 from memory, 5.4 so); with a last group that is
+// fetched with the elements before it that fill it up, which count as nothing (element by element behind the others / behind a branch / so, from memory: bf16 14242 x 790 10.0 / 10.3 / 7.2, f16 20000 x 1003
+// 15.5 / 12.2 / 11.7, 16384 x 2047 20.5 / 16.9 / 15.2, 100000 x 27 7.0 / 5.7 / 5.4); of less than a group, element by element.
+enum RowTail { TAIL_WHOLE, TAIL_PART, TAIL_NARROW };
+template <int DT, int KIND, int NPT, int TAIL> __global__ void __launch_bounds__(256)
 reduce_short_rows_kernel(const typename Elem<DT>::T* src, int64_t rows, int64_t cols, int64_t ld, int clear, typename Elem<DT>::T* dst, int lanes_log2) {
   typedef typename Elem<DT>::T T;
   constexpr int G = 16 / sizeof(T), SETS = 4 / NPT;
@@ -255,19 +261,20 @@ reduce_short_rows_kernel(const typename Elem<DT>::T* src, int64_t rows, int64_t 
   const int64_t blocks = (rows + rows_per_set * SETS - 1) / (rows_per_set * SETS);
   for (int64_t rb = blockIdx.x; rb < blocks; rb += gridDim.x) {
     T in[SETS][NPT][G];
-    const bool narrow = cols < G;  // rows of less than a group go element by element
+    bool inside[SETS][NPT];
 #pragma unroll
     for (int t = 0; t < SETS; ++t) {
       const int64_t r = (rb * SETS + t) * rows_per_set + (threadIdx.x >> lanes_log2);
 #pragma unroll
       for (int q = 0; q < NPT; ++q) {
-        const int64_t c0 = (int64_t)(q * lanes + lane) * G;
-        if (r >= rows || c0 >= cols) continue;
-        // (a last group that is not whole with the elements before it that fill it up)
-        if (!narrow) *(v4u*)in[t][q] = load16(src + r * ld + (c0 + G <= cols ? c0 : cols - G));
-        else
+        const int c0 = (q * lanes + lane) * G;
+        inside[t][q] = r < rows && c0 < (int)cols;
+        if (!inside[t][q]) continue;
+        const T* at = src + r * ld;
+        if constexpr (TAIL == TAIL_NARROW) {
 #pragma unroll
-          for (int e = 0; e < G; ++e) in[t][q][e] = src[r * ld + (e < cols ? e : 0)];
+          for (int e = 0; e < G; ++e) in[t][q][e] = at[e < (int)cols ? e : 0];
+        } else *(v4u*)in[t][q] = load16(at + (TAIL == TAIL_WHOLE || c0 + G <= (int)cols ? c0 : (int)cols - G));
       }
     }
 #pragma unroll
@@ -277,16 +284,11 @@ reduce_short_rows_kernel(const typename Elem<DT>::T* src, int64_t rows, int64_t 
       float acc = Op<KIND>::id();
 #pragma unroll
       for (int q = 0; q < NPT; ++q) {
-        const int64_t c0 = (int64_t)(q * lanes + lane) * G;
-        if (live && c0 + G <= cols) {
+        if (!inside[t][q]) continue;
+        const int past = (q * lanes + lane + 1) * G - (int)cols;
+        const int lo = TAIL == TAIL_PART && past > 0 ? past : 0, hi = TAIL == TAIL_NARROW ? (int)cols : G;
 #pragma unroll
-          for (int e = 0; e < G; ++e) acc = Op<KIND>::f(acc, Elem<DT>::load(in[t][q][e]));
-        } else if (live && c0 < cols) {
-          const int lo = narrow ? 0 : (int)(c0 + G - cols), hi = narrow ? (int)cols : G;
-#pragma unroll
-          for (int e = 0; e < G; ++e)
-            if (e >= lo && e < hi) acc = Op<KIND>::f(acc, Elem<DT>::load(in[t][q][e]));
-        }
+        for (int e = 0; e < G; ++e) acc = Op<KIND>::f(acc, TAIL == TAIL_WHOLE || (e >= lo && e < hi) ? Elem<DT>::load(in[t][q][e]) : Op<KIND>::id());
       }
       for (int off = lanes >> 1; off >= 1; off >>= 1) acc = Op<KIND>::f(acc, __shfl_xor(acc, off, 64));
       if (live && lane == 0) dst[r] = Elem<DT>::store(clear ? acc : Op<KIND>::f(Elem<DT>::load(dst[r]), acc));
@@ -531,16 +533,26 @@ template <int DT, int KIND> hipError_t reduce_t(const void* src, int64_t rows, i
       while (lanes_log2 < 6 && (int64_t(1) << lanes_log2) < gpr) ++lanes_log2;
       const int64_t rows_per_step = (256 >> lanes_log2) * (gpr <= 64 ? 4 : (gpr <= 128 ? 2 : 1)), blocks = (rows + rows_per_step - 1) / rows_per_step;
       const dim3 grid((unsigned)(blocks < kMaxGrid ? blocks : kMaxGrid));
-      if (gpr <= 64) hipLaunchKernelGGL((reduce_short_rows_kernel<DT, KIND, 1>), grid, dim3(256), 0, s, (const T*)src, rows, cols, ld, clear, (T*)dst, lanes_log2);
-      else if (gpr <= 128) hipLaunchKernelGGL((reduce_short_rows_kernel<DT, KIND, 2>), grid, dim3(256), 0, s, (const T*)src, rows, cols, ld, clear, (T*)dst, lanes_log2);
-      else hipLaunchKernelGGL((reduce_short_rows_kernel<DT, KIND, 4>), grid, dim3(256), 0, s, (const T*)src, rows, cols, ld, clear, (T*)dst, lanes_log2);
+      auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, (const T*)src, rows, cols, ld, clear, (T*)dst, lanes_log2); };
+      const bool whole = cols % G == 0;
+#define FRISK_REDUCE_SHORT(NPT) { if (whole) launch(reduce_short_rows_kernel<DT, KIND, NPT, TAIL_WHOLE>); else launch(reduce_short_rows_kernel<DT, KIND, NPT, TAIL_PART>); }
+      if (cols < G) launch(reduce_short_rows_kernel<DT, KIND, 1, TAIL_NARROW>);
+      else if (gpr <= 64) FRISK_REDUCE_SHORT(1)
+      else if (gpr <= 128) FRISK_REDUCE_SHORT(2)
+      else FRISK_REDUCE_SHORT(4)
+#undef FRISK_REDUCE_SHORT
     } else {
       const dim3 grid((unsigned)(rows < kMaxGrid ? rows : kMaxGrid), (unsigned)slices);
-      const bool streamed = rows * cols * (int64_t)sizeof(T) > (int64_t)64 << 20;
+      const bool aligned = (((uintptr_t)src | ld * sizeof(T)) & 15) == 0, large = rows * cols * (int64_t)sizeof(T) > (int64_t)64 << 20;
+      // 512 lanes where they have three groups each or the rows are few (us 256 / 512 lanes: f32 4000 x 8192 18.9 / 18.0, f16 2048 x 16384 11.7 / 11.5, bf16 1000 x 9000 5.6 / 5.2; but 1126 and
+      // 1354 groups of more rows, f32 4111 x 4501 10.8 / 11.9, bf16 6199 x 10825 21.3 / 22.1)
+      const bool wide = gpr > 1536 || (gpr > 1024 && rows <= 1024);
       auto launch = [&](auto kernel, int threads) { hipLaunchKernelGGL(kernel, grid, dim3(threads), 0, s, (const T*)src, rows, cols, ld, clear, (T*)dst, partial); };
-      if (gpr > 1024) { if (streamed) launch(reduce_rows_kernel<DT, KIND, 512, true>, 512); else launch(reduce_rows_kernel<DT, KIND, 512, false>, 512); }
-      else if (streamed) launch(reduce_rows_kernel<DT, KIND, 256, true>, 256);
-      else launch(reduce_rows_kernel<DT, KIND, 256, false>, 256);
+#define FRISK_REDUCE_ROWS(LOADS) { if (wide) launch(reduce_rows_kernel<DT, KIND, 512, LOADS>, 512); else launch(reduce_rows_kernel<DT, KIND, 256, LOADS>, 256); }
+      if (aligned) FRISK_REDUCE_ROWS(LOADS_PAST)
+      else if (large) FRISK_REDUCE_ROWS(LOADS_FROM_BOUNDARY)
+      else FRISK_REDUCE_ROWS(LOADS_CACHED)
+#undef FRISK_REDUCE_ROWS
     }
   } else if (tall) {
     int lanes_log2 = 0;

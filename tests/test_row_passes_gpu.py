@@ -220,3 +220,27 @@ def test_columns_of_long_rows_in_one_launch_and_beyond(hip, dt, tdt):
                     hip.reduce(dt, x.data_ptr(), rows, cols, ld, 0, "add", False, d.data_ptr(), ws.data_ptr() if with_ws else None, need if with_ws else 0, torch.cuda.current_stream().cuda_stream)
                     torch.cuda.synchronize()
                     assert torch.equal(d[:cols].float(), x[:, :cols].float().sum(0) + 7) and float(d[cols]) == 7.0, (rows, cols, ld, with_ws)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt,tdt", [(O.F32, "float32"), (O.F16, "float16"), (O.BF16, "bfloat16")])
+def test_row_reductions_on_and_off_boundaries(hip, dt, tdt):
+    """rows of whole groups and not, on 16-byte boundaries and off them, on 256 and 512 lanes and on lanes of a wave with one, two and four groups each; what lies between the rows is no number.  Whole
+    numbers whose sums every type holds: the same bits in any order"""
+    import torch
+    tdt = getattr(torch, tdt)
+    G = 16 // torch.empty(0, dtype=tdt).element_size()
+    g = torch.Generator(device="cuda").manual_seed(11)
+    stream = torch.cuda.current_stream().cuda_stream
+    for rows, cols in ((1030, 1300 * G), (1030, 1300 * G + 1), (1030, 1536 * G - 1), (1030, 1537 * G), (1024, 1025 * G), (1030, 1024 * G), (1030, 257 * G - 1), (2000, 256 * G), (2000, 129 * G), (2000, 128 * G - 1), (2000, 65 * G - 1),
+                       (2000, 64 * G), (5000, 3 * G), (5000, 3 * G + 1), (5000, G), (5000, G - 1)):
+        for ld, shift in ((-(-cols // G) * G, 0), (-(-cols // G) * G + G, 0), (cols + 1, 0), (-(-cols // G) * G, 1)):
+            base = torch.full((shift + rows * ld,), float("nan"), device="cuda", dtype=tdt)
+            x = base[shift:].view(rows, ld)
+            x[:, :cols] = (torch.rand(rows, cols, device="cuda", generator=g) < 0.06).to(tdt) * (2 * torch.randint(0, 2, (rows, cols), device="cuda", generator=g) - 1).to(tdt)
+            for kind in ("add", "min"):
+                d = torch.full((rows + 1,), 7.0, device="cuda", dtype=tdt)
+                hip.reduce(dt, x.data_ptr(), rows, cols, ld, 1, kind, True, d.data_ptr(), None, 0, stream)
+                torch.cuda.synchronize()
+                want = x[:, :cols].float().sum(1) if kind == "add" else x[:, :cols].float().amin(1)
+                assert torch.equal(d[:rows].float(), want) and float(d[rows]) == 7.0, (rows, cols, ld, shift, kind)
