@@ -108,11 +108,13 @@ template <bool SUM, int THREADS> __device__ __forceinline__ float block_all(floa
 // elements before it that fill it up (which enter the sum as their own lane's): every access is 16 bytes of the row and all loads of a row are under way
 // together.  Fetched element by element behind the others, that group held up every row by a memory latency: us before / now, f16 10069 x 4946 49.5 / 33.7,
 // 2490 x 2453 11.8 / 6.9, 870 x 16370 20.0 / 10.4 (with 512 lanes: 12.5 with 256), f32 5531 x 1315 17.6 / 10.6, 394 x 9229 (two launches before) 11.9 / 6.9;
-// rows that are whole groups gain by the shorter reductions, f16 8192 x 8192 47.3 / 43.5, which a plain copy takes 39 for.
-// STREAMED, for views that the last-level cache does not hold beside their result: the loads pass the caches by (8192 x 8192 f16 43.5, 45.0 without; but 870 x 16370
-// 10.4 without, 11.9 with), and where rows start off 16-byte boundaries the groups start at the first boundary, what lies before it being a group that overlaps
-// like the last one: stores that cross lines half way cost memory traffic (4426 x 15161 f16 54.9 at the rows' starts, 47.5 so; out of the cache 7.1 either way, 545 x 12163).
-template <int DT, int NPT, int THREADS, bool STREAMED>
+// rows that are whole groups gain by the shorter reductions and what HELD says, f16 8192 x 8192 45.3 / 38.9, which a plain copy takes 39 for.
+// HELD: rows of whole groups on 16-byte boundaries know of no other group.  On 128-byte lines and up to 56 MiB they are read past the caches (f16 4096 x 4096 out of the last-level cache 10.6 us through
+// the caches, 9.0 past them, f32 3000 x 4096 15.5 / 13.4), beyond through them (4096 x 8192 from memory 20.6 us, 23.2 past them, 8192 x 8192 38.9 / 42.7).  Others are read through the caches (870 x 16370 10.4,
+// 11.9 past them), and past them in views that the last-level cache does not hold beside their result; there, where rows start off 16-byte boundaries, the groups start at the first boundary, what lies
+// before it being a group that overlaps like the last one: stores that cross lines half way cost memory traffic (4426 x 15161 f16 54.9 at the rows' starts, 47.5 so; out of the cache 7.1 either way, 545 x 12163).
+enum HeldRows { HELD_WHOLE_PAST, HELD_WHOLE, HELD_CACHED, HELD_FROM_BOUNDARY };
+template <int DT, int NPT, int THREADS, int HELD>
 __global__ void __launch_bounds__(THREADS) softmax_held_rows_kernel(const typename SElem<DT>::T* src, int64_t sld, typename SElem<DT>::T* dst, int64_t dld, int64_t rows,
                                                                     int cols, float c, float* lse) {
   typedef typename SElem<DT>::T T;
@@ -122,8 +124,8 @@ __global__ void __launch_bounds__(THREADS) softmax_held_rows_kernel(const typena
     const T* x = src + r * sld;
     T* y = dst + r * dld;
     // groups 0 .. full - 1 from element `head` on, then the one that ends with the row, then the one it starts with
-    const int head = STREAMED ? (int)((0 - (uintptr_t)y) & 15) / (int)sizeof(T) : 0;
-    const int full = (cols - head) / G, body = head + full * G, tail = cols - body, groups = full + (tail > 0) + (head > 0);
+    const int head = HELD == HELD_FROM_BOUNDARY ? (int)((0 - (uintptr_t)y) & 15) / (int)sizeof(T) : 0;
+    const int full = (cols - head) / G, body = head + full * G, tail = HELD <= HELD_WHOLE ? 0 : cols - body, groups = full + (tail > 0) + (head > 0);
     T in[NPT][G];
     int at[NPT];
 #pragma unroll
@@ -131,8 +133,8 @@ __global__ void __launch_bounds__(THREADS) softmax_held_rows_kernel(const typena
       const int g = q * THREADS + (int)threadIdx.x;
       at[q] = g < full ? head + g * G : (tail > 0 && g == full ? cols - G : 0);
       if (g < groups) {
-        if constexpr (STREAMED) *(v4u*)in[q] = __builtin_nontemporal_load((const v4u_any*)(x + at[q]));
-        else *(v4u*)in[q] = *(const v4u_any*)(x + at[q]);
+        if constexpr (HELD == HELD_CACHED || HELD == HELD_WHOLE) *(v4u*)in[q] = *(const v4u_any*)(x + at[q]);
+        else *(v4u*)in[q] = __builtin_nontemporal_load((const v4u_any*)(x + at[q]));
       }
     }
     float v[NPT][G], mx = -INFINITY;
@@ -203,9 +205,12 @@ __global__ void __launch_bounds__(256) softmax_rows_kernel(const typename SElem<
 
 // Rows of at most 256 groups of 16 bytes: 2^lanes_log2 <= 64 lanes of one wave share a row, each holding up to NPT groups in
 // registers, and combine maximum and sum by shuffles (no LDS, no barrier); a work-group holds 256 >> lanes_log2 rows.
-template <int DT, int NPT>
+// TAIL: rows of whole groups (with the code for another last group, of any length, f16 32768 x 512 17.7 us, 14.4 so, 100000 x 64 from memory 8.2 / 7.1, 8192 x 1024 8.0 / 6.5); with a last
+// group that is read and written with the elements before it, which are another lane's (bf16 14242 x 790 beside the code for less than one 11.9 us, 10.5 so); of less than a group, element by element.
+enum RowTail { TAIL_WHOLE, TAIL_PART, TAIL_NARROW };
+template <int DT, int NPT, int TAIL>
 __global__ void __launch_bounds__(256) softmax_short_rows_kernel(const typename SElem<DT>::T* src, int64_t sld, typename SElem<DT>::T* dst, int64_t dld, int64_t rows,
-                                                                 int64_t cols, float c, float* lse, int lanes_log2) {
+                                                                 int cols, float c, float* lse, int lanes_log2) {
   typedef typename SElem<DT>::T T;
   constexpr int G = 16 / (int)sizeof(T);
   const int lanes = 1 << lanes_log2, lane = threadIdx.x & (lanes - 1), rows_per_group = 256 >> lanes_log2;
@@ -217,31 +222,26 @@ __global__ void __launch_bounds__(256) softmax_short_rows_kernel(const typename 
     T* y = dst + r * dld;
     float v[NPT][G];
     T in[NPT][G];
-    // a last group that is not whole is read and written with the elements before it, `twice` of them, which are another lane's; a row of less
-    // than a group goes element by element
-    const bool narrow = cols < G;
-    int64_t at[NPT];
-    int twice[NPT];
+    int at[NPT], twice[NPT];  // where a group starts, and how many of its elements are another lane's
     bool inside[NPT];
 #pragma unroll
     for (int q = 0; q < NPT; ++q) {
-      const int64_t c0 = (int64_t)(q * lanes + lane) * G;
+      const int c0 = (q * lanes + lane) * G;
       inside[q] = live && c0 < cols;
-      twice[q] = !narrow && c0 + G > cols ? (int)(c0 + G - cols) : 0;
+      twice[q] = TAIL == TAIL_PART && c0 + G > cols ? c0 + G - cols : 0;
       at[q] = c0 - twice[q];
-      if (inside[q]) {
-        if (!narrow) *(v4u*)in[q] = __builtin_nontemporal_load((const v4u_any*)(x + at[q]));
-        else
+      if (!inside[q]) continue;
+      if constexpr (TAIL == TAIL_NARROW) {
 #pragma unroll
-          for (int e = 0; e < G; ++e) in[q][e] = x[e < cols ? e : 0];
-      }
+        for (int e = 0; e < G; ++e) in[q][e] = x[e < cols ? e : 0];
+      } else *(v4u*)in[q] = __builtin_nontemporal_load((const v4u_any*)(x + at[q]));
     }
     float mx = -INFINITY;
 #pragma unroll
     for (int q = 0; q < NPT; ++q)
 #pragma unroll
       for (int e = 0; e < G; ++e) {
-        v[q][e] = inside[q] && (!narrow || e < cols) ? SElem<DT>::load(in[q][e]) * c : -INFINITY;
+        v[q][e] = inside[q] && (TAIL != TAIL_NARROW || e < cols) ? SElem<DT>::load(in[q][e]) * c : -INFINITY;
         mx = fmaxf(mx, v[q][e]);
       }
     for (int off = lanes >> 1; off >= 1; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
@@ -251,7 +251,7 @@ __global__ void __launch_bounds__(256) softmax_short_rows_kernel(const typename 
 #pragma unroll
       for (int e = 0; e < G; ++e) {
         v[q][e] = __builtin_amdgcn_exp2f(v[q][e] - mx);
-        sum += e >= twice[q] ? v[q][e] : 0.f;
+        sum += TAIL != TAIL_PART || e >= twice[q] ? v[q][e] : 0.f;
       }
     for (int off = lanes >> 1; off >= 1; off >>= 1) sum += __shfl_xor(sum, off, 64);
     const float inv = 1.f / sum;
@@ -261,11 +261,11 @@ __global__ void __launch_bounds__(256) softmax_short_rows_kernel(const typename 
       T out[G];
 #pragma unroll
       for (int e = 0; e < G; ++e) out[e] = SElem<DT>::store(v[q][e] * inv);
-      if (!narrow) __builtin_nontemporal_store(*(const v4u*)out, (v4u_any*)(y + at[q]));
-      else
+      if constexpr (TAIL == TAIL_NARROW) {
 #pragma unroll
         for (int e = 0; e < G; ++e)
           if (e < cols) y[e] = out[e];
+      } else __builtin_nontemporal_store(*(const v4u*)out, (v4u_any*)(y + at[q]));
     }
     if (lse && live && lane == 0) lse[r] = mx + __builtin_amdgcn_logf(sum);
   }
@@ -321,9 +321,9 @@ __global__ void __launch_bounds__(256) softmax_split_write_kernel(const typename
   if (lse && blockIdx.y == 0 && threadIdx.x == 0) lse[blockIdx.x] = ref;
 }
 
-// groups of a row that a work-group holds, and bytes of a view from which on its rows stream past the caches (with the result they are most of the 256 MiB of
-// the last-level cache)
-constexpr int64_t kHeldGroups = 4096, kStreamedBytes = (int64_t)112 << 20;
+// groups of a row that a work-group holds, bytes of a view from which on its rows stream past the caches (with the result they are most of the 256 MiB of
+// the last-level cache), and bytes up to which rows of whole groups on lines do
+constexpr int64_t kHeldGroups = 4096, kStreamedBytes = (int64_t)112 << 20, kPastBytes = (int64_t)56 << 20;
 
 template <int DT> hipError_t launch_typed(const void* src, int64_t sld, void* dst, int64_t dld, int64_t rows, int64_t cols, float c, float* lse, float* partial,
                                           int slices, hipStream_t s) {
@@ -344,17 +344,29 @@ template <int DT> hipError_t launch_typed(const void* src, int64_t sld, void* ds
     while (lanes_log2 < 6 && (int64_t(1) << lanes_log2) < groups) ++lanes_log2;
     const int64_t rows_per_group = 256 >> lanes_log2, blocks = (rows + rows_per_group - 1) / rows_per_group;
     const dim3 sgrid((unsigned)(blocks < (1 << 22) ? blocks : (1 << 22)));
-    if (groups <= 64) hipLaunchKernelGGL((softmax_short_rows_kernel<DT, 1>), sgrid, dim3(256), 0, s, x, sld, y, dld, rows, cols, c, lse, lanes_log2);
-    else if (groups <= 128) hipLaunchKernelGGL((softmax_short_rows_kernel<DT, 2>), sgrid, dim3(256), 0, s, x, sld, y, dld, rows, cols, c, lse, lanes_log2);
-    else hipLaunchKernelGGL((softmax_short_rows_kernel<DT, 4>), sgrid, dim3(256), 0, s, x, sld, y, dld, rows, cols, c, lse, lanes_log2);
+    auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, sgrid, dim3(256), 0, s, x, sld, y, dld, rows, (int)cols, c, lse, lanes_log2); };
+    const bool whole = cols % G == 0;
+#define FRISK_SOFTMAX_SHORT(NPT) { if (whole) launch(softmax_short_rows_kernel<DT, NPT, TAIL_WHOLE>); else launch(softmax_short_rows_kernel<DT, NPT, TAIL_PART>); }
+    if (cols < G) launch(softmax_short_rows_kernel<DT, 1, TAIL_NARROW>);
+    else if (groups <= 64) FRISK_SOFTMAX_SHORT(1)
+    else if (groups <= 128) FRISK_SOFTMAX_SHORT(2)
+    else FRISK_SOFTMAX_SHORT(4)
+#undef FRISK_SOFTMAX_SHORT
     return hipGetLastError();
   }
   if (groups <= kHeldGroups) {
-    const bool streamed = rows * cols * (int64_t)sizeof(T) > kStreamedBytes;
-    const int64_t most = groups + (streamed && (((uintptr_t)y | dld * sizeof(T)) & 15) ? 1 : 0);  // a row that starts off a boundary may have a group more
+    const int64_t bytes = rows * cols * (int64_t)sizeof(T);
+    const uintptr_t starts = (uintptr_t)x | (uintptr_t)y | sld * sizeof(T) | dld * sizeof(T);
+    const bool whole = cols % G == 0 && starts % 16 == 0, past = whole && starts % 128 == 0 && bytes <= kPastBytes, large = !whole && bytes > kStreamedBytes;
+    const int64_t most = groups + (large ? 1 : 0);  // a row that starts off a boundary may have a group more
     auto launch = [&](auto kernel, int threads) { hipLaunchKernelGGL(kernel, dim3(grid), dim3(threads), 0, s, x, sld, y, dld, rows, (int)cols, c, lse); };
 #define FRISK_SOFTMAX_HELD(NPT, THREADS) \
-  if (most <= NPT * THREADS) { if (streamed) launch(softmax_held_rows_kernel<DT, NPT, THREADS, true>, THREADS); else launch(softmax_held_rows_kernel<DT, NPT, THREADS, false>, THREADS); }
+  if (most <= NPT * THREADS) {                                                                          \
+    if (past) launch(softmax_held_rows_kernel<DT, NPT, THREADS, HELD_WHOLE_PAST>, THREADS);             \
+    else if (whole) launch(softmax_held_rows_kernel<DT, NPT, THREADS, HELD_WHOLE>, THREADS);            \
+    else if (large) launch(softmax_held_rows_kernel<DT, NPT, THREADS, HELD_FROM_BOUNDARY>, THREADS);    \
+    else launch(softmax_held_rows_kernel<DT, NPT, THREADS, HELD_CACHED>, THREADS);                      \
+  }
     FRISK_SOFTMAX_HELD(2, 256)
     else FRISK_SOFTMAX_HELD(3, 256)
     else FRISK_SOFTMAX_HELD(2, 512)

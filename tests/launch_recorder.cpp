@@ -5,6 +5,7 @@
 //   launch_recorder kept
 //   launch_recorder block <dtype> <rows> <cols> <operands: m = rows x cols, r = one value a row, s = that times a constant, c = one a column>
 //   launch_recorder reduce <dtype> <rows> <cols> <leading dimension> <dim> <bytes from the source to a 256-byte boundary> <workspace: 1 what the library asks for, 0 none>
+//   launch_recorder softmax <dtype> <rows> <cols> <leading dimension> <bytes from either matrix to a 256-byte boundary>
 #include <hip/hip_runtime_api.h>
 #include <algorithm>
 #include <chrono>
@@ -142,11 +143,19 @@ static int reduce(char** arg) {
   return 0;
 }
 
+static int softmax(char** arg) {
+  const int dtype = std::atoi(arg[0]);
+  const int64_t rows = std::atoll(arg[1]), cols = std::atoll(arg[2]), ld = std::atoll(arg[3]);
+  std::printf("status %d\n", frisk_hip_softmax(dtype, (char*)at(0) + std::atoi(arg[4]), ld, (char*)at(1) + std::atoi(arg[4]), ld, rows, cols, 1.f, nullptr, nullptr, 0, nullptr));
+  return 0;
+}
+
 int main(int argc, char** argv) {
   const std::string what = argc > 1 ? argv[1] : "";
   if (what == "gemm" && argc == 10) return gemm(argv + 2);
   if (what == "kept") return kept();
   if (what == "reduce" && argc == 9) return reduce(argv + 2);
+  if (what == "softmax" && argc == 7) return softmax(argv + 2);
   if (what == "block" && argc == 6) return block(argv + 2);
   return 2;
 }

@@ -140,3 +140,20 @@ def test_row_reductions_by_what_their_rows_are(recorded, dt, rows, cols, ld, off
     which, a, b = kernel.split()
     got = re.search(r"reduce_short_rows_kernelILi%dELi0ELi(\d+)ELi(\d+)E" % dt if which == "short" else r"reduce_rows_kernelILi%dELi0ELi(\d+)ELi(\d+)E" % dt, name)
     assert status == 0 and got and got.groups() == (a, b), name
+
+
+@pytest.mark.parametrize("dt,rows,cols,ld,off,kernel", [
+    # <groups a lane, rows of whole groups 0 / a part 1 / less than a group 2>
+    (R.F16, 32768, 512, 512, 0, "short 1 0"), (R.F16, 100000, 27, 27, 0, "short 1 1"), (R.F16, 100000, 7, 8, 0, "short 1 2"), (R.F32, 300000, 3, 3, 0, "short 1 2"), (R.F16, 8192, 1024, 1025, 2, "short 2 0"),
+    (R.BF16, 14242, 790, 790, 0, "short 2 1"), (R.F32, 8192, 1024, 1024, 0, "short 4 0"), (R.F32, 8192, 1023, 1024, 0, "short 4 1"),
+    # <groups a lane, lanes, whole groups on lines past the caches 0 / whole groups 1 / any through them 2 / any past them from a row's first boundary on 3>
+    (R.F16, 4096, 4096, 4096, 0, "held 2 256 0"), (R.F32, 3000, 4096, 4096, 0, "held 2 512 0"), (R.F16, 3584, 8192, 8192, 0, "held 2 512 0"), (R.F16, 3585, 8192, 8192, 0, "held 2 512 1"), (R.F16, 8192, 8192, 8192, 0, "held 2 512 1"),
+    (R.F16, 4096, 4000, 4000, 0, "held 2 256 1"), (R.F16, 4096, 4096, 4096, 16, "held 2 256 1"), (R.F16, 4096, 4096, 4096, 2, "held 2 256 2"), (R.F16, 4096, 4095, 4096, 0, "held 2 256 2"), (R.F16, 8192, 8192, 8193, 0, "held 3 512 3"),
+    (R.F16, 870, 16370, 16370, 0, "held 4 512 2"), (R.F16, 4426, 15161, 15161, 0, "held 4 512 3"), (R.F16, 64, 32768, 32768, 0, "held 9 512 0")])
+def test_softmax_by_what_its_rows_are(recorded, dt, rows, cols, ld, off, kernel):
+    """rows of whole groups on kernels that know of no others; past the caches where that was the faster way"""
+    status, launches = recorded("softmax", dt, rows, cols, ld, off)
+    (name, *_), = launches
+    which, *want = kernel.split()
+    got = re.search(r"softmax_%s_rows_kernelILi%d" % (which, dt) + r"ELi(\d+)" * len(want) + "E", name)
+    assert status == 0 and got and list(got.groups()) == want, name

@@ -244,3 +244,32 @@ def test_row_reductions_on_and_off_boundaries(hip, dt, tdt):
                 torch.cuda.synchronize()
                 want = x[:, :cols].float().sum(1) if kind == "add" else x[:, :cols].float().amin(1)
                 assert torch.equal(d[:rows].float(), want) and float(d[rows]) == 7.0, (rows, cols, ld, shift, kind)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt,tdt,tol", [(O.F32, "float32", 2e-5), (O.F16, "float16", 2e-3), (O.BF16, "bfloat16", 8e-3)])
+def test_softmax_of_whole_groups(hip, dt, tdt, tol):
+    """rows of whole groups, on 128-byte lines and off them, at the edges of what a number of groups per lane holds, up to 56 MiB and beyond, into another matrix and in place; what lies between
+    the rows stays as it is.  Bar: that of the other softmax tests."""
+    import torch
+    tdt = getattr(torch, tdt)
+    es = torch.empty(0, dtype=tdt).element_size()
+    G = 16 // es
+    g = torch.Generator(device="cuda").manual_seed(13)
+    stream = torch.cuda.current_stream().cuda_stream
+    views = [(5, G * k, pad) for k in (1, 3, 64, 65, 128, 129, 256, 257, 512, 513, 768, 769, 1024, 1025, 1536, 1537, 2048, 2049, 3072, 3073, 4096) for pad in (0, G)]
+    views += [(1000, 24, 0), (1000, G, G), (-(-(56 << 20) // (512 * 16)) + 1, 512 * G, 0), (-(-(120 << 20) // (600 * 16)), 600 * G, 0)]
+    for rows, cols, pad in views:
+        ld = cols + pad
+        x = torch.full((rows, ld), float("nan"), device="cuda", dtype=tdt)
+        x[:, :cols] = (torch.randn(rows, cols, device="cuda", generator=g) * 3).to(tdt)
+        z = x[:, :cols].double() * (1.25 * 0.6931471805599453)
+        want = torch.softmax(z, 1)
+        scale = torch.maximum(want, want.square().mean().sqrt())
+        for y in (torch.full_like(x, 5.0), x):
+            beside = y[:, cols:].clone()
+            hip.softmax(dt, x.data_ptr(), ld, y.data_ptr(), ld, rows, cols, 1.25, None, stream)
+            torch.cuda.synchronize()
+            assert bool(((y[:, :cols].double() - want).abs() <= tol * scale + (2.0 ** -25 if dt == O.F16 else 0)).all()), (rows, cols, ld)
+            assert torch.equal(y[:, cols:].nan_to_num(3.0), beside.nan_to_num(3.0)), (rows, cols, ld)
+        del z, want, scale
