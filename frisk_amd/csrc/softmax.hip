@@ -108,9 +108,10 @@ template <bool SUM, int THREADS> __device__ __forceinline__ float block_all(floa
 // elements before it that fill it up (which enter the sum as their own lane's): every access is 16 bytes of the row and all loads of a row are under way
 // together.  Fetched element by element behind the others, that group held up every row by a memory latency: us before / now, f16 10069 x 4946 49.5 / 33.7,
 // 2490 x 2453 11.8 / 6.9, 870 x 16370 20.0 / 10.4 (with 512 lanes: 12.5 with 256), f32 5531 x 1315 17.6 / 10.6, 394 x 9229 (two launches before) 11.9 / 6.9;
-// rows that are whole groups gain by the shorter reductions and what HELD says, f16 8192 x 8192 45.3 / 38.9, which a plain copy takes 39 for.
+// rows that are whole groups gain by the shorter reductions, f16 8192 x 8192 47.3 / 43.0, which a plain copy takes 39 for.
 // HELD: rows of whole groups on 16-byte boundaries know of no other group.  On 128-byte lines and up to 56 MiB they are read past the caches (f16 4096 x 4096 out of the last-level cache 10.6 us through
-// the caches, 9.0 past them, f32 3000 x 4096 15.5 / 13.4), beyond through them (4096 x 8192 from memory 20.6 us, 23.2 past them, 8192 x 8192 38.9 / 42.7).  Others are read through the caches (870 x 16370 10.4,
+// the caches, 9.0 past them, f32 3000 x 4096 15.5 / 13.4), beyond through them (4096 x 8192 20.6 us, 23.2 past them), and past them again where the last-level cache does not hold the view beside its result (8192 x 8192
+// behind the pass that wrote it 43.9 through them, 43.0 past them).  Others are read through the caches (870 x 16370 10.4,
 // 11.9 past them), and past them in views that the last-level cache does not hold beside their result; there, where rows start off 16-byte boundaries, the groups start at the first boundary, what lies
 // before it being a group that overlaps like the last one: stores that cross lines half way cost memory traffic (4426 x 15161 f16 54.9 at the rows' starts, 47.5 so; out of the cache 7.1 either way, 545 x 12163).
 enum HeldRows { HELD_WHOLE_PAST, HELD_WHOLE, HELD_CACHED, HELD_FROM_BOUNDARY };
@@ -322,7 +323,7 @@ __global__ void __launch_bounds__(256) softmax_split_write_kernel(const typename
 }
 
 // groups of a row that a work-group holds, bytes of a view from which on its rows stream past the caches (with the result they are most of the 256 MiB of
-// the last-level cache), and bytes up to which rows of whole groups on lines do
+// the last-level cache), and bytes up to which rows of whole groups on lines do too
 constexpr int64_t kHeldGroups = 4096, kStreamedBytes = (int64_t)112 << 20, kPastBytes = (int64_t)56 << 20;
 
 template <int DT> hipError_t launch_typed(const void* src, int64_t sld, void* dst, int64_t dld, int64_t rows, int64_t cols, float c, float* lse, float* partial,
@@ -357,7 +358,7 @@ template <int DT> hipError_t launch_typed(const void* src, int64_t sld, void* ds
   if (groups <= kHeldGroups) {
     const int64_t bytes = rows * cols * (int64_t)sizeof(T);
     const uintptr_t starts = (uintptr_t)x | (uintptr_t)y | sld * sizeof(T) | dld * sizeof(T);
-    const bool whole = cols % G == 0 && starts % 16 == 0, past = whole && starts % 128 == 0 && bytes <= kPastBytes, large = !whole && bytes > kStreamedBytes;
+    const bool whole = cols % G == 0 && starts % 16 == 0, past = whole && (bytes > kStreamedBytes || (starts % 128 == 0 && bytes <= kPastBytes)), large = !whole && bytes > kStreamedBytes;
     const int64_t most = groups + (large ? 1 : 0);  // a row that starts off a boundary may have a group more
     auto launch = [&](auto kernel, int threads) { hipLaunchKernelGGL(kernel, dim3(grid), dim3(threads), 0, s, x, sld, y, dld, rows, (int)cols, c, lse); };
 #define FRISK_SOFTMAX_HELD(NPT, THREADS) \

@@ -191,10 +191,11 @@ template <int KIND> __device__ __forceinline__ float wave_reduce(float v) {
 // With gridDim.y == 1 the result goes to dst (combined with the old value unless clear), else to partial[y][row].
 // A row's last group, where it is not whole, is fetched first, with the elements before it that fill it up, which are left out: every load is 16 bytes of the row, those of a lane are under way
 // together, and the loop over the whole groups knows nothing of it.  us element by element behind the loop / as a group of the loop / so, from memory: f16 3000 x 4095 9.7 / 7.3 / 7.3, 2490 x 2453
-// 7.0 / 5.4 / 5.1, 10069 x 4946 20.2 / 18.4 / 16.1, f32 5531 x 1315 10.0 / 7.8 / 7.6; rows of whole groups, f16 2177 x 8944 8.4 / 9.8 / 8.4, 4096 x 8192 11.5 / 12.4 / 11.6.
-// LOADS: rows on 16-byte boundaries are read past the caches (through them f16 4096 x 8192 from the last-level cache 11.2, 9.4 so, f32 3000 x 4096 8.8 / 6.8); off them, groups that straddle 128-byte lines would
-// be fetched twice: through the caches in views that the last-level cache may hold (f16 2490 x 4453 out of it 5.14 past them, 4.96 so; f32 5531 x 1315 6.5 / 6.3), and beyond, past them with the groups starting at a row's first
-// boundary, what lies before it being a group that overlaps like the last (bf16 6199 x 10825 27.4 at the rows' starts, 21.3 so).
+// 7.0 / 5.4 / 5.1, 10069 x 4946 20.2 / 18.4 / 16.1, f32 5531 x 1315 10.0 / 7.8 / 7.6; rows of whole groups, f16 2177 x 8944 8.4 / 9.8 / 8.7, 1024 x 16384 7.2 / 8.4 / 7.3.
+// LOADS: views of up to 64 MiB are read through the caches, where the call behind often finds them: cast, row sums, (x - s c) g + b and softmax in a row of 4096 x 8192 f16 93.6 us so, 96.8 with sums
+// past the caches, f32 3029 x 3796 60.8 / 64.5, 131 drawn views 1.003 times as fast.  (On their own, rows on 16-byte boundaries would be read sooner past them: out of the last-level cache f16 4096 x 8192 9.4 us,
+// 11.2 so, from memory 11.6 / 12.3; off them, groups that straddle 128-byte lines are fetched twice there, 2490 x 4453 5.14 us, 4.96 so.)  Beyond, past them, with the groups starting at a row's first
+// boundary where rows start off one, what lies before it being a group that overlaps like the last (bf16 6199 x 10825 27.4 at the rows' starts, 21.3 so).
 enum RowLoads { LOADS_CACHED, LOADS_PAST, LOADS_FROM_BOUNDARY };
 template <int DT, int KIND, int THREADS, int LOADS> __global__ void __launch_bounds__(THREADS)
 reduce_rows_kernel(const typename Elem<DT>::T* src, int64_t rows, int64_t cols, int64_t ld, int clear, typename Elem<DT>::T* dst, float* partial) {
@@ -549,9 +550,9 @@ template <int DT, int KIND> hipError_t reduce_t(const void* src, int64_t rows, i
       const bool wide = gpr > 1536 || (gpr > 1024 && rows <= 1024);
       auto launch = [&](auto kernel, int threads) { hipLaunchKernelGGL(kernel, grid, dim3(threads), 0, s, (const T*)src, rows, cols, ld, clear, (T*)dst, partial); };
 #define FRISK_REDUCE_ROWS(LOADS) { if (wide) launch(reduce_rows_kernel<DT, KIND, 512, LOADS>, 512); else launch(reduce_rows_kernel<DT, KIND, 256, LOADS>, 256); }
-      if (aligned) FRISK_REDUCE_ROWS(LOADS_PAST)
-      else if (large) FRISK_REDUCE_ROWS(LOADS_FROM_BOUNDARY)
-      else FRISK_REDUCE_ROWS(LOADS_CACHED)
+      if (!large) FRISK_REDUCE_ROWS(LOADS_CACHED)
+      else if (aligned) FRISK_REDUCE_ROWS(LOADS_PAST)
+      else FRISK_REDUCE_ROWS(LOADS_FROM_BOUNDARY)
 #undef FRISK_REDUCE_ROWS
     }
   } else if (tall) {

@@ -130,11 +130,11 @@ def test_column_reductions_in_one_launch_or_in_slices(recorded, dt, rows, cols, 
     (R.F16, 20000, 1000, 1000, 0, "short 2 0"), (R.F16, 20000, 1003, 1003, 0, "short 2 1"), (R.BF16, 5878, 864, 865, 2, "short 2 0"), (R.F32, 7313, 464, 464, 0, "short 2 0"), (R.F16, 100000, 24, 24, 0, "short 1 0"),
     (R.F16, 100000, 27, 27, 0, "short 1 1"), (R.F16, 100000, 7, 8, 0, "short 1 2"), (R.F32, 300000, 3, 3, 0, "short 1 2"), (R.F32, 5000, 1023, 1024, 0, "short 4 1"), (R.F32, 5000, 1024, 1024, 0, "short 4 0"),
     # <lanes, through the caches 0 / past them 1 / past them from a row's first boundary on 2>
-    (R.F16, 4096, 8192, 8192, 0, "rows 256 1"), (R.F32, 3000, 4096, 4096, 0, "rows 256 1"), (R.F16, 8192, 8192, 8192, 0, "rows 256 1"), (R.F16, 3000, 4095, 4096, 0, "rows 256 1"), (R.F16, 3000, 4095, 4095, 0, "rows 256 0"),
-    (R.F16, 4096, 8192, 8192, 2, "rows 256 0"), (R.F16, 10069, 4946, 4946, 0, "rows 256 2"), (R.F16, 8192, 8192, 8192, 2, "rows 256 2"), (R.F16, 2177, 8944, 8944, 0, "rows 256 1"), (R.BF16, 1024, 9000, 9000, 0, "rows 512 1"),
-    (R.BF16, 1025, 9000, 9000, 0, "rows 256 1"), (R.F32, 4000, 6144, 6144, 0, "rows 256 1"), (R.F32, 4000, 6148, 6148, 0, "rows 512 1"), (R.F16, 4426, 15161, 15161, 0, "rows 512 2"), (R.F32, 394, 9229, 9229, 0, "rows 512 0")])
+    (R.F16, 4096, 8192, 8192, 0, "rows 256 0"), (R.F32, 3000, 4096, 4096, 0, "rows 256 0"), (R.F16, 8192, 8192, 8192, 0, "rows 256 1"), (R.F16, 8200, 4095, 4096, 0, "rows 256 1"), (R.F16, 3000, 4095, 4095, 0, "rows 256 0"),
+    (R.F16, 10069, 4946, 4946, 0, "rows 256 2"), (R.F16, 8192, 8192, 8192, 2, "rows 256 2"), (R.F16, 2177, 8944, 8944, 0, "rows 256 0"), (R.BF16, 1024, 9000, 9000, 0, "rows 512 0"),
+    (R.BF16, 1025, 9000, 9000, 0, "rows 256 0"), (R.F32, 4000, 6144, 6144, 0, "rows 256 1"), (R.F32, 4000, 6148, 6148, 0, "rows 512 1"), (R.F16, 4426, 15161, 15161, 0, "rows 512 2"), (R.F32, 394, 9229, 9229, 0, "rows 512 0")])
 def test_row_reductions_by_what_their_rows_are(recorded, dt, rows, cols, ld, off, kernel):
-    """rows of whole groups on kernels that know of no others, rows on 16-byte boundaries past the caches, 512 lanes where they have work"""
+    """rows of whole groups on kernels that know of no others; past the caches beyond 64 MiB; 512 lanes where they have work"""
     status, launches = recorded("reduce", dt, rows, cols, ld, 1, off, 1)
     (name, *_), = launches
     which, a, b = kernel.split()
@@ -146,8 +146,8 @@ def test_row_reductions_by_what_their_rows_are(recorded, dt, rows, cols, ld, off
     # <groups a lane, rows of whole groups 0 / a part 1 / less than a group 2>
     (R.F16, 32768, 512, 512, 0, "short 1 0"), (R.F16, 100000, 27, 27, 0, "short 1 1"), (R.F16, 100000, 7, 8, 0, "short 1 2"), (R.F32, 300000, 3, 3, 0, "short 1 2"), (R.F16, 8192, 1024, 1025, 2, "short 2 0"),
     (R.BF16, 14242, 790, 790, 0, "short 2 1"), (R.F32, 8192, 1024, 1024, 0, "short 4 0"), (R.F32, 8192, 1023, 1024, 0, "short 4 1"),
-    # <groups a lane, lanes, whole groups on lines past the caches 0 / whole groups 1 / any through them 2 / any past them from a row's first boundary on 3>
-    (R.F16, 4096, 4096, 4096, 0, "held 2 256 0"), (R.F32, 3000, 4096, 4096, 0, "held 2 512 0"), (R.F16, 3584, 8192, 8192, 0, "held 2 512 0"), (R.F16, 3585, 8192, 8192, 0, "held 2 512 1"), (R.F16, 8192, 8192, 8192, 0, "held 2 512 1"),
+    # <groups a lane, lanes, whole groups past the caches 0 / through them 1 / any through them 2 / any past them from a row's first boundary on 3>
+    (R.F16, 4096, 4096, 4096, 0, "held 2 256 0"), (R.F32, 3000, 4096, 4096, 0, "held 2 512 0"), (R.F16, 3584, 8192, 8192, 0, "held 2 512 0"), (R.F16, 3585, 8192, 8192, 0, "held 2 512 1"), (R.F16, 7168, 8192, 8192, 0, "held 2 512 1"), (R.F16, 7169, 8192, 8192, 0, "held 2 512 0"), (R.F16, 8192, 8192, 8200, 0, "held 2 512 0"),
     (R.F16, 4096, 4000, 4000, 0, "held 2 256 1"), (R.F16, 4096, 4096, 4096, 16, "held 2 256 1"), (R.F16, 4096, 4096, 4096, 2, "held 2 256 2"), (R.F16, 4096, 4095, 4096, 0, "held 2 256 2"), (R.F16, 8192, 8192, 8193, 0, "held 3 512 3"),
     (R.F16, 870, 16370, 16370, 0, "held 4 512 2"), (R.F16, 4426, 15161, 15161, 0, "held 4 512 3"), (R.F16, 64, 32768, 32768, 0, "held 9 512 0")])
 def test_softmax_by_what_its_rows_are(recorded, dt, rows, cols, ld, off, kernel):
