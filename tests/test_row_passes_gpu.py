@@ -273,3 +273,25 @@ def test_softmax_of_whole_groups(hip, dt, tdt, tol):
             assert bool(((y[:, :cols].double() - want).abs() <= tol * scale + (2.0 ** -25 if dt == O.F16 else 0)).all()), (rows, cols, ld)
             assert torch.equal(y[:, cols:].nan_to_num(3.0), beside.nan_to_num(3.0)), (rows, cols, ld)
         del z, want, scale
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("cols", [4100, 5003, 6144])
+def test_sums_of_rows_on_256_lanes_are_no_further_from_the_exact_ones_than_on_512(hip, cols):
+    """fp32 rows of 1025 to 1536 groups, more than 1024 of them, against the error of 512 lanes that add their elements one after the other, then in pairs"""
+    import torch
+    rows, lanes = 2000, 512
+    vals = O.normal(rows * cols, 65, 0, 1.0).astype(np.float32).reshape(rows, cols)
+    exact = vals.astype(np.float64).sum(1)
+    chains = np.zeros((rows, lanes), np.float32)
+    for c in range(0, cols, 4 * lanes):
+        for e in range(4):
+            part = vals[:, c + e:min(c + 4 * lanes, cols):4]
+            chains[:, :part.shape[1]] += part
+    while chains.shape[1] > 1:
+        half = chains.shape[1] // 2
+        chains = chains[:, :half] + chains[:, half:]
+    x, d = torch.from_numpy(vals).cuda(), torch.empty(rows, device="cuda")
+    hip.reduce(O.F32, x.data_ptr(), rows, cols, cols, 1, "add", True, d.data_ptr(), None, 0, torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    assert np.linalg.norm(d.cpu().numpy().astype(np.float64) - exact) <= np.linalg.norm(chains[:, 0].astype(np.float64) - exact)
