@@ -71,6 +71,7 @@ struct EwArgs {
   int code[2 * kChunk];
   float imm[2 * kChunk];
   RowScale scale0, scale1;  // HELD_SCALED
+  int past;                 // halves: stores pass the caches
 };
 
 // ---- the interpreter loop.  EACH: one instruction per column.  Handlers lie 256 bytes apart, in the order of Step; NEXT fetches
@@ -422,10 +423,8 @@ __attribute__((amdgpu_waves_per_eu(four_waves(DT, HELD, DEPTH, ROWS == ROWS_UNIF
           if (mine_a < 4) store_half<decltype(streamed)::value>(out_at, top, 0, mine_a);
           if (mine_b < 4) store_half<decltype(streamed)::value>(out_at + apart * 4, top, 1, mine_b);
         };
-        // past the caches, but for rows of up to 32 columns, whose halves are parts of lines
         if (row < p.rows) {
-          if constexpr (ROWS == ROWS_UNIFORM) store(StreamedTag<true>{});
-          else if (lanes_log2 >= 3) {
+          if (p.past) {
             asm volatile("");  // (these keep the compiler from making one store of the two, which is then not streamed)
             store(StreamedTag<true>{});
           } else {
@@ -556,6 +555,13 @@ template <int DT> void launch_held(int held, bool scaled, const dim3& grid, cons
 
 }  // namespace
 
+// 32-bit bodies store past the caches, but for those of one operand that walks the rows and of values of the row, which as a rule have just been reduced from it, in views of more than kPastUpTo bytes and up to
+// kPastFrom, the size of the last-level cache: between the reduction that has read the operand and a softmax that reads the result, stores through the caches leave more to be found there.  us past / through, cast, row
+// sums, (x - s c) g + b and softmax together: 8192 x 8192 324 / 319 (319 before stores passed the caches; the body alone in that row 98.5 / 88.3), 16384 x 4096 314 / 307, 6000 x 8000 237 / 231, 4096 x 8192 171 / 163, 4111 x 4501
+// 109 / 106, 50000 x 400 113 / 109, 100000 x 600 294 / 284; 4096 x 4096 and 3029 x 3796 even; 16384 x 16384 1294 / 1313.  On their own, operands from memory, bodies are 1 to 4 % faster past the caches ((x - s c) g + b of
+// 8192 x 8192 96.8 / 98.4, exp2(x) c 94.7 / 98.4, x + y 137.3 / 138.6).  Rows of up to 32 columns, whose halves are parts of lines, never pass them.
+constexpr int64_t kPastUpTo = (int64_t)64 << 20, kPastFrom = (int64_t)256 << 20;
+
 hipError_t launch_elementwise(const EwParams& given, hipStream_t s) {
   EwParams p = given;
   // A dense view is one row, down which no lane walks and fetches ahead.  A 16-bit one that gives every lane more than one group is folded to
@@ -637,6 +643,8 @@ hipError_t launch_elementwise(const EwParams& given, hipStream_t s) {
   a.head = operand(prog.head); a.walk2 = operand(prog.walk2);
   a.row0 = operand(prog.row0); a.row1 = operand(prog.row1); a.col0 = operand(prog.col0); a.col1 = operand(prog.col1);
   a.scale0 = prog.scale0; a.scale1 = prog.scale1;
+  const int64_t bytes = p.rows * p.cols * 4;
+  a.past = lanes_log2 >= 3 && (prog.walk2 >= 0 || !per_row || bytes <= kPastUpTo || bytes > kPastFrom);
   a.n_steps = prog.n;
   __builtin_memcpy(a.code, prog.code, sizeof a.code);
   __builtin_memcpy(a.imm, prog.imm, sizeof a.imm);

@@ -295,3 +295,20 @@ def test_sums_of_rows_on_256_lanes_are_no_further_from_the_exact_ones_than_on_51
     hip.reduce(O.F32, x.data_ptr(), rows, cols, cols, 1, "add", True, d.data_ptr(), None, 0, torch.cuda.current_stream().cuda_stream)
     torch.cuda.synchronize()
     assert np.linalg.norm(d.cpu().numpy().astype(np.float64) - exact) <= np.linalg.norm(chains[:, 0].astype(np.float64) - exact)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,cols", [(4100, 4096), (4097, 4097), (8, 2097153), (50000, 400), (45003, 403), (600000, 33), (600000, 31), (9000, 7500)])
+def test_32_bit_bodies_of_views_on_either_side_of_64_and_256_mib(hip, rows, cols):
+    """stores through the caches and past them, of rows of whole groups and not, longer than a wave and shorter, into another matrix and into its own operand; every operation rounds once, as torch's do"""
+    import torch
+    g, ld, stream = torch.Generator(device="cuda").manual_seed(14), cols + 1, torch.cuda.current_stream().cuda_stream
+    x = torch.randn(rows, ld, device="cuda", generator=g)
+    r, c = torch.randn(rows, device="cuda", generator=g), torch.randn(cols, device="cuda", generator=g)
+    desc = hip.make_elementwise_desc([("input", 0), ("input", 1), ("const", 0.5), "mul", "sub", ("input", 2), "mul"], [(O.F32, ld, 1), (O.F32, 1, 0), (O.F32, 0, 1)], O.F32, rows, cols, out_ld=ld)
+    want = (x[:, :cols] - r[:, None] * 0.5) * c
+    for out in (torch.full_like(x, 3.0), x):
+        beside = out[:, cols:].clone()
+        hip.elementwise(desc, [x.data_ptr(), r.data_ptr(), c.data_ptr()], out.data_ptr(), stream)
+        torch.cuda.synchronize()
+        assert torch.equal(out[:, :cols], want) and torch.equal(out[:, cols:], beside)
