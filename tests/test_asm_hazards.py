@@ -187,3 +187,16 @@ def test_stores_under_a_condition_do_not_wait_for_everything_under_way(tmp_path)
     assert subprocess.run(cmd, capture_output=True).returncode == 0
     listing = out.read_text()
     assert "scratch_" not in listing and listing.count("global_store_dwordx4") > 400 and len(re.findall(r"vmcnt\(0\)", listing)) < 200
+
+
+@pytest.mark.skipif(not (os.path.exists(HIPCC) or shutil.which("hipcc")), reason="needs hipcc to produce the ISA listing")
+def test_the_smallest_fp32_products_have_one_body(tmp_path):
+    """the fp32 edge tiles whose waves split K: 2184 instructions, 2508 with bodies of their own for whole tiles, those that C ends in and a few columns"""
+    src, out = tmp_path / "edge.hip", tmp_path / "edge.s"
+    src.write_text('#include "gemm_kernel.hip.inc"\nnamespace frisk {\n'
+                   "template __global__ void gemm_kernel<GemmCfg<FRISK_F32, 0, 0, 32, 32, 128, 1, 1, 2, false, false, 4, 2, 32, true>>(GemmParams);\n}\n")
+    cmd = [HIPCC if os.path.exists(HIPCC) else "hipcc", "--offload-arch=gfx950", "-O3", "-std=c++17", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+           "-I" + os.path.join(ROOT, "include"), "-I" + CSRC, "-Wno-unused-command-line-argument", "--cuda-device-only", "-S", str(src), "-o", str(out)]
+    assert subprocess.run(cmd, capture_output=True).returncode == 0
+    listing = out.read_text()
+    assert "scratch_" not in listing and 1500 < len(re.findall(r"^\s+(?:[sv]|global|flat|ds|buffer)_", listing, re.M)) <= 2300
