@@ -741,7 +741,7 @@ static int follow_up(const std::vector<Variant>& list, const KernelEntry* k, con
 // Problems whose M and N are multiples of 256 are not here: they have split-K kernels of their own (2048x1280x8192 runs in 4 slices).
 // Error against 64 bits, fp32 C of fp16 1137x2880x11968: 6.9e-7 in one chain, 3.5e-7 in four.
 //
-// The least K of 16- and 8-bit types: where operands from memory, or the weights alone, gain (0.97 to 1.00 in a few of 150 measured at a line).  With both operands in the last-level cache, as in a
+// The least K of 16- and 8-bit types: where operands from memory, or the weights alone, gain (0.92 to 1.00 in a few of 300 measured at a line: fp16 2043x1144x7488 NN with the weights alone 46.7 / 50.9).  With both operands in the last-level cache, as in a
 // call repeated on the same buffers, a product at its line runs at 0.82 to 1.35 times its former speed, at 1.3 times that K at 0.92 to 1.42.  At the lines (and beyond), all from memory / the weights alone / all
 // from the cache, three to seven shapes in two layouts:
 struct DeepLine { int64_t k16, k8, k8_nk; };  // k8_nk: of 8-bit types against B [N][K]

@@ -9,7 +9,7 @@
 // assembly over fixed registers: a step is two lane reads of the program, a jump to its handler and 8 vector instructions in
 // place, the operand picked by the register index mode.  (As a C++ switch the compiler joins the values of all cases after every
 // step by register moves: 327 vector, 300 scalar and 120 branch instructions per group of 8 columns for (x - s * c) * g + b; here
-// 109, 125 and 34.)  That body on 8192 x 8192 f16: 137 us before, 45 now (a plain copy: 39); log2(max(x, c) / (x + c)), bound by
+// 109, 125 and 34.)  That body on 8192 x 8192 f16: 137 us before, 42.5 now on the same buffers, 49.4 with operands from memory (a plain copy: 38.8, 41.7); log2(max(x, c) / (x + c)), bound by
 // the vector pipe in its division, 123 -> 69.5; x + y 80 -> 58; rows off 16-byte boundaries (4095 x 8191) 369 -> 29.
 // Operands that are the same for every row stay in registers while the lane's columns do, values of one per row stay one
 // register, and what the next groups need from memory is fetched while the current one is evaluated.  All arithmetic is
@@ -41,8 +41,8 @@ constexpr int kSlotS0 = 0, kSlotX = 8, kSlotCol0 = 16, kSlotCol1 = 24, kSlotWalk
 constexpr int kChunk = 64;  // steps in one register of a wave, one per lane; STEP_MORE goes on to the second register
 // What an operand of one value per row goes through before the steps see it: value * mul + add, one operation with a constant (or none) whose other part changes
 // nothing, so that it rounds once as that operation does.  Done on a row's value it is one instruction a group; as steps on eight columns a lane, with the value
-// below the top kept meanwhile, it was four steps in place of one: (x - s c) g + b of 8192 x 8192 f16 48.7 us as steps, 45.1 so, bf16
-// 3077 x 3724 12.1 / 10.9, 12208 x 658 12.4 / 10.8, 6199 x 10825 54.5 / 51.9; f32, which memory bounds, even.  Programs without such a constant run on kernels without the multiply-add
+// below the top kept meanwhile, it was four steps in place of one: (x - s c) g + b as steps / so, from memory, 8192 x 8192 f16 51.1 us / 49.4, bf16
+// 3077 x 3724 12.4 / 11.5, 12208 x 658 12.4 / 10.9, 6199 x 10825 even (on the same buffers 49.6 / 44.5); f32, which memory bounds, even.  Programs without such a constant run on kernels without the multiply-add
 // (HELD_ALL): under it they were 1 to 2 % slower, f16 100000 x 24 x g + y 6.9 us, 6.2 without, x s 6.0 / 5.6, 3168 x 2891 (x - s) g + b 13.65 / 13.3, x g + b 12.93 / 12.69, 4096 x 4096 15.15 / 14.95.
 struct RowScale { float mul = 1.f, add = -0.f; };
 struct EwSteps {
@@ -253,9 +253,9 @@ __attribute__((amdgpu_waves_per_eu(four_waves(DT, HELD, DEPTH, ROWS == ROWS_UNIF
   const int64_t groups = (p.cols + V - 1) / V, slabs = (groups + lanes - 1) >> lanes_log2, row_blocks = (p.rows + row_step - 1) / row_step;
   constexpr bool narrow = ROWS == ROWS_NARROW;
   // HALVES: a lane's 8 columns of 32-bit operands are 4 and 4, a slab's lanes side by side in either half, so that every access of a wave is one run of memory.  (With a
-  // lane's two accesses side by side each takes half of every line, and stores past the caches, which halves allow, would write lines twice.  us side by side / so, f32: (x - s c) g + b of
-  // 4096 x 4096 29.1 / 23.0, 2875 x 5713 30.3 / 25.5, 20000 x 300 15.3 / 11.6, 8192 x 8192 104.2 / 100.3, exp2(x) c of 4095 x 8191 50.4 / 42.0, x + y of 1500 x 2000 8.8 / 7.5; halves with stores through
-  // the caches 26.9, 28.8, 14.2.)
+  // lane's two accesses side by side each takes half of every line, and stores past the caches, which halves allow, would write lines twice.  us side by side / so, f32 from memory: (x - s c) g + b of
+  // 4096 x 4096 28.9 / 27.7, 2000 x 2500 15.7 / 13.2, 4111 x 4501 37.6 / 33.3, 8192 x 8192 102.4 / 96.8, exp2(x) c of 4111 x 4501 29.6 / 25.7, x + y of 1500 x 2000 9.9 / 9.0; halves with stores through
+  // the caches 27.2, 14.5, 35.4, 98.4, 27.7, 9.6.)
   constexpr bool HALVES = DT == FRISK_F32 && !narrow;
   // step i of a chunk of the program in lane i: a lane read instead of a dependent scalar load
   int code_reg[2] = {p.code[threadIdx.x & 63], 0}, imm_reg[2] = {__builtin_bit_cast(int, p.imm[threadIdx.x & 63]), 0};
